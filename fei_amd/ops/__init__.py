@@ -66,7 +66,8 @@ def _try_load() -> None:
                                _i, _i, _vp]
     lib.fei_advance.argtypes = [_vp, _vp, _i, _i, _vp]
     lib.fei_attn_prefill.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp,
-                                     _i, _i, _i, _i, _i, _i, _f, _i, _l, _vp]
+                                     _i, _i, _i, _i, _i, _i, _f, _i, _l, _i,
+                                     _vp, _vp, _vp]
     lib.fei_mfma_probe.argtypes = [_vp, _vp, _vp, _vp]
     lib.fei_gemv.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp]
     lib.fei_gemm_m8.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp]
@@ -332,11 +333,30 @@ def attn_prefill(q, k_cache, v_cache, pos0, scale: Optional[float] = None,
     assert q.stride(3) == 1 and q.stride(2) == D
     assert q.stride(0) == S * q.stride(1)
     assert out.is_contiguous()
+    if not q.numel():
+        return out
+    splits = _prefill_splits(B * Hkv, S * (Hq // Hkv), k_cache.shape[2])
+    po = pml = None
+    if splits > 1:
+        ws = torch.empty(B * S * Hq * splits * (D + 2), dtype=torch.float32,
+                         device=q.device)
+        po, pml = _ptr(ws), _ptr(ws) + B * S * Hq * splits * D * 4
     lib.fei_attn_prefill(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
                          _ptr(pos0), _ptr(kv_len), B, S, Hq, Hkv, D,
                          k_cache.shape[2], scale, 1 if causal else 0,
-                         q.stride(1), _stream())
+                         q.stride(1), splits, po, pml, _stream())
     return out
+
+
+def _prefill_splits(heads: int, rows: int, max_seq: int) -> int:
+    """Shares of the keys that the prompt attention's blocks of 128 rows are
+    cut into, so that few rows over many keys fill the chip's 512 places (two
+    blocks per CU). How many keys there are is known on the device only; the
+    kernel uses fewer shares where one would have under three tiles of 64."""
+    blocks = heads * -(-rows // 128)
+    if blocks > 192:
+        return 1
+    return max(1, min(16, -(-512 // blocks), max_seq // 192))
 
 
 def _ref_bidir(q, k_cache, v_cache, kv_len, scale):

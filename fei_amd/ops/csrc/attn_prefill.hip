@@ -1,207 +1,333 @@
-// Flash-style causal GQA prefill attention for gfx950 (MFMA
-// mfma_f32_16x16x32_bf16, LDS-staged K/V tiles, online softmax).
-// Semantics: fei_amd/ops/reference.py::attn_prefill — q [B,S,Hq,D] (roped),
-// caches [B,Hkv,max_seq,D] already hold the roped K and V for positions
-// [0, pos0+S); q token s attends cache [0, pos0+s] (causal) or [0, kv_len)
-// (bidirectional, used by the bge encoder path).
+// Causal (or bidirectional) GQA attention of prompt rows over contiguous
+// caches, gfx950. Semantics: fei_amd/ops/reference.py::attn_prefill - q
+// [B,S,Hq,D] (roped), caches [B,Hkv,max_seq,D] already hold the roped K and V
+// for positions [0, pos0+S); q token s attends cache [0, pos0+s] (causal) or
+// [0, kv_len) (bidirectional, the encoder's).
 //
-// Structure (v1, correctness-first; guide: cdna_hip_programming.md §5/§B):
-//   grid (ceil(S/64), Hq, B); block 256 = 4 waves; wave w owns q rows
-//   [qt*64 + 16w, +16). K/V tiles of 32 keys staged in LDS, shared by the
-//   4 waves. Per tile: QK^T = 4 MFMAs per 16-key chunk (K-dim = D in steps
-//   of 32), per-row online softmax in-register (16-lane shfl groups), P
-//   staged through LDS to re-shape C-layout -> A-layout, PV = D/16 MFMAs.
+// A row is a (token, query head) pair of one kv head, token-major, so that all
+// heads of a group share the tiles of K and V. A block takes 128 rows, a wave
+// 32 of them, over tiles of 64 keys that direct loads bring to LDS one tile
+// ahead. Scores are computed transposed (K times Q^T, 32x32x16): a lane has 32
+// scores of ONE row, so that the softmax needs a single exchange between lanes,
+// and its weights are, as they lie, the second operand of V^T times P^T, whose
+// sums again belong to the lane's row. K and V lie in LDS as in memory but for
+// a permutation of a row's 16-byte (K) or 32-byte (V) places by the row, which
+// spreads the fragment reads over the banks; V is turned by the transposing
+// LDS read.
 //
-// Fragment maps used (verified on hardware by k_mfma_probe / test_ops_gpu):
-//   A[16x32]: lane l -> A[l&15][8*(l>>4)+j], j=0..7
-//   B[32x16]: lane l -> B[8*(l>>4)+j][l&15]
-//   C[16x16]: lane l, reg r -> C[4*(l>>4)+r][l&15]
-#include "fei_common.h"
+// What bounds it: per 64 keys a wave has 32 matrix instructions (1024 cycles
+// at D = 128) and about as many cycles of softmax; two blocks per CU overlap
+// the two, and the LDS reads (32 KB a wave) take as long again. Measured against
+// a wave of 16 queries of one head with the values turned on the way into LDS:
+// 2048 tokens, 32/8 heads of 128: 282 -> 50 us (690 TFLOP/s of the causal
+// half); 6 x 1001 tokens, heads of 64: 235 -> 42; 64 x 256, 12 heads of 64,
+// not causal: 59 -> 29; 75 tokens over 1875 keys: 139 -> 20 with splits (24
+// blocks without).
+#include "fei_mma.h"
 
 namespace {
 
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+typedef __attribute__((ext_vector_type(4))) u32 u32x4;
+
+constexpr int ROWS = 128;              // rows per block
+constexpr int KEYS = 64;               // keys per tile
+constexpr float M_NONE = -3.0e38f;     // maximum of a row without keys
+
+__device__ __forceinline__ f32x16 mma32(s16x8 a, s16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+      __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+      0);
+}
+
+// v of this lane and of lane ^ 32
+__device__ __forceinline__ f32x2 both_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(
+      __builtin_bit_cast(u32, v), __builtin_bit_cast(u32, v), false, false);
+  const u32 lo = r[0], hi = r[1];
+  return f32x2{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
+}
+
+// Keys that a block of rows reads: tiles [t0, t1) of n keys, cut into splits of
+// at least three tiles.
+__device__ __forceinline__ void split_tiles(int n, int splits, int split,
+                                            int& t0, int& t1) {
+  const int nt = (n + KEYS - 1) / KEYS;
+  const int per = max((nt + splits - 1) / splits, 3);
+  t0 = split * per;
+  t1 = min(nt, t0 + per);
+}
+
+struct Prefill {
+  const u16 *q, *kc, *vc;
+  u16* out;
+  float *po, *pml;                     // partial results of splits
+  const int *pos0, *kv_len;
+  int S, G, Hkv, heads, tiles, max_seq, causal, splits;
+  float scale;
+  long q_ts;
+};
+
+// Keys that the rows up to r_hi of batch row b see.
+__device__ __forceinline__ int keys_of(const Prefill& a, int b, int r_hi) {
+  const int n = a.causal ? a.pos0[b] + r_hi / a.G + 1 : a.kv_len[b];
+  return min(n, a.max_seq);
+}
+
+// Tile of the j-th block of a kv head. Causal tiles cost as much as they have
+// keys before them. Where all blocks fit on the chip at once (two per CU), the
+// second half takes the light ones upwards, so that a CU's pair costs the same
+// everywhere; otherwise the heavy ones go first.
+__device__ __forceinline__ int tile_of(const Prefill& a, int j) {
+  const int half = (a.tiles + 1) / 2;
+  if (a.causal && a.heads * a.tiles <= 512 && j >= half) return j - half;
+  return a.tiles - 1 - j;
+}
+
+template <int D, bool SPLIT>
+__global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
+  constexpr int KS = D / 16;           // steps of a score product
+  constexpr int DT = D / 32;           // tiles of 32 value columns
+  constexpr int LPR = D / 8;           // 16-byte places of a cache row
+  constexpr int RPI = 64 / LPR;        // rows of a load of 64 lanes
+  constexpr int LOADS = KEYS / RPI / 4;    // a wave's, of K and of V each
+  __shared__ __align__(16) u16 buf[2][2][KEYS * D];
+  const int head = blockIdx.x % a.heads, j = blockIdx.x / a.heads;
+  const int tile = tile_of(a, SPLIT ? j / a.splits : j);
+  const int split = SPLIT ? j % a.splits : 0;
+  const int b = head / a.Hkv, hkv = head - b * a.Hkv;
+  const int R = a.S * a.G, row0 = tile * ROWS;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l31 = lane & 31, h = lane >> 5;
+  const int n = keys_of(a, b, min(row0 + ROWS, R) - 1);
+  const int r = row0 + wid * 32 + l31;
+  const int s = min(r, R - 1) / a.G, g = min(r, R - 1) - s * a.G;
+  const long prow = ((long)head * R + r) * a.splits + split;
+  int t0 = 0, t1 = (n + KEYS - 1) / KEYS;
+  if (SPLIT) {
+    split_tiles(n, a.splits, split, t0, t1);
+    if (t0 >= t1 && split) {           // no keys: the sums are never read
+      if (h == 0 && r < R) *(f32x2*)(a.pml + prow * 2) = f32x2{M_NONE, 0.f};
+      return;
+    }
+  }
+
+  // last key that the lane's row sees; first tile that needs a mask; keys past
+  // the wave's last row are skipped
+  const int lim = a.causal ? min(a.pos0[b] + s, n - 1) : n - 1;
+  const int r_first = min(row0 + wid * 32, R - 1);
+  const int r_last = min(row0 + wid * 32 + 31, R - 1);
+  const int lim_lo = a.causal ? min(a.pos0[b] + r_first / a.G, n - 1) : n - 1;
+  const int lim_hi = a.causal ? min(a.pos0[b] + r_last / a.G, n - 1) : n - 1;
+
+  // a negative scale turns the queries round, a zero one clears them, so that
+  // the largest score stays the largest after scaling
+  const float c = a.scale == 0.f ? 1.f : fabsf(a.scale) * El<u16>::base;
+  const u32 flip = a.scale < 0.f ? 0x80008000u : 0u;
+  const u32 keep = a.scale == 0.f ? 0u : 0xffffffffu;
+  s16x8 fq[KS];
+  {
+    const u16* qp = a.q + ((long)b * a.S + s) * a.q_ts +
+                    (long)(hkv * a.G + g) * D + 8 * h;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      u32x4 v = *(const u32x4*)(qp + k * 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (v[e] ^ flip) & keep;
+      fq[k] = __builtin_bit_cast(s16x8, v);
+    }
+  }
+
+  const u16* kb = a.kc + (long)head * a.max_seq * D;
+  const u16* vb = a.vc + (long)head * a.max_seq * D;
+  const u32 lds =
+      (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)&buf[0][0][0];
+  auto load = [&](int t, int p) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int at = wid * LOADS + i;
+      const int row = at * RPI + lane / LPR, place = lane % LPR;
+      const int off = min(t * KEYS + row, n - 1) * D;
+      const int ck = place ^ (row & 7);
+      const int cv = (((place >> 1) ^ (row & (D / 16 - 1))) << 1) | (place & 1);
+      load_lds(kb + off + ck * 8, lds + (p * 2 * KEYS * D + at * 512) * 2);
+      load_lds(vb + off + cv * 8, lds + ((p * 2 + 1) * KEYS * D + at * 512) * 2);
+    }
+  };
+
+  float m = M_NONE, l = 0.f;
+  f32x16 o[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
+
+  if (t0 < t1) load(t0, 0);
+  for (int t = t0; t < t1; ++t) {
+    const int p = (t - t0) & 1;
+    // the tile is there, and all waves are done with the other buffer
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (t + 1 < t1) load(t + 1, p ^ 1);
+    if (t * KEYS > lim_hi) continue;
+    const u16* kt = buf[p][0];
+    const u16* vt = buf[p][1];
+
+    f32x16 sc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sc[i][e] = 0.f;
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+        sc[i] = mma32(ld8(kt + (i * 32 + l31) * D +
+                          (((k * 2 + h) ^ (l31 & 7)) << 3)),
+                      fq[k], sc[i]);
+    }
+    // register e of sc[i] is key t * 64 + i * 32 + 8 (e / 4) + 4 h + e % 4
+    if (t * KEYS + KEYS - 1 > lim_lo) {
+      const int d = lim - t * KEYS - 4 * h;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (i * 32 + 8 * (e / 4) + e % 4 > d) sc[i][e] = -1.f / 0.f;
+    }
+    float mx = fmaxf(sc[0][0], sc[1][0]);
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(fmaxf(mx, sc[0][e]), sc[1][e]);
+    const f32x2 two = both_halves(mx);
+    mx = fmaxf(two[0], two[1]) * c;
+    // the maximum may lag behind by 2^8: weights and sums are float32 with
+    // room for that, and most tiles leave the sums as they are
+    if (__any(mx > m + 8.f)) {
+      const float mn = fmaxf(m, mx);
+      const float al = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= al;
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[i][e] *= al;
+    }
+    s16x8 fp[4];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float ps = 0.f;
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        u32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int at = hf * 8 + 2 * e;
+          const f32x2 x = {
+              __builtin_amdgcn_exp2f(fmaf(sc[i][at], c, -m)),
+              __builtin_amdgcn_exp2f(fmaf(sc[i][at + 1], c, -m))};
+          ps += x[0] + x[1];
+          w[e] = __builtin_bit_cast(u32, __builtin_convertvector(x, bf16x2));
+        }
+        fp[i * 2 + hf] = __builtin_bit_cast(s16x8, w);
+      }
+      l += ps;
+    }
+    // a lane reads 4 values of a column at a time, in the order of the keys
+    // that its weights have: 16 i + 4 h + 0..3, then + 8
+    const int vr = 4 * h + ((lane & 15) >> 2), vc0 = (lane >> 4) & 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const u16* vp = vt + (i * 16 + vr) * D +
+                        (((dt * 2 + vc0) ^ (vr & (D / 16 - 1))) << 4) +
+                        (lane & 3) * 4;
+        o[dt] = mma32(turn8(vp, vp + 8 * D), fp[i], o[dt]);
+      }
+  }
+
+  const f32x2 lt = both_halves(l);
+  l = lt[0] + lt[1];
+  if (r >= R) return;
+  // column dt * 32 + 8 i + 4 h + 0..3 in registers 4 i .. of o[dt]
+  if (SPLIT) {
+    int u0, u1;
+    split_tiles(n, a.splits, 1, u0, u1);
+    if (u0 < u1) {                     // there are other splits
+      float* po = a.po + prow * D + 4 * h;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          *(f32x4*)(po + dt * 32 + 8 * i) =
+              f32x4{o[dt][4 * i], o[dt][4 * i + 1], o[dt][4 * i + 2],
+                    o[dt][4 * i + 3]};
+      if (h == 0) *(f32x2*)(a.pml + prow * 2) = f32x2{m, l};
+      return;
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  u16* op = a.out + (((long)b * a.S + s) * a.Hkv * a.G + hkv * a.G + g) * D +
+            4 * h;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      u16 v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = El<u16>::st(o[dt][4 * i + e] * inv);
+      __builtin_memcpy(op + dt * 32 + 8 * i, v, sizeof(v));
+    }
+}
+
+// Sums of the splits of a row; one wave per row, rows that one split finished
+// are left alone.
 template <int D>
 __global__ void __launch_bounds__(256)
-k_attn_prefill(const u16* __restrict__ q, const u16* __restrict__ kc,
-               const u16* __restrict__ vc, u16* __restrict__ out,
-               const int* __restrict__ pos0, const int* __restrict__ kv_len,
-               int B, int S, int Hq, int Hkv, int max_seq, float scale,
-               int causal, long q_ts) {
-  constexpr int DC = D / 16;       // d-chunks (8 for D=128)
-  constexpr int KS = D / 32;       // K-dim steps per QK^T mfma chain
-  constexpr int KV = 64;           // keys per LDS tile (one barrier per 64)
-  constexpr int NC = KV / 16;      // 16-key score chunks per tile
-  constexpr int KA = KV / 32;      // P A-fragments per tile (K=32 each)
-  const int qt = blockIdx.x;       // 64-row q tile
-  const int hq = blockIdx.y;
-  const int b = blockIdx.z;
-  const int hkv = hq / (Hq / Hkv);
-  const int tid = threadIdx.x;
-  const int w = tid >> 6;          // wave 0..3
-  const int lane = tid & 63;
-  const int l15 = lane & 15;
-  const int lg = lane >> 4;        // 16-lane group 0..3
-
-  // K tile: row-major with a T2 XOR swizzle (guide Guideline 4): read
-  // column-slice-wise with ds_read_b128, swizzling the 16-byte slot index
-  // by (row&7) spreads each 16-lane group over 8 slots.
-  // V tile: stored TRANSPOSED [col][key] in 8-key blocks so the PV
-  // B-fragment (8 consecutive keys of one column) is ONE 16-byte vector
-  // read — the r02 ablation (experimental/prefill_ablate.hip) measured
-  // the per-element PV gather at 56% of the kernel. The 8-key block
-  // index is XOR-swizzled by (col&7) to break the 128-byte column
-  // stride's bank pattern (<=2-way). The transpose cost moves to the
-  // staging scatter: 8 ds_write_b16 per global vec8 — 4x fewer LDS ops
-  // than the per-element PV reads they replace.
-  __shared__ u16 kt[64][D];
-  __shared__ u16 vtT[D][64];
-  __shared__ u16 p_lds[4][16][64];
-#define SWZ16(row, col8) ((col8) ^ ((row) & 7))
-#define VT_OFF(col, key) \
-  ((col) * 64 + \
-   ((((key) >> 3) ^ ((col) & 7) ^ (((col) >> 3) & 7)) << 3) + ((key) & 7))
-
-  const int p0 = pos0[b];
-  const int q_hi = min(qt * 64 + 64, S);           // exclusive rel row bound
-  const int kv_end = causal ? (p0 + q_hi) : kv_len[b];
-
-  // ---- load Q fragments (row = l&15 within this wave's 16-row block) ----
-  const int qrow_rel = qt * 64 + w * 16 + l15;     // A-fragment row
-  const int qrow_ld = min(qrow_rel, S - 1);        // clamp for tail
-  s16x8 a_q[KS];
-  {
-    const u16* qp = q + ((long)b * S + qrow_ld) * q_ts + (long)hq * D + 8 * lg;
+k_attn_prefill_combine(const Prefill a) {
+  const int R = a.S * a.G, lane = threadIdx.x & 63;
+  const long id = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (id >= (long)a.heads * R) return;
+  const int head = id / R, r = id - (long)head * R;
+  const int b = head / a.Hkv, hkv = head - b * a.Hkv;
+  int u0, u1;
+  split_tiles(keys_of(a, b, min(r / ROWS * ROWS + ROWS, R) - 1), a.splits, 1,
+              u0, u1);
+  if (u0 >= u1) return;
+  const float* ml = a.pml + id * a.splits * 2;
+  float m = M_NONE;
+  for (int i = 0; i < a.splits; ++i) m = fmaxf(m, ml[2 * i]);
+  float l = 0.f, o[D / 64];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-      a_q[ks] = *(const s16x8*)(qp + ks * 32);
+  for (int e = 0; e < D / 64; ++e) o[e] = 0.f;
+  for (int i = 0; i < a.splits; ++i) {
+    if (i && ml[2 * i + 1] == 0.f && ml[2 * i] == M_NONE) continue;
+    const float w = __builtin_amdgcn_exp2f(ml[2 * i] - m);
+    l = fmaf(w, ml[2 * i + 1], l);
+    const float* po = a.po + (id * a.splits + i) * D + lane * (D / 64);
+#pragma unroll
+    for (int e = 0; e < D / 64; ++e) o[e] = fmaf(w, po[e], o[e]);
   }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  const int s = r / a.G, g = r - s * a.G;
+  u16* op = a.out + (((long)b * a.S + s) * a.Hkv * a.G + hkv * a.G + g) * D +
+            lane * (D / 64);
+#pragma unroll
+  for (int e = 0; e < D / 64; ++e) op[e] = El<u16>::st(o[e] * inv);
+}
 
-  // online-softmax state per C row r (replicated across the 16-lane group)
-  float m_row[4], l_row[4];
-  f32x4 o_acc[DC];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) { m_row[r] = -1.0f / 0.0f; l_row[r] = 0.f; }
-#pragma unroll
-  for (int dc = 0; dc < DC; ++dc) o_acc[dc] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const u16* kbase = kc + ((long)b * Hkv + hkv) * max_seq * D;
-  const u16* vbase = vc + ((long)b * Hkv + hkv) * max_seq * D;
-
-  const int ntiles = (kv_end + KV - 1) / KV;
-  for (int t = 0; t < ntiles; ++t) {
-    // ---- stage K/V tile (KV keys x D), zero-padded past kv_end ----------
-    __syncthreads();                                // vt/kt reuse protection
-    {
-      const int nv8 = KV * D / 8;                   // vec8 slots in a tile
-      for (int i = tid; i < nv8; i += 256) {
-        const int key = i / (D / 8);
-        const int col8 = i % (D / 8);
-        const int kk = t * KV + key;
-        const int dst = key * (D / 8) + SWZ16(key, col8);
-        s16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-        s16x8 v8 = z;
-        if (kk < kv_end) {
-          ((s16x8*)kt)[dst] = *(const s16x8*)(kbase + (long)kk * D + col8 * 8);
-          v8 = *(const s16x8*)(vbase + (long)kk * D + col8 * 8);
-        } else {
-          ((s16x8*)kt)[dst] = z;
-        }
-        // V transposed scatter (VT_OFF block swizzle)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          ((u16*)vtT)[VT_OFF(col8 * 8 + j, key)] = (u16)v8[j];
-      }
-    }
-    __syncthreads();
-
-    // ---- QK^T: NC 16-key chunks ---------------------------------------
-    f32x4 sfrag[NC];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int krow = c * 16 + l15;
-        const int kcol8 = SWZ16(krow, ks * 4 + lg);
-        const s16x8 b_k = *(const s16x8*)(&((s16x8*)kt)[krow * (D / 8) + kcol8]);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_q[ks], b_k, acc, 0, 0, 0);
-      }
-      sfrag[c] = acc;
-    }
-
-    // ---- mask + online softmax ----------------------------------------
-    float p_val[NC][4];
-    float alpha[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int qrow_abs = p0 + qt * 64 + w * 16 + 4 * lg + r;
-      float sv[NC];
-      float mx = -1.0f / 0.0f;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        sv[c] = sfrag[c][r] * scale;
-        const int key = t * KV + c * 16 + l15;
-        if (key >= kv_end || (causal && key > qrow_abs)) sv[c] = -1.0f / 0.0f;
-        mx = fmaxf(mx, sv[c]);
-      }
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-      const float m_new = fmaxf(m_row[r], mx);
-      alpha[r] = __expf(m_row[r] - m_new);          // 0 on first tile
-      m_row[r] = m_new;
-      float psum = 0.f;
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        p_val[c][r] = (sv[c] == -1.0f / 0.0f) ? 0.f : __expf(sv[c] - m_new);
-        psum += p_val[c][r];
-      }
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) psum += __shfl_xor(psum, off);
-      l_row[r] = l_row[r] * alpha[r] + psum;
-    }
-
-    // ---- rescale O, stage P (C-layout -> A-layout via LDS) -------------
-#pragma unroll
-    for (int dc = 0; dc < DC; ++dc)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o_acc[dc][r] *= alpha[r];
-#pragma unroll
-    for (int c = 0; c < NC; ++c)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        p_lds[w][4 * lg + r][c * 16 + l15] = f2bf(p_val[c][r]);
-    // same-wave LDS RAW: compiler inserts lgkmcnt waits; no barrier needed
-    // (p_lds[w] is private to wave w).
-
-    // ---- PV: KA P-fragments of K=32 each -------------------------------
-    s16x8 a_p[KA];
-#pragma unroll
-    for (int ka = 0; ka < KA; ++ka)
-      a_p[ka] = *(const s16x8*)(&p_lds[w][l15][ka * 32 + 8 * lg]);
-#pragma unroll
-    for (int dc = 0; dc < DC; ++dc) {
-      const int col = dc * 16 + l15;
-#pragma unroll
-      for (int ka = 0; ka < KA; ++ka) {
-        // 8 consecutive keys of this column = one 16-byte read
-        const s16x8 b_v = *(const s16x8*)(
-            &((u16*)vtT)[VT_OFF(col, ka * 32 + 8 * lg)]);
-        o_acc[dc] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_p[ka], b_v,
-                                                            o_acc[dc], 0, 0, 0);
-      }
-    }
-  }
-
-  // ---- epilogue: O / l, store ------------------------------------------
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int srow = qt * 64 + w * 16 + 4 * lg + r;
-    if (srow >= S) continue;
-    const float inv_l = l_row[r] > 0.f ? 1.f / l_row[r] : 0.f;
-    u16* orow = out + (((long)b * S + srow) * Hq + hq) * D;
-#pragma unroll
-    for (int dc = 0; dc < DC; ++dc)
-      orow[dc * 16 + l15] = f2bf(o_acc[dc][r] * inv_l);
+template <int D>
+void launch_prefill(const Prefill& a, hipStream_t stream) {
+  const dim3 grid((unsigned)a.heads * a.tiles * a.splits);
+  if (a.splits > 1) {
+    hipLaunchKernelGGL((k_attn_prefill<D, true>), grid, dim3(256), 0, stream,
+                       a);
+    const long rows = (long)a.heads * a.S * a.G;
+    hipLaunchKernelGGL(k_attn_prefill_combine<D>, dim3((rows + 3) / 4),
+                       dim3(256), 0, stream, a);
+  } else {
+    hipLaunchKernelGGL((k_attn_prefill<D, false>), grid, dim3(256), 0, stream,
+                       a);
   }
 }
 
@@ -209,22 +335,21 @@ k_attn_prefill(const u16* __restrict__ q, const u16* __restrict__ kc,
 
 extern "C" {
 
+// po [B * Hkv, S * G, splits, D] and pml [.., splits, 2] float32, where
+// splits > 1.
 void fei_attn_prefill(const void* q, const void* k_cache, const void* v_cache,
-                      void* out, const int* pos0, const int* kv_len,
-                      int B, int S, int Hq, int Hkv, int D, int max_seq,
-                      float scale, int causal, long q_ts, hipStream_t stream) {
-  dim3 grid((S + 63) / 64, Hq, B);
-  if (D == 128) {
-    hipLaunchKernelGGL(k_attn_prefill<128>, grid, dim3(256), 0, stream,
-                       (const u16*)q, (const u16*)k_cache, (const u16*)v_cache,
-                       (u16*)out, pos0, kv_len, B, S, Hq, Hkv, max_seq, scale,
-                       causal, q_ts);
-  } else if (D == 64) {
-    hipLaunchKernelGGL(k_attn_prefill<64>, grid, dim3(256), 0, stream,
-                       (const u16*)q, (const u16*)k_cache, (const u16*)v_cache,
-                       (u16*)out, pos0, kv_len, B, S, Hq, Hkv, max_seq, scale,
-                       causal, q_ts);
-  }
+                      void* out, const int* pos0, const int* kv_len, int B,
+                      int S, int Hq, int Hkv, int D, int max_seq, float scale,
+                      int causal, long q_ts, int splits, float* po, float* pml,
+                      hipStream_t stream) {
+  const int G = Hq / Hkv;
+  const Prefill a{(const u16*)q, (const u16*)k_cache, (const u16*)v_cache,
+                  (u16*)out,     po,     pml,  pos0,  kv_len,
+                  S,             G,      Hkv,  B * Hkv,
+                  (S * G + ROWS - 1) / ROWS,   max_seq, causal, splits,
+                  scale,         q_ts};
+  if (D == 128) launch_prefill<128>(a, stream);
+  else if (D == 64) launch_prefill<64>(a, stream);
 }
 
 // ---------------------------------------------------------------------------

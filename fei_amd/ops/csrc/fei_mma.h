@@ -67,6 +67,32 @@ __device__ __forceinline__ void st8(float* p, f32x8 v) {
 __device__ __forceinline__ float get8(s16x8 v, int j) { return bf2f((u16)v[j]); }
 __device__ __forceinline__ float get8(f32x8 v, int j) { return v[j]; }
 
+// 64 lanes x 16 bytes from memory straight into LDS, lane i at lds + 16 i
+// (a byte address, the same in all lanes).
+__device__ __forceinline__ void load_lds(const u16* src, u32 lds) {
+  u32 keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds)
+      : "memory");
+}
+
+// For each group of 16 lanes, lane i of it at the 4 values (i % 4) * 4 of row
+// i / 4 of a 4 x 16 tile in LDS: column i, that is value i of the four rows.
+__device__ __forceinline__ s16x4 turn4(const u16* p) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+}
+__device__ __forceinline__ s16x8 turn8(const u16* p, const u16* q) {
+  const s16x4 a = turn4(p), b = turn4(q);
+  return __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
 // Reductions over the 16 lanes of a DPP row (lanes 16i .. 16i+15), by
 // rotations: every lane gets the result, no LDS traffic.
 template <int N>

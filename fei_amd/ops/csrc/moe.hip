@@ -190,21 +190,6 @@ k_moe_gemm(T* __restrict__ out, const T* __restrict__ x,
   }
 }
 
-// 64 lanes x 16 bytes from memory straight into LDS, lane i at lds + 16 i
-// (a byte address, the same in all lanes).
-__device__ __forceinline__ void load_lds(const u16* src, u32 lds) {
-  u32 keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(src), "s"(lds)
-      : "memory");
-}
-
 // The same for bfloat16 with K % 64 == 0 and N % 4 == 0: tiles of 128 slots x
 // 32 WI columns, 4 waves of 64 slots x 16 WI columns, S LDS buffers of 64
 // steps of K filled by direct loads. The 16-byte places of a row are permuted
