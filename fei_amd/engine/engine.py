@@ -1,13 +1,11 @@
 """LocalEngine: the MI355X inference engine behind the Assistant.
 
 The decode step (the agent-tok/s hot path) is fully device-resident.
-The bf16 default is the PLAIN chain (r02: non-temporal weight loads made
-it +2% over the fused-norm chain, profiles/r02_decode_nt.md):
-  rmsnorm -> QKV GEMV -> split-K decode attention (in-kernel RoPE +
-  KV-append) -> combine -> O GEMV -> fused add+rmsnorm -> gate/up GEMV
-  with fused SwiGLU -> down GEMV -> fused add+rmsnorm
-(9 nt-streaming kernels/layer; FEI_FUSED_NORM=1 restores the 5-kernel
-norm-prologue chain, which remains the fp8 decode path), then the
+Up to three rows (tensor parallel: never) a layer is six launches:
+  QKV GEMV (norm inside) -> split-K decode attention (in-kernel RoPE +
+  KV-append) -> combine -> O GEMV (adds to the residual) -> gate/up GEMV
+  (norm and SwiGLU inside) -> down GEMV (adds to the residual)
+and with more rows rmsnorm, products, fused add+rmsnorm; then the
 lm_head GEMV, the sampling kernel (writes the next input token + the
 out_tokens ring ON DEVICE) and the position advance —
 the whole step is captured once into a hipGraph (torch.cuda.CUDAGraph)
@@ -110,12 +108,8 @@ class LocalEngine:
         env = _os.environ.get("FEI_FUSED_ATTN")
         self.fused_attn = env not in ("0", "false") if env is not None \
             else False
-        # fused-norm chain default flipped in r02: after the non-temporal
-        # weight fix the PLAIN path (separate rmsnorm + nt GEMVs) measured
-        # FASTER (271.8 vs 266.4 tok/s, same-box A/B r2c30) — the norm
-        # prologue's per-element VALU chain throttles the GEMV stream to
-        # ~3-5 TB/s vs 6.6 plain. The fused chain stays for fp8 decode
-        # (its kernels are norm-fused) and via FEI_FUSED_NORM=1.
+        # FEI_FUSED_NORM: whether a batch-1 step reads fp8 weights where
+        # there are some (it does by default)
         self._fused_norm_env = _os.environ.get("FEI_FUSED_NORM")
         self.seed = seed
         self.temperature = 0.0       # graph-captured; set before capture

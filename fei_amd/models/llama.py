@@ -208,23 +208,20 @@ class LlamaModel:
         the TP hot loop samples on shards and gathers 8 bytes/seq instead,
         engine._decode_step_tp).
         ``fused_norm`` (tp=1 only): the residual stream stays inside the
-        GEMV kernels — norm-prologue QKV/gate-up, residual-epilogue O/down;
-        5 kernels per layer instead of 9."""
-        # the fused-norm chain's per-wave norm prologue scales with B
-        # (recomputes all B rows' sumsq per wave): batch 1 only — B=8
-        # measured 572 vs 1130 tok/s on the plain path (docs/BENCHMARKS.md).
-        # The r02 byte-form of that gate (B*C*2 <= 8 KB) also excluded
-        # hidden > 4096 at B=1, silently dropping 70B fp8 decode to the
-        # bf16 plain chain (measured 40.4 == bf16 vs r01's 41.3 with fp8
-        # engaged); the batch gate is B==1 with a separate LDS-budget cap.
-        if fused_norm and self.tp_size == 1 and token.shape[0] == 1 and \
-                self.spec.hidden_size * 2 <= 32 * 1024:
+        GEMV kernels — norm in QKV/gate-up, residual add in O/down; 6 kernels
+        per layer instead of 9. On the GPU always so for few rows."""
+        # Up to three rows the GEMVs hold the norms and the residual
+        # themselves: six launches a layer for nine (8B, batch 1: 3.54 ->
+        # 3.15 ms a step). On the CPU the caller's choice stays.
+        B = token.shape[0]
+        fits = B <= 3 and B * self.spec.hidden_size * 2 <= 64 * 1024
+        if self.tp_size == 1 and fits and (self.emb.is_cuda or
+                                           (fused_norm and B == 1)):
             return self._forward_decode_fused_norm(
                 token, pos, k_caches, v_caches, attn_splits, workspace,
-                fused_attn, attn_out)
+                fused_attn, attn_out, fused_norm)
         s = self.spec
-        B = token.shape[0]
-        h = F.embedding(token.long(), self.emb)          # residual stream
+        h = F.embedding(token, self.emb)                 # residual stream
         scale = 1.0 / math.sqrt(self.D)
         n_layers = len(self.layers)
         x = ops.rmsnorm(h, self.layers[0].norm_attn, s.norm_eps)
@@ -288,19 +285,11 @@ class LlamaModel:
 
     def _forward_decode_fused_norm(self, token, pos, k_caches, v_caches,
                                    attn_splits, workspace, fused_attn,
-                                   attn_out):
+                                   attn_out, use_fp8):
         s = self.spec
         B = token.shape[0]
-        fp8 = getattr(self, "fp8", None)
-        # fp8 norm-GEMVs stage B*C bf16 activations in LDS and recompute
-        # all B norms per wave — measured slower than bf16 already at B=2
-        # (386 vs 410 tok/s) and 3.5x slower at B=8. fp8 pays for B=1
-        # agent decode only (any hidden size whose row fits the 32 KB
-        # dynamic-LDS budget — the old 8 KB byte gate wrongly excluded
-        # 70B's hidden=8192 at B=1).
-        if fp8 is not None and (B != 1 or s.hidden_size * 2 > 32 * 1024):
-            fp8 = None
-        h = F.embedding(token.long(), self.emb).contiguous()
+        fp8 = getattr(self, "fp8", None) if use_fp8 and B == 1 else None
+        h = F.embedding(token, self.emb)
         scale = 1.0 / math.sqrt(self.D)
         # norm-precompute chain (opt-in FEI_NORM_PRECOMP=1; measured loss,
         # see __init__): each residual GEMV's epilogue accumulates the next

@@ -69,7 +69,8 @@ def _try_load() -> None:
                                      _i, _i, _i, _i, _i, _i, _f, _i, _l, _i,
                                      _vp, _vp, _vp]
     lib.fei_mfma_probe.argtypes = [_vp, _vp, _vp, _vp]
-    lib.fei_gemv.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp]
+    lib.fei_gemv.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _i,
+                             _vp, _vp]
     lib.fei_gemm_m8.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp]
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
@@ -89,19 +90,8 @@ def _try_load() -> None:
     lib.fei_add_layernorm.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _f,
                                       _i, _vp]
     lib.fei_gelu.argtypes = [_vp, _vp, _l, _vp]
-    lib.fei_gemv_norm_fp8.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _i,
-                                      _f, _vp]
-    lib.fei_gemv_res_fp8.argtypes = [_vp, _vp, _vp, _vp, _i, _i, _i, _vp]
-    lib.fei_gemv_swiglu_norm_fp8.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i,
-                                             _i, _f, _vp]
     lib.fei_quant_fp8_rows.argtypes = [_vp, _vp, _vp, _i, _i, _vp]
-    lib.fei_gemv_swiglu.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp]
     lib.fei_prefetch.argtypes = [_vp, _l, _vp, _i, _vp]
-    lib.fei_gemv_res.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp]
-    lib.fei_gemv_norm.argtypes = [_vp, _vp, _vp, _vp, _i, _i, _i, _f, _i, _vp,
-                                  _vp]
-    lib.fei_gemv_swiglu_norm.argtypes = [_vp, _vp, _vp, _vp, _i, _i, _i, _f,
-                                         _i, _vp, _vp]
     _mixers.declare(lib)
     _moe.declare(lib)
     _sigmoid_attn.declare(lib)
@@ -537,13 +527,21 @@ def mfma_probe(A: torch.Tensor, B: torch.Tensor) -> torch.Tensor:
 
 # -- decode GEMV dispatch ----------------------------------------------------
 
-# Nontemporal weight loads for ALL decode GEMVs: in the real decode loop
-# every weight byte is cache-cold (the 15 GB per-step cycle flushes the
-# 256 MB L3), so NT never hurts and avoids polluting L2/L3 for the hot
-# activations — measured 257.2 vs 255.6 tok/s on the 8B headline. The
-# microbench that suggested a 512 MB threshold was L3-warm across runs.
-# FEI_GEMV_NT_MIN (bytes) restores a threshold.
-_GEMV_NT_MIN_BYTES = int(os.environ.get("FEI_GEMV_NT_MIN", 0))
+# What becomes of a GEMV's sums (csrc/gemv.hip).
+_BF16, _RES, _SWIGLU = 0, 1, 2
+
+
+def _launch_gemv(out, x2, gain, w, wscale, N: int, eps: float, epi: int,
+                 ssq=None) -> None:
+    M, K = x2.shape
+    if M not in _GEMV_ROWS:
+        raise ValueError(f"the GEMV takes {_GEMV_ROWS} rows, got {M}")
+    opt = lambda t: None if t is None else _ptr(t)
+    require_lib().fei_gemv(_ptr(out), _ptr(x2), opt(gain), _ptr(w),
+                           opt(wscale), M, N, K, eps, epi, opt(ssq),
+                           _stream())
+
+
 # Fused split-K combine in decode attention (per-head reducer splits poll
 # sc1 done-flags and reduce the partials in-kernel; needs the 3-element
 # workspace). Verified token-identical and measured at PARITY with the
@@ -562,15 +560,22 @@ def _gemm_m8_ok(M: int, N: int, K: int) -> bool:
     return 4 <= M <= 8 and K % 1024 == 0 and N % 16 == 0
 
 
+_GEMV_ROWS = (1, 2, 3, 4, 8)
+
+
 def _gemv_ok(M: int, K: int) -> bool:
-    return M in (1, 2, 4, 8) and K % 8 == 0
+    return M in _GEMV_ROWS and K % 8 == 0
+
+
+def _norm_ok(M: int, K: int) -> bool:
+    """Whether the normed rows fit the GEMV's LDS."""
+    return _gemv_ok(M, K) and M * K * 2 <= 128 * 1024
 
 
 def linear_decode(x: torch.Tensor, w: torch.Tensor,
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """F.linear for skinny M: hand-rolled streaming GEMV on GPU
-    (profiles/r01: rocBLAS reaches ~4 TB/s on M=1; streaming reaches the
-    flat-read ceiling). Falls back to torch for unsupported shapes/CPU."""
+    """F.linear for skinny M: streaming GEMV or MFMA tile on GPU. Falls back
+    to torch for unsupported shapes/CPU."""
     M = x.numel() // x.shape[-1]
     K = x.shape[-1]
     N = w.shape[0]
@@ -580,7 +585,6 @@ def linear_decode(x: torch.Tensor, w: torch.Tensor,
     x2 = x.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
-    nt = 1 if (N * K * 2 >= _GEMV_NT_MIN_BYTES) else 0
     if _gemm_m8_ok(M, N, K):
         # MFMA tile: beats the VALU GEMV at every llama batch shape
         # (1.27-1.65x — profiles/r02_batch_attention.md addendum).
@@ -589,7 +593,7 @@ def linear_decode(x: torch.Tensor, w: torch.Tensor,
         lib.fei_gemm_m8(_ptr(out), _ptr(x2), _ptr(w), M, N, K, 0,
                         _stream())
         return out
-    lib.fei_gemv(_ptr(out), _ptr(x2), _ptr(w), M, N, K, nt, _stream())
+    _launch_gemv(out, x2, None, w, None, N, 0.0, _BF16)
     return out
 
 
@@ -605,7 +609,6 @@ def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
     x2 = x.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*x.shape[:-1], I, dtype=x.dtype, device=x.device)
-    nt = 1 if (2 * I * K * 2 >= _GEMV_NT_MIN_BYTES) else 0
     if _gemm_m8_ok(M, 2 * I, K):
         # MFMA over the stacked [2I, K] weight (its [M, 2I] output is
         # k_swiglu's packed input): 68.3 -> ~47 us on the 8B gate/up at
@@ -615,8 +618,7 @@ def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
                         _stream())
         lib.fei_swiglu(_ptr(out), _ptr(gu), M, I, _stream())
         return out
-    lib.fei_gemv_swiglu(_ptr(out), _ptr(x2), _ptr(wgu), M, I, K, nt,
-                        _stream())
+    _launch_gemv(out, x2, None, wgu, None, I, 0.0, _SWIGLU)
     return out
 
 
@@ -625,23 +627,17 @@ def gemv_res(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
     """res += x @ w^T (epilogue residual add; in place on res [M,N]).
 
     ``ssq_out`` [M] f32, pre-zeroed: the kernel also accumulates the
-    sum-of-squares of the updated residual rows so a following
-    gemv_norm/gemv_swiglu_norm can skip its sumsq prologue pass (pass the
-    same tensor as their ``ssq``). Ignored on the CPU fallback — consumers
-    recompute exactly there."""
+    sum-of-squares of the updated residual rows, which a following
+    gemv_norm/gemv_swiglu_norm takes as ``ssq``. Ignored on the CPU fallback —
+    consumers recompute exactly there."""
     M = x.numel() // x.shape[-1]
     K = x.shape[-1]
-    N = w.shape[0]
     if not x.is_cuda or not _gemv_ok(M, K):
         lin = torch.nn.functional.linear(x, w)
         res.copy_((res.float() + lin.float().view_as(res)).to(res.dtype))
         return res
-    lib = require_lib()
-    x2 = x.contiguous().view(M, K)
-    nt = 1 if (N * K * 2 >= _GEMV_NT_MIN_BYTES) else 0
-    lib.fei_gemv_res(_ptr(res), _ptr(x2), _ptr(w), M, N, K, nt,
-                     _ptr(ssq_out) if ssq_out is not None else None,
-                     _stream())
+    _launch_gemv(res, x.contiguous().view(M, K), None, w, None, w.shape[0],
+                 0.0, _RES, ssq_out)
     return res
 
 
@@ -649,23 +645,23 @@ def gemv_norm(res: torch.Tensor, wnorm: torch.Tensor, w: torch.Tensor,
               eps: float = 1e-5,
               out: Optional[torch.Tensor] = None,
               ssq: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """out = rmsnorm(res)*wnorm @ w^T (norm-prologue GEMV).
+    """out = rmsnorm(res)*wnorm @ w^T, the norm inside the product.
 
-    ``ssq`` [M] f32: precomputed sum-of-squares of res rows (from a prior
-    gemv_res ``ssq_out``); skips the prologue pass over res."""
+    ``ssq`` [M] f32: the sums of squares of res rows, if the caller has them
+    (from a prior gemv_res ``ssq_out``)."""
     M = res.numel() // res.shape[-1]
     K = res.shape[-1]
     N = w.shape[0]
     if not res.is_cuda or not _gemv_ok(M, K):
         return torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w)
-    lib = require_lib()
-    r2 = res.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*res.shape[:-1], N, dtype=res.dtype, device=res.device)
-    nt = 1 if (N * K * 2 >= _GEMV_NT_MIN_BYTES) else 0
-    lib.fei_gemv_norm(_ptr(out), _ptr(r2), _ptr(wnorm), _ptr(w), M, N, K,
-                      eps, nt, _ptr(ssq) if ssq is not None else None,
-                      _stream())
+    if not _norm_ok(M, K):
+        _launch_gemv(out, rmsnorm(res, wnorm, eps).view(M, K), None, w, None,
+                     N, 0.0, _BF16)
+        return out
+    _launch_gemv(out, res.contiguous().view(M, K), wnorm, w, None, N, eps,
+                 _BF16, ssq)
     return out
 
 
@@ -680,15 +676,14 @@ def gemv_swiglu_norm(res: torch.Tensor, wnorm: torch.Tensor,
     I = wgu.shape[0] // 2
     if not res.is_cuda or not _gemv_ok(M, K):
         return swiglu(torch.nn.functional.linear(rmsnorm(res, wnorm, eps), wgu))
-    lib = require_lib()
-    r2 = res.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*res.shape[:-1], I, dtype=res.dtype, device=res.device)
-    nt = 1 if (wgu.shape[0] * K * 2 >= _GEMV_NT_MIN_BYTES) else 0
-    lib.fei_gemv_swiglu_norm(_ptr(out), _ptr(r2), _ptr(wnorm), _ptr(wgu),
-                             M, I, K, eps, nt,
-                             _ptr(ssq) if ssq is not None else None,
-                             _stream())
+    if not _norm_ok(M, K):
+        _launch_gemv(out, rmsnorm(res, wnorm, eps).view(M, K), None, wgu,
+                     None, I, 0.0, _SWIGLU)
+        return out
+    _launch_gemv(out, res.contiguous().view(M, K), wnorm, wgu, None, I, eps,
+                 _SWIGLU, ssq)
     return out
 
 
@@ -827,12 +822,10 @@ def gemv_norm_fp8(res, wnorm, w8, wscale, eps: float = 1e-5,
         return torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w)
     assert M * K * 2 <= 64 * 1024, \
         "fp8 norm-GEMV stages M*K bf16 activations in LDS (<=64 KB)"
-    lib = require_lib()
-    r2 = res.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*res.shape[:-1], N, dtype=res.dtype, device=res.device)
-    lib.fei_gemv_norm_fp8(_ptr(out), _ptr(r2), _ptr(wnorm), _ptr(w8),
-                          _ptr(wscale), M, N, K, eps, _stream())
+    _launch_gemv(out, res.contiguous().view(M, K), wnorm, w8, wscale, N, eps,
+                 _BF16)
     return out
 
 
@@ -845,10 +838,8 @@ def gemv_res_fp8(x, w8, wscale, res) -> torch.Tensor:
         lin = torch.nn.functional.linear(x, w)
         res.copy_((res.float() + lin.float().view_as(res)).to(res.dtype))
         return res
-    lib = require_lib()
-    x2 = x.contiguous().view(M, K)
-    lib.fei_gemv_res_fp8(_ptr(res), _ptr(x2), _ptr(w8), _ptr(wscale),
-                         M, N, K, _stream())
+    _launch_gemv(res, x.contiguous().view(M, K), None, w8, wscale, N, 0.0,
+                 _RES)
     return res
 
 
@@ -861,10 +852,8 @@ def gemv_swiglu_norm_fp8(res, wnorm, w8, wscale, eps: float = 1e-5,
         w = ref.dequant_fp8(w8, wscale).to(res.dtype)
         return swiglu(torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w))
     assert M * K * 2 <= 64 * 1024
-    lib = require_lib()
-    r2 = res.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*res.shape[:-1], I, dtype=res.dtype, device=res.device)
-    lib.fei_gemv_swiglu_norm_fp8(_ptr(out), _ptr(r2), _ptr(wnorm), _ptr(w8),
-                                 _ptr(wscale), M, I, K, eps, _stream())
+    _launch_gemv(out, res.contiguous().view(M, K), wnorm, w8, wscale, I, eps,
+                 _SWIGLU)
     return out

@@ -1,356 +1,292 @@
-// Skinny-M GEMV kernels for the decode hot path (gfx950).
-// out[M, N] = x[M, K] @ W[N, K]^T  — torch F.linear weight layout (W row-
-// major over K). M <= 8 (decode batch), K % 512 == 0.
+// Products of few rows with a weight matrix, the decode step's (gfx950):
+// out[M, N] = x[M, K] @ W[N, K]^T, F.linear's layout.
 //
-// Design: two W rows per wave, streamed with 16 B/lane coalesced loads
-// (64 lanes x 16 B = 2 cachelines per instruction; 2 rows = 2 independent
-// load streams for memory-level parallelism); x read straight through
-// L1/L2 (8-28 KB, cache-hot — LDS staging only added startup latency);
-// per-lane f32 dot then wave shfl reduce. This is pure HBM streaming —
-// rocBLAS's tiled GEMM kernels reach only ~4 TB/s on M=1 shapes
-// (profiles/r01), streaming reaches the flat-read ceiling.
-//
-// fei_gemv_swiglu fuses the MLP gate/up pair: wave computes both dots
-// (rows n and n+N) and writes silu(g)*u — kills the separate swiglu
-// kernel and the 2*I-wide intermediate.
-#include "fei_common.h"
+// k_gemv streams the weights, bfloat16 or fp8 (e4m3fn, a scale per row), through
+// the vector units; from M = 4 on k_gemm_m8 (below) uses the matrix units.
+#include <type_traits>
+
 #include "fei_epilogue.h"
+#include "fei_mma.h"
 
 namespace {
 
-template <int M, bool NT>
+typedef __attribute__((ext_vector_type(4))) u32 u32x4;
+
+enum { GEMV_BF16 = 0, GEMV_RES = 1, GEMV_SWIGLU = 2 };
+
+// Sum over a wave, added in the order of a butterfly from lane ^ 32 down to
+// lane ^ 1, without LDS.
+__device__ __forceinline__ float wave_sum(float v) {
+  const u32 a = __builtin_bit_cast(u32, v);
+  const auto p = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  v = __builtin_bit_cast(float, p0) + __builtin_bit_cast(float, p1);
+  const u32 b = __builtin_bit_cast(u32, v);
+  const auto q = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const u32 q0 = q[0], q1 = q[1];
+  return row16_sum(__builtin_bit_cast(float, q0) +
+                   __builtin_bit_cast(float, q1));
+}
+
+// A wave streams two rows of w, 4 loads of 16 bytes a lane from each at a time
+// and the next 4 before it uses them; all waves of a product are on the chip at
+// once, so what counts is how soon their loads are out and how many. x goes to
+// LDS meanwhile: its loads are issued first (loads come back in order), and the
+// barriers leave the weights in flight. NORM: x is a residual under an RMS norm
+// with gains, which the block takes on the way to LDS (rounded to bfloat16 there,
+// as a norm kernel's result is). KS = 4: the block's waves share two rows. LDS = false:
+// x from L1/L2, for rows that LDS has no room for. GEMV_RES adds to out in
+// place; GEMV_SWIGLU: w has N rows of gates, then N of up, a wave takes a pair.
+// ssq (may be null): with GEMV_RES gets the sums of squares of the new rows
+// added, with NORM has those of x.
+//
+// Bound by HBM and, at decode sizes, by the 3 us that a launch and the first
+// loads take. In a graph of launches over cold weights, M = 1, against two rows
+// a wave in plain loops (and for NORM a norm's launch of 4.6 us in front):
+// 6144 x 4096 with norm 10.8 us (9.7 + 4.6), 4096 x 4096 7.8 (7.9),
+// 2 x 14336 x 4096 SwiGLU with norm 36.8 (36.3 + 4.6), 4096 x 14336 20.8
+// (24.9), 128256 x 4096 151 (165). fp8: 7.1 (10), 5.7 (6.5), 20.4 (44.5),
+// 13.7 (13). Two or eight loads a row in flight, four rows a wave, or rows
+// shared by 2 waves are slower at nearly every size.
+template <int M, int KS, bool NORM, int EPI, bool FP8, bool LDS>
 __global__ void __launch_bounds__(256)
 k_gemv(u16* __restrict__ out, const u16* __restrict__ x,
-       const u16* __restrict__ w, int N, int K) {
-  // 4 waves per block, TWO W rows per wave: two independent load streams
-  // per wave double the in-flight memory requests (the fused swiglu kernel
-  // streams 2 rows/wave and measures ~25 % more bandwidth than 1 row/wave).
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int n0 = blockIdx.x * 8 + wid * 2;
-  if (n0 >= N) return;
-  const u16* xs = x;                          // L1/L2-hot, no staging
-  const bool two = (n0 + 1) < N;
-
-  const s16x8* wrow0 = (const s16x8*)(w + (long)n0 * K);
-  const s16x8* wrow1 = (const s16x8*)(w + (long)(n0 + (two ? 1 : 0)) * K);
-  float acc0[M], acc1[M];
+       const u16* __restrict__ gain, const void* __restrict__ wp,
+       const float* __restrict__ wscale, int N, int K, float eps,
+       float* __restrict__ ssq) {
+  constexpr int E = FP8 ? 16 : 8;          // weights of a 16-byte load
+  constexpr int U = KS > 1 ? 2 : 4;        // loads of a row in flight
+  constexpr int R = 2;                     // rows of w
+  constexpr int WV = 4 / KS;               // waves side by side
+  extern __shared__ __align__(16) u16 xs[];   // the rows, normed
+  __shared__ float red[4][M];
+  __shared__ float part[KS > 1 ? 4 : 1][R][M];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ks = KS > 1 ? wid % KS : 0;
+  // SWIGLU: half of a wave's rows are gates, the others the same of up
+  constexpr int RO = EPI == GEMV_SWIGLU ? R / 2 : R;     // results per wave
+  const int n0 = (blockIdx.x * WV + wid / KS) * RO;
+  const u32x4* w[R];
 #pragma unroll
-  for (int m = 0; m < M; ++m) { acc0[m] = 0.f; acc1[m] = 0.f; }
-  const int nv = K >> 3;                      // vec8 per row
-  for (int i = lane; i < nv; i += 64) {
-    s16x8 wv0, wv1;
-    if (NT) {
-      wv0 = __builtin_nontemporal_load(&wrow0[i]);
-      wv1 = __builtin_nontemporal_load(&wrow1[i]);
-    } else {
-      wv0 = wrow0[i];
-      wv1 = wrow1[i];
-    }
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      s16x8 xv = ((const s16x8*)(xs + m * K))[i];
-      acc0[m] += dot8_bf16(xv, wv0);
-      acc1[m] += dot8_bf16(xv, wv1);
-    }
+  for (int r = 0; r < R; ++r) {
+    long n = min(n0 + r % RO, N - 1);
+    if (EPI == GEMV_SWIGLU && r >= RO) n += N;
+    w[r] = (const u32x4*)((const char*)wp + n * K * (FP8 ? 1 : 2));
   }
+  const int nv = K / E;                    // loads of a row
+  const int per = KS > 1 ? ((nv + 63) / 64 + KS - 1) / KS * 64 : nv;
+  const int lo = ks * per, hi = KS > 1 ? min(nv, lo + per) : nv;
+  // x first: loads come back in order
+  constexpr int XV = NORM && M == 1 ? 4 : 8;
+  const int nx = M * (K / 8);
+  s16x8 x0[XV], g0[NORM ? XV : 1];
+  auto gain_at = [&](int c) {
+    return ((const s16x8*)gain)[M == 1 ? c : c % (K / 8)];
+  };
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    float v0 = wave_reduce_sum(acc0[m]);
-    float v1 = wave_reduce_sum(acc1[m]);
-    if (lane == 0) {
-      out[(long)m * N + n0] = f2bf(v0);
-      if (two) out[(long)m * N + n0 + 1] = f2bf(v1);
-    }
+  for (int i = 0; LDS && i < XV; ++i) {
+    const int c = min(tid + i * 256, nx - 1);
+    x0[i] = ((const s16x8*)x)[c];
+    if (NORM) g0[i] = gain_at(c);
   }
-}
-
-// gate/up + SwiGLU fused: W = [gate rows (N) ; up rows (N)] stacked, out[M,N]
-template <int M, bool NT>
-__global__ void __launch_bounds__(256)
-k_gemv_swiglu(u16* __restrict__ out, const u16* __restrict__ x,
-              const u16* __restrict__ w, int N, int K) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int n = blockIdx.x * 4 + wid;
-  if (n >= N) return;
-  const u16* xs = x;                          // L1/L2-hot, no staging
-
-  const s16x8* grow = (const s16x8*)(w + (long)n * K);
-  const s16x8* urow = (const s16x8*)(w + (long)(n + N) * K);
-  float accg[M], accu[M];
+  u32x4 v[U][R], nxt[U][R];
+  auto fetch = [&](u32x4 (&d)[U][R], int i0) {
 #pragma unroll
-  for (int m = 0; m < M; ++m) { accg[m] = 0.f; accu[m] = 0.f; }
-  const int nv = K >> 3;
-  for (int i = lane; i < nv; i += 64) {
-    s16x8 gv = NT ? __builtin_nontemporal_load(&grow[i]) : grow[i];
-    s16x8 uv = NT ? __builtin_nontemporal_load(&urow[i]) : urow[i];
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int m = 0; m < M; ++m) {
-      s16x8 xv = ((const s16x8*)(xs + m * K))[i];
-      accg[m] += dot8_bf16(xv, gv);
-      accu[m] += dot8_bf16(xv, uv);
-    }
-  }
+      for (int r = 0; r < R; ++r)
+        d[u][r] = __builtin_nontemporal_load(w[r] + i0 + u * 64 + lane);
+  };
+  auto fetch_tail = [&](u32x4 (&d)[U][R], int i0) {
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    float g = wave_reduce_sum(accg[m]);
-    float u = wave_reduce_sum(accu[m]);
-    if (lane == 0) {
-      const float silu = g / (1.f + __expf(-g));
-      out[(long)m * N + n] = f2bf(silu * u);
-    }
-  }
-}
-
-}  // namespace
-
-extern "C" {
-
-void fei_gemv(void* out, const void* x, const void* w, int M, int N, int K,
-              int nontemporal, hipStream_t stream) {
-  dim3 grid((N + 7) / 8);
-  const size_t lds = 0;
-#define LG(MV, NTV) hipLaunchKernelGGL((k_gemv<MV, NTV>), grid, dim3(256), \
-                                       lds, stream, (u16*)out, \
-                                       (const u16*)x, (const u16*)w, N, K)
-#define LGD(MV) do { if (nontemporal) LG(MV, true); else LG(MV, false); } while (0)
-  switch (M) {
-    case 1: LGD(1); break;
-    case 2: LGD(2); break;
-    case 4: LGD(4); break;
-    case 8: LGD(8); break;
-    default: break;   // wrapper validates
-  }
-#undef LGD
-#undef LG
-}
-
-void fei_gemv_swiglu(void* out, const void* x, const void* w, int M, int N,
-                     int K, int nontemporal, hipStream_t stream) {
-  dim3 grid((N + 3) / 4);
-  const size_t lds = 0;
-#define LG(MV, NTV) hipLaunchKernelGGL((k_gemv_swiglu<MV, NTV>), grid, \
-                                  dim3(256), lds, stream, (u16*)out, \
-                                  (const u16*)x, (const u16*)w, N, K)
-#define LGD(MV) do { if (nontemporal) LG(MV, true); else LG(MV, false); } while (0)
-  switch (M) {
-    case 1: LGD(1); break;
-    case 2: LGD(2); break;
-    case 4: LGD(4); break;
-    case 8: LGD(8); break;
-    default: break;
-  }
-#undef LGD
-#undef LG
-}
-
-}  // extern "C"
-
-// ---------------------------------------------------------------------------
-// Fused-chain GEMV variants (tp=1 decode): the residual stream never leaves
-// the GEMV kernels —
-//   k_gemv_res:  res[m,n] += x[m,:] @ W[n,:]      (epilogue residual add)
-//   k_gemv_norm: out = rmsnorm(res)*wn @ W^T      (norm prologue; every wave
-//                recomputes the row's sumsq from L1/L2-hot res — cheaper
-//                than a separate kernel + intermediate round trip)
-//   k_gemv_swiglu_norm: norm prologue + fused gate/up + SwiGLU
-// ---------------------------------------------------------------------------
-
-namespace {
-
-template <int M>
-__device__ __forceinline__ void norm_factors(const u16* __restrict__ res,
-                                             int K, float eps, int lane,
-                                             float inv[M]) {
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const s16x8* row = (const s16x8*)(res + (long)m * K);
-    float ss = 0.f;
-    const int nv = K >> 3;
-    for (int i = lane; i < nv; i += 64) {
-      s16x8 v = row[i];
+      for (int r = 0; r < R; ++r)
+        if (i0 + u * 64 + lane < hi)
+          d[u][r] = __builtin_nontemporal_load(w[r] + i0 + u * 64 + lane);
+  };
+  auto get = [&](u32x4 (&d)[U][R], int i0) {
+    if (i0 + U * 64 <= hi) fetch(d, i0);
+    else if (i0 < hi) fetch_tail(d, i0);
+  };
+  get(v, lo);
+  float inv[M];
+  if (NORM) {
+    float ss[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) ss[m] = 0.f;
+    auto square = [&](int c, s16x8 xv) {
+      float s = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float f = bf2f((u16)v[j]);
-        ss = fmaf(f, f, ss);
+        const float f = bf2f((u16)xv[j]);
+        s = fmaf(f, f, s);
       }
-    }
-    ss = wave_reduce_sum(ss);
-    inv[m] = rsqrtf(ss / (float)K + eps);
-  }
-}
-
-// ssq (nullable): per-row sum-of-squares of the UPDATED residual,
-// accumulated across workgroups (LDS reduce + one atomicAdd per WG) so the
-// NEXT norm-prologue GEMV can skip its sumsq pass over res (the prologue
-// stalls every wave on an L2-latency-bound read of the whole row before any
-// W bytes stream — measured ~7-13 us per fused GEMV, profiles/r01).
-// Caller zeroes ssq before the step; kernels on one stream order the
-// producer before the consumer. Squares are taken of the bf16-ROUNDED
-// stored value so the result matches what a separate k_rmsnorm would see.
-template <int M, bool NT>
-__global__ void __launch_bounds__(256)
-k_gemv_res(u16* __restrict__ res, const u16* __restrict__ x,
-           const u16* __restrict__ w, int N, int K, float* __restrict__ ssq) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int n0 = blockIdx.x * 8 + wid * 2;
-  const bool active = n0 < N;   // inactive waves still reach the barrier
-  const bool two = (n0 + 1) < N;
-  const s16x8* wrow0 = (const s16x8*)(w + (long)(active ? n0 : 0) * K);
-  const s16x8* wrow1 = (const s16x8*)(w + (long)(active ? n0 + (two ? 1 : 0) : 0) * K);
-  float acc0[M], acc1[M], mysq[M];
-#pragma unroll
-  for (int m = 0; m < M; ++m) { acc0[m] = 0.f; acc1[m] = 0.f; mysq[m] = 0.f; }
-  const int nv = K >> 3;
-  if (active) {
-    for (int i = lane; i < nv; i += 64) {
-      s16x8 wv0 = NT ? __builtin_nontemporal_load(&wrow0[i]) : wrow0[i];
-      s16x8 wv1 = NT ? __builtin_nontemporal_load(&wrow1[i]) : wrow1[i];
-#pragma unroll
-      for (int m = 0; m < M; ++m) {
-        s16x8 xv = ((const s16x8*)(x + (long)m * K))[i];
-        acc0[m] += dot8_bf16(xv, wv0);
-        acc1[m] += dot8_bf16(xv, wv1);
-      }
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const float v0 = wave_reduce_sum(acc0[m]);
-    const float v1 = wave_reduce_sum(acc1[m]);
-    if (lane == 0 && active) {
-      u16* r = res + (long)m * N + n0;
-      const u16 b0 = f2bf(bf2f(r[0]) + v0);
-      r[0] = b0;
-      const float f0 = bf2f(b0);
-      mysq[m] = f0 * f0;
-      if (two) {
-        const u16 b1 = f2bf(bf2f(r[1]) + v1);
-        r[1] = b1;
-        const float f1 = bf2f(b1);
-        mysq[m] += f1 * f1;
-      }
-    }
-  }
-  if (ssq) {                         // uniform across the block
-    __shared__ float sred[4][M];
-    if (lane == 0) {
-#pragma unroll
-      for (int m = 0; m < M; ++m) sred[wid][m] = mysq[m];
-    }
-    __syncthreads();
-    if (tid == 0) {
 #pragma unroll
       for (int m = 0; m < M; ++m)
-        atomicAdd(&ssq[m], sred[0][m] + sred[1][m] + sred[2][m] + sred[3][m]);
-    }
-  }
-}
-
-template <int M, bool NT>
-__global__ void __launch_bounds__(256)
-k_gemv_norm(u16* __restrict__ out, const u16* __restrict__ res,
-            const u16* __restrict__ wn, const u16* __restrict__ w,
-            int N, int K, float eps, const float* __restrict__ ssq) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int n0 = blockIdx.x * 8 + wid * 2;
-  if (n0 >= N) return;
-  float inv[M];
-  if (ssq) {     // sumsq precomputed by the producing k_gemv_res epilogue
+        ss[m] += M == 1 || c / (K / 8) == m ? s : 0.f;
+    };
 #pragma unroll
-    for (int m = 0; m < M; ++m)
-      inv[m] = rsqrtf(ssq[m] / (float)K + eps);
-  } else {
-    norm_factors<M>(res, K, eps, lane, inv);
-  }
-  const bool two = (n0 + 1) < N;
-  const s16x8* wrow0 = (const s16x8*)(w + (long)n0 * K);
-  const s16x8* wrow1 = (const s16x8*)(w + (long)(n0 + (two ? 1 : 0)) * K);
-  float acc0[M], acc1[M];
-#pragma unroll
-  for (int m = 0; m < M; ++m) { acc0[m] = 0.f; acc1[m] = 0.f; }
-  const int nv = K >> 3;
-  for (int i = lane; i < nv; i += 64) {
-    s16x8 wv0 = NT ? __builtin_nontemporal_load(&wrow0[i]) : wrow0[i];
-    s16x8 wv1 = NT ? __builtin_nontemporal_load(&wrow1[i]) : wrow1[i];
-    s16x8 wnv = ((const s16x8*)wn)[i];
+    for (int i = 0; i < XV; ++i)
+      if (tid + i * 256 < nx) square(tid + i * 256, x0[i]);
+    for (int c = tid + XV * 256; c < nx; c += 256)
+      square(c, ((const s16x8*)x)[c]);
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-      s16x8 xv = ((const s16x8*)(res + (long)m * K))[i];
+      ss[m] = wave_sum(ss[m]);
+      if (lane == 0) red[wid][m] = ss[m];
+    }
+    // not __syncthreads: the weights stay in flight
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        // match k_rmsnorm's rounding: the normed activation is quantised
-        // to bf16 before the dot (reference semantics)
-        const float xn = bf2f(f2bf(bf2f((u16)xv[j]) * inv[m] * bf2f((u16)wnv[j])));
-        acc0[m] = fmaf(xn, bf2f((u16)wv0[j]), acc0[m]);
-        acc1[m] = fmaf(xn, bf2f((u16)wv1[j]), acc1[m]);
+    for (int m = 0; m < M; ++m)
+      inv[m] = rsqrtf((ssq ? ssq[m] : red[0][m] + red[1][m] + red[2][m] +
+                                          red[3][m]) / (float)K + eps);
+  }
+  auto stage = [&](int c, s16x8 xv, s16x8 gv) {
+    if (NORM) {
+      float f = inv[0];
+#pragma unroll
+      for (int m = 1; m < M; ++m) f = c / (K / 8) == m ? inv[m] : f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        xv[j] = (short)El<u16>::st(bf2f((u16)xv[j]) * f * bf2f((u16)gv[j]));
+    }
+    ((s16x8*)xs)[c] = xv;
+  };
+#pragma unroll
+  for (int i = 0; LDS && i < XV; ++i)
+    if (tid + i * 256 < nx) stage(tid + i * 256, x0[i], g0[NORM ? i : 0]);
+  for (int c = tid + XV * 256; LDS && c < nx; c += 256)
+    stage(c, ((const s16x8*)x)[c], NORM ? gain_at(c) : x0[0]);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+
+  float acc[R][M];
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[r][m] = 0.f;
+  auto dot = [&](const u32x4 (&d)[R], int i) {
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      s16x8 xv[E / 8];
+#pragma unroll
+      for (int q = 0; q < E / 8; ++q)
+        xv[q] = ld8((LDS ? xs : x) + (long)m * K + i * E + q * 8);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (FP8) {
+          float s = 0.f;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const u32 t = d[r][q];
+            const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(t, false);
+            const f32x2 b = __builtin_amdgcn_cvt_pk_f32_fp8(t, true);
+            const s16x8 y = xv[q / 2 * (E / 8 - 1)];
+            s = fmaf(a[0], bf2f((u16)y[q % 2 * 4]), s);
+            s = fmaf(a[1], bf2f((u16)y[q % 2 * 4 + 1]), s);
+            s = fmaf(b[0], bf2f((u16)y[q % 2 * 4 + 2]), s);
+            s = fmaf(b[1], bf2f((u16)y[q % 2 * 4 + 3]), s);
+          }
+          acc[r][m] += s;
+        } else {
+          acc[r][m] += dot8_bf16(xv[0], __builtin_bit_cast(s16x8, d[r]));
+        }
       }
     }
+  };
+  for (int i0 = lo; i0 < hi; i0 += U * 64) {
+    get(nxt, i0 + U * 64);
+    if (i0 + U * 64 <= hi) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) dot(v[u], i0 + u * 64 + lane);
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (i0 + u * 64 + lane < hi) dot(v[u], i0 + u * 64 + lane);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[u][r] = nxt[u][r];
   }
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const float v0 = wave_reduce_sum(acc0[m]);
-    const float v1 = wave_reduce_sum(acc1[m]);
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int m = 0; m < M; ++m) acc[r][m] = wave_sum(acc[r][m]);
+  if (KS > 1) {
     if (lane == 0) {
-      out[(long)m * N + n0] = f2bf(v0);
-      if (two) out[(long)m * N + n0 + 1] = f2bf(v1);
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int m = 0; m < M; ++m) part[wid][r][m] = acc[r][m];
     }
+    __syncthreads();
+    if (ks) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        acc[r][m] = part[wid][r][m];
+#pragma unroll
+        for (int k = 1; k < KS; ++k) acc[r][m] += part[wid + k][r][m];
+      }
+  }
+  if (lane) return;
+  float sq[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    sq[m] = 0.f;
+#pragma unroll
+    for (int r = 0; r < RO; ++r) {
+      const int n = n0 + r;
+      if (n >= N) break;
+      float y = acc[r][m];
+      if (FP8) y *= wscale[n];
+      u16* o = out + (long)m * N + n;
+      if (EPI == GEMV_SWIGLU) {
+        float u = acc[r + R - RO][m];
+        if (FP8) u *= wscale[n + N];
+        *o = f2bf(y / (1.f + __expf(-y)) * u);
+      } else if (EPI == GEMV_RES) {
+        const u16 t = f2bf(bf2f(*o) + y);
+        *o = t;
+        sq[m] = fmaf(bf2f(t), bf2f(t), sq[m]);
+      } else {
+        *o = f2bf(y);
+      }
+    }
+    if (EPI == GEMV_RES && ssq) atomicAdd(&ssq[m], sq[m]);
   }
 }
 
-template <int M, bool NT>
-__global__ void __launch_bounds__(256)
-k_gemv_swiglu_norm(u16* __restrict__ out, const u16* __restrict__ res,
-                   const u16* __restrict__ wn, const u16* __restrict__ w,
-                   int N, int K, float eps, const float* __restrict__ ssq) {
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wid = tid >> 6;
-  const int n = blockIdx.x * 4 + wid;
-  if (n >= N) return;
-  float inv[M];
-  if (ssq) {
-#pragma unroll
-    for (int m = 0; m < M; ++m)
-      inv[m] = rsqrtf(ssq[m] / (float)K + eps);
-  } else {
-    norm_factors<M>(res, K, eps, lane, inv);
+template <int M, bool NORM, int EPI, bool FP8>
+void launch_gemv(void* out, const void* x, const void* gain, const void* w,
+                 const float* wscale, int N, int K, float eps, float* ssq,
+                 hipStream_t stream) {
+  const size_t lds = (size_t)M * K * 2;
+  auto go = [&](auto kernel, int blocks, size_t bytes) {
+    // beyond 64 KB a kernel has to ask
+    if (bytes > 65536)
+      (void)hipFuncSetAttribute((const void*)kernel,
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)bytes);
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), bytes, stream,
+                       (u16*)out, (const u16*)x, (const u16*)gain, w, wscale,
+                       N, K, eps, ssq);
+  };
+  const int per = EPI == GEMV_SWIGLU ? 4 : 8;          // results per block
+  if constexpr (!NORM) {
+    if (lds > 65536)
+      return go(k_gemv<M, 1, false, EPI, FP8, false>, (N + per - 1) / per, 0);
+    // Few long rows: a wave per two rows would be one per SIMD. 2048 x 8192:
+    // 8.4 us against 9.1 (fp8 5.7, 6.8); 2048 x 2048: 4.5 against 4.3.
+    if constexpr (EPI != GEMV_SWIGLU)
+      if (N <= 2048 && K >= 4096)
+        return go(k_gemv<M, 4, false, EPI, FP8, true>, (N + 1) / 2, lds);
   }
-  const s16x8* grow = (const s16x8*)(w + (long)n * K);
-  const s16x8* urow = (const s16x8*)(w + (long)(n + N) * K);
-  float accg[M], accu[M];
-#pragma unroll
-  for (int m = 0; m < M; ++m) { accg[m] = 0.f; accu[m] = 0.f; }
-  const int nv = K >> 3;
-  for (int i = lane; i < nv; i += 64) {
-    s16x8 gv = NT ? __builtin_nontemporal_load(&grow[i]) : grow[i];
-    s16x8 uv = NT ? __builtin_nontemporal_load(&urow[i]) : urow[i];
-    s16x8 wnv = ((const s16x8*)wn)[i];
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      s16x8 xv = ((const s16x8*)(res + (long)m * K))[i];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float xn = bf2f(f2bf(bf2f((u16)xv[j]) * inv[m] * bf2f((u16)wnv[j])));
-        accg[m] = fmaf(xn, bf2f((u16)gv[j]), accg[m]);
-        accu[m] = fmaf(xn, bf2f((u16)uv[j]), accu[m]);
-      }
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const float g = wave_reduce_sum(accg[m]);
-    const float u = wave_reduce_sum(accu[m]);
-    if (lane == 0)
-      out[(long)m * N + n] = f2bf(g / (1.f + __expf(-g)) * u);
-  }
+  go(k_gemv<M, 1, NORM, EPI, FP8, true>, (N + per - 1) / per, lds);
 }
 
 // Cache prefetch: stream a weight region through normal (cache-filling)
@@ -373,6 +309,42 @@ k_prefetch(const u16* __restrict__ w, long n_vec8, float* __restrict__ sink) {
 
 extern "C" {
 
+// epi: what becomes of the sums (see above). gain null: no norm. wscale null:
+// bfloat16 weights. M is 1, 2, 3, 4 or 8; with a norm M * K * 2 is at most
+// 128 KB (the callers see to both).
+void fei_gemv(void* out, const void* x, const void* gain, const void* w,
+              const float* wscale, int M, int N, int K, float eps, int epi,
+              float* ssq, hipStream_t stream) {
+  auto run = [&](auto m, auto norm, auto e, auto fp8) {
+    launch_gemv<m.value, norm.value, e.value, fp8.value>(
+        out, x, gain, w, wscale, N, K, eps, ssq, stream);
+  };
+  auto by_weights = [&](auto m, auto norm, auto e) {
+    if (wscale) run(m, norm, e, std::true_type{});
+    else run(m, norm, e, std::false_type{});
+  };
+  auto by_rows = [&](auto norm, auto e) {
+    switch (M) {
+      case 1: return by_weights(std::integral_constant<int, 1>{}, norm, e);
+      case 2: return by_weights(std::integral_constant<int, 2>{}, norm, e);
+      case 3: return by_weights(std::integral_constant<int, 3>{}, norm, e);
+      case 4: return by_weights(std::integral_constant<int, 4>{}, norm, e);
+      case 8: return by_weights(std::integral_constant<int, 8>{}, norm, e);
+      default: return;
+    }
+  };
+  auto by_epi = [&](auto norm) {
+    if (epi == GEMV_RES)
+      by_rows(norm, std::integral_constant<int, GEMV_RES>{});
+    else if (epi == GEMV_SWIGLU)
+      by_rows(norm, std::integral_constant<int, GEMV_SWIGLU>{});
+    else
+      by_rows(norm, std::integral_constant<int, GEMV_BF16>{});
+  };
+  if (gain) by_epi(std::true_type{});
+  else by_epi(std::false_type{});
+}
+
 void fei_prefetch(const void* w, long bytes, void* sink, int n_blocks,
                   hipStream_t stream) {
   const long n_vec8 = bytes / 16;
@@ -380,56 +352,6 @@ void fei_prefetch(const void* w, long bytes, void* sink, int n_blocks,
   hipLaunchKernelGGL(k_prefetch, dim3(n_blocks), dim3(256), 0, stream,
                      (const u16*)w, n_vec8, (float*)sink);
 }
-
-#define DISPATCH_M(FN, ...) \
-  switch (M) { \
-    case 1: FN(1, __VA_ARGS__); break; \
-    case 2: FN(2, __VA_ARGS__); break; \
-    case 4: FN(4, __VA_ARGS__); break; \
-    case 8: FN(8, __VA_ARGS__); break; \
-    default: break; \
-  }
-
-void fei_gemv_res(void* res, const void* x, const void* w, int M, int N,
-                  int K, int nontemporal, void* ssq, hipStream_t stream) {
-  dim3 grid((N + 7) / 8);
-#define LR(MV, NTV) hipLaunchKernelGGL((k_gemv_res<MV, NTV>), grid, \
-    dim3(256), 0, stream, (u16*)res, (const u16*)x, (const u16*)w, N, K, \
-    (float*)ssq)
-#define LRD(MV, _ignored) do { if (nontemporal) LR(MV, true); else LR(MV, false); } while (0)
-  DISPATCH_M(LRD, 0)
-#undef LRD
-#undef LR
-}
-
-void fei_gemv_norm(void* out, const void* res, const void* wn, const void* w,
-                   int M, int N, int K, float eps, int nontemporal,
-                   const void* ssq, hipStream_t stream) {
-  dim3 grid((N + 7) / 8);
-#define LN(MV, NTV) hipLaunchKernelGGL((k_gemv_norm<MV, NTV>), grid, \
-    dim3(256), 0, stream, (u16*)out, (const u16*)res, (const u16*)wn, \
-    (const u16*)w, N, K, eps, (const float*)ssq)
-#define LND(MV, _ignored) do { if (nontemporal) LN(MV, true); else LN(MV, false); } while (0)
-  DISPATCH_M(LND, 0)
-#undef LND
-#undef LN
-}
-
-void fei_gemv_swiglu_norm(void* out, const void* res, const void* wn,
-                          const void* w, int M, int N, int K, float eps,
-                          int nontemporal, const void* ssq,
-                          hipStream_t stream) {
-  dim3 grid((N + 3) / 4);
-#define LS(MV, NTV) hipLaunchKernelGGL((k_gemv_swiglu_norm<MV, NTV>), grid, \
-    dim3(256), 0, stream, (u16*)out, (const u16*)res, (const u16*)wn, \
-    (const u16*)w, N, K, eps, (const float*)ssq)
-#define LSD(MV, _ignored) do { if (nontemporal) LS(MV, true); else LS(MV, false); } while (0)
-  DISPATCH_M(LSD, 0)
-#undef LSD
-#undef LS
-}
-
-#undef DISPATCH_M
 
 }  // extern "C"
 

@@ -72,3 +72,60 @@ def test_attn_prefill_geometries(lib, D, S, Hq, Hkv, T, pos0, kv_len, scale):
     # weights and results are each rounded to bfloat16 once: 2^-9 of each
     # weight times its value, and 2^-9 of the result
     assert row_err(got, want) < 2 ** -7
+
+
+# -- decode GEMVs ----------------------------------------------------------------
+
+def rms64(x, g, eps):
+    x = x.double()
+    return x * torch.rsqrt((x * x).mean(-1, keepdim=True) + eps) * g.double()
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 8, 16),            # less than one load a lane
+    (1, 9, 2064),          # odd rows, a few loads past the full ones
+    (2, 2048, 4096),       # rows shared by four waves
+    (2, 33, 8208),         # the same with a remainder
+    (3, 2050, 4112),
+    (1, 130, 14336),
+    (3, 17, 14336),        # more activations than 64 KB
+    (4, 24, 4096),
+    (8, 11, 2048),
+    (8, 10, 4096),
+    (8, 6, 8192),          # 128 KB of LDS
+])
+def test_gemv_geometries(lib, M, N, K, fp8):
+    """Norm inside or not, plain, residual and SwiGLU sums, both kinds of
+    weights. Sums are float32 and rounded to bfloat16 once: 2^-9 of a value,
+    2^-8 allowed. Normed rows are rounded once more, for a SwiGLU before both
+    products: 3 * 2^-9 in all, 2^-7 allowed."""
+    if fp8 and M * K * 2 > 65536:
+        pytest.skip("the fp8 products refuse rows of this size")
+    x, g = randbf(M, K, seed=M), randbf(K, seed=3) * 0.2 + 1
+    w = randbf(2 * N, K, seed=N, scale=K ** -0.5)
+    res = randbf(M, N, seed=5)
+    w64, w1 = w.double(), w
+    if fp8:
+        w1, sc = lib.quant_fp8(w)
+        w64 = w1.view(torch.float8_e4m3fn).double() * sc.double()[:, None]
+    half = (lambda t: t[:N].contiguous())
+    xn = rms64(x, g, 1e-5)
+    x64 = x.double()
+    r = res.clone()
+    if fp8:
+        got = lib.gemv_norm_fp8(x, g, half(w1), half(sc))
+        sw = lib.gemv_swiglu_norm_fp8(x, g, w1, sc)
+        lib.gemv_res_fp8(x, half(w1), half(sc), r)
+    else:
+        got = lib.gemv_norm(x, g, half(w))
+        sw = lib.gemv_swiglu_norm(x, g, w)
+        lib.gemv_res(x, half(w), r)
+        plain = torch.empty_like(r)
+        lib._launch_gemv(plain, x, None, half(w), None, N, 0.0, lib._BF16)
+        assert row_err(plain, x64 @ w64[:N].T) < 2 ** -8
+    tol = 2 ** -7
+    assert row_err(got, xn @ w64[:N].T) < tol
+    assert row_err(r, res.double() + x64 @ w64[:N].T) < 2 ** -8
+    y = xn @ w64.T
+    assert row_err(sw, torch.nn.functional.silu(y[:, :N]) * y[:, N:]) < tol
