@@ -80,16 +80,9 @@ class LocalEngine:
             use_hip_graph = self.is_gpu
         self.use_graph = use_hip_graph and self.is_gpu
         import os as _os
-        # split-K decode attention: splits x Hkv x B workgroups. 4 splits
-        # (32 WGs on a 256-CU chip) starved KV bandwidth at agent context
-        # lengths (r01: 4 -> 32 measured +41% at seq 3400). Two r02
-        # post-nt sweeps (r2c27, r2c32): 16 vs 32 differ only within
-        # run-to-run noise (±2%) below ~4k context, while 32 is robustly
-        # ahead at 8k (249 vs 217 tok/s) — 32 stays the B<=2 default.
-        # Batches multiply the grid by B, so B>=4 halves the split count
-        # (batch-8: splits 32 -> 16 measured 6.34 -> 5.85 ms/step; 4/8/16
-        # within noise — the grid already fills the chip at 16).
-        # The combine kernel now stages up to 64 splits for experiments.
+        # Blocks of 128 keys per kv head and sequence; those past the context
+        # leave at once, so more cost little. 32 hold 4096 keys in one round;
+        # with four sequences and more, 16 fill the chip.
         env_splits = _os.environ.get("FEI_ATTN_SPLITS")
         if env_splits:
             self.attn_splits = int(env_splits)
@@ -268,15 +261,9 @@ class LocalEngine:
         # sized from self.attn_splits (NOT the ctor arg: FEI_ATTN_SPLITS
         # overrides it, and an undersized workspace is an out-of-bounds
         # write in the split kernel)
-        # 3rd element: zeroed per-split done-flag buffer [B*Hkv_l*splits]
-        # selecting the FUSED split-K combine (split 0 of each (b, hkv)
-        # pair polls the flags and reduces the partials in-kernel — no
-        # separate combine launch per layer).
         self.attn_ws = (
             torch.zeros(self.B, Hq_l, self.attn_splits, D, dtype=torch.float32, device=device),
             torch.zeros(self.B, Hq_l, self.attn_splits, 2, dtype=torch.float32, device=device),
-            torch.zeros(self.B * self.model.hkv_l * self.attn_splits,
-                        dtype=torch.int32, device=device),
         )
         self.attn_out = torch.zeros(self.B, Hq_l, D, dtype=self.dtype,
                                     device=device)
@@ -431,12 +418,6 @@ class LocalEngine:
             k[:, :, kv_rows].copy_(sk)
         for v, sv in zip(self.v_caches, saved_v):
             v[:, :, kv_rows].copy_(sv)
-        # fused-combine done-flags are (pos, layer)-tagged: the warmup ran
-        # at pos 1..2, and the first real replay may run at those same
-        # positions — stale matching tags would let the in-kernel reducer
-        # read partials before the current step's splits wrote them.
-        if len(self.attn_ws) >= 3:
-            self.attn_ws[2].zero_()
         torch.cuda.synchronize()
         self._graph = g
         self._graph_params = (self.temperature, self.seed)
@@ -519,11 +500,6 @@ class LocalEngine:
             # granule tags are pos-keyed, so stale tags must be cleared
             for t in self._stream_ws.values():
                 t.zero_()
-        # same pos-keyed-tag rule for the fused-combine done flags: a new
-        # request replays earlier positions, and a stale matching tag would
-        # release the in-kernel reducer before this step's splits published
-        if self.is_gpu and len(self.attn_ws) >= 3:
-            self.attn_ws[2].zero_()
         # Cap to the context budget BEFORE chunking (mirrors _prep_prompt's
         # cap for the from_pos>0 prefix-cached path, which bypasses it):
         # keep the TAIL of the new tokens — a mid-loop break would silently

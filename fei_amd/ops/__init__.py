@@ -57,10 +57,8 @@ def _try_load() -> None:
                                        _i, _i, _i, _i, _i, _l, _l, _vp]
     lib.fei_rope_kv_prefill.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                         _i, _i, _i, _i, _i, _i, _l, _l, _vp]
-    lib.fei_attn_decode.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp,
-                                    _i, _i, _i, _i, _i, _i, _f, _l,
-                                    _vp, _vp, _vp, _l, _vp, _vp, _i, _vp]
-    lib.fei_attn_decode_combine.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp]
+    lib.fei_attn_decode.argtypes = ([_vp] * 8 + [_i] * 8 + [_f, _l] +
+                                    [_vp] * 3 + [_l, _vp])
     lib.fei_swiglu.argtypes = [_vp, _vp, _l, _i, _vp]
     lib.fei_sample.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _u64,
                                _i, _i, _vp]
@@ -84,9 +82,6 @@ def _try_load() -> None:
                                      _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                      _vp, _vp, _vp, _i, _i, _i, _i, _i,
                                      _i, _i, _f, _f, _vp]
-    lib.fei_attn_decode_paged.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
-                                          _i, _i, _i, _i, _i, _i, _i, _f,
-                                          _l, _vp, _vp, _vp, _l, _vp]
     lib.fei_add_layernorm.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _f,
                                       _i, _vp]
     lib.fei_gelu.argtypes = [_vp, _vp, _l, _vp]
@@ -221,7 +216,9 @@ def attn_decode(q, k_cache, v_cache, pos, splits: int = 32,
     """Single-token GQA attention over n = pos[b]+1 cache entries.
     q [B,Hq,D] -> out [B,Hq,D]. The length is read on DEVICE (hipGraph).
     When (k, v, table) are given, the kernel also fuses the step's RoPE +
-    KV-append: q is the RAW qkv view and cache[pos] is written in-kernel."""
+    KV-append: q is the RAW qkv view and cache[pos] is written in-kernel.
+    ``workspace``: float32 [B,Hq,splits,D] and [B,Hq,splits,2]; more entries,
+    and ``layer``, are taken and not used."""
     B, Hq, D = q.shape
     scale = scale if scale is not None else 1.0 / math.sqrt(D)
     if not q.is_cuda:
@@ -229,52 +226,42 @@ def attn_decode(q, k_cache, v_cache, pos, splits: int = 32,
             rope_kv_decode(q, k, v, k_cache, v_cache, pos, table)
         seqlen = pos + 1
         return ref.attn_decode(q, k_cache, v_cache, seqlen, scale)
-    lib = require_lib()
-    arrive = None
+    return _launch_attn_decode(q, k_cache, v_cache, None, k_cache.shape[2], 0,
+                               k_cache.shape[1], pos, splits, scale,
+                               workspace, out, k, v, table)
+
+
+def _launch_attn_decode(q, kc, vc, blocks, max_seq: int, bs_log: int,
+                        Hkv: int, pos, splits: int, scale: float, workspace,
+                        out, k, v, rope) -> torch.Tensor:
+    """Contiguous caches (``blocks`` None) or paged pools."""
+    B, Hq, D = q.shape
     if workspace is None:
         part_o = torch.empty(B, Hq, splits, D, dtype=torch.float32, device=q.device)
         part_ml = torch.empty(B, Hq, splits, 2, dtype=torch.float32, device=q.device)
     else:
         part_o, part_ml = workspace[0], workspace[1]
-        # a 3rd workspace element (zeroed int32 [B*Hkv*splits] per-split
-        # done-flag buffer) selects the FUSED combine: split 0 of each
-        # (b, hkv) pair polls the flags and reduces the partials in-kernel,
-        # and the separate combine launch is skipped (FEI_FUSED_CMB=0 opts
-        # out for A/B; pass `layer` so the flag tags stay unique across the
-        # layers of one step).
-        if len(workspace) >= 3 and _FUSED_CMB:
-            arrive = workspace[2]
         assert part_o.shape[2] == splits and part_ml.shape[2] == splits, \
             f"workspace sized for {part_o.shape[2]} splits, kernel asked {splits}"
     if out is None:
-        out = torch.empty_like(q)
-    Hkv = k_cache.shape[1]
+        out = torch.empty(B, Hq, D, dtype=q.dtype, device=q.device)
     assert q.stride(2) == 1 and q.stride(1) == D
-    # the kernel's V lane maps tile 256 threads by D/2 and D/8 — both must
-    # divide the block (holds for the llama head dims 64/128; D=96 would
-    # silently under-cover a tile)
+    # a lane's share of a row: D/16 columns
     assert D in (64, 128), f"decode attention supports D in (64,128), got {D}"
-    assert splits <= 64, "combine kernel stages at most 64 split partials"
-    if table is not None:
+    assert splits <= 64, "the combine kernel takes at most 64 splits"
+    assert Hq // Hkv <= 16, "at most 16 query heads per kv head"
+    if rope is not None:
         assert k is not None and v is not None
         assert k.stride(1) == D and k.stride(0) == v.stride(0)
-        kin, vin, cs, kv_bs = _ptr(k), _ptr(v), _ptr(table), k.stride(0)
+        kin, vin, cs, kv_bs = _ptr(k), _ptr(v), _ptr(rope), k.stride(0)
     else:
         kin = vin = cs = None
         kv_bs = 0
-    if arrive is not None:
-        assert arrive.dtype == torch.int32 and \
-            arrive.numel() >= B * Hkv * splits
-    lib.fei_attn_decode(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(part_o),
-                        _ptr(part_ml), _ptr(pos), B, Hq, Hkv, D,
-                        k_cache.shape[2], splits, scale, q.stride(0),
-                        kin, vin, cs, kv_bs,
-                        _ptr(out) if arrive is not None else None,
-                        _ptr(arrive) if arrive is not None else None,
-                        layer, _stream())
-    if arrive is None:
-        lib.fei_attn_decode_combine(_ptr(out), _ptr(part_o), _ptr(part_ml),
-                                    B, Hq, D, splits, _stream())
+    require_lib().fei_attn_decode(
+        _ptr(q), _ptr(kc), _ptr(vc), None if blocks is None else _ptr(blocks),
+        _ptr(part_o), _ptr(part_ml), _ptr(out), _ptr(pos), B, Hq, Hkv, D,
+        max_seq, bs_log, 0 if blocks is None else blocks.shape[1], splits,
+        scale, q.stride(0), kin, vin, cs, kv_bs, _stream())
     return out
 
 
@@ -542,15 +529,10 @@ def _launch_gemv(out, x2, gain, w, wscale, N: int, eps: float, epi: int,
                            _stream())
 
 
-# Fused split-K combine in decode attention (per-head reducer splits poll
-# sc1 done-flags and reduce the partials in-kernel; needs the 3-element
-# workspace). Verified token-identical and measured at PARITY with the
-# separate k_attn_decode_combine launch (275.5 vs 275.8 tok/s on the 8B
-# chain — in a captured graph the combine launch already overlaps the
-# attention grid's drain, so there was no boundary to win; the full
-# 4-protocol measurement ladder is profiles/r02_fused_combine.md).
-# Opt-in via FEI_FUSED_CMB=1; the launch form stays the default.
-_FUSED_CMB = os.environ.get("FEI_FUSED_CMB", "0") == "1"
+# Kept for callers that set it: a decode attention's splits are always added by
+# a launch of their own (adding them in the attention kernel behind flags was
+# no faster, profiles/r02_fused_combine.md).
+_FUSED_CMB = False
 
 
 def _gemm_m8_ok(M: int, N: int, K: int) -> bool:
@@ -739,33 +721,9 @@ def attn_decode_paged(q, k_pool, v_pool, block_table, pos, splits: int = 32,
                 kc[b, :, j * BS:(j + 1) * BS] = k_pool[blk]
                 vc[b, :, j * BS:(j + 1) * BS] = v_pool[blk]
         return ref.attn_decode(q, kc, vc, pos + 1, scale)
-    lib = require_lib()
-    if workspace is None:
-        part_o = torch.empty(B, Hq, splits, D, dtype=torch.float32, device=q.device)
-        part_ml = torch.empty(B, Hq, splits, 2, dtype=torch.float32, device=q.device)
-    else:
-        part_o, part_ml = workspace
-        assert part_o.shape[2] == splits and part_ml.shape[2] == splits
-    if out is None:
-        out = torch.empty_like(q)
-    assert q.stride(2) == 1 and q.stride(1) == D
-    assert D in (64, 128), f"paged attention supports D in (64,128), got {D}"
-    assert splits <= 64
-    if table is not None:
-        assert k is not None and v is not None
-        assert k.stride(1) == D and k.stride(0) == v.stride(0)
-        kin, vin, cs, kv_bs = _ptr(k), _ptr(v), _ptr(table), k.stride(0)
-    else:
-        kin = vin = cs = None
-        kv_bs = 0
-    lib.fei_attn_decode_paged(_ptr(q), _ptr(k_pool), _ptr(v_pool),
-                              _ptr(block_table), _ptr(part_o), _ptr(part_ml),
-                              _ptr(pos), B, Hq, Hkv, D, bs_log,
-                              block_table.shape[1], splits, scale,
-                              q.stride(0), kin, vin, cs, kv_bs, _stream())
-    lib.fei_attn_decode_combine(_ptr(out), _ptr(part_o), _ptr(part_ml),
-                                B, Hq, D, splits, _stream())
-    return out
+    return _launch_attn_decode(
+        q, k_pool, v_pool, block_table, block_table.shape[1] << bs_log,
+        bs_log, Hkv, pos, splits, scale, workspace, out, k, v, table)
 
 
 def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,

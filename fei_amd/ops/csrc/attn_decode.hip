@@ -1,0 +1,391 @@
+// Decode attention: one new token per sequence over its cached keys, split over
+// the keys, all heads of a group together; caches [B,Hkv,max_seq,D] or paged
+// pools [blocks,Hkv,BS,D] behind a block table. n = pos[b] + 1 keys, read on
+// the device, so that a captured launch serves every length. With cos_sin the
+// step's RoPE and the cache row of the new token are made here too.
+//
+// A wave takes chunks of 32 keys by itself. Scores are computed transposed (K
+// times Q^T, 16x16x32: a lane has 8 scores of ONE head), so that the weights
+// lie in the registers as the second operand of V^T times P^T; a lane loads 8
+// keys x D/16 columns of V and turns them in registers. Keys and values never
+// pass LDS, and nothing but the end of a block has a barrier. Roped queries and
+// weights enter the bfloat16 products as a high and a low part (about 16 bits).
+// The chunks go to the blocks' waves in order, so that short contexts end in
+// few blocks (one: it writes the result), and the rest leave at once.
+//
+// Bound by latency (position, table, rows, combine) up to some MB of keys, by
+// HBM beyond. Per layer in a captured step, against a thread per key with the
+// products on the vector units and the scores exchanged through LDS: 300 keys,
+// 32/8 heads of 64: 11.1 -> 4.7 us; 512 and 3400 keys, 32/8 of 128: 12.6 -> 5.2
+// and 20.0 -> 6.6; 8 sequences of up to 2047 keys (43 MB): 26.9 -> 13.4; 20 of
+// up to 600 in pages of 16, heads of 64: 50 -> 17. The combine takes 4 to 5, a
+// launch's least.
+#include "fei_attn.h"
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) u32 u32x4;
+typedef __attribute__((ext_vector_type(2))) u32 u32x2;
+
+constexpr float M_NONE = -3.0e38f;       // maximum of no keys
+constexpr int CHUNK = 32;                // keys of a wave at a time
+constexpr int WAVES = 4;
+
+struct DecodeAttn {
+  const u16* q;
+  u16 *kc, *vc;
+  const int* table;                      // paged: [B, W]
+  float *po, *pml;                       // [B,Hq,splits,D], [B,Hq,splits,2]
+  u16* out;
+  const int* pos;
+  const u16 *kin, *vin;
+  const float* cs;
+  int G, Hkv, max_seq, bs_log, W, splits;
+  float scale;
+  long q_bs, kv_bs;
+};
+
+__device__ __forceinline__ int keys_at(const DecodeAttn& a, int b) {
+  return min(a.pos[b] + 1, a.max_seq);
+}
+// Splits that have keys.
+__device__ __forceinline__ int used_splits(const DecodeAttn& a, int n) {
+  return min(a.splits, (n + CHUNK * WAVES - 1) / (CHUNK * WAVES));
+}
+
+__device__ __forceinline__ f32x2 swap32(float v) {
+  const u32 u = __builtin_bit_cast(u32, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const u32 r0 = r[0], r1 = r[1];
+  return f32x2{__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1)};
+}
+__device__ __forceinline__ f32x2 swap16(float v) {
+  const u32 u = __builtin_bit_cast(u32, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const u32 r0 = r[0], r1 = r[1];
+  return f32x2{__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1)};
+}
+// Over the four lanes of a head, lane % 16 alike.
+__device__ __forceinline__ float head_max(float v) {
+  f32x2 t = swap32(v);
+  t = swap16(fmaxf(t[0], t[1]));
+  return fmaxf(t[0], t[1]);
+}
+__device__ __forceinline__ float head_sum(float v) {
+  f32x2 t = swap32(v);
+  t = swap16(t[0] + t[1]);
+  return t[0] + t[1];
+}
+
+// x1 and x2: dimensions d .. d + 7 and d + D/2 .. of a head; cs: their pairs.
+__device__ __forceinline__ void rope8(float (&x1)[8], float (&x2)[8],
+                                      const float* cs) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const f32x4 t = *(const f32x4*)(cs + 4 * i);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const float u = x1[2 * i + j], w = x2[2 * i + j];
+      x1[2 * i + j] = u * t[2 * j] - w * t[2 * j + 1];
+      x2[2 * i + j] = w * t[2 * j] + u * t[2 * j + 1];
+    }
+  }
+}
+
+template <int N>
+__device__ __forceinline__ void rope_row(float (&x)[N][8], const float* cs,
+                                         int lg) {
+#pragma unroll
+  for (int k = 0; k < N / 2; ++k)
+    rope8(x[k], x[k + N / 2], cs + (k * 32 + 8 * lg) * 2);
+}
+
+template <int D, bool PAGED, bool ROPE>
+__global__ void __launch_bounds__(64 * WAVES, D == 64 ? 4 : 3)
+k_attn_decode(const DecodeAttn a) {
+  constexpr int KS = D / 32;             // steps of a score product
+  constexpr int VC = D / 16;             // columns of V a lane loads
+  typedef __attribute__((ext_vector_type(VC / 2))) u32 vrow;
+  extern __shared__ __align__(16) float so[];      // [WAVES][G][D], then m, l
+  const int split = blockIdx.x, hkv = blockIdx.y, b = blockIdx.z;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, lg = lane >> 4;
+  const int n = keys_at(a, b), last = n - 1;
+  const int chunks = (n + CHUNK - 1) / CHUNK;
+  if (split * WAVES >= chunks) return;
+  const int G = a.G, Hq = a.Hkv * G;
+
+  auto row = [&](int key) {
+    if (PAGED) {
+      const int blk = a.table[(long)b * a.W + (key >> a.bs_log)];
+      return ((((long)blk * a.Hkv + hkv) << a.bs_log) +
+              (key & ((1 << a.bs_log) - 1))) * D;
+    }
+    return (((long)b * a.Hkv + hkv) * a.max_seq + key) * D;
+  };
+  const float* cs = ROPE ? a.cs + (long)last * D : nullptr;
+
+  // queries, head lane % 16 (what the lanes past the last head compute is not
+  // used)
+  s16x8 qh[KS], ql[ROPE ? KS : 1];
+  {
+    const u16* qp = a.q + (long)b * a.q_bs +
+                    (long)(hkv * G + min(l15, G - 1)) * D + 8 * lg;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) qh[k] = ld8(qp + k * 32);
+    if (ROPE) {
+      float x[KS][8];
+#pragma unroll
+      for (int k = 0; k < KS; ++k)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[k][j] = bf2f((u16)qh[k][j]);
+      rope_row(x, cs, lg);
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        s16x8 p[2];
+        weight_parts(x[k], p);
+        qh[k] = p[0];
+        ql[k] = p[1];
+      }
+    }
+  }
+  const float c = a.scale * El<u16>::base;
+  // The wave with the last chunk makes the new token's row, for the cache and
+  // for itself; no other wave reads it.
+  __shared__ __align__(16) u16 fresh[2][D];
+  if (ROPE && (chunks - 1) % (a.splits * WAVES) == split * WAVES + wid &&
+      lane < D / 2) {
+    const u16* kp = a.kin + (long)b * a.kv_bs + (long)hkv * D + lane;
+    const u16* vp = a.vin + (long)b * a.kv_bs + (long)hkv * D + lane;
+    const f32x2 t = *(const f32x2*)(cs + 2 * lane);
+    const float u = bf2f(kp[0]), w = bf2f(kp[D / 2]);
+    const u16 row0[2] = {El<u16>::st(u * t[0] - w * t[1]), vp[0]};
+    const u16 row1[2] = {El<u16>::st(w * t[0] + u * t[1]), vp[D / 2]};
+    const long at = row(last) + lane;
+    a.kc[at] = fresh[0][lane] = row0[0];
+    a.kc[at + D / 2] = fresh[0][lane + D / 2] = row1[0];
+    a.vc[at] = fresh[1][lane] = row0[1];
+    a.vc[at + D / 2] = fresh[1][lane + D / 2] = row1[1];
+  }
+
+  float m = M_NONE, l = 0.f;
+  f32x4 o[VC];
+#pragma unroll
+  for (int e = 0; e < VC; ++e) o[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  for (int ch = split * WAVES + wid; ch < chunks; ch += a.splits * WAVES) {
+    const int k0 = ch * CHUNK;
+    s16x8 kf[2][KS];
+    vrow vf[8];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const u16* kp = a.kc + row(min(k0 + 16 * t + l15, last)) + 8 * lg;
+#pragma unroll
+      for (int k = 0; k < KS; ++k) kf[t][k] = ld8(kp + k * 32);
+    }
+#pragma unroll
+    for (int r = 0; r < 8; ++r)
+      vf[r] = *(const vrow*)(
+          a.vc + row(min(k0 + (r & 4) * 4 + 4 * lg + (r & 3), last)) +
+          VC * l15);
+    if (ROPE && ch == chunks - 1) {      // the new token's row is in LDS
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        if (k0 + 16 * t + l15 == last)
+#pragma unroll
+          for (int k = 0; k < KS; ++k) kf[t][k] = ld8(fresh[0] + 8 * lg + k * 32);
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        if (k0 + (r & 4) * 4 + 4 * lg + (r & 3) == last)
+          vf[r] = *(const vrow*)(fresh[1] + VC * l15);
+    }
+    if (k0 + CHUNK > n) {                // what lies past the keys counts 0
+#pragma unroll
+      for (int r = 0; r < 8; ++r)
+        if (k0 + (r & 4) * 4 + 4 * lg + (r & 3) > last)
+#pragma unroll
+          for (int e = 0; e < VC / 2; ++e) vf[r][e] = 0;
+    }
+    float s[8];                          // keys 4 lg + 0..3, then 16 on
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        acc = mma(kf[t][k], qh[k], acc);
+        if (ROPE) acc = mma(kf[t][k], ql[k], acc);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        s[4 * t + r] = k0 + 16 * t + 4 * lg + r > last ? -1.f / 0.f
+                                                       : acc[r] * c;
+    }
+    float mx = fmaxf(s[0], s[1]);
+#pragma unroll
+    for (int i = 2; i < 8; ++i) mx = fmaxf(mx, s[i]);
+    const float mn = fmaxf(m, head_max(mx));
+    const float al = __builtin_amdgcn_exp2f(m - mn);
+    m = mn;
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      s[i] = __builtin_amdgcn_exp2f(s[i] - mn);
+      ps += s[i];
+    }
+    l = fmaf(l, al, ps);
+    s16x8 p[2];
+    weight_parts(s, p);
+#pragma unroll
+    for (int w = 0; w < VC / 2; ++w)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        u32x4 t;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          t[i] = __builtin_amdgcn_perm(vf[2 * i + 1][w], vf[2 * i][w],
+                                       hf ? 0x07060302u : 0x05040100u);
+        const s16x8 va = __builtin_bit_cast(s16x8, t);
+        f32x4& oe = o[2 * w + hf];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) oe[r] *= al;
+        oe = mma(va, p[0], oe);
+        oe = mma(va, p[1], oe);
+      }
+  }
+  l = head_sum(l);
+  // column VC * (4 lg + r) + e of head l15 is o[e][r]
+  float* sml = so + WAVES * G * D;
+  if (l15 < G) {
+    float* dst = so + (wid * G + l15) * D;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int e = 0; e < VC; e += 4)
+        *(f32x4*)(dst + VC * (4 * lg + r) + e) =
+            f32x4{o[e][r], o[e + 1][r], o[e + 2][r], o[e + 3][r]};
+    if (lg == 0) {
+      sml[(wid * G + l15) * 2] = m;
+      sml[(wid * G + l15) * 2 + 1] = l;
+    }
+  }
+  __syncthreads();
+  const bool whole = used_splits(a, n) == 1;
+  for (int i = tid * 4; i < G * D; i += 64 * WAVES * 4) {
+    const int g = i / D, d = i - g * D;
+    float mm = M_NONE, ll = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) mm = fmaxf(mm, sml[(w * G + g) * 2]);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = __builtin_amdgcn_exp2f(sml[(w * G + g) * 2] - mm);
+      const f32x4 t = *(const f32x4*)(so + (w * G + g) * D + d);
+      ll = fmaf(f, sml[(w * G + g) * 2 + 1], ll);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = fmaf(f, t[e], v[e]);
+    }
+    const long hq = (long)b * Hq + hkv * G + g;
+    if (whole) {
+      const float inv = ll > 0.f ? 1.f / ll : 0.f;
+      u16 y[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) y[e] = El<u16>::st(v[e] * inv);
+      __builtin_memcpy(a.out + hq * D + d, y, sizeof(y));
+    } else {
+      *(f32x4*)(a.po + (hq * a.splits + split) * D + d) = v;
+      if (d == 0)
+        *(f32x2*)(a.pml + (hq * a.splits + split) * 2) = f32x2{mm, ll};
+    }
+  }
+}
+
+// out[b,hq] from the splits that have keys; nothing to do where one had all.
+// One block per head, 8 (D = 128) or 16 splits side by side.
+template <int D>
+__global__ void __launch_bounds__(256) k_attn_decode_combine(const DecodeAttn a) {
+  constexpr int SIDE = 256 / (D / 4);
+  __shared__ f32x4 part[SIDE][D / 4];
+  const long hq = blockIdx.x;
+  const int b = hq / (a.Hkv * a.G);
+  const int used = used_splits(a, keys_at(a, b));
+  if (used == 1) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int side = tid / (D / 4), d = tid % (D / 4);
+  const float* ml = a.pml + hq * a.splits * 2;
+  const f32x4* po = (const f32x4*)(a.po + hq * a.splits * D) + d;
+  const f32x2 t = lane < used ? *(const f32x2*)(ml + 2 * lane)
+                              : f32x2{M_NONE, 0.f};
+  float m = row16_max(t[0]);
+  f32x2 sw = swap16(m);
+  sw = swap32(fmaxf(sw[0], sw[1]));
+  m = fmaxf(sw[0], sw[1]);
+  float l = row16_sum(t[1] * __builtin_amdgcn_exp2f(t[0] - m));
+  sw = swap16(l);
+  sw = swap32(sw[0] + sw[1]);
+  l = sw[0] + sw[1];
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int s = side; s < used; s += SIDE) {
+    const float f = __builtin_amdgcn_exp2f(ml[2 * s] - m);
+    const f32x4 x = po[(long)s * (D / 4)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = fmaf(f, x[e], v[e]);
+  }
+  part[side][d] = v;
+  __syncthreads();
+  if (side) return;
+#pragma unroll
+  for (int i = 1; i < SIDE; ++i)
+    if (i < used)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += part[i][d][e];
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  u16 y[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = El<u16>::st(v[e] * inv);
+  __builtin_memcpy(a.out + hq * D + d * 4, y, sizeof(y));
+}
+
+template <int D>
+void launch_decode(const DecodeAttn& a, int B, hipStream_t stream) {
+  const dim3 grid(a.splits, a.Hkv, B), block(64 * WAVES);
+  const size_t lds = (size_t)WAVES * a.G * (D + 2) * sizeof(float);
+#define GO(PAGED, ROPE)                                                       \
+  hipLaunchKernelGGL((k_attn_decode<D, PAGED, ROPE>), grid, block, lds, stream, \
+                     a)
+  if (a.table) {
+    if (a.cs) GO(true, true); else GO(true, false);
+  } else {
+    if (a.cs) GO(false, true); else GO(false, false);
+  }
+#undef GO
+  if (a.splits > 1)
+    hipLaunchKernelGGL(k_attn_decode_combine<D>, dim3(B * a.Hkv * a.G),
+                       dim3(256), 0, stream, a);
+}
+
+}  // namespace
+
+// max_seq: rows of a head in a contiguous cache; of a paged one (table not
+// null) the positions that a row of the table can name. cs null: q is roped and
+// the new token's row is in the cache. Up to 16 query heads a kv head, up to 64
+// splits; D is 64 or 128.
+extern "C" void fei_attn_decode(const void* q, void* kc, void* vc,
+                                const int* table, float* po, float* pml,
+                                void* out, const int* pos, int B, int Hq,
+                                int Hkv, int D, int max_seq, int bs_log, int W,
+                                int splits, float scale, long q_bs,
+                                const void* kin, const void* vin,
+                                const float* cs, long kv_bs,
+                                hipStream_t stream) {
+  const DecodeAttn a{(const u16*)q, (u16*)kc,         (u16*)vc,
+                     table,         po,               pml,
+                     (u16*)out,     pos,              (const u16*)kin,
+                     (const u16*)vin, cs,             Hq / Hkv,
+                     Hkv,           max_seq,          bs_log,
+                     W,             splits,           scale,
+                     q_bs,          kv_bs};
+  if (D == 128) launch_decode<128>(a, B, stream);
+  else if (D == 64) launch_decode<64>(a, B, stream);
+}

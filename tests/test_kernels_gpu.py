@@ -129,3 +129,73 @@ def test_gemv_geometries(lib, M, N, K, fp8):
     assert row_err(r, res.double() + x64 @ w64[:N].T) < 2 ** -8
     y = xn @ w64.T
     assert row_err(sw, torch.nn.functional.silu(y[:, :N]) * y[:, N:]) < tol
+
+
+# -- decode attention --------------------------------------------------------------
+
+def rope64(x, pos, theta=500000.0):
+    D = x.shape[-1]
+    inv = theta ** (-torch.arange(0, D, 2, dtype=torch.float64, device=DEV) / D)
+    a = (pos.double().view(-1, 1) * inv).unsqueeze(1)
+    u, w = x[..., :D // 2].double(), x[..., D // 2:].double()
+    return torch.cat([u * a.cos() - w * a.sin(), w * a.cos() + u * a.sin()], -1)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,splits,lens", [
+    (8, 2, 4, [1, 2]),               # the new token alone
+    (3, 1, 32, [31, 32, 33]),        # around a wave's 32 keys, groups of 3
+    (8, 1, 16, [128, 129, 300]),     # one split, two
+    (16, 1, 2, [700]),               # more keys than one round of the splits
+    (4, 4, 64, [2000, 15, 1]),
+    (8, 2, 1, [257, 500]),
+])
+def test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, splits, lens):
+    """Against float64, over caches whose rows past each length are NaN, with
+    the step's RoPE and cache row made inside or before."""
+    from fei_amd.ops import reference as ref
+    B, BS, T = len(lens), 16, max(lens) + 5
+    W = (Hq + 2 * Hkv) * D
+    qkv = randbf(B, W, seed=sum(lens))
+    q, k, v = (qkv[:, a * D:b * D].view(B, -1, D) for a, b in
+               ((0, Hq), (Hq, Hq + Hkv), (Hq + Hkv, Hq + 2 * Hkv)))
+    pos = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    kc, vc = randbf(B, Hkv, T, D, seed=1), randbf(B, Hkv, T, D, seed=2)
+    for b, n in enumerate(lens):
+        kc[b, :, n - rope:] = vc[b, :, n - rope:] = float("nan")
+    args = dict(splits=splits)
+    if rope:
+        table = ref.rope_table(T, D, device=DEV)
+        args.update(k=k, v=v, table=table)
+    if paged:
+        nb = -(-T // BS)
+        perm = torch.randperm(B * nb, generator=torch.Generator().manual_seed(3))
+        bt = perm.view(B, nb).int().to(DEV)
+        pools = []
+        for c in (kc, vc):
+            pad = torch.full((B, Hkv, nb * BS, D), float("nan"), device=DEV,
+                             dtype=torch.bfloat16)
+            pad[:, :, :T] = c
+            p = torch.empty(B * nb, Hkv, BS, D, device=DEV, dtype=torch.bfloat16)
+            p[bt.view(-1).long()] = pad.view(B, Hkv, nb, BS, D).transpose(1, 2) \
+                .reshape(B * nb, Hkv, BS, D)
+            pools.append(p)
+        got = lib.attn_decode_paged(q, *pools, bt, pos, **args)
+        kn, vn = (p[bt.long()].transpose(1, 2).reshape(B, Hkv, nb * BS, D)[:, :, :T]
+                  for p in pools)
+    else:
+        got = lib.attn_decode(q, kc, vc, pos, **args)
+        kn, vn = kc, vc
+    q64 = rope64(q, pos) if rope else q.double()
+    k64 = rope64(k, pos)
+    for b, n in enumerate(lens):
+        if rope:                     # the row is in the cache now, rounded once
+            assert row_err(kn[b, :, n - 1], k64[b]) < 2 ** -8
+            assert torch.equal(vn[b, :, n - 1], v[b])
+        kk, vv = (t[b, :, :n].double().repeat_interleave(Hq // Hkv, 0)
+                  for t in (kn, vn))
+        p = torch.softmax((kk * q64[b].unsqueeze(1)).sum(-1) * D ** -0.5, -1)
+        # the result is rounded once: 2^-9
+        assert row_err(got[b], (p.unsqueeze(-1) * vv).sum(1)) < 2 ** -8
