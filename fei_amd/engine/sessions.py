@@ -278,35 +278,32 @@ class PagedSessionManager:
 
     def _forward_paged(self, token: torch.Tensor, pos: torch.Tensor,
                        table: torch.Tensor) -> torch.Tensor:
-        """Plain decode forward with block-table attention. Same GEMV /
-        norm kernels as LlamaModel.forward_decode (llama.py); RoPE + the
-        single-row KV append are torch-side (control plane — O(Hkv*D) per
-        session, independent of context length) and fully device-resident:
-        the block/offset of the appended row derive from `pos` and `table`
-        with gather/advanced indexing, so a whole step chain runs without
-        a host sync (step_chunk)."""
+        """Decode forward with block-table attention: the products of
+        LlamaModel.forward_decode (llama.py). Fully device-resident - the
+        appended row's block and offset derive from `pos` and `table` - so a
+        whole step chain runs without a host sync (step_chunk)."""
         m = self.model
         s = m.spec
         B = token.shape[0]
         BS = self.pool.block_size
-        h = F.embedding(token.long(), m.emb)
+        h = F.embedding(token, m.emb)
         scale = 1.0 / math.sqrt(m.D)
-        n_layers = len(m.layers)
-        x = ops.rmsnorm(h, m.layers[0].norm_attn, s.norm_eps)
-        pos_l = pos.long()
+        eps, n_layers = s.norm_eps, len(m.layers)
         gpu = m.device.type == "cuda"
+        fused = m.fused_rows(B)
         if not gpu:
+            pos_l = pos.long()
             blk = table.gather(1, (pos_l // BS).unsqueeze(1)) \
                 .squeeze(1).long()
             off = pos_l % BS
+        x = None if fused else ops.rmsnorm(h, m.layers[0].norm_attn, eps)
         for li, lw in enumerate(m.layers):
-            qkv = ops.linear_decode(x, lw.wqkv)
+            qkv = ops.gemv_norm(h, lw.norm_attn, lw.wqkv, eps) if fused \
+                else ops.linear_decode(x, lw.wqkv)
             q, k, v = m._qkv_views(qkv, B)
             kp, vp = self.pool.k[li], self.pool.v[li]
             if gpu:
-                # fused in-kernel RoPE + paged append (the eager torch
-                # rope/append chain was ~15 launches/layer — ~30% of the
-                # serving step)
+                # RoPE and the paged append are made in the kernel
                 att = ops.attn_decode_paged(q, kp, vp, table, pos,
                                             splits=self._splits(B),
                                             scale=scale,
@@ -321,13 +318,21 @@ class PagedSessionManager:
                                             splits=self._splits(B),
                                             scale=scale,
                                             workspace=self._workspace(B))
-            o = ops.linear_decode(att.reshape(B, -1), lw.wo)
-            x, h = ops.fused_add_rmsnorm(o, h, lw.norm_mlp, s.norm_eps)
+            att = att.reshape(B, -1)
+            if fused:
+                ops.gemv_res(att, lw.wo, h)
+                act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, eps)
+                ops.gemv_res(act, lw.wdown, h)
+                continue
+            o = ops.linear_decode(att, lw.wo)
+            x, h = ops.fused_add_rmsnorm(o, h, lw.norm_mlp, eps)
             act = ops.gemv_swiglu(x, lw.wgu)
             d = ops.linear_decode(act, lw.wdown)
             next_norm = (m.layers[li + 1].norm_attn if li + 1 < n_layers
                          else m.norm_f)
-            x, h = ops.fused_add_rmsnorm(d, h, next_norm, s.norm_eps)
+            x, h = ops.fused_add_rmsnorm(d, h, next_norm, eps)
+        if fused:
+            return ops.gemv_norm(h, m.norm_f, m.lm_head, eps)
         return ops.linear_decode(x, m.lm_head)
 
 

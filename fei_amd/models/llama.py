@@ -208,15 +208,15 @@ class LlamaModel:
         the TP hot loop samples on shards and gathers 8 bytes/seq instead,
         engine._decode_step_tp).
         ``fused_norm`` (tp=1 only): the residual stream stays inside the
-        GEMV kernels — norm in QKV/gate-up, residual add in O/down; 6 kernels
-        per layer instead of 9. On the GPU always so for few rows."""
-        # Up to three rows the GEMVs hold the norms and the residual
-        # themselves: six launches a layer for nine (8B, batch 1: 3.54 ->
-        # 3.15 ms a step). On the CPU the caller's choice stays.
+        GEMV kernels — norm in QKV/gate-up, residual add in O/down. On the
+        GPU always so for few rows; there it chooses fp8 weights at batch 1,
+        if the model has some."""
+        # Few rows: the products add to the residual and make the SwiGLU, up
+        # to three rows the norms too: six or eight launches a layer for nine
+        # or ten (8B, batch 1: 3.54 -> 3.15 ms a step). On the CPU the
+        # caller's choice stays.
         B = token.shape[0]
-        fits = B <= 3 and B * self.spec.hidden_size * 2 <= 64 * 1024
-        if self.tp_size == 1 and fits and (self.emb.is_cuda or
-                                           (fused_norm and B == 1)):
+        if self.fused_rows(B) or (fused_norm and B == 1 and self.tp_size == 1):
             return self._forward_decode_fused_norm(
                 token, pos, k_caches, v_caches, attn_splits, workspace,
                 fused_attn, attn_out, fused_norm)
@@ -251,6 +251,14 @@ class LlamaModel:
         if gather_logits:
             logits = all_gather_cat(logits, dim=-1, ctx=self.tp)
         return logits
+
+    def fused_rows(self, B: int) -> bool:
+        """Whether a step of B rows runs the chain whose products hold the
+        residual."""
+        lw = self.layers[0]
+        return self.tp_size == 1 and all(
+            ops.own_product(B, w)
+            for w in (lw.wqkv, lw.wo, lw.wgu, lw.wdown, self.lm_head))
 
     def forward_decode_stream(self, token, pos, k_caches, v_caches,
                               ws: dict, bufs) -> torch.Tensor:

@@ -69,7 +69,8 @@ def _try_load() -> None:
     lib.fei_mfma_probe.argtypes = [_vp, _vp, _vp, _vp]
     lib.fei_gemv.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _i,
                              _vp, _vp]
-    lib.fei_gemm_m8.argtypes = [_vp, _vp, _vp, _i, _i, _i, _i, _vp]
+    lib.fei_skinny.argtypes = ([_vp] * 3 + [_i] * 4 + [_vp, _f, _f, _i, _i] +
+                               [_vp, _vp, _l, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -535,13 +536,6 @@ def _launch_gemv(out, x2, gain, w, wscale, N: int, eps: float, epi: int,
 _FUSED_CMB = False
 
 
-def _gemm_m8_ok(M: int, N: int, K: int) -> bool:
-    # MFMA GEMM tile: A-fragment rows clamp to M-1 so M <= 16 is CORRECT,
-    # but at M = 16 hipBLASLt measured faster (serving-16: 2473 vs 2337
-    # tok/s) — route only the 4..8 range where the tile wins 1.27-1.65x
-    return 4 <= M <= 8 and K % 1024 == 0 and N % 16 == 0
-
-
 _GEMV_ROWS = (1, 2, 3, 4, 8)
 
 
@@ -554,53 +548,62 @@ def _norm_ok(M: int, K: int) -> bool:
     return _gemv_ok(M, K) and M * K * 2 <= 128 * 1024
 
 
+def _product(x: torch.Tensor, w: torch.Tensor, rows_out: int) -> Optional[str]:
+    """Which kernel takes x @ w^T: "skinny" (matrix units), "gemv", or None
+    (the library; CPU)."""
+    K = x.shape[-1]
+    M = x.numel() // K if K else 0
+    if not x.is_cuda or not M or not rows_out:
+        return None
+    if _mixers.skinny_ok(M, K, x, w):
+        return "skinny"
+    return "gemv" if _gemv_ok(M, K) else None
+
+
+def own_product(M: int, w: torch.Tensor) -> bool:
+    """Whether M rows of w's type (a tensor of their own) times w run in this
+    library's kernels, which add to a residual and make a SwiGLU without a
+    launch of its own."""
+    N, K = w.shape
+    return w.is_cuda and N > 0 and (_mixers.skinny_ok(M, K, w, w) or
+                                    _gemv_ok(M, K))
+
+
 def linear_decode(x: torch.Tensor, w: torch.Tensor,
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """F.linear for skinny M: streaming GEMV or MFMA tile on GPU. Falls back
-    to torch for unsupported shapes/CPU."""
+    """F.linear for skinny M: streaming GEMV or matrix-core tile on GPU. Falls
+    back to torch for unsupported shapes/CPU."""
     M = x.numel() // x.shape[-1]
-    K = x.shape[-1]
-    N = w.shape[0]
-    if not x.is_cuda or not (_gemv_ok(M, K) or _gemm_m8_ok(M, N, K)):
+    N, K = w.shape
+    how = _product(x, w, N)
+    if how is None:
         return torch.nn.functional.linear(x, w)
-    lib = require_lib()
     x2 = x.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=x.device)
-    if _gemm_m8_ok(M, N, K):
-        # MFMA tile: beats the VALU GEMV at every llama batch shape
-        # (1.27-1.65x — profiles/r02_batch_attention.md addendum).
-        # ALWAYS plain loads: the nt hint on the 16 B/lane staged W
-        # fetch measured 6.50 vs 5.01 ms/step at batch 8.
-        lib.fei_gemm_m8(_ptr(out), _ptr(x2), _ptr(w), M, N, K, 0,
-                        _stream())
-        return out
-    _launch_gemv(out, x2, None, w, None, N, 0.0, _BF16)
+    if how == "skinny":
+        _mixers.skinny(out, x2, w, N, _mixers.EPI_BF16)
+    else:
+        _launch_gemv(out, x2, None, w, None, N, 0.0, _BF16)
     return out
 
 
 def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Fused gate/up GEMV + SwiGLU: x [M,K] @ [2I,K]^T -> silu(g)*u [M,I]."""
+    """Fused gate/up product + SwiGLU: x [M,K] @ [2I,K]^T -> silu(g)*u [M,I]."""
     M = x.numel() // x.shape[-1]
     K = x.shape[-1]
     I = wgu.shape[0] // 2
-    if not x.is_cuda or not (_gemv_ok(M, K) or _gemm_m8_ok(M, 2 * I, K)):
+    how = _product(x, wgu, I)
+    if how is None:
         return swiglu(torch.nn.functional.linear(x, wgu))
-    lib = require_lib()
     x2 = x.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*x.shape[:-1], I, dtype=x.dtype, device=x.device)
-    if _gemm_m8_ok(M, 2 * I, K):
-        # MFMA over the stacked [2I, K] weight (its [M, 2I] output is
-        # k_swiglu's packed input): 68.3 -> ~47 us on the 8B gate/up at
-        # batch 8 vs the fused VALU kernel
-        gu = torch.empty(M, 2 * I, dtype=x.dtype, device=x.device)
-        lib.fei_gemm_m8(_ptr(gu), _ptr(x2), _ptr(wgu), M, 2 * I, K, 0,
-                        _stream())
-        lib.fei_swiglu(_ptr(out), _ptr(gu), M, I, _stream())
-        return out
-    _launch_gemv(out, x2, None, wgu, None, I, 0.0, _SWIGLU)
+    if how == "skinny":
+        _mixers.skinny(out, x2, wgu, I, _mixers.EPI_SWIGLU, act=out, stride=I)
+    else:
+        _launch_gemv(out, x2, None, wgu, None, I, 0.0, _SWIGLU)
     return out
 
 
@@ -613,13 +616,19 @@ def gemv_res(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
     gemv_norm/gemv_swiglu_norm takes as ``ssq``. Ignored on the CPU fallback —
     consumers recompute exactly there."""
     M = x.numel() // x.shape[-1]
-    K = x.shape[-1]
-    if not x.is_cuda or not _gemv_ok(M, K):
+    N, K = w.shape
+    how = _product(x, w, N)
+    if ssq_out is not None and how == "skinny" and _gemv_ok(M, K):
+        how = "gemv"
+    if how is None:
         lin = torch.nn.functional.linear(x, w)
         res.copy_((res.float() + lin.float().view_as(res)).to(res.dtype))
-        return res
-    _launch_gemv(res, x.contiguous().view(M, K), None, w, None, w.shape[0],
-                 0.0, _RES, ssq_out)
+    elif how == "skinny":
+        _mixers.skinny(res, x.contiguous().view(M, K), w, N,
+                       _mixers.EPI_RES_BF16)
+    else:
+        _launch_gemv(res, x.contiguous().view(M, K), None, w, None, N, 0.0,
+                     _RES, ssq_out)
     return res
 
 
@@ -632,16 +641,14 @@ def gemv_norm(res: torch.Tensor, wnorm: torch.Tensor, w: torch.Tensor,
     ``ssq`` [M] f32: the sums of squares of res rows, if the caller has them
     (from a prior gemv_res ``ssq_out``)."""
     M = res.numel() // res.shape[-1]
-    K = res.shape[-1]
-    N = w.shape[0]
-    if not res.is_cuda or not _gemv_ok(M, K):
+    N, K = w.shape
+    how = _product(res, w, N)
+    if how is None:
         return torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w)
+    if how == "skinny" or not _norm_ok(M, K):
+        return linear_decode(rmsnorm(res, wnorm, eps), w, out)
     if out is None:
         out = torch.empty(*res.shape[:-1], N, dtype=res.dtype, device=res.device)
-    if not _norm_ok(M, K):
-        _launch_gemv(out, rmsnorm(res, wnorm, eps).view(M, K), None, w, None,
-                     N, 0.0, _BF16)
-        return out
     _launch_gemv(out, res.contiguous().view(M, K), wnorm, w, None, N, eps,
                  _BF16, ssq)
     return out
@@ -656,14 +663,13 @@ def gemv_swiglu_norm(res: torch.Tensor, wnorm: torch.Tensor,
     M = res.numel() // res.shape[-1]
     K = res.shape[-1]
     I = wgu.shape[0] // 2
-    if not res.is_cuda or not _gemv_ok(M, K):
+    how = _product(res, wgu, I)
+    if how is None:
         return swiglu(torch.nn.functional.linear(rmsnorm(res, wnorm, eps), wgu))
+    if how == "skinny" or not _norm_ok(M, K):
+        return gemv_swiglu(rmsnorm(res, wnorm, eps), wgu, out)
     if out is None:
         out = torch.empty(*res.shape[:-1], I, dtype=res.dtype, device=res.device)
-    if not _norm_ok(M, K):
-        _launch_gemv(out, rmsnorm(res, wnorm, eps).view(M, K), None, wgu,
-                     None, I, 0.0, _SWIGLU)
-        return out
     _launch_gemv(out, res.contiguous().view(M, K), wnorm, wgu, None, I, eps,
                  _SWIGLU, ssq)
     return out

@@ -2,13 +2,20 @@
 #pragma once
 #include "fei_common.h"
 
-enum { EPI_BF16 = 0, EPI_F32 = 1, EPI_RES = 2, EPI_PARALLEL = 3 };
+enum {
+  EPI_BF16 = 0,
+  EPI_F32 = 1,
+  EPI_RES = 2,        // added to float32
+  EPI_PARALLEL = 3,
+  EPI_RES_BF16 = 4,   // added to bfloat16
+  EPI_SWIGLU = 5,     // of a gate and an up product, to act
+};
 
 struct Epilogue {
   const float* bias;   // per column, may be null
   float scale;
   float cap;           // 0: no softcap
-  // EPI_PARALLEL: n_mix columns go to out, the next n_router to router, of
+  // EPI_SWIGLU: rows of act are ``as`` apart. EPI_PARALLEL: n_mix columns go to out, the next n_router to router, of
   // the rest relu(.)^2 to act, whose rows are ``as`` apart
   int n_mix, n_router;
   float* router;
@@ -33,6 +40,8 @@ __device__ __forceinline__ void epilogue(void* out, int row, int N, int col,
   const long at = (long)row * N + col;
   if (EPI == EPI_BF16) {
     ((u16*)out)[at] = f2bf(v);
+  } else if (EPI == EPI_RES_BF16) {
+    ((u16*)out)[at] = f2bf(bf2f(((u16*)out)[at]) + v);
   } else if (EPI == EPI_RES) {
     ((float*)out)[at] += v * ep.scale;
   } else if (EPI == EPI_F32) {

@@ -2,7 +2,7 @@
 // out[M, N] = x[M, K] @ W[N, K]^T, F.linear's layout.
 //
 // k_gemv streams the weights, bfloat16 or fp8 (e4m3fn, a scale per row), through
-// the vector units; from M = 4 on k_gemm_m8 (below) uses the matrix units.
+// the vector units; from M = 4 on k_skinny (below) uses the matrix units.
 #include <type_traits>
 
 #include "fei_epilogue.h"
@@ -356,143 +356,212 @@ void fei_prefetch(const void* w, long bytes, void* sink, int n_blocks,
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// MFMA M<=8 GEMM: out[M, N] = x[M, K] @ W[N, K]^T for the decode batch
-// path. Four VALU-kernel variants measured slower than the pipelined
-// k_gemv<8> (profiles/r02_batch_attention.md); this MFMA tile beats it
-// on every llama shape (qkv 1.45x, o 1.43x, down 1.27x, stacked gate/up
-// 1.65x — experimental/gemv_mfma.hip, numerics exact vs the VALU form).
-// Structure: 16 n-rows per workgroup, each of NW waves owns K/NW with
-// wave-private double-buffered LDS staging (register prefetch overlaps
-// the next tile's loads with the current tile's MFMAs; same-wave ds
-// ordering needs no barriers), one end-of-kernel cross-wave C reduce.
-// A-fragment rows clamp to M-1: the duplicate rows only produce C rows
-// >= M, which are never written. Requires K % 1024 == 0, N % 16 == 0
-// (the wrapper routes other shapes to k_gemv).
-#define GEMM_NT 16
-#define GEMM_KC 128
-#define GSWZ(row, col8) ((col8) ^ ((row) & 7))
-
+// The same for 4 to 64 rows on the matrix units. The block's four waves share K;
+// a wave streams 16 RT rows of w and the rows of x, 64 of K a stage, S stages
+// ahead, by direct loads into LDS of its own, so that nothing but the sum at the
+// end has a barrier. A load takes 8 whole lines of 128 bytes (fragments read
+// from memory directly, 16 lanes on 16 rows, come one lane a cycle: 4096 x 4096
+// in 9.6 us, 28672 x 4096 in 52); the 16-byte places of a row are permuted by
+// the row, so that the fragment reads spread over the banks.
+//
+// Bound by HBM, and with many rows by the loads of x, of which a block repeats
+// all. Measured with cold weights in a graph, 8 rows, against tiles through
+// registers with 4 KB a wave in flight: 6144 x 4096 16.0 -> 10.6 us, 4096 x 4096
+// 10.3 -> 7.8, 28672 x 4096 53 -> 41, 4096 x 14336 29 -> 20.2, 128256 x 4096 190
+// -> 172. 20 rows, against the library: 3072 x 2048 11.9 -> 5.8, 2048 x 2048
+// 10.9 -> 5.5, 16384 x 2048 17.6 -> 14.6, 2048 x 8192 14.9 -> 13.7.
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) float f32x4_g;
+// As load_lds, for what is read once.
+__device__ __forceinline__ void load_lds_nt(const u16* src, u32 lds) {
+  u32 keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off nt\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds)
+      : "memory");
+}
 
-template <bool NTW, int EPI, int NW = 4>
-__global__ void __launch_bounds__(NW * 64)
-k_gemm_m8(void* __restrict__ outp, const u16* __restrict__ x,
-          const u16* __restrict__ w, int M, int N, int K, Epilogue ep) {
-  const int n0 = blockIdx.x * GEMM_NT;
-  const int tid = threadIdx.x;
-  const int wv = tid >> 6;
-  const int lane = tid & 63;
+// XL: groups of 8 rows of x. N: results a row of x; with EPI_SWIGLU w has N
+// rows of gates, then N of up, and half of a wave's tiles are either.
+template <int EPI, int XL, int RT, int S>
+__global__ void __launch_bounds__(256)
+k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
+         const u16* __restrict__ w, int M, int N, int K, Epilogue ep) {
+  constexpr int MT = (XL + 1) / 2;
+  constexpr int LOADS = 2 * RT + XL, STAGE = LOADS * 512;
+  constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : RT;
+  extern __shared__ __align__(16) u16 buf[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, lg = lane >> 4;
-  __shared__ u16 wt[NW][2][GEMM_NT * GEMM_KC];
-  __shared__ float cred[NW][16][16];
-
-  f32x4_g acc = {0.f, 0.f, 0.f, 0.f};
-  const int kq = K / NW;
-  const int nv8 = GEMM_KC / 8;
-  const int k_lo = wv * kq, k_hi = (wv + 1) * kq;
-  const int arow = l15 < M ? l15 : M - 1;
-  const int srow = lane / 4, scol8 = (lane % 4) * 4;
-  auto fetch = [&](int k0, s16x8 r[4]) {
+  const int n0 = blockIdx.x * 16 * RO;
+  const int r8 = lane >> 3, c8 = ((lane & 7) ^ r8) * 8;
+  const int steps = K / 64, per = (steps + 3) / 4;
+  const int lo = wid * per, hi = min(steps, lo + per);
+  const u16* src[LOADS];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const s16x8* p = (const s16x8*)(w + (long)(n0 + srow) * K + k0 +
-                                      (scol8 + j) * 8);
-      r[j] = NTW ? __builtin_nontemporal_load(p) : *p;
-    }
-  };
-  auto put = [&](int buf, s16x8 r[4]) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      ((s16x8*)wt[wv][buf])[srow * nv8 + GSWZ(srow, scol8 + j)] = r[j];
-  };
-  s16x8 pre[4];
-  fetch(k_lo, pre);
-  put(0, pre);
-  int buf = 0;
-  for (int k0 = k_lo; k0 < k_hi; k0 += GEMM_KC) {
-    if (k0 + GEMM_KC < k_hi) fetch(k0 + GEMM_KC, pre);
-#pragma unroll
-    for (int kb = 0; kb < GEMM_KC / 32; ++kb) {
-      const s16x8 a_frag =
-          *(const s16x8*)(x + (long)arow * K + k0 + kb * 32 + lg * 8);
-      const int col8 = kb * 4 + lg;
-      const s16x8 b_frag =
-          ((s16x8*)wt[wv][buf])[l15 * nv8 + GSWZ(l15, col8)];
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_frag, b_frag, acc,
-                                                    0, 0, 0);
-    }
-    if (k0 + GEMM_KC < k_hi) put(buf ^ 1, pre);
-    buf ^= 1;
+  for (int i = 0; i < 2 * RT; ++i) {
+    long n = min(n0 + i % (2 * RO) * 8 + r8, N - 1);
+    if (i >= 2 * RO) n += N;
+    src[i] = w + n * K + c8;
   }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) cred[wv][lg * 4 + r][l15] = acc[r];
+  for (int i = 0; i < XL; ++i)
+    src[2 * RT + i] = x + (long)min(i * 8 + r8, M - 1) * K + c8;
+  u16* mine = buf + wid * S * STAGE;
+  const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)mine;
+  // past the end the last stage is read again, into a buffer that is free
+  auto load = [&](int step, int b) {
+    const int k = min(step, steps - 1) * 64;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const u32 at = lds + (b * STAGE + i * 512) * 2;
+      if (i < 2 * RT) load_lds_nt(src[i] + k, at);
+      else load_lds(src[i] + k, at);
+    }
+  };
+  f32x4 acc[RT][MT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < S; ++s) load(lo + s, s);
+  int b = 0;
+  for (int s = lo; s < hi; ++s) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * LOADS) : "memory");
+    const u16* bw = mine + b * STAGE;
+    const u16* bx = bw + RT * 1024;
+    s16x8 fa[2][RT], fb[2][MT];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int c = ((kk * 4 + lg) ^ (l15 & 7)) * 8;
+#pragma unroll
+      for (int i = 0; i < RT; ++i) fa[kk][i] = ld8(bw + (i * 16 + l15) * 64 + c);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        // an odd group of 8 rows stands in for the one after it
+        const int r = XL >= 2 * j + 2 ? l15 : l15 & 7;
+        fb[kk][j] = ld8(bx + (j * 16 + r) * 64 + c);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    load(s + S, b);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+          acc[i][j] = mma(fa[kk][i], fb[kk][j], acc[i][j]);
+    b = b == S - 1 ? 0 : b + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (wv == 0) {
-    for (int i = lane; i < M * 16; i += 64) {
-      const int m = i / 16, n = i % 16;
-      float v = cred[0][m][n] + cred[1][m][n] + cred[2][m][n] + cred[3][m][n];
+  f32x4* red = (f32x4*)buf;
 #pragma unroll
-      for (int c = 4; c < NW; ++c) v += cred[c][m][n];
-      epilogue<EPI>(outp, m, N, n0 + n, v, ep);
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+      red[((i * MT + j) * 4 + wid) * 64 + lane] = acc[i][j];
+  __syncthreads();
+  auto sum = [&](int t) {
+    const f32x4* p = red + t * 256 + lane;
+    f32x4 v = p[0];
+#pragma unroll
+    for (int k = 1; k < 4; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += p[k * 64][e];
+    return v;
+  };
+  // results 4 lg + 0..3 of a tile, of row l15
+  for (int t = wid; t < RO * MT; t += 4) {
+    const int m = t % MT * 16 + l15, n = n0 + t / MT * 16 + 4 * lg;
+    f32x4 v = sum(t);
+    if (EPI == EPI_SWIGLU) {
+      const f32x4 u = sum(t + RO * MT);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = v[e] / (1.f + __expf(-v[e])) * u[e];
+    }
+    if (m >= M) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (n + e >= N) break;
+      if (EPI == EPI_SWIGLU) ep.act[m * ep.as + n + e] = f2bf(v[e]);
+      else epilogue<EPI>(outp, m, N, n + e, v[e], ep);
     }
   }
+}
+
+template <int EPI, int XL, int RT, int S>
+void launch_skinny(void* out, const void* x, const void* w, int M, int N,
+                   int K, const Epilogue& ep, hipStream_t stream) {
+  constexpr int MT = (XL + 1) / 2;
+  constexpr int stages = 4 * S * (2 * RT + XL), sums = RT * MT * 4;
+  constexpr int lds = (stages > sums ? stages : sums) * 1024;
+  constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : RT;
+  if (lds > 65536)                        // beyond that a kernel has to ask
+    (void)hipFuncSetAttribute((const void*)k_skinny<EPI, XL, RT, S>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  hipLaunchKernelGGL((k_skinny<EPI, XL, RT, S>),
+                     dim3((N + 16 * RO - 1) / (16 * RO)), dim3(256), lds,
+                     stream, out, (const u16*)x, (const u16*)w, M, N, K, ep);
+}
+
+// Few rows of w (under 320 tiles, little more than one a CU): small tiles, so
+// that all CUs load. 4096 rows, 8 of x: 7.8 us against 9.9; 6144: 12.1, 10.6.
+// Many with more than 24 rows of x: wide tiles, so that x is repeated less.
+// 28672 x 4096, 32 rows: 46 us against 50; 64: 55, 66.
+template <int EPI, int XL>
+void by_tiles(void* out, const void* x, const void* w, int M, int N, int K,
+              const Epilogue& ep, hipStream_t stream) {
+  const int rows = EPI == EPI_SWIGLU ? 2 * N : N;
+  if constexpr (XL >= 4)
+    if (rows >= 16384)
+      return launch_skinny<EPI, XL, 4, 2>(out, x, w, M, N, K, ep, stream);
+  if constexpr (EPI != EPI_SWIGLU)
+    if (rows < 5120)
+      return launch_skinny<EPI, XL, 1, (XL < 4 ? 3 : 2)>(out, x, w, M, N, K,
+                                                         ep, stream);
+  launch_skinny<EPI, XL, 2, 2>(out, x, w, M, N, K, ep, stream);
+}
+
+template <int EPI>
+void by_rows(void* out, const void* x, const void* w, int M, int N, int K,
+             const Epilogue& ep, hipStream_t stream) {
+  if (M <= 8) by_tiles<EPI, 1>(out, x, w, M, N, K, ep, stream);
+  else if (M <= 16) by_tiles<EPI, 2>(out, x, w, M, N, K, ep, stream);
+  else if (M <= 24) by_tiles<EPI, 3>(out, x, w, M, N, K, ep, stream);
+  else if (M <= 32) by_tiles<EPI, 4>(out, x, w, M, N, K, ep, stream);
+  else if (M <= 48) by_tiles<EPI, 6>(out, x, w, M, N, K, ep, stream);
+  else by_tiles<EPI, 8>(out, x, w, M, N, K, ep, stream);
 }
 
 }  // namespace
 
-// float32 results: residual != 0 adds to out, otherwise out is
-// softcap(acc * scale, cap) + bias (cap 0: none; bias may be null). With few
-// columns more waves share out K, so that the weight stream fills the chip.
-extern "C" void fei_gemm_m8_f32(void* out, const void* x, const void* w,
-                                const float* bias, int M, int N, int K,
-                                int residual, float scale, float cap,
-                                hipStream_t stream) {
-  dim3 grid(N / GEMM_NT);
-  const Epilogue ep{bias, scale, cap};
-#define M8(EPI, NW)                                                         \
-  hipLaunchKernelGGL((k_gemm_m8<false, EPI, NW>), grid, dim3(NW * 64), 0,   \
-                     stream, out, (const u16*)x, (const u16*)w, M, N, K, ep)
-#define BY_NW(EPI)                                                          \
-  do {                                                                      \
-    if (N <= 4096 && K % 2048 == 0) M8(EPI, 16);                            \
-    else if (N <= 8192) M8(EPI, 8);                                         \
-    else M8(EPI, 4);                                                        \
-  } while (0)
-  if (residual) BY_NW(EPI_RES); else BY_NW(EPI_F32);
-#undef BY_NW
-#undef M8
-}
-
-// All products of a parallel layer's input (see EPI_PARALLEL).
-extern "C" void fei_gemm_m8_parallel_in(void* out, float* router,
-                                        const void* x, const void* w,
-                                        void* act, long as, int M, int n_mix,
-                                        int n_router, int N, int K,
-                                        hipStream_t stream) {
-  const Epilogue ep{nullptr, 1.f,    0.f,       n_mix,
-                    n_router, router, (u16*)act, as};
-  if (N <= 8192)
-    hipLaunchKernelGGL((k_gemm_m8<false, EPI_PARALLEL, 8>),
-                       dim3(N / GEMM_NT), dim3(512), 0, stream, out,
-                       (const u16*)x, (const u16*)w, M, N, K, ep);
-  else
-    hipLaunchKernelGGL((k_gemm_m8<false, EPI_PARALLEL, 4>),
-                       dim3(N / GEMM_NT), dim3(256), 0, stream, out,
-                       (const u16*)x, (const u16*)w, M, N, K, ep);
-}
-
-extern "C" void fei_gemm_m8(void* out, const void* x, const void* w, int M,
-                            int N, int K, int nontemporal,
-                            hipStream_t stream) {
-  dim3 grid(N / GEMM_NT);
-  if (nontemporal)
-    hipLaunchKernelGGL((k_gemm_m8<true, EPI_BF16>), grid, dim3(256), 0,
-                       stream, out, (const u16*)x, (const u16*)w, M, N, K,
-                       Epilogue{});
-  else
-    hipLaunchKernelGGL((k_gemm_m8<false, EPI_BF16>), grid, dim3(256), 0,
-                       stream, out, (const u16*)x, (const u16*)w, M, N, K,
-                       Epilogue{});
+// 1 to 64 rows, K % 64 == 0, rows of x and w 16-byte aligned. See Epilogue for
+// what becomes of the sums and which of the arguments that takes.
+extern "C" void fei_skinny(void* out, const void* x, const void* w, int M,
+                           int N, int K, int epi, const float* bias,
+                           float scale, float cap, int n_mix, int n_router,
+                           float* router, void* act, long as,
+                           hipStream_t stream) {
+  const Epilogue ep{bias, scale, cap, n_mix, n_router, router, (u16*)act, as};
+  switch (epi) {
+#define CASE(E)                                                      \
+  case E: return by_rows<E>(out, x, w, M, N, K, ep, stream)
+    CASE(EPI_BF16);
+    CASE(EPI_F32);
+    CASE(EPI_RES);
+    CASE(EPI_PARALLEL);
+    CASE(EPI_RES_BF16);
+    CASE(EPI_SWIGLU);
+#undef CASE
+    default: return;
+  }
 }

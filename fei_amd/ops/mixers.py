@@ -34,9 +34,6 @@ def declare(lib: ctypes.CDLL) -> None:
     lib.fei_gemv_gain.argtypes = [_vp] * 4 + [_f] + [_i] * 3 + [_vp]
     lib.fei_gemv_parallel_in.argtypes = (
         [_vp] * 5 + [_f] + [_vp, _l] + [_i] * 5 + [_vp])
-    lib.fei_gemm_m8_parallel_in.argtypes = (
-        [_vp] * 5 + [_l] + [_i] * 5 + [_vp])
-    lib.fei_gemm_m8_f32.argtypes = [_vp] * 4 + [_i] * 4 + [_f, _f, _vp]
     lib.fei_latent_decode.argtypes = (
         [_vp, _l, _vp, _l] + [_vp] * 10 + [_i] * 8 +
         [_f, _i, _f, _i, _i, _i, _vp])
@@ -161,10 +158,28 @@ def _gemv_rows(T: int, K: int, t: torch.Tensor) -> bool:
     return T in (1, 2, 4, 8) and K % 8 == 0 and t.dtype == torch.bfloat16
 
 
-def _m8(T: int, K: int, t: torch.Tensor, *cols: int) -> bool:
-    """Rows and sizes that the small matrix-core tile takes."""
-    return (4 <= T <= 8 and K % 1024 == 0 and t.dtype == torch.bfloat16
-            and all(n % 16 == 0 for n in cols))
+# What becomes of a skinny product's sums (csrc/fei_epilogue.h).
+EPI_BF16, EPI_F32, EPI_RES, EPI_PARALLEL, EPI_RES_BF16, EPI_SWIGLU = range(6)
+SKINNY_ROWS = 32     # most rows of the matrix-core tile for few rows
+
+
+def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Rows and sizes that the matrix-core tile for few rows takes: its loads
+    are of 16 bytes, 128 a row. Under 4 rows the vector units are faster; beyond
+    32 the tile's repeated reads of x cost more than the library's."""
+    return (4 <= T <= SKINNY_ROWS and K > 0 and K % 64 == 0
+            and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous()
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def skinny(out, x, w, n: int, epi: int, bias=None, scale: float = 1.0,
+           cap: float = 0.0, n_mix: int = 0, router=None, act=None,
+           stride: int = 0) -> None:
+    """x [T, K] with the rows of ``w``: ``n`` results a row."""
+    T, K = x.shape
+    _lib().fei_skinny(_p(out), _p(x), _p(w), T, n, K, epi, _p(bias), scale,
+                      cap, n_mix, 0 if router is None else router.shape[1],
+                      _p(router), _p(act), stride, _stream())
 
 
 def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,
@@ -173,16 +188,12 @@ def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,
     silu(gate) * up of n2, gate and up being the next ``ff`` rows each, into
     ``act`` (a column range of a wider buffer)."""
     T, K = n1.shape
-    if n1.is_cuda and _m8(T, K, n1, n_mix, 2 * ff):
+    if n1.is_cuda and skinny_ok(T, K, n1, w_in):
         proj = torch.empty(T, n_mix, dtype=n1.dtype, device=n1.device)
-        _lib().fei_gemm_m8(_p(proj), _p(n1), _p(w_in), T, n_mix, K, 0,
-                           _stream())
+        skinny(proj, n1, w_in, n_mix, EPI_BF16)
         if ff:
-            gu = torch.empty(T, 2 * ff, dtype=n1.dtype, device=n1.device)
-            _lib().fei_gemm_m8(_p(gu), _p(n2), _p(w_in[n_mix:]), T, 2 * ff, K,
-                               0, _stream())
-            _lib().fei_swiglu_rows(_p(act), act.stride(0), _p(gu), 2 * ff, T,
-                                   ff, 0, _stream())
+            skinny(None, n2, w_in[n_mix:], ff, EPI_SWIGLU, act=act,
+                   stride=act.stride(0))
         return proj
     if n1.is_cuda and _gemv_rows(T, K, n1):
         proj = torch.empty(T, n_mix, dtype=n1.dtype, device=n1.device)
@@ -214,7 +225,7 @@ def parallel_in(h: GainNormed, w_in: torch.Tensor, n_mix: int, ff: int,
     T, K = x.shape
     n = n_mix + ff + n_router
     gpu = x.is_cuda and h.dtype == torch.bfloat16
-    if h.inside or (gpu and _m8(T, K, w_in, n)):
+    if h.inside or (gpu and skinny_ok(T, K, h.rows, w_in)):
         proj = torch.empty(T, n_mix, dtype=h.dtype, device=x.device)
         router = torch.empty(T, n_router, dtype=torch.float32,
                              device=x.device) if n_router else None
@@ -223,9 +234,8 @@ def parallel_in(h: GainNormed, w_in: torch.Tensor, n_mix: int, ff: int,
                 _p(proj), _p(router), _p(x), _p(w_in), _p(norm.gain), norm.eps,
                 _p(act), act.stride(0), T, n_mix, n_router, n, K, _stream())
         else:
-            _lib().fei_gemm_m8_parallel_in(
-                _p(proj), _p(router), _p(h.rows), _p(w_in), _p(act),
-                act.stride(0), T, n_mix, n_router, n, K, _stream())
+            skinny(proj, h.rows, w_in, n, EPI_PARALLEL, n_mix=n_mix,
+                   router=router, act=act, stride=act.stride(0))
         return proj, router
     rows = h.rows
     proj = torch.nn.functional.linear(rows, w_in[:n_mix])
@@ -271,9 +281,8 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
                     mult: float = 1.0) -> torch.Tensor:
     """x + mult * (a @ w^T), float32; x may be overwritten with it."""
     T, K = a.shape
-    if a.is_cuda and _m8(T, K, a, w.shape[0]):
-        _lib().fei_gemm_m8_f32(_p(x), _p(a), _p(w), None, T, w.shape[0], K, 1,
-                               mult, 0.0, _stream())
+    if a.is_cuda and skinny_ok(T, K, a, w):
+        skinny(x, a, w, w.shape[0], EPI_RES, scale=mult)
         return x
     if a.is_cuda and _gemv_rows(T, K, a):
         _lib().fei_gemv_f32(_p(x), _p(a), _p(w), None, T, w.shape[0], K, 1,
@@ -289,10 +298,9 @@ def linear_f32(a: torch.Tensor, w: torch.Tensor,
                bias: torch.Tensor) -> torch.Tensor:
     """a @ w^T + bias, float32."""
     T, K = a.shape
-    if a.is_cuda and _m8(T, K, a, w.shape[0]):
+    if a.is_cuda and skinny_ok(T, K, a, w):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=a.device)
-        _lib().fei_gemm_m8_f32(_p(out), _p(a), _p(w), _p(bias), T, w.shape[0],
-                               K, 0, 1.0, 0.0, _stream())
+        skinny(out, a, w, w.shape[0], EPI_F32, bias=bias)
         return out
     if a.is_cuda and _gemv_rows(T, K, a):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=a.device)
@@ -309,10 +317,9 @@ def logits_head(y: torch.Tensor, w: torch.Tensor, scale: float,
     if not y.is_cuda:
         return ref.softcap_logits(_mm_f32(y, w, None), scale, cap)
     c = float(cap or 0.0)
-    if _m8(T, K, y, w.shape[0]):
+    if skinny_ok(T, K, y, w):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=y.device)
-        _lib().fei_gemm_m8_f32(_p(out), _p(y), _p(w), None, T, w.shape[0], K,
-                               0, scale, c, _stream())
+        skinny(out, y, w, w.shape[0], EPI_F32, scale=scale, cap=c)
         return out
     if _gemv_rows(T, K, y):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=y.device)

@@ -199,3 +199,51 @@ def test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, splits, lens):
         p = torch.softmax((kk * q64[b].unsqueeze(1)).sum(-1) * D ** -0.5, -1)
         # the result is rounded once: 2^-9
         assert row_err(got[b], (p.unsqueeze(-1) * vv).sum(1)) < 2 ** -8
+
+
+# -- products of few rows on the matrix units ------------------------------------
+
+@pytest.mark.parametrize("M", [4, 8, 9, 17, 25, 32])
+@pytest.mark.parametrize("N,K", [
+    (16, 64),              # one stage, three waves without any
+    (20, 320),             # five stages for four waves, a part of a tile
+    (5120, 192),           # tiles of 32 rows
+    (8200, 64),            # SwiGLU: tiles of 64 rows, the last in part
+    (2048, 4160),
+])
+def test_skinny_geometries(lib, M, N, K):
+    """Each kind of result, against float64: float32 sums, rounded to
+    bfloat16 once where the result is (2^-9; 2^-8 allowed)."""
+    from fei_amd.ops import mixers as mx
+    x, w = randbf(M, K, seed=M), randbf(2 * N, K, seed=N, scale=K ** -0.5)
+    assert mx.skinny_ok(M, K, x, w)
+    y = x.double() @ w.double().T
+    a, b = y[:, :N], y[:, N:]
+    w1 = w[:N].contiguous()
+    out = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    mx.skinny(out, x, w1, N, mx.EPI_BF16)
+    assert row_err(out, a) < 2 ** -8
+    res = randbf(M, N, seed=1)
+    want = res.double() + a
+    mx.skinny(res, x, w1, N, mx.EPI_RES_BF16)
+    assert row_err(res, want) < 2 ** -8
+    wide = torch.zeros(M, N + 24, device=DEV, dtype=torch.bfloat16)
+    mx.skinny(None, x, w, N, mx.EPI_SWIGLU, act=wide[:, 8:], stride=N + 24)
+    assert row_err(wide[:, 8:8 + N], torch.nn.functional.silu(a) * b) < 2 ** -8
+    assert not wide[:, :8].any() and not wide[:, 8 + N:].any()
+    bias = torch.randn(N, device=DEV)
+    f = torch.empty(M, N, device=DEV)
+    mx.skinny(f, x, w1, N, mx.EPI_F32, bias=bias, scale=0.5, cap=3.0)
+    assert row_err(f, 3 * torch.tanh(a * 0.5 / 3) + bias.double()) < 1e-5
+    mx.skinny(f.copy_(want), x, w1, N, mx.EPI_RES, scale=0.25)
+    assert row_err(f, want.float().double() + 0.25 * a) < 1e-5
+    n_mix, n_r = N - 12, 4
+    proj = torch.empty(M, n_mix, device=DEV, dtype=torch.bfloat16)
+    router = torch.empty(M, n_r, device=DEV)
+    act = torch.zeros(M, 16, device=DEV, dtype=torch.bfloat16)
+    mx.skinny(proj, x, w1, N, mx.EPI_PARALLEL, n_mix=n_mix, router=router,
+              act=act[:, 4:], stride=16)
+    assert row_err(proj, a[:, :n_mix]) < 2 ** -8
+    assert row_err(router, a[:, n_mix:n_mix + n_r]) < 1e-5
+    assert (act[:, 4:12].double() - a[:, -8:].clamp(min=0) ** 2).abs().max() \
+        < 2 ** -8 * (a[:, -8:] ** 2).max()
