@@ -382,23 +382,22 @@ class LlamaModel:
         n_layers = len(self.layers)
         x = ops.rmsnorm(h, self.layers[0].norm_attn, s.norm_eps)
         for li, lw in enumerate(self.layers):
-            qkv = F.linear(x, lw.wqkv)                    # [B,S,W]
+            qkv = ops.linear_decode(x, lw.wqkv)           # [B,S,W]
             qkv2 = qkv.view(B * S, -1)
             q, k, v = self._qkv_views(qkv2, B, S)
             ops.rope_kv_prefill(q, k, v, k_caches[li], v_caches[li], pos0, self.rope)
             att = ops.attn_prefill(q, k_caches[li], v_caches[li], pos0, scale=scale)
-            o = F.linear(att.reshape(B, S, -1), lw.wo)
+            o = ops.linear_decode(att.reshape(B, S, -1), lw.wo)
             all_reduce_sum(o, self.tp)
             x, h = ops.fused_add_rmsnorm(o, h, lw.norm_mlp, s.norm_eps)
-            gu = F.linear(x, lw.wgu)
-            act = ops.swiglu(gu)
-            d = F.linear(act, lw.wdown)
+            act = ops.gemv_swiglu(x, lw.wgu)
+            d = ops.linear_decode(act, lw.wdown)
             all_reduce_sum(d, self.tp)
             next_norm = (self.layers[li + 1].norm_attn if li + 1 < n_layers
                          else self.norm_f)
             x, h = ops.fused_add_rmsnorm(d, h, next_norm, s.norm_eps)
         last = x if all_positions else x[:, -1, :]
-        logits = F.linear(last, self.lm_head)
+        logits = ops.linear_decode(last, self.lm_head)
         logits = all_gather_cat(logits, dim=-1, ctx=self.tp)
         return logits
 

@@ -247,3 +247,32 @@ def test_skinny_geometries(lib, M, N, K):
     assert row_err(router, a[:, n_mix:n_mix + n_r]) < 1e-5
     assert (act[:, 4:12].double() - a[:, -8:].clamp(min=0) ** 2).abs().max() \
         < 2 ** -8 * (a[:, -8:] ** 2).max()
+
+
+# -- RoPE of a prompt --------------------------------------------------------------
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,D,pad", [
+    (1, 1, 1, 1, 64, 0), (2, 33, 5, 1, 128, 0), (1, 7, 4, 2, 24, 0),
+    (1, 9, 3, 3, 64, 3),         # rows that start at no multiple of 16 bytes
+])
+def test_rope_prefill_geometries(lib, B, S, Hq, Hkv, D, pad):
+    from fei_amd.ops import reference as ref
+    W, T = (Hq + 2 * Hkv) * D + pad, S + 9
+    buf = randbf(B * S * W + 8, seed=S)
+    parts = [buf.as_strided((B, S, H, D), (S * W, W, D, 1), o * D + (pad and 1))
+             for H, o in ((Hq, 0), (Hkv, Hq), (Hkv, Hq + Hkv))]
+    q, k, v = parts
+    q0 = q.clone()
+    pos0 = torch.arange(B, dtype=torch.int32, device=DEV) * 4 + 3
+    kc, vc = (torch.zeros(B, Hkv, T, D, device=DEV, dtype=torch.bfloat16)
+              for _ in range(2))
+    lib.rope_kv_prefill(q, k, v, kc, vc, pos0, ref.rope_table(T, D, device=DEV))
+    for b in range(B):
+        p = torch.arange(S, device=DEV) + pos0[b]
+        # angles are float32, results rounded once
+        assert row_err(q[b], rope64(q0[b], p)) < 2 ** -8
+        assert row_err(kc[b, :, p].transpose(0, 1), rope64(k[b], p)) < 2 ** -8
+        assert torch.equal(vc[b, :, p].transpose(0, 1), v[b])
+    rest = torch.ones(T, dtype=torch.bool, device=DEV)
+    rest[p] = False
+    assert not kc[-1][:, rest].any() and not vc[-1][:, rest].any()
