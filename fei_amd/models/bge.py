@@ -94,20 +94,20 @@ class BgeEncoder:
                   else torch.full((B,), S, dtype=torch.int32, device=self.device))
         pos0 = torch.zeros(B, dtype=torch.int32, device=self.device)
         for lw in self.layers:
-            qkv = (F.linear(h, lw["wqkv"]) + lw["bqkv"]).view(B, S, 3, H, D)
-            q = qkv[:, :, 0].contiguous()
-            k = qkv[:, :, 1].transpose(1, 2).contiguous()   # [B,H,S,D] "cache"
-            v = qkv[:, :, 2].transpose(1, 2).contiguous()
-            att = ops.attn_prefill(q.to(self.dtype), k.to(self.dtype),
-                                   v.to(self.dtype), pos0, scale=scale,
-                                   causal=False, kv_len=kv_len)
-            o = F.linear(att.reshape(B, S, H * D), lw["wo"]) + lw["bo"]
-            h = ops.layernorm(o.to(self.dtype), lw["ln1_w"], lw["ln1_b"],
-                              self.eps, residual=h)
-            inner = ops.gelu((F.linear(h, lw["wi"]) + lw["bi"]).to(self.dtype))
-            o2 = F.linear(inner, lw["wo2"]) + lw["bo2"]
-            h = ops.layernorm(o2.to(self.dtype), lw["ln2_w"], lw["ln2_b"],
-                              self.eps, residual=h)
+            qkv = ops.linear_bias(h, lw["wqkv"], lw["bqkv"]) \
+                .view(B, S, 3, H, D)
+            # the attention reads queries, keys and values where they are
+            q, k, v = qkv.unbind(2)
+            att = ops.attn_prefill(q, k.transpose(1, 2), v.transpose(1, 2),
+                                   pos0, scale=scale, causal=False,
+                                   kv_len=kv_len)
+            o = ops.linear_bias(att.reshape(B, S, H * D), lw["wo"], lw["bo"])
+            h = ops.layernorm(o, lw["ln1_w"], lw["ln1_b"], self.eps,
+                              residual=h)
+            inner = ops.linear_bias(h, lw["wi"], lw["bi"], act_gelu=True)
+            o2 = ops.linear_bias(inner, lw["wo2"], lw["bo2"])
+            h = ops.layernorm(o2, lw["ln2_w"], lw["ln2_b"], self.eps,
+                              residual=h)
         hf = h.float()
         if lengths is not None:
             mask = (torch.arange(S, device=self.device).unsqueeze(0)

@@ -65,12 +65,12 @@ def _try_load() -> None:
     lib.fei_advance.argtypes = [_vp, _vp, _i, _i, _vp]
     lib.fei_attn_prefill.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp,
                                      _i, _i, _i, _i, _i, _i, _f, _i, _l, _i,
-                                     _vp, _vp, _vp]
+                                     _vp, _vp, _l, _l, _l, _vp]
     lib.fei_mfma_probe.argtypes = [_vp, _vp, _vp, _vp]
     lib.fei_gemv.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _i,
                              _vp, _vp]
     lib.fei_skinny.argtypes = ([_vp] * 3 + [_i] * 4 + [_vp, _f, _f, _i, _i] +
-                               [_vp, _vp, _l, _vp])
+                               [_vp, _vp, _l, _vp, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -313,6 +313,7 @@ def attn_prefill(q, k_cache, v_cache, pos0, scale: Optional[float] = None,
     assert out.is_contiguous()
     if not q.numel():
         return out
+    k_cache, v_cache = _cache_rows(k_cache, v_cache)
     splits = _prefill_splits(B * Hkv, S * (Hq // Hkv), k_cache.shape[2])
     po = pml = None
     if splits > 1:
@@ -322,8 +323,21 @@ def attn_prefill(q, k_cache, v_cache, pos0, scale: Optional[float] = None,
     lib.fei_attn_prefill(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(out),
                          _ptr(pos0), _ptr(kv_len), B, S, Hq, Hkv, D,
                          k_cache.shape[2], scale, 1 if causal else 0,
-                         q.stride(1), splits, po, pml, _stream())
+                         q.stride(1), splits, po, pml, k_cache.stride(0),
+                         k_cache.stride(1), k_cache.stride(2), _stream())
     return out
+
+
+def _cache_rows(k: torch.Tensor, v: torch.Tensor):
+    """Caches as the prompt attention's loads of 16 bytes take them: contiguous
+    rows, all 16-byte aligned, both laid out alike; copies where they are not
+    (what it reads is not written to)."""
+    def fits(t):
+        return (t.stride(3) == 1 and t.data_ptr() % 16 == 0
+                and all(s % 8 == 0 for s in t.stride()[:3]))
+    if k.stride() == v.stride() and fits(k) and fits(v):
+        return k, v
+    return (t.clone(memory_format=torch.contiguous_format) for t in (k, v))
 
 
 def _prefill_splits(heads: int, rows: int, max_seq: int) -> int:
@@ -748,6 +762,22 @@ def layernorm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor,
                           _ptr(bias), rows, x2.shape[-1], eps,
                           1 if residual is not None else 0, _stream())
     return out
+
+
+def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
+                act_gelu: bool = False) -> torch.Tensor:
+    """x @ w^T + bias, and its GELU if asked for (encoder blocks)."""
+    M = x.numel() // max(x.shape[-1], 1)
+    if (x.is_cuda and x.is_contiguous() and bias.dtype == torch.bfloat16
+            and _mixers.skinny_ok(M, x.shape[-1], x, w)):
+        out = torch.empty(*x.shape[:-1], w.shape[0], dtype=x.dtype,
+                          device=x.device)
+        _mixers.skinny(out, x.view(M, -1), w, w.shape[0],
+                       _mixers.EPI_GELU if act_gelu else _mixers.EPI_BF16,
+                       bias16=bias)
+        return out
+    y = torch.nn.functional.linear(x, w, bias)
+    return gelu(y) if act_gelu else y
 
 
 def gelu(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

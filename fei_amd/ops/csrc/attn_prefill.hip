@@ -68,6 +68,7 @@ struct Prefill {
   int S, G, Hkv, heads, tiles, max_seq, causal, splits;
   float scale;
   long q_ts;
+  long kv_b, kv_h, kv_t;               // strides of the caches
 };
 
 // Keys that the rows up to r_hi of batch row b see.
@@ -141,8 +142,8 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
     }
   }
 
-  const u16* kb = a.kc + (long)head * a.max_seq * D;
-  const u16* vb = a.vc + (long)head * a.max_seq * D;
+  const u16* kb = a.kc + b * a.kv_b + hkv * a.kv_h;
+  const u16* vb = a.vc + b * a.kv_b + hkv * a.kv_h;
   const u32 lds =
       (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)&buf[0][0][0];
   auto load = [&](int t, int p) {
@@ -150,7 +151,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
     for (int i = 0; i < LOADS; ++i) {
       const int at = wid * LOADS + i;
       const int row = at * RPI + lane / LPR, place = lane % LPR;
-      const int off = min(t * KEYS + row, n - 1) * D;
+      const long off = min(t * KEYS + row, n - 1) * a.kv_t;
       const int ck = place ^ (row & 7);
       const int cv = (((place >> 1) ^ (row & (D / 16 - 1))) << 1) | (place & 1);
       load_lds(kb + off + ck * 8, lds + (p * 2 * KEYS * D + at * 512) * 2);
@@ -335,19 +336,20 @@ void launch_prefill(const Prefill& a, hipStream_t stream) {
 
 extern "C" {
 
-// po [B * Hkv, S * G, splits, D] and pml [.., splits, 2] float32, where
+// Strides of both caches by batch row, head and position; rows of D values,
+// 16-byte aligned. po [B * Hkv, S * G, splits, D] and pml [.., splits, 2] float32, where
 // splits > 1.
 void fei_attn_prefill(const void* q, const void* k_cache, const void* v_cache,
                       void* out, const int* pos0, const int* kv_len, int B,
                       int S, int Hq, int Hkv, int D, int max_seq, float scale,
                       int causal, long q_ts, int splits, float* po, float* pml,
-                      hipStream_t stream) {
+                      long kv_b, long kv_h, long kv_t, hipStream_t stream) {
   const int G = Hq / Hkv;
   const Prefill a{(const u16*)q, (const u16*)k_cache, (const u16*)v_cache,
                   (u16*)out,     po,     pml,  pos0,  kv_len,
                   S,             G,      Hkv,  B * Hkv,
                   (S * G + ROWS - 1) / ROWS,   max_seq, causal, splits,
-                  scale,         q_ts};
+                  scale,         q_ts,   kv_b, kv_h,  kv_t};
   if (D == 128) launch_prefill<128>(a, stream);
   else if (D == 64) launch_prefill<64>(a, stream);
 }

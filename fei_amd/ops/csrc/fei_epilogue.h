@@ -9,6 +9,7 @@ enum {
   EPI_PARALLEL = 3,
   EPI_RES_BF16 = 4,   // added to bfloat16
   EPI_SWIGLU = 5,     // of a gate and an up product, to act
+  EPI_GELU = 6,       // bfloat16
 };
 
 struct Epilogue {
@@ -21,11 +22,27 @@ struct Epilogue {
   float* router;
   u16* act;
   long as;
+  const u16* bias16;   // EPI_BF16, EPI_GELU: per column, may be null
 };
 
 __device__ __forceinline__ float softcap(float v, float scale, float cap) {
   v *= scale;
   return cap > 0.f ? cap * tanhf(v / cap) : v;
+}
+
+// x Phi(x), erf by its rational approximation times exp(-x^2 / 2) (Abramowitz and
+// Stegun, Handbook of Mathematical Functions, 7.1.26; 1.5e-7 at most). Taken from
+// the side of the tail, so that nothing cancels there.
+__device__ __forceinline__ float gelu_erf(float x) {
+  const float z = fabsf(x) * 0.70710678118654752f;
+  const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, z, 1.f));
+  float p = fmaf(t, 1.061405429f, -1.453152027f);
+  p = fmaf(t, p, 1.421413741f);
+  p = fmaf(t, p, -0.284496736f);
+  p = fmaf(t, p, 0.254829592f);
+  // half of erfc(z)
+  const float q = 0.5f * t * p * __expf(-z * z);
+  return x * (x < 0.f ? q : 1.f - q);
 }
 
 __device__ __forceinline__ float relu2(float v) {
@@ -38,8 +55,9 @@ template <int EPI>
 __device__ __forceinline__ void epilogue(void* out, int row, int N, int col,
                                          float v, const Epilogue& ep) {
   const long at = (long)row * N + col;
-  if (EPI == EPI_BF16) {
-    ((u16*)out)[at] = f2bf(v);
+  if (EPI == EPI_BF16 || EPI == EPI_GELU) {
+    if (ep.bias16) v += bf2f(ep.bias16[col]);
+    ((u16*)out)[at] = f2bf(EPI == EPI_GELU ? gelu_erf(v) : v);
   } else if (EPI == EPI_RES_BF16) {
     ((u16*)out)[at] = f2bf(bf2f(((u16*)out)[at]) + v);
   } else if (EPI == EPI_RES) {

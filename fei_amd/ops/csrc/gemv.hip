@@ -550,8 +550,9 @@ extern "C" void fei_skinny(void* out, const void* x, const void* w, int M,
                            int N, int K, int epi, const float* bias,
                            float scale, float cap, int n_mix, int n_router,
                            float* router, void* act, long as,
-                           hipStream_t stream) {
-  const Epilogue ep{bias, scale, cap, n_mix, n_router, router, (u16*)act, as};
+                           const void* bias16, hipStream_t stream) {
+  const Epilogue ep{bias,   scale,     cap, n_mix,              n_router,
+                    router, (u16*)act, as,  (const u16*)bias16};
   switch (epi) {
 #define CASE(E)                                                      \
   case E: return by_rows<E>(out, x, w, M, N, K, ep, stream)
@@ -561,6 +562,7 @@ extern "C" void fei_skinny(void* out, const void* x, const void* w, int M,
     CASE(EPI_PARALLEL);
     CASE(EPI_RES_BF16);
     CASE(EPI_SWIGLU);
+    CASE(EPI_GELU);
 #undef CASE
     default: return;
   }

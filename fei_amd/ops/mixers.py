@@ -159,7 +159,8 @@ def _gemv_rows(T: int, K: int, t: torch.Tensor) -> bool:
 
 
 # What becomes of a skinny product's sums (csrc/fei_epilogue.h).
-EPI_BF16, EPI_F32, EPI_RES, EPI_PARALLEL, EPI_RES_BF16, EPI_SWIGLU = range(6)
+(EPI_BF16, EPI_F32, EPI_RES, EPI_PARALLEL, EPI_RES_BF16, EPI_SWIGLU,
+ EPI_GELU) = range(7)
 SKINNY_ROWS = 32     # most rows of the matrix-core tile for few rows
 
 
@@ -174,12 +175,12 @@ def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def skinny(out, x, w, n: int, epi: int, bias=None, scale: float = 1.0,
            cap: float = 0.0, n_mix: int = 0, router=None, act=None,
-           stride: int = 0) -> None:
+           stride: int = 0, bias16=None) -> None:
     """x [T, K] with the rows of ``w``: ``n`` results a row."""
     T, K = x.shape
     _lib().fei_skinny(_p(out), _p(x), _p(w), T, n, K, epi, _p(bias), scale,
                       cap, n_mix, 0 if router is None else router.shape[1],
-                      _p(router), _p(act), stride, _stream())
+                      _p(router), _p(act), stride, _p(bias16), _stream())
 
 
 def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,

@@ -223,6 +223,11 @@ def test_skinny_geometries(lib, M, N, K):
     out = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
     mx.skinny(out, x, w1, N, mx.EPI_BF16)
     assert row_err(out, a) < 2 ** -8
+    b16 = randbf(N, seed=2)
+    mx.skinny(out, x, w1, N, mx.EPI_BF16, bias16=b16)
+    assert row_err(out, a + b16.double()) < 2 ** -8
+    mx.skinny(out, x, w1, N, mx.EPI_GELU, bias16=b16)
+    assert row_err(out, torch.nn.functional.gelu(a + b16.double())) < 2 ** -8
     res = randbf(M, N, seed=1)
     want = res.double() + a
     mx.skinny(res, x, w1, N, mx.EPI_RES_BF16)
@@ -276,3 +281,52 @@ def test_rope_prefill_geometries(lib, B, S, Hq, Hkv, D, pad):
     rest = torch.ones(T, dtype=torch.bool, device=DEV)
     rest[p] = False
     assert not kc[-1][:, rest].any() and not vc[-1][:, rest].any()
+
+
+# -- encoder ---------------------------------------------------------------------
+
+@pytest.mark.parametrize("cols", [8, 512, 520, 768, 1032, 2048, 2056])
+@pytest.mark.parametrize("rows", [1, 5])
+def test_layernorm_widths(lib, rows, cols):
+    """Float32 statistics; the result is rounded once (2^-9)."""
+    x, r = randbf(rows, cols, seed=1) + 3, randbf(rows, cols, seed=2)
+    w, b = randbf(cols, seed=3), randbf(cols, seed=4)
+    for res in (None, r):
+        y = x.double() + (0 if res is None else r.double())
+        want = torch.nn.functional.layer_norm(y, (cols,), w.double(),
+                                              b.double(), 1e-6)
+        assert row_err(lib.layernorm(x, w, b, 1e-6, residual=res), want) < 2 ** -8
+
+
+def test_gelu_all_bfloat16(lib):
+    """Every bfloat16 but -inf."""
+    x = torch.arange(1 << 16, device=DEV, dtype=torch.int32).to(torch.int16) \
+        .view(torch.bfloat16)
+    got, want = lib.gelu(x), torch.nn.functional.gelu(x.double())
+    ok = x.isfinite()
+    err = (got.double() - want).abs()[ok]
+    x64, w64 = x.double()[ok], want[ok]
+    # rounded once: 2^-9 of the value, or half the smallest bfloat16, 2^-133;
+    # 1.5e-7 of |x| from the approximation
+    most = 2 ** -8 * w64.abs() + 2e-7 * x64.abs().clamp(max=12) + 2.0 ** -133
+    assert (err <= most).all()
+    assert got[x == float("inf")].eq(float("inf")).all()
+    assert got[x.isnan()].isnan().all()
+
+
+def test_encoder_attention_reads_views(lib):
+    """Queries, keys and values as they lie in one projection, aligned or
+    not, give what contiguous copies give."""
+    B, S, H, D = 2, 70, 3, 64
+    lens = torch.tensor([70, 9], dtype=torch.int32, device=DEV)
+    zero = torch.zeros(B, dtype=torch.int32, device=DEV)
+    buf = randbf(B * S * 3 * H * D + 8, seed=4)
+    for shift in (0, 1):
+        qkv = buf[shift:shift + B * S * 3 * H * D].view(B, S, 3, H, D)
+        q, k, v = qkv.unbind(2)
+        got = lib.attn_prefill(q, k.transpose(1, 2), v.transpose(1, 2), zero,
+                               causal=False, kv_len=lens)
+        want = lib.attn_prefill(q.contiguous(), k.transpose(1, 2).contiguous(),
+                                v.transpose(1, 2).contiguous(), zero,
+                                causal=False, kv_len=lens)
+        assert torch.equal(got, want)
