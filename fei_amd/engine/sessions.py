@@ -290,40 +290,32 @@ class PagedSessionManager:
         scale = 1.0 / math.sqrt(m.D)
         eps, n_layers = s.norm_eps, len(m.layers)
         gpu = m.device.type == "cuda"
-        fused = m.fused_rows(B)
         if not gpu:
             pos_l = pos.long()
             blk = table.gather(1, (pos_l // BS).unsqueeze(1)) \
                 .squeeze(1).long()
             off = pos_l % BS
-        x = None if fused else ops.rmsnorm(h, m.layers[0].norm_attn, eps)
-        for li, lw in enumerate(m.layers):
-            qkv = ops.gemv_norm(h, lw.norm_attn, lw.wqkv, eps) if fused \
-                else ops.linear_decode(x, lw.wqkv)
+
+        def attend(li, qkv):
             q, k, v = m._qkv_views(qkv, B)
             kp, vp = self.pool.k[li], self.pool.v[li]
-            if gpu:
-                # RoPE and the paged append are made in the kernel
-                att = ops.attn_decode_paged(q, kp, vp, table, pos,
-                                            splits=self._splits(B),
-                                            scale=scale,
-                                            workspace=self._workspace(B),
-                                            k=k, v=v, table=m.rope)
-            else:
-                q_r = ref.apply_rope(q, pos_l, m.rope).contiguous()
-                k_r = ref.apply_rope(k, pos_l, m.rope)
-                kp[blk, :, off, :] = k_r
-                vp[blk, :, off, :] = v
-                att = ops.attn_decode_paged(q_r, kp, vp, table, pos,
-                                            splits=self._splits(B),
-                                            scale=scale,
-                                            workspace=self._workspace(B))
-            att = att.reshape(B, -1)
-            if fused:
-                ops.gemv_res(att, lw.wo, h)
-                act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, eps)
-                ops.gemv_res(act, lw.wdown, h)
-                continue
+            args = dict(splits=self._splits(B), scale=scale,
+                        workspace=self._workspace(B))
+            if gpu:      # RoPE and the paged append are made in the kernel
+                return ops.attn_decode_paged(q, kp, vp, table, pos, k=k, v=v,
+                                             table=m.rope, **args)
+            kp[blk, :, off, :] = ref.apply_rope(k, pos_l, m.rope)
+            vp[blk, :, off, :] = v
+            return ops.attn_decode_paged(
+                ref.apply_rope(q, pos_l, m.rope).contiguous(), kp, vp, table,
+                pos, **args)
+
+        if m.fused_rows(B):
+            sums = m.fused_layers(h, attend)
+            return ops.gemv_norm(h, m.norm_f, m.lm_head, eps, sums=sums)
+        x = ops.rmsnorm(h, m.layers[0].norm_attn, eps)
+        for li, lw in enumerate(m.layers):
+            att = attend(li, ops.linear_decode(x, lw.wqkv)).reshape(B, -1)
             o = ops.linear_decode(att, lw.wo)
             x, h = ops.fused_add_rmsnorm(o, h, lw.norm_mlp, eps)
             act = ops.gemv_swiglu(x, lw.wgu)
@@ -331,8 +323,6 @@ class PagedSessionManager:
             next_norm = (m.layers[li + 1].norm_attn if li + 1 < n_layers
                          else m.norm_f)
             x, h = ops.fused_add_rmsnorm(d, h, next_norm, eps)
-        if fused:
-            return ops.gemv_norm(h, m.norm_f, m.lm_head, eps)
         return ops.linear_decode(x, m.lm_head)
 
 

@@ -252,6 +252,19 @@ class LlamaModel:
             logits = all_gather_cat(logits, dim=-1, ctx=self.tp)
         return logits
 
+    def fused_layers(self, h: torch.Tensor, attend) -> Optional[torch.Tensor]:
+        """All layers over the residual ``h`` [rows, C], in place; fused_rows
+        has to allow the rows. ``attend(layer, qkv)`` gives the attention's
+        output. Returns what a norm's product takes as ``sums``."""
+        eps, sums = self.spec.norm_eps, None
+        for li, lw in enumerate(self.layers):
+            qkv = ops.gemv_norm(h, lw.norm_attn, lw.wqkv, eps, sums=sums)
+            att = attend(li, qkv)
+            sums = ops.add_product(att.reshape(h.shape[0], -1), lw.wo, h)
+            act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, eps, sums=sums)
+            sums = ops.add_product(act, lw.wdown, h)
+        return sums
+
     def fused_rows(self, B: int) -> bool:
         """Whether a step of B rows runs the chain whose products hold the
         residual."""
@@ -304,6 +317,7 @@ class LlamaModel:
         # norm's sumsq so the norm prologues collapse to one scalar read.
         # The layer-0 attention norm has no producing epilogue (embedding)
         # and keeps the full prologue.
+        sums = None
         ssq = (self._ssq_slots(B, h.device)
                if (self.norm_precomp and fp8 is None and h.is_cuda) else None)
         if ssq is not None:
@@ -320,7 +334,7 @@ class LlamaModel:
                                         s.norm_eps)
             else:
                 qkv = ops.gemv_norm(
-                    h, lw.norm_attn, lw.wqkv, s.norm_eps,
+                    h, lw.norm_attn, lw.wqkv, s.norm_eps, sums=sums,
                     ssq=ssq[2 * li - 1] if (ssq is not None and li > 0) else None)
             if pf:
                 # warm L2/L3 with this layer's gate/up weights while the
@@ -346,14 +360,16 @@ class LlamaModel:
                 act = ops.gemv_swiglu_norm_fp8(h, lw.norm_mlp, *q8["wgu"],
                                                s.norm_eps)
                 ops.gemv_res_fp8(act, *q8["wdown"], h)
+            elif ssq is None:
+                sums = ops.add_product(att.reshape(B, -1), lw.wo, h)
+                act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, s.norm_eps,
+                                           sums=sums)
+                sums = ops.add_product(act, lw.wdown, h)
             else:
-                ops.gemv_res(att.reshape(B, -1), lw.wo, h,
-                             ssq_out=ssq[2 * li] if ssq is not None else None)
-                act = ops.gemv_swiglu_norm(
-                    h, lw.norm_mlp, lw.wgu, s.norm_eps,
-                    ssq=ssq[2 * li] if ssq is not None else None)
-                ops.gemv_res(act, lw.wdown, h,
-                             ssq_out=ssq[2 * li + 1] if ssq is not None else None)
+                ops.gemv_res(att.reshape(B, -1), lw.wo, h, ssq_out=ssq[2 * li])
+                act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, s.norm_eps,
+                                           ssq=ssq[2 * li])
+                ops.gemv_res(act, lw.wdown, h, ssq_out=ssq[2 * li + 1])
         if pf:
             # rejoin the prefetch stream so graph capture sees all work
             # ordered (pure cache warming: no data dependency otherwise)
@@ -362,7 +378,8 @@ class LlamaModel:
             return ops.gemv_norm_fp8(h, self.norm_f, *self.fp8_lm_head,
                                      s.norm_eps)
         return ops.gemv_norm(h, self.norm_f, self.lm_head, s.norm_eps,
-                             ssq=ssq[-1] if ssq is not None else None)
+                             ssq=ssq[-1] if ssq is not None else None,
+                             sums=sums)
 
     def forward_prefill(
         self,
@@ -380,13 +397,25 @@ class LlamaModel:
         h = F.embedding(tokens.long(), self.emb)          # [B,S,C] residual
         scale = 1.0 / math.sqrt(self.D)
         n_layers = len(self.layers)
+
+        def attend(li, qkv):
+            q, k, v = self._qkv_views(qkv.view(B * S, -1), B, S)
+            ops.rope_kv_prefill(q, k, v, k_caches[li], v_caches[li], pos0,
+                                self.rope)
+            return ops.attn_prefill(q, k_caches[li], v_caches[li], pos0,
+                                    scale=scale)
+
+        if self.fused_rows(B * S):
+            sums = self.fused_layers(h.view(B * S, -1), attend)
+            if not all_positions and S > 1:
+                h, sums = h[:, -1, :], None
+            elif not all_positions:
+                h = h[:, -1, :]
+            return ops.gemv_norm(h, self.norm_f, self.lm_head, s.norm_eps,
+                                 sums=sums)
         x = ops.rmsnorm(h, self.layers[0].norm_attn, s.norm_eps)
         for li, lw in enumerate(self.layers):
-            qkv = ops.linear_decode(x, lw.wqkv)           # [B,S,W]
-            qkv2 = qkv.view(B * S, -1)
-            q, k, v = self._qkv_views(qkv2, B, S)
-            ops.rope_kv_prefill(q, k, v, k_caches[li], v_caches[li], pos0, self.rope)
-            att = ops.attn_prefill(q, k_caches[li], v_caches[li], pos0, scale=scale)
+            att = attend(li, ops.linear_decode(x, lw.wqkv))     # [B,S,W]
             o = ops.linear_decode(att.reshape(B, S, -1), lw.wo)
             all_reduce_sum(o, self.tp)
             x, h = ops.fused_add_rmsnorm(o, h, lw.norm_mlp, s.norm_eps)

@@ -70,7 +70,7 @@ def _try_load() -> None:
     lib.fei_gemv.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _i,
                              _vp, _vp]
     lib.fei_skinny.argtypes = ([_vp] * 3 + [_i] * 4 + [_vp, _f, _f, _i, _i] +
-                               [_vp, _vp, _l, _vp, _vp])
+                               [_vp, _vp, _l] + [_vp] * 3 + [_i, _f, _vp, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -557,9 +557,12 @@ def _gemv_ok(M: int, K: int) -> bool:
     return M in _GEMV_ROWS and K % 8 == 0
 
 
-def _norm_ok(M: int, K: int) -> bool:
-    """Whether the normed rows fit the GEMV's LDS."""
-    return _gemv_ok(M, K) and M * K * 2 <= 128 * 1024
+def _norm_inside(how: str, M: int, K: int, sums) -> bool:
+    """Whether a product takes rows under a norm: the GEMV keeps them in LDS;
+    the tile for few rows needs their sums of squares, and keeps the gains."""
+    if how == "skinny":
+        return sums is not None and K <= 16384
+    return M * K * 2 <= 128 * 1024
 
 
 def _product(x: torch.Tensor, w: torch.Tensor, rows_out: int) -> Optional[str]:
@@ -646,23 +649,45 @@ def gemv_res(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
     return res
 
 
+def add_product(x: torch.Tensor, w: torch.Tensor,
+                res: torch.Tensor) -> Optional[torch.Tensor]:
+    """gemv_res, for a chain: returns the sums of squares of the new rows by
+    tiles of columns, for the ``sums`` of the products that read them under a
+    norm, or None where those do not need them."""
+    M = x.numel() // x.shape[-1]
+    N, K = w.shape
+    if _product(x, w, N) != "skinny":
+        gemv_res(x, w, res)
+        return None
+    sums = torch.empty(M, -(-N // 16), dtype=torch.float32, device=x.device)
+    _mixers.skinny(res, x.contiguous().view(M, K), w, N, _mixers.EPI_RES_BF16,
+                   sums_out=sums)
+    return sums
+
+
 def gemv_norm(res: torch.Tensor, wnorm: torch.Tensor, w: torch.Tensor,
               eps: float = 1e-5,
               out: Optional[torch.Tensor] = None,
-              ssq: Optional[torch.Tensor] = None) -> torch.Tensor:
+              ssq: Optional[torch.Tensor] = None,
+              sums: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out = rmsnorm(res)*wnorm @ w^T, the norm inside the product.
 
     ``ssq`` [M] f32: the sums of squares of res rows, if the caller has them
-    (from a prior gemv_res ``ssq_out``)."""
+    (from a prior gemv_res ``ssq_out``). ``sums``: what add_product returned
+    for these rows."""
     M = res.numel() // res.shape[-1]
     N, K = w.shape
     how = _product(res, w, N)
     if how is None:
         return torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w)
-    if how == "skinny" or not _norm_ok(M, K):
+    if not _norm_inside(how, M, K, sums):
         return linear_decode(rmsnorm(res, wnorm, eps), w, out)
     if out is None:
         out = torch.empty(*res.shape[:-1], N, dtype=res.dtype, device=res.device)
+    if how == "skinny":
+        _mixers.skinny(out, res.contiguous().view(M, K), w, N,
+                       _mixers.EPI_BF16, norm=(wnorm, sums, eps))
+        return out
     _launch_gemv(out, res.contiguous().view(M, K), wnorm, w, None, N, eps,
                  _BF16, ssq)
     return out
@@ -671,19 +696,25 @@ def gemv_norm(res: torch.Tensor, wnorm: torch.Tensor, w: torch.Tensor,
 def gemv_swiglu_norm(res: torch.Tensor, wnorm: torch.Tensor,
                      wgu: torch.Tensor, eps: float = 1e-5,
                      out: Optional[torch.Tensor] = None,
-                     ssq: Optional[torch.Tensor] = None) -> torch.Tensor:
+                     ssq: Optional[torch.Tensor] = None,
+                     sums: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out = silu(g)*u where [g;u] = rmsnorm(res)*wnorm @ wgu^T.
-    ``ssq``: see gemv_norm."""
+    ``ssq``, ``sums``: see gemv_norm."""
     M = res.numel() // res.shape[-1]
     K = res.shape[-1]
     I = wgu.shape[0] // 2
     how = _product(res, wgu, I)
     if how is None:
         return swiglu(torch.nn.functional.linear(rmsnorm(res, wnorm, eps), wgu))
-    if how == "skinny" or not _norm_ok(M, K):
+    if not _norm_inside(how, M, K, sums):
         return gemv_swiglu(rmsnorm(res, wnorm, eps), wgu, out)
     if out is None:
         out = torch.empty(*res.shape[:-1], I, dtype=res.dtype, device=res.device)
+    if how == "skinny":
+        _mixers.skinny(None, res.contiguous().view(M, K), wgu, I,
+                       _mixers.EPI_SWIGLU, act=out, stride=I,
+                       norm=(wnorm, sums, eps))
+        return out
     _launch_gemv(out, res.contiguous().view(M, K), wnorm, wgu, None, I, eps,
                  _SWIGLU, ssq)
     return out

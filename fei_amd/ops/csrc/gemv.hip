@@ -386,12 +386,27 @@ __device__ __forceinline__ void load_lds_nt(const u16* src, u32 lds) {
       : "memory");
 }
 
+// The RMS norm of x inside the product, from the sums of squares that the
+// product before left.
+struct SkinnyNorm {
+  const u16* gain;     // null: none
+  const float* sums;   // [M, tiles], one per 16 columns of x
+  int tiles;
+  float eps;
+  float* sums_out;     // EPI_RES_BF16: the same of the new rows; may be null
+};
+
 // XL: groups of 8 rows of x. N: results a row of x; with EPI_SWIGLU w has N
-// rows of gates, then N of up, and half of a wave's tiles are either.
-template <int EPI, int XL, int RT, int S>
+// rows of gates, then N of up, and half of a wave's tiles are either. NORM: x is
+// a residual; its fragments take the gains on the way to the matrix units (rounded
+// then, as a norm kernel would), the sums the root mean square. 8 rows, 28672 x
+// 4096: 43 us for 41 and a norm's launch of 4.8; normed in full before the
+// products, with the root mean square waited for, it was 46.
+template <int EPI, int XL, int RT, int S, bool NORM>
 __global__ void __launch_bounds__(256)
 k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
-         const u16* __restrict__ w, int M, int N, int K, Epilogue ep) {
+         const u16* __restrict__ w, int M, int N, int K, Epilogue ep,
+         SkinnyNorm nm) {
   constexpr int MT = (XL + 1) / 2;
   constexpr int LOADS = 2 * RT + XL, STAGE = LOADS * 512;
   constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : RT;
@@ -430,8 +445,25 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // NORM: the gains go behind the stages; the sums of squares (of rows wid, wid
+  // + 4, ..) are asked for first and used last
+  const u16* gs = buf + 4 * S * STAGE;
+  constexpr int NR = NORM ? 2 * XL : 1;
+  float raw[NR][4];
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        raw[i][t] = nm.sums[(long)min(wid + 4 * i, M - 1) * nm.tiles +
+                            min(lane + 64 * t, nm.tiles - 1)];
+    for (int i = tid; i < K / 8; i += 256)
+      ((s16x8*)gs)[i] = ((const s16x8*)nm.gain)[i];
+  }
 #pragma unroll
   for (int s = 0; s < S; ++s) load(lo + s, s);
+  // the other waves' gains too; the stages stay in flight
+  if (NORM) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   int b = 0;
   for (int s = lo; s < hi; ++s) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * LOADS) : "memory");
@@ -450,8 +482,22 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
         fb[kk][j] = ld8(bx + (j * 16 + r) * 64 + c);
       }
     }
+    s16x8 fg[2];
+    if (NORM)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+        fg[kk] = ld8(gs + s * 64 + (kk * 4 + lg) * 8);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     load(s + S, b);
+    if (NORM)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            fb[kk][j][e] = (short)El<u16>::st(bf2f((u16)fb[kk][j][e]) *
+                                              bf2f((u16)fg[kk][e]));
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -462,6 +508,20 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
     b = b == S - 1 ? 0 : b + 1;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __shared__ float sinv[NORM ? XL * 8 : 1];
+  if (NORM) {
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      float ss = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        if (lane + 64 * t < nm.tiles) ss += raw[i][t];
+      for (int t = lane + 256; t < nm.tiles; t += 64)
+        ss += nm.sums[(long)min(wid + 4 * i, M - 1) * nm.tiles + t];
+      ss = wave_sum(ss);
+      if (lane == 0) sinv[wid + 4 * i] = rsqrtf(ss / (float)K + nm.eps);
+    }
+  }
   __syncthreads();
   f32x4* red = (f32x4*)buf;
 #pragma unroll
@@ -483,34 +543,58 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
   for (int t = wid; t < RO * MT; t += 4) {
     const int m = t % MT * 16 + l15, n = n0 + t / MT * 16 + 4 * lg;
     f32x4 v = sum(t);
+    const float inv = NORM ? sinv[min(m, XL * 8 - 1)] : 1.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] *= inv;
     if (EPI == EPI_SWIGLU) {
       const f32x4 u = sum(t + RO * MT);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = v[e] / (1.f + __expf(-v[e])) * u[e];
+      for (int e = 0; e < 4; ++e)
+        v[e] = v[e] / (1.f + __expf(-v[e])) * (u[e] * inv);
     }
-    if (m >= M) continue;
+    float sq = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      if (n + e >= N) break;
+      if (m >= M || n + e >= N) break;
       if (EPI == EPI_SWIGLU) ep.act[m * ep.as + n + e] = f2bf(v[e]);
       else epilogue<EPI>(outp, m, N, n + e, v[e], ep);
+      if (EPI == EPI_RES_BF16) {
+        const float y = bf2f(((u16*)outp)[(long)m * N + n + e]);
+        sq = fmaf(y, y, sq);
+      }
+    }
+    if (EPI == EPI_RES_BF16 && nm.sums_out) {
+      sq += __shfl_xor(sq, 16);
+      sq += __shfl_xor(sq, 32);
+      const int tile = n0 / 16 + t / MT;
+      if (lg == 0 && m < M && tile < nm.tiles)
+        nm.sums_out[(long)m * nm.tiles + tile] = sq;
     }
   }
 }
 
 template <int EPI, int XL, int RT, int S>
 void launch_skinny(void* out, const void* x, const void* w, int M, int N,
-                   int K, const Epilogue& ep, hipStream_t stream) {
+                   int K, const Epilogue& ep, const SkinnyNorm& nm,
+                   hipStream_t stream) {
   constexpr int MT = (XL + 1) / 2;
   constexpr int stages = 4 * S * (2 * RT + XL), sums = RT * MT * 4;
   constexpr int lds = (stages > sums ? stages : sums) * 1024;
   constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : RT;
-  if (lds > 65536)                        // beyond that a kernel has to ask
-    (void)hipFuncSetAttribute((const void*)k_skinny<EPI, XL, RT, S>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  hipLaunchKernelGGL((k_skinny<EPI, XL, RT, S>),
-                     dim3((N + 16 * RO - 1) / (16 * RO)), dim3(256), lds,
-                     stream, out, (const u16*)x, (const u16*)w, M, N, K, ep);
+  auto go = [&](auto kernel, int bytes) {
+    if (bytes > 65536)                    // beyond that a kernel has to ask
+      (void)hipFuncSetAttribute((const void*)kernel,
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                bytes);
+    hipLaunchKernelGGL(kernel, dim3((N + 16 * RO - 1) / (16 * RO)), dim3(256),
+                       bytes, stream, out, (const u16*)x, (const u16*)w, M, N,
+                       K, ep, nm);
+  };
+  if constexpr ((EPI == EPI_BF16 || EPI == EPI_SWIGLU) && XL <= 4)
+    if (nm.gain)
+      return go(k_skinny<EPI, XL, RT, S, true>,
+                (stages * 1024 + K * 2 > lds ? stages * 1024 + K * 2 : lds));
+  go(k_skinny<EPI, XL, RT, S, false>, lds);
 }
 
 // Few rows of w (under 320 tiles, little more than one a CU): small tiles, so
@@ -519,43 +603,48 @@ void launch_skinny(void* out, const void* x, const void* w, int M, int N,
 // 28672 x 4096, 32 rows: 46 us against 50; 64: 55, 66.
 template <int EPI, int XL>
 void by_tiles(void* out, const void* x, const void* w, int M, int N, int K,
-              const Epilogue& ep, hipStream_t stream) {
+              const Epilogue& ep, const SkinnyNorm& nm, hipStream_t stream) {
   const int rows = EPI == EPI_SWIGLU ? 2 * N : N;
   if constexpr (XL >= 4)
     if (rows >= 16384)
-      return launch_skinny<EPI, XL, 4, 2>(out, x, w, M, N, K, ep, stream);
+      return launch_skinny<EPI, XL, 4, 2>(out, x, w, M, N, K, ep, nm, stream);
   if constexpr (EPI != EPI_SWIGLU)
     if (rows < 5120)
       return launch_skinny<EPI, XL, 1, (XL < 4 ? 3 : 2)>(out, x, w, M, N, K,
-                                                         ep, stream);
-  launch_skinny<EPI, XL, 2, 2>(out, x, w, M, N, K, ep, stream);
+                                                         ep, nm, stream);
+  launch_skinny<EPI, XL, 2, 2>(out, x, w, M, N, K, ep, nm, stream);
 }
 
 template <int EPI>
 void by_rows(void* out, const void* x, const void* w, int M, int N, int K,
-             const Epilogue& ep, hipStream_t stream) {
-  if (M <= 8) by_tiles<EPI, 1>(out, x, w, M, N, K, ep, stream);
-  else if (M <= 16) by_tiles<EPI, 2>(out, x, w, M, N, K, ep, stream);
-  else if (M <= 24) by_tiles<EPI, 3>(out, x, w, M, N, K, ep, stream);
-  else if (M <= 32) by_tiles<EPI, 4>(out, x, w, M, N, K, ep, stream);
-  else if (M <= 48) by_tiles<EPI, 6>(out, x, w, M, N, K, ep, stream);
-  else by_tiles<EPI, 8>(out, x, w, M, N, K, ep, stream);
+             const Epilogue& ep, const SkinnyNorm& nm, hipStream_t stream) {
+  if (M <= 8) by_tiles<EPI, 1>(out, x, w, M, N, K, ep, nm, stream);
+  else if (M <= 16) by_tiles<EPI, 2>(out, x, w, M, N, K, ep, nm, stream);
+  else if (M <= 24) by_tiles<EPI, 3>(out, x, w, M, N, K, ep, nm, stream);
+  else if (M <= 32) by_tiles<EPI, 4>(out, x, w, M, N, K, ep, nm, stream);
+  else if (M <= 48) by_tiles<EPI, 6>(out, x, w, M, N, K, ep, nm, stream);
+  else by_tiles<EPI, 8>(out, x, w, M, N, K, ep, nm, stream);
 }
 
 }  // namespace
 
 // 1 to 64 rows, K % 64 == 0, rows of x and w 16-byte aligned. See Epilogue for
-// what becomes of the sums and which of the arguments that takes.
+// what becomes of the sums and which of the arguments that takes. gain (up to 32
+// rows, EPI_BF16 and EPI_SWIGLU; 16-byte aligned): x under an RMS norm with the
+// sums [M, tiles]. sums_out (EPI_RES_BF16): [M, tiles], tiles = N / 16 up.
 extern "C" void fei_skinny(void* out, const void* x, const void* w, int M,
                            int N, int K, int epi, const float* bias,
                            float scale, float cap, int n_mix, int n_router,
                            float* router, void* act, long as,
-                           const void* bias16, hipStream_t stream) {
+                           const void* bias16, const void* gain,
+                           const float* sums, int tiles, float eps,
+                           float* sums_out, hipStream_t stream) {
   const Epilogue ep{bias,   scale,     cap, n_mix,              n_router,
                     router, (u16*)act, as,  (const u16*)bias16};
+  const SkinnyNorm nm{(const u16*)gain, sums, tiles, eps, sums_out};
   switch (epi) {
 #define CASE(E)                                                      \
-  case E: return by_rows<E>(out, x, w, M, N, K, ep, stream)
+  case E: return by_rows<E>(out, x, w, M, N, K, ep, nm, stream)
     CASE(EPI_BF16);
     CASE(EPI_F32);
     CASE(EPI_RES);

@@ -175,12 +175,17 @@ def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def skinny(out, x, w, n: int, epi: int, bias=None, scale: float = 1.0,
            cap: float = 0.0, n_mix: int = 0, router=None, act=None,
-           stride: int = 0, bias16=None) -> None:
-    """x [T, K] with the rows of ``w``: ``n`` results a row."""
+           stride: int = 0, bias16=None, norm=None, sums_out=None) -> None:
+    """x [T, K] with the rows of ``w``: ``n`` results a row. ``norm``: (gains,
+    sums of squares, eps) of an RMS norm that x is under."""
     T, K = x.shape
+    gain, sums, eps = norm or (None, None, 0.0)
+    of = sums if sums is not None else sums_out
+    tiles = 0 if of is None else of.shape[1]
     _lib().fei_skinny(_p(out), _p(x), _p(w), T, n, K, epi, _p(bias), scale,
                       cap, n_mix, 0 if router is None else router.shape[1],
-                      _p(router), _p(act), stride, _p(bias16), _stream())
+                      _p(router), _p(act), stride, _p(bias16), _p(gain),
+                      _p(sums), tiles, eps, _p(sums_out), _stream())
 
 
 def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,

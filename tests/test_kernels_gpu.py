@@ -242,6 +242,22 @@ def test_skinny_geometries(lib, M, N, K):
     assert row_err(f, 3 * torch.tanh(a * 0.5 / 3) + bias.double()) < 1e-5
     mx.skinny(f.copy_(want), x, w1, N, mx.EPI_RES, scale=0.25)
     assert row_err(f, want.float().double() + 0.25 * a) < 1e-5
+    # a residual's next product under a norm: the sums of squares of its tiles
+    h = randbf(M, N, seed=6)
+    sums = lib.add_product(x, w1, h)
+    assert row_err(sums, (h.double() ** 2 @ torch.nn.functional.pad(
+        torch.eye(-(-N // 16), device=DEV, dtype=torch.float64)
+        .repeat_interleave(16, 0)[:N], (0, 0)))) < 1e-5
+    if N % 64 == 0:
+        g, w2 = randbf(N, seed=7), randbf(48, N, seed=8, scale=N ** -0.5)
+        # inputs rounded under their gains: 2^-9 of each product, up to twice
+        # that of a row of few results; a SwiGLU takes two of them with slopes
+        # of up to 1.1, 2.2 * 2^-8, and is rounded: under 2^-6
+        y2 = rms64(h, g, 1e-5) @ w2.double().T
+        assert row_err(lib.gemv_norm(h, g, w2, 1e-5, sums=sums), y2) < 2 ** -7
+        assert row_err(lib.gemv_swiglu_norm(h, g, w2, 1e-5, sums=sums),
+                       torch.nn.functional.silu(y2[:, :24]) * y2[:, 24:]) \
+            < 2 ** -6
     n_mix, n_r = N - 12, 4
     proj = torch.empty(M, n_mix, device=DEV, dtype=torch.bfloat16)
     router = torch.empty(M, n_r, device=DEV)
