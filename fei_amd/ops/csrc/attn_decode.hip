@@ -24,7 +24,6 @@
 
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) u32 u32x4;
 typedef __attribute__((ext_vector_type(2))) u32 u32x2;
 
 constexpr float M_NONE = -3.0e38f;       // maximum of no keys

@@ -27,28 +27,11 @@
 
 namespace {
 
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(4))) u32 u32x4;
 
 constexpr int ROWS = 128;              // rows per block
 constexpr int KEYS = 64;               // keys per tile
 constexpr float M_NONE = -3.0e38f;     // maximum of a row without keys
-
-__device__ __forceinline__ f32x16 mma32(s16x8 a, s16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-      __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
-      0);
-}
-
-// v of this lane and of lane ^ 32
-__device__ __forceinline__ f32x2 both_halves(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(
-      __builtin_bit_cast(u32, v), __builtin_bit_cast(u32, v), false, false);
-  const u32 lo = r[0], hi = r[1];
-  return f32x2{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
-}
 
 // Keys that a block of rows reads: tiles [t0, t1) of n keys, cut into splits of
 // at least three tiles.

@@ -30,7 +30,6 @@ __device__ __forceinline__ T part_of(float v, int i) {
 __device__ __forceinline__ void weight_parts(const float (&v)[8],
                                              s16x8 (&p)[2]) {
   typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-  typedef __attribute__((ext_vector_type(4))) u32 u32x4;
   u32x4 hi, lo;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

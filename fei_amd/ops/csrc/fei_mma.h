@@ -14,6 +14,16 @@ typedef __attribute__((ext_vector_type(8))) float f32x8;
 __device__ __forceinline__ f32x4 mma(s16x8 a, s16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+// 32x32x16: the lane's 8 elements k = 8*(lane/32) .. +7 of row or column lane%32;
+// the result's register e is row 8*(e/4) + 4*(lane/32) + e%4, column lane%32.
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) u32 u32x4;
+__device__ __forceinline__ f32x16 mma32(s16x8 a, s16x8 b, f32x16 c) {
+  typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+      __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+      0);
+}
 __device__ __forceinline__ f32x4 mma(f32x8 a, f32x8 b, f32x4 c) {
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -112,6 +122,14 @@ __device__ __forceinline__ float row16_sum(float v) {
   v += row_ror<4>(v);
   v += row_ror<2>(v);
   return v + row_ror<1>(v);
+}
+
+// v of the lane's half and of the other (lane ^ 32), in one order in both.
+__device__ __forceinline__ f32x2 both_halves(float v) {
+  const u32 u = __builtin_bit_cast(u32, v);
+  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  const u32 lo = r[0], hi = r[1];
+  return f32x2{__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi)};
 }
 
 // Precise sigmoid and silu.

@@ -10,7 +10,6 @@
 
 namespace {
 
-typedef __attribute__((ext_vector_type(4))) u32 u32x4;
 
 enum { GEMV_BF16 = 0, GEMV_RES = 1, GEMV_SWIGLU = 2 };
 

@@ -688,6 +688,225 @@ k_window_prefill(T* __restrict__ out, long os, const T* __restrict__ proj,
   }
 }
 
+// The same for bfloat16 heads of whole panels of 64 dimensions: dim and rot
+// multiples of 64, KP panels together; vdim = 64 VP. Four waves own 32 queries
+// each and half of every tile of 64 keys, four more the other halves; the two
+// sums of a query meet at the end. Scores are computed transposed (K times Q^T,
+// 32x32x16): a lane has 16 scores of ONE query, so that the softmax needs a
+// single exchange between lanes and the weights are, as they lie, the second
+// operand of V^T times P^T. Panels of keys and values come by direct loads one
+// tile ahead, the 16-byte (K) or 32-byte (V) places of a row permuted by the
+// row, and V is turned by the transposing LDS read; in the general kernel keys,
+// values and weights pass registers on the way to LDS and scores a reduction
+// over 16 lanes.
+//
+// Bound by the chain of tiles of the longest block: a prompt of 900 tokens has 8
+// blocks a head, the last of 15 tiles. 900 + 333 + 64 tokens, 16 heads of
+// 128 + 64 and 128, window 1024: 68 us in the general kernel, 37 here, 43 with
+// one wave for all keys of a tile (one wave on a SIMD: nothing runs while it
+// waits).
+constexpr float M_NONE = -3.0e38f;
+
+template <int KP, int VP>
+__global__ void __launch_bounds__(512, 2)
+k_window_panels(u16* __restrict__ out, long os, const u16* __restrict__ proj,
+                long ps, const u16* __restrict__ kv,
+                const u16* __restrict__ krot, const int* __restrict__ spans,
+                const int* __restrict__ tiles, int gate_off, Geo g) {
+  constexpr int KS = 4 * KP, DT = 2 * VP, PAN = 64 * 64;
+  extern __shared__ __align__(16) u16 buf[];       // [2][KP + VP][64][64]
+  const int h = blockIdx.x;
+  const int* sp = spans + tiles[blockIdx.y * 2] * 5;
+  const int row0 = sp[0], cnt = sp[1], pos0 = sp[2], key0 = sp[3], at0 = sp[4];
+  const int q0 = tiles[blockIdx.y * 2 + 1];
+  const int qn = min(128, cnt - q0);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int w = wave & 3, half = wave >> 2;        // queries 32 w, keys 32 half
+  const int l31 = lane & 31, hf = lane >> 5;
+  const long kvs = (long)g.heads * (g.dim + g.vdim);
+  const u16* kh = kv + (long)h * g.dim;
+  const u16* vh = kv + (long)g.heads * g.dim + (long)h * g.vdim;
+
+  // positions of this tile's queries and of the keys any of them sees
+  const int qa = pos0 + q0, qb = qa + qn - 1;
+  const int klo = max(first_key(qa, g.window), key0) & ~63;
+  const int wa = qa + w * 32, wb = min(wa + 31, qb);
+  const int wlo = max(first_key(min(wa, qb), g.window), key0);
+  const int r = min(w * 32 + l31, qn - 1);         // the lane's query
+  const int hi = qa + r, lo = max(first_key(hi, g.window), key0);
+
+  // a negative scale turns the queries round, a zero one clears them, so that
+  // the largest score stays the largest after scaling
+  const float c = g.scale == 0.f ? 1.f : fabsf(g.scale) * El<u16>::base;
+  const u32 flip = g.scale < 0.f ? 0x80008000u : 0u;
+  const u32 keep = g.scale == 0.f ? 0u : 0xffffffffu;
+  s16x8 fq[KS];
+  {
+    const u16* q = proj + (long)(row0 + q0 + r) * ps +
+                   (long)h * (g.dim + g.rot) + 8 * hf;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      u32x4 v = *(const u32x4*)(q + k * 16);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (v[e] ^ flip) & keep;
+      fq[k] = __builtin_bit_cast(s16x8, v);
+    }
+  }
+
+  const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)buf;
+  // the wave's 8 rows of each panel; the place's elements in a row
+  const int row = wave * 8 + (lane >> 3), place = lane & 7;
+  const int ck = (place ^ (row & 7)) << 3;
+  const int cv = ((((place >> 1) ^ row) & 3) << 4) + (place & 1) * 8;
+  auto load = [&](int t0, int p) {
+    const u32 to = lds + (p * (KP + VP) * PAN + wave * 512) * 2;
+    const int n = at0 + min(max(t0 + row, key0), qb) - key0;
+    const u16* kr = kh + n * kvs;
+    const u16* rr = krot + (long)n * g.rot - g.dim;
+#pragma unroll
+    for (int pan = 0; pan < KP; ++pan)
+      load_lds((pan * 64 < g.dim ? kr : rr) + pan * 64 + ck,
+               to + pan * PAN * 2);
+#pragma unroll
+    for (int pan = 0; pan < VP; ++pan)
+      load_lds(vh + n * kvs + pan * 64 + cv, to + (KP + pan) * PAN * 2);
+  };
+
+  float m = M_NONE, l = 0.f;
+  f32x16 o[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
+
+  load(klo, 0);
+  int p = 0;
+  for (int t0 = klo; t0 <= qb; t0 += 64, p ^= 1) {
+    // the tile is there, and all waves are done with the other buffer
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (t0 + 64 <= qb) load(t0 + 64, p ^ 1);
+    const int u0 = t0 + 32 * half;         // the wave's keys
+    if (u0 > wb || u0 + 31 < wlo) continue;
+    const u16* kt = buf + p * (KP + VP) * PAN + (half * 32 + l31) * 64;
+    const u16* vt = buf + (p * (KP + VP) + KP) * PAN + half * 32 * 64;
+    f32x16 s;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+      s = mma32(ld8(kt + (k / 4) * PAN + (((k % 4 * 2 + hf) ^ (l31 & 7)) << 3)),
+                fq[k], s);
+    // register e is key u0 + 8 (e / 4) + 4 hf + e % 4
+    if (u0 + 31 > wa || u0 < wlo || (g.window > 0 && wb - u0 >= g.window)) {
+      const int a = hi - u0 - 4 * hf, b = lo - u0 - 4 * hf;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int key = 8 * (e / 4) + e % 4;
+        if (key > a || key < b) s[e] = NEG_INF;
+      }
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    const f32x2 two = both_halves(mx);
+    mx = fmaxf(two[0], two[1]) * c;
+    // the maximum may lag behind by 2^8: see there, attn_prefill.hip
+    if (__any(mx > m + 8.f)) {
+      const float mn = fmaxf(m, mx);
+      const float al = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= al;
+#pragma unroll
+      for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[i][e] *= al;
+    }
+    const int vr = 4 * hf + ((lane & 15) >> 2), vc = (lane >> 4) & 1;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {          // 16 keys
+      float v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        v[e] = __builtin_amdgcn_exp2f(fmaf(s[i * 8 + e], c, -m));
+        l += v[e];
+      }
+      s16x8 fp[2];
+      weight_parts(v, fp);
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        const u16* vp = vt + (dt / 2) * PAN + (i * 16 + vr) * 64 +
+                        (((dt % 2 * 2 + vc) ^ (vr & 3)) << 4) + (lane & 3) * 4;
+        const s16x8 fv = turn8(vp, vp + 8 * 64);
+        o[dt] = mma32(fv, fp[0], o[dt]);
+        o[dt] = mma32(fv, fp[1], o[dt]);
+      }
+    }
+  }
+  const f32x2 lt = both_halves(l);
+  l = lt[0] + lt[1];
+
+  // the two halves of the keys: each wave keeps half of the dimensions and
+  // takes the other wave's sums of them
+  float* part = (float*)buf + (w * 64 + lane);     // [register][wave, lane]
+  float* ml = (float*)buf + 16 * DT * 256; // [half][max, sum][wave, lane]
+  __syncthreads();
+  ml[half * 512 + w * 64 + lane] = m;
+  ml[half * 512 + 256 + w * 64 + lane] = l;
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+    if (d / VP != half)
+#pragma unroll
+      for (int e = 0; e < 16; ++e)
+        part[(d * 16 + e) * 256] = o[d][e];
+  __syncthreads();
+  const float m2 = ml[(half ^ 1) * 512 + w * 64 + lane];
+  const float l2 = ml[(half ^ 1) * 512 + 256 + w * 64 + lane];
+  const float mt = fmaxf(m, m2);
+  float a1 = __builtin_amdgcn_exp2f(m - mt), a2 = __builtin_amdgcn_exp2f(m2 - mt);
+  if (w * 32 + l31 >= qn) return;
+  const float inv = 1.f / (l * a1 + l2 * a2);      // a query always sees itself
+  a1 *= inv;
+  a2 *= inv;
+  const long at = row0 + q0 + r;
+  const u16* gate = proj + at * ps + gate_off + (long)h * g.vdim + 4 * hf;
+  u16* dst = out + at * os + (long)h * g.vdim + 4 * hf;
+#pragma unroll
+  for (int d = 0; d < DT; ++d)
+    if (d / VP == half)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        u16 z[4], y[4];
+        __builtin_memcpy(z, gate + d * 32 + 8 * i, sizeof(z));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float v = o[d][4 * i + e] * a1 +
+                          part[(d * 16 + 4 * i + e) * 256] * a2;
+          y[e] = El<u16>::st(v * sigmoid_f(bf2f(z[e])));
+        }
+        __builtin_memcpy(dst + d * 32 + 8 * i, y, sizeof(y));
+      }
+}
+
+template <int KP, int VP>
+void launch_panels(u16* out, long os, const u16* proj, long ps, const u16* kv,
+                   const u16* krot, const int* spans, const int* tiles,
+                   int n_tiles, Geo g, hipStream_t stream) {
+  // tiles; afterwards the sums [16 DT][256] and [2][2][256]
+  constexpr int lds = (KP + VP) * 16384 > (32 * VP + 4) * 1024
+                          ? (KP + VP) * 16384 : (32 * VP + 4) * 1024;
+  static bool set = lds <= 65536;
+  if (!set) {
+    (void)hipFuncSetAttribute((const void*)k_window_panels<KP, VP>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    set = true;
+  }
+  const int gate_off = g.heads * (g.dim + g.rot) + g.kr + g.rot;
+  hipLaunchKernelGGL((k_window_panels<KP, VP>), dim3(g.heads, n_tiles),
+                     dim3(512), lds, stream, out, os, proj, ps, kv, krot,
+                     spans, tiles, gate_off, g);
+}
+
 template <typename T>
 int run_decode(T* out, long os, const T* proj, long ps, const T* wuk,
                const T* wuv, const float* nw, const float* rotab, T* rows,
@@ -780,6 +999,24 @@ void run_window(T* out, long os, const T* proj, long ps, const T* kv,
                 int n_tiles, Geo g, hipStream_t stream) {
   const int vec = g.dim % 8 == 0 && g.rot % 8 == 0 && g.vdim % 8 == 0 &&
                   ps % 8 == 0;
+  if constexpr (sizeof(T) == 2) {
+    // whole panels that fit LDS and registers; loads of 16 bytes, so aligned
+    const int kp = (g.dim + g.rot) / 64, vp = g.vdim / 64;
+    if (vec && g.dim % 64 == 0 && g.rot % 64 == 0 && g.vdim % 64 == 0 &&
+        kp >= 1 && kp <= 4 && vp >= 1 && vp <= 2 &&
+        (((uintptr_t)proj | (uintptr_t)kv | (uintptr_t)krot) & 15) == 0) {
+#define PANELS(KP)                                                           \
+  return vp == 1 ? launch_panels<KP, 1>(out, os, proj, ps, kv, krot, spans,  \
+                                        tiles, n_tiles, g, stream)           \
+                 : launch_panels<KP, 2>(out, os, proj, ps, kv, krot, spans,  \
+                                        tiles, n_tiles, g, stream)
+      if (kp == 1) PANELS(1);
+      if (kp == 2) PANELS(2);
+      if (kp == 3) PANELS(3);
+      PANELS(4);
+#undef PANELS
+    }
+  }
   const int ks = (g.dim + g.rot + 31) / 32, dc = (g.vdim + 15) / 16;
 #define WIN(KS, DC) launch_window<T, KS, DC>(out, os, proj, ps, kv, krot,    \
                                              spans, tiles, n_tiles, g, vec,  \

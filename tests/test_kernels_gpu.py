@@ -346,3 +346,62 @@ def test_encoder_attention_reads_views(lib):
                                 v.transpose(1, 2).contiguous(), zero,
                                 causal=False, kv_len=lens)
         assert torch.equal(got, want)
+
+
+# -- prompt attention over windows ---------------------------------------------
+
+@pytest.mark.parametrize("dims", [(128, 64, 128), (64, 0, 64), (64, 64, 128),
+                                  (192, 64, 64), (64, 0, 192), (96, 32, 64)])
+@pytest.mark.parametrize("window,parts,scale", [
+    (0, [(1, 1, 0), (2, 129, 0), (131, 33, 70)], 0.1),
+    (64, [(0, 200, 300), (200, 64, 0)], 0.1),
+    (65, [(0, 128, 63), (130, 31, 1000)], -0.1),
+    (1, [(0, 66, 5)], 0.1),
+    (1024, [(0, 300, 1100)], 0.0),
+])
+def test_window_prefill_geometries(lib, dims, window, parts, scale):
+    """Panels of 64 (the first four) and the general path, whose only
+    difference is the width of the heads."""
+    from fei_amd.ops import mixers as mx
+    (dim, rot, vdim), H, kr = dims, 3, 64
+    rows = max(r + n for r, n, _ in parts)
+    q_w = H * (dim + rot)
+    proj = randbf(rows, q_w + kr + rot + H * vdim, seed=rows)
+    spans, tiles, at = [], [], 0
+    for i, (r, n, pos0) in enumerate(parts):
+        k0 = max(0, pos0 - window + 1) if window else 0
+        spans.append([r, n, pos0, k0, at])
+        tiles += [[i, q] for q in range(0, n, 128)]
+        at += pos0 + n - k0
+    kv = randbf(at, H * (dim + vdim), seed=1)
+    krot = randbf(at, rot, seed=2)
+    out = torch.full((rows, H * vdim), 7.0, dtype=torch.bfloat16, device=DEV)
+    sp, tl = (torch.tensor(x, dtype=torch.int32, device=DEV)
+              for x in (spans, tiles))
+    p = mx._p
+    mx._lib().fei_window_prefill(
+        p(out), out.stride(0), p(proj), proj.stride(0), p(kv), p(krot), p(sp),
+        p(tl), len(tiles), H, dim, rot, vdim, kr, scale, window, 0,
+        mx._stream())
+    used = torch.zeros(rows, dtype=torch.bool)
+    for (r, n, pos0), (_, _, _, k0, a) in zip(parts, spans):
+        used[r:r + n] = True
+        m = pos0 + n - k0
+        q = proj[r:r + n, :q_w].double().view(n, H, dim + rot).transpose(0, 1)
+        keys = torch.cat(
+            [kv[a:a + m, :H * dim].double().view(m, H, dim),
+             krot[a:a + m].double()[:, None].expand(m, H, rot)], 2)
+        s = torch.matmul(q, keys.permute(1, 2, 0).contiguous()) * scale
+        qp = pos0 + torch.arange(n, device=DEV)[:, None]
+        kp = k0 + torch.arange(m, device=DEV)[None]
+        hide = kp > qp
+        if window:
+            hide |= qp - kp >= window
+        w = torch.softmax(s.masked_fill(hide, float("-inf")), -1)
+        v = kv[a:a + m, H * dim:].double().view(m, H, vdim).transpose(0, 1)
+        o = torch.matmul(w, v.contiguous()).transpose(0, 1).reshape(n, -1)
+        o = o * proj[r:r + n, q_w + kr + rot:].double().sigmoid()
+        # weights keep 16 bits, sums are float32: the rounding of the result
+        # (2^-9 an element, less in a row's norm) is what shows
+        assert row_err(out[r:r + n], o) < 2.0 ** -8
+    assert bool((out[~used.to(DEV)] == 7.0).all())
