@@ -399,8 +399,9 @@ struct SkinnyNorm {
 // rows of gates, then N of up, and half of a wave's tiles are either. NORM: x is
 // a residual; its fragments take the gains on the way to the matrix units (rounded
 // then, as a norm kernel would), the sums the root mean square. 8 rows, 28672 x
-// 4096: 43 us for 41 and a norm's launch of 4.8; normed in full before the
-// products, with the root mean square waited for, it was 46.
+// 4096: 42 us for 41 and a norm's launch of 4.8; normed in full before the
+// products, with the root mean square waited for, it was 46; with the gains
+// through registers, before the first stages could be asked for, 43.
 template <int EPI, int XL, int RT, int S, bool NORM>
 __global__ void __launch_bounds__(256)
 k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
@@ -465,13 +466,17 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
       for (int t = 0; t < 4; ++t)
         raw[i][t] = nm.sums[(long)min(wid + 4 * i, M - 1) * nm.tiles +
                             min(lane + 64 * t, nm.tiles - 1)];
-    for (int i = tid; i < K / 8; i += 256)
-      ((s16x8*)gs)[i] = ((const s16x8*)nm.gain)[i];
+    // 1 KB a load, to the end of a whole one
+    const u32 to = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)gs;
+    for (int i = wid * 512; i < K; i += 2048)
+      load_lds(nm.gain + min(i + lane * 8, K - 8), to + i * 2);
   }
 #pragma unroll
   for (int s = 0; s < S; ++s) load(s, s);
-  // the other waves' gains too; the stages stay in flight
-  if (NORM) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  // the gains of all waves; the stages stay in flight
+  if (NORM)
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(S * LOADS)
+                 : "memory");
   int b = 0;
   for (int s = 0; s < n; ++s) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * LOADS) : "memory");
@@ -503,9 +508,17 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
 #pragma unroll
         for (int j = 0; j < MT; ++j)
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            fb[kk][j][e] = (short)El<u16>::st(bf2f((u16)fb[kk][j][e]) *
-                                              bf2f((u16)fg[kk][e]));
+          for (int e = 0; e < 8; e += 2) {
+            typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+            typedef __attribute__((ext_vector_type(2))) short s16x2;
+            const f32x2 v = {bf2f((u16)fb[kk][j][e]) * bf2f((u16)fg[kk][e]),
+                             bf2f((u16)fb[kk][j][e + 1]) *
+                                 bf2f((u16)fg[kk][e + 1])};
+            const s16x2 y = __builtin_bit_cast(
+                s16x2, __builtin_convertvector(v, bf16x2));
+            fb[kk][j][e] = y[0];
+            fb[kk][j][e + 1] = y[1];
+          }
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
@@ -601,7 +614,7 @@ void launch_skinny(void* out, const void* x, const void* w, int M, int N,
   if constexpr ((EPI == EPI_BF16 || EPI == EPI_SWIGLU) && XL <= 4)
     if (nm.gain)
       return go(k_skinny<EPI, XL, RT, S, true>,
-                (stages * 1024 + K * 2 > lds ? stages * 1024 + K * 2 : lds));
+                max(lds, stages * 1024 + (K + 511) / 512 * 1024));
   go(k_skinny<EPI, XL, RT, S, false>, lds);
 }
 
