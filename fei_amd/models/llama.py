@@ -396,7 +396,6 @@ class LlamaModel:
         B, S = tokens.shape
         h = F.embedding(tokens.long(), self.emb)          # [B,S,C] residual
         scale = 1.0 / math.sqrt(self.D)
-        n_layers = len(self.layers)
 
         def attend(li, qkv):
             q, k, v = self._qkv_views(qkv.view(B * S, -1), B, S)
@@ -414,21 +413,59 @@ class LlamaModel:
             return ops.gemv_norm(h, self.norm_f, self.lm_head, s.norm_eps,
                                  sums=sums)
         x = ops.rmsnorm(h, self.layers[0].norm_attn, s.norm_eps)
+        if self.rows_in_parts(B * S, (*k_caches, *v_caches)):
+            x = self._layers_in_parts(x.view(B * S, -1), h.view(B * S, -1), S,
+                                      pos0, k_caches, v_caches).view(B, S, -1)
+        else:
+            x = self._layers(x, h, attend)
+        last = x if all_positions else x[:, -1, :]
+        logits = ops.linear_decode(last, self.lm_head)
+        logits = all_gather_cat(logits, dim=-1, ctx=self.tp)
+        return logits
+
+    def rows_in_parts(self, T: int, caches) -> bool:
+        """Whether a prompt of T rows runs products cut along K, whose parts
+        the next kernel sums (to caches of its type, 16 bytes at a time)."""
+        lw = self.layers[0]
+        return (self.tp_size == 1 and self.D % 16 == 0 and
+                all(ops.rows_ok(T, w) for w in (lw.wqkv, lw.wo, lw.wdown)) and
+                all(c.dtype == lw.wqkv.dtype and c.data_ptr() % 16 == 0
+                    for c in caches))
+
+    def _layers_in_parts(self, x, h, S, pos0, k_caches, v_caches):
+        """All layers over T rows x (normed) of the residual h -> the final
+        norm's rows."""
+        eps = self.spec.norm_eps
+        for li, lw in enumerate(self.layers):
+            q = ops.rope_kv_parts(ops.product_parts(x, lw.wqkv), S, self.hq_l,
+                                  k_caches[li], v_caches[li], pos0, self.rope)
+            att = ops.attn_prefill(q, k_caches[li], v_caches[li], pos0,
+                                   scale=1.0 / math.sqrt(self.D))
+            x = ops.add_norm_parts(
+                ops.product_parts(att.view(h.shape[0], -1), lw.wo), h,
+                lw.norm_mlp, eps)
+            act = ops.gemv_swiglu(x, lw.wgu)
+            x = ops.add_norm_parts(ops.product_parts(act, lw.wdown), h,
+                                   self._norm_after(li), eps)
+        return x
+
+    def _norm_after(self, li: int) -> torch.Tensor:
+        return (self.layers[li + 1].norm_attn if li + 1 < len(self.layers)
+                else self.norm_f)
+
+    def _layers(self, x, h, attend):
+        """The same by whole products."""
+        s = self.spec
         for li, lw in enumerate(self.layers):
             att = attend(li, ops.linear_decode(x, lw.wqkv))     # [B,S,W]
-            o = ops.linear_decode(att.reshape(B, S, -1), lw.wo)
+            o = ops.linear_decode(att.reshape(*h.shape[:-1], -1), lw.wo)
             all_reduce_sum(o, self.tp)
             x, h = ops.fused_add_rmsnorm(o, h, lw.norm_mlp, s.norm_eps)
             act = ops.gemv_swiglu(x, lw.wgu)
             d = ops.linear_decode(act, lw.wdown)
             all_reduce_sum(d, self.tp)
-            next_norm = (self.layers[li + 1].norm_attn if li + 1 < n_layers
-                         else self.norm_f)
-            x, h = ops.fused_add_rmsnorm(d, h, next_norm, s.norm_eps)
-        last = x if all_positions else x[:, -1, :]
-        logits = ops.linear_decode(last, self.lm_head)
-        logits = all_gather_cat(logits, dim=-1, ctx=self.tp)
-        return logits
+            x, h = ops.fused_add_rmsnorm(d, h, self._norm_after(li), s.norm_eps)
+        return x
 
     # -- checkpointing (safetensors) -----------------------------------------
 

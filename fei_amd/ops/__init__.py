@@ -22,6 +22,7 @@ import torch
 from fei_amd.ops import mixers as _mixers
 from fei_amd.ops import moe as _moe
 from fei_amd.ops import reference as ref
+from fei_amd.ops import rows as _rows
 from fei_amd.ops import sigmoid_attn as _sigmoid_attn
 from fei_amd.ops.mixers import (  # noqa: F401
     GainNorm, GainNormed, cat_cast, check_gla_geometry,
@@ -30,6 +31,8 @@ from fei_amd.ops.mixers import (  # noqa: F401
     norm_pair, parallel_in, residual_linear)
 from fei_amd.ops.moe import (  # noqa: F401
     check_moe_geometry, residual_moe, route)
+from fei_amd.ops.rows import (  # noqa: F401
+    add_norm_parts, product_parts, rope_kv_parts, rows_ok)
 from fei_amd.ops.sigmoid_attn import (  # noqa: F401
     check_sigmoid_geometry, sigmoid_attn_decode, sigmoid_attn_prefill)
 
@@ -89,6 +92,7 @@ def _try_load() -> None:
     lib.fei_quant_fp8_rows.argtypes = [_vp, _vp, _vp, _i, _i, _vp]
     lib.fei_prefetch.argtypes = [_vp, _l, _vp, _i, _vp]
     _mixers.declare(lib)
+    _rows.declare(lib)
     _moe.declare(lib)
     _sigmoid_attn.declare(lib)
     _LIB = lib
@@ -612,11 +616,16 @@ def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
     K = x.shape[-1]
     I = wgu.shape[0] // 2
     how = _product(x, wgu, I)
+    if how is None and x.is_cuda and _rows.swiglu_ok(M, x, wgu):
+        how = "rows"
     if how is None:
         return swiglu(torch.nn.functional.linear(x, wgu))
     x2 = x.contiguous().view(M, K)
     if out is None:
         out = torch.empty(*x.shape[:-1], I, dtype=x.dtype, device=x.device)
+    if how == "rows":
+        _rows.swiglu_product(x2, wgu, out)
+        return out
     if how == "skinny":
         _mixers.skinny(out, x2, wgu, I, _mixers.EPI_SWIGLU, act=out, stride=I)
     else:

@@ -1,0 +1,354 @@
+// Products of tens to hundreds of rows with a weight matrix (gfx950):
+// out[M, N] = x[M, K] @ W[N, K]^T in bfloat16 with float32 sums, where a library
+// product leaves the chip half idle or makes a result that takes another pass.
+#include "fei_mma.h"
+
+namespace {
+
+enum {
+  ROWS_PARTS = 0,      // float32 sums of a part of K, [parts][M][N]
+  ROWS_SWIGLU = 1,     // W has N rows of gates, then N of up; bfloat16
+};
+
+// Tiles of 32 XJ rows x 32 WI rows of W (SWIGLU: half of them gates, the others
+// the same of up), 4 waves of half by half, S LDS buffers of 64 steps of K filled
+// by direct loads. The 16-byte places of a row are permuted by the row, in the
+// address that a lane reads, so that the fragment reads of 16 rows spread over the
+// banks. Fragments of 32 steps are read ahead of the products with the 32 before;
+// reads and loads go out between the matrix instructions.
+//
+// blockIdx.y: a part of K. Column tiles start at different steps of their part:
+// rows of W often lie a multiple of 4 KB apart, and the same columns of all of
+// them would be on the same memory channels; not where x is more than an L2 holds,
+// which all tiles of columns read together then. An XCD gets consecutive tiles, four
+// of rows times all of columns, rows first, so that its L2 holds what they share.
+//
+// Bound by HBM for one tile of rows, by the loads to LDS (36 to 43 bytes a clock
+// and CU go through them) for more. Cold weights, 75 rows, against the library:
+// 4096 x 14336 in 8 parts 27 us (50), 4096 x 4096 in 4 11.4 (16.2), 6144 x 4096 in
+// 4 15.8 (23.8), 2 x 14336 x 4096 with SwiGLU 48 (53 + 4.5), 58 with all tiles
+// starting at the same step. Two buffers instead of four: 71.
+template <int XJ, int WI, int S, int EPI>
+__global__ void __launch_bounds__(256, S * (XJ + WI) <= 20 ? 2 : 1)
+k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
+       const u16* __restrict__ w, int M, int N, int K, int nx, int nm) {
+  constexpr int TM = 32 * XJ, TN = 32 * WI, MX = XJ > WI ? XJ : WI;
+  constexpr int CN = EPI == ROWS_SWIGLU ? TN / 2 : TN;   // columns of out
+  constexpr int BUF = (TM + TN) * 64, LOADS = XJ + WI;
+  extern __shared__ __align__(16) u16 buf[];
+  const int total = nx * nm, per = (total + 7) / 8;
+  const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
+  const int g0 = id / (4 * nx) * 4, gm = min(4, nm - g0), gr = id - g0 * nx;
+  const int tile = gr / gm, n0 = tile * CN;
+  const int m0 = (g0 + gr % gm) * TM, cnt = min(TM, M - m0);
+  const int all = K / 64, first = (int)(blockIdx.y * (long)all / gridDim.y);
+  const int steps = (int)((blockIdx.y + 1) * (long)all / gridDim.y) - first;
+  const int turn = (long)M * K <= 2 << 20 ? tile * 3 % steps : 0;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, lg = lane >> 4;
+  // 8 rows a load; the place of a row's 8 values depends on the row
+  const int r8 = lane >> 3, c8 = ((lane & 7) ^ r8) * 8 + first * 64;
+  const u16* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < XJ; ++i)
+    src[i] = x + (long)(m0 + min((wid * XJ + i) * 8 + r8, cnt - 1)) * xs + c8;
+#pragma unroll
+  for (int i = 0; i < WI; ++i) {
+    int r = (wid * WI + i) * 8 + r8;       // row of the tile
+    long n;
+    if (EPI == ROWS_SWIGLU) {              // a wave's half: gates, then up
+      const int half = r / (TN / 2), q = r % (TN / 2), up = q / (TN / 4);
+      n = min(n0 + half * (TN / 4) + q % (TN / 4), N - 1) + (long)up * N;
+    } else {
+      n = min(n0 + r, N - 1);
+    }
+    src[XJ + i] = w + n * K + c8;
+  }
+  const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)buf;
+  // past the end the last step is read again, into a buffer that is free
+  auto load = [&](int step, int b, int i) {
+    int t = min(step, steps - 1) + turn;
+    t = t < steps ? t : t - steps;
+    load_lds(src[i] + t * 64,
+             lds + b * BUF * 2 + (i < XJ ? (wid * XJ + i) * 1024
+                                         : TM * 128 + (wid * WI + i - XJ) * 1024));
+  };
+  const int xm = (wid & 1) * 16 * XJ, wm = (wid >> 1) * 16 * WI;
+  struct Frags {
+    s16x8 w[WI], x[XJ];
+  };
+  auto read = [&](Frags& f, int b, int kk, int i) {
+    const int c = ((kk * 4 + lg) ^ (l15 & 7)) * 8;
+    const u16* bx = buf + b * BUF;
+    if (i < XJ) f.x[i] = ld8(bx + (xm + i * 16 + l15) * 64 + c);
+    if (i < WI) f.w[i] = ld8(bx + (TM + wm + i * 16 + l15) * 64 + c);
+  };
+  f32x4 acc[WI][XJ];
+#pragma unroll
+  for (int i = 0; i < WI; ++i)
+#pragma unroll
+    for (int j = 0; j < XJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto product = [&](const Frags& f, int i) {
+    if (i >= WI) return;
+#pragma unroll
+    for (int j = 0; j < XJ; ++j) acc[i][j] = mma(f.w[i], f.x[j], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) load(s, s, i);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * LOADS)
+               : "memory");
+  Frags f0, f1;
+#pragma unroll
+  for (int i = 0; i < MX; ++i) read(f0, 0, 0, i);
+  int b = 0;                               // buffer of step k
+  for (int k = 0; k < steps; ++k) {
+#pragma unroll
+    for (int i = 0; i < MX; ++i) {
+      read(f1, b, 1, i);
+      product(f0, i);
+    }
+    // all waves have the second half of buffer b, which can be filled again,
+    // and the loads of the next one have arrived
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(
+                     (S - 2) * LOADS)
+                 : "memory");
+    const int nb = b == S - 1 ? 0 : b + 1;
+#pragma unroll
+    for (int i = 0; i < MX; ++i) {
+      read(f0, nb, 0, i);
+      load(k + S, b, i);
+      if (MX + i < LOADS) load(k + S, b, MX + i);
+      product(f1, i);
+    }
+    b = nb;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // results 4 lg + 0..3 of a column group, of row l15
+  constexpr int CI = EPI == ROWS_SWIGLU ? WI / 2 : WI;
+#pragma unroll
+  for (int j = 0; j < XJ; ++j) {
+    const int r = xm + j * 16 + l15;
+    if (r >= cnt) continue;
+#pragma unroll
+    for (int i = 0; i < CI; ++i) {
+      const int n = n0 + (wid >> 1) * 16 * CI + i * 16 + 4 * lg;
+      if (n >= N) continue;
+      const long at = (long)(m0 + r) * N + n;
+      if (EPI == ROWS_SWIGLU) {
+        u16 v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float g = acc[i][j][e];
+          v[e] = f2bf(g / (1.f + __expf(-g)) * acc[CI + i][j][e]);
+        }
+        __builtin_memcpy((u16*)outp + at, v, sizeof(v));
+      } else {
+        *(f32x4*)((float*)outp + (long)blockIdx.y * M * N + at) = acc[i][j];
+      }
+    }
+  }
+}
+
+template <int XJ, int WI, int S, int EPI>
+void launch(void* out, const void* x, long xs, const void* w, int M, int N,
+            int K, int parts, hipStream_t stream) {
+  constexpr int lds = S * 32 * (XJ + WI) * 128;
+  constexpr int CN = EPI == ROWS_SWIGLU ? 16 * WI : 32 * WI;
+  static bool set = lds <= 65536;          // beyond that a kernel has to ask
+  if (!set) {
+    (void)hipFuncSetAttribute((const void*)k_rows<XJ, WI, S, EPI>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    set = true;
+  }
+  const int nx = (N + CN - 1) / CN, nm = (M + 32 * XJ - 1) / (32 * XJ);
+  hipLaunchKernelGGL((k_rows<XJ, WI, S, EPI>),
+                     dim3((nx * nm + 7) / 8 * 8, parts), dim3(256), lds, stream,
+                     out, (const u16*)x, xs, (const u16*)w, M, N, K, nx, nm);
+}
+
+template <int WI, int S, int EPI>
+void by_rows(int xj, void* out, const void* x, long xs, const void* w, int M,
+             int N, int K, int parts, hipStream_t stream) {
+  if (xj == 2) launch<2, WI, S, EPI>(out, x, xs, w, M, N, K, parts, stream);
+  else if (xj == 3) launch<3, WI, S, EPI>(out, x, xs, w, M, N, K, parts, stream);
+  else launch<4, WI, S, EPI>(out, x, xs, w, M, N, K, parts, stream);
+}
+
+// The sums of the parts of a product, added to a bfloat16 residual, and its RMS
+// norm: what follows a product inside a layer. A row a block, 8 columns a thread
+// at a time. 75 rows of 4096, 8 parts: 5.0 us, as long as the norm of a whole
+// product took; latency of a launch and two passes over a row.
+__global__ void __launch_bounds__(512)
+k_parts_norm(u16* __restrict__ out, u16* __restrict__ res,
+             const float* __restrict__ parts, int np,
+             const u16* __restrict__ gain, int rows, int cols, float eps) {
+  __shared__ float red[8];
+  const int tid = threadIdx.x, nv = cols >> 3;
+  const long row = blockIdx.x, step = (long)rows * cols;
+  s16x8* rr = (s16x8*)(res + row * cols);
+  float ss = 0.f;
+  for (int i = tid; i < nv; i += 512) {
+    const s16x8 old = rr[i];
+    const float* p = parts + row * cols + i * 8;
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < np; ++k) {
+      const f32x8 q = ld8(p + k * step);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] += q[j];
+    }
+    s16x8 y;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const u16 b = f2bf(bf2f((u16)old[j]) + v[j]);
+      y[j] = (short)b;
+      ss = fmaf(bf2f(b), bf2f(b), ss);
+    }
+    rr[i] = y;
+  }
+  ss = wave_reduce_sum(ss);
+  if ((tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) ss += red[k];
+  const float inv = rsqrtf(ss / (float)cols + eps);
+  for (int i = tid; i < nv; i += 512) {
+    const s16x8 v = rr[i], g = ((const s16x8*)gain)[i];
+    s16x8 y;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      y[j] = (short)f2bf(bf2f((u16)v[j]) * inv * bf2f((u16)g[j]));
+    ((s16x8*)(out + row * cols))[i] = y;
+  }
+}
+
+// The parts of a product with the projections of q, k and v: q to rows of its own
+// and k to the cache under RoPE, v to the cache. A thread takes dimensions
+// 8 i .. 8 i + 7 of a head and their partners D/2 on; D % 16 == 0. 75 tokens, 32/8
+// heads of 128, 4 parts: 4.8 us, for 3.4 to sum the parts and 3.5 for RoPE.
+__global__ void __launch_bounds__(256)
+k_rope_kv_parts(u16* __restrict__ q, const float* __restrict__ parts, int np,
+                u16* __restrict__ kc, u16* __restrict__ vc,
+                const float* __restrict__ cos_sin, const int* __restrict__ pos0,
+                long units, long step, int S, int Hq, int Hkv, int D,
+                int max_seq) {
+  const int per = D / 16, heads = Hq + 2 * Hkv;
+  const long u = (long)blockIdx.x * 256 + threadIdx.x;
+  if (u >= units) return;
+  const int i = (int)(u % per) * 8;
+  const long th = u / per;                 // token and head
+  const int h = (int)(th % heads);
+  const long tok = th / heads;
+  const int b = (int)(tok / S), p = pos0[b] + (int)(tok - (long)b * S);
+  const float* src = parts + th * D + i;
+  float x1[8], x2[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x1[j] = x2[j] = 0.f;
+#pragma unroll 4
+  for (int k = 0; k < np; ++k) {
+    const f32x8 a = ld8(src + k * step), c = ld8(src + k * step + D / 2);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      x1[j] += a[j];
+      x2[j] += c[j];
+    }
+  }
+  u16* dst;
+  if (h < Hq) {
+    dst = q + (tok * Hq + h) * D + i;
+  } else {
+    const int hk = h - Hq;
+    dst = (hk < Hkv ? kc : vc) +
+          (((long)b * Hkv + hk % Hkv) * max_seq + p) * D + i;
+  }
+  if (h < Hq + Hkv) {
+    const float* cs = cos_sin + ((long)p * (D / 2) + i) * 2;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float a = x1[j], c = x2[j];
+      x1[j] = a * cs[2 * j] - c * cs[2 * j + 1];
+      x2[j] = c * cs[2 * j] + a * cs[2 * j + 1];
+    }
+  }
+  s16x8 y1, y2;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    y1[j] = (short)f2bf(x1[j]);
+    y2[j] = (short)f2bf(x2[j]);
+  }
+  *(s16x8*)dst = y1;
+  *(s16x8*)(dst + D / 2) = y2;
+}
+
+// The sums of the parts, times a scale, added to float32.
+__global__ void __launch_bounds__(256)
+k_parts_add(float* __restrict__ out, const float* __restrict__ parts, int np,
+            long n4, float scale) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int k = 0; k < np; ++k) {
+    const f32x4 q = ((const f32x4*)parts)[k * n4 + i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += q[e];
+  }
+  f32x4 y = ((f32x4*)out)[i];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) y[e] = fmaf(scale, v[e], y[e]);
+  ((f32x4*)out)[i] = y;
+}
+
+}  // namespace
+
+extern "C" {
+
+// K % 64 == 0 and at least 64 a part, N % 4 == 0; rows of x (xs apart) and w on 16
+// bytes. xj: 32 rows of x a tile, 2 to 4; wide: 128 rows of w a tile, else 64.
+// swiglu: bfloat16 [M, N] of one part; else float32 [parts, M, N].
+void fei_rows(void* out, const void* x, long xs, const void* w, int M, int N,
+              int K, int swiglu, int xj, int wide, int parts,
+              hipStream_t stream) {
+#define ROWS(E)                                                            \
+  wide ? by_rows<4, 4, E>(xj, out, x, xs, w, M, N, K, parts, stream)       \
+       : by_rows<2, 3, E>(xj, out, x, xs, w, M, N, K, parts, stream)
+  if (swiglu) ROWS(ROWS_SWIGLU);
+  else ROWS(ROWS_PARTS);
+#undef ROWS
+}
+
+void fei_parts_norm(void* out, void* res, const float* parts, int np,
+                    const void* gain, int rows, int cols, float eps,
+                    hipStream_t stream) {
+  hipLaunchKernelGGL(k_parts_norm, dim3(rows), dim3(512), 0, stream, (u16*)out,
+                     (u16*)res, parts, np, (const u16*)gain, rows, cols, eps);
+}
+
+// parts [np][B * S][(Hq + 2 Hkv) * D], q [B * S][Hq][D]; D % 16 == 0, all on 16
+// bytes
+void fei_rope_kv_parts(void* q, const float* parts, int np, void* k_cache,
+                       void* v_cache, const float* cos_sin, const int* pos0,
+                       int B, int S, int Hq, int Hkv, int D, int max_seq,
+                       hipStream_t stream) {
+  const long rows = (long)B * S * (Hq + 2 * Hkv), units = rows * (D / 16);
+  hipLaunchKernelGGL(k_rope_kv_parts, dim3((units + 255) / 256), dim3(256), 0,
+                     stream, (u16*)q, parts, np, (u16*)k_cache, (u16*)v_cache,
+                     cos_sin, pos0, units, rows * D, S, Hq, Hkv, D, max_seq);
+}
+
+// out += scale * the sums; n % 4 == 0 values a part, all on 16 bytes
+void fei_parts_add(float* out, const float* parts, int np, long n, float scale,
+                   hipStream_t stream) {
+  hipLaunchKernelGGL(k_parts_add, dim3((n / 4 + 255) / 256), dim3(256), 0,
+                     stream, out, parts, np, n / 4, scale);
+}
+
+}  // extern "C"

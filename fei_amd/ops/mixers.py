@@ -14,6 +14,8 @@ from typing import Optional, Tuple
 import torch
 
 from fei_amd.ops import reference as ref
+from fei_amd.ops import rows as _rows
+from fei_amd.ops.rows import SKINNY_ROWS
 
 _c = ctypes
 _vp, _i, _f, _l = _c.c_void_p, _c.c_int, _c.c_float, _c.c_long
@@ -161,7 +163,6 @@ def _gemv_rows(T: int, K: int, t: torch.Tensor) -> bool:
 # What becomes of a skinny product's sums (csrc/fei_epilogue.h).
 (EPI_BF16, EPI_F32, EPI_RES, EPI_PARALLEL, EPI_RES_BF16, EPI_SWIGLU,
  EPI_GELU) = range(7)
-SKINNY_ROWS = 32     # most rows of the matrix-core tile for few rows
 
 
 def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -296,6 +297,9 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
         return x
     if not a.is_cuda or a.dtype == torch.float32:
         return x + mult * _mm_f32(a, w, None)
+    if _rows.add_ok(x, a, w):
+        _rows.add_product(x, a, w, mult)
+        return x
     return torch.addmm(x, a, w.t(), out_dtype=torch.float32, alpha=mult,
                        out=x)
 

@@ -405,3 +405,96 @@ def test_window_prefill_geometries(lib, dims, window, parts, scale):
         # (2^-9 an element, less in a row's norm) is what shows
         assert row_err(out[r:r + n], o) < 2.0 ** -8
     assert bool((out[~used.to(DEV)] == 7.0).all())
+
+
+# -- products of tens of rows ----------------------------------------------------
+
+@pytest.mark.parametrize("M,N,K", [
+    (33, 64, 64), (64, 72, 128), (65, 200, 192), (96, 128, 1024),
+    (97, 2048, 2048), (128, 4096, 4096), (129, 1000, 1088), (256, 136, 8192),
+    (75, 6144, 4096),
+])
+def test_product_parts(lib, M, N, K):
+    x, w = randbf(M, K + 64, seed=M)[:, :K], randbf(N, K, seed=N)
+    assert lib.rows_ok(M, w)
+    parts = lib.product_parts(x, w)
+    want = x.double() @ w.double().t()
+    # float32 sums of K products
+    assert row_err(parts.sum(0), want) < 2.0 ** -22 * K ** 0.5
+    h, gain = randbf(M, N, seed=3, scale=K ** 0.5), randbf(N, seed=4)
+    res = h.clone()
+    y = lib.add_norm_parts(parts, res, gain, 1e-5)
+    new = (h.double() + want)
+    assert row_err(res, new) < 2.0 ** -8
+    inv = (res.double().pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()
+    assert row_err(y, res.double() * inv * gain.double()) < 2.0 ** -8
+    if N >= 64 and K >= 4096:
+        from fei_amd.ops import rows
+        acc = torch.randn(M, N, device=DEV)
+        want = acc.double() + 0.3 * want
+        assert rows.add_ok(acc, x, w)
+        rows.add_product(acc, x, w, 0.3)
+        assert row_err(acc, want) < 2.0 ** -22 * K ** 0.5
+
+
+@pytest.mark.parametrize("M,I,K", [
+    (33, 8, 64), (64, 64, 256), (75, 1000, 512), (128, 14336, 128),
+    (256, 8192, 192), (200, 72, 1024),
+])
+def test_rows_swiglu(lib, M, I, K):
+    from fei_amd.ops import rows
+    x, w = randbf(M, K, seed=M), randbf(2 * I, K, seed=I, scale=K ** -0.5)
+    assert rows.swiglu_ok(M, x, w)
+    gu = x.double() @ w.double().t()
+    want = torch.nn.functional.silu(gu[:, :I]) * gu[:, I:]
+    assert row_err(lib.gemv_swiglu(x, w), want) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,D", [(1, 33, 4, 2, 128), (3, 17, 3, 1, 64),
+                                          (2, 40, 2, 2, 16), (1, 75, 32, 8, 128)])
+def test_rope_kv_parts(lib, B, S, Hq, Hkv, D):
+    """Against the kernel for whole products."""
+    T, W = B * S, (Hq + 2 * Hkv) * D
+    parts = torch.randn(3, T, W, device=DEV)
+    table = torch.randn(200, D // 2, 2, device=DEV)
+    pos0 = torch.arange(B, device=DEV, dtype=torch.int32) * 7
+    kc, vc = (torch.zeros(B, Hkv, 200, D, dtype=torch.bfloat16, device=DEV)
+              for _ in range(2))
+    kr, vr = kc.clone(), vc.clone()
+    q = lib.rope_kv_parts(parts, S, Hq, kc, vc, pos0, table)
+    qkv = parts.sum(0).bfloat16()
+    q0, k0, v0 = (qkv[:, a * D:b * D].view(B, S, b - a, D) for a, b in (
+        (0, Hq), (Hq, Hq + Hkv), (Hq + Hkv, Hq + 2 * Hkv)))
+    lib.rope_kv_prefill(q0, k0, v0, kr, vr, pos0, table)
+    # there the sums are rounded before they are turned, here only after
+    for a, b in ((q, q0), (kc, kr), (vc, vr)):
+        d = (a.double() - b.double()).abs().amax()
+        assert d <= 2.0 ** -7 * b.double().abs().amax()
+    assert torch.equal(vc, vr)
+
+
+@pytest.mark.parametrize("B,S", [(1, 33), (2, 20), (1, 128), (2, 65), (1, 200)])
+def test_prompt_in_parts_matches_whole_products(lib, B, S):
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+    spec = dataclasses.replace(get_spec("llama3-1b"), num_layers=2,
+                               vocab_size=512)
+    m = LlamaModel(spec, torch.device(DEV), torch.bfloat16, seed=1,
+                   max_seq_len=256)
+    toks = torch.randint(0, 512, (B, S), device=DEV)
+    pos0 = torch.arange(B, dtype=torch.int32, device=DEV) * 3
+
+    def run(parts):
+        if not parts:
+            m.rows_in_parts = lambda T, caches: False
+        kc, vc = ([torch.zeros(B, spec.num_kv_heads, 256, m.D,
+                               dtype=torch.bfloat16, device=DEV)
+                   for _ in range(2)] for _ in range(2))
+        return m.forward_prefill(toks, pos0, kc, vc, all_positions=True), kc, vc
+    assert m.rows_in_parts(B * S, [])
+    (a, ka, va), (b, kb, vb) = run(True), run(False)
+    # a rounding of 2^-9 here and there, through two layers
+    assert row_err(a, b.double()) < 2.0 ** -5
+    for x, y in zip(ka + va, kb + vb):
+        assert row_err(x.flatten(), y.double().flatten()) < 2.0 ** -6
