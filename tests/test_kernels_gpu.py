@@ -498,3 +498,21 @@ def test_prompt_in_parts_matches_whole_products(lib, B, S):
     assert row_err(a, b.double()) < 2.0 ** -5
     for x, y in zip(ka + va, kb + vb):
         assert row_err(x.flatten(), y.double().flatten()) < 2.0 ** -6
+
+
+@pytest.mark.parametrize("B,S,lengths", [(1, 4, None), (1, 24, None),
+                                         (4, 8, [8, 1, 3, 5]), (2, 16, [16, 9]),
+                                         (32, 1, None)])
+def test_encoder_layers_from_one_call(lib, B, S, lengths):
+    from fei_amd.models.bge import BgeEncoder
+    m = BgeEncoder(device=torch.device(DEV))
+    ids = torch.randint(0, 1000, (B, S), device=DEV)
+    n = None if lengths is None else torch.tensor(lengths, device=DEV)
+    got = m.encode_ids(ids, n)
+    before, lib.encoder_layers = lib.encoder_layers, lambda *a: None
+    try:
+        want = m.encode_ids(ids, n)
+    finally:
+        lib.encoder_layers = before
+    # the same kernels in the same order
+    assert torch.equal(got, want)
