@@ -506,19 +506,36 @@ void fei_moe_plan(int* order, int* place, int* tiles, int* count,
                      tiles, count, ids, n, E, top, rows, max_tiles);
 }
 
-// bits: 1 = float32, 2 = tiles of 128 slots (else 32)
+// bits: 1 = float32, 2 = tiles of 128 slots (else 32); likely: tiles if all experts
+// have as many slots
 void fei_moe_gemm(void* out, const void* x, const void* w, const int* order,
-                  const int* tiles, const int* count, int max_tiles, int N,
-                  int K, int act, int bits, hipStream_t stream) {
+                  const int* tiles, const int* count, int max_tiles,
+                  int likely, int N, int K, int act, int bits,
+                  hipStream_t stream) {
   if (bits & 2) {
-    // 192 columns a block unless they are wasted or leave CUs without a block
-    const int c6 = (N + 191) / 192, c4 = (N + 127) / 128;
-    if (c6 * max_tiles >= 512 && c6 * 192 * 10 <= c4 * 128 * 11)
-      launch_big<6, 2>((u16*)out, (const u16*)x, (const u16*)w, order, tiles,
-                       count, max_tiles, N, K, act, stream);
-    else
-      launch_big<4, 2>((u16*)out, (const u16*)x, (const u16*)w, order, tiles,
-                       count, max_tiles, N, K, act, stream);
+// 128 or 192 columns a block, with two buffers (two blocks a CU) or three
+    // (one, whose loads are further ahead: 0.7 of the time where every CU has
+    // one block to do). What a round of blocks takes goes with the rows that a
+    // step loads, 32 (WI + 4). 6824 slots of 16 experts, 64 tiles: 768 columns
+    // of 2048 in 30.7 us (192, three buffers; others 40 to 45), 2048 of 768 in
+    // 39.6 (128, two; 43 to 46). 2800 slots: 22.1 (128, three; 28 to 36) and
+    // 22.5 (128, two; 24 to 30).
+    auto cost = [&](int wi, int per_round) {
+      const long blocks = (long)likely * ((N + 32 * wi - 1) / (32 * wi));
+      return ((blocks + per_round - 1) / per_round) * (wi + 4) *
+             (per_round == 256 ? 7 : 10);
+    };
+    const long c42 = cost(4, 512), c62 = cost(6, 512), c43 = cost(4, 256),
+               c63 = cost(6, 256);
+    const long least = min(min(c42, c62), min(c43, c63));
+#define BIG(WI, S)                                                          \
+  launch_big<WI, S>((u16*)out, (const u16*)x, (const u16*)w, order, tiles,  \
+                    count, max_tiles, N, K, act, stream)
+    if (c42 == least) BIG(4, 2);
+    else if (c62 == least) BIG(6, 2);
+    else if (c43 == least) BIG(4, 3);
+    else BIG(6, 3);
+#undef BIG
     return;
   }
   const dim3 grid((N + 63) / 64, max_tiles);

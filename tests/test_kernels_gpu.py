@@ -516,3 +516,42 @@ def test_encoder_layers_from_one_call(lib, B, S, lengths):
         lib.encoder_layers = before
     # the same kernels in the same order
     assert torch.equal(got, want)
+
+
+# -- grouped products ------------------------------------------------------------
+
+@pytest.mark.parametrize("T,E,top,N,K", [
+    (300, 4, 2, 512, 256),       # 128 columns, three buffers
+    (2000, 16, 4, 768, 128),     # 192, three
+    (2000, 16, 4, 2048, 64),     # 128, two
+    (2000, 16, 4, 1344, 192),    # 192, two
+    (400, 3, 1, 20, 320),        # a part of a block, steps that do not divide
+])
+def test_moe_gemm_blocks(lib, T, E, top, N, K):
+    """Each size of block of the grouped product, with experts that have more
+    and fewer rows than their share."""
+    from fei_amd.ops import mixers as mx
+    n = T * top
+    x, w = randbf(T, K, seed=T), randbf(E, N, K, seed=N, scale=K ** -0.5)
+    g = torch.Generator(device=DEV).manual_seed(2)
+    score = torch.randn(T, E, generator=g, device=DEV)
+    score[:, 0] += 0.3
+    ids = score.topk(top, 1).indices.int().contiguous()
+    most = min(n, n // 128 + E)
+    likely = min(most, E * -(-n // (E * 128)))
+    order, place = (torch.empty(n, dtype=torch.int32, device=DEV)
+                    for _ in range(2))
+    tiles = torch.empty(most, 3, dtype=torch.int32, device=DEV)
+    count = torch.empty(1, dtype=torch.int32, device=DEV)
+    p, st, lb = mx._p, mx._stream(), mx._lib()
+    lb.fei_moe_plan(p(order), p(place), p(tiles), p(count), p(ids), n, E, top,
+                    128, most, st)
+    out = torch.full((n, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    lb.fei_moe_gemm(p(out), p(x), p(w), p(order), p(tiles), p(count), most,
+                    likely, N, K, 0, 2, st)
+    want = torch.empty(T, top, N, dtype=torch.float64, device=DEV)
+    for e in range(E):
+        t, k = (ids == e).nonzero(as_tuple=True)
+        want[t, k] = x[t].double() @ w[e].double().t()
+    got = out[place.view(T, top).long()]
+    assert row_err(got.view(n, N), want.view(n, N)) < 2.0 ** -8
