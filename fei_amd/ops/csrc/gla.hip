@@ -126,17 +126,18 @@ __device__ __forceinline__ f32x4 ld4(const T* p, int lim, int vec) {
 }
 
 // Values of columns e0 .. e0+NE-1, transposed, zero past the chunk and past
-// vdim. A thread turns 4 tokens x 4 columns.
+// vdim. A thread (tid, of 256) turns 4 tokens x 4 columns.
 template <typename T, int NE>
-__device__ __forceinline__ void stage_vt(float* vt, const T* __restrict__ proj,
-                                         long ps, const Gla& g, int h, int row0,
-                                         int n, int e0, int vec) {
+__device__ __forceinline__ void stage_vt(float* vt, int tid,
+                                         const T* __restrict__ proj, long ps,
+                                         const Gla& g, int h, int row0, int n,
+                                         int e0, int vec) {
   constexpr int Q = NE / 4;
   constexpr int NU = (Q * 16 + 255) / 256;
   f32x4 x[NU][4];
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int i = threadIdx.x + u * 256;
+    const int i = tid + u * 256;
     const int e = i % Q * 4, t = i / Q * 4;
     const int lim = i < Q * 16 ? g.vdim - e0 - e : 0;
 #pragma unroll
@@ -147,7 +148,7 @@ __device__ __forceinline__ void stage_vt(float* vt, const T* __restrict__ proj,
   }
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
-    const int i = threadIdx.x + u * 256;
+    const int i = tid + u * 256;
     const int e = i % Q * 4, t = i / Q * 4;
     if (i < Q * 16)
 #pragma unroll
@@ -195,7 +196,7 @@ k_gla_state(float* __restrict__ U, const float* __restrict__ G,
         *(f32x4*)(kt + tr_at(d + c, t >> 2)) = v;
       }
   }
-  stage_vt<T, 64>(vt, proj, ps, g, h, row0, n, e0, vec);
+  stage_vt<T, 64>(vt, threadIdx.x, proj, ps, g, h, row0, n, e0, vec);
   __syncthreads();
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int l15 = lane & 15, lg = lane >> 4;
@@ -349,21 +350,28 @@ k_gla_scores(float* __restrict__ A, const float* __restrict__ G,
   }
 }
 
-// o = (q exp(G)) S + A V, head norm, gate. grid (chunks, heads); wave w owns
-// 16 tokens and all of vdim, which goes by tiles of 32 columns held in LDS.
-// DK = ceil(dim / 32), NV = ceil(vdim / 32), both rounded up.
-template <typename T, int DK, int NV>
-__global__ void __launch_bounds__(256)
+// o = (q exp(G)) S + A V, head norm, gate. grid (chunks, heads). vdim goes by
+// tiles of 32 columns held in LDS, NG of them at a time, each by four waves of 16
+// tokens. DK = ceil(dim / 32), NV = ceil(vdim / 32), both rounded up.
+//
+// Bound by the latency of a tile's loads, with few blocks on the chip (22 chunks x
+// 8 heads at 1297 tokens): all tiles one after the other took 55 us (dim 128,
+// vdim 256), four at a time 41, a quarter of it the float32 matrix units.
+template <typename T, int DK, int NV, int NG>
+__global__ void __launch_bounds__(256 * NG)
 k_gla_out(T* __restrict__ out, long os, const float* __restrict__ S,
           const float* __restrict__ A, const float* __restrict__ G,
           const T* __restrict__ proj, long ps, const float* __restrict__ nw,
           const int* __restrict__ chunks, Gla g, float eps, int vec) {
-  constexpr int DS = DK * 32 + 4;
-  __shared__ __align__(16) float st[32 * DS];
-  __shared__ __align__(16) float vt[32 * CH];
+  constexpr int DS = DK * 32 + 4, TILE = 32 * (DS + CH);
+  extern __shared__ __align__(16) float lds[];      // [NG][TILE]
+  __shared__ float part[NG][CH];
   const int row0 = chunks[blockIdx.x * 3 + 1], n = chunks[blockIdx.x * 3 + 2];
   const int h = blockIdx.y;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int tid = threadIdx.x & 255, grp = threadIdx.x >> 8;
+  float* st = lds + grp * TILE;
+  float* vt = st + 32 * DS;
+  const int w = tid >> 6, lane = tid & 63;
   const int l15 = lane & 15, lg = lane >> 4;
   const float scale = 1.f / sqrtf((float)g.dim);
   const float* s0 = S + ((long)blockIdx.x * g.heads + h) * g.vdim * g.dim;
@@ -389,27 +397,31 @@ k_gla_out(T* __restrict__ out, long os, const float* __restrict__ S,
     aa[k] = ld8(A + (((long)blockIdx.x * g.heads + h) * CH + t) * CH + k * 32 +
                 8 * lg);
 
-  f32x4 o[NV * 2];
+  constexpr int NT = NV / NG;              // tiles of a group
+  f32x4 o[NT * 2];
 #pragma unroll
-  for (int v = 0; v < NV; ++v) {
-    const int e0 = v * 32;
-    if (e0 < g.vdim) {                     // uniform
-      __syncthreads();
+  for (int v = 0; v < NT; ++v) {
+    const int e0 = (v * NG + grp) * 32;
+    o[v * 2] = o[v * 2 + 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    if (e0 < g.vdim) {                     // uniform in the group
       f32x4 x[DK];
 #pragma unroll
       for (int u = 0; u < DK; ++u) {
-        const int i = threadIdx.x + u * 256;
+        const int i = tid + u * 256;
         const int e = i / (DK * 8), d = i % (DK * 8) * 4;
         x[u] = ld4<float>(s0 + (long)(e0 + e) * g.dim + d,
                           e0 + e < g.vdim ? g.dim - d : 0, vec);
       }
 #pragma unroll
       for (int u = 0; u < DK; ++u) {
-        const int i = threadIdx.x + u * 256;
+        const int i = tid + u * 256;
         *(f32x4*)(st + i / (DK * 8) * DS + i % (DK * 8) * 4) = x[u];
       }
-      stage_vt<T, 32>(vt, proj, ps, g, h, row0, n, e0, vec);
-      __syncthreads();
+      stage_vt<T, 32>(vt, tid, proj, ps, g, h, row0, n, e0, vec);
+    }
+    __syncthreads();
+    if (e0 < g.vdim) {
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -421,24 +433,30 @@ k_gla_out(T* __restrict__ out, long os, const float* __restrict__ S,
           acc = mma(aa[k], tr_ld8(vt, c * 16 + l15, k * 32 + 8 * lg), acc);
         o[v * 2 + c] = acc;
       }
-    } else {
-      o[v * 2] = o[v * 2 + 1] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
   }
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     float ss = 0.f;                        // columns past vdim are zero
 #pragma unroll
-    for (int c = 0; c < NV * 2; ++c) ss = fmaf(o[c][r], o[c][r], ss);
+    for (int c = 0; c < NT * 2; ++c) ss = fmaf(o[c][r], o[c][r], ss);
     ss = row16_sum(ss);
+    if (l15 == 0) part[grp][w * 16 + 4 * lg + r] = ss;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
     const int tr = w * 16 + 4 * lg + r;
     if (tr >= n) continue;
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < NG; ++k) ss += part[k][tr];
     const float inv = 1.f / sqrtf(ss / (float)g.vdim + eps);
     const T* gate = proj + (long)(row0 + tr) * ps + g.g_off() + h * g.vdim;
     T* dst = out + (long)(row0 + tr) * os + h * g.vdim;
 #pragma unroll
-    for (int c = 0; c < NV * 2; ++c) {
-      const int e = c * 16 + l15;
+    for (int c = 0; c < NT * 2; ++c) {
+      const int e = ((c >> 1) * NG + grp) * 32 + (c & 1) * 16 + l15;
       if (e < g.vdim) {
         const float gv = El<T>::ld(gate[e]);
         dst[e] = El<T>::st(o[c][r] * inv * nw[e] * gv * sigmoid_f(gv));
@@ -558,6 +576,24 @@ void launch_state(float* U, const float* G, const T* proj, long ps,
                      stream, U, G, proj, ps, chunks, g, vec);
 }
 
+template <typename T, int DK, int NV>
+void launch_out(T* out, long os, const float* U, const float* A, const float* G,
+                const T* proj, long ps, const float* nw, const int* chunks,
+                int n, Gla g, float eps, int vec, hipStream_t stream) {
+  // four tiles at a time, two where there are no more or LDS has no room
+  constexpr int NG = NV >= 4 && DK <= 4 ? 4 : 2;
+  constexpr int lds = NG * 32 * (DK * 32 + 4 + CH) * 4;
+  static bool set = lds <= 65536;
+  if (!set) {
+    (void)hipFuncSetAttribute((const void*)k_gla_out<T, DK, NV, NG>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    set = true;
+  }
+  hipLaunchKernelGGL((k_gla_out<T, DK, NV, NG>), dim3(n, g.heads),
+                     dim3(256 * NG), lds, stream, out, os, U, A, G, proj, ps,
+                     nw, chunks, g, eps, vec);
+}
+
 template <typename T>
 void run_gla_prefill(T* out, long os, const T* proj, long ps, const float* a2,
                      const float* bias, const float* nw, float* states,
@@ -579,10 +615,9 @@ void run_gla_prefill(T* out, long os, const T* proj, long ps, const float* a2,
                      stream, U, G, states, chunks, spans, slots, g);
   hipLaunchKernelGGL(k_gla_scores<T>, dim3(n, g.heads), dim3(256), 0, stream,
                      A, G, proj, ps, chunks, g, vec);
-  const dim3 go(n, g.heads);
 #define OUT(DK, NV)                                                         \
-  hipLaunchKernelGGL((k_gla_out<T, DK, NV>), go, dim3(256), 0, stream, out, \
-                     os, U, A, G, proj, ps, nw, chunks, g, eps, vec)
+  launch_out<T, DK, NV>(out, os, U, A, G, proj, ps, nw, chunks, n, g, eps,  \
+                        vec, stream)
 #define BY_NV(DK)                           \
   do {                                      \
     if (g.vdim <= 64) OUT(DK, 2);           \

@@ -555,3 +555,47 @@ def test_moe_gemm_blocks(lib, T, E, top, N, K):
         want[t, k] = x[t].double() @ w[e].double().t()
     got = out[place.view(T, top).long()]
     assert row_err(got.view(n, N), want.view(n, N)) < 2.0 ** -8
+
+
+# -- gated linear attention over prompts ---------------------------------------------
+
+@pytest.mark.parametrize("dim,vdim", [
+    (16, 40), (32, 100), (64, 256), (128, 300), (128, 33), (136, 64),
+    (200, 256), (256, 512), (30, 510), (128, 256),
+])
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-5),
+                                       (torch.bfloat16, 2.0 ** -8)])
+def test_gla_prompt_tiles(lib, dim, vdim, dtype, tol):
+    """Each count of column tiles a block takes at once, the last ones in part,
+    against the recurrence token by token on the CPU. float32: sums of 256
+    terms and 16 ulp of the exponentials; bfloat16: one rounding."""
+    from types import SimpleNamespace as NS
+    from fei_amd.ops import mixers as mx
+    H, rank = 2, 8
+    parts = [(0, 70, 0), (70, 64, 0), (134, 1, 0)]
+    T = 135
+    g = torch.Generator().manual_seed(dim + vdim)
+    rand = lambda *s: torch.randn(*s, generator=g)
+    m = NS(heads=H, dim=dim, vdim=vdim, gate_rank=rank, tau=8.0)
+    w = NS(a2=rand(H * dim, rank) * 0.3, bias=rand(H * dim),
+           norm=rand(vdim).abs() + 0.5, eps=1e-5)
+    proj = rand(T, 2 * H * dim + 2 * H * vdim + rank).to(dtype)
+    chunks, spans = [], []
+    for i, (row, n, pos0) in enumerate(parts):
+        spans.append([len(chunks), -(-n // 64), pos0, i])
+        chunks += [[i, row + a, min(64, n - a)] for a in range(0, n, 64)]
+
+    def run(dev):
+        up = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)
+        batch = NS(portions=parts, n_dec=0, slots=up([2, 0, 1]),
+                   chunk_plan=lambda: (up(chunks), up(spans)))
+        out = torch.zeros(T, H * vdim, dtype=dtype, device=dev)
+        states = torch.ones(4, H, vdim, dim, device=dev)
+        mx.gla_prefill(proj.to(dev), out, m,
+                       NS(**{k: v.to(dev) if torch.is_tensor(v) else v
+                             for k, v in vars(w).items()}), batch, states)
+        return out.cpu(), states.cpu()
+    (got, s), (want, s0) = run(DEV), run("cpu")
+    assert row_err(got, want.double()) < tol * (1 if dtype == torch.float32 else 2)
+    assert row_err(s[:3].flatten(1), s0[:3].double().flatten(1)) < 2e-5
+    assert bool((s[3] == 1).all())
