@@ -123,13 +123,13 @@ class PagedSessionManager:
             with torch.cuda.stream(side):
                 for _ in range(2):
                     lg = self._forward_paged(tk, ps, bt)
-                    tk.copy_(lg.argmax(dim=-1))
+                    tk.copy_(ops.argmax(lg))
                     ps.add_(1)
             torch.cuda.current_stream().wait_stream(side)
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g):
                 lg = self._forward_paged(tk, ps, bt)
-                tk.copy_(lg.argmax(dim=-1))
+                tk.copy_(ops.argmax(lg))
                 ps.add_(1)
             torch.cuda.synchronize()
         except Exception as e:                      # pragma: no cover - GPU
@@ -243,7 +243,7 @@ class PagedSessionManager:
             steps = []
             for _ in range(chunk):
                 logits = self._forward_paged(token, pos, table)
-                token = logits.argmax(dim=-1)
+                token = ops.argmax(logits)
                 steps.append(token)
                 pos = pos + 1
             allt = torch.stack(steps, dim=1).tolist()      # the one sync
@@ -409,7 +409,7 @@ class StepSessionManager(PagedSessionManager):
         for e in entries:
             self.sessions[e.seq].pos += len(e.tokens)
         if emits:
-            for s, t in zip(emits, logits.argmax(dim=-1).tolist()):
+            for s, t in zip(emits, ops.argmax(logits).tolist()):
                 self._emit(s, int(t))
         return len(entries)
 
@@ -444,7 +444,7 @@ class StepSessionManager(PagedSessionManager):
         steps = []
         for _ in range(n):
             logits = self.model.forward(batch, self.runner.cache)
-            batch.tokens = logits.argmax(dim=-1)
+            batch.tokens = ops.argmax(logits)
             batch.pos += 1
             steps.append(batch.tokens)
         rows = torch.stack(steps, dim=1).tolist()

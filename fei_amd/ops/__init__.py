@@ -74,6 +74,7 @@ def _try_load() -> None:
                              _vp, _vp]
     lib.fei_skinny.argtypes = ([_vp] * 3 + [_i] * 4 + [_vp, _f, _f, _i, _i] +
                                [_vp, _vp, _l] + [_vp] * 3 + [_i, _f, _vp, _vp])
+    lib.fei_argmax.argtypes = [_vp] * 3 + [_i] * 4 + [_vp]
     lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
                                        [_f, _f, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
@@ -386,6 +387,20 @@ def swiglu(gate_up: torch.Tensor,
     if out is None:
         out = torch.empty(*gu.shape[:-1], inter, dtype=gu.dtype, device=gu.device)
     lib.fei_swiglu(_ptr(out), _ptr(gu), rows, inter, _stream())
+    return out
+
+
+def argmax(x: torch.Tensor) -> torch.Tensor:
+    """x.argmax(-1) of rows [B, V]: the first of the largest values."""
+    if not (x.is_cuda and x.dim() == 2 and x.is_contiguous() and x.numel()
+            and x.dtype in (torch.bfloat16, torch.float32)):
+        return x.argmax(dim=-1)
+    B, V = x.shape
+    chunks = max(1, min(64, 512 // B, -(-V // 2048)))
+    out = torch.empty(B, dtype=torch.int64, device=x.device)
+    part = torch.empty(B, chunks, dtype=torch.int64, device=x.device)
+    require_lib().fei_argmax(_ptr(out), _ptr(part), _ptr(x), B, V, chunks,
+                             1 if x.dtype == torch.float32 else 0, _stream())
     return out
 
 

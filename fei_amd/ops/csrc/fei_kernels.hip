@@ -397,6 +397,82 @@ void fei_advance(int* pos, int* step, int B, int max_pos,
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
+// First place of the largest value of each row (NaN above all, as in torch's
+// argmax): ordered bits above the inverted place, so that one maximum of whole
+// numbers decides. A row in chunks, a block each, then a wave per row. 20 x 128256
+// bfloat16: 4.6 + 4.5 us, torch 41.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ u64 rank_of(float v, int i) {
+  u32 u = __builtin_bit_cast(u32, v + 0.f);          // -0 counts as 0
+  u = v != v ? ~0u : u & 0x80000000u ? ~u : u | 0x80000000u;
+  return (u64)u << 32 | (u32)~i;
+}
+__device__ __forceinline__ u64 wave_max(u64 v) {
+#pragma unroll
+  for (int off = 32; off; off >>= 1) {
+    const u64 o = __shfl_xor(v, off);
+    v = o > v ? o : v;
+  }
+  return v;
+}
+
+template <typename T, bool VEC>
+__global__ void __launch_bounds__(256)
+k_argmax_chunk(u64* __restrict__ part, const T* __restrict__ x, int cols,
+               int per) {
+  constexpr int E = VEC ? 16 / sizeof(T) : 1;
+  const T* row = x + (long)blockIdx.y * cols;
+  const int lo = blockIdx.x * per, hi = min(cols, lo + per);
+  u64 best = 0;
+#pragma unroll 4
+  for (int i = lo + threadIdx.x * E; i < hi; i += 256 * E) {
+    T v[E];
+    __builtin_memcpy(v, VEC ? __builtin_assume_aligned(row + i, 16) : row + i,
+                     sizeof(v));
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const u64 r = rank_of(logit(v[j]), i + j);
+      best = r > best ? r : best;
+    }
+  }
+  __shared__ u64 red[4];
+  best = wave_max(best);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = best;
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int i = 1; i < 4; ++i) best = red[i] > best ? red[i] : best;
+  part[(long)blockIdx.y * gridDim.x + blockIdx.x] = best;
+}
+
+__global__ void __launch_bounds__(64)
+k_argmax_row(long* __restrict__ out, const u64* __restrict__ part, int chunks) {
+  const u64* p = part + (long)blockIdx.x * chunks;
+  u64 best = 0;
+  for (int i = threadIdx.x; i < chunks; i += 64) best = p[i] > best ? p[i] : best;
+  best = wave_max(best);
+  if (threadIdx.x == 0) out[blockIdx.x] = (u32)~(u32)best;
+}
+
+// x [rows, cols] -> out [rows]; part [rows, chunks]
+extern "C" void fei_argmax(long* out, u64* part, const void* x, int rows,
+                           int cols, int chunks, int f32, hipStream_t stream) {
+  const int per = (cols + chunks * 8 - 1) / (chunks * 8) * 8;
+  const dim3 grid(chunks, rows);
+  const bool vec = cols % 8 == 0 && (uintptr_t)x % 16 == 0;
+#define GO(T, V)                                                           \
+  hipLaunchKernelGGL((k_argmax_chunk<T, V>), grid, dim3(256), 0, stream,   \
+                     part, (const T*)x, cols, per)
+  if (f32) {
+    if (vec) GO(float, true); else GO(float, false);
+  } else {
+    if (vec) GO(u16, true); else GO(u16, false);
+  }
+#undef GO
+  hipLaunchKernelGGL(k_argmax_row, dim3(rows), dim3(64), 0, stream, out, part,
+                     chunks);
+}
+
+// ---------------------------------------------------------------------------
 // One-pass sampler for small B: grid (B), block 1024 = 16 waves streaming
 // the whole vocab row; replaces the partial+final pair (one node, no
 // workspace round trip).

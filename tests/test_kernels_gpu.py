@@ -599,3 +599,24 @@ def test_gla_prompt_tiles(lib, dim, vdim, dtype, tol):
     assert row_err(got, want.double()) < tol * (1 if dtype == torch.float32 else 2)
     assert row_err(s[:3].flatten(1), s0[:3].double().flatten(1)) < 2e-5
     assert bool((s[3] == 1).all())
+
+
+# -- largest values ----------------------------------------------------------------
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("B,V", [(1, 1), (3, 7), (20, 128256), (2, 2049),
+                                 (600, 64), (5, 50257)])
+def test_argmax_is_the_first(lib, dtype, B, V):
+    """Ties, infinities, NaN and zeros of both signs."""
+    g = torch.Generator(device=DEV).manual_seed(V)
+    x = torch.randn(B, V, generator=g, device=DEV).to(dtype)
+    rows = [x, (x * 2).round(), -x.abs() * 0.0, torch.full_like(x, -float("inf"))]
+    y = x.clone()
+    y[:, V // 2:] = float("nan")
+    z = x.clone()
+    z[:, V // 3] = float("inf")
+    for t in (*rows, y, z):
+        got = lib.argmax(t)
+        assert got.dtype == torch.int64
+        # argmax of the CPU: the first of equals, NaN above all
+        assert torch.equal(got.cpu(), t.float().cpu().argmax(-1))
