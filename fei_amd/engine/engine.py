@@ -1,7 +1,7 @@
 """LocalEngine: the MI355X inference engine behind the Assistant.
 
 The decode step (the agent-tok/s hot path) is fully device-resident.
-Up to three rows (tensor parallel: never) a layer is six launches:
+Few rows (tensor parallel: never) are six launches a layer:
   QKV GEMV (norm inside) -> split-K decode attention (in-kernel RoPE +
   KV-append) -> combine -> O GEMV (adds to the residual) -> gate/up GEMV
   (norm and SwiGLU inside) -> down GEMV (adds to the residual)

@@ -211,10 +211,9 @@ class LlamaModel:
         GEMV kernels — norm in QKV/gate-up, residual add in O/down. On the
         GPU always so for few rows; there it chooses fp8 weights at batch 1,
         if the model has some."""
-        # Few rows: the products add to the residual and make the SwiGLU, up
-        # to three rows the norms too: six or eight launches a layer for nine
-        # or ten (8B, batch 1: 3.54 -> 3.15 ms a step). On the CPU the
-        # caller's choice stays.
+        # Few rows: the products add to the residual, make the SwiGLU and take
+        # rows under a norm: six launches a layer for nine or ten (8B, batch 1:
+        # 3.54 -> 3.15 ms a step). On the CPU the caller's choice stays.
         B = token.shape[0]
         if self.fused_rows(B) or (fused_norm and B == 1 and self.tp_size == 1):
             return self._forward_decode_fused_norm(

@@ -593,7 +593,7 @@ def _product(x: torch.Tensor, w: torch.Tensor, rows_out: int) -> Optional[str]:
     M = x.numel() // K if K else 0
     if not x.is_cuda or not M or not rows_out:
         return None
-    if _mixers.skinny_ok(M, K, x, w):
+    if _mixers.skinny_ok(M, K, x, w, 2):
         return "skinny"
     return "gemv" if _gemv_ok(M, K) else None
 
@@ -603,7 +603,7 @@ def own_product(M: int, w: torch.Tensor) -> bool:
     library's kernels, which add to a residual and make a SwiGLU without a
     launch of its own."""
     N, K = w.shape
-    return w.is_cuda and N > 0 and (_mixers.skinny_ok(M, K, w, w) or
+    return w.is_cuda and N > 0 and (_mixers.skinny_ok(M, K, w, w, 2) or
                                     _gemv_ok(M, K))
 
 

@@ -2,7 +2,7 @@
 // out[M, N] = x[M, K] @ W[N, K]^T, F.linear's layout.
 //
 // k_gemv streams the weights, bfloat16 or fp8 (e4m3fn, a scale per row), through
-// the vector units; from M = 4 on k_skinny (below) uses the matrix units.
+// the vector units; from M = 2 on k_skinny (below) uses the matrix units.
 #include <type_traits>
 
 #include "fei_epilogue.h"
@@ -355,7 +355,7 @@ void fei_prefetch(const void* w, long bytes, void* sink, int n_blocks,
 }  // extern "C"
 
 // ---------------------------------------------------------------------------
-// The same for 4 to 64 rows on the matrix units. The block's four waves share K;
+// The same for 2 to 64 rows on the matrix units. The block's four waves share K;
 // a wave streams 16 RT rows of w and the rows of x, 64 of K a stage, S stages
 // ahead, by direct loads into LDS of its own, so that nothing but the sum at the
 // end has a barrier. A load takes 8 whole lines of 128 bytes (fragments read

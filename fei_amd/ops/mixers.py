@@ -165,11 +165,15 @@ def _gemv_rows(T: int, K: int, t: torch.Tensor) -> bool:
  EPI_GELU) = range(7)
 
 
-def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
+def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor,
+              least: int = 3) -> bool:
     """Rows and sizes that the matrix-core tile for few rows takes: its loads
-    are of 16 bytes, 128 a row. Under 4 rows the vector units are faster; beyond
-    32 the tile's repeated reads of x cost more than the library's."""
-    return (4 <= T <= SKINNY_ROWS and K > 0 and K % 64 == 0
+    are of 16 bytes, 128 a row. From 3 rows on it beats the vector units (whole
+    decoding steps, 3 rows: 3.24 ms for 4.75 on 8B, 0.79 for 1.12 on 1B), from 2
+    (``least``) where it also makes the norm or adds to the residual (3.01 for
+    3.54, 0.84 for 0.88); beyond 32 its repeated reads of x cost more than the
+    library's."""
+    return (least <= T <= SKINNY_ROWS and K > 0 and K % 64 == 0
             and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous()
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 

@@ -203,7 +203,7 @@ def test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, splits, lens):
 
 # -- products of few rows on the matrix units ------------------------------------
 
-@pytest.mark.parametrize("M", [4, 8, 9, 17, 25, 32])
+@pytest.mark.parametrize("M", [3, 4, 8, 9, 17, 25, 32])
 @pytest.mark.parametrize("N,K", [
     (16, 64),              # one stage, three waves without any
     (20, 320),             # five stages for four waves, a part of a tile
