@@ -76,7 +76,7 @@ def _try_load() -> None:
                                [_vp, _vp, _l] + [_vp] * 3 + [_i, _f, _vp, _vp])
     lib.fei_argmax.argtypes = [_vp] * 3 + [_i] * 4 + [_vp]
     lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
-                                       [_f, _f, _vp])
+                                       [_f, _f, _i, _vp, _vp, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -837,6 +837,13 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
     return gelu(y) if act_gelu else y
 
 
+# Rows up to which all layers are launched from one call; one by one, with the
+# library's products, they take 1.6 ms and more from Python (12 layers of 768), of
+# which the GPU works a part: 100 rows 820 us, 512 956, 1000 981. Beyond, the
+# library's products are the faster ones and the GPU is never idle.
+ENCODER_ROWS = 1024
+
+
 def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
                    pos0: torch.Tensor, kv_len: torch.Tensor,
                    eps: float) -> Optional[torch.Tensor]:
@@ -847,7 +854,9 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
     B, S, C = h.shape
     M, HD = B * S, heads * dim
     if not (h.is_cuda and h.is_contiguous() and dim in (64, 128)
-            and _mixers.skinny_ok(M, C, h, h) and HD % 64 == inner % 64 == 0
+            and h.dtype == torch.bfloat16 and 2 < M <= ENCODER_ROWS
+            and C % 64 == HD % 64 == inner % 64 == 0
+            and h.data_ptr() % 16 == 0
             and all(t.dtype == torch.bfloat16 and t.is_contiguous()
                     for t in weights)):
         return None
@@ -859,10 +868,17 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
         return torch.empty(M, n, dtype=h.dtype, device=h.device)
     h1, tmp = rows(C), rows(C)
     qkv, att, mid = rows(3 * HD), rows(HD), rows(inner)
+    splits = _prefill_splits(B * heads, S, S)
+    po = pml = None
+    if splits > 1:
+        ws = torch.empty(M * heads * splits * (dim + 2), dtype=torch.float32,
+                         device=h.device)
+        po, pml = _ptr(ws), _ptr(ws) + M * heads * splits * dim * 4
     require_lib().fei_encoder_layers(
         (_vp * len(ptrs))(*ptrs), len(ptrs) // 12, _ptr(h), _ptr(h1),
         _ptr(tmp), _ptr(qkv), _ptr(att), _ptr(mid), _ptr(pos0), _ptr(kv_len),
-        B, S, heads, dim, C, inner, 1.0 / math.sqrt(dim), eps, _stream())
+        B, S, heads, dim, C, inner, 1.0 / math.sqrt(dim), eps, splits, po, pml,
+        _stream())
     return h
 
 

@@ -1,6 +1,7 @@
 // Products of tens to hundreds of rows with a weight matrix (gfx950):
 // out[M, N] = x[M, K] @ W[N, K]^T in bfloat16 with float32 sums, where a library
 // product leaves the chip half idle or makes a result that takes another pass.
+#include "fei_epilogue.h"
 #include "fei_mma.h"
 
 namespace {
@@ -8,6 +9,8 @@ namespace {
 enum {
   ROWS_PARTS = 0,      // float32 sums of a part of K, [parts][M][N]
   ROWS_SWIGLU = 1,     // W has N rows of gates, then N of up; bfloat16
+  ROWS_BIAS = 2,       // with a bias per column; bfloat16
+  ROWS_GELU = 3,       // of that
 };
 
 // Tiles of 32 XJ rows x 32 WI rows of W (SWIGLU: half of them gates, the others
@@ -31,7 +34,8 @@ enum {
 template <int XJ, int WI, int S, int EPI>
 __global__ void __launch_bounds__(256, S * (XJ + WI) <= 20 ? 2 : 1)
 k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
-       const u16* __restrict__ w, int M, int N, int K, int nx, int nm) {
+       const u16* __restrict__ w, const u16* __restrict__ bias, int M, int N,
+       int K, int nx, int nm) {
   constexpr int TM = 32 * XJ, TN = 32 * WI, MX = XJ > WI ? XJ : WI;
   constexpr int CN = EPI == ROWS_SWIGLU ? TN / 2 : TN;   // columns of out
   constexpr int BUF = (TM + TN) * 64, LOADS = XJ + WI;
@@ -147,6 +151,15 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
           v[e] = f2bf(g / (1.f + __expf(-g)) * acc[CI + i][j][e]);
         }
         __builtin_memcpy((u16*)outp + at, v, sizeof(v));
+      } else if (EPI >= ROWS_BIAS) {
+        u16 v[4], add[4];
+        __builtin_memcpy(add, bias + n, sizeof(add));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float y = acc[i][j][e] + bf2f(add[e]);
+          v[e] = f2bf(EPI == ROWS_GELU ? gelu_erf(y) : y);
+        }
+        __builtin_memcpy((u16*)outp + at, v, sizeof(v));
       } else {
         *(f32x4*)((float*)outp + (long)blockIdx.y * M * N + at) = acc[i][j];
       }
@@ -156,7 +169,7 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
 
 template <int XJ, int WI, int S, int EPI>
 void launch(void* out, const void* x, long xs, const void* w, int M, int N,
-            int K, int parts, hipStream_t stream) {
+            int K, int parts, hipStream_t stream, const void* bias = nullptr) {
   constexpr int lds = S * 32 * (XJ + WI) * 128;
   constexpr int CN = EPI == ROWS_SWIGLU ? 16 * WI : 32 * WI;
   static bool set = lds <= 65536;          // beyond that a kernel has to ask
@@ -168,7 +181,8 @@ void launch(void* out, const void* x, long xs, const void* w, int M, int N,
   const int nx = (N + CN - 1) / CN, nm = (M + 32 * XJ - 1) / (32 * XJ);
   hipLaunchKernelGGL((k_rows<XJ, WI, S, EPI>),
                      dim3((nx * nm + 7) / 8 * 8, parts), dim3(256), lds, stream,
-                     out, (const u16*)x, xs, (const u16*)w, M, N, K, nx, nm);
+                     out, (const u16*)x, xs, (const u16*)w, (const u16*)bias, M,
+                     N, K, nx, nm);
 }
 
 template <int WI, int S, int EPI>
@@ -323,6 +337,17 @@ void fei_rows(void* out, const void* x, long xs, const void* w, int M, int N,
   if (swiglu) ROWS(ROWS_SWIGLU);
   else ROWS(ROWS_PARTS);
 #undef ROWS
+}
+
+// The same sizes; out [M, N] bfloat16 with a bias per column, and GELU of it. Tiles
+// of 64 x 64: an encoder's products are small (12 to 48 of these tiles for 64
+// rows), and what counts is that many CUs load.
+void fei_rows_bias(void* out, const void* x, const void* w, const void* bias,
+                   int M, int N, int K, int gelu, hipStream_t stream) {
+  if (gelu)
+    launch<2, 2, 3, ROWS_GELU>(out, x, K, w, M, N, K, 1, stream, bias);
+  else
+    launch<2, 2, 3, ROWS_BIAS>(out, x, K, w, M, N, K, 1, stream, bias);
 }
 
 void fei_parts_norm(void* out, void* res, const float* parts, int np,

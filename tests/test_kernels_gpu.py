@@ -203,7 +203,7 @@ def test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, splits, lens):
 
 # -- products of few rows on the matrix units ------------------------------------
 
-@pytest.mark.parametrize("M", [3, 4, 8, 9, 17, 25, 32])
+@pytest.mark.parametrize("M", [3, 4, 8, 9, 17, 25, 32, 40, 64])
 @pytest.mark.parametrize("N,K", [
     (16, 64),              # one stage, three waves without any
     (20, 320),             # five stages for four waves, a part of a tile
@@ -216,7 +216,7 @@ def test_skinny_geometries(lib, M, N, K):
     bfloat16 once where the result is (2^-9; 2^-8 allowed)."""
     from fei_amd.ops import mixers as mx
     x, w = randbf(M, K, seed=M), randbf(2 * N, K, seed=N, scale=K ** -0.5)
-    assert mx.skinny_ok(M, K, x, w)
+    assert mx.skinny_ok(M, K, x, w) == (M <= 32)
     y = x.double() @ w.double().T
     a, b = y[:, :N], y[:, N:]
     w1 = w[:N].contiguous()
@@ -242,6 +242,18 @@ def test_skinny_geometries(lib, M, N, K):
     assert row_err(f, 3 * torch.tanh(a * 0.5 / 3) + bias.double()) < 1e-5
     mx.skinny(f.copy_(want), x, w1, N, mx.EPI_RES, scale=0.25)
     assert row_err(f, want.float().double() + 0.25 * a) < 1e-5
+    n_mix, n_r = N - 12, 4
+    proj = torch.empty(M, n_mix, device=DEV, dtype=torch.bfloat16)
+    router = torch.empty(M, n_r, device=DEV)
+    act = torch.zeros(M, 16, device=DEV, dtype=torch.bfloat16)
+    mx.skinny(proj, x, w1, N, mx.EPI_PARALLEL, n_mix=n_mix, router=router,
+              act=act[:, 4:], stride=16)
+    assert row_err(proj, a[:, :n_mix]) < 2 ** -8
+    assert row_err(router, a[:, n_mix:n_mix + n_r]) < 1e-5
+    assert (act[:, 4:12].double() - a[:, -8:].clamp(min=0) ** 2).abs().max() \
+        < 2 ** -8 * (a[:, -8:] ** 2).max()
+    if M > 32:
+        return
     # a residual's next product under a norm: the sums of squares of its tiles
     h = randbf(M, N, seed=6)
     sums = lib.add_product(x, w1, h)
@@ -258,16 +270,6 @@ def test_skinny_geometries(lib, M, N, K):
         assert row_err(lib.gemv_swiglu_norm(h, g, w2, 1e-5, sums=sums),
                        torch.nn.functional.silu(y2[:, :24]) * y2[:, 24:]) \
             < 2 ** -6
-    n_mix, n_r = N - 12, 4
-    proj = torch.empty(M, n_mix, device=DEV, dtype=torch.bfloat16)
-    router = torch.empty(M, n_r, device=DEV)
-    act = torch.zeros(M, 16, device=DEV, dtype=torch.bfloat16)
-    mx.skinny(proj, x, w1, N, mx.EPI_PARALLEL, n_mix=n_mix, router=router,
-              act=act[:, 4:], stride=16)
-    assert row_err(proj, a[:, :n_mix]) < 2 ** -8
-    assert row_err(router, a[:, n_mix:n_mix + n_r]) < 1e-5
-    assert (act[:, 4:12].double() - a[:, -8:].clamp(min=0) ** 2).abs().max() \
-        < 2 ** -8 * (a[:, -8:] ** 2).max()
 
 
 # -- RoPE of a prompt --------------------------------------------------------------
@@ -502,7 +504,8 @@ def test_prompt_in_parts_matches_whole_products(lib, B, S):
 
 @pytest.mark.parametrize("B,S,lengths", [(1, 4, None), (1, 24, None),
                                          (4, 8, [8, 1, 3, 5]), (2, 16, [16, 9]),
-                                         (32, 1, None)])
+                                         (32, 1, None), (1, 33, None),
+                                         (3, 50, [50, 1, 20]), (1, 300, None)])
 def test_encoder_layers_from_one_call(lib, B, S, lengths):
     from fei_amd.models.bge import BgeEncoder
     m = BgeEncoder(device=torch.device(DEV))
@@ -514,8 +517,28 @@ def test_encoder_layers_from_one_call(lib, B, S, lengths):
         want = m.encode_ids(ids, n)
     finally:
         lib.encoder_layers = before
-    # the same kernels in the same order
-    assert torch.equal(got, want)
+    if B * S <= 32:      # the same kernels in the same order
+        assert torch.equal(got, want)
+    else:
+        # 8 roundings a layer, 2^-9 / sqrt(3) each, that differ on either side:
+        # sqrt(2 * 96) of them make 0.016; twice that
+        assert row_err(got, want.double()) < 2.0 ** -5
+
+
+@pytest.mark.parametrize("gelu", [False, True])
+@pytest.mark.parametrize("M,N,K", [(33, 4, 64), (64, 768, 3072), (65, 100, 128),
+                                   (500, 2304, 768)])
+def test_rows_bias(lib, gelu, M, N, K):
+    from fei_amd.ops import rows
+    x, w, b = randbf(M, K, seed=M), randbf(N, K, seed=N, scale=K ** -0.5), \
+        randbf(N, seed=1)
+    out = torch.full((M, N), float("nan"), device=DEV, dtype=torch.bfloat16)
+    rows._lib().fei_rows_bias(*(t.data_ptr() for t in (out, x, w, b)), M, N, K,
+                              int(gelu), rows._stream())
+    want = x.double() @ w.double().t() + b.double()
+    if gelu:
+        want = torch.nn.functional.gelu(want)
+    assert row_err(out, want) < 2.0 ** -8
 
 
 # -- grouped products ------------------------------------------------------------
