@@ -302,36 +302,52 @@ k_attn_decode(const DecodeAttn a) {
 }
 
 // out[b,hq] from the splits that have keys; nothing to do where one had all.
-// One block per head, 8 (D = 128) or 16 splits side by side.
+// One block per head, 8 (D = 128) or 16 splits side by side. Bound by the latency
+// of a launch and its loads: those of the first 16 splits go out with that of the
+// position, before it is known how many there are (what lies there otherwise is
+// not used).
 template <int D>
 __global__ void __launch_bounds__(256) k_attn_decode_combine(const DecodeAttn a) {
   constexpr int SIDE = 256 / (D / 4);
   __shared__ f32x4 part[SIDE][D / 4];
   const long hq = blockIdx.x;
   const int b = hq / (a.Hkv * a.G);
-  const int used = used_splits(a, keys_at(a, b));
-  if (used == 1) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int side = tid / (D / 4), d = tid % (D / 4);
-  const float* ml = a.pml + hq * a.splits * 2;
+  const f32x2* ml = (const f32x2*)(a.pml + hq * a.splits * 2);
   const f32x4* po = (const f32x4*)(a.po + hq * a.splits * D) + d;
-  const f32x2 t = lane < used ? *(const f32x2*)(ml + 2 * lane)
-                              : f32x2{M_NONE, 0.f};
+  constexpr int PRE = 16 / SIDE;
+  f32x4 x[PRE];
+#pragma unroll
+  for (int i = 0; i < PRE; ++i)
+    x[i] = po[(long)min(side + i * SIDE, a.splits - 1) * (D / 4)];
+  f32x2 t = ml[min(lane, a.splits - 1)];
+  const int used = used_splits(a, keys_at(a, b));
+  if (used == 1) return;
+  if (lane >= used) t = f32x2{M_NONE, 0.f};
   float m = row16_max(t[0]);
   f32x2 sw = swap16(m);
   sw = swap32(fmaxf(sw[0], sw[1]));
   m = fmaxf(sw[0], sw[1]);
-  float l = row16_sum(t[1] * __builtin_amdgcn_exp2f(t[0] - m));
+  const float w = __builtin_amdgcn_exp2f(t[0] - m);    // of split ``lane``
+  float l = row16_sum(t[1] * w);
   sw = swap16(l);
   sw = swap32(sw[0] + sw[1]);
   l = sw[0] + sw[1];
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int s = side; s < used; s += SIDE) {
-    const float f = __builtin_amdgcn_exp2f(ml[2 * s] - m);
-    const f32x4 x = po[(long)s * (D / 4)];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = fmaf(f, x[e], v[e]);
+  for (int i = 0; i < PRE; ++i) {
+    const float f = __shfl(w, side + i * SIDE);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      v[e] = side + i * SIDE < used ? fmaf(f, x[i][e], v[e]) : v[e];
+  }
+#pragma unroll 4
+  for (int s = side + 16; s < used; s += SIDE) {
+    const float f = __builtin_amdgcn_exp2f(ml[s][0] - m);
+    const f32x4 y = po[(long)s * (D / 4)];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = fmaf(f, y[e], v[e]);
   }
   part[side][d] = v;
   __syncthreads();
