@@ -76,7 +76,7 @@ def _try_load() -> None:
                                [_vp, _vp, _l] + [_vp] * 3 + [_i, _f, _vp, _vp])
     lib.fei_argmax.argtypes = [_vp] * 3 + [_i] * 4 + [_vp]
     lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
-                                       [_f, _f, _i, _vp, _vp, _vp])
+                                       [_f, _f, _i] + [_vp] * 3 + [_i, _i, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -839,7 +839,7 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
 
 # Rows up to which all layers are launched from one call; one by one, with the
 # library's products, they take 1.6 ms and more from Python (12 layers of 768), of
-# which the GPU works a part: 100 rows 820 us, 512 956, 1000 981. Beyond, the
+# which the GPU works a part: 100 rows 667 us, 512 848, 1000 979. Beyond, the
 # library's products are the faster ones and the GPU is never idle.
 ENCODER_ROWS = 1024
 
@@ -874,11 +874,18 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
         ws = torch.empty(M * heads * splits * (dim + 2), dtype=torch.float32,
                          device=h.device)
         po, pml = _ptr(ws), _ptr(ws) + M * heads * splits * dim * 4
+    # parts of K for about a tile of 64 x 64 a CU, of 256 steps at least
+    tiles = -(-M // 64) * -(-C // 64)
+    p1, p2 = (min(256 // tiles, 8, k // 256) if M > 64 and C <= 2048 else 0
+              for k in (HD, inner))
+    p1, p2 = (p if p > 1 else 0 for p in (p1, p2))
+    parts = torch.empty(max(p1, p2, 1) * M * C, dtype=torch.float32,
+                        device=h.device)
     require_lib().fei_encoder_layers(
         (_vp * len(ptrs))(*ptrs), len(ptrs) // 12, _ptr(h), _ptr(h1),
         _ptr(tmp), _ptr(qkv), _ptr(att), _ptr(mid), _ptr(pos0), _ptr(kv_len),
         B, S, heads, dim, C, inner, 1.0 / math.sqrt(dim), eps, splits, po, pml,
-        _stream())
+        _ptr(parts), p1, p2, _stream())
     return h
 
 

@@ -11,6 +11,13 @@ void fei_skinny(void* out, const void* x, const void* w, int M, int N, int K,
                 int tiles, float eps, float* sums_out, hipStream_t stream);
 void fei_rows_bias(void* out, const void* x, const void* w, const void* bias,
                    int M, int N, int K, int gelu, hipStream_t stream);
+void fei_rows(void* out, const void* x, long xs, const void* w, int M, int N,
+              int K, int swiglu, int xj, int wide, int parts,
+              hipStream_t stream);
+void fei_parts_layernorm(void* out, const float* parts, int np,
+                         const void* bias, const void* res, const void* gain,
+                         const void* shift, int rows, int cols, float eps,
+                         hipStream_t stream);
 void fei_attn_prefill(const void* q, const void* k_cache, const void* v_cache,
                       void* out, const int* pos0, const int* kv_len, int B,
                       int S, int Hq, int Hkv, int D, int max_seq, float scale,
@@ -23,13 +30,15 @@ void fei_add_layernorm(void* out, const void* x, const void* res,
 // w: 12 a layer, in the order in which they are read below; h [B * S, C] is
 // replaced by the layers' result; h1 and tmp as h, qkv [B * S, 3 H D],
 // att [B * S, H D], inner [B * S, I]. What fei_skinny and fei_attn_prefill ask of
-// their rows holds for all. splits, po, pml: see fei_attn_prefill.
+// their rows holds for all. splits, po, pml: see fei_attn_prefill. parts: room
+// for the larger of p1 and p2 times B * S * C floats, and as many parts of the
+// output and the outer product's K, for more than 64 rows (0: whole products).
 void fei_encoder_layers(const void* const* w, int layers, void* h, void* h1,
                         void* tmp, void* qkv, void* att, void* inner,
                         const int* pos0, const int* kv_len, int B, int S, int H,
                         int D, int C, int I, float scale, float eps,
-                        int splits, float* po, float* pml,
-                        hipStream_t stream) {
+                        int splits, float* po, float* pml, float* parts,
+                        int p1, int p2, hipStream_t stream) {
   const int M = B * S, HD = H * D;
   auto product = [&](void* out, const void* x, const void* const* wb, int N,
                      int K, int epi) {
@@ -41,16 +50,26 @@ void fei_encoder_layers(const void* const* w, int layers, void* h, void* h1,
     fei_skinny(out, x, wb[0], M, N, K, epi, nullptr, 1.f, 0.f, 0, 0, nullptr,
                nullptr, 0, wb[1], nullptr, nullptr, 0, 0.f, nullptr, stream);
   };
+  // to = LayerNorm(x W^T + b + from). Few tiles: K in parts, which the norm sums
+  // (12 layers of 768: 100 rows 667 us for 819, 512 848 for 954)
+  auto residual = [&](void* to, const void* from, const void* x,
+                      const void* const* wb, int K, int np) {
+    if (np) {
+      fei_rows(parts, x, K, wb[0], M, C, K, 0, 2, 0, np, stream);
+      return fei_parts_layernorm(to, parts, np, wb[1], from, wb[2], wb[3], M, C,
+                                 eps, stream);
+    }
+    product(tmp, x, wb, C, K, EPI_BF16);
+    fei_add_layernorm(to, tmp, from, wb[2], wb[3], M, C, eps, 1, stream);
+  };
   for (int l = 0; l < layers; ++l, w += 12) {
     product(qkv, h, w, 3 * HD, C, EPI_BF16);
     fei_attn_prefill(qkv, (u16*)qkv + HD, (u16*)qkv + 2 * HD, att, pos0, kv_len,
                      B, S, H, H, D, S, scale, 0, 3L * HD, splits, po, pml,
                      3L * S * HD, D, 3L * HD, stream);
-    product(tmp, att, w + 2, C, HD, EPI_BF16);
-    fei_add_layernorm(h1, tmp, h, w[4], w[5], M, C, eps, 1, stream);
+    residual(h1, h, att, w + 2, HD, p1);
     product(inner, h1, w + 6, I, C, EPI_GELU);
-    product(tmp, inner, w + 8, C, I, EPI_BF16);
-    fei_add_layernorm(h, tmp, h1, w[10], w[11], M, C, eps, 1, stream);
+    residual(h, h1, inner, w + 8, I, p2);
   }
 }
 

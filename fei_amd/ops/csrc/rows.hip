@@ -244,6 +244,65 @@ k_parts_norm(u16* __restrict__ out, u16* __restrict__ res,
   }
 }
 
+// LayerNorm of the sum of the parts, a bias and a residual: what follows an
+// encoder's product. A wave per row, V times 8 columns a lane; bound by the latency
+// of a launch and of the parts, as the norm of a whole product is.
+template <int V>
+__global__ void __launch_bounds__(256)
+k_parts_layernorm(u16* __restrict__ out, const float* __restrict__ parts, int np,
+                  const u16* __restrict__ bias, const u16* __restrict__ res,
+                  const u16* __restrict__ gain, const u16* __restrict__ shift,
+                  int rows, int cols, float eps) {
+  const int lane = threadIdx.x & 63, nv = cols >> 3;
+  const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const long step = (long)rows * cols;
+  float v[V][8], sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = lane + 64 * i;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = 0.f;
+    if (c >= nv) continue;
+    const s16x8 r = ((const s16x8*)(res + row * cols))[c];
+    const s16x8 b = ((const s16x8*)bias)[c];
+    const float* p = parts + row * cols + c * 8;
+#pragma unroll 4
+    for (int k = 0; k < np; ++k) {
+      const f32x8 q = ld8(p + k * step);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[i][j] += q[j];
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[i][j] += bf2f((u16)b[j]) + bf2f((u16)r[j]);
+      sum += v[i][j];
+    }
+  }
+  const float mean = wave_reduce_sum(sum) / (float)cols;
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < V; ++i)
+    if (lane + 64 * i < nv)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        v[i][j] -= mean;
+        sq = fmaf(v[i][j], v[i][j], sq);
+      }
+  const float inv = rsqrtf(wave_reduce_sum(sq) / (float)cols + eps);
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int c = lane + 64 * i;
+    if (c >= nv) continue;
+    const s16x8 g = ((const s16x8*)gain)[c], b = ((const s16x8*)shift)[c];
+    s16x8 y;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      y[j] = (short)f2bf(fmaf(v[i][j] * inv, bf2f((u16)g[j]), bf2f((u16)b[j])));
+    ((s16x8*)(out + row * cols))[c] = y;
+  }
+}
+
 // The parts of a product with the projections of q, k and v: q to rows of its own
 // and k to the cache under RoPE, v to the cache. A thread takes dimensions
 // 8 i .. 8 i + 7 of a head and their partners D/2 on; D % 16 == 0. 75 tokens, 32/8
@@ -355,6 +414,20 @@ void fei_parts_norm(void* out, void* res, const float* parts, int np,
                     hipStream_t stream) {
   hipLaunchKernelGGL(k_parts_norm, dim3(rows), dim3(512), 0, stream, (u16*)out,
                      (u16*)res, parts, np, (const u16*)gain, rows, cols, eps);
+}
+
+// cols % 8 == 0, at most 2048; out may be none of the inputs
+void fei_parts_layernorm(void* out, const float* parts, int np,
+                         const void* bias, const void* res, const void* gain,
+                         const void* shift, int rows, int cols, float eps,
+                         hipStream_t stream) {
+#define GO(V)                                                                \
+  hipLaunchKernelGGL(k_parts_layernorm<V>, dim3((rows + 3) / 4), dim3(256), 0, \
+                     stream, (u16*)out, parts, np, (const u16*)bias,          \
+                     (const u16*)res, (const u16*)gain, (const u16*)shift,    \
+                     rows, cols, eps)
+  if (cols <= 1024) GO(2); else GO(4);
+#undef GO
 }
 
 // parts [np][B * S][(Hq + 2 Hkv) * D], q [B * S][Hq][D]; D % 16 == 0, all on 16

@@ -17,6 +17,8 @@ SKINNY_ROWS = 32     # most rows of the matrix-core tile for few rows
 def declare(lib: ctypes.CDLL) -> None:
     lib.fei_rows.argtypes = [_vp, _vp, _l, _vp] + [_i] * 7 + [_vp]
     lib.fei_rows_bias.argtypes = [_vp] * 4 + [_i] * 4 + [_vp]
+    lib.fei_parts_layernorm.argtypes = ([_vp, _vp, _i] + [_vp] * 4 +
+                                        [_i, _i, _f, _vp])
     lib.fei_parts_norm.argtypes = [_vp, _vp, _vp, _i, _vp, _i, _i, _f, _vp]
     lib.fei_rope_kv_parts.argtypes = [_vp, _vp, _i] + [_vp] * 4 + [_i] * 6 + [_vp]
     lib.fei_parts_add.argtypes = [_vp, _vp, _i, _l, _f, _vp]

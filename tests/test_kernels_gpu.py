@@ -643,3 +643,21 @@ def test_argmax_is_the_first(lib, dtype, B, V):
         assert got.dtype == torch.int64
         # argmax of the CPU: the first of equals, NaN above all
         assert torch.equal(got.cpu(), t.float().cpu().argmax(-1))
+
+
+@pytest.mark.parametrize("M,C,p", [(1, 8, 1), (5, 512, 3), (70, 768, 8),
+                                   (66, 1024, 2), (9, 1032, 5), (6, 2048, 4)])
+def test_parts_layernorm(lib, M, C, p):
+    from fei_amd.ops import rows
+    parts = torch.randn(p, M, C, device=DEV)
+    bias, res, gain, shift = (randbf(*s, seed=i) for i, s in enumerate(
+        ((C,), (M, C), (C,), (C,))))
+    out = torch.full((M + 1, C), float("nan"), device=DEV, dtype=torch.bfloat16)
+    rows._lib().fei_parts_layernorm(
+        out.data_ptr(), parts.data_ptr(), p, bias.data_ptr(), res.data_ptr(),
+        gain.data_ptr(), shift.data_ptr(), M, C, 1e-6, rows._stream())
+    x = parts.double().sum(0) + bias.double() + res.double()
+    want = torch.nn.functional.layer_norm(x, (C,), gain.double(),
+                                          shift.double(), 1e-6)
+    assert row_err(out[:M], want) < 2.0 ** -8
+    assert bool(out[M].isnan().all())
