@@ -100,14 +100,7 @@ class BgeEncoder:
                                  H, D, s.intermediate_size, pos0, kv_len,
                                  self.eps)
         h = few if few is not None else self._layers(h, pos0, kv_len)
-        hf = h.float()
-        if lengths is not None:
-            mask = (torch.arange(S, device=self.device).unsqueeze(0)
-                    < lengths.unsqueeze(1)).float().unsqueeze(-1)
-            pooled = (hf * mask).sum(1) / mask.sum(1).clamp_min(1.0)
-        else:
-            pooled = hf.mean(dim=1)
-        return F.normalize(pooled, dim=-1)
+        return ops.pool_unit(h, kv_len)
 
     def _layers(self, h: torch.Tensor, pos0: torch.Tensor,
                 kv_len: torch.Tensor) -> torch.Tensor:

@@ -74,6 +74,7 @@ def _try_load() -> None:
                              _vp, _vp]
     lib.fei_skinny.argtypes = ([_vp] * 3 + [_i] * 4 + [_vp, _f, _f, _i, _i] +
                                [_vp, _vp, _l] + [_vp] * 3 + [_i, _f, _vp, _vp])
+    lib.fei_pool_unit.argtypes = [_vp] * 3 + [_i] * 3 + [_vp]
     lib.fei_argmax.argtypes = [_vp] * 3 + [_i] * 4 + [_vp]
     lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
                                        [_f, _f, _i] + [_vp] * 3 + [_i, _i, _vp])
@@ -887,6 +888,25 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
         B, S, heads, dim, C, inner, 1.0 / math.sqrt(dim), eps, splits, po, pml,
         _ptr(parts), p1, p2, _stream())
     return h
+
+
+def pool_unit(h: torch.Tensor, lens: torch.Tensor) -> torch.Tensor:
+    """Mean of the first lens[b] rows of h [B, S, C], scaled to length 1 ->
+    [B, C] float32."""
+    B, S, C = h.shape
+    if not (h.is_cuda and h.dtype == torch.bfloat16 and h.is_contiguous()
+            and h.numel() and C % 8 == 0 and C <= 2048
+            and h.data_ptr() % 16 == 0 and lens.device == h.device
+            and lens.dtype == torch.int32
+            and lens.is_contiguous()):
+        mask = (torch.arange(S, device=h.device).unsqueeze(0)
+                < lens.unsqueeze(1)).float().unsqueeze(-1)
+        mean = (h.float() * mask).sum(1) / mask.sum(1).clamp_min(1.0)
+        return torch.nn.functional.normalize(mean, dim=-1)
+    out = torch.empty(B, C, dtype=torch.float32, device=h.device)
+    require_lib().fei_pool_unit(_ptr(out), _ptr(h), _ptr(lens), B, S, C,
+                                _stream())
+    return out
 
 
 def gelu(x: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

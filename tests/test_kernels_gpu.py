@@ -661,3 +661,20 @@ def test_parts_layernorm(lib, M, C, p):
                                           shift.double(), 1e-6)
     assert row_err(out[:M], want) < 2.0 ** -8
     assert bool(out[M].isnan().all())
+
+
+@pytest.mark.parametrize("B,S,C,lens", [
+    (1, 1, 8, [1]), (3, 7, 768, [7, 0, 3]), (2, 513, 768, [513, 200]),
+    (2, 40, 2048, [40, 99]), (5, 9, 1032, [9, 1, 2, -3, 5]), (1, 300, 64, [300]),
+])
+def test_pool_unit(lib, B, S, C, lens):
+    """Rows past a length, or past the text, do not count; no row: zeros."""
+    h = randbf(B, S, C, seed=S)
+    got = lib.pool_unit(h, torch.tensor(lens, dtype=torch.int32, device=DEV))
+    for b, n in enumerate(lens):
+        x = h[b, :max(n, 0)].double()
+        want = torch.nn.functional.normalize(
+            x.sum(0) / max(x.shape[0], 1), dim=0)
+        # float32 sums of up to 513 terms, the partial ones short
+        assert float((got[b] - want).norm()) < 1e-5
+        assert n > 0 or not got[b].any()
