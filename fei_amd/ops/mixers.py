@@ -156,8 +156,30 @@ class GainNormed:
                 and self.x.shape[0] > 0)
 
 
-def _gemv_rows(T: int, K: int, t: torch.Tensor) -> bool:
-    return T in (1, 2, 4, 8) and K % 8 == 0 and t.dtype == torch.bfloat16
+def plain(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether pointers stand for x [.., K] and w [N, K] in a kernel: bfloat16,
+    without gaps, of sizes that fit, on one device; and nobody asks for a
+    gradient, which the library's products have."""
+    return (x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
+            and x.is_contiguous() and w.is_contiguous()
+            and x.shape[-1] == w.shape[1] and x.device == w.device
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
+def _dense(t: torch.Tensor, dtype: torch.dtype, like: torch.Tensor,
+           *shape: int) -> bool:
+    """Whether a pointer stands for t of this type and shape."""
+    return (t.dtype == dtype and t.shape == shape and t.is_contiguous()
+            and t.device == like.device)
+
+
+def gemv_sizes(T: int, K: int) -> bool:
+    return T in (1, 2, 4, 8) and K % 8 == 0
+
+
+def _gemv_rows(T: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
+    return gemv_sizes(T, K) and plain(x, w)
 
 
 # What becomes of a skinny product's sums (csrc/fei_epilogue.h).
@@ -174,7 +196,7 @@ def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor,
     3.54, 0.84 for 0.88); beyond 32 its repeated reads of x cost more than the
     library's."""
     return (least <= T <= SKINNY_ROWS and K > 0 and K % 64 == 0
-            and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous()
+            and plain(x, w)
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
@@ -199,14 +221,16 @@ def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,
     silu(gate) * up of n2, gate and up being the next ``ff`` rows each, into
     ``act`` (a column range of a wider buffer)."""
     T, K = n1.shape
-    if n1.is_cuda and skinny_ok(T, K, n1, w_in):
+    own = n1.is_cuda and (not ff or (
+        n2.shape == n1.shape and plain(n2, w_in) and n2.data_ptr() % 16 == 0))
+    if own and skinny_ok(T, K, n1, w_in):
         proj = torch.empty(T, n_mix, dtype=n1.dtype, device=n1.device)
         skinny(proj, n1, w_in, n_mix, EPI_BF16)
         if ff:
             skinny(None, n2, w_in[n_mix:], ff, EPI_SWIGLU, act=act,
                    stride=act.stride(0))
         return proj
-    if n1.is_cuda and _gemv_rows(T, K, n1):
+    if own and _gemv_rows(T, K, n1, w_in):
         proj = torch.empty(T, n_mix, dtype=n1.dtype, device=n1.device)
         _lib().fei_gemv_mix_in(_p(proj), _p(act), _p(n1), _p(n2), _p(w_in),
                                act.stride(0), T, n_mix, ff, K, 1, _stream())
@@ -292,16 +316,17 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
                     mult: float = 1.0) -> torch.Tensor:
     """x + mult * (a @ w^T), float32; x may be overwritten with it."""
     T, K = a.shape
-    if a.is_cuda and skinny_ok(T, K, a, w):
+    own = a.is_cuda and _dense(x, torch.float32, a, T, w.shape[0])
+    if own and skinny_ok(T, K, a, w):
         skinny(x, a, w, w.shape[0], EPI_RES, scale=mult)
         return x
-    if a.is_cuda and _gemv_rows(T, K, a):
+    if own and _gemv_rows(T, K, a, w):
         _lib().fei_gemv_f32(_p(x), _p(a), _p(w), None, T, w.shape[0], K, 1,
                             mult, 0.0, 1, _stream())
         return x
     if not a.is_cuda or a.dtype == torch.float32:
         return x + mult * _mm_f32(a, w, None)
-    if _rows.add_ok(x, a, w):
+    if own and _rows.add_ok(x, a, w):
         _rows.add_product(x, a, w, mult)
         return x
     return torch.addmm(x, a, w.t(), out_dtype=torch.float32, alpha=mult,
@@ -312,11 +337,12 @@ def linear_f32(a: torch.Tensor, w: torch.Tensor,
                bias: torch.Tensor) -> torch.Tensor:
     """a @ w^T + bias, float32."""
     T, K = a.shape
-    if a.is_cuda and skinny_ok(T, K, a, w):
+    own = a.is_cuda and _dense(bias, torch.float32, a, w.shape[0])
+    if own and skinny_ok(T, K, a, w):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=a.device)
         skinny(out, a, w, w.shape[0], EPI_F32, bias=bias)
         return out
-    if a.is_cuda and _gemv_rows(T, K, a):
+    if own and _gemv_rows(T, K, a, w):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=a.device)
         _lib().fei_gemv_f32(_p(out), _p(a), _p(w), _p(bias), T, w.shape[0], K,
                             0, 1.0, 0.0, 1, _stream())
@@ -335,7 +361,7 @@ def logits_head(y: torch.Tensor, w: torch.Tensor, scale: float,
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=y.device)
         skinny(out, y, w, w.shape[0], EPI_F32, scale=scale, cap=c)
         return out
-    if _gemv_rows(T, K, y):
+    if _gemv_rows(T, K, y, w):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=y.device)
         _lib().fei_gemv_f32(_p(out), _p(y), _p(w), None, T, w.shape[0], K, 0,
                             scale, c, 1, _stream())

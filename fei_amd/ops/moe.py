@@ -14,8 +14,8 @@ from typing import Tuple
 import torch
 
 from fei_amd.ops import reference as ref
-from fei_amd.ops.mixers import (GainNormed, _f32, _gemv_rows, _lib, _p,
-                                _stream, residual_linear)
+from fei_amd.ops.mixers import (GainNormed, _f32, _lib, _p, _stream,
+                                gemv_sizes, residual_linear)
 
 _c = ctypes
 _vp, _i, _f, _l = _c.c_void_p, _c.c_int, _c.c_float, _c.c_long
@@ -69,7 +69,8 @@ def residual_moe(x: torch.Tensor, h: GainNormed, router: torch.Tensor,
     if T == 0:
         return x
     dev, st, lib = x.device, _stream(), _lib()
-    if _gemv_rows(T, C, up) and ff % 8 == 0 and a.shape[1] % 8 == 0:
+    if gemv_sizes(T, C) and up.dtype == torch.bfloat16 and ff % 8 == 0 \
+            and a.shape[1] % 8 == 0:
         ids = torch.empty(T, f.top, dtype=torch.int32, device=dev)
         w = torch.empty(T, f.top, dtype=torch.float32, device=dev)
         act = torch.empty(T * f.top, ff, dtype=up.dtype, device=dev)

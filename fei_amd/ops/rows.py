@@ -137,7 +137,9 @@ def add_ok(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether x += a @ w^T runs in parts: of a short K the second launch costs
     what they gain (200 rows, 2048 x 2048: 11 us in the library)."""
     return (rows_ok(a.shape[0], w) and w.shape[1] >= 4096
-            and a.dtype == w.dtype and x.dtype == torch.float32
+            and a.dtype == w.dtype and a.shape[1] == w.shape[1]
+            and a.device == w.device == x.device and x.dtype == torch.float32
+            and x.shape == (a.shape[0], w.shape[0])
             and x.is_contiguous() and x.data_ptr() % 16 == 0)
 
 
