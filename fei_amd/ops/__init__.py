@@ -587,14 +587,29 @@ def _norm_inside(how: str, M: int, K: int, sums) -> bool:
     return M * K * 2 <= 128 * 1024
 
 
-def _product(x: torch.Tensor, w: torch.Tensor, rows_out: int) -> Optional[str]:
+def _product(x: torch.Tensor, w: torch.Tensor, rows_out: int,
+             out: Optional[torch.Tensor] = None) -> Optional[str]:
     """Which kernel takes x @ w^T: "skinny" (matrix units), "gemv", or None
-    (the library; CPU)."""
+    (the library; CPU). ``out``: where the caller wants the results."""
     K = x.shape[-1]
     M = x.numel() // K if K else 0
     if not x.is_cuda or not M or not rows_out:
         return None
-    if _mixers.skinny_ok(M, K, x, w, 2):
+    return _kernel_for(x, w, M, K) if _fits(out, x, M * rows_out) else None
+
+
+def _fits(out: Optional[torch.Tensor], x: torch.Tensor, n: int) -> bool:
+    """Whether a kernel can write its n results, of x's type, to out."""
+    return out is None or (out.dtype == x.dtype and out.numel() == n
+                           and out.is_contiguous() and out.device == x.device)
+
+
+def _kernel_for(x: torch.Tensor, w: torch.Tensor, M: int,
+                K: int) -> Optional[str]:
+    if not _mixers.match(x, w):
+        return None
+    # the callers copy rows with gaps; a copy is aligned
+    if _mixers.skinny_sizes(M, K, x if x.is_contiguous() else w, w, 2):
         return "skinny"
     return "gemv" if _gemv_ok(M, K) else None
 
@@ -604,17 +619,15 @@ def own_product(M: int, w: torch.Tensor) -> bool:
     library's kernels, which add to a residual and make a SwiGLU without a
     launch of its own."""
     N, K = w.shape
-    return w.is_cuda and N > 0 and (_mixers.skinny_ok(M, K, w, w, 2) or
-                                    _gemv_ok(M, K))
+    return w.is_cuda and N > 0 and _kernel_for(w, w, M, K) is not None
 
 
 def linear_decode(x: torch.Tensor, w: torch.Tensor,
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """F.linear for skinny M: streaming GEMV or matrix-core tile on GPU. Falls
     back to torch for unsupported shapes/CPU."""
-    M = x.numel() // x.shape[-1]
-    N, K = w.shape
-    how = _product(x, w, N)
+    M, K, N = x.numel() // x.shape[-1], x.shape[-1], w.shape[0]
+    how = _product(x, w, N, out)
     if how is None:
         return torch.nn.functional.linear(x, w)
     x2 = x.contiguous().view(M, K)
@@ -633,8 +646,9 @@ def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
     M = x.numel() // x.shape[-1]
     K = x.shape[-1]
     I = wgu.shape[0] // 2
-    how = _product(x, wgu, I)
-    if how is None and x.is_cuda and _rows.swiglu_ok(M, x, wgu):
+    how = _product(x, wgu, I, out)
+    if (how is None and x.is_cuda and _rows.swiglu_ok(M, x, wgu)
+            and _mixers.match(x, wgu) and _fits(out, x, M * I)):
         how = "rows"
     if how is None:
         return swiglu(torch.nn.functional.linear(x, wgu))
@@ -659,14 +673,15 @@ def gemv_res(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
     sum-of-squares of the updated residual rows, which a following
     gemv_norm/gemv_swiglu_norm takes as ``ssq``. Ignored on the CPU fallback —
     consumers recompute exactly there."""
-    M = x.numel() // x.shape[-1]
-    N, K = w.shape
-    how = _product(x, w, N)
+    M, K, N = x.numel() // x.shape[-1], x.shape[-1], w.shape[0]
+    how = _product(x, w, N, res)
     if ssq_out is not None and how == "skinny" and _gemv_ok(M, K):
         how = "gemv"
     if how is None:
         lin = torch.nn.functional.linear(x, w)
         res.copy_((res.float() + lin.float().view_as(res)).to(res.dtype))
+        if ssq_out is not None and x.is_cuda:
+            ssq_out += res.float().reshape(M, N).pow(2).sum(-1)
     elif how == "skinny":
         _mixers.skinny(res, x.contiguous().view(M, K), w, N,
                        _mixers.EPI_RES_BF16)
@@ -681,9 +696,8 @@ def add_product(x: torch.Tensor, w: torch.Tensor,
     """gemv_res, for a chain: returns the sums of squares of the new rows by
     tiles of columns, for the ``sums`` of the products that read them under a
     norm, or None where those do not need them."""
-    M = x.numel() // x.shape[-1]
-    N, K = w.shape
-    if _product(x, w, N) != "skinny":
+    M, K, N = x.numel() // x.shape[-1], x.shape[-1], w.shape[0]
+    if _product(x, w, N, res) != "skinny":
         gemv_res(x, w, res)
         return None
     sums = torch.empty(M, -(-N // 16), dtype=torch.float32, device=x.device)
@@ -702,9 +716,8 @@ def gemv_norm(res: torch.Tensor, wnorm: torch.Tensor, w: torch.Tensor,
     ``ssq`` [M] f32: the sums of squares of res rows, if the caller has them
     (from a prior gemv_res ``ssq_out``). ``sums``: what add_product returned
     for these rows."""
-    M = res.numel() // res.shape[-1]
-    N, K = w.shape
-    how = _product(res, w, N)
+    M, K, N = res.numel() // res.shape[-1], res.shape[-1], w.shape[0]
+    how = _product(res, w, N, out)
     if how is None:
         return torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w)
     if not _norm_inside(how, M, K, sums):
@@ -730,7 +743,7 @@ def gemv_swiglu_norm(res: torch.Tensor, wnorm: torch.Tensor,
     M = res.numel() // res.shape[-1]
     K = res.shape[-1]
     I = wgu.shape[0] // 2
-    how = _product(res, wgu, I)
+    how = _product(res, wgu, I, out)
     if how is None:
         return swiglu(torch.nn.functional.linear(rmsnorm(res, wnorm, eps), wgu))
     if not _norm_inside(how, M, K, sums):
@@ -826,8 +839,8 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
                 act_gelu: bool = False) -> torch.Tensor:
     """x @ w^T + bias, and its GELU if asked for (encoder blocks)."""
     M = x.numel() // max(x.shape[-1], 1)
-    if (x.is_cuda and x.is_contiguous() and bias.dtype == torch.bfloat16
-            and _mixers.skinny_ok(M, x.shape[-1], x, w)):
+    if (x.is_cuda and _mixers.skinny_ok(M, x.shape[-1], x, w)
+            and _mixers.dense(bias, torch.bfloat16, x, w.shape[0])):
         out = torch.empty(*x.shape[:-1], w.shape[0], dtype=x.dtype,
                           device=x.device)
         _mixers.skinny(out, x.view(M, -1), w, w.shape[0],

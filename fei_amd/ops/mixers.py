@@ -156,18 +156,23 @@ class GainNormed:
                 and self.x.shape[0] > 0)
 
 
-def plain(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether pointers stand for x [.., K] and w [N, K] in a kernel: bfloat16,
-    without gaps, of sizes that fit, on one device; and nobody asks for a
-    gradient, which the library's products have."""
+def match(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether pointers stand for x [.., K], or a copy without gaps, and w
+    [N, K] in a kernel: bfloat16, w without gaps, sizes that fit, on one device;
+    and nobody asks for a gradient, which the library's products have."""
     return (x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
-            and x.is_contiguous() and w.is_contiguous()
-            and x.shape[-1] == w.shape[1] and x.device == w.device
+            and w.is_contiguous() and x.shape[-1] == w.shape[1]
+            and x.device == w.device
             and not (torch.is_grad_enabled()
                      and (x.requires_grad or w.requires_grad)))
 
 
-def _dense(t: torch.Tensor, dtype: torch.dtype, like: torch.Tensor,
+def plain(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """The same for x as it lies."""
+    return x.is_contiguous() and match(x, w)
+
+
+def dense(t: torch.Tensor, dtype: torch.dtype, like: torch.Tensor,
            *shape: int) -> bool:
     """Whether a pointer stands for t of this type and shape."""
     return (t.dtype == dtype and t.shape == shape and t.is_contiguous()
@@ -187,8 +192,8 @@ def _gemv_rows(T: int, K: int, x: torch.Tensor, w: torch.Tensor) -> bool:
  EPI_GELU) = range(7)
 
 
-def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor,
-              least: int = 3) -> bool:
+def skinny_sizes(T: int, K: int, x: torch.Tensor, w: torch.Tensor,
+                 least: int = 3) -> bool:
     """Rows and sizes that the matrix-core tile for few rows takes: its loads
     are of 16 bytes, 128 a row. From 3 rows on it beats the vector units (whole
     decoding steps, 3 rows: 3.24 ms for 4.75 on 8B, 0.79 for 1.12 on 1B), from 2
@@ -196,8 +201,12 @@ def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor,
     3.54, 0.84 for 0.88); beyond 32 its repeated reads of x cost more than the
     library's."""
     return (least <= T <= SKINNY_ROWS and K > 0 and K % 64 == 0
-            and plain(x, w)
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def skinny_ok(T: int, K: int, x: torch.Tensor, w: torch.Tensor,
+              least: int = 3) -> bool:
+    return skinny_sizes(T, K, x, w, least) and plain(x, w)
 
 
 def skinny(out, x, w, n: int, epi: int, bias=None, scale: float = 1.0,
@@ -316,7 +325,7 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
                     mult: float = 1.0) -> torch.Tensor:
     """x + mult * (a @ w^T), float32; x may be overwritten with it."""
     T, K = a.shape
-    own = a.is_cuda and _dense(x, torch.float32, a, T, w.shape[0])
+    own = a.is_cuda and dense(x, torch.float32, a, T, w.shape[0])
     if own and skinny_ok(T, K, a, w):
         skinny(x, a, w, w.shape[0], EPI_RES, scale=mult)
         return x
@@ -337,7 +346,7 @@ def linear_f32(a: torch.Tensor, w: torch.Tensor,
                bias: torch.Tensor) -> torch.Tensor:
     """a @ w^T + bias, float32."""
     T, K = a.shape
-    own = a.is_cuda and _dense(bias, torch.float32, a, w.shape[0])
+    own = a.is_cuda and dense(bias, torch.float32, a, w.shape[0])
     if own and skinny_ok(T, K, a, w):
         out = torch.empty(T, w.shape[0], dtype=torch.float32, device=a.device)
         skinny(out, a, w, w.shape[0], EPI_F32, bias=bias)

@@ -43,6 +43,67 @@ def test_few_rows_want_plain_tensors(T):
         assert mx.plain(x, leaf)
 
 
+@pytest.mark.parametrize("M", [1, 3, 5, 8, 32])
+def test_products_want_plain_weights(M):
+    """Which kernel, if any; it needs no GPU to say so."""
+    for K, how in ((128, "gemv" if M == 1 else "skinny"),
+                   (72, "gemv" if M in (1, 3, 8) else None), (70, None)):
+        x, w = rand(M, K), rand(48, K)
+        assert ops._kernel_for(x, w, M, K) == how
+        assert ops._kernel_for(rand(M, 2 * K)[:, K:], w, M, K) == how
+        leaf = rand(48, K).requires_grad_()
+        for a, b in [(x.float(), w.float()), (x.half(), w.half()),
+                     (x.float(), w), (x, rand(K, 48).t()), (x, leaf),
+                     (x, rand(48, 2 * K)[:, :K]), (x, rand(48, K + 8)),
+                     (x, w[0])]:
+            assert ops._kernel_for(a, b, M, K) is None
+        with torch.no_grad():
+            assert ops._kernel_for(x, leaf, M, K) == how
+    out = rand(M, 48)
+    assert ops._fits(None, x, M * 48) and ops._fits(out, x, M * 48)
+    for bad in (out.float(), rand(M, 49), rand(M, 96)[:, :48] if M > 1 else rand(2, 48)):
+        assert not ops._fits(bad, x, M * 48)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 3, 5, 8, 9, 32, 40])
+def test_products_of_other_types_and_layouts(M):
+    F = torch.nn.functional
+    K, N = 128, 96
+    for dtype, tol in ((torch.float32, 1e-5), (torch.float16, 2 ** -10),
+                       (torch.bfloat16, 2 ** -8)):
+        make = dict(dev=DEV, dtype=dtype, scale=K ** -0.5)
+        x = rand(M, K, seed=1, dev=DEV, dtype=dtype)
+        for w in (rand(N, K, seed=2, **make), rand(K, N, seed=2, **make).t(),
+                  rand(N, 2 * K, seed=2, **make)[:, K:]):
+            y = x.double() @ w.double().t()
+            assert row_err(ops.linear_decode(x, w), y) < tol
+            wide = rand(M, 2 * N, seed=3, dev=DEV, dtype=dtype)
+            for res in (wide[:, N:], wide[:, N:].contiguous()):
+                left, want = wide[:, :N].clone(), res.double() + y
+                # sums rounded before they are added, in the library
+                ops.gemv_res(x, w, res)
+                assert row_err(res, want) < 2 * tol
+                assert torch.equal(wide[:, :N], left)
+            b = rand(2 * N, seed=4, dev=DEV, dtype=dtype)
+            for bias in (b[:N], b[::2]):
+                got = ops.linear_bias(x, w, bias)
+                assert row_err(got, y + bias.double()) < tol
+            if dtype == torch.bfloat16:
+                want = F.silu(y[:, :N // 2]) * y[:, N // 2:]
+                # rounded once, in the library twice before
+                assert row_err(ops.gemv_swiglu(x, w), want) < 2 ** -6
+        for w in (w[:, :64].contiguous(), w.cpu().contiguous()):
+            for call in (lambda: ops.linear_decode(x, w),
+                         lambda: ops.linear_bias(x, w, b[:N]),
+                         lambda: ops.gemv_swiglu(x, w)):
+                with pytest.raises(RuntimeError):
+                    call()
+    leaf = w.to(DEV).requires_grad_()
+    ops.linear_decode(x, leaf).sum().backward()
+    assert row_err(leaf.grad, x.double().sum(0).expand(N, K)) < 2 ** -7
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 3, 4, 8, 9, 32, 40])
 def test_views_of_few_rows(T):
