@@ -46,7 +46,8 @@ k_pool_unit(float* __restrict__ out, const u16* __restrict__ h,
   sq = 0.f;
 #pragma unroll
   for (int k = 0; k < 16; ++k) sq += red[k];
-  const float norm = fmaxf(sqrtf(sq), 1e-12f);
+  const float len = sqrtf(sq);
+  const float norm = len < 1e-12f ? 1e-12f : len;   // NaN stays
   for (int i = tid; i < C; i += 1024) out[(long)b * C + i] = part[i] / norm;
 }
 

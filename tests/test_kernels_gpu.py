@@ -678,3 +678,20 @@ def test_pool_unit(lib, B, S, C, lens):
         # float32 sums of up to 513 terms, the partial ones short
         assert float((got[b] - want).norm()) < 1e-5
         assert n > 0 or not got[b].any()
+
+
+def test_pool_unit_keeps_nan_and_inf(lib):
+    """As in torch: a NaN in one column makes a text's whole result NaN, an
+    infinity the others zero; texts beside it are as without."""
+    h = randbf(4, 9, 768, seed=1)
+    h[1, 3, 5], h[2, 8, 700] = float("nan"), float("inf")
+    h[3, 4, 0] = float("nan")                       # past the length
+    lens = torch.tensor([9, 9, 9, 4], dtype=torch.int32, device=DEV)
+    got = lib.pool_unit(h, lens)
+    assert got[1].isnan().all()
+    assert got[2, 700].isnan() and not got[2, :700].any() \
+        and not got[2, 701:].any()
+    for b in (0, 3):
+        want = torch.nn.functional.normalize(
+            h[b, :lens[b]].double().mean(0), dim=0)
+        assert float((got[b] - want).norm()) < 1e-5
