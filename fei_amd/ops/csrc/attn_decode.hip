@@ -9,17 +9,20 @@
 // lie in the registers as the second operand of V^T times P^T; a lane loads 8
 // keys x D/16 columns of V and turns them in registers. Keys and values never
 // pass LDS, and nothing but the end of a block has a barrier. Roped queries and
-// weights enter the bfloat16 products as a high and a low part (about 16 bits).
+// weights enter the bfloat16 products as three parts, whose sum is the float32
+// value: 3e-7 of a row's float32 result is what the whole is off by, as much as
+// products on the vector units (4e-7); with two parts it was 3e-6, 6 % faster. An
+// infinite key or value makes a row NaN (0 times it, in a part).
 // The chunks go to the blocks' waves in order, so that short contexts end in
 // few blocks (one: it writes the result), and the rest leave at once.
 //
 // Bound by latency (position, table, rows, combine) up to some MB of keys, by
-// HBM beyond. Per layer in a captured step, against a thread per key with the
-// products on the vector units and the scores exchanged through LDS: 300 keys,
-// 32/8 heads of 64: 11.1 -> 4.7 us; 512 and 3400 keys, 32/8 of 128: 12.6 -> 5.2
-// and 20.0 -> 6.6; 8 sequences of up to 2047 keys (43 MB): 26.9 -> 13.4; 20 of
-// up to 600 in pages of 16, heads of 64: 50 -> 7.8. The combine takes 4 to 5, a
-// launch's least.
+// HBM beyond. Per layer with the combine in a graph of 16, against a thread per
+// key with the products on the vector units and the scores exchanged through LDS:
+// 300 keys, 32/8 heads of 64: 13.5 -> 6.1 us; 512, 3400 and 8000 keys, 32/8 of
+// 128: 15.7 -> 8.2, 21.4 -> 9.7 and 25.3 -> 13.7; 8 sequences of 2047: 32.5 ->
+// 20.4; 32 of 500: 72 -> 21.2; 20 of 600, heads of 64: 49 -> 12.4. The combine
+// takes 4 to 5, a launch's least.
 #include "fei_attn.h"
 
 namespace {
@@ -76,6 +79,26 @@ __device__ __forceinline__ float head_sum(float v) {
   return t[0] + t[1];
 }
 
+// Eight float32 values as three fragments of bfloat16, largest first. Each part
+// is what the ones before leave, rounded; what two of them leave has 8 bits, so
+// that the sum of the three is the value.
+__device__ __forceinline__ void parts3(const float (&v)[8], s16x8 (&p)[3]) {
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  u32x4 w[3];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    f32x2 x = {v[2 * i], v[2 * i + 1]};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      w[k][i] = __builtin_bit_cast(u32, __builtin_convertvector(x, bf16x2));
+      x = f32x2{x[0] - __builtin_bit_cast(float, w[k][i] << 16),
+                x[1] - __builtin_bit_cast(float, w[k][i] & 0xffff0000u)};
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) p[k] = __builtin_bit_cast(s16x8, w[k]);
+}
+
 // x1 and x2: dimensions d .. d + 7 and d + D/2 .. of a head; cs: their pairs.
 __device__ __forceinline__ void rope8(float (&x1)[8], float (&x2)[8],
                                       const float* cs) {
@@ -99,13 +122,23 @@ __device__ __forceinline__ void rope_row(float (&x)[N][8], const float* cs,
     rope8(x[k], x[k + N / 2], cs + (k * 32 + 8 * lg) * 2);
 }
 
+// Of roped queries of 128 dimensions two parts wait in LDS: in registers, of which
+// three blocks a CU leave 168, 8 spilled (8 x 2047 keys 23.8 us for 20.4).
+constexpr bool parts_in_lds(int D, bool rope) { return rope && D > 64; }
+// A wave's floats in LDS: its sums at the end, those parts before.
+template <int D, bool ROPE>
+__host__ __device__ constexpr int wave_floats(int G) {
+  return parts_in_lds(D, ROPE) && G * D < D / 32 * 2 * 256 ? D / 32 * 2 * 256
+                                                           : G * D;
+}
+
 template <int D, bool PAGED, bool ROPE>
 __global__ void __launch_bounds__(64 * WAVES, D == 64 ? 4 : 3)
 k_attn_decode(const DecodeAttn a) {
   constexpr int KS = D / 32;             // steps of a score product
   constexpr int VC = D / 16;             // columns of V a lane loads
   typedef __attribute__((ext_vector_type(VC / 2))) u32 vrow;
-  extern __shared__ __align__(16) float so[];      // [WAVES][G][D], then m, l
+  extern __shared__ __align__(16) float so[];      // [WAVES][G][D], m and l
   const int side = gridDim.x / a.Hkv, hkv = blockIdx.x / side;
   const int split = blockIdx.z * side + blockIdx.x - hkv * side;
   const int b = blockIdx.y;
@@ -129,25 +162,30 @@ k_attn_decode(const DecodeAttn a) {
 
   // queries, head lane % 16 (what the lanes past the last head compute is not
   // used)
-  s16x8 qh[KS], ql[ROPE ? KS : 1];
+  constexpr int NQ = ROPE ? 3 : 1;       // parts; an unroped query is one
+  constexpr int NR = parts_in_lds(D, ROPE) ? 1 : NQ;   // of them in registers
+  int mine = wid * (wave_floats<D, ROPE>(G) / 4) + lane;
+  s16x8 qf[KS][NR];
   {
     const u16* qp = a.q + (long)b * a.q_bs +
                     (long)(hkv * G + min(l15, G - 1)) * D + 8 * lg;
 #pragma unroll
-    for (int k = 0; k < KS; ++k) qh[k] = ld8(qp + k * 32);
-    if (ROPE) {
+    for (int k = 0; k < KS; ++k) qf[k][0] = ld8(qp + k * 32);
+    if constexpr (ROPE) {
       float x[KS][8];
 #pragma unroll
       for (int k = 0; k < KS; ++k)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) x[k][j] = bf2f((u16)qh[k][j]);
+        for (int j = 0; j < 8; ++j) x[k][j] = bf2f((u16)qf[k][0][j]);
       rope_row(x, cs, lg);
 #pragma unroll
       for (int k = 0; k < KS; ++k) {
-        s16x8 p[2];
-        weight_parts(x[k], p);
-        qh[k] = p[0];
-        ql[k] = p[1];
+        s16x8 p[3];
+        parts3(x[k], p);
+#pragma unroll
+        for (int i = 0; i < NR; ++i) qf[k][i] = p[i];
+#pragma unroll
+        for (int i = NR; i < NQ; ++i) ((s16x8*)so)[mine + (k * 2 + i - 1) * 64] = p[i];
       }
     }
   }
@@ -208,14 +246,18 @@ k_attn_decode(const DecodeAttn a) {
 #pragma unroll
           for (int e = 0; e < VC / 2; ++e) vf[r][e] = 0;
     }
+    if (NR < NQ) asm volatile("" : "+v"(mine));      // read each time
+    const s16x8* rest = (const s16x8*)so + mine;
     float s[8];                          // keys 4 lg + 0..3, then 16 on
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < KS; ++k) {
-        acc = mma(kf[t][k], qh[k], acc);
-        if (ROPE) acc = mma(kf[t][k], ql[k], acc);
+#pragma unroll
+        for (int i = NQ - 1; i >= 0; --i)
+          acc = mma(kf[t][k], i < NR ? qf[k][i % NR] : rest[(k * 2 + i - 1) * 64],
+                    acc);
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r)
@@ -235,8 +277,8 @@ k_attn_decode(const DecodeAttn a) {
       ps += s[i];
     }
     l = fmaf(l, al, ps);
-    s16x8 p[2];
-    weight_parts(s, p);
+    s16x8 p[3];
+    parts3(s, p);
 #pragma unroll
     for (int w = 0; w < VC / 2; ++w)
 #pragma unroll
@@ -250,15 +292,16 @@ k_attn_decode(const DecodeAttn a) {
         f32x4& oe = o[2 * w + hf];
 #pragma unroll
         for (int r = 0; r < 4; ++r) oe[r] *= al;
-        oe = mma(va, p[0], oe);
-        oe = mma(va, p[1], oe);
+#pragma unroll
+        for (int i = 2; i >= 0; --i) oe = mma(va, p[i], oe);
       }
   }
   l = head_sum(l);
   // column VC * (4 lg + r) + e of head l15 is o[e][r]
-  float* sml = so + WAVES * G * D;
+  constexpr auto stride = wave_floats<D, ROPE>;
+  float* sml = so + WAVES * stride(G);
   if (l15 < G) {
-    float* dst = so + (wid * G + l15) * D;
+    float* dst = so + wid * stride(G) + l15 * D;
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
@@ -281,7 +324,7 @@ k_attn_decode(const DecodeAttn a) {
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       const float f = __builtin_amdgcn_exp2f(sml[(w * G + g) * 2] - mm);
-      const f32x4 t = *(const f32x4*)(so + (w * G + g) * D + d);
+      const f32x4 t = *(const f32x4*)(so + w * stride(G) + g * D + d);
       ll = fmaf(f, sml[(w * G + g) * 2 + 1], ll);
 #pragma unroll
       for (int e = 0; e < 4; ++e) v[e] = fmaf(f, t[e], v[e]);
@@ -374,9 +417,9 @@ void launch_decode(const DecodeAttn& a, int B, hipStream_t stream) {
                                            (CHUNK * WAVES)));
   const int side = min(all, 16);
   const dim3 grid(a.Hkv * side, B, (all + side - 1) / side), block(64 * WAVES);
-  const size_t lds = (size_t)WAVES * a.G * (D + 2) * sizeof(float);
 #define GO(PAGED, ROPE)                                                       \
-  hipLaunchKernelGGL((k_attn_decode<D, PAGED, ROPE>), grid, block, lds, stream, \
+  hipLaunchKernelGGL((k_attn_decode<D, PAGED, ROPE>), grid, block,            \
+                     WAVES * (wave_floats<D, ROPE>(a.G) + 2 * a.G) * 4, stream, \
                      a)
   if (a.table) {
     if (a.cs) GO(true, true); else GO(true, false);

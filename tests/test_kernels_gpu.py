@@ -201,6 +201,45 @@ def test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, splits, lens):
         assert row_err(got[b], (p.unsqueeze(-1) * vv).sum(1)) < 2 ** -8
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,n,size", [(8, 2, 700, 1), (4, 4, 300, 4),
+                                           (16, 1, 1000, 1)])
+def test_attn_decode_sums_are_float32(lib, D, rope, Hq, Hkv, n, size):
+    """The splits' sums, which are not rounded to bfloat16: queries under RoPE
+    and weights keep float32's 24 bits. Scores are of size ``size`` squared; D
+    roundings of 2^-24 make theirs, and what comes of it is relative to the
+    result: 1e-6. Weights or queries of 16 bits are 2e-6 and more off."""
+    from fei_amd.ops import reference as ref
+    W, T, splits = (Hq + 2 * Hkv) * D, n + 3, 8
+    qkv = randbf(1, W, seed=n) * size
+    q, k, v = (qkv[:, a * D:b * D].view(1, -1, D) for a, b in
+               ((0, Hq), (Hq, Hq + Hkv), (Hq + Hkv, Hq + 2 * Hkv)))
+    kc, vc = randbf(1, Hkv, T, D, seed=1), randbf(1, Hkv, T, D, seed=2)
+    pos = torch.tensor([n - 1], dtype=torch.int32, device=DEV)
+    table = ref.rope_table(T, D, device=DEV)
+    po = torch.zeros(1, Hq, splits, D, device=DEV)
+    ml = torch.zeros(1, Hq, splits, 2, device=DEV)
+    ml[..., 0] = -3e38
+    lib.attn_decode(q, kc, vc, pos, splits=splits, workspace=(po, ml),
+                    **(dict(k=k, v=v, table=table) if rope else {}))
+    used = min(splits, -(-n // 128))
+    assert used > 1 and not ml[:, :, used:, 1].any()
+    top = ml[0, ..., 0].double().amax(-1, keepdim=True)
+    w = torch.exp2(ml[0, ..., 0].double() - top)
+    got = (po[0].double() * w.unsqueeze(-1)).sum(1) \
+        / (ml[0, ..., 1].double() * w).sum(-1, keepdim=True)
+    q64 = q[0].double()
+    if rope:                           # by the same float32 angles
+        c, s = table.view(T, D // 2, 2)[n - 1].double().unbind(-1)
+        a, b = q64.split(D // 2, -1)
+        q64 = torch.cat([a * c - b * s, b * c + a * s], -1)
+    kk, vv = (t[0, :, :n].double().repeat_interleave(Hq // Hkv, 0)
+              for t in (kc, vc))
+    p = torch.softmax((kk * q64.unsqueeze(1)).sum(-1) * D ** -0.5, -1)
+    assert row_err(got, (p.unsqueeze(-1) * vv).sum(1)) < 1e-6
+
+
 # -- products of few rows on the matrix units ------------------------------------
 
 @pytest.mark.parametrize("M", [3, 4, 8, 9, 17, 25, 32, 40, 64])
