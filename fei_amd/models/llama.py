@@ -315,10 +315,13 @@ class LlamaModel:
         # see __init__): each residual GEMV's epilogue accumulates the next
         # norm's sumsq so the norm prologues collapse to one scalar read.
         # The layer-0 attention norm has no producing epilogue (embedding)
-        # and keeps the full prologue.
+        # and keeps the full prologue. Of one row only: with more the products
+        # that take the norm inside have their own sums, and the one buffer has
+        # to stay where a captured step writes it.
         sums = None
         ssq = (self._ssq_slots(B, h.device)
-               if (self.norm_precomp and fp8 is None and h.is_cuda) else None)
+               if (self.norm_precomp and B == 1 and fp8 is None
+                   and h.is_cuda) else None)
         if ssq is not None:
             ssq.zero_()
         pf = self.prefetch_mb > 0 and fp8 is None and h.is_cuda

@@ -236,3 +236,57 @@ def test_hbm_sized_kv_decodes_past_nominal_window():
             else True
     finally:
         eng.shutdown()
+
+
+def test_norm_precompute_is_for_one_row(monkeypatch):
+    """A step of several rows takes no sums of squares by atomics (its products
+    would drop them), and leaves the buffer alone that a captured step of one
+    row writes to."""
+    from fei_amd import ops
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+
+    dev = torch.device("cuda:0")
+    m = LlamaModel(get_spec("llama3-tiny"), dev, torch.bfloat16, seed=9,
+                   max_seq_len=128)
+    m.norm_precomp = True
+    asked = []
+    real = ops.gemv_res
+    monkeypatch.setattr(ops, "gemv_res", lambda *a, **k: (
+        asked.append(k.get("ssq_out") is not None), real(*a, **k))[1])
+
+    held = []                    # what a captured step reads stays alive
+
+    def step(B, fn):
+        kc, vc = m.new_kv_cache(B, 128)
+        tok = torch.arange(B, dtype=torch.int32, device=dev) + 7
+        pos = torch.full((B,), 3, dtype=torch.int32, device=dev)
+        held.append((kc, vc, tok, pos))
+        return fn(lambda: m.forward_decode(tok, pos, kc, vc))
+
+    def capture(fn):
+        fn()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = fn()
+        return g, out
+
+    g, out = step(1, capture)
+    assert asked and all(asked)
+    kept = m._ssq.data_ptr()
+    want = step(1, lambda fn: fn()).clone()
+    for B in (2, 3, 8):
+        del asked[:]
+        got = step(B, lambda fn: fn())
+        assert not any(asked)
+        m.norm_precomp = False
+        plain = step(B, lambda fn: fn())
+        m.norm_precomp = True
+        assert torch.equal(got, plain)
+        assert m._ssq.data_ptr() == kept
+        g.replay()
+        torch.cuda.synchronize()
+        # the sums are added by atomics, in any order
+        err = (out.float() - want.float()).abs().max()
+        assert err <= 2e-2 * want.float().abs().max()
