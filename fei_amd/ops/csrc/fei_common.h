@@ -86,4 +86,16 @@ __device__ __forceinline__ float hash_uniform(u64 x) {
   return ((float)m + 1.0f) * (1.0f / 16777216.0f);
 }
 
+// Says that launches of the kernel use ``bytes`` of LDS, which has to be said beyond
+// 64 KB with what the kernel declares itself (under 16 KB everywhere here). It is a
+// device that is told, and threads have devices of their own: said at every launch,
+// under 0.1 us of its 3.3.
+template <typename Kernel>
+inline void allow_lds(Kernel* kernel, size_t bytes) {
+  if (bytes > 48 * 1024)
+    (void)hipFuncSetAttribute((const void*)kernel,
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)bytes);
+}
+
 #define HIP_CHECK_LAUNCH() do { } while (0)

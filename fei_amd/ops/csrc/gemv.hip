@@ -266,11 +266,7 @@ void launch_gemv(void* out, const void* x, const void* gain, const void* w,
                  hipStream_t stream) {
   const size_t lds = (size_t)M * K * 2;
   auto go = [&](auto kernel, int blocks, size_t bytes) {
-    // beyond 64 KB a kernel has to ask
-    if (bytes > 65536)
-      (void)hipFuncSetAttribute((const void*)kernel,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)bytes);
+    allow_lds(kernel, bytes);
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), bytes, stream,
                        (u16*)out, (const u16*)x, (const u16*)gain, w, wscale,
                        N, K, eps, ssq);
@@ -603,10 +599,7 @@ void launch_skinny(void* out, const void* x, const void* w, int M, int N,
   constexpr int lds = (stages > sums ? stages : sums) * 1024;
   constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : RT;
   auto go = [&](auto kernel, int bytes) {
-    if (bytes > 65536)                    // beyond that a kernel has to ask
-      (void)hipFuncSetAttribute((const void*)kernel,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                bytes);
+    allow_lds(kernel, bytes);
     hipLaunchKernelGGL(kernel, dim3((N + 16 * RO - 1) / (16 * RO)), dim3(256),
                        bytes, stream, out, (const u16*)x, (const u16*)w, M, N,
                        K, ep, nm);

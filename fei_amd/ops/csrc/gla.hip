@@ -564,13 +564,7 @@ void launch_state(float* U, const float* G, const T* proj, long ps,
                   const int* chunks, int n, Gla g, int vec,
                   hipStream_t stream) {
   const size_t lds = 4 * (DT * 16 + 64) * CH;
-  static bool set = false;
-  if (!set) {
-    (void)hipFuncSetAttribute((const void*)k_gla_state<T, DT>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    set = true;
-  }
+  allow_lds(k_gla_state<T, DT>, lds);
   hipLaunchKernelGGL((k_gla_state<T, DT>),
                      dim3(n, g.heads, (g.vdim + 63) / 64), dim3(256), lds,
                      stream, U, G, proj, ps, chunks, g, vec);
@@ -583,12 +577,7 @@ void launch_out(T* out, long os, const float* U, const float* A, const float* G,
   // four tiles at a time, two where there are no more or LDS has no room
   constexpr int NG = NV >= 4 && DK <= 4 ? 4 : 2;
   constexpr int lds = NG * 32 * (DK * 32 + 4 + CH) * 4;
-  static bool set = lds <= 65536;
-  if (!set) {
-    (void)hipFuncSetAttribute((const void*)k_gla_out<T, DK, NV, NG>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    set = true;
-  }
+  allow_lds(k_gla_out<T, DK, NV, NG>, lds);
   hipLaunchKernelGGL((k_gla_out<T, DK, NV, NG>), dim3(n, g.heads),
                      dim3(256 * NG), lds, stream, out, os, U, A, G, proj, ps,
                      nw, chunks, g, eps, vec);

@@ -895,12 +895,7 @@ void launch_panels(u16* out, long os, const u16* proj, long ps, const u16* kv,
   // tiles; afterwards the sums [16 DT][256] and [2][2][256]
   constexpr int lds = (KP + VP) * 16384 > (32 * VP + 4) * 1024
                           ? (KP + VP) * 16384 : (32 * VP + 4) * 1024;
-  static bool set = lds <= 65536;
-  if (!set) {
-    (void)hipFuncSetAttribute((const void*)k_window_panels<KP, VP>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    set = true;
-  }
+  allow_lds(k_window_panels<KP, VP>, lds);
   const int gate_off = g.heads * (g.dim + g.rot) + g.kr + g.rot;
   hipLaunchKernelGGL((k_window_panels<KP, VP>), dim3(g.heads, n_tiles),
                      dim3(512), lds, stream, out, os, proj, ps, kv, krot,
@@ -938,13 +933,7 @@ int run_decode(T* out, long os, const T* proj, long ps, const T* wuk,
   const dim3 gd(splits, (g.heads + 16 * nh - 1) / (16 * nh), B);
 #define DEC(N, H)                                                            \
   do {                                                                       \
-    static bool set = false;                                                 \
-    if (!set) {                                                              \
-      (void)hipFuncSetAttribute((const void*)k_latent_decode<T, N, H>,       \
-                                hipFuncAttributeMaxDynamicSharedMemorySize,  \
-                                160 * 1024);                                 \
-      set = true;                                                            \
-    }                                                                        \
+    allow_lds(k_latent_decode<T, N, H>, lds(KT));                            \
     hipLaunchKernelGGL((k_latent_decode<T, N, H>), gd, dim3(256 * H),        \
                        lds(KT), stream, qa, rows, part_o, part_ml, pos,      \
                        table, W, bs_log, g, splits, KT, Rs, R % 8 == 0);     \
@@ -979,13 +968,7 @@ void launch_window(T* out, long os, const T* proj, long ps, const T* kv,
   constexpr int NW = sizeof(T) == 2 ? 8 : 4;
   const size_t lds = sizeof(T) * (64 * (KS * 32 + 8) + DC * 16 * 64 +
                                   NW * Parts<T>::n * 16 * 72);
-  static bool set = false;
-  if (!set) {
-    (void)hipFuncSetAttribute((const void*)k_window_prefill<T, KS, DC, NW>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    set = true;
-  }
+  allow_lds(k_window_prefill<T, KS, DC, NW>, lds);
   const dim3 grid(g.heads, n_tiles, NW == 8 ? 1 : 2);
   const int gate_off = g.heads * (g.dim + g.rot) + g.kr + g.rot;
   hipLaunchKernelGGL((k_window_prefill<T, KS, DC, NW>), grid, dim3(NW * 64), lds,

@@ -316,13 +316,7 @@ void launch_big(u16* out, const u16* x, const u16* w, const int* order,
                 const int* tiles, const int* count, int max_tiles, int N,
                 int K, int act, hipStream_t stream) {
   constexpr int lds = S * (128 + 32 * WI) * 64 * 2;
-  static bool set = false;
-  if (!set) {
-    (void)hipFuncSetAttribute((const void*)k_moe_gemm_big<WI, S>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lds);
-    set = true;
-  }
+  allow_lds(k_moe_gemm_big<WI, S>, lds);
   const int nx = (N + 32 * WI - 1) / (32 * WI);
   hipLaunchKernelGGL((k_moe_gemm_big<WI, S>),
                      dim3((nx * max_tiles + 7) / 8 * 8), dim3(256), lds,

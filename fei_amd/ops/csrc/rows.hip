@@ -172,12 +172,7 @@ void launch(void* out, const void* x, long xs, const void* w, int M, int N,
             int K, int parts, hipStream_t stream, const void* bias = nullptr) {
   constexpr int lds = S * 32 * (XJ + WI) * 128;
   constexpr int CN = EPI == ROWS_SWIGLU ? 16 * WI : 32 * WI;
-  static bool set = lds <= 65536;          // beyond that a kernel has to ask
-  if (!set) {
-    (void)hipFuncSetAttribute((const void*)k_rows<XJ, WI, S, EPI>,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-    set = true;
-  }
+  allow_lds(k_rows<XJ, WI, S, EPI>, lds);
   const int nx = (N + CN - 1) / CN, nm = (M + 32 * XJ - 1) / (32 * XJ);
   hipLaunchKernelGGL((k_rows<XJ, WI, S, EPI>),
                      dim3((nx * nm + 7) / 8 * 8, parts), dim3(256), lds, stream,

@@ -761,13 +761,6 @@ k_sig_combine(T* __restrict__ out, long os, const float* __restrict__ part,
   out[(long)b * os + c] = El<T>::st(v);
 }
 
-template <typename K>
-void allow_lds(K kernel) {
-  (void)hipFuncSetAttribute((const void*)kernel,
-                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                            160 * 1024);
-}
-
 template <typename T>
 void run_decode(T* out, long os, float* part, const T* proj, long ps, T* rows,
                 float* states, Conv cv, const float* bias, const int* pos,
@@ -778,13 +771,9 @@ void run_decode(T* out, long os, float* part, const T* proj, long ps, T* rows,
   const bool vec = g.dim % 8 == 0 && g.vdim % 8 == 0;
 #define DEC(KS, CPL, VEC)                                                    \
   do {                                                                       \
-    static bool set = false;                                                 \
-    if (!set) {                                                              \
-      allow_lds(k_sig_decode<T, KS, CPL, VEC>);                              \
-      set = true;                                                            \
-    }                                                                        \
     const size_t lds = sizeof(T) * (17 * (KS * 32 + 8) + CPL * 16) +         \
                        4 * 4 * (hg < 16 ? hg : 16) * (CPL * 16 + 4);         \
+    allow_lds(k_sig_decode<T, KS, CPL, VEC>, lds);                           \
     hipLaunchKernelGGL((k_sig_decode<T, KS, CPL, VEC>), grid, dim3(256),     \
                        lds, stream, out, os, part, proj, ps, rows, states,   \
                        cv, bias, pos, slots, table, W, bs_log, g, splits,    \
@@ -862,13 +851,9 @@ void launch_prefill(T* out, long os, const T* q, const T* rows,
   constexpr int QS = sizeof(T) == 2 && KS <= 4 && DC <= 8 ? 2 : 1;
   constexpr int NW = sizeof(T) == 2 ? 8 / QS : 4;
   constexpr int NQ = NW * 16 * QS;
-  static bool set = false;
-  if (!set) {
-    allow_lds(k_sig_prefill<T, KS, DC, NW, QS, VEC>);
-    set = true;
-  }
   const size_t lds = sizeof(T) * (64 * (KS * 32 + 8) + DC * 16 * 64) +
                      16 * (NQ + 68);
+  allow_lds(k_sig_prefill<T, KS, DC, NW, QS, VEC>, lds);
   const dim3 grid(g.heads, n_tiles, 128 / NQ);
   hipLaunchKernelGGL((k_sig_prefill<T, KS, DC, NW, QS, VEC>), grid,
                      dim3(NW * 64), lds, stream, out, os, q, rows, bias,
