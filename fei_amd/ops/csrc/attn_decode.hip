@@ -147,8 +147,13 @@ k_attn_decode(const DecodeAttn a) {
   const int l15 = lane & 15, lg = lane >> 4;
   const int n = keys_at(a, b), last = n - 1;
   const int chunks = (n + CHUNK - 1) / CHUNK, used = used_splits(a, n);
-  if (split >= used) return;
   const int G = a.G, Hq = a.Hkv * G;
+  if (split >= used) {
+    if (used <= 0 && split == 0)         // no key: zeros
+      for (int i = tid; i < G * D; i += 64 * WAVES)
+        a.out[((long)b * Hq + hkv * G) * D + i] = 0;
+    return;
+  }
 
   auto row = [&](int key) {
     if (PAGED) {

@@ -201,6 +201,33 @@ def test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, splits, lens):
         assert row_err(got[b], (p.unsqueeze(-1) * vv).sum(1)) < 2 ** -8
 
 
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("T,splits", [(64, 4), (512, 1), (512, 8)])
+def test_attn_decode_without_keys(lib, paged, T, splits):
+    """A position before the first: zeros, whether one block or several would
+    have the keys, and no cache row."""
+    from fei_amd.ops import reference as ref
+    B, Hq, Hkv, D, BS = 3, 4, 2, 64, 16
+    q, k, v = (randbf(B, H, D, seed=H) for H in (Hq, Hkv, Hkv + 5))
+    v = v[:, :Hkv].contiguous()
+    pos = torch.tensor([-1, 5, -200], dtype=torch.int32, device=DEV)
+    shape = (B * (T // BS), Hkv, BS, D) if paged else (B, Hkv, T, D)
+    kc, vc = (torch.zeros(shape, device=DEV, dtype=torch.bfloat16)
+              for _ in range(2))
+    out = torch.full((B, Hq, D), float("nan"), device=DEV, dtype=torch.bfloat16)
+    args = dict(splits=splits, k=k, v=v, out=out,
+                table=ref.rope_table(T, D, device=DEV))
+    if paged:
+        bt = torch.arange(shape[0], device=DEV, dtype=torch.int32).view(B, -1)
+        lib.attn_decode_paged(q, kc, vc, bt, pos, **args)
+        kc, vc = (c.view(B, T // BS, Hkv, BS, D) for c in (kc, vc))
+    else:
+        lib.attn_decode(q, kc, vc, pos, **args)
+    assert not out[0].any() and not out[2].any() and out[1].isfinite().all()
+    for c in (kc, vc):
+        assert not c[0].any() and not c[2].any() and c[1].any()
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("rope", [False, True])
 @pytest.mark.parametrize("Hq,Hkv,n,size", [(8, 2, 700, 1), (4, 4, 300, 4),
