@@ -220,7 +220,7 @@ class LlamaModel:
                 token, pos, k_caches, v_caches, attn_splits, workspace,
                 fused_attn, attn_out, fused_norm)
         s = self.spec
-        h = F.embedding(token, self.emb)                 # residual stream
+        h = self._embed(token)                           # residual stream
         scale = 1.0 / math.sqrt(self.D)
         n_layers = len(self.layers)
         x = ops.rmsnorm(h, self.layers[0].norm_attn, s.norm_eps)
@@ -250,6 +250,13 @@ class LlamaModel:
         if gather_logits:
             logits = all_gather_cat(logits, dim=-1, ctx=self.tp)
         return logits
+
+    def _embed(self, token: torch.Tensor) -> torch.Tensor:
+        """Rows of whole numbers of any type; F.embedding takes two of them as
+        they are, without a launch to convert."""
+        if token.dtype not in (torch.int32, torch.int64):
+            token = token.long()
+        return F.embedding(token, self.emb)
 
     def fused_layers(self, h: torch.Tensor, attend) -> Optional[torch.Tensor]:
         """All layers over the residual ``h`` [rows, C], in place; fused_rows
@@ -309,7 +316,7 @@ class LlamaModel:
         s = self.spec
         B = token.shape[0]
         fp8 = getattr(self, "fp8", None) if use_fp8 and B == 1 else None
-        h = F.embedding(token, self.emb)
+        h = self._embed(token)
         scale = 1.0 / math.sqrt(self.D)
         # norm-precompute chain (opt-in FEI_NORM_PRECOMP=1; measured loss,
         # see __init__): each residual GEMV's epilogue accumulates the next

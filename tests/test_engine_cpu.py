@@ -571,3 +571,16 @@ def test_hbm_seq_plumbing_cpu():
     assert eng.max_seq_len == eng.spec.max_seq_len
     out = eng.generate("abc", max_new_tokens=4, stop_on_eos=False)
     assert len(out["token_ids"]) == 4
+
+
+@pytest.mark.parametrize("dtype", [torch.int16, torch.uint8, torch.int32,
+                                   torch.int64])
+@pytest.mark.parametrize("fused", [False, True])
+def test_decode_takes_tokens_of_any_whole_type(dtype, fused):
+    m = LlamaModel(get_spec("llama3-tiny"), torch.device("cpu"), torch.float32,
+                   seed=1, max_seq_len=16)
+    pos = torch.zeros(1, dtype=torch.int32)
+    a, b = (m.forward_decode(torch.tensor([7]).to(t), pos, *m.new_kv_cache(1, 16),
+                             fused_norm=fused) for t in (dtype, torch.int64))
+    assert torch.equal(a, b)
+
