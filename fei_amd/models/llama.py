@@ -315,7 +315,10 @@ class LlamaModel:
                                    attn_out, use_fp8):
         s = self.spec
         B = token.shape[0]
-        fp8 = getattr(self, "fp8", None) if use_fp8 and B == 1 else None
+        # fp8 pays for one row, of up to 16384: the products that read it hold
+        # 32 KB of activations in LDS
+        fp8 = (getattr(self, "fp8", None)
+               if use_fp8 and B == 1 and s.hidden_size <= 16384 else None)
         h = self._embed(token)
         scale = 1.0 / math.sqrt(self.D)
         # norm-precompute chain (opt-in FEI_NORM_PRECOMP=1; measured loss,

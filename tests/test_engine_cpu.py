@@ -584,3 +584,23 @@ def test_decode_takes_tokens_of_any_whole_type(dtype, fused):
                              fused_norm=fused) for t in (dtype, torch.int64))
     assert torch.equal(a, b)
 
+
+@pytest.mark.parametrize("hidden,fp8", [(256, True), (16384, True),
+                                        (16448, False)])
+def test_fp8_rows_that_the_products_hold(hidden, fp8):
+    """Wider models decode with the weights as they were loaded."""
+    import dataclasses
+    spec = dataclasses.replace(
+        get_spec("llama3-tiny"), hidden_size=hidden, num_layers=1, num_heads=1,
+        num_kv_heads=1, intermediate_size=64, vocab_size=64)
+    m = LlamaModel(spec, torch.device("cpu"), torch.float32, seed=1,
+                   max_seq_len=8)
+    tok, pos = torch.tensor([7]), torch.zeros(1, dtype=torch.int32)
+    run = lambda fused: m.forward_decode(tok, pos, *m.new_kv_cache(1, 8),
+                                         fused_norm=fused)
+    want = run(False)
+    m.quantize_fp8()
+    got = run(True)
+    off = float((got - want).norm() / want.norm())
+    assert off > 1e-3 if fp8 else off < 1e-5
+
