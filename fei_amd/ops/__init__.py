@@ -394,9 +394,10 @@ def swiglu(gate_up: torch.Tensor,
 def argmax(x: torch.Tensor) -> torch.Tensor:
     """x.argmax(-1) of rows [B, V]: the first of the largest values."""
     if not (x.is_cuda and x.dim() == 2 and x.is_contiguous() and x.numel()
+            and x.shape[0] <= 65535 and x.shape[1] < 1 << 30
             and x.dtype in (torch.bfloat16, torch.float32)):
         return x.argmax(dim=-1)
-    B, V = x.shape
+    B, V = x.shape               # rows are the second dimension of a grid
     chunks = max(1, min(64, 512 // B, -(-V // 2048)))
     out = torch.empty(B, dtype=torch.int64, device=x.device)
     part = torch.empty(B, chunks, dtype=torch.int64, device=x.device)

@@ -695,7 +695,7 @@ def test_gla_prompt_tiles(lib, dim, vdim, dtype, tol):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("B,V", [(1, 1), (3, 7), (20, 128256), (2, 2049),
-                                 (600, 64), (5, 50257)])
+                                 (600, 64), (5, 50257), (65535, 3), (65536, 3)])
 def test_argmax_is_the_first(lib, dtype, B, V):
     """Ties, infinities, NaN and zeros of both signs."""
     g = torch.Generator(device=DEV).manual_seed(V)
