@@ -500,14 +500,14 @@ void fei_moe_plan(int* order, int* place, int* tiles, int* count,
                      tiles, count, ids, n, E, top, rows, max_tiles);
 }
 
-// bits: 1 = float32, 2 = tiles of 128 slots (else 32); likely: tiles if all experts
-// have as many slots
+// bits: 1 = float32, 2 = tiles of 128 slots (else 32); likely: tiles to expect, for
+// the choice of blocks alone
 void fei_moe_gemm(void* out, const void* x, const void* w, const int* order,
                   const int* tiles, const int* count, int max_tiles,
                   int likely, int N, int K, int act, int bits,
                   hipStream_t stream) {
   if (bits & 2) {
-// 128 or 192 columns a block, with two buffers (two blocks a CU) or three
+    // 128 or 192 columns a block, with two buffers (two blocks a CU) or three
     // (one, whose loads are further ahead: 0.7 of the time where every CU has
     // one block to do). What a round of blocks takes goes with the rows that a
     // step loads, 32 (WI + 4). 6824 slots of 16 experts, 64 tiles: 768 columns

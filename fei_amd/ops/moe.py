@@ -9,6 +9,7 @@ tiles each belong to one expert.
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Tuple
 
 import torch
@@ -55,6 +56,18 @@ def route(logits: torch.Tensor, top: int, scale: float
     return ids, w
 
 
+def likely_tiles(n: int, E: int, rows: int) -> int:
+    """Tiles of ``rows`` slots to expect of n slots that are dealt to E experts
+    by chance: an expert has n / E of them, give or take the root of that, and
+    a tile more or fewer if it comes over an edge. Blocks of the grouped product
+    are chosen by it, and one tile too many for a round of them takes another
+    round (1908 rows, 16 experts, top 4: 65 tiles, 48 us for 35)."""
+    share, full = n / E, -(-n // (E * rows))
+    past = lambda edge: 0.5 * math.erfc(abs(edge - share) / (2 * share) ** 0.5)
+    fewer = past((full - 1) * rows) if full > 1 else 0.0
+    return round(E * (full + past(full * rows) - fewer))
+
+
 def residual_moe(x: torch.Tensor, h: GainNormed, router: torch.Tensor,
                  a: torch.Tensor, w_o: torch.Tensor, up: torch.Tensor,
                  down: torch.Tensor, f, mult: float) -> torch.Tensor:
@@ -93,7 +106,7 @@ def residual_moe(x: torch.Tensor, h: GainNormed, router: torch.Tensor,
         and n >= 32 * E
     rows = 128 if big else 32
     max_tiles = min(n, n // rows + E)
-    likely = min(max_tiles, E * -(-n // (E * rows)))
+    likely = min(max_tiles, likely_tiles(n, E, rows))
     meta = torch.empty(2 * n + 3 * max_tiles + 1, dtype=torch.int32,
                        device=dev)
     order, place = meta[:n], meta[n:2 * n]

@@ -138,3 +138,21 @@ def test_views_of_few_rows(T):
         assert row_err(act[:, ff:2 * ff],
                        torch.nn.functional.silu(g) * u) < 2 ** -6
         assert not act[:, :ff].any() and not act[:, 2 * ff:].any()
+
+
+@pytest.mark.parametrize("E,top,rows", [(16, 4, 128), (8, 2, 128), (4, 1, 32),
+                                        (64, 8, 128)])
+def test_tiles_to_expect(E, top, rows):
+    """Against experts drawn by chance."""
+    from fei_amd.ops.moe import likely_tiles
+    g = torch.Generator().manual_seed(E)
+    for T in (300, 500, 800, 900, 1000, 1500, 1908, 2048, 4000):
+        n = T * top
+        if n < 32 * E:
+            continue
+        seen = []
+        for _ in range(30):
+            ids = torch.rand(T, E, generator=g).topk(top, 1).indices.flatten()
+            seen.append(int((-(-ids.bincount(minlength=E) // rows)).sum()))
+        # the mean of 30, and that top choices of a row are never the same
+        assert abs(likely_tiles(n, E, rows) - sum(seen) / 30) < 1 + 0.05 * E
