@@ -580,11 +580,13 @@ def _gemv_ok(M: int, K: int) -> bool:
     return M in _GEMV_ROWS and K % 8 == 0
 
 
-def _norm_inside(how: str, M: int, K: int, sums) -> bool:
+def _norm_inside(how: str, M: int, K: int, sums, wnorm) -> bool:
     """Whether a product takes rows under a norm: the GEMV keeps them in LDS;
-    the tile for few rows needs their sums of squares, and keeps the gains."""
+    the tile for few rows needs their sums of squares, and keeps the gains,
+    which go to LDS by loads that have to be aligned."""
     if how == "skinny":
-        return sums is not None and K <= 16384
+        return (sums is not None and K <= 16384
+                and wnorm.data_ptr() % 16 == 0)
     return M * K * 2 <= 128 * 1024
 
 
@@ -721,7 +723,7 @@ def gemv_norm(res: torch.Tensor, wnorm: torch.Tensor, w: torch.Tensor,
     how = _product(res, w, N, out)
     if how is None:
         return torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w)
-    if not _norm_inside(how, M, K, sums):
+    if not _norm_inside(how, M, K, sums, wnorm):
         return linear_decode(rmsnorm(res, wnorm, eps), w, out)
     if out is None:
         out = torch.empty(*res.shape[:-1], N, dtype=res.dtype, device=res.device)
@@ -747,7 +749,7 @@ def gemv_swiglu_norm(res: torch.Tensor, wnorm: torch.Tensor,
     how = _product(res, wgu, I, out)
     if how is None:
         return swiglu(torch.nn.functional.linear(rmsnorm(res, wnorm, eps), wgu))
-    if not _norm_inside(how, M, K, sums):
+    if not _norm_inside(how, M, K, sums, wnorm):
         return gemv_swiglu(rmsnorm(res, wnorm, eps), wgu, out)
     if out is None:
         out = torch.empty(*res.shape[:-1], I, dtype=res.dtype, device=res.device)

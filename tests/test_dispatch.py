@@ -65,6 +65,36 @@ def test_products_want_plain_weights(M):
         assert not ops._fits(bad, x, M * 48)
 
 
+def test_gains_in_lds_are_aligned():
+    K, sums = 128, torch.zeros(4, 8)
+    buf = torch.zeros(K + 8, dtype=torch.bfloat16)
+    assert buf.data_ptr() % 16 == 0
+    for at, inside in ((0, True), (1, False), (2, False), (4, False), (8, True)):
+        assert ops._norm_inside("skinny", 4, K, sums, buf[at:at + K]) == inside
+        assert ops._norm_inside("gemv", 4, K, None, buf[at:at + K])
+    assert not ops._norm_inside("skinny", 4, K, None, buf[:K])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 32])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+def test_gains_anywhere(M, shift):
+    K, N = 256, 64
+    x, h = rand(M, K, seed=1, dev=DEV), rand(M, K, seed=2, dev=DEV)
+    w0 = rand(K, K, seed=3, dev=DEV, scale=K ** -0.5)
+    w = rand(N, K, seed=4, dev=DEV, scale=K ** -0.5)
+    gain = (1 + 0.2 * rand(K + 8, seed=5, dev=DEV))[shift:shift + K]
+    sums = ops.add_product(x, w0, h)
+    h64 = h.double()
+    y = (h64 * (h64.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()
+         * gain.double()) @ w.double().t()
+    # rows rounded under their gains, results once more
+    assert row_err(ops.gemv_norm(h, gain, w, 1e-5, sums=sums), y) < 2 ** -7
+    want = torch.nn.functional.silu(y[:, :N // 2]) * y[:, N // 2:]
+    assert row_err(ops.gemv_swiglu_norm(h, gain, w, 1e-5, sums=sums),
+                   want) < 2 ** -6
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [1, 3, 5, 8, 9, 32, 40])
 def test_products_of_other_types_and_layouts(M):
