@@ -567,12 +567,6 @@ def _launch_gemv(out, x2, gain, w, wscale, N: int, eps: float, epi: int,
                            _stream())
 
 
-# Kept for callers that set it: a decode attention's splits are always added by
-# a launch of their own (adding them in the attention kernel behind flags was
-# no faster, profiles/r02_fused_combine.md).
-_FUSED_CMB = False
-
-
 _GEMV_ROWS = (1, 2, 3, 4, 8)
 
 
