@@ -584,26 +584,26 @@ def _norm_inside(how: str, M: int, K: int, sums, wnorm) -> bool:
     return M * K * 2 <= 128 * 1024
 
 
-def _product(x: torch.Tensor, w: torch.Tensor, rows_out: int,
+def _product(x: torch.Tensor, w: torch.Tensor, M: int, K: int, rows_out: int,
              out: Optional[torch.Tensor] = None) -> Optional[str]:
-    """Which kernel takes x @ w^T: "skinny" (matrix units), "gemv", or None
-    (the library; CPU). ``out``: where the caller wants the results."""
-    K = x.shape[-1]
-    M = x.numel() // K if K else 0
-    if not x.is_cuda or not M or not rows_out:
+    """Which kernel takes the M rows x @ w^T: "skinny" (matrix units), "gemv",
+    or None (the library; CPU). ``out``: where the caller wants the results."""
+    if not (x.is_cuda and M and rows_out and (
+            out is None or _fits(out, x, M * rows_out))):
         return None
-    return _kernel_for(x, w, M, K) if _fits(out, x, M * rows_out) else None
+    return _kernel_for(x, w, M, K)
 
 
 def _fits(out: Optional[torch.Tensor], x: torch.Tensor, n: int) -> bool:
     """Whether a kernel can write its n results, of x's type, to out."""
-    return out is None or (out.dtype == x.dtype and out.numel() == n
-                           and out.is_contiguous() and out.device == x.device)
+    return out is None or (out.dtype is x.dtype and out.numel() == n
+                           and out.is_contiguous()
+                           and out.get_device() == x.get_device())
 
 
 def _kernel_for(x: torch.Tensor, w: torch.Tensor, M: int,
                 K: int) -> Optional[str]:
-    if not _mixers.match(x, w):
+    if not _mixers.match(x, w, K):
         return None
     # the callers copy rows with gaps; a copy is aligned
     if _mixers.skinny_sizes(M, K, x if x.is_contiguous() else w, w, 2):
@@ -623,8 +623,9 @@ def linear_decode(x: torch.Tensor, w: torch.Tensor,
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """F.linear for skinny M: streaming GEMV or matrix-core tile on GPU. Falls
     back to torch for unsupported shapes/CPU."""
-    M, K, N = x.numel() // x.shape[-1], x.shape[-1], w.shape[0]
-    how = _product(x, w, N, out)
+    K, N = x.shape[-1], w.shape[0]
+    M = x.numel() // K
+    how = _product(x, w, M, K, N, out)
     if how is None:
         return torch.nn.functional.linear(x, w)
     x2 = x.contiguous().view(M, K)
@@ -640,12 +641,11 @@ def linear_decode(x: torch.Tensor, w: torch.Tensor,
 def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Fused gate/up product + SwiGLU: x [M,K] @ [2I,K]^T -> silu(g)*u [M,I]."""
-    M = x.numel() // x.shape[-1]
-    K = x.shape[-1]
-    I = wgu.shape[0] // 2
-    how = _product(x, wgu, I, out)
+    K, I = x.shape[-1], wgu.shape[0] // 2
+    M = x.numel() // K
+    how = _product(x, wgu, M, K, I, out)
     if (how is None and x.is_cuda and _rows.swiglu_ok(M, x, wgu)
-            and _mixers.match(x, wgu) and _fits(out, x, M * I)):
+            and _mixers.match(x, wgu, K) and _fits(out, x, M * I)):
         how = "rows"
     if how is None:
         return swiglu(torch.nn.functional.linear(x, wgu))
@@ -670,8 +670,9 @@ def gemv_res(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
     sum-of-squares of the updated residual rows, which a following
     gemv_norm/gemv_swiglu_norm takes as ``ssq``. Ignored on the CPU fallback —
     consumers recompute exactly there."""
-    M, K, N = x.numel() // x.shape[-1], x.shape[-1], w.shape[0]
-    how = _product(x, w, N, res)
+    K, N = x.shape[-1], w.shape[0]
+    M = x.numel() // K
+    how = _product(x, w, M, K, N, res)
     if ssq_out is not None and how == "skinny" and _gemv_ok(M, K):
         how = "gemv"
     if how is None:
@@ -693,8 +694,9 @@ def add_product(x: torch.Tensor, w: torch.Tensor,
     """gemv_res, for a chain: returns the sums of squares of the new rows by
     tiles of columns, for the ``sums`` of the products that read them under a
     norm, or None where those do not need them."""
-    M, K, N = x.numel() // x.shape[-1], x.shape[-1], w.shape[0]
-    if _product(x, w, N, res) != "skinny":
+    K, N = x.shape[-1], w.shape[0]
+    M = x.numel() // K
+    if _product(x, w, M, K, N, res) != "skinny":
         gemv_res(x, w, res)
         return None
     sums = torch.empty(M, -(-N // 16), dtype=torch.float32, device=x.device)
@@ -713,8 +715,9 @@ def gemv_norm(res: torch.Tensor, wnorm: torch.Tensor, w: torch.Tensor,
     ``ssq`` [M] f32: the sums of squares of res rows, if the caller has them
     (from a prior gemv_res ``ssq_out``). ``sums``: what add_product returned
     for these rows."""
-    M, K, N = res.numel() // res.shape[-1], res.shape[-1], w.shape[0]
-    how = _product(res, w, N, out)
+    K, N = res.shape[-1], w.shape[0]
+    M = res.numel() // K
+    how = _product(res, w, M, K, N, out)
     if how is None:
         return torch.nn.functional.linear(rmsnorm(res, wnorm, eps), w)
     if not _norm_inside(how, M, K, sums, wnorm):
@@ -737,10 +740,9 @@ def gemv_swiglu_norm(res: torch.Tensor, wnorm: torch.Tensor,
                      sums: Optional[torch.Tensor] = None) -> torch.Tensor:
     """out = silu(g)*u where [g;u] = rmsnorm(res)*wnorm @ wgu^T.
     ``ssq``, ``sums``: see gemv_norm."""
-    M = res.numel() // res.shape[-1]
-    K = res.shape[-1]
-    I = wgu.shape[0] // 2
-    how = _product(res, wgu, I, out)
+    K, I = res.shape[-1], wgu.shape[0] // 2
+    M = res.numel() // K
+    how = _product(res, wgu, M, K, I, out)
     if how is None:
         return swiglu(torch.nn.functional.linear(rmsnorm(res, wnorm, eps), wgu))
     if not _norm_inside(how, M, K, sums, wnorm):

@@ -13,6 +13,7 @@ from typing import Optional, Tuple
 
 import torch
 
+import fei_amd.ops as _ops     # half made yet: it imports this
 from fei_amd.ops import reference as ref
 from fei_amd.ops import rows as _rows
 from fei_amd.ops.rows import SKINNY_ROWS
@@ -53,13 +54,11 @@ def declare(lib: ctypes.CDLL) -> None:
 
 
 def _lib() -> ctypes.CDLL:
-    from fei_amd import ops
-    return ops.require_lib()
+    return _ops.require_lib()
 
 
 def _stream() -> int:
-    from fei_amd import ops
-    return ops._stream()
+    return _ops._stream()
 
 
 def _p(t: Optional[torch.Tensor]):
@@ -156,20 +155,26 @@ class GainNormed:
                 and self.x.shape[0] > 0)
 
 
-def match(x: torch.Tensor, w: torch.Tensor) -> bool:
+_BF16 = torch.bfloat16
+
+
+def match(x: torch.Tensor, w: torch.Tensor, K: int) -> bool:
     """Whether pointers stand for x [.., K], or a copy without gaps, and w
     [N, K] in a kernel: bfloat16, w without gaps, sizes that fit, on one device;
     and nobody asks for a gradient, which the library's products have."""
-    return (x.dtype == w.dtype == torch.bfloat16 and w.dim() == 2
-            and w.is_contiguous() and x.shape[-1] == w.shape[1]
-            and x.device == w.device
-            and not (torch.is_grad_enabled()
-                     and (x.requires_grad or w.requires_grad)))
+    # 1 us, once or twice a launch: get_device, which is -1 of the CPU, is a
+    # third of what comparing devices takes
+    size = w.shape
+    return (x.dtype is _BF16 and w.dtype is _BF16 and len(size) == 2
+            and size[1] == K and w.is_contiguous()
+            and x.get_device() == w.get_device()
+            and not ((x.requires_grad or w.requires_grad)
+                     and torch.is_grad_enabled()))
 
 
 def plain(x: torch.Tensor, w: torch.Tensor) -> bool:
     """The same for x as it lies."""
-    return x.is_contiguous() and match(x, w)
+    return x.is_contiguous() and match(x, w, x.shape[-1])
 
 
 def dense(t: torch.Tensor, dtype: torch.dtype, like: torch.Tensor,

@@ -8,6 +8,8 @@ from typing import Tuple
 
 import torch
 
+import fei_amd.ops as _ops     # half made yet: it imports this
+
 _vp, _i, _f, _l = (ctypes.c_void_p, ctypes.c_int, ctypes.c_float,
                    ctypes.c_long)
 
@@ -25,13 +27,11 @@ def declare(lib: ctypes.CDLL) -> None:
 
 
 def _lib() -> ctypes.CDLL:
-    from fei_amd import ops
-    return ops.require_lib()
+    return _ops.require_lib()
 
 
 def _stream() -> int:
-    from fei_amd import ops
-    return ops._stream()
+    return _ops._stream()
 
 
 def _p(t: torch.Tensor) -> int:

@@ -547,7 +547,7 @@ def test_gemv_ssq_chain(lib, M, K):
     wn = randbf(K, seed=333, scale=0.5)
     w2 = randbf(N, K, seed=334, scale=0.02)
     wgu = randbf(2 * I, K, seed=335, scale=0.02)
-    assert lib._product(res, w2, N) == "gemv"
+    assert lib._product(res, w2, M, K, N) == "gemv"
 
     want = res.double() + x.double() @ w.double().t()
     ssq = torch.zeros(M, dtype=torch.float32, device=res.device)
