@@ -2,10 +2,10 @@
 (BERT-style: 12 layers, 768 hidden, 12 heads, post-LayerNorm residual
 blocks, GELU MLP, biased linears).
 
-Products of few rows run in this library's matrix-core tile (up to 32 rows all
-layers are launched from one call), others in the BLAS library; bidirectional
-attention in the HIP prompt kernel (causal=0), LayerNorm with the residual and
-GELU in HIP kernels. Weights are random-init — there is no network for
+Up to 1024 rows all layers are launched from one call (ops.encoder_layers), their
+products in this library's matrix-core tiles; beyond, and for one or two rows, the
+products are the BLAS library's. Bidirectional attention runs in the HIP prompt
+kernel (causal=0), LayerNorm with the residual and GELU in HIP kernels. Weights are random-init — there is no network for
 checkpoints — but the architecture matches bge-base so real weights could
 be loaded via the same tensors.
 

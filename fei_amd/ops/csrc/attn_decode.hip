@@ -12,7 +12,7 @@
 // weights enter the bfloat16 products as three parts, whose sum is the float32
 // value: 3e-7 of a row's float32 result is what the whole is off by, as much as
 // products on the vector units (4e-7); with two parts it was 3e-6, 6 % faster. An
-// infinite key or value makes a row NaN (0 times it, in a part).
+// infinite key or value gives NaN (0 times it, in a part).
 // The chunks go to the blocks' waves in order, so that short contexts end in
 // few blocks (one: it writes the result), and the rest leave at once.
 //
@@ -21,8 +21,8 @@
 // key with the products on the vector units and the scores exchanged through LDS:
 // 300 keys, 32/8 heads of 64: 13.5 -> 6.1 us; 512, 3400 and 8000 keys, 32/8 of
 // 128: 15.7 -> 8.2, 21.4 -> 9.7 and 25.3 -> 13.7; 8 sequences of 2047: 32.5 ->
-// 20.4; 32 of 500: 72 -> 21.2; 20 of 600, heads of 64: 49 -> 12.4. The combine
-// takes 4 to 5, a launch's least.
+// 20.4; 32 of 500: 72 -> 21.2; 20 of 600, heads of 64: 49 -> 12.4. The combine is
+// 3.3 (heads of 64) to 5 of it, a launch's least.
 #include "fei_attn.h"
 
 namespace {
@@ -55,12 +55,6 @@ __device__ __forceinline__ int used_splits(const DecodeAttn& a, int n) {
   return min(a.splits, (n + CHUNK * WAVES - 1) / (CHUNK * WAVES));
 }
 
-__device__ __forceinline__ f32x2 swap32(float v) {
-  const u32 u = __builtin_bit_cast(u32, v);
-  const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-  const u32 r0 = r[0], r1 = r[1];
-  return f32x2{__builtin_bit_cast(float, r0), __builtin_bit_cast(float, r1)};
-}
 __device__ __forceinline__ f32x2 swap16(float v) {
   const u32 u = __builtin_bit_cast(u32, v);
   const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
@@ -69,12 +63,12 @@ __device__ __forceinline__ f32x2 swap16(float v) {
 }
 // Over the four lanes of a head, lane % 16 alike.
 __device__ __forceinline__ float head_max(float v) {
-  f32x2 t = swap32(v);
+  f32x2 t = both_halves(v);
   t = swap16(fmaxf(t[0], t[1]));
   return fmaxf(t[0], t[1]);
 }
 __device__ __forceinline__ float head_sum(float v) {
-  f32x2 t = swap32(v);
+  f32x2 t = both_halves(v);
   t = swap16(t[0] + t[1]);
   return t[0] + t[1];
 }
@@ -375,12 +369,12 @@ __global__ void __launch_bounds__(256) k_attn_decode_combine(const DecodeAttn a)
   if (lane >= used) t = f32x2{M_NONE, 0.f};
   float m = row16_max(t[0]);
   f32x2 sw = swap16(m);
-  sw = swap32(fmaxf(sw[0], sw[1]));
+  sw = both_halves(fmaxf(sw[0], sw[1]));
   m = fmaxf(sw[0], sw[1]);
   const float w = __builtin_amdgcn_exp2f(t[0] - m);    // of split ``lane``
   float l = row16_sum(t[1] * w);
   sw = swap16(l);
-  sw = swap32(sw[0] + sw[1]);
+  sw = both_halves(sw[0] + sw[1]);
   l = sw[0] + sw[1];
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll

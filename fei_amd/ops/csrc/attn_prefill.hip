@@ -17,12 +17,12 @@
 //
 // What bounds it: per 64 keys a wave has 32 matrix instructions (1024 cycles
 // at D = 128) and about as many cycles of softmax; two blocks per CU overlap
-// the two, and the LDS reads (32 KB a wave) take as long again. Measured against
-// a wave of 16 queries of one head with the values turned on the way into LDS:
-// 2048 tokens, 32/8 heads of 128: 282 -> 50 us (690 TFLOP/s of the causal
-// half); 6 x 1001 tokens, heads of 64: 235 -> 42; 64 x 256, 12 heads of 64,
-// not causal: 59 -> 29; 75 tokens over 1875 keys: 139 -> 20 with splits (24
-// blocks without).
+// the two, and the LDS reads (32 KB a wave) take as long again. Measured in a
+// model's layers against a wave of 16 queries of one head with the values turned
+// on the way into LDS: 2048 tokens, 32/8 heads of 128: 282 -> 63 us (545 TFLOP/s
+// of the causal half); 6 x 1001 tokens, heads of 64: 235 -> 49; 64 x 256, 12 heads
+// of 64, not causal: 59 -> 32; 75 tokens over 1875 keys: 139 -> 20 with splits and
+// their combine (24 blocks without).
 #include "fei_mma.h"
 
 namespace {

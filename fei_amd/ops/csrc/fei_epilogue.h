@@ -16,8 +16,9 @@ struct Epilogue {
   const float* bias;   // per column, may be null
   float scale;
   float cap;           // 0: no softcap
-  // EPI_SWIGLU: rows of act are ``as`` apart. EPI_PARALLEL: n_mix columns go to out, the next n_router to router, of
-  // the rest relu(.)^2 to act, whose rows are ``as`` apart
+  // EPI_SWIGLU: rows of act are ``as`` apart. EPI_PARALLEL: n_mix columns go to
+  // out, the next n_router to router, of the rest relu(.)^2 to act, whose rows
+  // are ``as`` apart
   int n_mix, n_router;
   float* router;
   u16* act;
