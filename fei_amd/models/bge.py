@@ -5,9 +5,9 @@ blocks, GELU MLP, biased linears).
 Up to 1024 rows all layers are launched from one call (ops.encoder_layers), their
 products in this library's matrix-core tiles; beyond, and for one or two rows, the
 products are the BLAS library's. Bidirectional attention runs in the HIP prompt
-kernel (causal=0), LayerNorm with the residual and GELU in HIP kernels. Weights are random-init — there is no network for
-checkpoints — but the architecture matches bge-base so real weights could
-be loaded via the same tensors.
+kernel (causal=0), LayerNorm with the residual and GELU in HIP kernels. Weights are
+random-init — there is no network for checkpoints — but the architecture matches
+bge-base so real weights could be loaded via the same tensors.
 
 Output: mean-pooled last hidden state, L2-normalised — [B, hidden].
 """

@@ -622,7 +622,7 @@ def own_product(M: int, w: torch.Tensor) -> bool:
 def linear_decode(x: torch.Tensor, w: torch.Tensor,
                   out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """F.linear for skinny M: streaming GEMV or matrix-core tile on GPU. Falls
-    back to torch for unsupported shapes/CPU."""
+    back to torch for unsupported shapes, types and layouts, and on the CPU."""
     K, N = x.shape[-1], w.shape[0]
     M = x.numel() // K
     how = _product(x, w, M, K, N, out)
