@@ -474,9 +474,16 @@ class LlamaModel:
             all_reduce_sum(o, self.tp)
             x, h = ops.fused_add_rmsnorm(o, h, lw.norm_mlp, s.norm_eps)
             act = ops.gemv_swiglu(x, lw.wgu)
-            d = ops.linear_decode(act, lw.wdown)
+            T, norm = act.numel() // act.shape[-1], self._norm_after(li)
+            act = act.view(T, -1)
+            if self.tp_size == 1 and ops.tile_parts_ok(T, act, lw.wdown):
+                x = ops.add_norm_parts(ops.tile_parts(act, lw.wdown),
+                                       h.view(T, -1), norm,
+                                       s.norm_eps).view_as(h)
+                continue
+            d = ops.linear_decode(act, lw.wdown).view_as(h)
             all_reduce_sum(d, self.tp)
-            x, h = ops.fused_add_rmsnorm(d, h, self._norm_after(li), s.norm_eps)
+            x, h = ops.fused_add_rmsnorm(d, h, norm, s.norm_eps)
         return x
 
     # -- checkpointing (safetensors) -----------------------------------------

@@ -24,6 +24,7 @@ from fei_amd.ops import moe as _moe
 from fei_amd.ops import reference as ref
 from fei_amd.ops import rows as _rows
 from fei_amd.ops import sigmoid_attn as _sigmoid_attn
+from fei_amd.ops import tiles as _tiles
 from fei_amd.ops.mixers import (  # noqa: F401
     GainNorm, GainNormed, cat_cast, check_gla_geometry,
     check_latent_geometry, embed_pos, gain_logits, gla_decode, gla_prefill,
@@ -35,6 +36,8 @@ from fei_amd.ops.rows import (  # noqa: F401
     add_norm_parts, product_parts, rope_kv_parts, rows_ok)
 from fei_amd.ops.sigmoid_attn import (  # noqa: F401
     check_sigmoid_geometry, sigmoid_attn_decode, sigmoid_attn_prefill)
+from fei_amd.ops.tiles import (  # noqa: F401
+    parts_ok as tile_parts_ok, product_parts as tile_parts)
 
 _LIB: Optional[ctypes.CDLL] = None
 _LIB_ERR: Optional[str] = None
@@ -97,6 +100,7 @@ def _try_load() -> None:
     lib.fei_prefetch.argtypes = [_vp, _l, _vp, _i, _vp]
     _mixers.declare(lib)
     _rows.declare(lib)
+    _tiles.declare(lib)
     _moe.declare(lib)
     _sigmoid_attn.declare(lib)
     _LIB = lib
@@ -638,15 +642,26 @@ def linear_decode(x: torch.Tensor, w: torch.Tensor,
     return out
 
 
+def _many_rows(M: int, x: torch.Tensor, wgu: torch.Tensor) -> Optional[str]:
+    """The kernel of more than a few rows that makes a SwiGLU, if one does."""
+    if _rows.swiglu_ok(M, x, wgu):
+        return "rows"
+    # a copy of rows with gaps is aligned
+    if (wgu.shape[0] % 16 == 0
+            and _tiles.tile_ok(M, x if x.is_contiguous() else wgu, wgu)):
+        return "tile"
+    return None
+
+
 def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Fused gate/up product + SwiGLU: x [M,K] @ [2I,K]^T -> silu(g)*u [M,I]."""
     K, I = x.shape[-1], wgu.shape[0] // 2
     M = x.numel() // K
     how = _product(x, wgu, M, K, I, out)
-    if (how is None and x.is_cuda and _rows.swiglu_ok(M, x, wgu)
-            and _mixers.match(x, wgu, K) and _fits(out, x, M * I)):
-        how = "rows"
+    if (how is None and M and x.is_cuda and _mixers.match(x, wgu, K)
+            and _fits(out, x, M * I)):
+        how = _many_rows(M, x, wgu)
     if how is None:
         return swiglu(torch.nn.functional.linear(x, wgu))
     x2 = x.contiguous().view(M, K)
@@ -654,6 +669,9 @@ def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
         out = torch.empty(*x.shape[:-1], I, dtype=x.dtype, device=x.device)
     if how == "rows":
         _rows.swiglu_product(x2, wgu, out)
+        return out
+    if how == "tile":
+        _tiles.product(x2, wgu, out.view(M, I), I, _tiles.TILE_SWIGLU)
         return out
     if how == "skinny":
         _mixers.skinny(out, x2, wgu, I, _mixers.EPI_SWIGLU, act=out, stride=I)
@@ -845,6 +863,15 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
         _mixers.skinny(out, x.view(M, -1), w, w.shape[0],
                        _mixers.EPI_GELU if act_gelu else _mixers.EPI_BF16,
                        bias16=bias)
+        return out
+    if (act_gelu and x.is_cuda and _mixers.plain(x, w)
+            and _tiles.tile_ok(M, x, w)
+            and _mixers.dense(bias, torch.bfloat16, x, w.shape[0])
+            and bias.data_ptr() % 16 == 0):
+        out = torch.empty(*x.shape[:-1], w.shape[0], dtype=x.dtype,
+                          device=x.device)
+        _tiles.product(x.view(M, -1), w, out.view(M, -1), w.shape[0],
+                       _tiles.TILE_GELU, bias)
         return out
     y = torch.nn.functional.linear(x, w, bias)
     return gelu(y) if act_gelu else y

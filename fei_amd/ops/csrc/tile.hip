@@ -1,0 +1,391 @@
+// Products of hundreds of rows and more with a weight matrix (gfx950):
+// out[M, N] = x[M, K] @ W[N, K]^T in bfloat16 with float32 sums, where what follows
+// the product is done on its sums, or K is cut so that all CUs have a tile.
+#include <algorithm>
+
+#include "fei_epilogue.h"
+#include "fei_mma.h"
+
+namespace {
+
+enum {
+  TILE_BF16 = 0,
+  TILE_SWIGLU = 1,     // W has N rows of gates, then N of up
+  TILE_GELU = 2,       // with a bias per column
+  TILE_RELU2 = 3,
+  TILE_PARTS = 4,      // float32 sums of a part of K, [parts][M][N]
+};
+
+struct First { static constexpr int value = 0; };
+struct Second { static constexpr int value = 1; };
+
+__device__ __forceinline__ int uniform(int v) {
+  return __builtin_amdgcn_readfirstlane(v);
+}
+
+// 64 lanes x 16 bytes from ``base`` (the same in all lanes) + off straight into LDS,
+// lane i at lds + 16 i. m0 is not kept: nothing else here uses it.
+__device__ __forceinline__ void load_lds_from(const u16* base, u32 off, u32 lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, %1"
+      :: "v"(off), "s"(base), "s"(lds)
+      : "memory");
+}
+
+struct TileArgs {
+  void* out;
+  const u16* x;
+  const u16* w;
+  const u16* bias;
+  long os, xs;         // rows of out and x are this far apart
+  int M, N, K, nx, nm, parts;
+};
+
+// A block: 8 waves, two on a SIMD, that share tiles of 32 WM XI rows of x and
+// 32 WN WI rows of W (SWIGLU: half of them gates, the others the same of up),
+// WN = 8 / WM, 64 steps of K at a time. Both operands come in halves; a wave has
+// XI x WI fragments of each of the four quarters. Waves 0-3 are one
+// barrier ahead of waves 4-7, so that of the two waves on a SIMD one multiplies
+// while the other reads fragments and sends loads. A step is two such turns:
+//   first half of x, both of W -> its two quarters of the tile
+//   second half of x           -> the other two
+// Each group loads its half of x and W, straight to LDS, two steps ahead of the
+// products, in two buffers: what a turn has read is free when the turn's barrier
+// is past (reads are waited for in front of it), and is filled again in the next.
+// Loads are waited for a turn before they are read, by their number, so that
+// those of a step and more stay in flight. The stream of loads runs on
+// into the block's next tile, and results are written while the other group
+// multiplies: a tile's first loads and last stores cost little then.
+//
+// The 16-byte places of a row in LDS are permuted by the row, in the address that
+// a lane loads from, so that the reads of 16 rows spread over the banks. Row
+// i of a fragment of W is row 4 WI (i / 4) + 4 j + i % 4 of the wave's, j the
+// fragment, so that a lane has 4 WI consecutive columns of a row of out.
+//
+// Blocks of an XCD take consecutive tiles, eight of rows times all of columns, rows
+// first: its L2 holds what they share. XCDs start at different steps of K, or
+// all would read the same columns of W, rows of which lie a power of two apart,
+// from the same memory channels.
+//
+// Bound by the matrix units: 2310 cycles a step of 256 x 256 x 64, of which they
+// need 2048, at the 1.7 to 2.1 GHz that the card keeps under this load; four turns
+// of one quarter took 2510, and more where both groups ran the same branching code.
+// Against the library, us: 2 x 14336 x 4096 of 2048 rows with SwiGLU 348 (360 + 33
+// for the pass of its own); 3072 x 768 of 16384 with bias and GELU 104
+// (68.5 + 52); 4096 x 14336 of 2048 in two parts 170 (204); 8192^3 706 (700).
+template <int WM, int XI, int WI, int EPI>
+__global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
+  constexpr int WN = 8 / WM;
+  constexpr int HA = 16 * WM * XI, HB = 16 * WN * WI;   // rows of a half
+  constexpr int TM = 2 * HA, TN = 2 * HB;
+  constexpr int PA = HA / 32, PB = HB / 32;             // loads of a wave
+  constexpr bool PAIR = EPI == TILE_SWIGLU;
+  constexpr int CN = PAIR ? HB : TN;                    // columns of out
+  constexpr int STAGE = (TM + TN) * 64;
+  extern __shared__ __align__(16) u16 buf[];
+  u16* const lbias = buf + 2 * STAGE;                   // [4 tiles][512]
+  const int M = g.M, N = g.N, K = g.K, parts = g.parts;
+  const int total = g.nx * g.nm, tiles = total * parts, per = (tiles + 7) / 8;
+  const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
+  const int lim = min(per, tiles - xcd * per);          // tiles of the XCD
+  if (slot >= lim) return;
+  const int all = K / 64;
+  const bool spread = (long)M * K <= 2 << 20;
+  struct Tile { int m0, n0, part, first, steps, turn; };
+  auto locate = [&](int i) __attribute__((always_inline)) {
+    Tile t;
+    int id = xcd * per + i;
+    t.part = uniform(id / total);
+    id -= t.part * total;
+    const int g0 = uniform(id / (8 * g.nx)) * 8, gm = min(8, g.nm - g0);
+    const int gr = id - g0 * g.nx, c = uniform(gr / gm);
+    t.n0 = c * CN;
+    t.m0 = (g0 + gr - c * gm) * TM;
+    t.first = uniform((int)((u32)(t.part * all) / (u32)parts));
+    t.steps = uniform((int)((u32)((t.part + 1) * all) / (u32)parts)) - t.first;
+    t.turn = uniform((u32)(xcd * t.steps / 8 + (spread ? 3 * c : 0)) % (u32)t.steps);
+    return t;
+  };
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = uniform(tid >> 6), grp = wid >> 2, w4 = wid & 3;
+  const int wm = WM == 4 ? w4 : grp, wn = WM == 4 ? grp : w4;
+  const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)buf;
+
+  // the wave's stream of loads: its pieces of 8 rows of its group's halves
+  Tile ld = locate(slot);
+  int li = slot, lk = 0, ltile = 0;
+  u32 ls = 0;                              // buffer, in bytes
+  u32 oa[PA], ob[PB];
+  const u16 *pa, *pb;
+  auto aim = [&]() __attribute__((always_inline)) {
+    // a lane's share is made anew for each tile: kept, it would not fit
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int r8 = ln >> 3, c8 = ln & 7;
+    const int ma = ld.m0 + grp * HA, last_a = max(M - 1 - ma, 0);
+    pa = g.x + min(ma, M - 1) * g.xs + ld.first * 64;
+#pragma unroll
+    for (int i = 0; i < PA; ++i)
+      oa[i] = (u32)min((w4 * PA + i) * 8 + r8, last_a) * (u32)(g.xs * 2) +
+              (c8 ^ r8) * 16;
+    const int nb = PAIR ? ld.n0 : ld.n0 + grp * HB, last_b = max(N - 1 - nb, 0);
+    pb = g.w + ((long)min(nb, N - 1) + (PAIR && grp ? N : 0)) * K +
+         ld.first * 64;
+#pragma unroll
+    for (int i = 0; i < PB; ++i) {
+      const int r = (w4 * PB + i) * 8 + r8;
+      const int f = (r & 3) | ((r % (16 * WI) / (4 * WI)) & 1) << 2;
+      ob[i] = (u32)min(r, last_b) * (u32)(K * 2) + (c8 ^ f) * 16;
+    }
+    if (EPI == TILE_GELU && wid == 0)
+      load_lds_from(g.bias, (u32)min(ld.n0 + (ln & 31) * 8, N - 8) * 2,
+                    lds + 4 * STAGE + (ltile & 3) * 1024);
+  };
+  aim();
+  auto column = [&]() __attribute__((always_inline)) {
+    const int t = lk + ld.turn;
+    return (t < ld.steps ? t : t - ld.steps) * 64;
+  };
+  auto load_a = [&]() __attribute__((always_inline)) {
+    const u16* p = pa + column();
+    const u32 d = lds + ls + (grp * HA + w4 * PA * 8) * 128;
+#pragma unroll
+    for (int i = 0; i < PA; ++i) load_lds_from(p, oa[i], d + i * 1024);
+  };
+  auto load_b = [&]() __attribute__((always_inline)) {
+    const u16* p = pb + column();
+    const u32 d = lds + ls + (TM + grp * HB + w4 * PB * 8) * 128;
+#pragma unroll
+    for (int i = 0; i < PB; ++i) load_lds_from(p, ob[i], d + i * 1024);
+  };
+  // past the block's last step that one is read again: the waits count loads
+  auto advance = [&]() __attribute__((always_inline)) {
+    ls ^= STAGE * 2;
+    if (__builtin_expect(lk + 1 < ld.steps, 1)) {
+      ++lk;
+    } else if (li + slots < lim) {
+      li += slots;
+      ++ltile;
+      ld = locate(li);
+      lk = 0;
+      aim();
+    }
+  };
+
+  s16x8 fa[XI][2], fb[2][WI][2];
+  const int l15 = lane & 15, lg = lane >> 4;
+  const int pl0 = (lg ^ (l15 & 7)) * 8, pl1 = ((4 + lg) ^ (l15 & 7)) * 8;
+  const int xa = (wm * 16 * XI + l15) * 64;
+  const int wa = (TM + wn * 16 * WI + 4 * WI * (l15 >> 2) + (l15 & 3)) * 64;
+  int cs = 0;                              // buffer of the products
+  auto read_a = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      const u16* p = buf + cs + xa + (h * HA + i * 16) * 64;
+      fa[i][0] = ld8(p + pl0);
+      fa[i][1] = ld8(p + pl1);
+    }
+  };
+  auto read_b = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < WI; ++j) {
+      const u16* p = buf + cs + wa + (h * HB + 4 * j) * 64;
+      fb[h][j][0] = ld8(p + pl0);
+      fb[h][j][1] = ld8(p + pl1);
+    }
+  };
+  f32x4 acc[2][2][XI][WI];
+  auto clear = [&](auto ha, auto hb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < XI; ++i)
+#pragma unroll
+      for (int j = 0; j < WI; ++j)
+        acc[ha.value][hb.value][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  };
+  clear(First{}, First{});
+  clear(First{}, Second{});
+  clear(Second{}, First{});
+  clear(Second{}, Second{});
+  auto barrier = [&]() __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_barrier" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // until all but a step's loads, the last sent, have arrived
+  auto wait = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PA + PB) : "memory");
+  };
+  auto product = [&](auto ha) __attribute__((always_inline)) {
+    constexpr int a = decltype(ha)::value;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    barrier();
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+        for (int i = 0; i < XI; ++i)
+#pragma unroll
+          for (int j = 0; j < WI; ++j)
+            acc[a][b][i][j] = mma(fb[b][j][kk], fa[i][kk], acc[a][b][i][j]);
+    __builtin_amdgcn_s_setprio(0);
+    barrier();
+  };
+  // results of a quarter of the tile (SWIGLU: of a half's gates and ups)
+  auto store = [&](auto ha, auto hb, const Tile& t, int tile)
+                   __attribute__((always_inline)) {
+    constexpr int a = decltype(ha)::value, b = decltype(hb)::value, V = 4 * WI;
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    const int nr = b * HB + wn * 16 * WI + V * (ln >> 4), n = t.n0 + nr;
+    u16 add[V];
+    if (EPI == TILE_GELU)
+#pragma unroll
+      for (int j = 0; j < WI; ++j)
+        __builtin_memcpy(add + 4 * j, lbias + (tile & 3) * 512 + nr + 4 * j, 8);
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+      const int m = t.m0 + a * HA + wm * 16 * XI + i * 16 + (ln & 15);
+      if (m < M && n < N) {
+        if (EPI == TILE_PARTS) {
+          float* p = (float*)g.out + ((long)t.part * M + m) * N + n;
+#pragma unroll
+          for (int j = 0; j < WI; ++j)
+            if (n + 4 * j < N) *(f32x4*)(p + 4 * j) = acc[a][b][i][j];
+        } else {
+          u16 v[V];
+#pragma unroll
+          for (int j = 0; j < WI; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              float y = acc[a][b][i][j][e];
+              if (PAIR) y = y / (1.f + __expf(-y)) * acc[a][1][i][j][e];
+              if (EPI == TILE_GELU) y = gelu_erf(y + bf2f(add[j * 4 + e]));
+              if (EPI == TILE_RELU2) y = relu2(y);
+              v[j * 4 + e] = El<u16>::st(y);
+            }
+          u16* p = (u16*)g.out + m * g.os + n;
+          constexpr int W = WI % 2 ? 4 : 8;             // of a store; N % 8 == 0
+#pragma unroll
+          for (int c = 0; c < V; c += W)
+            if (n + c < N)
+              __builtin_memcpy(__builtin_assume_aligned(p + c, 2 * W), v + c,
+                               2 * W);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);   // a row at a time: registers
+    }
+    clear(ha, hb);
+    if (PAIR) clear(ha, Second{});
+  };
+
+  int ct = 0;
+  auto step = [&](const Tile& t, auto lastc, auto gc)
+                  __attribute__((always_inline)) {
+    constexpr bool last = decltype(lastc)::value, late = decltype(gc)::value;
+    read_a(0);
+    read_b(0);
+    read_b(1);
+    if (late) {
+      load_a();
+      advance();
+      wait();                        // this step's second half of x
+    }
+    product(First{});
+    read_a(1);
+    if (!late) load_a();
+    load_b();
+    if (!late) advance();
+    wait();                          // all else of the next step
+    if (last) {
+      store(First{}, First{}, t, ct);
+      if (!PAIR) store(First{}, Second{}, t, ct);
+    }
+    product(Second{});
+    if (last) {
+      store(Second{}, First{}, t, ct);
+      if (!PAIR) store(Second{}, Second{}, t, ct);
+    }
+    cs ^= STAGE;
+  };
+  // one loop a group, so that neither branches on it
+  auto run = [&](auto gc) __attribute__((always_inline)) {
+    for (int i = slot; i < lim; i += slots, ++ct) {
+      const Tile t = locate(i);
+      for (int k = 0; k < t.steps - 1; ++k) step(t, First{}, gc);
+      step(t, Second{}, gc);
+    }
+  };
+  if (grp == 0) {
+    load_a();
+    load_b();
+    advance();
+    load_a();
+    load_b();
+    advance();
+    wait();
+    barrier();
+    run(First{});
+    barrier();
+  } else {
+    load_b();
+    load_a();
+    advance();
+    load_b();
+    wait();
+    barrier();
+    barrier();
+    run(Second{});
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <int WM, int XI, int WI, int EPI>
+void launch(TileArgs g, hipStream_t stream) {
+  constexpr int TM = 32 * WM * XI, TN = 32 * (8 / WM) * WI;
+  constexpr int CN = EPI == TILE_SWIGLU ? TN / 2 : TN;
+  constexpr int lds = 2 * (TM + TN) * 128 + 4096;
+  allow_lds(k_tile<WM, XI, WI, EPI>, lds);
+  g.nx = (g.N + CN - 1) / CN;
+  g.nm = (g.M + TM - 1) / TM;
+  // a block a CU
+  const int blocks = std::min(256L, ((long)g.nx * g.nm * g.parts + 7) / 8 * 8);
+  hipLaunchKernelGGL((k_tile<WM, XI, WI, EPI>), dim3(blocks), dim3(512), lds,
+                     stream, g);
+}
+
+template <int EPI>
+void by_size(int rows, int width, const TileArgs& g, hipStream_t stream) {
+  if (rows == 192) launch<2, 3, 2, EPI>(g, stream);
+  else if (rows == 128) launch<2, 2, 2, EPI>(g, stream);
+  else if (width == 256) launch<2, 4, 2, EPI>(g, stream);
+  else if (width == 192) launch<4, 2, 3, EPI>(g, stream);
+  else launch<4, 2, 2, EPI>(g, stream);
+}
+
+}  // namespace
+
+extern "C" {
+
+// Rows of x (xs apart) and w on 16 bytes, K % 64 == 0 and at least 64 a part,
+// N % 8 == 0; rows of out (os apart) on 16 bytes, as the bias. A tile has rows x width
+// rows of x and w: 256 x 256, 192 or 128, 192 x 256, 128 x 256. epi: see above; parts
+// are 1 but for TILE_PARTS.
+void fei_tile(void* out, long os, const void* x, long xs, const void* w,
+              const void* bias, int M, int N, int K, int epi, int rows,
+              int width, int parts, hipStream_t stream) {
+  const TileArgs g = {out, (const u16*)x, (const u16*)w, (const u16*)bias,
+                      os, xs, M, N, K, 0, 0, parts};
+  switch (epi) {
+    case TILE_BF16: return by_size<TILE_BF16>(rows, width, g, stream);
+    case TILE_SWIGLU: return by_size<TILE_SWIGLU>(rows, width, g, stream);
+    case TILE_GELU: return by_size<TILE_GELU>(rows, width, g, stream);
+    case TILE_RELU2: return by_size<TILE_RELU2>(rows, width, g, stream);
+    case TILE_PARTS: return by_size<TILE_PARTS>(rows, width, g, stream);
+  }
+}
+
+}  // extern "C"

@@ -16,6 +16,7 @@ import torch
 import fei_amd.ops as _ops     # half made yet: it imports this
 from fei_amd.ops import reference as ref
 from fei_amd.ops import rows as _rows
+from fei_amd.ops import tiles as _tiles
 from fei_amd.ops.rows import SKINNY_ROWS
 
 _c = ctypes
@@ -229,6 +230,15 @@ def skinny(out, x, w, n: int, epi: int, bias=None, scale: float = 1.0,
                       _p(sums), tiles, eps, _p(sums_out), _stream())
 
 
+def _act_tile(x: torch.Tensor, w: torch.Tensor, ff: int,
+              act: torch.Tensor) -> bool:
+    """Whether the product of many rows writes its activations, ``ff`` a row, to
+    ``act`` itself."""
+    return (ff % 8 == 0 and plain(x, w) and _tiles.tile_ok(x.shape[0], x, w)
+            and act.dtype is _BF16 and act.stride(1) == 1
+            and act.stride(0) % 8 == 0 and act.data_ptr() % 16 == 0)
+
+
 def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,
            n_mix: int, ff: int, act: torch.Tensor) -> torch.Tensor:
     """All products of a layer's input: returns n1 @ w_in[:n_mix]^T and writes
@@ -250,7 +260,9 @@ def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,
                                act.stride(0), T, n_mix, ff, K, 1, _stream())
         return proj
     proj = torch.nn.functional.linear(n1, w_in[:n_mix])
-    if ff:
+    if ff and own and _act_tile(n2, w_in[n_mix:], ff, act):
+        _tiles.product(n2, w_in[n_mix:], act, ff, _tiles.TILE_SWIGLU)
+    elif ff:
         gu = torch.nn.functional.linear(n2, w_in[n_mix:])
         if n1.is_cuda:
             if T:
@@ -288,7 +300,9 @@ def parallel_in(h: GainNormed, w_in: torch.Tensor, n_mix: int, ff: int,
         return proj, router
     rows = h.rows
     proj = torch.nn.functional.linear(rows, w_in[:n_mix])
-    if ff:
+    if ff and gpu and _act_tile(rows, w_in[n_mix:], ff, act):
+        _tiles.product(rows, w_in[n_mix:], act, ff, _tiles.TILE_RELU2)
+    elif ff:
         up = torch.nn.functional.linear(rows, w_in[n_mix:])
         if not x.is_cuda:
             act.copy_(ref.square_relu(up))

@@ -1,0 +1,106 @@
+"""Products of hundreds of rows and more (csrc/tile.hip) with what follows them
+inside, or cut along K for the kernel after them. bfloat16 GPU tensors only."""
+
+from __future__ import annotations
+
+import ctypes
+from functools import lru_cache
+from typing import Optional, Tuple
+
+import torch
+
+import fei_amd.ops as _ops     # half made yet: it imports this
+
+_vp, _i, _l = ctypes.c_void_p, ctypes.c_int, ctypes.c_long
+
+# csrc/tile.hip
+TILE_BF16, TILE_SWIGLU, TILE_GELU, TILE_RELU2, TILE_PARTS = range(5)
+
+CUS = 256
+# Rows of x and w a tile, and us of a step of 64 of K: with one tile on the chip, and
+# what comes on top with one on every CU, when the card lowers its clock.
+TILES = ((256, 256, 0.95, 0.38), (256, 192, 0.82, 0.25), (192, 256, 0.82, 0.25),
+         (256, 128, 0.66, 0.17), (128, 256, 0.66, 0.17))
+
+
+def declare(lib: ctypes.CDLL) -> None:
+    lib.fei_tile.argtypes = [_vp, _l, _vp, _l, _vp, _vp] + [_i] * 7 + [_vp]
+
+
+def _p(t: Optional[torch.Tensor]):
+    return None if t is None else t.data_ptr()
+
+
+def tile_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether M rows x times w run here; x's rows may lie apart."""
+    K = w.shape[-1]
+    return (M > 128 and w.is_cuda and w.dim() == 2 and K > 0 and K % 64 == 0
+            and w.shape[0] > 0 and w.shape[0] % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.stride(-1) == 1 and x.stride(-2) % 8 == 0)
+
+
+def _time(M: int, cols: int, K: int, parts: int, rows: int, width: int,
+          alone: float, full: float) -> float:
+    """About how many us a product takes: rounds of tiles over the CUs."""
+    tiles = -(-M // rows) * -(-cols // width) * parts
+    rounds = -(-tiles // CUS)
+    return rounds * (-(-K // 64 // parts) * (alone + full * tiles /
+                                             (CUS * rounds)) + 3.0)
+
+
+@lru_cache(maxsize=1024)
+def size_for(M: int, cols: int, K: int) -> Tuple[int, int]:
+    """Rows of x and of w a tile for a product with ``cols`` of them.
+    16384 x 768 in 192 columns a tile is one full round, 24 us; in 256 three quarters
+    of one, 26; 16384 x 3072 three rounds of 256, 70, four of 192, 89."""
+    return min(TILES, key=lambda t: _time(M, cols, K, 1, *t))[:2]
+
+
+def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, N: int,
+            epi: int, bias: Optional[torch.Tensor] = None) -> None:
+    """x [M, K] with the rows of ``w``: N results a row, for tile_ok; rows of
+    ``out`` on 16 bytes."""
+    K = x.shape[1]
+    size = size_for(x.shape[0], w.shape[0], K)
+    _launch(out, x, w, N, epi, size, bias)
+
+
+def _launch(out, x, w, N, epi, size, bias=None, parts=1) -> None:
+    M, K = x.shape
+    _ops.require_lib().fei_tile(
+        _p(out), out.stride(-2), _p(x), x.stride(0), _p(w), _p(bias), M, N, K,
+        epi, *size, parts, _ops._stream())
+
+
+def parts_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x @ w^T is faster in parts of K that the norm after it sums: a long
+    K, and results for less than half of the CUs' tiles. With the norm, against the
+    library's product and a norm: 4096 x 14336 of 512 rows 66 us (95), 1000 106
+    (138), 2048 187 (212); 2048 x 8192 of 512 32 (35), 2048 72 (79), 4000 117 (121);
+    of 6006 172 (166). 4096 x 4096 is a draw."""
+    N, K = w.shape
+    return (K >= 8192 and M > 256 and tile_ok(M, x, w)
+            and _ops._mixers.match(x, w, x.shape[-1])
+            and 2 * -(-M // 256) * -(-N // 256) <= CUS)
+
+
+@lru_cache(maxsize=1024)
+def parts_for(M: int, N: int, K: int) -> Tuple[Tuple[int, int], int]:
+    """Rows of x and of w a tile, and parts of K. A part's sums are written and
+    read once, 8 bytes at about 4.5 TB/s."""
+    tile, p = min(((t, p) for t in TILES for p in range(1, 9)),
+                  key=lambda c: _time(M, N, K, c[1], *c[0]) +
+                  c[1] * M * N * 1.8e-6)
+    return tile[:2], p
+
+
+def product_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [M, K] @ w^T as float32 parts [p, M, N] that are to be summed, for
+    parts_ok."""
+    M, K = x.shape
+    N = w.shape[0]
+    size, p = parts_for(M, N, K)
+    out = torch.empty(p, M, N, dtype=torch.float32, device=x.device)
+    _launch(out, x, w, N, TILE_PARTS, size, None, p)
+    return out

@@ -1,0 +1,104 @@
+"""Products of hundreds of rows (csrc/tile.hip) against float64."""
+
+import pytest
+import torch
+
+from fei_amd import ops
+from fei_amd.ops import mixers as mx
+from fei_amd.ops import tiles
+
+DEV = "cuda:0"
+F = torch.nn.functional
+
+
+def rand(*shape, seed=0, dev=DEV, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    return (torch.randn(*shape, generator=g) * scale).to(dev, torch.bfloat16)
+
+
+def err(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+def test_what_tiles_take():
+    """It needs no GPU to say so; CPU tensors are for torch."""
+    x, w = rand(300, 128, dev="cpu"), rand(64, 128, dev="cpu")
+    assert not tiles.tile_ok(300, x, w)
+    for M in (129, 257, 300, 1301, 2048, 6006, 16384):
+        for N, K in ((64, 64), (768, 768), (4096, 14336), (28672, 4096)):
+            assert tiles.size_for(M, N, K) in [t[:2] for t in tiles.TILES]
+            size, p = tiles.parts_for(M, N, K)
+            assert size in [t[:2] for t in tiles.TILES] and 1 <= p <= 8
+    # one full round of the CUs in tiles of 192 columns, not 3/4 of one of 256
+    assert tiles.size_for(16384, 768, 768) == (256, 192)
+
+
+# one step of K, an odd and an even number of them; one row and one 8 columns past a
+# tile, and short of it; more tiles than CUs, with few steps each
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [
+    (256, 256, 64), (257, 264, 128), (191, 248, 192), (385, 776, 320),
+    (1000, 1536, 1088), (5000, 4104, 64), (4100, 3080, 192)])
+@pytest.mark.parametrize("size", [t[:2] for t in tiles.TILES])
+def test_tile(M, N, K, size):
+    # rows of x and out are ranges of wider ones; nothing is written beside them
+    x = rand(M, K + 8, seed=1)[:, :K]
+    w, b = rand(2 * N, K, seed=2, scale=K ** -0.5), rand(N, seed=3)
+    y = x.double() @ w.double().t()
+    u, g = y[:, N:], y[:, :N]
+    # a result is rounded once, by 2^-9 at most, 0.3 of that in the mean; GELU's and
+    # SwiGLU's own errors are float32's
+    for epi, bias, want in (
+            (tiles.TILE_BF16, None, g), (tiles.TILE_SWIGLU, None, F.silu(g) * u),
+            (tiles.TILE_GELU, b, F.gelu(g + b.double())),
+            (tiles.TILE_RELU2, None, g.clamp_min(0) ** 2)):
+        wide = torch.full((M, N + 16), 7.0, device=DEV, dtype=torch.bfloat16)
+        ww = w if epi == tiles.TILE_SWIGLU else w[:N]
+        tiles._launch(wide[:, 8:N + 8], x, ww, N, epi, size, bias)
+        assert err(wide[:, 8:N + 8], want) < 2 ** -9
+        assert bool((wide[:, :8] == 7).all() and (wide[:, N + 8:] == 7).all())
+    for p in (1, 2, 3, 5):
+        if K // 64 < p:
+            continue
+        parts = torch.full((p, M, N), 7.0, device=DEV)
+        tiles._launch(parts, x, w[:N], N, tiles.TILE_PARTS, size, None, p)
+        # float32 sums of K terms in any order: 2^-24 sqrt(K) of their size and
+        # less; 4e-7 seen
+        assert err(parts.double().sum(0), g) < 2 ** -24 * max(K ** 0.5, 16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,I,K", [(129, 64, 128), (300, 100, 192),
+                                   (700, 1024, 256), (300, 64, 72)])
+def test_swiglu_of_many_rows(M, I, K):
+    """Through the public op; sizes that tiles do not take go to the library."""
+    x, w = rand(M, 2 * K, seed=1), rand(2 * I, K, seed=2, scale=K ** -0.5)
+    for a in (x[:, :K].contiguous(), x[:, K:]):
+        y = a.double() @ w.double().t()
+        want = F.silu(y[:, :I]) * y[:, I:]
+        if I % 8:      # beyond 32 rows the SwiGLU pass takes whole vectors
+            assert not tiles.tile_ok(M, a, w[:I])
+            continue
+        # rounded once, in the library and its pass twice before
+        assert err(ops.gemv_swiglu(a, w), want) < 2 ** -8
+        out = torch.full((M, 2 * I), 7.0, device=DEV, dtype=torch.bfloat16)
+        n2 = a.contiguous()
+        mx.mix_in(n2, n2, torch.cat([w[:8], w]), 8, I, out[:, I:])
+        assert err(out[:, I:], want) < 2 ** -8
+        assert bool((out[:, :I] == 7).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(257, 256, 8192), (600, 2048, 8256),
+                                   (1500, 1024, 10240)])
+def test_parts_and_their_norm(M, N, K):
+    x, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
+    h, gain = rand(M, N, seed=3), rand(N, seed=4)
+    assert ops.tile_parts_ok(M, x, w)
+    assert not ops.tile_parts_ok(M, x.float(), w)
+    assert not ops.tile_parts_ok(M, x[:, 64:], w)
+    want = h.double() + x.double() @ w.double().t()
+    out = ops.add_norm_parts(ops.tile_parts(x, w), h, gain, 1e-5)
+    assert err(h, want) < 2 ** -9
+    norm = want * (want.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()
+    assert err(out, norm * gain.double()) < 2 ** -8
