@@ -9,6 +9,8 @@
 // launched for the largest possible number of tiles.
 //
 // T is u16 (bfloat16 bits) or float.
+#include <type_traits>
+
 #include "fei_common.h"
 #include "fei_epilogue.h"
 #include "fei_mma.h"
@@ -231,9 +233,8 @@ k_moe_gemm_big(u16* __restrict__ out, const u16* __restrict__ x,
     src[4 + i] = we + (long)min(n0 + (wid * WI + i) * 8 + r8, N - 1) * K + c8;
   const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)buf;
   const int steps = K / 64;
-  // past the end the last steps are read again, into a buffer that is free
   auto load = [&](int step, int b, int i) {
-    load_lds(src[i] + min(step, steps - 1) * 64,
+    load_lds(src[i] + step * 64,
              lds + b * BUF * 2 +
                  (i < 4 ? (wid * 4 + i) * 1024
                         : 16384 + (wid * WI + i - 4) * 1024));
@@ -253,12 +254,23 @@ k_moe_gemm_big(u16* __restrict__ out, const u16* __restrict__ x,
   for (int i = 0; i < WI; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // until ``ahead`` steps of those asked for, the last, are still on the way
+  auto wait = [&](int ahead) {
+    static_assert(S <= 3, "more steps to tell apart");
+    if (S > 2 && ahead > 1)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+    else if (ahead > 0)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
 #pragma unroll
   for (int s = 0; s < S; ++s)
+    if (s < steps)
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load(s, s, i);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * LOADS)
-               : "memory");
+      for (int i = 0; i < LOADS; ++i) load(s, s, i);
+  wait(min(S, steps) - 1);
+  asm volatile("s_barrier" ::: "memory");
   Frags f0, f1;
 #pragma unroll
   for (int i = 0; i < WI; ++i) read(f0, 0, 0, i);
@@ -267,7 +279,7 @@ k_moe_gemm_big(u16* __restrict__ out, const u16* __restrict__ x,
   // before. At the barrier all waves have the second half of buffer b, which
   // can be filled again, and the loads of the next one have arrived. Reads
   // and loads go out between the matrix instructions.
-  for (int k = 0; k < steps; ++k) {
+  auto step = [&](int k, auto more) {
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
       read(f1, b, 1, i);
@@ -276,23 +288,28 @@ k_moe_gemm_big(u16* __restrict__ out, const u16* __restrict__ x,
         acc[i][j] = mma(f0.w[i], f0.x[j], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(
-                     (S - 2) * LOADS)
-                 : "memory");
+    if (more.value) wait(S - 2);
+    else wait(min(S - 2, steps - 2 - k));
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const int nb = b == S - 1 ? 0 : b + 1;
 #pragma unroll
     for (int i = 0; i < WI; ++i) {
       read(f0, nb, 0, i);
-      load(k + S, b, i);
-      if (WI + i < LOADS) load(k + S, b, WI + i);
+      if (more.value) {
+        load(k + S, b, i);
+        if (WI + i < LOADS) load(k + S, b, WI + i);
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         acc[i][j] = mma(f1.w[i], f1.x[j], acc[i][j]);
       __builtin_amdgcn_sched_barrier(0);
     }
     b = nb;
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
+  // nothing is asked for past the end: 12 steps would become 15
+  int k = 0;
+  for (; k + S < steps; ++k) step(k, std::true_type{});
+  for (; k < steps; ++k) step(k, std::false_type{});
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     const int r = xm + j * 16 + l15;

@@ -1,6 +1,8 @@
 // Products of tens to hundreds of rows with a weight matrix (gfx950):
 // out[M, N] = x[M, K] @ W[N, K]^T in bfloat16 with float32 sums, where a library
 // product leaves the chip half idle or makes a result that takes another pass.
+#include <type_traits>
+
 #include "fei_epilogue.h"
 #include "fei_mma.h"
 
@@ -72,9 +74,8 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
     src[XJ + i] = w + n * K + c8;
   }
   const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)buf;
-  // past the end the last step is read again, into a buffer that is free
   auto load = [&](int step, int b, int i) {
-    int t = min(step, steps - 1) + turn;
+    int t = step + turn;
     t = t < steps ? t : t - steps;
     load_lds(src[i] + t * 64,
              lds + b * BUF * 2 + (i < XJ ? (wid * XJ + i) * 1024
@@ -101,17 +102,29 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
     for (int j = 0; j < XJ; ++j) acc[i][j] = mma(f.w[i], f.x[j], acc[i][j]);
     __builtin_amdgcn_sched_barrier(0);
   };
+  // until ``ahead`` steps of those asked for, the last, are still on the way
+  auto wait = [&](int ahead) {
+    if (S > 3 && ahead > 2)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * LOADS) : "memory");
+    else if (S > 2 && ahead > 1)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * LOADS) : "memory");
+    else if (ahead > 0)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  };
 #pragma unroll
   for (int s = 0; s < S; ++s)
+    if (s < steps)
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load(s, s, i);
-  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * LOADS)
-               : "memory");
+      for (int i = 0; i < LOADS; ++i) load(s, s, i);
+  wait(min(S, steps) - 1);
+  asm volatile("s_barrier" ::: "memory");
   Frags f0, f1;
 #pragma unroll
   for (int i = 0; i < MX; ++i) read(f0, 0, 0, i);
   int b = 0;                               // buffer of step k
-  for (int k = 0; k < steps; ++k) {
+  auto step = [&](int k, auto more) {
 #pragma unroll
     for (int i = 0; i < MX; ++i) {
       read(f1, b, 1, i);
@@ -119,19 +132,25 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
     }
     // all waves have the second half of buffer b, which can be filled again,
     // and the loads of the next one have arrived
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(
-                     (S - 2) * LOADS)
-                 : "memory");
+    if (more.value) wait(S - 2);
+    else wait(min(S - 2, steps - 2 - k));
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const int nb = b == S - 1 ? 0 : b + 1;
 #pragma unroll
     for (int i = 0; i < MX; ++i) {
       read(f0, nb, 0, i);
-      load(k + S, b, i);
-      if (MX + i < LOADS) load(k + S, b, MX + i);
+      if (more.value) {
+        load(k + S, b, i);
+        if (MX + i < LOADS) load(k + S, b, MX + i);
+      }
       product(f1, i);
     }
     b = nb;
-  }
+  };
+  // nothing is asked for past the end: 16 steps would become 20
+  int k = 0;
+  for (; k + S < steps; ++k) step(k, std::true_type{});
+  for (; k < steps; ++k) step(k, std::false_type{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // results 4 lg + 0..3 of a column group, of row l15
   constexpr int CI = EPI == ROWS_SWIGLU ? WI / 2 : WI;

@@ -116,6 +116,7 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
   // the wave's stream of loads: its pieces of 8 rows of its group's halves
   Tile ld = locate(slot);
   int li = slot, lk = 0, ltile = 0;
+  bool live = true;                        // there are steps left to load
   u32 ls = 0;                              // buffer, in bytes
   u32 oa[PA], ob[PB];
   const u16 *pa, *pb;
@@ -149,18 +150,19 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     return (t < ld.steps ? t : t - ld.steps) * 64;
   };
   auto load_a = [&]() __attribute__((always_inline)) {
+    if (!live) return;
     const u16* p = pa + column();
     const u32 d = lds + ls + (grp * HA + w4 * PA * 8) * 128;
 #pragma unroll
     for (int i = 0; i < PA; ++i) load_lds_from(p, oa[i], d + i * 1024);
   };
   auto load_b = [&]() __attribute__((always_inline)) {
+    if (!live) return;
     const u16* p = pb + column();
     const u32 d = lds + ls + (TM + grp * HB + w4 * PB * 8) * 128;
 #pragma unroll
     for (int i = 0; i < PB; ++i) load_lds_from(p, ob[i], d + i * 1024);
   };
-  // past the block's last step that one is read again: the waits count loads
   auto advance = [&]() __attribute__((always_inline)) {
     ls ^= STAGE * 2;
     if (__builtin_expect(lk + 1 < ld.steps, 1)) {
@@ -171,6 +173,8 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
       ld = locate(li);
       lk = 0;
       aim();
+    } else {
+      live = false;
     }
   };
 
@@ -213,9 +217,13 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     asm volatile("s_barrier" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
   };
-  // until all but a step's loads, the last sent, have arrived
-  auto wait = [&]() __attribute__((always_inline)) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PA + PB) : "memory");
+  // until all but a step's loads, the last sent, have arrived; behind the end all
+  // but those of a half of x where ``half``
+  auto wait = [&](auto half) __attribute__((always_inline)) {
+    if (__builtin_expect(live, 1))
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PA + PB) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(half.value * PA) : "memory");
   };
   auto product = [&](auto ha) __attribute__((always_inline)) {
     constexpr int a = decltype(ha)::value;
@@ -291,15 +299,15 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     read_b(1);
     if (late) {
       load_a();
+      wait(First{});                       // this step's second half of x
       advance();
-      wait();                        // this step's second half of x
     }
     product(First{});
     read_a(1);
     if (!late) load_a();
     load_b();
+    wait(gc);                              // all else of the next step
     if (!late) advance();
-    wait();                          // all else of the next step
     if (last) {
       store(First{}, First{}, t, ct);
       if (!PAIR) store(First{}, Second{}, t, ct);
@@ -325,8 +333,8 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     advance();
     load_a();
     load_b();
+    wait(First{});
     advance();
-    wait();
     barrier();
     run(First{});
     barrier();
@@ -335,7 +343,7 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     load_a();
     advance();
     load_b();
-    wait();
+    wait(Second{});
     barrier();
     barrier();
     run(Second{});
