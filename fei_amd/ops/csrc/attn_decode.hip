@@ -31,7 +31,9 @@ typedef __attribute__((ext_vector_type(2))) u32 u32x2;
 
 constexpr float M_NONE = -3.0e38f;       // maximum of no keys
 constexpr int CHUNK = 32;                // keys of a wave at a time
-constexpr int WAVES = 4;
+constexpr int SHARE = 4;                 // waves of a block where keys are split
+// of one that has all keys of a head: as many as the registers allow
+constexpr int whole_waves(int D) { return D == 64 ? 16 : 8; }
 
 struct DecodeAttn {
   const u16* q;
@@ -51,6 +53,7 @@ __device__ __forceinline__ int keys_at(const DecodeAttn& a, int b) {
   return min(a.pos[b] + 1, a.max_seq);
 }
 // Splits that have keys.
+template <int WAVES>
 __device__ __forceinline__ int used_splits(const DecodeAttn& a, int n) {
   return min(a.splits, (n + CHUNK * WAVES - 1) / (CHUNK * WAVES));
 }
@@ -126,8 +129,8 @@ __host__ __device__ constexpr int wave_floats(int G) {
                                                            : G * D;
 }
 
-template <int D, bool PAGED, bool ROPE>
-__global__ void __launch_bounds__(64 * WAVES, D == 64 ? 4 : 3)
+template <int D, bool PAGED, bool ROPE, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES, D == 64 ? 4 : WAVES > 4 ? 2 : 3)
 k_attn_decode(const DecodeAttn a) {
   constexpr int KS = D / 32;             // steps of a score product
   constexpr int VC = D / 16;             // columns of V a lane loads
@@ -140,7 +143,7 @@ k_attn_decode(const DecodeAttn a) {
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, lg = lane >> 4;
   const int n = keys_at(a, b), last = n - 1;
-  const int chunks = (n + CHUNK - 1) / CHUNK, used = used_splits(a, n);
+  const int chunks = (n + CHUNK - 1) / CHUNK, used = used_splits<WAVES>(a, n);
   const int G = a.G, Hq = a.Hkv * G;
   if (split >= used) {
     if (used <= 0 && split == 0)         // no key: zeros
@@ -364,7 +367,7 @@ __global__ void __launch_bounds__(256) k_attn_decode_combine(const DecodeAttn a)
   for (int i = 0; i < PRE; ++i)
     x[i] = po[(long)min(side + i * SIDE, a.splits - 1) * (D / 4)];
   f32x2 t = ml[min(lane, a.splits - 1)];
-  const int used = used_splits(a, keys_at(a, b));
+  const int used = used_splits<SHARE>(a, keys_at(a, b));
   if (used == 1) return;
   if (lane >= used) t = f32x2{M_NONE, 0.f};
   float m = row16_max(t[0]);
@@ -406,26 +409,50 @@ __global__ void __launch_bounds__(256) k_attn_decode_combine(const DecodeAttn a)
   __builtin_memcpy(a.out + hq * D + d * 4, y, sizeof(y));
 }
 
+template <int D, int WAVES>
+void launch_waves(const DecodeAttn& a, dim3 grid, hipStream_t stream) {
+  const int lds = WAVES * (wave_floats<D, false>(a.G) + 2 * a.G) * 4;
+  const int roped = WAVES * (wave_floats<D, true>(a.G) + 2 * a.G) * 4;
+#define GO(PAGED, ROPE)                                                     \
+  allow_lds(k_attn_decode<D, PAGED, ROPE, WAVES>, ROPE ? roped : lds);      \
+  hipLaunchKernelGGL((k_attn_decode<D, PAGED, ROPE, WAVES>), grid,          \
+                     dim3(64 * WAVES), ROPE ? roped : lds, stream, a)
+  if (a.table) {
+    if (a.cs) { GO(true, true); } else { GO(true, false); }
+  } else {
+    if (a.cs) { GO(false, true); } else { GO(false, false); }
+  }
+#undef GO
+}
+
+// Keys up to which a block takes all of a head's, given how many heads of keys there
+// are: then nothing is left to combine. Split and combined, or whole, us in a graph:
+// 1 sequence of 256 keys and 8 heads of 64 6.7, 6.2; of 320 6.6, 6.8; 8 of 576 9.0,
+// 8.0, of 1024 9.7, 11.0; 20 of 600 in pages 12.7, 9.5; 32 of 2048 34.0, 29.3. Heads
+// of 128, 8 sequences of 320 9.2, 8.8, of 448 9.5, 10.1; 12 of 512 12.4, 12.5; 24 of
+// 2048 46.7, 41.9. Beyond 2048 one long sequence among short ones would be alone on
+// its CUs.
+inline int whole_keys(int heads, int D) {
+  if (heads >= 160) return 2048;
+  if (heads < 64) return 256;
+  return D == 64 ? 768 : heads < 96 ? 320 : 512;
+}
+
 template <int D>
-void launch_decode(const DecodeAttn& a, int B, hipStream_t stream) {
+void launch_decode(DecodeAttn a, int B, hipStream_t stream) {
+  if (a.max_seq > CHUNK * SHARE && a.max_seq <= whole_keys(a.Hkv * B, D)) {
+    a.splits = 1;
+    return launch_waves<D, whole_waves(D)>(a, dim3(a.Hkv, B), stream);
+  }
   // Splits that no sequence can have are not launched, and those beyond 16 come
   // last: a block waits for the position to know that it has no keys, and keeps
   // its place meanwhile. 20 sequences of up to 600 keys in pages, 16 splits
   // asked for: 15.9 -> 7.8 us.
-  const int all = max(1, min(a.splits, (a.max_seq + CHUNK * WAVES - 1) /
-                                           (CHUNK * WAVES)));
+  const int all = max(1, min(a.splits, (a.max_seq + CHUNK * SHARE - 1) /
+                                           (CHUNK * SHARE)));
   const int side = min(all, 16);
-  const dim3 grid(a.Hkv * side, B, (all + side - 1) / side), block(64 * WAVES);
-#define GO(PAGED, ROPE)                                                       \
-  hipLaunchKernelGGL((k_attn_decode<D, PAGED, ROPE>), grid, block,            \
-                     WAVES * (wave_floats<D, ROPE>(a.G) + 2 * a.G) * 4, stream, \
-                     a)
-  if (a.table) {
-    if (a.cs) GO(true, true); else GO(true, false);
-  } else {
-    if (a.cs) GO(false, true); else GO(false, false);
-  }
-#undef GO
+  launch_waves<D, SHARE>(a, dim3(a.Hkv * side, B, (all + side - 1) / side),
+                         stream);
   if (all > 1)
     hipLaunchKernelGGL(k_attn_decode_combine<D>, dim3(B * a.Hkv * a.G),
                        dim3(256), 0, stream, a);

@@ -236,6 +236,26 @@ def test_attn_decode_without_keys(lib, paged, T, splits):
 
 
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,lens", [
+    (8, 2, [1, 129, 251]),           # little room
+    (32, 2, [250]),                  # groups of 16: the most LDS
+    (12, 4, [31, 33, 63, 257, 288] * 4),         # 64 heads and more
+    (8, 8, [700, 511, 513, 1, 97, 300, 400, 512]),
+    (8, 8, list(range(960, 1160, 10))),          # 160 heads: several rounds
+])
+def test_attn_decode_in_one_block(lib, D, paged, rope, Hq, Hkv, lens):
+    """Where a block takes all keys of a head."""
+    test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, 8, lens)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+def test_attn_decode_in_one_block_without_keys(lib, paged):
+    test_attn_decode_without_keys(lib, paged, 192, 4)
+
+
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("rope", [False, True])
 @pytest.mark.parametrize("Hq,Hkv,n,size", [(8, 2, 700, 1), (4, 4, 300, 4),
                                            (16, 1, 1000, 1)])
