@@ -1,8 +1,19 @@
 // All layers of an encoder, launched from one call: over few rows its kernels take
 // 4 to 10 us each, less than it takes to launch them one by one from Python.
 #include "fei_epilogue.h"
+#include "fei_mma.h"
 
 namespace {
+
+// Sum over a wave without LDS.
+__device__ __forceinline__ float wave_sum(float v) {
+  f32x2 t = both_halves(v);
+  const u32 b = __builtin_bit_cast(u32, t[0] + t[1]);
+  const auto q = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const u32 q0 = q[0], q1 = q[1];
+  return row16_sum(__builtin_bit_cast(float, q0) +
+                   __builtin_bit_cast(float, q1));
+}
 
 // Mean of a text's first len rows, to length 1: out [B, C] float32. A block per
 // text; a thread has 8 columns of every SIDEth row. Bound by latency, and by what
@@ -49,6 +60,202 @@ k_pool_unit(float* __restrict__ out, const u16* __restrict__ h,
   const float len = sqrtf(sq);
   const float norm = len < 1e-12f ? 1e-12f : len;   // NaN stays
   for (int i = tid; i < C; i += 1024) out[(long)b * C + i] = part[i] / norm;
+}
+
+// out = LayerNorm(x + res) W^T + bias, or GELU of it: what an encoder's layer does
+// behind each of its two residual products, for up to 8 XL rows of C <= 1024. Each
+// block makes the norm of all rows for itself, to LDS, in twelve waves, while four
+// others have their first rows of W on the way, which they multiply as k_skinny
+// (gemv.hip) does. Block b writes normed rows b, b + gridDim.x, .. to ``normed``,
+// which is none of the inputs.
+//
+// Bound by latency and, from 32 rows on, by the norm's own work on one CU: 16 rows of
+// W and 24 of x take 7 us, a launch of 3.8 for the norm and one of 5 otherwise; in
+// all four waves, in front of the products, 9. Whole encoders, 12 layers of 768,
+// fused and not: 8 rows 341 us, 374; 16 383, 392; 24 392, 411; 32 448, 443; 64 661,
+// 513.
+constexpr int NORM_WAVES = 12;             // beside four that multiply
+
+template <int XL, bool GELU>
+__global__ void __launch_bounds__(64 * (4 + NORM_WAVES))
+k_norm_product(u16* __restrict__ out, const u16* __restrict__ x,
+               const u16* __restrict__ res, const u16* __restrict__ gain,
+               const u16* __restrict__ shift, u16* __restrict__ normed,
+               const u16* __restrict__ w, const u16* __restrict__ bias, int M,
+               int N, int C, float eps) {
+  constexpr int MT = (XL + 1) / 2, R = XL * 8, S = 3;
+  constexpr int NR = (R + NORM_WAVES - 1) / NORM_WAVES;  // a wave's rows
+  extern __shared__ __align__(16) u16 buf[];             // rows of w, of x
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, lg = lane >> 4;
+  const int n0 = blockIdx.x * 16;
+  const int r8 = lane >> 3, c8 = ((lane & 7) ^ r8) * 8;
+  const int steps = C / 64, per = (steps + 3) / 4;
+  const int lo = min(wid * per, steps - 1);
+  const int n = wid < 4 ? max(min(steps, (wid + 1) * per) - wid * per, 0) : 0;
+  const int turn = n ? blockIdx.x * 3 % n : 0;
+  auto at = [&](int s) {
+    const int t = s + turn;
+    return lo + (t < n ? t : t - n);
+  };
+  const u16* src[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    src[i] = w + (long)min(n0 + i * 8 + r8, N - 1) * C + c8;
+  u16* mine = buf + wid * S * 1024;
+  u16* xs = buf + 4 * S * 1024;
+  const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)mine;
+  auto load = [&](int step, int b) {
+    if (step >= n) return;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      load_lds(src[i] + at(step) * 64, lds + (b * 1024 + i * 512) * 2);
+  };
+  const int nv = C >> 3;
+  if (wid < 4) {
+#pragma unroll
+    for (int s = 0; s < S; ++s) load(s, s);
+  } else {
+    // rows wid - 4 and every 12th on; 8 columns lane and lane + 64 of each
+    s16x8 xv[NR][2], rv[NR][2], gv[2], sv[2];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const long row = min(wid - 4 + NORM_WAVES * i, M - 1);
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        const int c = min(lane + 64 * v, nv - 1);
+        xv[i][v] = ((const s16x8*)(x + row * C))[c];
+        rv[i][v] = ((const s16x8*)(res + row * C))[c];
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const int c = min(lane + 64 * v, nv - 1);
+      gv[v] = ((const s16x8*)gain)[c];
+      sv[v] = ((const s16x8*)shift)[c];
+    }
+    const bool both = lane + 64 < nv, one = lane < nv;
+    float f[NR][2][8], sum[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      float t = 0.f, t0 = 0.f;             // in the order of k_layernorm_wave
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        t0 = t;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          f[i][v][j] = bf2f((u16)xv[i][v][j]) + bf2f((u16)rv[i][v][j]);
+          t += f[i][v][j];
+        }
+      }
+      sum[i] = wave_sum(both ? t : one ? t0 : 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const float mean = sum[i] / (float)C;
+      float t = 0.f, t0 = 0.f;
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        t0 = t;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          f[i][v][j] -= mean;
+          t = fmaf(f[i][v][j], f[i][v][j], t);
+        }
+      }
+      sum[i] = wave_sum(both ? t : one ? t0 : 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const float inv = rsqrtf(sum[i] / (float)C + eps);
+      const int row = wid - 4 + NORM_WAVES * i;
+#pragma unroll
+      for (int v = 0; v < 2; ++v) {
+        const int c = lane + 64 * v;
+        s16x8 o;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          o[j] = (short)El<u16>::st(fmaf(f[i][v][j] * inv,
+                                         bf2f((u16)gv[v][j]),
+                                         bf2f((u16)sv[v][j])));
+        if (c < nv && row < R) {
+          st8(xs + ((c >> 3) * R + row) * 64 + ((c & 7) ^ (row & 7)) * 8, o);
+          if (row < M && row % gridDim.x == blockIdx.x)
+            st8(normed + (long)row * C + c * 8, o);
+        }
+      }
+    }
+  }
+  // not __syncthreads: the rows of w stay on the way
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  f32x4 acc[MT];
+#pragma unroll
+  for (int j = 0; j < MT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int b = 0;
+  for (int s = 0; s < n; ++s) {
+    if (n - s > 2) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+    else if (n - s > 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const u16* bw = mine + b * 1024;
+    const u16* bx = xs + at(s) * R * 64;
+    s16x8 fa[2], fb[2][MT];
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      const int c = ((kk * 4 + lg) ^ (l15 & 7)) * 8;
+      fa[kk] = ld8(bw + l15 * 64 + c);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) {
+        // an odd group of 8 rows stands in for the one after it
+        const int r = XL >= 2 * j + 2 ? l15 : l15 & 7;
+        fb[kk][j] = ld8(bx + (j * 16 + r) * 64 + c);
+      }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    load(s + S, b);
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[j] = mma(fa[kk], fb[kk][j], acc[j]);
+    b = b == S - 1 ? 0 : b + 1;
+  }
+  __syncthreads();
+  f32x4* red = (f32x4*)buf;
+#pragma unroll
+  for (int j = 0; j < MT; ++j)
+    if (wid < 4) red[(j * 4 + wid) * 64 + lane] = acc[j];
+  __syncthreads();
+  for (int t = wid; t < MT; t += 4 + NORM_WAVES) {
+    const f32x4* p = red + t * 256 + lane;
+    f32x4 v = p[0];
+#pragma unroll
+    for (int k = 1; k < 4; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += p[k * 64][e];
+    const int m = t * 16 + l15, c = n0 + 4 * lg;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (m >= M || c + e >= N) break;
+      const float y = v[e] + bf2f(bias[c + e]);
+      out[(long)m * N + c + e] = f2bf(GELU ? gelu_erf(y) : y);
+    }
+  }
+}
+
+template <bool GELU>
+void norm_product(u16* out, const u16* x, const u16* res, const u16* gain,
+                  const u16* shift, u16* normed, const u16* w, const u16* bias,
+                  int M, int N, int C, float eps, hipStream_t stream) {
+  auto go = [&](auto kernel, int xl) {
+    const int lds = 24576 + xl * 8 * C * 2;
+    allow_lds(kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3((N + 15) / 16),
+                       dim3(64 * (4 + NORM_WAVES)), lds, stream, out, x, res,
+                       gain, shift, normed, w, bias, M, N, C, eps);
+  };
+  if (M <= 8) go(k_norm_product<1, GELU>, 1);
+  else if (M <= 16) go(k_norm_product<2, GELU>, 2);
+  else go(k_norm_product<3, GELU>, 3);
 }
 
 }  // namespace
@@ -121,6 +328,32 @@ void fei_encoder_layers(const void* const* w, int layers, void* h, void* h1,
     product(tmp, x, wb, C, K, EPI_BF16);
     fei_add_layernorm(to, tmp, from, wb[2], wb[3], M, C, eps, 1, stream);
   };
+  if (M <= 24 && C <= 1024) {
+    // the norms inside the products behind them, but the last
+    auto behind = [&](void* out, const void* res, const void* const* norm,
+                      void* normed, const void* const* wb, int N, bool gelu) {
+      auto run = [&](auto launch) {
+        launch((u16*)out, (const u16*)tmp, (const u16*)res,
+               (const u16*)norm[0], (const u16*)norm[1], (u16*)normed,
+               (const u16*)wb[0], (const u16*)wb[1], M, N, C, eps, stream);
+      };
+      if (gelu) run(norm_product<true>);
+      else run(norm_product<false>);
+    };
+    for (int l = 0; l < layers; ++l, w += 12) {
+      if (l) behind(qkv, h1, w - 2, h, w, 3 * HD, false);
+      else product(qkv, h, w, 3 * HD, C, EPI_BF16);
+      fei_attn_prefill(qkv, (u16*)qkv + HD, (u16*)qkv + 2 * HD, att, pos0,
+                       kv_len, B, S, H, H, D, S, scale, 0, 3L * HD, splits, po,
+                       pml, 3L * S * HD, D, 3L * HD, stream);
+      product(tmp, att, w + 2, C, HD, EPI_BF16);
+      behind(inner, h, w + 4, h1, w + 6, I, true);
+      product(tmp, inner, w + 8, C, I, EPI_BF16);
+    }
+    if (layers)
+      fei_add_layernorm(h, tmp, h1, w[-2], w[-1], M, C, eps, 1, stream);
+    return;
+  }
   for (int l = 0; l < layers; ++l, w += 12) {
     product(qkv, h, w, 3 * HD, C, EPI_BF16);
     fei_attn_prefill(qkv, (u16*)qkv + HD, (u16*)qkv + 2 * HD, att, pos0, kv_len,

@@ -648,12 +648,18 @@ k_layernorm_wave(u16* __restrict__ out, const u16* __restrict__ x,
   const int nv = cols >> 3;
   const s16x8* xr = (const s16x8*)(x + (long)row * cols);
   const s16x8* rr = (const s16x8*)(res + (long)row * cols);
-  s16x8 xv[V], rv[RES ? V : 1];
+  s16x8 xv[V], rv[RES ? V : 1], wv[V], bv[V];
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     const int at = min(lane + 64 * i, nv - 1);
     xv[i] = xr[at];
     if (RES) rv[i] = rr[at];
+  }
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    const int at = min(lane + 64 * i, nv - 1);
+    wv[i] = ((const s16x8*)w)[at];
+    bv[i] = ((const s16x8*)bias)[at];
   }
   float f[V][8], sum = 0.f;
 #pragma unroll
@@ -678,11 +684,11 @@ k_layernorm_wave(u16* __restrict__ out, const u16* __restrict__ x,
   for (int i = 0; i < V; ++i) {
     const int at = lane + 64 * i;
     if (at >= nv) break;
-    const s16x8 wv = ((const s16x8*)w)[at], bv = ((const s16x8*)bias)[at];
     s16x8 o;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      o[j] = (short)f2bf(f[i][j] * inv * bf2f((u16)wv[j]) + bf2f((u16)bv[j]));
+      o[j] = (short)f2bf(f[i][j] * inv * bf2f((u16)wv[i][j]) +
+                         bf2f((u16)bv[i][j]));
     ((s16x8*)(out + (long)row * cols))[at] = o;
   }
 }

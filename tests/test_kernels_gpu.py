@@ -623,6 +623,35 @@ def test_encoder_layers_from_one_call(lib, B, S, lengths):
         assert row_err(got, want.double()) < 2.0 ** -5
 
 
+@pytest.mark.parametrize("B,S", [(3, 1), (1, 8), (1, 9), (2, 8), (1, 17), (5, 5)])
+@pytest.mark.parametrize("heads,inner", [(12, 3072), (1, 64), (16, 128)])
+def test_encoder_norms_inside_products(lib, B, S, heads, inner):
+    """Up to 24 rows: the same sums in the same order as with a launch for each
+    norm, at the edges of the rows, and of widths that leave lanes without columns
+    or a wave without steps."""
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.bge import BgeEncoder
+    C = heads * 64
+    spec = dataclasses.replace(get_spec("bge-base"), num_layers=3, num_heads=heads,
+                               num_kv_heads=heads, hidden_size=C,
+                               intermediate_size=inner)
+    m = BgeEncoder(spec, device=torch.device(DEV))
+    for i, lw in enumerate(m.layers):
+        for n in ("ln1_w", "ln2_w"):
+            lw[n].copy_(1 + randbf(C, seed=i) * 0.2)
+        for n in ("bqkv", "bo", "bi", "bo2", "ln1_b", "ln2_b"):
+            lw[n].copy_(randbf(lw[n].numel(), seed=i + 9) * 0.1)
+    ids = torch.randint(0, 1000, (B, S), device=DEV)
+    got = m.encode_ids(ids)
+    before, lib.encoder_layers = lib.encoder_layers, lambda *a: None
+    try:
+        want = m.encode_ids(ids)
+    finally:
+        lib.encoder_layers = before
+    assert got.isfinite().all() and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("gelu", [False, True])
 @pytest.mark.parametrize("M,N,K", [(33, 4, 64), (64, 768, 3072), (65, 100, 128),
                                    (500, 2304, 768)])
