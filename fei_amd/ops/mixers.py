@@ -357,6 +357,9 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
     if own and _rows.add_ok(x, a, w):
         _rows.add_product(x, a, w, mult)
         return x
+    if own and _tiles.add_ok(x, a, w):
+        _rows.add_parts(x, _tiles.product_parts(a, w), mult)
+        return x
     return torch.addmm(x, a, w.t(), out_dtype=torch.float32, alpha=mult,
                        out=x)
 

@@ -146,6 +146,11 @@ def add_ok(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
 def add_product(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
                 mult: float) -> None:
     """x += mult * (a @ w^T), for add_ok."""
-    parts = product_parts(a, w)
+    add_parts(x, product_parts(a, w), mult)
+
+
+def add_parts(x: torch.Tensor, parts: torch.Tensor, mult: float) -> None:
+    """x += mult * the sum of the parts, float32 on 16 bytes, a multiple of 4
+    values."""
     _lib().fei_parts_add(_p(x), _p(parts), parts.shape[0], x.numel(), mult,
                          _stream())

@@ -102,3 +102,18 @@ def test_parts_and_their_norm(M, N, K):
     assert err(h, want) < 2 ** -9
     norm = want * (want.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()
     assert err(out, norm * gain.double()) < 2 ** -8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(257, 8, 8192), (300, 2048, 10240),
+                                   (1706, 1000, 8256), (300, 2048, 8128)])
+def test_residual_of_many_rows(M, N, K):
+    """In parts of K, or (short K, a residual between others') in the library."""
+    a, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
+    x = rand(M, N + 2, seed=3).float()
+    for res in (x[:, :N].contiguous(), x[:, 2:]):
+        assert tiles.add_ok(res, a, w) == (K >= 8192 and N % 8 == 0
+                                           and res.data_ptr() % 16 == 0)
+        want = res.double() + 0.5 * (a.double() @ w.double().t())
+        # float32 sums of K products and one addition
+        assert err(mx.residual_linear(res, a, w, 0.5), want) < 2 ** -24 * K ** 0.5
