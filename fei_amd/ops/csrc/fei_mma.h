@@ -92,6 +92,20 @@ __device__ __forceinline__ void load_lds(const u16* src, u32 lds) {
       : "memory");
 }
 
+// As load_lds, for what is read once.
+__device__ __forceinline__ void load_lds_nt(const u16* src, u32 lds) {
+  u32 keep;
+  asm volatile(
+      "s_mov_b32 %0, m0\n\t"
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %1, off nt\n\t"
+      "s_mov_b32 m0, %0"
+      : "=&s"(keep)
+      : "v"(src), "s"(lds)
+      : "memory");
+}
+
 // For each group of 16 lanes, lane i of it at the 4 values (i % 4) * 4 of row
 // i / 4 of a 4 x 16 tile in LDS: column i, that is value i of the four rows.
 __device__ __forceinline__ s16x4 turn4(const u16* p) {

@@ -367,20 +367,6 @@ void fei_prefetch(const void* w, long bytes, void* sink, int n_blocks,
 // 10.9 -> 5.5, 16384 x 2048 17.6 -> 14.6, 2048 x 8192 14.9 -> 13.7.
 namespace {
 
-// As load_lds, for what is read once.
-__device__ __forceinline__ void load_lds_nt(const u16* src, u32 lds) {
-  u32 keep;
-  asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off nt\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(keep)
-      : "v"(src), "s"(lds)
-      : "memory");
-}
-
 // The RMS norm of x inside the product, from the sums of squares that the
 // product before left.
 struct SkinnyNorm {

@@ -34,13 +34,23 @@ enum {
 // 4 15.8 (23.8), 2 x 14336 x 4096 with SwiGLU 48 (53 + 4.5), 58 with all tiles
 // starting at the same step. Two buffers instead of four: 71. Among the other
 // kernels of a layer the four take 29.7, 13.4, 17.2 and 49.8.
-template <int XJ, int WI, int S, int EPI>
+//
+// ONCE: there is one tile of rows, so that w is read once and need not push x out of
+// the L2: 75 rows 26.6 -> 24.3, 14.9 -> 14.4, 45.9 -> 44.8, 40 rows of the last 43.7
+// -> 38.3; two tiles share what they read (200 rows, 2 x 14336 x 4096 in tiles of
+// 64 columns 92 -> 117).
+template <int XJ, int WI, int S, int EPI, bool ONCE>
 __global__ void __launch_bounds__(256, S * (XJ + WI) <= 20 ? 2 : 1)
 k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
        const u16* __restrict__ w, const u16* __restrict__ bias, int M, int N,
        int K, int nx, int nm) {
   constexpr int TM = 32 * XJ, TN = 32 * WI, MX = XJ > WI ? XJ : WI;
   constexpr int CN = EPI == ROWS_SWIGLU ? TN / 2 : TN;   // columns of out
+  // whether nothing is asked for past the end, so that 16 steps do not become 20. Else
+  // the last step is read again, into a buffer that is free: the second loop costs
+  // registers, and more than it gains where steps are many (2 x 14336 x 4096 with
+  // SwiGLU, 96 rows 45.1 us, 46.0 with one loop; 128 53.4, 50.3; 256 99.7, 86.7)
+  constexpr bool EXACT = EPI != ROWS_SWIGLU || WI == 2 || (ONCE && XJ < 4);
   constexpr int BUF = (TM + TN) * 64, LOADS = XJ + WI;
   extern __shared__ __align__(16) u16 buf[];
   const int total = nx * nm, per = (total + 7) / 8;
@@ -75,11 +85,13 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
   }
   const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)buf;
   auto load = [&](int step, int b, int i) {
-    int t = step + turn;
+    int t = (EXACT ? step : min(step, steps - 1)) + turn;
     t = t < steps ? t : t - steps;
-    load_lds(src[i] + t * 64,
-             lds + b * BUF * 2 + (i < XJ ? (wid * XJ + i) * 1024
-                                         : TM * 128 + (wid * WI + i - XJ) * 1024));
+    const u32 to = lds + b * BUF * 2 +
+                   (i < XJ ? (wid * XJ + i) * 1024
+                           : TM * 128 + (wid * WI + i - XJ) * 1024);
+    if (ONCE && i >= XJ) load_lds_nt(src[i] + t * 64, to);
+    else load_lds(src[i] + t * 64, to);
   };
   const int xm = (wid & 1) * 16 * XJ, wm = (wid >> 1) * 16 * WI;
   struct Frags {
@@ -115,10 +127,10 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
   };
 #pragma unroll
   for (int s = 0; s < S; ++s)
-    if (s < steps)
+    if (!EXACT || s < steps)
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) load(s, s, i);
-  wait(min(S, steps) - 1);
+  wait(EXACT ? min(S, steps) - 1 : S - 1);
   asm volatile("s_barrier" ::: "memory");
   Frags f0, f1;
 #pragma unroll
@@ -147,10 +159,10 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
     }
     b = nb;
   };
-  // nothing is asked for past the end: 16 steps would become 20
   int k = 0;
-  for (; k + S < steps; ++k) step(k, std::true_type{});
-  for (; k < steps; ++k) step(k, std::false_type{});
+  for (; EXACT ? k + S < steps : k < steps; ++k) step(k, std::true_type{});
+  if (EXACT)
+    for (; k < steps; ++k) step(k, std::false_type{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   // results 4 lg + 0..3 of a column group, of row l15
   constexpr int CI = EPI == ROWS_SWIGLU ? WI / 2 : WI;
@@ -187,25 +199,33 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
   }
 }
 
-template <int XJ, int WI, int S, int EPI>
+template <int XJ, int WI, int S, int EPI, bool ONCE>
 void launch(void* out, const void* x, long xs, const void* w, int M, int N,
             int K, int parts, hipStream_t stream, const void* bias = nullptr) {
   constexpr int lds = S * 32 * (XJ + WI) * 128;
   constexpr int CN = EPI == ROWS_SWIGLU ? 16 * WI : 32 * WI;
-  allow_lds(k_rows<XJ, WI, S, EPI>, lds);
+  allow_lds(k_rows<XJ, WI, S, EPI, ONCE>, lds);
   const int nx = (N + CN - 1) / CN, nm = (M + 32 * XJ - 1) / (32 * XJ);
-  hipLaunchKernelGGL((k_rows<XJ, WI, S, EPI>),
+  hipLaunchKernelGGL((k_rows<XJ, WI, S, EPI, ONCE>),
                      dim3((nx * nm + 7) / 8 * 8, parts), dim3(256), lds, stream,
                      out, (const u16*)x, xs, (const u16*)w, (const u16*)bias, M,
                      N, K, nx, nm);
 }
 
-template <int WI, int S, int EPI>
+// Four buffers, but three for 128 rows of x and 64 of w, of which two blocks fit a
+// CU then. 75 rows, 64 of w, three -> four: 4096 x 4096 in 4 parts 10.8 -> 10.0 us,
+// 2 x 8192 x 2048 with SwiGLU 17.4 -> 15.4; 128 rows 7.6 -> 7.8 of 2048 x 2048.
+template <int WI, int EPI>
 void by_rows(int xj, void* out, const void* x, long xs, const void* w, int M,
              int N, int K, int parts, hipStream_t stream) {
-  if (xj == 2) launch<2, WI, S, EPI>(out, x, xs, w, M, N, K, parts, stream);
-  else if (xj == 3) launch<3, WI, S, EPI>(out, x, xs, w, M, N, K, parts, stream);
-  else launch<4, WI, S, EPI>(out, x, xs, w, M, N, K, parts, stream);
+#define GO(XJ, S)                                                             \
+  M <= 32 * XJ                                                                \
+      ? launch<XJ, WI, S, EPI, true>(out, x, xs, w, M, N, K, parts, stream)   \
+      : launch<XJ, WI, S, EPI, false>(out, x, xs, w, M, N, K, parts, stream)
+  if (xj == 2) GO(2, 4);
+  else if (xj == 3) GO(3, 4);
+  else GO(4, (WI == 2 ? 3 : 4));
+#undef GO
 }
 
 // The sums of the parts of a product, added to a bfloat16 residual, and its RMS
@@ -406,8 +426,8 @@ void fei_rows(void* out, const void* x, long xs, const void* w, int M, int N,
               int K, int swiglu, int xj, int wide, int parts,
               hipStream_t stream) {
 #define ROWS(E)                                                            \
-  wide ? by_rows<4, 4, E>(xj, out, x, xs, w, M, N, K, parts, stream)       \
-       : by_rows<2, 3, E>(xj, out, x, xs, w, M, N, K, parts, stream)
+  wide ? by_rows<4, E>(xj, out, x, xs, w, M, N, K, parts, stream)       \
+       : by_rows<2, E>(xj, out, x, xs, w, M, N, K, parts, stream)
   if (swiglu) ROWS(ROWS_SWIGLU);
   else ROWS(ROWS_PARTS);
 #undef ROWS
@@ -419,9 +439,9 @@ void fei_rows(void* out, const void* x, long xs, const void* w, int M, int N,
 void fei_rows_bias(void* out, const void* x, const void* w, const void* bias,
                    int M, int N, int K, int gelu, hipStream_t stream) {
   if (gelu)
-    launch<2, 2, 3, ROWS_GELU>(out, x, K, w, M, N, K, 1, stream, bias);
+    launch<2, 2, 3, ROWS_GELU, false>(out, x, K, w, M, N, K, 1, stream, bias);
   else
-    launch<2, 2, 3, ROWS_BIAS>(out, x, K, w, M, N, K, 1, stream, bias);
+    launch<2, 2, 3, ROWS_BIAS, false>(out, x, K, w, M, N, K, 1, stream, bias);
 }
 
 void fei_parts_norm(void* out, void* res, const float* parts, int np,
