@@ -11,13 +11,20 @@
 // scores of ONE row, so that the softmax needs a single exchange between lanes,
 // and its weights are, as they lie, the second operand of V^T times P^T, whose
 // sums again belong to the lane's row. K and V lie in LDS as in memory but for
-// a permutation of a row's 16-byte (K) or 32-byte (V) places by the row, which
-// spreads the fragment reads over the banks; V is turned by the transposing
-// LDS read.
+// a permutation of a row's places by the row, which spreads the fragment reads over
+// the banks; V is turned by the transposing LDS read. The products with the values
+// stand between the exponentials of the next 16 keys, one for two or four.
 //
 // What bounds it: per 64 keys a wave has 32 matrix instructions (1024 cycles
-// at D = 128) and about as many cycles of softmax; two blocks per CU overlap
-// the two, and the LDS reads (32 KB a wave) take as long again. Measured in a
+// at D = 128) and 900 of softmax, and the two waves of a SIMD overlap little of them:
+// a tile takes 2400. Counters (2 x 2048 tokens): matrix units 36 % of the time, vector
+// units 36, LDS 18 (36 before its reads were free of bank conflicts, which by itself
+// gained nothing). Two groups of waves that take turns, in step, at products and
+// softmax and share the keys of a block's rows were no faster (2048 tokens 50.5 us,
+// heads of 64, 6 x 1001, 58). Against all products behind all exponentials and a
+// lane's addresses made anew for each tile: 2048 tokens, 32/8 heads of 128, 55 -> 51
+// us, over 2048 more 116 -> 107; 6 x 1001, heads of 64, 43 -> 40; 64 x 256, 12 heads,
+// not causal 28 -> 26. Measured in a
 // model's layers against a wave of 16 queries of one head with the values turned
 // on the way into LDS: 2048 tokens, 32/8 heads of 128: 282 -> 63 us (545 TFLOP/s
 // of the causal half); 6 x 1001 tokens, heads of 64: 235 -> 49; 64 x 256, 12 heads
@@ -59,6 +66,18 @@ struct Prefill {
 __device__ __forceinline__ int keys_of(const Prefill& a, int b, int r_hi) {
   const int n = a.causal ? a.pos0[b] + r_hi / a.G + 1 : a.kv_len[b];
   return min(n, a.max_seq);
+}
+
+// By what the 16-byte places of a row of K or V in LDS are turned round, so that the
+// fragment reads take all 64 banks: 16 lanes read a place of 16 rows of K, 32 lanes
+// two of 32 bytes of 4 rows of V; a row fills the banks (D = 128) or half of them.
+template <int D>
+__device__ __forceinline__ int key_turn(int row) {
+  return D == 128 ? row & 15 : row >> 1 & 7;
+}
+template <int D>
+__device__ __forceinline__ int value_turn(int row) {
+  return D == 128 ? (row & 3) * 4 : (row & 2) * 2;
 }
 
 // Tile of the j-th block of a kv head. Causal tiles cost as much as they have
@@ -130,16 +149,35 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   const u16* vb = a.vc + b * a.kv_b + hkv * a.kv_h;
   const u32 lds =
       (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)&buf[0][0][0];
-  auto load = [&](int t, int p) {
+  // what a lane loads of a tile, in bytes from its first row: the wave's LOADS times
+  // RPI rows, of V behind that of K. A tile that ends past the keys reads its last
+  // one again.
+  u32 at[2][LOADS];
+  const int lrow = wid * LOADS * RPI + lane / LPR, place = lane % LPR;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int at = wid * LOADS + i;
-      const int row = at * RPI + lane / LPR, place = lane % LPR;
-      const long off = min(t * KEYS + row, n - 1) * a.kv_t;
-      const int ck = place ^ (row & 7);
-      const int cv = (((place >> 1) ^ (row & (D / 16 - 1))) << 1) | (place & 1);
-      load_lds(kb + off + ck * 8, lds + (p * 2 * KEYS * D + at * 512) * 2);
-      load_lds(vb + off + cv * 8, lds + ((p * 2 + 1) * KEYS * D + at * 512) * 2);
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = lrow + i * RPI;
+    at[0][i] = row * (u32)a.kv_t * 2 + (place ^ key_turn<D>(row)) * 16;
+    at[1][i] = row * (u32)a.kv_t * 2 + (place ^ value_turn<D>(row)) * 16;
+  }
+  const bool near = a.kv_t < 1 << 24;      // such offsets have 32 bits
+  auto load = [&](int t, auto which) __attribute__((always_inline)) {
+    constexpr int V = decltype(which)::value;
+    const u16* base = V ? vb : kb;
+    const u32 to = lds + (((t - t0) & 1) * 2 + V) * KEYS * D * 2 +
+                   wid * LOADS * 1024;
+    if (near && t * KEYS + KEYS <= n) {
+      base += (long)t * KEYS * a.kv_t;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) load_lds_from(base, at[V][i], to + i * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        const int row = lrow + i * RPI;
+        const int c = place ^ (V ? value_turn<D>(row) : key_turn<D>(row));
+        load_lds(base + (long)min(t * KEYS + row, n - 1) * a.kv_t + c * 8,
+                 to + i * 1024);
+      }
     }
   };
 
@@ -150,26 +188,61 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
 
-  if (t0 < t1) load(t0, 0);
+  // Step k of a score product of tile t, 32 keys of it.
+  auto key = [&](int t, int k, int i) __attribute__((always_inline)) {
+    return ld8(buf[(t - t0) & 1][0] + (i * 32 + l31) * D +
+               (((k * 2 + h) ^ key_turn<D>(l31)) << 3));
+  };
+  // 32 columns of 16 keys, 4 values of a column at a time in the order of the keys
+  // that the lane's weights have: 16 i + 4 h + 0..3, then + 8
+  const int vr = 4 * h + ((lane & 15) >> 2), vc0 = (lane >> 4) & 1;
+  auto value = [&](int t, int i, int dt) __attribute__((always_inline)) {
+    const u16* vp = buf[(t - t0) & 1][1] + (i * 16 + vr) * D +
+                    (((dt * 4 + vc0 * 2) ^ value_turn<D>(vr)) << 3) +
+                    (lane & 3) * 4;
+    return turn8(vp, vp + 8 * D);
+  };
+  if (t0 < t1) {
+    load(t0, First{});
+    load(t0, Second{});
+  }
   for (int t = t0; t < t1; ++t) {
-    const int p = (t - t0) & 1;
     // the tile is there, and all waves are done with the other buffer
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (t + 1 < t1) load(t + 1, p ^ 1);
+    if (t + 1 < t1) {
+      load(t + 1, First{});
+      load(t + 1, Second{});
+    }
     if (t * KEYS > lim_hi) continue;
-    const u16* kt = buf[p][0];
-    const u16* vt = buf[p][1];
-
     f32x16 sc[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int e = 0; e < 16; ++e) sc[i][e] = 0.f;
+    s16x8 vf[DT];
+    if constexpr (D == 128) {
+      // fragments 8 products ahead; heads of 64 would lose the fourth wave of a SIMD
+      // by the registers (6 x 1001 tokens 40.4 -> 41.8 us; of 128 73.3 -> 70.2)
+      constexpr int AHEAD = 8;
+      s16x8 kf[AHEAD];
+#pragma unroll
+      for (int x = 0; x < AHEAD; ++x) kf[x] = key(t, x / 2, x % 2);
+#pragma unroll
+      for (int x = 0; x < 2 * KS; ++x) {
+        sc[x % 2] = mma32(kf[x % AHEAD], fq[x / 2], sc[x % 2]);
+        if (x + AHEAD < 2 * KS)
+          kf[x % AHEAD] = key(t, (x + AHEAD) / 2, (x + AHEAD) % 2);
+        else if (x + DT >= 2 * KS)
+          vf[x + DT - 2 * KS] = value(t, 0, x + DT - 2 * KS);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
 #pragma unroll
       for (int k = 0; k < KS; ++k)
-        sc[i] = mma32(ld8(kt + (i * 32 + l31) * D +
-                          (((k * 2 + h) ^ (l31 & 7)) << 3)),
-                      fq[k], sc[i]);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) sc[i] = mma32(key(t, k, i), fq[k], sc[i]);
+#pragma unroll
+      for (int j = 0; j < DT; ++j) vf[j] = value(t, 0, j);
     }
     // register e of sc[i] is key t * 64 + i * 32 + 8 (e / 4) + 4 h + e % 4
     if (t * KEYS + KEYS - 1 > lim_lo) {
@@ -197,38 +270,36 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] *= al;
     }
-    s16x8 fp[4];
+    // weights of 16 keys at a time; between them, the products with the 16 before
+    s16x8 fp;
+    float ps = 0.f;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      float ps = 0.f;
+    for (int i = 0; i < 4; ++i) {
+      float x[8];
+      u32x4 w;
 #pragma unroll
-      for (int hf = 0; hf < 2; ++hf) {
-        u32x4 w;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int at = hf * 8 + 2 * e;
-          const f32x2 x = {
-              __builtin_amdgcn_exp2f(fmaf(sc[i][at], c, -m)),
-              __builtin_amdgcn_exp2f(fmaf(sc[i][at + 1], c, -m))};
-          ps += x[0] + x[1];
-          w[e] = __builtin_bit_cast(u32, __builtin_convertvector(x, bf16x2));
+      for (int u = 0; u < 8; ++u) {
+        if (i && u % (8 / DT) == 0) {
+          const int j = u / (8 / DT);
+          o[j] = mma32(vf[j], fp, o[j]);
+          vf[j] = value(t, i, j);
         }
-        fp[i * 2 + hf] = __builtin_bit_cast(s16x8, w);
+        x[u] = __builtin_amdgcn_exp2f(fmaf(sc[i >> 1][(i & 1) * 8 + u], c, -m));
+        if (u & 1) {
+          ps += x[u - 1] + x[u];
+          w[u >> 1] = __builtin_bit_cast(
+              u32, __builtin_convertvector(f32x2{x[u - 1], x[u]}, bf16x2));
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      l += ps;
+      fp = __builtin_bit_cast(s16x8, w);
+      if (i & 1) {
+        l += ps;
+        ps = 0.f;
+      }
     }
-    // a lane reads 4 values of a column at a time, in the order of the keys
-    // that its weights have: 16 i + 4 h + 0..3, then + 8
-    const int vr = 4 * h + ((lane & 15) >> 2), vc0 = (lane >> 4) & 1;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
-        const u16* vp = vt + (i * 16 + vr) * D +
-                        (((dt * 2 + vc0) ^ (vr & (D / 16 - 1))) << 4) +
-                        (lane & 3) * 4;
-        o[dt] = mma32(turn8(vp, vp + 8 * D), fp[i], o[dt]);
-      }
+    for (int j = 0; j < DT; ++j) o[j] = mma32(vf[j], fp, o[j]);
   }
 
   const f32x2 lt = both_halves(l);

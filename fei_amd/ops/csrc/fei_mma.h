@@ -92,6 +92,21 @@ __device__ __forceinline__ void load_lds(const u16* src, u32 lds) {
       : "memory");
 }
 
+// 64 lanes x 16 bytes from ``base`` (the same in all lanes) + off straight into LDS,
+// lane i at lds + 16 i. m0 is not kept: nothing else may use it.
+__device__ __forceinline__ void load_lds_from(const u16* base, u32 off, u32 lds) {
+  asm volatile(
+      "s_mov_b32 m0, %2\n\t"
+      "s_nop 0\n\t"
+      "global_load_lds_dwordx4 %0, %1"
+      :: "v"(off), "s"(base), "s"(lds)
+      : "memory");
+}
+
+// A constant that a lambda can take.
+struct First { static constexpr int value = 0; };
+struct Second { static constexpr int value = 1; };
+
 // As load_lds, for what is read once.
 __device__ __forceinline__ void load_lds_nt(const u16* src, u32 lds) {
   u32 keep;

@@ -16,22 +16,8 @@ enum {
   TILE_PARTS = 4,      // float32 sums of a part of K, [parts][M][N]
 };
 
-struct First { static constexpr int value = 0; };
-struct Second { static constexpr int value = 1; };
-
 __device__ __forceinline__ int uniform(int v) {
   return __builtin_amdgcn_readfirstlane(v);
-}
-
-// 64 lanes x 16 bytes from ``base`` (the same in all lanes) + off straight into LDS,
-// lane i at lds + 16 i. m0 is not kept: nothing else here uses it.
-__device__ __forceinline__ void load_lds_from(const u16* base, u32 off, u32 lds) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1"
-      :: "v"(off), "s"(base), "s"(lds)
-      : "memory");
 }
 
 struct TileArgs {
