@@ -356,9 +356,13 @@ def _prefill_splits(heads: int, rows: int, max_seq: int) -> int:
     """Shares of the keys that the prompt attention's blocks of 128 rows are
     cut into, so that few rows over many keys fill the chip's 512 places (two
     blocks per CU). How many keys there are is known on the device only; the
-    kernel uses fewer shares where one would have under three tiles of 64."""
+    kernel uses fewer shares where one would have under three tiles of 64, and
+    one where there are few keys in all (of ``max_seq`` the same is asked here).
+    Between the products of a model 250 rows of 32 heads of 128 over 2050 keys
+    take 130 us less a call in 8 shares than in 4; over warm keys the fewer
+    are as fast."""
     blocks = heads * -(-rows // 128)
-    if blocks > 192:
+    if blocks > 192 or max_seq <= 64 * (9 + blocks // 6):
         return 1
     return max(1, min(16, -(-512 // blocks), max_seq // 192))
 

@@ -41,22 +41,12 @@ constexpr int ROWS = 128;              // rows per block
 constexpr int KEYS = 64;               // keys per tile
 constexpr float M_NONE = -3.0e38f;     // maximum of a row without keys
 
-// Keys that a block of rows reads: tiles [t0, t1) of n keys, cut into splits of
-// at least three tiles.
-__device__ __forceinline__ void split_tiles(int n, int splits, int split,
-                                            int& t0, int& t1) {
-  const int nt = (n + KEYS - 1) / KEYS;
-  const int per = max((nt + splits - 1) / splits, 3);
-  t0 = split * per;
-  t1 = min(nt, t0 + per);
-}
-
 struct Prefill {
   const u16 *q, *kc, *vc;
   u16* out;
   float *po, *pml;                     // partial results of splits
   const int *pos0, *kv_len;
-  int S, G, Hkv, heads, tiles, max_seq, causal, splits;
+  int S, G, Hkv, heads, tiles, max_seq, causal, splits, alone;
   float scale;
   long q_ts;
   long kv_b, kv_h, kv_t;               // strides of the caches
@@ -66,6 +56,23 @@ struct Prefill {
 __device__ __forceinline__ int keys_of(const Prefill& a, int b, int r_hi) {
   const int n = a.causal ? a.pos0[b] + r_hi / a.G + 1 : a.kv_len[b];
   return min(n, a.max_seq);
+}
+
+// Keys that a block of rows reads: tiles [t0, t1) of n keys. They are cut into splits
+// of at least three where the last row of the batch row sees more than ``alone`` tiles
+// (asked of one block of rows by itself, those of few keys would have them all and be
+// the last: 500 tokens over 1800 keys 58 us for 39). How many it takes is what the
+// results of splits and the combine cost, which grow with the rows: 9 tiles and one
+// more for six blocks. In one, and in two or three: 33 rows of 32 heads of 128 over
+// 333 keys 11.7 us, 12.2; 150 over 450 13.2, 16.2; 500 over 500 15.1, 22.7, over 800
+// 20.1, 29.2, over 2300 44.3, 41.0.
+__device__ __forceinline__ void split_tiles(const Prefill& a, int b, int n,
+                                            int split, int& t0, int& t1) {
+  const int nt = (n + KEYS - 1) / KEYS;
+  const bool cut = keys_of(a, b, a.S * a.G - 1) > a.alone * KEYS;
+  const int per = cut ? max((nt + a.splits - 1) / a.splits, 3) : nt;
+  t0 = split * per;
+  t1 = min(nt, t0 + per);
 }
 
 // By what the 16-byte places of a row of K or V in LDS are turned round, so that the
@@ -112,7 +119,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   const long prow = ((long)head * R + r) * a.splits + split;
   int t0 = 0, t1 = (n + KEYS - 1) / KEYS;
   if (SPLIT) {
-    split_tiles(n, a.splits, split, t0, t1);
+    split_tiles(a, b, n, split, t0, t1);
     if (t0 >= t1 && split) {           // no keys: the sums are never read
       if (h == 0 && r < R) *(f32x2*)(a.pml + prow * 2) = f32x2{M_NONE, 0.f};
       return;
@@ -308,7 +315,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   // column dt * 32 + 8 i + 4 h + 0..3 in registers 4 i .. of o[dt]
   if (SPLIT) {
     int u0, u1;
-    split_tiles(n, a.splits, 1, u0, u1);
+    split_tiles(a, b, n, 1, u0, u1);
     if (u0 < u1) {                     // there are other splits
       float* po = a.po + prow * D + 4 * h;
 #pragma unroll
@@ -348,8 +355,8 @@ k_attn_prefill_combine(const Prefill a) {
   const int head = id / R, r = id - (long)head * R;
   const int b = head / a.Hkv, hkv = head - b * a.Hkv;
   int u0, u1;
-  split_tiles(keys_of(a, b, min(r / ROWS * ROWS + ROWS, R) - 1), a.splits, 1,
-              u0, u1);
+  split_tiles(a, b, keys_of(a, b, min(r / ROWS * ROWS + ROWS, R) - 1), 1, u0,
+              u1);
   if (u0 >= u1) return;
   // a lane has the maximum and the sum of a split
   const float* ml = a.pml + id * a.splits * 2;
@@ -417,11 +424,12 @@ void fei_attn_prefill(const void* q, const void* k_cache, const void* v_cache,
                       int S, int Hq, int Hkv, int D, int max_seq, float scale,
                       int causal, long q_ts, int splits, float* po, float* pml,
                       long kv_b, long kv_h, long kv_t, hipStream_t stream) {
-  const int G = Hq / Hkv;
+  const int G = Hq / Hkv, tiles = (S * G + ROWS - 1) / ROWS;
   const Prefill a{(const u16*)q, (const u16*)k_cache, (const u16*)v_cache,
                   (u16*)out,     po,     pml,  pos0,  kv_len,
                   S,             G,      Hkv,  B * Hkv,
-                  (S * G + ROWS - 1) / ROWS,   max_seq, causal, splits,
+                  tiles,         max_seq, causal, splits,
+                  9 + B * Hkv * tiles / 6,
                   scale,         q_ts,   kv_b, kv_h,  kv_t};
   if (D == 128) launch_prefill<128>(a, stream);
   else if (D == 64) launch_prefill<64>(a, stream);
