@@ -635,6 +635,10 @@ def linear_decode(x: torch.Tensor, w: torch.Tensor,
     M = x.numel() // K
     how = _product(x, w, M, K, N, out)
     if how is None:
+        # M > 256 for one: nothing is asked of few rows that they have not been
+        if (M > 256 and out is None and x.is_cuda and w.dim() == 2
+                and x.is_contiguous() and _tiles.linear_ok(M, x, w)):
+            return _tiles.linear(x.view(M, K), w).view(*x.shape[:-1], N)
         return torch.nn.functional.linear(x, w)
     x2 = x.contiguous().view(M, K)
     if out is None:

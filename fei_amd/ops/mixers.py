@@ -230,6 +230,13 @@ def skinny(out, x, w, n: int, epi: int, bias=None, scale: float = 1.0,
                       _p(sums), tiles, eps, _p(sums_out), _stream())
 
 
+def _linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [T, K] @ w^T of more rows than the kernels for few take."""
+    if x.stride(-1) == 1 and _tiles.linear_ok(x.shape[0], x, w):
+        return _tiles.linear(x, w)
+    return torch.nn.functional.linear(x, w)
+
+
 def _act_tile(x: torch.Tensor, w: torch.Tensor, ff: int,
               act: torch.Tensor) -> bool:
     """Whether the product of many rows writes its activations, ``ff`` a row, to
@@ -259,7 +266,7 @@ def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,
         _lib().fei_gemv_mix_in(_p(proj), _p(act), _p(n1), _p(n2), _p(w_in),
                                act.stride(0), T, n_mix, ff, K, 1, _stream())
         return proj
-    proj = torch.nn.functional.linear(n1, w_in[:n_mix])
+    proj = _linear(n1, w_in[:n_mix])
     if ff and own and _act_tile(n2, w_in[n_mix:], ff, act):
         _tiles.product(n2, w_in[n_mix:], act, ff, _tiles.TILE_SWIGLU)
     elif ff:
@@ -299,7 +306,7 @@ def parallel_in(h: GainNormed, w_in: torch.Tensor, n_mix: int, ff: int,
                    router=router, act=act, stride=act.stride(0))
         return proj, router
     rows = h.rows
-    proj = torch.nn.functional.linear(rows, w_in[:n_mix])
+    proj = _linear(rows, w_in[:n_mix])
     if ff and gpu and _act_tile(rows, w_in[n_mix:], ff, act):
         _tiles.product(rows, w_in[n_mix:], act, ff, _tiles.TILE_RELU2)
     elif ff:

@@ -19,8 +19,8 @@ TILE_BF16, TILE_SWIGLU, TILE_GELU, TILE_RELU2, TILE_PARTS = range(5)
 CUS = 256
 # Rows of x and w a tile, and us of a step of 64 of K: with one tile on the chip, and
 # what comes on top with one on every CU, when the card lowers its clock.
-TILES = ((256, 256, 0.95, 0.38), (256, 192, 0.82, 0.25), (192, 256, 0.82, 0.25),
-         (256, 128, 0.66, 0.17), (128, 256, 0.66, 0.17))
+TILES = ((256, 256, 1.0, 0.46), (256, 192, 0.875, 0.36), (192, 256, 0.82, 0.34),
+         (256, 128, 0.73, 0.13), (128, 256, 0.73, 0.13))
 
 
 def declare(lib: ctypes.CDLL) -> None:
@@ -52,9 +52,25 @@ def _time(M: int, cols: int, K: int, parts: int, rows: int, width: int,
 @lru_cache(maxsize=1024)
 def size_for(M: int, cols: int, K: int) -> Tuple[int, int]:
     """Rows of x and of w a tile for a product with ``cols`` of them.
-    16384 x 768 in 192 columns a tile is one full round, 24 us; in 256 three quarters
-    of one, 26; 16384 x 3072 three rounds of 256, 70, four of 192, 89."""
+    6006 x 3072, K = 2048, in tiles of 192 rows takes two rounds, three quarters full, 69
+    us; in 256 x 256 two, a little over half full, 86; 16384 x 3072, K = 768, three rounds
+    of 256, 70, four of 192, 89."""
     return min(TILES, key=lambda t: _time(M, cols, K, 1, *t))[:2]
+
+
+def linear_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether x [M, K] @ w^T is faster here than in the library: where K is 1024 to
+    2048 and the tiles fill the CUs to 0.86 PFLOP/s. Against the library, us: 3072 x 2048 of 6006 rows 69 (82), of 4000 41
+    (43), of 3000 36 (36), of 2048 29 (27); 5000 x 2048 of 1301 31 (34), of 2600 48 (62);
+    3648 x 2048 of 1706 30 (33); 6144 x 2048 of 1301 35 (43), of 1030 32 (31); the worst
+    that the rule takes 6144 x 2048 of 2600 64 (62). Of 4096 x 4096 and 6144 x 4096 neither
+    is better by more than 5 % up to 6006 rows."""
+    N, K = w.shape
+    if (not 1024 <= K <= 2048 or M <= 256 or not tile_ok(M, x, w)
+            or not _ops._mixers.match(x, w, x.shape[-1])):
+        return False
+    size = next(t for t in TILES if t[:2] == size_for(M, N, K))
+    return 2 * M * N * K > 0.86e9 * _time(M, N, K, 1, *size)
 
 
 def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, N: int,
@@ -64,6 +80,13 @@ def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, N: int,
     K = x.shape[1]
     size = size_for(x.shape[0], w.shape[0], K)
     _launch(out, x, w, N, epi, size, bias)
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x [M, K] @ w^T, for linear_ok."""
+    out = torch.empty(x.shape[0], w.shape[0], dtype=x.dtype, device=x.device)
+    product(x, w, out, w.shape[0], TILE_BF16)
+    return out
 
 
 def _launch(out, x, w, N, epi, size, bias=None, parts=1) -> None:

@@ -117,3 +117,22 @@ def test_residual_of_many_rows(M, N, K):
         want = res.double() + 0.5 * (a.double() @ w.double().t())
         # float32 sums of K products and one addition
         assert err(mx.residual_linear(res, a, w, 0.5), want) < 2 ** -24 * K ** 0.5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1301, 5704, 2048), (4001, 3072, 1984),
+                                   (3777, 2568, 1088), (300, 512, 2048)])
+def test_plain_products_of_many_rows(M, N, K):
+    """Through the public op and inside a layer's input, rows with gaps too; the last
+    is the library's."""
+    x, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
+    want = x.double() @ w.double().t()
+    assert tiles.linear_ok(M, x, w) == (M > 300)
+    # a result is rounded once, by 2^-9 at most
+    assert err(ops.linear_decode(x.view(1, M, K), w)[0], want) < 2 ** -9
+    for rows in (x, rand(M, K + 8, seed=1)[:, :K]):
+        want = rows.double() @ w.double().t()
+        assert err(mx.mix_in(rows, None, w, N, 0, rows), want) < 2 ** -9
+    v = w.clone().requires_grad_()           # gradients are the library's
+    assert not tiles.linear_ok(M, x, v)
+    assert ops.linear_decode(x, v).requires_grad
