@@ -256,7 +256,7 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
               float y = acc[a][b][i][j][e];
-              if (PAIR) y = y / (1.f + __expf(-y)) * acc[a][1][i][j][e];
+              if (PAIR) y = swiglu(y, acc[a][1][i][j][e]);
               if (EPI == TILE_GELU) y = gelu_erf(y + bf2f(add[j * 4 + e]));
               if (EPI == TILE_RELU2) y = relu2(y);
               v[j * 4 + e] = El<u16>::st(y);
