@@ -139,17 +139,25 @@ class BokenexModel(StepModel):
         None). ``on_run(r, residual)`` is called after every layer."""
         s, dt = self.spec, self.dtype
         x = ops.embed_pos(batch.tokens, batch.pos, self.emb, self.pos_emb)
+        rows = None
         for r, (lw, L) in enumerate(zip(self.layers, s.layers)):
             n_mix, mlp = L.mixer.out_cols, lw.mlp
             ff = mlp.act_cols if mlp is not None else 0
             cat = torch.empty(x.shape[0], n_mix + ff, dtype=dt,
                               device=x.device)
-            h = ops.GainNormed(x, lw.norm, dt)
+            h = ops.GainNormed(x, lw.norm, dt, rows)
+            rows = None
             proj, router = ops.parallel_in(
                 h, lw.w_in, L.mixer.in_rows, ff,
                 mlp.router_rows if mlp is not None else 0, cat[:, n_mix:])
             lw.mixer.run(proj, cat[:, :n_mix], batch, cache, r, {})
-            if router is None:
+            if router is None and on_run is None and r + 1 < len(self.layers):
+                after = self.layers[r + 1].norm
+                x, normed = ops.residual_norms(x, cat, lw.w_out, after.cols,
+                                               None, after.eps, dt,
+                                               s.residual_mult)
+                rows = normed and normed[0]
+            elif router is None:
                 x = ops.residual_linear(x, cat, lw.w_out, s.residual_mult)
             else:
                 x = ops.residual_moe(x, h, router, cat, lw.w_out, mlp.up,

@@ -147,19 +147,28 @@ class TobaraxModel(StepModel):
         s, dt = self.spec, self.dtype
         x = torch.nn.functional.embedding(batch.tokens, self.emb).float()
         x0 = x.clone() if s.loop is not None else None
+        normed = None
         for r, run in enumerate(s.runs):
             if run.enters_pass is not None:
                 x = ops.linear_f32(ops.cat_cast(x, x0, dt), self.loop_in,
                                    self.loop_step[run.enters_pass])
             lw, L = self.layers[run.layer], s.layers[run.layer]
-            n1, n2 = ops.norm_pair(x, lw.norm1, lw.norm2, s.norm_eps, dt)
+            n1, n2 = normed or ops.norm_pair(x, lw.norm1, lw.norm2, s.norm_eps,
+                                             dt)
             n_mix, ff = L.mixer.out_cols, L.ff or 0
             cat = torch.empty(x.shape[0], n_mix + ff, dtype=dt,
                               device=x.device)
             proj = ops.mix_in(n1, n2, lw.w_in, L.mixer.in_rows, ff,
                               cat[:, n_mix:])
             lw.mixer.run(proj, cat[:, :n_mix], batch, cache, r, self._rot)
-            x = ops.residual_linear(x, cat, lw.w_out)
+            # the norms behind the residual, unless it goes elsewhere first
+            after = s.runs[r + 1] if r + 1 < len(s.runs) else None
+            if on_run is None and after and after.enters_pass is None:
+                nw = self.layers[after.layer]
+                x, normed = ops.residual_norms(x, cat, lw.w_out, nw.norm1,
+                                               nw.norm2, s.norm_eps, dt)
+            else:
+                x, normed = ops.residual_linear(x, cat, lw.w_out), None
             if on_run is not None:
                 on_run(r, x)
         if batch.want_rows is not None:

@@ -415,6 +415,65 @@ k_parts_add(float* __restrict__ out, const float* __restrict__ parts, int np,
   ((f32x4*)out)[i] = y;
 }
 
+// The same, and both norms of the new rows (o2 may be null): what follows the product
+// that ends a layer. A row a block, four columns a thread and turn, of which four turns
+// stay in registers. 1301 rows of 2048, 4 parts: in two launches 11 us and 7; bound by
+// reading the parts, at 5 TB/s.
+__global__ void __launch_bounds__(256)
+k_parts_add_norms(u16* __restrict__ o1, u16* __restrict__ o2,
+                  float* __restrict__ x, const float* __restrict__ parts, int np,
+                  const float* __restrict__ w1, const float* __restrict__ w2,
+                  long step, int C, float scale, float eps) {
+  constexpr int KEEP = 4;
+  __shared__ float red[4];
+  const int tid = threadIdx.x, nv = C >> 2;
+  const long row = blockIdx.x;
+  f32x4* xr = (f32x4*)(x + row * C);
+  const f32x4* pr = (const f32x4*)(parts + row * C);
+  float ss = 0.f;
+  auto add = [&](int i) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = 0; k < np; ++k) {
+      const f32x4 q = pr[k * (step >> 2) + i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += q[e];
+    }
+    f32x4 y = xr[i];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[e] = fmaf(scale, v[e], y[e]);
+      ss = fmaf(y[e], y[e], ss);
+    }
+    xr[i] = y;
+    return y;
+  };
+  f32x4 y[KEEP];
+#pragma unroll
+  for (int k = 0; k < KEEP; ++k)
+    if (tid + k * 256 < nv) y[k] = add(tid + k * 256);
+  for (int i = tid + KEEP * 256; i < nv; i += 256) add(i);
+  ss = block_reduce_sum(ss, red);
+  const float inv = 1.f / sqrtf(ss / (float)C + eps);
+  auto norm = [&](int i, f32x4 v) {
+    const f32x4 a = ((const f32x4*)w1)[i];
+    u16 t[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] = El<u16>::st(v[e] * inv * a[e]);
+    __builtin_memcpy(o1 + row * C + i * 4, t, sizeof(t));
+    if (o2) {
+      const f32x4 b = ((const f32x4*)w2)[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) t[e] = El<u16>::st(v[e] * inv * b[e]);
+      __builtin_memcpy(o2 + row * C + i * 4, t, sizeof(t));
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < KEEP; ++k)
+    if (tid + k * 256 < nv) norm(tid + k * 256, y[k]);
+  for (int i = tid + KEEP * 256; i < nv; i += 256) norm(i, xr[i]);
+}
+
 }  // namespace
 
 extern "C" {
@@ -482,6 +541,16 @@ void fei_parts_add(float* out, const float* parts, int np, long n, float scale,
                    hipStream_t stream) {
   hipLaunchKernelGGL(k_parts_add, dim3((n / 4 + 255) / 256), dim3(256), 0,
                      stream, out, parts, np, n / 4, scale);
+}
+
+// x [rows, C] float32 += scale * the sums, and its norms with gains w1 and w2 in
+// bfloat16 (o2, w2 may be null); C % 4 == 0, all on 16 bytes, o1 and o2 on 8
+void fei_parts_add_norms(void* o1, void* o2, float* x, const float* parts,
+                         int np, const float* w1, const float* w2, int rows,
+                         int C, float scale, float eps, hipStream_t stream) {
+  hipLaunchKernelGGL(k_parts_add_norms, dim3(rows), dim3(256), 0, stream,
+                     (u16*)o1, (u16*)o2, x, parts, np, w1, w2, (long)rows * C, C,
+                     scale, eps);
 }
 
 }  // extern "C"

@@ -137,9 +137,10 @@ class GainNormed:
     commute with a product, so a product of a row or two takes x as it is
     and makes the norm inside; the others take the normed ``rows``."""
 
-    def __init__(self, x: torch.Tensor, norm: GainNorm, dtype: torch.dtype):
+    def __init__(self, x: torch.Tensor, norm: GainNorm, dtype: torch.dtype,
+                 rows: Optional[torch.Tensor] = None):
         self.x, self.norm, self.dtype = x, norm, dtype
-        self._rows: Optional[torch.Tensor] = None
+        self._rows = rows
 
     @property
     def rows(self) -> torch.Tensor:
@@ -369,6 +370,28 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
         return x
     return torch.addmm(x, a, w.t(), out_dtype=torch.float32, alpha=mult,
                        out=x)
+
+
+def residual_norms(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
+                   w1: torch.Tensor, w2: Optional[torch.Tensor], eps: float,
+                   dtype: torch.dtype, mult: float = 1.0
+                   ) -> Tuple[torch.Tensor, Optional[Tuple]]:
+    """residual_linear, and the norm_pair of its result where one kernel makes
+    both: that of many rows, whose product comes in parts. Else None, and who
+    needs the norms asks for them."""
+    T, C = x.shape
+    gains = [w1] if w2 is None else [w1, w2]
+    if (a.is_cuda and dtype is _BF16 and dense(x, torch.float32, a, T, C)
+            and all(dense(g, torch.float32, a, C) and g.data_ptr() % 16 == 0
+                    and not (g.requires_grad and torch.is_grad_enabled())
+                    for g in gains)
+            and a.shape[0] == T and w.shape[0] == C and C % 4 == 0):
+        parts = (_rows.product_parts(a, w) if _rows.add_ok(x, a, w)
+                 else _tiles.product_parts(a, w) if _tiles.add_ok(x, a, w)
+                 else None)
+        if parts is not None:
+            return x, _rows.add_parts_norms(x, parts, mult, w1, w2, eps)
+    return residual_linear(x, a, w, mult), None
 
 
 def linear_f32(a: torch.Tensor, w: torch.Tensor,

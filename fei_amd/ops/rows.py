@@ -4,7 +4,7 @@ kernel after them sums, or with the SwiGLU inside. bfloat16 GPU tensors only."""
 from __future__ import annotations
 
 import ctypes
-from typing import Tuple
+from typing import Optional, Tuple
 
 import torch
 
@@ -24,6 +24,8 @@ def declare(lib: ctypes.CDLL) -> None:
     lib.fei_parts_norm.argtypes = [_vp, _vp, _vp, _i, _vp, _i, _i, _f, _vp]
     lib.fei_rope_kv_parts.argtypes = [_vp, _vp, _i] + [_vp] * 4 + [_i] * 6 + [_vp]
     lib.fei_parts_add.argtypes = [_vp, _vp, _i, _l, _f, _vp]
+    lib.fei_parts_add_norms.argtypes = (
+        [_vp] * 4 + [_i] + [_vp] * 2 + [_i, _i, _f, _f, _vp])
 
 
 def _lib() -> ctypes.CDLL:
@@ -154,3 +156,17 @@ def add_parts(x: torch.Tensor, parts: torch.Tensor, mult: float) -> None:
     values."""
     _lib().fei_parts_add(_p(x), _p(parts), parts.shape[0], x.numel(), mult,
                          _stream())
+
+
+def add_parts_norms(x: torch.Tensor, parts: torch.Tensor, mult: float,
+                    w1: torch.Tensor, w2: Optional[torch.Tensor], eps: float
+                    ) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """add_parts to x [M, C], and its norms with the float32 gains in bfloat16."""
+    M, C = x.shape
+    o1 = torch.empty(M, C, dtype=torch.bfloat16, device=x.device)
+    o2 = None if w2 is None else torch.empty_like(o1)
+    _lib().fei_parts_add_norms(
+        _p(o1), None if o2 is None else _p(o2), _p(x), _p(parts),
+        parts.shape[0], _p(w1), None if w2 is None else _p(w2), M, C, mult,
+        eps, _stream())
+    return o1, o2

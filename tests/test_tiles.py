@@ -136,3 +136,27 @@ def test_plain_products_of_many_rows(M, N, K):
     v = w.clone().requires_grad_()           # gradients are the library's
     assert not tiles.linear_ok(M, x, v)
     assert ops.linear_decode(x, v).requires_grad
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,pair", [
+    (40, 8, 4096, True), (256, 1000, 4160, False), (257, 2048, 8192, True),
+    (300, 4104, 8256, True), (300, 256, 4096, False)])
+def test_residual_and_its_norms(M, N, K, pair):
+    """What one kernel makes of a product in parts, some columns and more than its
+    registers hold; the last is in the library, which leaves the norms to others."""
+    a, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
+    x, g = rand(M, N, seed=3).float(), rand(2, N, seed=4).float()
+    want = x.double() + 0.5 * (a.double() @ w.double().t())
+    y, normed = mx.residual_norms(x, a, w, g[0], g[1] if pair else None, 1e-3,
+                                  torch.bfloat16, 0.5)
+    # float32 sums of K products and one addition
+    assert err(y, want) < 2 ** -24 * K ** 0.5
+    assert (normed is None) == (K == 4096 and M > 256)
+    if normed is None:
+        return
+    norm = want * (want.pow(2).mean(-1, keepdim=True) + 1e-3).rsqrt()
+    # rounded once, by 2^-9 at most
+    assert err(normed[0], norm * g[0].double()) < 2 ** -9
+    assert err(normed[1], norm * g[1].double()) < 2 ** -9 if pair \
+        else normed[1] is None
