@@ -266,9 +266,10 @@ class LlamaModel:
         for li, lw in enumerate(self.layers):
             qkv = ops.gemv_norm(h, lw.norm_attn, lw.wqkv, eps, sums=sums)
             att = attend(li, qkv)
-            sums = ops.add_product(att.reshape(h.shape[0], -1), lw.wo, h)
+            sums = ops.add_product(att.reshape(h.shape[0], -1), lw.wo, h,
+                                   True)
             act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, eps, sums=sums)
-            sums = ops.add_product(act, lw.wdown, h)
+            sums = ops.add_product(act, lw.wdown, h, True)
         return sums
 
     def fused_rows(self, B: int) -> bool:
@@ -373,10 +374,10 @@ class LlamaModel:
                                                s.norm_eps)
                 ops.gemv_res_fp8(act, *q8["wdown"], h)
             elif ssq is None:
-                sums = ops.add_product(att.reshape(B, -1), lw.wo, h)
+                sums = ops.add_product(att.reshape(B, -1), lw.wo, h, True)
                 act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, s.norm_eps,
                                            sums=sums)
-                sums = ops.add_product(act, lw.wdown, h)
+                sums = ops.add_product(act, lw.wdown, h, True)
             else:
                 ops.gemv_res(att.reshape(B, -1), lw.wo, h, ssq_out=ssq[2 * li])
                 act = ops.gemv_swiglu_norm(h, lw.norm_mlp, lw.wgu, s.norm_eps,

@@ -715,17 +715,20 @@ def gemv_res(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
     return res
 
 
-def add_product(x: torch.Tensor, w: torch.Tensor,
-                res: torch.Tensor) -> Optional[torch.Tensor]:
+def add_product(x: torch.Tensor, w: torch.Tensor, res: torch.Tensor,
+                any_tiles: bool = False) -> Optional[torch.Tensor]:
     """gemv_res, for a chain: returns the sums of squares of the new rows by
-    tiles of columns, for the ``sums`` of the products that read them under a
-    norm, or None where those do not need them."""
+    tiles of 16 columns, for the ``sums`` of the products that read them under a
+    norm, or None where those do not need them. ``any_tiles``: of any number of
+    columns, which leaves the kernel its choice of blocks."""
     K, N = x.shape[-1], w.shape[0]
     M = x.numel() // K
     if _product(x, w, M, K, N, res) != "skinny":
         gemv_res(x, w, res)
         return None
-    sums = torch.empty(M, -(-N // 16), dtype=torch.float32, device=x.device)
+    # blocks have 8 columns where with 16 CUs would be left without
+    sums = torch.empty(M, -(-N // (8 if any_tiles and N <= 2048 else 16)),
+                       dtype=torch.float32, device=x.device)
     _mixers.skinny(res, x.contiguous().view(M, K), w, N, _mixers.EPI_RES_BF16,
                    sums_out=sums)
     return sums

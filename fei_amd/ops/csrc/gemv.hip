@@ -371,10 +371,11 @@ namespace {
 // product before left.
 struct SkinnyNorm {
   const u16* gain;     // null: none
-  const float* sums;   // [M, tiles], one per 16 columns of x
+  const float* sums;   // [M, tiles], together of all columns of x
   int tiles;
   float eps;
-  float* sums_out;     // EPI_RES_BF16: the same of the new rows; may be null
+  float* sums_out;     // EPI_RES_BF16: the same of the new rows; may be null. With
+                       // tiles of N / 8 they are of 8 columns each
 };
 
 // XL: groups of 8 rows of x. N: results a row of x; with EPI_SWIGLU w has N
@@ -390,13 +391,14 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
          const u16* __restrict__ w, int M, int N, int K, Epilogue ep,
          SkinnyNorm nm) {
   constexpr int MT = (XL + 1) / 2;
-  constexpr int LOADS = 2 * RT + XL, STAGE = LOADS * 512;
-  constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : RT;
+  constexpr int WL = RT ? 2 * RT : 1, FR = RT ? RT : 1;  // loads, fragments of w
+  constexpr int LOADS = WL + XL, STAGE = LOADS * 512;
+  constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : FR;
   extern __shared__ __align__(16) u16 buf[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l15 = lane & 15, lg = lane >> 4;
-  const int n0 = blockIdx.x * 16 * RO;
+  const int n0 = blockIdx.x * (RT ? 16 * RO : 8);
   const int r8 = lane >> 3, c8 = ((lane & 7) ^ r8) * 8;
   const int steps = K / 64, per = (steps + 3) / 4;
   const int lo = min(wid * per, steps - 1);
@@ -411,14 +413,14 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
   };
   const u16* src[LOADS];
 #pragma unroll
-  for (int i = 0; i < 2 * RT; ++i) {
+  for (int i = 0; i < WL; ++i) {
     long row = min(n0 + i % (2 * RO) * 8 + r8, N - 1);
     if (i >= 2 * RO) row += N;
     src[i] = w + row * K + c8;
   }
 #pragma unroll
   for (int i = 0; i < XL; ++i)
-    src[2 * RT + i] = x + (long)min(i * 8 + r8, M - 1) * K + c8;
+    src[WL + i] = x + (long)min(i * 8 + r8, M - 1) * K + c8;
   u16* mine = buf + wid * S * STAGE;
   const u32 lds = (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)mine;
   // nothing is asked for past the end: a wave often has few more stages than it asks
@@ -430,13 +432,13 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const u32 to = lds + (b * STAGE + i * 512) * 2;
-      if (i < 2 * RT) load_lds_nt(src[i] + k, to);
+      if (i < WL) load_lds_nt(src[i] + k, to);
       else load_lds(src[i] + k, to);
     }
   };
-  f32x4 acc[RT][MT];
+  f32x4 acc[FR][MT];
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+  for (int i = 0; i < FR; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // NORM: the gains go behind the stages; the sums of squares (of rows wid, wid
@@ -481,13 +483,14 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
   for (int s = 0; s < n; ++s) {
     wait(min(S, n - s) - 1);
     const u16* bw = mine + b * STAGE;
-    const u16* bx = bw + RT * 1024;
-    s16x8 fa[2][RT], fb[2][MT];
+    const u16* bx = bw + WL * 512;
+    s16x8 fa[2][FR], fb[2][MT];
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk) {
       const int c = ((kk * 4 + lg) ^ (l15 & 7)) * 8;
 #pragma unroll
-      for (int i = 0; i < RT; ++i) fa[kk][i] = ld8(bw + (i * 16 + l15) * 64 + c);
+      for (int i = 0; i < FR; ++i)     // 8 rows stand for the next 8 as well
+        fa[kk][i] = ld8(bw + (i * 16 + (RT ? l15 : l15 & 7)) * 64 + c);
 #pragma unroll
       for (int j = 0; j < MT; ++j) {
         // an odd group of 8 rows stands in for the one after it
@@ -522,7 +525,7 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
 #pragma unroll
     for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
-      for (int i = 0; i < RT; ++i)
+      for (int i = 0; i < FR; ++i)
 #pragma unroll
         for (int j = 0; j < MT; ++j)
           acc[i][j] = mma(fa[kk][i], fb[kk][j], acc[i][j]);
@@ -546,7 +549,7 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
   __syncthreads();
   f32x4* red = (f32x4*)buf;
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+  for (int i = 0; i < FR; ++i)
 #pragma unroll
     for (int j = 0; j < MT; ++j)
       red[((i * MT + j) * 4 + wid) * 64 + lane] = acc[i][j];
@@ -576,7 +579,7 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
     float sq = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      if (m >= M || n + e >= N) break;
+      if (m >= M || n + e >= N || (!RT && lg > 1)) break;
       if (EPI == EPI_SWIGLU) ep.act[m * ep.as + n + e] = f2bf(v[e]);
       else epilogue<EPI>(outp, m, N, n + e, v[e], ep);
       if (EPI == EPI_RES_BF16) {
@@ -587,7 +590,7 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
     if (EPI == EPI_RES_BF16 && nm.sums_out) {
       sq += __shfl_xor(sq, 16);
       sq += __shfl_xor(sq, 32);
-      const int tile = n0 / 16 + t / MT;
+      const int tile = n0 / (RT ? 16 : 8) + t / MT;
       if (lg == 0 && m < M && tile < nm.tiles)
         nm.sums_out[(long)m * nm.tiles + tile] = sq;
     }
@@ -599,12 +602,13 @@ void launch_skinny(void* out, const void* x, const void* w, int M, int N,
                    int K, const Epilogue& ep, const SkinnyNorm& nm,
                    hipStream_t stream) {
   constexpr int MT = (XL + 1) / 2;
-  constexpr int stages = 4 * S * (2 * RT + XL), sums = RT * MT * 4;
+  constexpr int WL = RT ? 2 * RT : 1, sums = (RT ? RT : 1) * MT * 4;
+  constexpr int stages = 4 * S * (WL + XL);
   constexpr int lds = (stages > sums ? stages : sums) * 1024;
-  constexpr int RO = EPI == EPI_SWIGLU ? RT / 2 : RT;
+  constexpr int cols = EPI == EPI_SWIGLU ? 8 * RT : 8 * WL;
   auto go = [&](auto kernel, int bytes) {
     allow_lds(kernel, bytes);
-    hipLaunchKernelGGL(kernel, dim3((N + 16 * RO - 1) / (16 * RO)), dim3(256),
+    hipLaunchKernelGGL(kernel, dim3((N + cols - 1) / cols), dim3(256),
                        bytes, stream, out, (const u16*)x, (const u16*)w, M, N,
                        K, ep, nm);
   };
@@ -615,6 +619,12 @@ void launch_skinny(void* out, const void* x, const void* w, int M, int N,
   go(k_skinny<EPI, XL, RT, S, false>, lds);
 }
 
+// Rows of w for 128 tiles of 16 and fewer: tiles of 8 (RT = 0), half of whose products
+// are for nothing, but which twice as many CUs load. 2048 x 8192, 8 rows 11.4 -> 9.0 us,
+// 20 14.3 -> 11.6, 64 24.1 -> 21.6; 2048 x 2048, 20 rows 6.1 -> 5.5; 768 x 3072, 24 rows
+// 6.8 -> 5.8. What a CU gets through is 60 KB a us of w and x together, whatever the
+// stages in flight (2 to 8), waves (4 to 16) and first steps. The sums of squares that
+// these leave are of 8 columns, for which the caller has to have room.
 // Few rows of w (under 320 tiles, little more than one a CU): small tiles, so
 // that all CUs load. 4096 rows, 8 of x: 7.8 us against 9.9; 6144: 12.1, 10.6.
 // Many with more than 24 rows of x: wide tiles, so that x is repeated less.
@@ -626,10 +636,14 @@ void by_tiles(void* out, const void* x, const void* w, int M, int N, int K,
   if constexpr (XL >= 4)
     if (rows >= 16384)
       return launch_skinny<EPI, XL, 4, 2>(out, x, w, M, N, K, ep, nm, stream);
-  if constexpr (EPI != EPI_SWIGLU)
+  if constexpr (EPI != EPI_SWIGLU) {
+    if (rows <= 2048 && (!nm.sums_out || nm.tiles >= (N + 7) / 8))
+      return launch_skinny<EPI, XL, 0, (XL < 4 ? 4 : 3)>(out, x, w, M, N, K, ep,
+                                                         nm, stream);
     if (rows < 5120)
       return launch_skinny<EPI, XL, 1, (XL < 4 ? 3 : 2)>(out, x, w, M, N, K,
                                                          ep, nm, stream);
+  }
   launch_skinny<EPI, XL, 2, 2>(out, x, w, M, N, K, ep, nm, stream);
 }
 
@@ -649,7 +663,8 @@ void by_rows(void* out, const void* x, const void* w, int M, int N, int K,
 // 1 to 64 rows, K % 64 == 0, rows of x and w 16-byte aligned. See Epilogue for
 // what becomes of the sums and which of the arguments that takes. gain (up to 32
 // rows, EPI_BF16 and EPI_SWIGLU; 16-byte aligned): x under an RMS norm with the
-// sums [M, tiles]. sums_out (EPI_RES_BF16): [M, tiles], tiles = N / 16 up.
+// sums [M, tiles]. sums_out (EPI_RES_BF16): [M, tiles], tiles = N / 16 up, or, of N up
+// to 2048, N / 8 up.
 extern "C" void fei_skinny(void* out, const void* x, const void* w, int M,
                            int N, int K, int epi, const float* bias,
                            float scale, float cap, int n_mix, int n_router,

@@ -366,6 +366,31 @@ def test_skinny_geometries(lib, M, N, K):
             < 2 ** -6
 
 
+@pytest.mark.parametrize("M", [2, 8, 9, 24, 32])
+@pytest.mark.parametrize("N,K", [(16, 64), (200, 320), (2048, 192), (2056, 64),
+                                 (4000, 128)])
+def test_skinny_blocks_of_8_columns(lib, M, N, K):
+    """Up to 2048 columns and past them: sums of squares by blocks, a last block in
+    part, waves without steps; the products that read the rows under a norm."""
+    x, w = randbf(M, K, seed=1), randbf(N, K, seed=2, scale=K ** -0.5)
+    h, res = randbf(M, N, seed=3), randbf(M, N, seed=3)
+    want = h.double() + x.double() @ w.double().T
+    sums = lib.add_product(x, w, h, any_tiles=True)
+    # rounded once, by 2^-9 at most; the sums of squares are of what is written
+    assert row_err(h, want) < 2 ** -8
+    cols = 8 if N <= 2048 else 16
+    sq = torch.nn.functional.pad(h.double() ** 2, (0, -N % cols))
+    assert row_err(sums, sq.view(M, -1, cols).sum(-1)) < 1e-5
+    assert row_err(lib.add_product(x, w, res),
+                   torch.nn.functional.pad(res.double() ** 2, (0, -N % 16))
+                   .view(M, -1, 16).sum(-1)) < 1e-5
+    if N % 64 == 0:
+        g, w2 = randbf(N, seed=4), randbf(48, N, seed=5, scale=N ** -0.5)
+        # 2^-9 of each product, up to twice that of a row of few results
+        assert row_err(lib.gemv_norm(h, g, w2, 1e-5, sums=sums),
+                       rms64(h, g, 1e-5) @ w2.double().T) < 2 ** -7
+
+
 # -- RoPE of a prompt --------------------------------------------------------------
 
 @pytest.mark.parametrize("B,S,Hq,Hkv,D,pad", [
