@@ -233,7 +233,8 @@ def skinny(out, x, w, n: int, epi: int, bias=None, scale: float = 1.0,
 
 def _linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x [T, K] @ w^T of more rows than the kernels for few take."""
-    if x.stride(-1) == 1 and _tiles.linear_ok(x.shape[0], x, w):
+    if (x.shape[0] > 256 and x.stride(-1) == 1
+            and _tiles.linear_ok(x.shape[0], x, w)):
         return _tiles.linear(x, w)
     return torch.nn.functional.linear(x, w)
 
@@ -380,6 +381,8 @@ def residual_norms(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
     both: that of many rows, whose product comes in parts. Else None, and who
     needs the norms asks for them."""
     T, C = x.shape
+    if T <= SKINNY_ROWS:
+        return residual_linear(x, a, w, mult), None
     gains = [w1] if w2 is None else [w1, w2]
     if (a.is_cuda and dtype is _BF16 and dense(x, torch.float32, a, T, C)
             and all(dense(g, torch.float32, a, C) and g.data_ptr() % 16 == 0

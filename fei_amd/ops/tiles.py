@@ -31,11 +31,24 @@ def _p(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
 
+def _memory(*tensors: torch.Tensor) -> bool:
+    """Whether the tensors are what lies at their pointers, and nothing follows what
+    is done to them: tracing, transforms, tangents and dispatch modes are for the
+    library's operations."""
+    c = torch._C                 # 2 us
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+            and c._functorch.peek_interpreter_stack() is None
+            and torch.autograd.forward_ad._current_level < 0
+            and not c._len_torch_dispatch_stack()
+            and c._get_tracing_state() is None
+            and not torch.compiler.is_compiling())
+
+
 def tile_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether M rows x times w run here; x's rows may lie apart."""
     K = w.shape[-1]
     return (M > 128 and w.is_cuda and w.dim() == 2 and K > 0 and K % 64 == 0
-            and w.shape[0] > 0 and w.shape[0] % 8 == 0
+            and w.shape[0] > 0 and w.shape[0] % 8 == 0 and _memory(x, w)
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
             and x.stride(-1) == 1 and x.stride(-2) % 8 == 0)
 
@@ -66,7 +79,7 @@ def linear_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     that the rule takes 6144 x 2048 of 2600 64 (62). Of 4096 x 4096 and 6144 x 4096 neither
     is better by more than 5 % up to 6006 rows."""
     N, K = w.shape
-    if (not 1024 <= K <= 2048 or M <= 256 or not tile_ok(M, x, w)
+    if (M <= 256 or not 1024 <= K <= 2048 or not tile_ok(M, x, w)
             or not _ops._mixers.match(x, w, x.shape[-1])):
         return False
     size = next(t for t in TILES if t[:2] == size_for(M, N, K))

@@ -160,3 +160,33 @@ def test_residual_and_its_norms(M, N, K, pair):
     assert err(normed[0], norm * g[0].double()) < 2 ** -9
     assert err(normed[1], norm * g[1].double()) < 2 ** -9 if pair \
         else normed[1] is None
+
+
+def test_tensors_that_are_more_than_memory():
+    """Tiles leave them to the library; no GPU is needed to say which they are."""
+    x = rand(4, 8, dev="cpu")
+    w = torch.nn.Parameter(x)
+    assert tiles._memory(x, w)
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(tiles._memory(t)), t)[1])(x[None])
+    with torch.autograd.forward_ad.dual_level():
+        seen.append(tiles._memory(x))
+    with torch._subclasses.FakeTensorMode():
+        seen.append(tiles._memory(x))
+    torch.jit.trace(lambda t: (seen.append(tiles._memory(t)), t + 1)[1], x,
+                    check_trace=False)
+    assert len(seen) >= 4 and not any(seen)
+
+
+@pytest.mark.gpu
+def test_many_rows_under_transforms():
+    M, N, K = 1301, 5704, 2048
+    x, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
+    v = rand(M, K, seed=3)
+    assert tiles.linear_ok(M, x, w)
+    y, dy = torch.func.jvp(lambda t: ops.linear_decode(t, w), (x,), (v,))
+    # results are rounded once, by 2^-9 at most
+    assert err(y, x.double() @ w.double().t()) < 2 ** -9
+    assert err(dy, v.double() @ w.double().t()) < 2 ** -9
+    both = torch.func.vmap(lambda t: ops.linear_decode(t, w))(torch.stack([x, v]))
+    assert err(both[1], v.double() @ w.double().t()) < 2 ** -9
