@@ -448,6 +448,11 @@ void launch_decode(DecodeAttn a, int B, hipStream_t stream) {
   // last: a block waits for the position to know that it has no keys, and keeps
   // its place meanwhile. 20 sequences of up to 600 keys in pages, 16 splits
   // asked for: 15.9 -> 7.8 us.
+  // Nor more blocks than the chip has places (three on a CU, four of heads of 64), or
+  // the last would begin when others end: 16 sequences of up to 900 keys, 8 heads of
+  // 128, 6 splits 15.3 us, 16 18.5; 8 of 3000 12 24.6, 16 27.5; 12 of 2047, the worst
+  // of it, 8 26.7, 16 25.9.
+  a.splits = max(1, min(a.splits, (D == 64 ? 1024 : 768) / (a.Hkv * B)));
   const int all = max(1, min(a.splits, (a.max_seq + CHUNK * SHARE - 1) /
                                            (CHUNK * SHARE)));
   const int side = min(all, 16);

@@ -250,6 +250,16 @@ def test_attn_decode_in_one_block(lib, D, paged, rope, Hq, Hkv, lens):
     test_attn_decode_geometries(lib, D, paged, rope, Hq, Hkv, 8, lens)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,lens", [
+    (16, 8, [1500, 1, 700, 129, 128, 900] * 3),  # 144 heads: fewer splits than asked
+    (10, 10, list(range(1200, 1350, 10))),       # 150
+])
+def test_attn_decode_as_many_blocks_as_places(lib, D, paged, Hq, Hkv, lens):
+    test_attn_decode_geometries(lib, D, paged, True, Hq, Hkv, 16, lens)
+
+
 @pytest.mark.parametrize("paged", [False, True])
 def test_attn_decode_in_one_block_without_keys(lib, paged):
     test_attn_decode_without_keys(lib, paged, 192, 4)
