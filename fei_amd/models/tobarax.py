@@ -148,7 +148,8 @@ class TobaraxModel(StepModel):
         x = torch.nn.functional.embedding(batch.tokens, self.emb).float()
         x0 = x.clone() if s.loop is not None else None
         normed = None
-        for r, run in enumerate(s.runs):
+        runs = s.runs            # made anew each time
+        for r, run in enumerate(runs):
             if run.enters_pass is not None:
                 x = ops.linear_f32(ops.cat_cast(x, x0, dt), self.loop_in,
                                    self.loop_step[run.enters_pass])
@@ -162,7 +163,7 @@ class TobaraxModel(StepModel):
                               cat[:, n_mix:])
             lw.mixer.run(proj, cat[:, :n_mix], batch, cache, r, self._rot)
             # the norms behind the residual, unless it goes elsewhere first
-            after = s.runs[r + 1] if r + 1 < len(s.runs) else None
+            after = runs[r + 1] if r + 1 < len(runs) else None
             if on_run is None and after and after.enters_pass is None:
                 nw = self.layers[after.layer]
                 x, normed = ops.residual_norms(x, cat, lw.w_out, nw.norm1,

@@ -243,7 +243,8 @@ def _act_tile(x: torch.Tensor, w: torch.Tensor, ff: int,
               act: torch.Tensor) -> bool:
     """Whether the product of many rows writes its activations, ``ff`` a row, to
     ``act`` itself."""
-    return (ff % 8 == 0 and plain(x, w) and _tiles.tile_ok(x.shape[0], x, w)
+    return (x.shape[0] > 128 and ff % 8 == 0 and plain(x, w)
+            and _tiles.tile_ok(x.shape[0], x, w)
             and act.dtype is _BF16 and act.stride(1) == 1
             and act.stride(0) % 8 == 0 and act.data_ptr() % 16 == 0)
 
@@ -373,6 +374,14 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
                        out=x)
 
 
+def _gain(g: torch.Tensor, C: int, like: torch.Tensor) -> bool:
+    """Whether a pointer stands for C float32 gains, four at a time."""
+    return (g.dtype is torch.float32 and g.shape[0] == C and C % 4 == 0
+            and g.dim() == 1 and g.is_contiguous() and g.data_ptr() % 16 == 0
+            and g.get_device() == like.get_device()
+            and not (g.requires_grad and torch.is_grad_enabled()))
+
+
 def residual_norms(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
                    w1: torch.Tensor, w2: Optional[torch.Tensor], eps: float,
                    dtype: torch.dtype, mult: float = 1.0
@@ -383,12 +392,9 @@ def residual_norms(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
     T, C = x.shape
     if T <= SKINNY_ROWS:
         return residual_linear(x, a, w, mult), None
-    gains = [w1] if w2 is None else [w1, w2]
-    if (a.is_cuda and dtype is _BF16 and dense(x, torch.float32, a, T, C)
-            and all(dense(g, torch.float32, a, C) and g.data_ptr() % 16 == 0
-                    and not (g.requires_grad and torch.is_grad_enabled())
-                    for g in gains)
-            and a.shape[0] == T and w.shape[0] == C and C % 4 == 0):
+    if (dtype is _BF16 and a.is_cuda and a.shape[0] == T and w.shape[0] == C
+            and _gain(w1, C, a) and (w2 is None or _gain(w2, C, a))
+            and dense(x, torch.float32, a, T, C)):
         parts = (_rows.product_parts(a, w) if _rows.add_ok(x, a, w)
                  else _tiles.product_parts(a, w) if _tiles.add_ok(x, a, w)
                  else None)
