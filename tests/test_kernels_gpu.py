@@ -148,6 +148,21 @@ def rope64(x, pos, theta=500000.0):
     return torch.cat([u * a.cos() - w * a.sin(), w * a.cos() + u * a.sin()], -1)
 
 
+def test_attn_prefill_rows_far_apart(lib):
+    """Cache rows so far from each other that a tile's offsets have more than 32
+    bits."""
+    n, S, D, far = 70, 40, 64, 1 << 25
+    room = torch.empty(n * far, dtype=torch.bfloat16, device=DEV)
+    k, v = (room[i * D:].as_strided((1, 1, n, D), (n * far, n * far, far, 1))
+            for i in range(2))
+    k.copy_(randbf(1, 1, n, D, seed=1))
+    v.copy_(randbf(1, 1, n, D, seed=2))
+    q = randbf(1, S, 2, D, seed=3)
+    p0 = torch.tensor([n - S], dtype=torch.int32, device=DEV)
+    assert torch.equal(lib.attn_prefill(q, k, v, p0),
+                       lib.attn_prefill(q, k.contiguous(), v.contiguous(), p0))
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("paged", [False, True])
 @pytest.mark.parametrize("rope", [False, True])
