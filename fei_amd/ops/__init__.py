@@ -270,6 +270,8 @@ def _launch_attn_decode(q, kc, vc, blocks, max_seq: int, bs_log: int,
     else:
         kin = vin = cs = None
         kv_bs = 0
+    if not B:
+        return out
     require_lib().fei_attn_decode(
         _ptr(q), _ptr(kc), _ptr(vc), None if blocks is None else _ptr(blocks),
         _ptr(part_o), _ptr(part_ml), _ptr(out), _ptr(pos), B, Hq, Hkv, D,

@@ -468,7 +468,7 @@ void launch_decode(DecodeAttn a, int B, hipStream_t stream) {
 // max_seq: rows of a head in a contiguous cache; of a paged one (table not
 // null) the positions that a row of the table can name. cs null: q is roped and
 // the new token's row is in the cache. Up to 16 query heads a kv head, up to 64
-// splits; D is 64 or 128.
+// splits; D is 64 or 128. Nothing is launched for an empty batch.
 extern "C" void fei_attn_decode(const void* q, void* kc, void* vc,
                                 const int* table, float* po, float* pml,
                                 void* out, const int* pos, int B, int Hq,
@@ -477,6 +477,7 @@ extern "C" void fei_attn_decode(const void* q, void* kc, void* vc,
                                 const void* kin, const void* vin,
                                 const float* cs, long kv_bs,
                                 hipStream_t stream) {
+  if (B <= 0 || Hkv <= 0) return;
   const DecodeAttn a{(const u16*)q, (u16*)kc,         (u16*)vc,
                      table,         po,               pml,
                      (u16*)out,     pos,              (const u16*)kin,

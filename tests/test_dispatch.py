@@ -1,6 +1,9 @@
 """Which calls the kernels for few rows take: those whose tensors are what the
 kernels read through a bare pointer. The others get what the library gives."""
 
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -186,3 +189,34 @@ def test_tiles_to_expect(E, top, rows):
             seen.append(int((-(-ids.bincount(minlength=E) // rows)).sum()))
         # the mean of 30, and that top choices of a row are never the same
         assert abs(likely_tiles(n, E, rows) - sum(seen) / 30) < 1 + 0.05 * E
+
+
+@pytest.mark.parametrize("T", [64, 192, 1024])
+@pytest.mark.parametrize("D", [64, 128])
+def test_attn_decode_of_no_sequences_returns(D, T):
+    """Whichever way as many positions would go; in a process of its own, which it
+    would end. Nothing is launched, so it needs no GPU."""
+    if not ops.kernels_available():
+        pytest.skip("the kernels are not built")
+    call = ("from fei_amd import ops; ops.require_lib().fei_attn_decode("
+            "*[None] * 8, 0, 8, 2, {}, {}, 0, 0, 4, 1.0, 0, None, None, None, 0, "
+            "None)").format(D, T)
+    done = subprocess.run([sys.executable, "-c", call], capture_output=True,
+                          text=True, timeout=300)
+    assert done.returncode == 0, done
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [64, 192, 1024])
+def test_attn_decode_of_an_empty_batch(T):
+    q = rand(0, 8, 64, dev=DEV)
+    pos = torch.zeros(0, dtype=torch.int32, device=DEV)
+    kc = rand(0, 2, T, 64, dev=DEV)
+    assert ops.attn_decode(q, kc, kc, pos, splits=4).shape == (0, 8, 64)
+    pool = rand(4, 2, 16, 64, dev=DEV)
+    table = torch.zeros(0, T // 16, dtype=torch.int32, device=DEV)
+    assert ops.attn_decode_paged(q, pool, pool, table, pos,
+                                 splits=4).shape == (0, 8, 64)
+    torch.cuda.synchronize()
+    with pytest.raises(AssertionError):      # what is refused stays so
+        ops.attn_decode(q, kc, kc, pos, splits=65)
