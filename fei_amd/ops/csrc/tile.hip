@@ -364,8 +364,8 @@ void by_size(int rows, int width, const TileArgs& g, hipStream_t stream) {
 
 extern "C" {
 
-// Rows of x (xs apart) and w on 16 bytes, K % 64 == 0 and at least 64 a part,
-// N % 8 == 0; rows of out (os apart) on 16 bytes, as the bias. A tile has rows x width
+// Rows of x (xs apart) and w on 16 bytes and less than 2^24 values apart, K % 64 == 0
+// and at least 64 a part, N % 8 == 0; rows of out (os apart) on 16 bytes, as the bias. A tile has rows x width
 // rows of x and w: 256 x 256, 192 or 128, 192 x 256, 128 x 256. epi: see above; parts
 // are 1 but for TILE_PARTS.
 void fei_tile(void* out, long os, const void* x, long xs, const void* w,

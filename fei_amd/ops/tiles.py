@@ -17,6 +17,7 @@ _vp, _i, _l = ctypes.c_void_p, ctypes.c_int, ctypes.c_long
 TILE_BF16, TILE_SWIGLU, TILE_GELU, TILE_RELU2, TILE_PARTS = range(5)
 
 CUS = 256
+FAR = 1 << 24        # rows this far apart: what 128 of them span takes more than 32 bits
 # Rows of x and w a tile, and us of a step of 64 of K: with one tile on the chip, and
 # what comes on top with one on every CU, when the card lowers its clock.
 TILES = ((256, 256, 1.0, 0.46), (256, 192, 0.875, 0.36), (192, 256, 0.82, 0.34),
@@ -44,13 +45,20 @@ def _memory(*tensors: torch.Tensor) -> bool:
             and not torch.compiler.is_compiling())
 
 
+def _near(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether 16 bytes at a time and 32-bit offsets from a tile's first row reach
+    the rows of both."""
+    return (x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+            and x.stride(-1) == 1 and x.stride(-2) % 8 == 0
+            and x.stride(-2) < FAR and w.shape[-1] < FAR)
+
+
 def tile_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether M rows x times w run here; x's rows may lie apart."""
     K = w.shape[-1]
     return (M > 128 and w.is_cuda and w.dim() == 2 and K > 0 and K % 64 == 0
             and w.shape[0] > 0 and w.shape[0] % 8 == 0 and _memory(x, w)
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
-            and x.stride(-1) == 1 and x.stride(-2) % 8 == 0)
+            and _near(x, w))
 
 
 def _time(M: int, cols: int, K: int, parts: int, rows: int, width: int,

@@ -33,6 +33,36 @@ def test_what_tiles_take():
     assert tiles.size_for(16384, 768, 768) == (256, 192)
 
 
+def test_how_far_apart_rows_may_lie():
+    """A lane's offset in bytes from a tile's first row has 32 bits, for up to 127 rows
+    and 128 bytes."""
+    w = torch.empty(64, 64, device="meta")
+    for far in (64, 72, tiles.FAR - 8, tiles.FAR, tiles.FAR + 8, 1 << 26):
+        x = torch.empty_strided((129, 64), (far, 1), device="meta")
+        assert tiles._near(x, w) == (far < tiles.FAR)
+        assert not tiles._near(x, w) or 127 * far * 2 + 128 < 1 << 32
+    wide = torch.empty(8, tiles.FAR, device="meta")
+    assert not tiles._near(wide[:129], wide)
+
+
+@pytest.mark.gpu
+def test_rows_far_apart():
+    """Rows as far apart as tiles take them and further, which are the library's."""
+    M, N, K = 257, 1024, 8192
+    w = rand(N, K, seed=2, scale=K ** -0.5)
+    near, res = rand(M, K, seed=1), rand(M, N, seed=3).float()
+    y = near.double() @ w.double().t()
+    for far in (tiles.FAR - 8, tiles.FAR):
+        x = torch.empty_strided((M, K), (far, 1), device=DEV,
+                                dtype=torch.bfloat16).copy_(near)
+        assert tiles.tile_ok(M, x, w) == (far < tiles.FAR)
+        # float32 sums of K products and one addition; a result rounded once
+        assert err(mx.residual_linear(res.clone(), x, w),
+                   res.double() + y) < 2 ** -24 * K ** 0.5
+        assert err(mx.mix_in(x, None, w, N, 0, x), y) < 2 ** -9
+        del x
+
+
 # one step of K, an odd and an even number of them; one row and one 8 columns past a
 # tile, and short of it; more tiles than CUs, with few steps each
 @pytest.mark.gpu
