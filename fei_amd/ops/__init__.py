@@ -657,7 +657,7 @@ def _many_rows(M: int, x: torch.Tensor, wgu: torch.Tensor) -> Optional[str]:
     if _rows.swiglu_ok(M, x, wgu):
         return "rows"
     # a copy of rows with gaps is aligned
-    if (wgu.shape[0] % 16 == 0
+    if (wgu.shape[0] % 16 == 0 and _tiles.types_ok(x)
             and _tiles.tile_ok(M, x if x.is_contiguous() else wgu, wgu)):
         return "tile"
     return None
@@ -879,6 +879,7 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
         return out
     if (act_gelu and x.is_cuda and _mixers.plain(x, w)
             and _tiles.tile_ok(M, x, w)
+            and _tiles.types_ok(bias)
             and _mixers.dense(bias, torch.bfloat16, x, w.shape[0])
             and bias.data_ptr() % 16 == 0):
         out = torch.empty(*x.shape[:-1], w.shape[0], dtype=x.dtype,

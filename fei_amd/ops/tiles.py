@@ -8,6 +8,7 @@ from functools import lru_cache
 from typing import Optional, Tuple
 
 import torch
+from torch.utils._device import DeviceContext
 
 import fei_amd.ops as _ops     # half made yet: it imports this
 
@@ -32,15 +33,25 @@ def _p(t: Optional[torch.Tensor]):
     return None if t is None else t.data_ptr()
 
 
+def types_ok(*tensors: torch.Tensor) -> bool:
+    """Whether the tensors are of no class that does more than torch's own."""
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+
+
 def _memory(*tensors: torch.Tensor) -> bool:
     """Whether the tensors are what lies at their pointers, and nothing follows what
-    is done to them: tracing, transforms, tangents and dispatch modes are for the
-    library's operations."""
-    c = torch._C                 # 2 us
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
+    is done to them: tracing, transforms, tangents, modes and casts to another type are
+    for the library's operations."""
+    c = torch._C                 # 2.5 us
+    return (types_ok(*tensors)
             and c._functorch.peek_interpreter_stack() is None
             and torch.autograd.forward_ad._current_level < 0
             and not c._len_torch_dispatch_stack()
+            # that of a default device changes nothing here
+            and all(type(c._get_function_stack_at(i)) is DeviceContext
+                    for i in range(c._len_torch_function_stack()))
+            and (not torch.is_autocast_enabled("cuda")
+                 or torch.get_autocast_dtype("cuda") is torch.bfloat16)
             and c._get_tracing_state() is None
             and not torch.compiler.is_compiling())
 
@@ -136,7 +147,8 @@ def add_ok(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
     (150); 2048 x 14336 of 1706 97 (124); 4096 x 10240 of 1900 143 (147); 4096 x
     25600 of 1030 207 (319). 2048 x 4096 of 1301 40 (32): there the pass costs more
     than the parts gain."""
-    return (parts_ok(a.shape[0], a, w) and x.data_ptr() % 16 == 0
+    return (parts_ok(a.shape[0], a, w) and types_ok(x)
+            and x.data_ptr() % 16 == 0
             and not (x.requires_grad and torch.is_grad_enabled()))
 
 

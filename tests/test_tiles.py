@@ -192,6 +192,19 @@ def test_residual_and_its_norms(M, N, K, pair):
         else normed[1] is None
 
 
+class Recorder(torch.overrides.TorchFunctionMode):
+    def __init__(self):
+        self.seen = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen.append(func)
+        return func(*args, **(kwargs or {}))
+
+
+class Tagged(torch.Tensor):
+    """A class of its own, as users make them."""
+
+
 def test_tensors_that_are_more_than_memory():
     """Tiles leave them to the library; no GPU is needed to say which they are."""
     x = rand(4, 8, dev="cpu")
@@ -205,7 +218,30 @@ def test_tensors_that_are_more_than_memory():
         seen.append(tiles._memory(x))
     torch.jit.trace(lambda t: (seen.append(tiles._memory(t)), t + 1)[1], x,
                     check_trace=False)
-    assert len(seen) >= 4 and not any(seen)
+    with Recorder():
+        seen.append(tiles._memory(x))
+    seen.append(tiles._memory(x, x.as_subclass(Tagged)))
+    for dtype in (torch.float16, torch.bfloat16):
+        before = torch.get_autocast_dtype("cuda")
+        torch.set_autocast_enabled("cuda", True)
+        torch.set_autocast_dtype("cuda", dtype)
+        try:             # bfloat16 stays as it is
+            seen.append(tiles._memory(x) != (dtype is torch.bfloat16))
+        finally:
+            torch.set_autocast_enabled("cuda", False)
+            torch.set_autocast_dtype("cuda", before)
+    assert len(seen) >= 8 and not any(seen)
+    with torch.device("cpu"):                # a default for new tensors
+        assert tiles._memory(x)
+    # rows with gaps, of which a copy goes to the kernel
+    wide = rand(300, 256, dev="cpu").as_subclass(Tagged)[:, :128]
+    ok, tiles.tile_ok = tiles.tile_ok, lambda M, a, b: tiles._memory(a, b)
+    try:
+        w = rand(64, 128, dev="cpu")
+        assert ops._many_rows(300, torch.Tensor(wide.float())[:, :128], w)
+        assert ops._many_rows(300, wide, w) is None
+    finally:
+        tiles.tile_ok = ok
 
 
 @pytest.mark.gpu
@@ -220,3 +256,11 @@ def test_many_rows_under_transforms():
     assert err(dy, v.double() @ w.double().t()) < 2 ** -9
     both = torch.func.vmap(lambda t: ops.linear_decode(t, w))(torch.stack([x, v]))
     assert err(both[1], v.double() @ w.double().t()) < 2 ** -9
+    # what follows torch's operations sees one, and a cast is made
+    with Recorder() as mode:
+        ops.linear_decode(x, w)
+    assert F.linear in mode.seen
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert ops.linear_decode(x, w).dtype == torch.float16
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(ops.linear_decode(x, w), tiles.linear(x, w))
