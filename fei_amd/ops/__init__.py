@@ -652,12 +652,15 @@ def linear_decode(x: torch.Tensor, w: torch.Tensor,
     return out
 
 
-def _many_rows(M: int, x: torch.Tensor, wgu: torch.Tensor) -> Optional[str]:
-    """The kernel of more than a few rows that makes a SwiGLU, if one does."""
+def _many_rows(M: int, x: torch.Tensor, wgu: torch.Tensor,
+               out: Optional[torch.Tensor] = None) -> Optional[str]:
+    """The kernel of more than a few rows that makes a SwiGLU, if one does. Tiles
+    write 16 bytes at a time."""
     if _rows.swiglu_ok(M, x, wgu):
         return "rows"
     # a copy of rows with gaps is aligned
     if (wgu.shape[0] % 16 == 0 and _tiles.types_ok(x)
+            and (out is None or out.data_ptr() % 16 == 0)
             and _tiles.tile_ok(M, x if x.is_contiguous() else wgu, wgu)):
         return "tile"
     return None
@@ -671,7 +674,7 @@ def gemv_swiglu(x: torch.Tensor, wgu: torch.Tensor,
     how = _product(x, wgu, M, K, I, out)
     if (how is None and M and x.is_cuda and _mixers.match(x, wgu, K)
             and _fits(out, x, M * I)):
-        how = _many_rows(M, x, wgu)
+        how = _many_rows(M, x, wgu, out)
     if how is None:
         return swiglu(torch.nn.functional.linear(x, wgu))
     x2 = x.contiguous().view(M, K)

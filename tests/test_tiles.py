@@ -119,6 +119,20 @@ def test_swiglu_of_many_rows(M, I, K):
 
 
 @pytest.mark.gpu
+def test_swiglu_of_many_rows_to_a_place_between():
+    """Results that start on any 2 bytes: nothing is written beside them."""
+    M, I, K = 300, 64, 128
+    x, w = rand(M, K, seed=1), rand(2 * I, K, seed=2, scale=K ** -0.5)
+    y = x.double() @ w.double().t()
+    for at in (0, 1, 4, 8):
+        room = torch.full((M * I + 16,), 7.0, device=DEV, dtype=torch.bfloat16)
+        got = ops.gemv_swiglu(x, w, room[at:at + M * I].view(M, I))
+        # rounded once, in the library and its pass twice before
+        assert err(got, F.silu(y[:, :I]) * y[:, I:]) < 2 ** -8
+        assert bool((room[:at] == 7).all() and (room[at + M * I:] == 7).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(257, 256, 8192), (600, 2048, 8256),
                                    (1500, 1024, 10240)])
 def test_parts_and_their_norm(M, N, K):
@@ -240,6 +254,10 @@ def test_tensors_that_are_more_than_memory():
         w = rand(64, 128, dev="cpu")
         assert ops._many_rows(300, torch.Tensor(wide.float())[:, :128], w)
         assert ops._many_rows(300, wide, w) is None
+        x, room = rand(300, 128, dev="cpu"), rand(300 * 32 + 8, dev="cpu")
+        for at in range(9):              # results on 16 bytes
+            out = room[at:at + 300 * 32]
+            assert bool(ops._many_rows(300, x, w, out)) == (at % 8 == 0)
     finally:
         tiles.tile_ok = ok
 
