@@ -661,7 +661,7 @@ def _many_rows(M: int, x: torch.Tensor, wgu: torch.Tensor,
     # a copy of rows with gaps is aligned
     if (wgu.shape[0] % 16 == 0 and _tiles.types_ok(x)
             and (out is None or out.data_ptr() % 16 == 0)
-            and _tiles.tile_ok(M, x if x.is_contiguous() else wgu, wgu)):
+            and _tiles.act_ok(M, x if x.is_contiguous() else wgu, wgu)):
         return "tile"
     return None
 
@@ -881,7 +881,7 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
                        bias16=bias)
         return out
     if (act_gelu and x.is_cuda and _mixers.plain(x, w)
-            and _tiles.tile_ok(M, x, w)
+            and _tiles.act_ok(M, x, w)
             and _tiles.types_ok(bias)
             and _mixers.dense(bias, torch.bfloat16, x, w.shape[0])
             and bias.data_ptr() % 16 == 0):

@@ -244,7 +244,7 @@ def _act_tile(x: torch.Tensor, w: torch.Tensor, ff: int,
     """Whether the product of many rows writes its activations, ``ff`` a row, to
     ``act`` itself."""
     return (x.shape[0] > 128 and ff % 8 == 0 and plain(x, w)
-            and _tiles.tile_ok(x.shape[0], x, w)
+            and _tiles.act_ok(x.shape[0], x, w)
             and act.dtype is _BF16 and act.stride(1) == 1
             and act.stride(0) % 8 == 0 and act.data_ptr() % 16 == 0)
 

@@ -90,6 +90,13 @@ def size_for(M: int, cols: int, K: int) -> Tuple[int, int]:
     return min(TILES, key=lambda t: _time(M, cols, K, 1, *t))[:2]
 
 
+@lru_cache(maxsize=1024)
+def _rate(M: int, cols: int, K: int) -> float:
+    """About how many PFLOP/s the tiles of a product reach: few where there are few, or
+    where a last round has few."""
+    return 2e-9 * M * cols * K / min(_time(M, cols, K, 1, *t) for t in TILES)
+
+
 def linear_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether x [M, K] @ w^T is faster here than in the library: where K is 1024 to
     2048 and the tiles fill the CUs to 0.86 PFLOP/s. Against the library, us: 3072 x 2048 of 6006 rows 69 (82), of 4000 41
@@ -98,11 +105,21 @@ def linear_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     that the rule takes 6144 x 2048 of 2600 64 (62). Of 4096 x 4096 and 6144 x 4096 neither
     is better by more than 5 % up to 6006 rows."""
     N, K = w.shape
-    if (M <= 256 or not 1024 <= K <= 2048 or not tile_ok(M, x, w)
-            or not _ops._mixers.match(x, w, x.shape[-1])):
-        return False
-    size = next(t for t in TILES if t[:2] == size_for(M, N, K))
-    return 2 * M * N * K > 0.86e9 * _time(M, N, K, 1, *size)
+    return (M > 256 and 1024 <= K <= 2048 and tile_ok(M, x, w)
+            and _ops._mixers.match(x, w, x.shape[-1]) and _rate(M, N, K) > 0.86)
+
+
+def act_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the product of all of w's rows with an activation inside is faster here
+    than in the library with a pass for it. Over 43 sizes of 8 to 28672 results and K of
+    64 to 14336, 129 to 8192 rows, nowhere by more than 5 % slower from 0.7 PFLOP/s on, and
+    past K = 8192, which the library cuts, from 0.86. Without a rule, us: GELU of 256 x
+    4096, 300 rows 56 (14), 1024 x 1024, 1000 rows 23 (15); SwiGLU of 2 x 1024 x 2048, 1000
+    rows 29 (21); relu^2 of 6144 x 4096, 512 rows 55 (42). What the rule leaves out that
+    would gain most: SwiGLU of 2 x 2048 x 512, 1301 rows 13 (22)."""
+    N, K = w.shape
+    return (tile_ok(M, x, w)
+            and _rate(M, N, K) > (0.7 if K <= 8192 else 0.86))
 
 
 def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, N: int,

@@ -33,6 +33,17 @@ def test_what_tiles_take():
     assert tiles.size_for(16384, 768, 768) == (256, 192)
 
 
+def test_when_activations_go_into_tiles():
+    """Where those fill the CUs: not of few rows and results, whatever K."""
+    for M, N, K in ((129, 8, 64), (300, 256, 4096), (1000, 1024, 1024), (8192, 64, 256),
+                    (1000, 2048, 2048), (512, 6144, 4096), (700, 512, 8192),
+                    (2048, 2048, 8192), (1301, 4096, 14336), (129, 28672, 4096)):
+        assert tiles._rate(M, N, K) < (0.7 if K <= 8192 else 0.86)
+    for M, N, K in ((16384, 3072, 768), (2048, 28672, 4096), (6006, 16384, 2048),
+                    (1301, 12288, 2048), (1000, 6144, 4096), (4096, 4096, 14336)):
+        assert tiles._rate(M, N, K) > (0.7 if K <= 8192 else 0.86)
+
+
 def test_how_far_apart_rows_may_lie():
     """A lane's offset in bytes from a tile's first row has 32 bits, for up to 127 rows
     and 128 bytes."""
@@ -119,10 +130,31 @@ def test_swiglu_of_many_rows(M, I, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,I,K", [(2600, 2056, 1088), (2049, 2048, 512),
+                                   (2600, 2056, 1080)])
+def test_activations_of_many_rows(M, I, K):
+    """Through the public ops, where tiles take them; the last is the library's."""
+    x, w = rand(M, K, seed=1), rand(2 * I, K, seed=2, scale=K ** -0.5)
+    b = rand(2 * I, seed=3)
+    assert (ops._many_rows(M, x, w) == "tile") == (K % 64 == 0)
+    y = x.double() @ w.double().t()
+    # rounded once, in the library and its pass twice before
+    assert err(ops.gemv_swiglu(x, w), F.silu(y[:, :I]) * y[:, I:]) < 2 ** -8
+    assert err(ops.linear_bias(x.view(1, M, K), w, b, True)[0],
+               F.gelu(y + b.double())) < 2 ** -8
+    out = torch.full((M, 3 * I), 7.0, device=DEV, dtype=torch.bfloat16)
+    h = mx.GainNormed(x.float(), None, torch.bfloat16, x)
+    mx.parallel_in(h, w, 0, 2 * I, 0, out[:, I:])
+    assert err(out[:, I:], y.clamp_min(0) ** 2) < 2 ** -8
+    assert bool((out[:, :I] == 7).all())
+
+
+@pytest.mark.gpu
 def test_swiglu_of_many_rows_to_a_place_between():
     """Results that start on any 2 bytes: nothing is written beside them."""
-    M, I, K = 300, 64, 128
+    M, I, K = 2048, 2048, 512
     x, w = rand(M, K, seed=1), rand(2 * I, K, seed=2, scale=K ** -0.5)
+    assert ops._many_rows(M, x, w) == "tile"
     y = x.double() @ w.double().t()
     for at in (0, 1, 4, 8):
         room = torch.full((M * I + 16,), 7.0, device=DEV, dtype=torch.bfloat16)
@@ -249,7 +281,7 @@ def test_tensors_that_are_more_than_memory():
         assert tiles._memory(x)
     # rows with gaps, of which a copy goes to the kernel
     wide = rand(300, 256, dev="cpu").as_subclass(Tagged)[:, :128]
-    ok, tiles.tile_ok = tiles.tile_ok, lambda M, a, b: tiles._memory(a, b)
+    ok, tiles.act_ok = tiles.act_ok, lambda M, a, b: tiles._memory(a, b)
     try:
         w = rand(64, 128, dev="cpu")
         assert ops._many_rows(300, torch.Tensor(wide.float())[:, :128], w)
@@ -259,7 +291,7 @@ def test_tensors_that_are_more_than_memory():
             out = room[at:at + 300 * 32]
             assert bool(ops._many_rows(300, x, w, out)) == (at % 8 == 0)
     finally:
-        tiles.tile_ok = ok
+        tiles.act_ok = ok
 
 
 @pytest.mark.gpu
