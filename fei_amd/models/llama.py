@@ -477,7 +477,8 @@ class LlamaModel:
             act = ops.gemv_swiglu(x, lw.wgu)
             T, norm = act.numel() // act.shape[-1], self._norm_after(li)
             act = act.view(T, -1)
-            if self.tp_size == 1 and ops.tile_parts_ok(T, act, lw.wdown):
+            if (self.tp_size == 1 and ops.tile_parts_pay(T, lw.wdown)
+                    and ops.tile_parts_ok(T, act, lw.wdown)):
                 x = ops.add_norm_parts(ops.tile_parts(act, lw.wdown),
                                        h.view(T, -1), norm,
                                        s.norm_eps).view_as(h)

@@ -367,7 +367,7 @@ def residual_linear(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
     if own and _rows.add_ok(x, a, w):
         _rows.add_product(x, a, w, mult)
         return x
-    if own and _tiles.add_ok(x, a, w):
+    if own and _tiles.parts_pay(T, w) and _tiles.add_ok(x, a, w):
         _rows.add_parts(x, _tiles.product_parts(a, w), mult)
         return x
     return torch.addmm(x, a, w.t(), out_dtype=torch.float32, alpha=mult,
@@ -396,8 +396,8 @@ def residual_norms(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor,
             and _gain(w1, C, a) and (w2 is None or _gain(w2, C, a))
             and dense(x, torch.float32, a, T, C)):
         parts = (_rows.product_parts(a, w) if _rows.add_ok(x, a, w)
-                 else _tiles.product_parts(a, w) if _tiles.add_ok(x, a, w)
-                 else None)
+                 else _tiles.product_parts(a, w)
+                 if _tiles.parts_pay(T, w) and _tiles.add_ok(x, a, w) else None)
         if parts is not None:
             return x, _rows.add_parts_norms(x, parts, mult, w1, w2, eps)
     return residual_linear(x, a, w, mult), None

@@ -112,7 +112,7 @@ def linear_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
 def act_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the product of all of w's rows with an activation inside is faster here
     than in the library with a pass for it. Over 43 sizes of 8 to 28672 results and K of
-    64 to 14336, 129 to 8192 rows, nowhere by more than 5 % slower from 0.7 PFLOP/s on, and
+    64 to 14336, 129 to 8192 rows, nowhere by more than 6 % slower from 0.7 PFLOP/s on, and
     past K = 8192, which the library cuts, from 0.86. Without a rule, us: GELU of 256 x
     4096, 300 rows 56 (14), 1024 x 1024, 1000 rows 23 (15); SwiGLU of 2 x 1024 x 2048, 1000
     rows 29 (21); relu^2 of 6144 x 4096, 512 rows 55 (42). What the rule leaves out that
@@ -146,8 +146,9 @@ def _launch(out, x, w, N, epi, size, bias=None, parts=1) -> None:
 
 
 def parts_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether x @ w^T is faster in parts of K that the norm after it sums: a long
-    K, and results for less than half of the CUs' tiles. With the norm, against the
+    """Whether x @ w^T may run in parts of K that the norm after it sums: a long
+    K, and results for less than half of the CUs' tiles, so that it is faster if there
+    are not too few (parts_pay). With the norm, against the
     library's product and a norm: 4096 x 14336 of 512 rows 66 us (95), 1000 106
     (138), 2048 187 (212); 2048 x 8192 of 512 32 (35), 2048 72 (79), 4000 117 (121);
     of 6006 172 (166). 4096 x 4096 is a draw."""
@@ -155,6 +156,17 @@ def parts_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     return (K >= 8192 and M > 256 and tile_ok(M, x, w)
             and _ops._mixers.match(x, w, x.shape[-1])
             and 2 * -(-M // 256) * -(-N // 256) <= CUS)
+
+
+def parts_pay(M: int, w: torch.Tensor) -> bool:
+    """Whether products with w that parts_ok takes have the tiles for it: of few results
+    a row eight parts leave most CUs without, and the library cuts K further; and of
+    just half of the CUs' tiles, up to K = 10240, it is as good. With float32 results
+    added, K = 8192, 257 rows, us: 8 results 19 (12), 256 23 (16), 512 25 (23), 768 26
+    (23), 1000 26 (29), 1024 25 (27); 1024 of 8192 rows 126 (115)."""
+    N, K = w.shape
+    return N >= 1000 and (K >= 10240
+                          or 2 * -(-M // 256) * -(-N // 256) < CUS)
 
 
 def add_ok(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:

@@ -44,6 +44,15 @@ def test_when_activations_go_into_tiles():
         assert tiles._rate(M, N, K) > (0.7 if K <= 8192 else 0.86)
 
 
+def test_when_parts_of_k_pay():
+    for M, N, K, pays in ((257, 992, 8192, False), (257, 1000, 8192, True),
+                          (300, 4096, 14336, True), (8192, 1024, 8192, False),
+                          (8192, 1024, 10240, True), (8191, 960, 14336, False),
+                          (4096, 2048, 8192, False), (4096, 1792, 8192, True)):
+        w = torch.empty(N, K, device="meta")
+        assert tiles.parts_pay(M, w) == pays
+
+
 def test_how_far_apart_rows_may_lie():
     """A lane's offset in bytes from a tile's first row has 32 bits, for up to 127 rows
     and 128 bytes."""
@@ -193,6 +202,23 @@ def test_residual_of_many_rows(M, N, K):
         want = res.double() + 0.5 * (a.double() @ w.double().t())
         # float32 sums of K products and one addition
         assert err(mx.residual_linear(res, a, w, 0.5), want) < 2 ** -24 * K ** 0.5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(257, 8, 8192), (300, 992, 8192),
+                                   (300, 1000, 8192)])
+def test_parts_of_few_results_stay_in_the_library(M, N, K, monkeypatch):
+    a, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
+    x, g = rand(M, N, seed=3).float(), rand(N, seed=4).float()
+    want = x.double() + a.double() @ w.double().t()
+    calls, parts = [], tiles.product_parts
+    monkeypatch.setattr(tiles, "product_parts",
+                        lambda *t: (calls.append(1), parts(*t))[1])
+    # float32 sums of K products and one addition
+    assert err(mx.residual_linear(x.clone(), a, w), want) < 2 ** -24 * K ** 0.5
+    y, normed = mx.residual_norms(x, a, w, g, None, 1e-3, torch.bfloat16)
+    assert err(y, want) < 2 ** -24 * K ** 0.5
+    assert len(calls) == 2 * (N >= 1000) and (normed is None) == (N < 1000)
 
 
 @pytest.mark.gpu
