@@ -97,16 +97,31 @@ def _rate(M: int, cols: int, K: int) -> float:
     return 2e-9 * M * cols * K / min(_time(M, cols, K, 1, *t) for t in TILES)
 
 
+@lru_cache(maxsize=1024)
+def _plain_pays(M: int, N: int, K: int) -> bool:
+    """Whether a product with nothing behind it is faster in tiles than in the library,
+    which whole rounds of 256 x 256 suit best, and three quarters of one of whole tiles:
+    3 to 14 % faster there (8192 x 2048, 4096 rows 98 us, 103 here; 6144 x 1024, 2048
+    rows 29, 31). Else from 0.88 PFLOP/s on (1.02 of more than a round where
+    K < 2048: 6144 x 1536, 3000 rows 64 us, 60 in the library). Of 657 sizes, M of 300 to
+    16384 and N of 768 to 16384, it takes 341, 222 of which gain 3 to 32 % (5000 x 1024,
+    2600 rows 30 us for 43; 8192 x 2048, 2600 rows 76 for 97; 3072 x 2048, 6006 rows 76 for
+    82), and at worst loses 6 (2560 x 1280, 6006 rows 37 for 35)."""
+    tiles = -(-M // 256) * -(-N // 256)
+    rounds = -(-tiles // CUS)
+    if N % 256 == 0 and (tiles == rounds * CUS or
+                         M % 256 == 0 and 4 * tiles >= 3 * rounds * CUS):
+        return False
+    return _rate(M, N, K) > (1.02 if K < 2048 and rounds > 1 else 0.88)
+
+
 def linear_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether x [M, K] @ w^T is faster here than in the library: where K is 1024 to
-    2048 and the tiles fill the CUs to 0.86 PFLOP/s. Against the library, us: 3072 x 2048 of 6006 rows 69 (82), of 4000 41
-    (43), of 3000 36 (36), of 2048 29 (27); 5000 x 2048 of 1301 31 (34), of 2600 48 (62);
-    3648 x 2048 of 1706 30 (33); 6144 x 2048 of 1301 35 (43), of 1030 32 (31); the worst
-    that the rule takes 6144 x 2048 of 2600 64 (62). Of 4096 x 4096 and 6144 x 4096 neither
-    is better by more than 5 % up to 6006 rows."""
+    """Whether x [M, K] @ w^T is faster here than in the library: of K 1024 to 2048
+    (of 4096 x 4096 and 6144 x 4096 neither is better by more than 5 % up to 6006
+    rows)."""
     N, K = w.shape
     return (M > 256 and 1024 <= K <= 2048 and tile_ok(M, x, w)
-            and _ops._mixers.match(x, w, x.shape[-1]) and _rate(M, N, K) > 0.86)
+            and _ops._mixers.match(x, w, x.shape[-1]) and _plain_pays(M, N, K))
 
 
 def act_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:

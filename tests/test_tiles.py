@@ -44,6 +44,16 @@ def test_when_activations_go_into_tiles():
         assert tiles._rate(M, N, K) > (0.7 if K <= 8192 else 0.86)
 
 
+def test_when_plain_products_pay():
+    """Not where the library's own tiles fill the CUs."""
+    for M, N, K, pays in ((8192, 16384, 1280, False), (4000, 8192, 2048, False),
+                          (2048, 6144, 1024, False), (2048, 3072, 2048, False),
+                          (3000, 6144, 1536, False), (300, 512, 2048, False),
+                          (6006, 3072, 2048, True), (2600, 5000, 1024, True),
+                          (1301, 5704, 2048, True), (4096, 2560, 1024, True)):
+        assert tiles._plain_pays(M, N, K) == pays
+
+
 def test_when_parts_of_k_pay():
     for M, N, K, pays in ((257, 992, 8192, False), (257, 1000, 8192, True),
                           (300, 4096, 14336, True), (8192, 1024, 8192, False),
