@@ -128,6 +128,41 @@ def test_tile(M, N, K, size):
 
 
 @pytest.mark.gpu
+def test_activations_of_every_value():
+    """All of bfloat16, and infinities and NaN that sums come to (as no factor, which
+    would meet zeros): the bits of the library's product and the pass behind it, which
+    divides."""
+    every = torch.arange(1 << 16, dtype=torch.int32, device=DEV).to(torch.int16)
+    every = every.view(torch.bfloat16)
+    every = every[every.isfinite()]
+    big = every.abs().max()
+    M, K, N = len(every) + 4, 64, 16
+    x = torch.zeros(M, K, device=DEV, dtype=torch.bfloat16)
+    x[:-4, 0], x[:, 2] = every, 1.0
+    x[-4, 0], x[-3, 0], x[-2, :2], x[-1, :2] = big, -big, big, -big
+    w = torch.zeros(2 * N, K, device=DEV, dtype=torch.bfloat16)
+    w[:N, 0] = 1.0
+    w[8:N, 0], w[8:N, 1] = 2.0, -2.0         # infinities, and their difference
+    w[N:, 2] = torch.tensor([1, -1, 0.5, 3, 1e30, 1e-30, 2.0 ** 100, 0] * 2)
+    y = F.linear(x, w)
+    assert y[-4, 8].isinf() and y[-2, 8].isnan() and y[-2, N:].isfinite().all()
+    none = torch.zeros(N, device=DEV, dtype=torch.bfloat16)
+    for epi, ww, want in (
+            (tiles.TILE_BF16, w[:N], y[:, :N]),
+            (tiles.TILE_SWIGLU, w, ops.swiglu(y)),
+            (tiles.TILE_GELU, w[:N], ops.gelu(y[:, :N].contiguous())),
+            (tiles.TILE_RELU2, w[:N], mx.ref.square_relu(y[:, :N]).bfloat16())):
+        out = torch.empty(M, N, device=DEV, dtype=torch.bfloat16)
+        tiles._launch(out, x, ww, N, epi, (256, 256), none)
+        if epi == tiles.TILE_RELU2:          # a NaN is not above 0
+            want = want.where(~y[:, :N].isnan(), torch.zeros_like(want))
+        assert torch.equal(out.isnan(), want.isnan())
+        ok = ~want.isnan()
+        differ = out[ok] != want[ok]
+        assert not differ.any(), (epi, out[ok][differ][:8], want[ok][differ][:8])
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,I,K", [(129, 64, 128), (300, 100, 192),
                                    (700, 1024, 256), (300, 64, 72)])
 def test_swiglu_of_many_rows(M, I, K):
