@@ -429,11 +429,14 @@ void launch_waves(const DecodeAttn& a, dim3 grid, hipStream_t stream) {
 // are: then nothing is left to combine. Split and combined, or whole, us in a graph:
 // 1 sequence of 256 keys and 8 heads of 64 6.7, 6.2; of 320 6.6, 6.8; 8 of 576 9.0,
 // 8.0, of 1024 9.7, 11.0; 20 of 600 in pages 12.7, 9.5; 32 of 2048 34.0, 29.3. Heads
-// of 128, 8 sequences of 320 9.2, 8.8, of 448 9.5, 10.1; 12 of 512 12.4, 12.5; 24 of
-// 2048 46.7, 41.9. Beyond 2048 one long sequence among short ones would be alone on
-// its CUs.
+// of 128, 8 sequences of 320 9.2, 8.8, of 448 9.5, 10.1; 12 of 512 12.4, 12.5; 20 of
+// 1024 21.8, 19.7, of half that 17.0, 11.8. One long sequence among short ones is alone
+// on its CUs: 20 of 60 keys, but one of 512 9.5, 9.5, of 640 9.3, 10.6, of 1024 13.3,
+// 14.3, of 2048 17.4, 23.6, so that beyond 1024 keys are split. For the same reason
+// there are as many splits as were asked for, however many sequences: with no more
+// blocks than places, 64 of which one had 8192 keys took 80 us for 41.
 inline int whole_keys(int heads, int D) {
-  if (heads >= 160) return 2048;
+  if (heads >= 160) return 1024;
   if (heads < 64) return 256;
   return D == 64 ? 768 : heads < 96 ? 320 : 512;
 }
@@ -448,11 +451,6 @@ void launch_decode(DecodeAttn a, int B, hipStream_t stream) {
   // last: a block waits for the position to know that it has no keys, and keeps
   // its place meanwhile. 20 sequences of up to 600 keys in pages, 16 splits
   // asked for: 15.9 -> 7.8 us.
-  // Nor more blocks than the chip has places (three on a CU, four of heads of 64), or
-  // the last would begin when others end: 16 sequences of up to 900 keys, 8 heads of
-  // 128, 6 splits 15.3 us, 16 18.5; 8 of 3000 12 24.6, 16 27.5; 12 of 2047, the worst
-  // of it, 8 26.7, 16 25.9.
-  a.splits = max(1, min(a.splits, (D == 64 ? 1024 : 768) / (a.Hkv * B)));
   const int all = max(1, min(a.splits, (a.max_seq + CHUNK * SHARE - 1) /
                                            (CHUNK * SHARE)));
   const int side = min(all, 16);

@@ -259,6 +259,8 @@ def test_attn_decode_without_keys(lib, paged, T, splits):
     (12, 4, [31, 33, 63, 257, 288] * 4),         # 64 heads and more
     (8, 8, [700, 511, 513, 1, 97, 300, 400, 512]),
     (8, 8, list(range(960, 1160, 10))),          # 160 heads: several rounds
+    (8, 8, [60] * 19 + [1019]),      # one long one among short ones, the most in one
+    (8, 8, [1020] + [60] * 20),      # block and the fewest in several
 ])
 def test_attn_decode_in_one_block(lib, D, paged, rope, Hq, Hkv, lens):
     """Where a block takes all keys of a head."""
