@@ -329,7 +329,7 @@ def attn_prefill(q, k_cache, v_cache, pos0, scale: Optional[float] = None,
     if not q.numel():
         return out
     k_cache, v_cache = _cache_rows(k_cache, v_cache)
-    splits = _prefill_splits(B * Hkv, S * (Hq // Hkv), k_cache.shape[2])
+    splits = _prefill_splits(B, Hkv, S * (Hq // Hkv), k_cache.shape[2])
     po = pml = None
     if splits > 1:
         ws = torch.empty(B * S * Hq * splits * (D + 2), dtype=torch.float32,
@@ -355,17 +355,16 @@ def _cache_rows(k: torch.Tensor, v: torch.Tensor):
     return (t.clone(memory_format=torch.contiguous_format) for t in (k, v))
 
 
-def _prefill_splits(heads: int, rows: int, max_seq: int) -> int:
+def _prefill_splits(B: int, Hkv: int, rows: int, max_seq: int) -> int:
     """Shares of the keys that the prompt attention's blocks of 128 rows are
     cut into, so that few rows over many keys fill the chip's 512 places (two
     blocks per CU). How many keys there are is known on the device only; the
     kernel uses fewer shares where one would have under three tiles of 64, and
-    one where there are few keys in all (of ``max_seq`` the same is asked here).
-    Between the products of a model 250 rows of 32 heads of 128 over 2050 keys
-    take 130 us less a call in 8 shares than in 4; over warm keys the fewer
-    are as fast."""
-    blocks = heads * -(-rows // 128)
-    if blocks > 192 or max_seq <= 64 * (9 + blocks // 6):
+    one where there are few keys in all. Of ``max_seq`` that is asked here, for
+    half of the ``B`` and one more as if they were long; a launch without shares
+    saves 3 us and more."""
+    blocks = B * Hkv * -(-rows // 128)
+    if blocks > 192 or max_seq <= 64 * 6 + Hkv * rows * (B + 1) // 20:
         return 1
     return max(1, min(16, -(-512 // blocks), max_seq // 192))
 
@@ -926,7 +925,7 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
         return torch.empty(M, n, dtype=h.dtype, device=h.device)
     h1, tmp = rows(C), rows(C)
     qkv, att, mid = rows(3 * HD), rows(HD), rows(inner)
-    splits = _prefill_splits(B * heads, S, S)
+    splits = _prefill_splits(B, heads, S, S)
     po = pml = None
     if splits > 1:
         ws = torch.empty(M * heads * splits * (dim + 2), dtype=torch.float32,

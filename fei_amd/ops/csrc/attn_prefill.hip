@@ -40,13 +40,15 @@ constexpr int MAX_SPLITS = 16;
 constexpr int ROWS = 128;              // rows per block
 constexpr int KEYS = 64;               // keys per tile
 constexpr float M_NONE = -3.0e38f;     // maximum of a row without keys
+constexpr float DONE = -1.f;           // sum of a row that one split finished
 
 struct Prefill {
   const u16 *q, *kc, *vc;
   u16* out;
   float *po, *pml;                     // partial results of splits
   const int *pos0, *kv_len;
-  int S, G, Hkv, heads, tiles, max_seq, causal, splits, alone;
+  int B, S, G, Hkv, heads, tiles, max_seq, causal, splits;
+  int share;                           // keys for the rows of a batch row: cut_keys
   float scale;
   long q_ts;
   long kv_b, kv_h, kv_t;               // strides of the caches
@@ -58,21 +60,29 @@ __device__ __forceinline__ int keys_of(const Prefill& a, int b, int r_hi) {
   return min(n, a.max_seq);
 }
 
-// Keys that a block of rows reads: tiles [t0, t1) of n keys. They are cut into splits
-// of at least three where the last row of the batch row sees more than ``alone`` tiles
-// (asked of one block of rows by itself, those of few keys would have them all and be
-// the last: 500 tokens over 1800 keys 58 us for 39). How many it takes is what the
-// results of splits and the combine cost, which grow with the rows: 9 tiles and one
-// more for six blocks. In one, and in two or three: 33 rows of 32 heads of 128 over
-// 333 keys 11.7 us, 12.2; 150 over 450 13.2, 16.2; 500 over 500 15.1, 22.7, over 800
-// 20.1, 29.2, over 2300 44.3, 41.0.
-__device__ __forceinline__ void split_tiles(const Prefill& a, int b, int n,
-                                            int split, int& t0, int& t1) {
-  const int nt = (n + KEYS - 1) / KEYS;
-  const bool cut = keys_of(a, b, a.S * a.G - 1) > a.alone * KEYS;
-  const int per = cut ? max((nt + a.splits - 1) / a.splits, 3) : nt;
-  t0 = split * per;
-  t1 = min(nt, t0 + per);
+// Whether the keys of a batch row are cut into splits: where its last row sees more than
+// few (asked of one block of rows by itself, those of few keys would have them all and be
+// the last: 500 tokens over 1800 keys 58 us for 39). How many are few is what the results
+// of splits and the combine cost, which grow with the rows that are cut: 3 tiles, and a
+// key for 14 rows of the batch rows that are cut. In one and cut, us, over room for 8192
+// keys, 32 heads of 128, 8 of keys: 150 tokens over 300 keys 19.0, 19.3, over 600 23.9,
+// 21.1; 300 over 600 27.1, 31.1; 500 over 600 31.0, 33.8, over 1000 38.0, 36.1; 4 x 75
+// over 600 24.0, 28.8, over 1800 44.5, 41.7, where three of the four begin 42.5, 33.0.
+constexpr int FEW = 3 * KEYS;
+__device__ __forceinline__ bool cut_keys(const Prefill& a, int b) {
+  const int last = a.S * a.G - 1, n = keys_of(a, b, last);
+  if (n <= FEW + a.share || a.B == 1) return n > FEW + a.share;
+  int cut = 0;                           // batch rows that would be, by themselves
+  for (int i = 0; i < a.B; i += 64) {
+    const int at = i + (threadIdx.x & 63);
+    cut += __popcll(__ballot(at < a.B && keys_of(a, min(at, a.B - 1), last) >
+                                             FEW + a.share));
+  }
+  return n > FEW + cut * a.share;
+}
+// Tiles of a split of n keys.
+__device__ __forceinline__ int split_tiles(const Prefill& a, int n) {
+  return max(((n + KEYS - 1) / KEYS + a.splits - 1) / a.splits, 3);
 }
 
 // By what the 16-byte places of a row of K or V in LDS are turned round, so that the
@@ -106,9 +116,14 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   constexpr int LOADS = KEYS / RPI / 4;    // a wave's, of K and of V each
   __shared__ __align__(16) u16 buf[2][2][KEYS * D];
   const int head = blockIdx.x % a.heads, j = blockIdx.x / a.heads;
-  const int tile = tile_of(a, SPLIT ? j / a.splits : j);
-  const int split = SPLIT ? j % a.splits : 0;
   const int b = head / a.Hkv, hkv = head - b * a.Hkv;
+  // where nothing is cut the first splits come first, so that each has a CU by itself,
+  // and the others leave at once (4 x 150 rows over 1950 keys 56 us -> 38); else those of
+  // a tile, so that two on a CU are of unlike tiles (75 over 4000 31.8 -> 30.1)
+  const bool cut = SPLIT && cut_keys(a, b);
+  const int split = !SPLIT ? 0 : cut ? j % a.splits : j / a.tiles;
+  if (SPLIT && !cut && split) return;
+  const int tile = tile_of(a, cut ? j / a.splits : j);
   const int R = a.S * a.G, row0 = tile * ROWS;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -118,8 +133,10 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   const int s = min(r, R - 1) / a.G, g = min(r, R - 1) - s * a.G;
   const long prow = ((long)head * R + r) * a.splits + split;
   int t0 = 0, t1 = (n + KEYS - 1) / KEYS;
-  if (SPLIT) {
-    split_tiles(a, b, n, split, t0, t1);
+  if (cut) {
+    const int per = split_tiles(a, n);
+    t0 = split * per;
+    t1 = min(t1, t0 + per);
     if (t0 >= t1 && split) {           // no keys: the sums are never read
       if (h == 0 && r < R) *(f32x2*)(a.pml + prow * 2) = f32x2{M_NONE, 0.f};
       return;
@@ -314,9 +331,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   if (r >= R) return;
   // column dt * 32 + 8 i + 4 h + 0..3 in registers 4 i .. of o[dt]
   if (SPLIT) {
-    int u0, u1;
-    split_tiles(a, b, n, 1, u0, u1);
-    if (u0 < u1) {                     // there are other splits
+    if (cut && split_tiles(a, n) * KEYS < n) {   // there are other splits
       float* po = a.po + prow * D + 4 * h;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
@@ -328,6 +343,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
       if (h == 0) *(f32x2*)(a.pml + prow * 2) = f32x2{m, l};
       return;
     }
+    if (h == 0) *(f32x2*)(a.pml + prow * 2) = f32x2{M_NONE, DONE};
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
   u16* op = a.out + (((long)b * a.S + s) * a.Hkv * a.G + hkv * a.G + g) * D +
@@ -354,10 +370,6 @@ k_attn_prefill_combine(const Prefill a) {
   if (id >= (long)a.heads * R) return;
   const int head = id / R, r = id - (long)head * R;
   const int b = head / a.Hkv, hkv = head - b * a.Hkv;
-  int u0, u1;
-  split_tiles(a, b, keys_of(a, b, min(r / ROWS * ROWS + ROWS, R) - 1), 1, u0,
-              u1);
-  if (u0 >= u1) return;
   // a lane has the maximum and the sum of a split
   const float* ml = a.pml + id * a.splits * 2;
   float m = M_NONE, l = 0.f;
@@ -365,6 +377,11 @@ k_attn_prefill_combine(const Prefill a) {
     m = ml[2 * lane];
     l = ml[2 * lane + 1];
   }
+  // known sooner than the sums are here
+  if (keys_of(a, b, R - 1) <= FEW + a.share) return;
+  if (__builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(
+          __builtin_bit_cast(int, l))) == DONE)
+    return;
   const u64 used = __ballot(lane == 0 || l != 0.f || m != M_NONE);
   float top = m;
 #pragma unroll
@@ -427,9 +444,9 @@ void fei_attn_prefill(const void* q, const void* k_cache, const void* v_cache,
   const int G = Hq / Hkv, tiles = (S * G + ROWS - 1) / ROWS;
   const Prefill a{(const u16*)q, (const u16*)k_cache, (const u16*)v_cache,
                   (u16*)out,     po,     pml,  pos0,  kv_len,
-                  S,             G,      Hkv,  B * Hkv,
-                  tiles,         max_seq, causal, splits,
-                  9 + B * Hkv * tiles / 6,
+                  B,             S,      G,    Hkv,
+                  B * Hkv,       tiles,  max_seq, causal, splits,
+                  Hkv * S * G / 14,
                   scale,         q_ts,   kv_b, kv_h,  kv_t};
   if (D == 128) launch_prefill<128>(a, stream);
   else if (D == 64) launch_prefill<64>(a, stream);

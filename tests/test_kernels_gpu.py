@@ -52,6 +52,11 @@ def attend64(q, k, v, pos0, scale, kv_len=None):
     (40, 4, 2, 64, [10], None, 0.0),            # all keys alike
     (65, 3, 3, 65, [0, 0, 0], [65, 1, 0], None),   # no key at all
     (70, 2, 2, 4000, [0, 0], [4000, 129], None),
+    # rows of a batch that are cut and not: one long one, as many as make none
+    # worth it, more than a wave's lanes
+    (150, 12, 3, 1400, [900, 0, 20, 300], None, None),
+    (150, 12, 3, 1400, [900, 950, 800, 960], None, None),
+    (3, 4, 1, 1300, [1200] * 3 + [0, 700] * 33 + [1000], None, None),
 ])
 def test_attn_prefill_geometries(lib, D, S, Hq, Hkv, T, pos0, kv_len, scale):
     B, W = len(pos0), (Hq + 2 * Hkv) * D
