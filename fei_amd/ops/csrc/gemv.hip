@@ -405,8 +405,9 @@ k_skinny(void* __restrict__ outp, const u16* __restrict__ x,
   const int n = max(min(steps, (wid + 1) * per) - wid * per, 0);
   // blocks start at different steps: rows often lie a multiple of 4 KB apart,
   // and the same columns of all of them would be on the same memory channels (a
-  // decoding step of 8 rows, 32 layers of 4096: 3669 -> 3422 us)
-  const int turn = n ? blockIdx.x * 3 % n : 0;
+  // decoding step of 8 rows, 32 layers of 4096: 3669 -> 3422 us). Two blocks of 8 columns
+  // start where one of 16 does, so that either gives the same bits
+  const int turn = n ? blockIdx.x / (RT ? 1 : 2) * 3 % n : 0;
   auto at = [&](int s) {
     const int t = s + turn;
     return lo + (t < n ? t : t - n);

@@ -423,6 +423,17 @@ def test_skinny_blocks_of_8_columns(lib, M, N, K):
                        rms64(h, g, 1e-5) @ w2.double().T) < 2 ** -7
 
 
+@pytest.mark.parametrize("M", [2, 8, 9, 24, 32])
+@pytest.mark.parametrize("N,K", [(128, 1024), (2048, 8192), (1000, 320)])
+def test_skinny_blocks_of_8_and_16_columns_agree(lib, M, N, K):
+    """To the last bit: the encoder has both in front of the same rows."""
+    x, w = randbf(M, K, seed=1), randbf(N, K, seed=2, scale=K ** -0.5)
+    h = [randbf(M, N, seed=3) for _ in range(2)]
+    for any_tiles in (False, True):
+        lib.add_product(x, w, h[any_tiles], any_tiles)
+    assert torch.equal(*h)
+
+
 # -- RoPE of a prompt --------------------------------------------------------------
 
 @pytest.mark.parametrize("B,S,Hq,Hkv,D,pad", [
