@@ -49,8 +49,10 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
   // whether nothing is asked for past the end, so that 16 steps do not become 20. Else
   // the last step is read again, into a buffer that is free: the second loop costs
   // registers, and more than it gains where steps are many (2 x 14336 x 4096 with
-  // SwiGLU, 96 rows 45.1 us, 46.0 with one loop; 128 53.4, 50.3; 256 99.7, 86.7)
-  constexpr bool EXACT = EPI != ROWS_SWIGLU || WI == 2 || (ONCE && XJ < 4);
+  // SwiGLU, 96 rows 45.1 us, 46.0 with one loop; 128 53.4, 50.3; 256 99.7, 86.7; parts
+  // of 4096 x 14336, 128 rows 30.1, 31.9; 200 50.7, 46.9; 256 52.2, 49.8)
+  constexpr bool EXACT =
+      WI == 2 || (ONCE && (XJ < 4 || EPI != ROWS_SWIGLU));
   constexpr int BUF = (TM + TN) * 64, LOADS = XJ + WI;
   extern __shared__ __align__(16) u16 buf[];
   const int total = nx * nm, per = (total + 7) / 8;
