@@ -93,7 +93,8 @@ __device__ __forceinline__ void load_lds(const u16* src, u32 lds) {
 }
 
 // 64 lanes x 16 bytes from ``base`` (the same in all lanes) + off straight into LDS,
-// lane i at lds + 16 i. m0 is not kept: nothing else may use it.
+// lane i at lds + 16 i. m0 is not kept, and being reserved cannot be named as changed:
+// nothing else in a kernel may use it, which tests/test_kernel_sources.py looks at.
 __device__ __forceinline__ void load_lds_from(const u16* base, u32 off, u32 lds) {
   asm volatile(
       "s_mov_b32 m0, %2\n\t"
