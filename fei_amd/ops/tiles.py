@@ -69,7 +69,8 @@ def tile_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
     K = w.shape[-1]
     return (M > 128 and w.is_cuda and w.dim() == 2 and K > 0 and K % 64 == 0
             and w.shape[0] > 0 and w.shape[0] % 8 == 0 and _memory(x, w)
-            and _near(x, w))
+            # a launch goes to the current device, the library's to the tensors'
+            and w.get_device() == torch.cuda.current_device() and _near(x, w))
 
 
 def _time(M: int, cols: int, K: int, parts: int, rows: int, width: int,

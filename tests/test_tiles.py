@@ -366,6 +366,31 @@ def test_tensors_that_are_more_than_memory():
 
 
 @pytest.mark.gpu
+def test_tensors_of_another_device_are_the_library_s(monkeypatch):
+    M, N, K = 1301, 5704, 2048
+    x, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
+    assert tiles.linear_ok(M, x, w) and tiles.act_ok(M, x, w)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert not tiles.linear_ok(M, x, w) and not tiles.act_ok(M, x, w)
+    long = rand(1024, 8192)
+    assert not tiles.parts_ok(300, rand(300, 8192), long)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("I", [2048, 2052, 2056])
+def test_swiglu_wants_a_multiple_of_8_columns(I):
+    """Gates and ups are a multiple of 8 together before they are one each."""
+    M, K = 2049, 512
+    x, w = rand(M, K, seed=1), rand(2 * I, K, seed=2)
+    assert tiles.act_ok(M, x, w)
+    assert (ops._many_rows(M, x, w) == "tile") == (I % 8 == 0)
+    act = torch.empty(M, 2056, device=DEV, dtype=torch.bfloat16)
+    assert mx._act_tile(x, w, I, act) == (I % 8 == 0)
+    assert not mx._act_tile(x, w, 2048, act[:, 4:])      # rows not on 16 bytes
+    assert not mx._act_tile(x, w, 2048, act.float())
+
+
+@pytest.mark.gpu
 def test_many_rows_under_transforms():
     M, N, K = 1301, 5704, 2048
     x, w = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5)
