@@ -72,8 +72,8 @@ k_pool_unit(float* __restrict__ out, const u16* __restrict__ h,
 // Bound by latency and, from 32 rows on, by the norm's own work on one CU: 16 rows of
 // W and 24 of x take 7 us, a launch of 3.8 for the norm and one of 5 otherwise; in
 // all four waves, in front of the products, 9. Whole encoders, 12 layers of 768,
-// fused and not: 8 rows 341 us, 374; 16 383, 392; 24 392, 411; 32 448, 443; 64 661,
-// 513.
+// fused and not: 8 rows 341 us, 374; 16 383, 392; 24 392, 411; of more rows, in variants
+// that are not kept, 32 448, 443; 64 661, 513.
 constexpr int NORM_WAVES = 12;             // beside four that multiply
 
 template <int XL, bool GELU>

@@ -1,5 +1,5 @@
 // Common helpers for fei_amd gfx950 kernels.
-// CDNA4 only: wave64, MFMA, LDS per /opt/skills/guides/cdna_hip_programming.md.
+// CDNA4 only: waves of 64 lanes, matrix units, 160 KB of LDS a CU.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

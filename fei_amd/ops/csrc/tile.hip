@@ -59,8 +59,8 @@ struct TileArgs {
 // need 2048, at the 1.7 to 2.1 GHz that the card keeps under this load; four turns
 // of one quarter took 2510, and more where both groups ran the same branching code.
 // Against the library, us: 2 x 14336 x 4096 of 2048 rows with SwiGLU 348 (360 + 33
-// for the pass of its own); 3072 x 768 of 16384 with bias and GELU 104
-// (68.5 + 52); 4096 x 14336 of 2048 in two parts 170 (204); 8192^3 706 (700).
+// for the pass of its own); 3072 x 768 of 16384 with bias and GELU 104 to
+// 109 (68.5 + 52); 4096 x 14336 of 2048 in two parts 170 (204); 8192^3 706 (700).
 template <int WM, int XI, int WI, int EPI>
 __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
   constexpr int WN = 8 / WM;
