@@ -2,9 +2,10 @@
 (BERT-style: 12 layers, 768 hidden, 12 heads, post-LayerNorm residual
 blocks, GELU MLP, biased linears).
 
-Up to 1024 rows all layers are launched from one call (ops.encoder_layers), their
-products in this library's matrix-core tiles; beyond, and for one or two rows, the
-products are the BLAS library's. Bidirectional attention runs in the HIP prompt
+Of more than 640 rows, only those that texts have are run (ops.encoder_packed): padding
+is left out on the device. Up to 1024, and of texts without lengths, all layers are
+launched from one call (ops.encoder_layers); both have their products in this library's
+matrix-core tiles. Beyond, and for one or two rows, the products are the BLAS library's. Bidirectional attention runs in the HIP prompt
 kernel (causal=0), LayerNorm with the residual and GELU in HIP kernels. Weights are
 random-init — there is no network for checkpoints — but the architecture matches
 bge-base so real weights could be loaded via the same tensors.
@@ -91,14 +92,19 @@ class BgeEncoder:
         H, D = s.num_heads, s.head_dim
         h = F.embedding(token_ids.long(), self.tok_emb) + \
             self.pos_emb[:S].unsqueeze(0)
-        h = ops.layernorm(h.to(self.dtype), self.emb_ln_w, self.emb_ln_b,
-                          self.eps)
+        h = h.to(self.dtype)
         kv_len = (lengths.to(torch.int32) if lengths is not None
                   else torch.full((B,), S, dtype=torch.int32, device=self.device))
+        weights = [lw[n] for lw in self.layers for n in NAMES]
+        if lengths is not None:
+            out = ops.encoder_packed(h, self.emb_ln_w, self.emb_ln_b, weights,
+                                     H, D, s.intermediate_size, kv_len, self.eps)
+            if out is not None:
+                return out
+        h = ops.layernorm(h, self.emb_ln_w, self.emb_ln_b, self.eps)
         pos0 = torch.zeros(B, dtype=torch.int32, device=self.device)
-        few = ops.encoder_layers(h, [lw[n] for lw in self.layers for n in NAMES],
-                                 H, D, s.intermediate_size, pos0, kv_len,
-                                 self.eps)
+        few = ops.encoder_layers(h, weights, H, D, s.intermediate_size, pos0,
+                                 kv_len, self.eps)
         h = few if few is not None else self._layers(h, pos0, kv_len)
         return ops.pool_unit(h, kv_len)
 

@@ -82,6 +82,8 @@ def _try_load() -> None:
     lib.fei_argmax.argtypes = [_vp] * 3 + [_i] * 4 + [_vp]
     lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
                                        [_f, _f, _i] + [_vp] * 3 + [_i, _i, _vp])
+    lib.fei_encoder_packed.argtypes = ([_vp, _i] + [_vp] * 12 + [_i] * 6 +
+                                       [_f, _f] + [_vp] * 2 + [_i, _i, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -944,6 +946,67 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
         B, S, heads, dim, C, inner, 1.0 / math.sqrt(dim), eps, splits, po, pml,
         _ptr(parts), p1, p2, _stream())
     return h
+
+
+# Rows, padding among them, from which those that texts have are packed, and up to which
+# their products run in tiles of 64 x 64, beyond in k_tile's. Us of 12 layers of 768,
+# texts of a quarter to all of the length (all of one length), with padding, in tiles of
+# 64, in k_tile's: 512 rows 618, 636 (670); 768 745, 658 (747); 1500 1631, 800 (1021),
+# 1094 (1136); 2560 1429, 1053 (1265), 1153 (1260); 3200 1431, 1150 (1537), 1250 (1369);
+# 5120 1694, 1550 (2164), 1522 (1747).
+ENCODER_PACKED_FROM = 640
+ENCODER_PACKED_ROWS = 3072
+
+
+def encoder_packed(emb: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor,
+                   weights, heads: int, dim: int, inner: int,
+                   lens: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
+    """An encoder over texts of unlike lengths: emb [B, S, C], before the norm with
+    ``gain`` and ``shift``, of which text b has lens[b] rows -> embeddings [B, C]
+    float32, or None where its kernels do not take them. Rows that no text has are left
+    out, without the host's knowing how many those are. ``weights``: see
+    encoder_layers."""
+    B, S, C = emb.shape
+    M, HD = B * S, heads * dim
+    tensors = [emb, gain, shift, *weights]
+    if not (emb.is_cuda and dim in (64, 128) and M > ENCODER_PACKED_FROM
+            and M * max(3 * HD, inner, C) < 1 << 31
+            and C % 64 == HD % 64 == inner % 64 == 0 and C <= 2048
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in tensors)
+            and lens.device == emb.device and lens.dtype == torch.int32
+            and lens.shape == (B,) and lens.is_contiguous()
+            and emb.get_device() == torch.cuda.current_device()
+            and _tiles._memory(*tensors, lens)
+            and _prefill_splits(B, heads, S, S) == 1):
+        return None
+
+    def rows(n):
+        return torch.empty(M, n, dtype=emb.dtype, device=emb.device)
+    room = [rows(n) for n in (C, C, C, 3 * HD, HD, inner)]
+    starts = torch.empty(B + 1, dtype=torch.int32, device=emb.device)
+    out = torch.empty(B, C, dtype=torch.float32, device=emb.device)
+    sizes = parts = None
+    if M > ENCODER_PACKED_ROWS:
+        best = [_tiles.parts_up_to(M, *c) for c in (
+            (3 * HD, C, 1), (C, HD), (inner, C, 1), (C, inner))]
+        sizes = (_i * 8)(*(v for size, _ in best for v in size))
+        p1, p2 = best[1][1], best[3][1]
+    else:
+        # as in encoder_layers, for two thirds of the rows
+        tiles = -(-M * 2 // 3 // 64) * -(-C // 64)
+        p1, p2 = (min(256 // tiles, 8, k // 256) for k in (HD, inner))
+    p1, p2 = (p if p > 1 else 0 for p in (p1, p2))
+    if p1 or p2:
+        parts = torch.empty(max(p1, p2) * M * C, dtype=torch.float32,
+                            device=emb.device)
+    require_lib().fei_encoder_packed(
+        (_vp * len(weights))(*(t.data_ptr() for t in weights)),
+        len(weights) // 12, _ptr(out), _ptr(emb), _ptr(gain), _ptr(shift),
+        *(_ptr(t) for t in room), _ptr(lens), _ptr(starts), B, S, heads, dim, C,
+        inner, 1.0 / math.sqrt(dim), eps, sizes,
+        None if parts is None else _ptr(parts), p1, p2, _stream())
+    return out
 
 
 def pool_unit(h: torch.Tensor, lens: torch.Tensor) -> torch.Tensor:

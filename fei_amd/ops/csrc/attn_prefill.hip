@@ -46,7 +46,7 @@ struct Prefill {
   const u16 *q, *kc, *vc;
   u16* out;
   float *po, *pml;                     // partial results of splits
-  const int *pos0, *kv_len;
+  const int *pos0, *kv_len, *starts;   // starts: the first row of each text, PACKED
   int B, S, G, Hkv, heads, tiles, max_seq, causal, splits;
   int share;                           // keys for the rows of a batch row: cut_keys
   float scale;
@@ -107,7 +107,9 @@ __device__ __forceinline__ int tile_of(const Prefill& a, int j) {
   return a.tiles - 1 - j;
 }
 
-template <int D, bool SPLIT>
+// PACKED: a row of the batch has kv_len[b] <= S tokens, whose queries, keys, values and
+// results are rows starts[b] and on; of those that it has not nothing is touched.
+template <int D, bool SPLIT, bool PACKED = false>
 __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   constexpr int KS = D / 16;           // steps of a score product
   constexpr int DT = D / 32;           // tiles of 32 value columns
@@ -124,7 +126,9 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   const int split = !SPLIT ? 0 : cut ? j % a.splits : j / a.tiles;
   if (SPLIT && !cut && split) return;
   const int tile = tile_of(a, cut ? j / a.splits : j);
-  const int R = a.S * a.G, row0 = tile * ROWS;
+  const int R = (PACKED ? keys_of(a, b, 0) : a.S) * a.G, row0 = tile * ROWS;
+  if (PACKED && row0 >= R) return;
+  const long tok0 = PACKED ? a.starts[b] : (long)b * a.S;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l31 = lane & 31, h = lane >> 5;
@@ -158,7 +162,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
   const u32 keep = a.scale == 0.f ? 0u : 0xffffffffu;
   s16x8 fq[KS];
   {
-    const u16* qp = a.q + ((long)b * a.S + s) * a.q_ts +
+    const u16* qp = a.q + (tok0 + s) * a.q_ts +
                     (long)(hkv * a.G + g) * D + 8 * h;
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
@@ -169,8 +173,8 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
     }
   }
 
-  const u16* kb = a.kc + b * a.kv_b + hkv * a.kv_h;
-  const u16* vb = a.vc + b * a.kv_b + hkv * a.kv_h;
+  const long kv0 = (PACKED ? tok0 * a.kv_t : b * a.kv_b) + hkv * a.kv_h;
+  const u16 *kb = a.kc + kv0, *vb = a.vc + kv0;
   const u32 lds =
       (u32)(uintptr_t)(__attribute__((address_space(3))) u16*)&buf[0][0][0];
   // what a lane loads of a tile, in bytes from its first row: the wave's LOADS times
@@ -346,8 +350,7 @@ __global__ void __launch_bounds__(256, 2) k_attn_prefill(const Prefill a) {
     if (h == 0) *(f32x2*)(a.pml + prow * 2) = f32x2{M_NONE, DONE};
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
-  u16* op = a.out + (((long)b * a.S + s) * a.Hkv * a.G + hkv * a.G + g) * D +
-            4 * h;
+  u16* op = a.out + ((tok0 + s) * a.Hkv * a.G + hkv * a.G + g) * D + 4 * h;
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -443,13 +446,33 @@ void fei_attn_prefill(const void* q, const void* k_cache, const void* v_cache,
                       long kv_b, long kv_h, long kv_t, hipStream_t stream) {
   const int G = Hq / Hkv, tiles = (S * G + ROWS - 1) / ROWS;
   const Prefill a{(const u16*)q, (const u16*)k_cache, (const u16*)v_cache,
-                  (u16*)out,     po,     pml,  pos0,  kv_len,
+                  (u16*)out,     po,     pml,  pos0,  kv_len, nullptr,
                   B,             S,      G,    Hkv,
                   B * Hkv,       tiles,  max_seq, causal, splits,
                   Hkv * S * G / 14,
                   scale,         q_ts,   kv_b, kv_h,  kv_t};
   if (D == 128) launch_prefill<128>(a, stream);
   else if (D == 64) launch_prefill<64>(a, stream);
+}
+
+// Attention of B texts of kv_len[b] of at most S tokens among themselves, whose rows lie
+// one behind another from row starts[b] on: q, k and v a row of 3 H D values, out of H D.
+// D is 64 or 128; all on 16 bytes. kv_len is taken at S where it is more.
+void fei_attn_packed(const void* qkv, void* out, const int* kv_len,
+                     const int* starts, int B, int S, int H, int D, float scale,
+                     hipStream_t stream) {
+  const int HD = H * D, tiles = (S + ROWS - 1) / ROWS;
+  const u16* p = (const u16*)qkv;
+  const Prefill a{p, p + HD, p + 2 * HD, (u16*)out, nullptr, nullptr, kv_len,
+                  kv_len, starts, B, S, 1, H, B * H, tiles, S, 0, 1, 0, scale,
+                  3L * HD, 0, D, 3L * HD};
+  const dim3 grid((unsigned)a.heads * tiles);
+  if (D == 128)
+    hipLaunchKernelGGL((k_attn_prefill<128, false, true>), grid, dim3(256), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((k_attn_prefill<64, false, true>), grid, dim3(256), 0,
+                       stream, a);
 }
 
 // ---------------------------------------------------------------------------

@@ -17,18 +17,21 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 // Mean of a text's first len rows, to length 1: out [B, C] float32. A block per
 // text; a thread has 8 columns of every SIDEth row. Bound by latency, and by what
-// one CU loads of a long text (256 rows of 768: 393 KB). In library operations it
+// one CU loads of a long text (256 rows of 768: 393 KB). starts: null, or the first row
+// of each text, where only the rows that texts have are there. In library operations it
 // is nine launches and six passes over the rows in float32: 64 texts of 256 about
 // 110 us for 8.6 here.
 __global__ void __launch_bounds__(1024)
 k_pool_unit(float* __restrict__ out, const u16* __restrict__ h,
-            const int* __restrict__ lens, int S, int C) {
+            const int* __restrict__ lens, const int* __restrict__ starts,
+            int S, int C) {
   extern __shared__ __align__(16) float part[];    // [sides][C]
   __shared__ float red[16];
   const int b = blockIdx.x, tid = threadIdx.x, nv = C >> 3;
   const int sides = 1024 / nv, side = tid / nv, c = tid - side * nv;
   const int n = min(max(lens[b], 0), S);
-  const s16x8* row = (const s16x8*)(h + (long)b * S * C) + c;
+  const long first = starts ? starts[b] : (long)b * S;
+  const s16x8* row = (const s16x8*)(h + first * C) + c;
   float v[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) v[j] = 0.f;
@@ -60,6 +63,38 @@ k_pool_unit(float* __restrict__ out, const u16* __restrict__ h,
   const float len = sqrtf(sq);
   const float norm = len < 1e-12f ? 1e-12f : len;   // NaN stays
   for (int i = tid; i < C; i += 1024) out[(long)b * C + i] = part[i] / norm;
+}
+
+// First row of each of B texts that lie one behind another, and behind the last the
+// number of rows in all. A text has lens[b] rows, at least none and at most S.
+__global__ void __launch_bounds__(1024)
+k_text_starts(int* __restrict__ starts, const int* __restrict__ lens, int B,
+              int S) {
+  __shared__ int sum[16];
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  int before = 0;
+  for (int b0 = 0; b0 < B; b0 += 1024) {
+    const int b = b0 + tid;
+    int v = b < B ? min(max(lens[b], 0), S) : 0;
+    const int n = v;
+#pragma unroll
+    for (int i = 1; i < 64; i *= 2) {
+      const int t = __shfl_up(v, i);
+      if (lane >= i) v += t;
+    }
+    __syncthreads();                       // the sums before have been read
+    if (lane == 63) sum[wid] = v;
+    __syncthreads();
+    int all = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      if (k < wid) v += sum[k];
+      all += sum[k];
+    }
+    if (b < B) starts[b] = before + v - n;
+    before += all;
+  }
+  if (tid == 0) starts[B] = before;
 }
 
 // out = LayerNorm(x + res) W^T + bias, or GELU of it: what an encoder's layer does
@@ -267,7 +302,7 @@ void fei_pool_unit(float* out, const void* h, const int* lens, int B, int S,
                    int C, hipStream_t stream) {
   const int sides = 1024 / (C / 8);
   hipLaunchKernelGGL(k_pool_unit, dim3(B), dim3(1024), sides * C * 4, stream,
-                     out, (const u16*)h, lens, S, C);
+                     out, (const u16*)h, lens, nullptr, S, C);
 }
 
 void fei_skinny(void* out, const void* x, const void* w, int M, int N, int K,
@@ -292,6 +327,87 @@ void fei_attn_prefill(const void* q, const void* k_cache, const void* v_cache,
 void fei_add_layernorm(void* out, const void* x, const void* res,
                        const void* w, const void* b, int rows, int cols,
                        float eps, int has_res, hipStream_t stream);
+
+void fei_rows_bias_of(void* out, const void* x, const void* w, const void* bias,
+                      int M, int N, int K, int gelu, const int* count,
+                      hipStream_t stream);
+void fei_rows_parts_of(float* out, const void* x, const void* w, int M, int N,
+                       int K, int parts, const int* count, hipStream_t stream);
+void fei_parts_layernorm_of(void* out, const float* parts, int np,
+                            const void* bias, const void* res, const void* gain,
+                            const void* shift, int rows, int cols, float eps,
+                            const int* count, hipStream_t stream);
+void fei_tile(void* out, long os, const void* x, long xs, const void* w,
+              const void* bias, int M, int N, int K, int epi, int rows,
+              int width, int parts, const int* count, hipStream_t stream);
+void fei_attn_packed(const void* qkv, void* out, const int* kv_len,
+                     const int* starts, int B, int S, int H, int D, float scale,
+                     hipStream_t stream);
+void fei_layernorm_packed(void* out, const void* x, const void* res,
+                          const void* w, const void* bias, int texts, int S,
+                          int cols, float eps, const int* starts,
+                          hipStream_t stream);
+
+// An encoder over the rows that its texts have, one behind another: out [B, C] float32.
+// emb [B, S, C] is what the first norm (gain, shift) takes; w: 12 a layer, as in
+// fei_encoder_layers; h, h1 and tmp have room for B * S rows of C, qkv of 3 H D, att of
+// H D, inner of I; starts for B + 1. How many rows there are only the device knows: grids
+// are made for all B * S, and blocks that have none leave. sizes: rows and width of the
+// tiles (fei_tile) of the four products of a layer; null: tiles of 64 x 64. p1, p2 and
+// parts as in fei_encoder_layers. All on 16 bytes, C and H D and I
+// multiples of 64, C <= 2048.
+//
+// 64 texts of 64 to 256 tokens, 10336 rows of 16384, 12 layers of 768: 3000 us; all
+// rows, with the library's products, 4005. Bound by the products, at 0.7 to 0.8 PFLOP/s
+// of tiles that fill the chip one and a half times. To find the number costs each kernel
+// a load before its first, 30 us of the 570 that 320 rows take in all.
+void fei_encoder_packed(const void* const* w, int layers, float* out,
+                        const void* emb, const void* gain, const void* shift,
+                        void* h, void* h1, void* tmp, void* qkv, void* att,
+                        void* inner, const int* lens, int* starts, int B, int S,
+                        int H, int D, int C, int I, float scale, float eps,
+                        const int* sizes, float* parts, int p1, int p2,
+                        hipStream_t stream) {
+  const int M = B * S, HD = H * D;
+  const int* count = starts + B;
+  hipLaunchKernelGGL(k_text_starts, dim3(1), dim3(1024), 0, stream, starts,
+                     lens, B, S);
+  fei_layernorm_packed(h, emb, nullptr, gain, shift, B, S, C, eps, starts,
+                       stream);
+  auto product = [&](int i, void* to, const void* x, const void* const* wb,
+                     int N, int K, bool gelu) {
+    constexpr int TILE_GELU = 2, TILE_BIAS = 5;
+    if (!sizes)
+      return fei_rows_bias_of(to, x, wb[0], wb[1], M, N, K, gelu, count, stream);
+    fei_tile(to, N, x, K, wb[0], wb[1], M, N, K, gelu ? TILE_GELU : TILE_BIAS,
+             sizes[2 * i], sizes[2 * i + 1], 1, count, stream);
+  };
+  auto residual = [&](int i, void* to, const void* from, const void* x,
+                      const void* const* wb, int K, int np) {
+    if (np) {
+      constexpr int TILE_PARTS = 4;
+      if (sizes)
+        fei_tile(parts, C, x, K, wb[0], nullptr, M, C, K, TILE_PARTS,
+                 sizes[2 * i], sizes[2 * i + 1], np, count, stream);
+      else
+        fei_rows_parts_of(parts, x, wb[0], M, C, K, np, count, stream);
+      return fei_parts_layernorm_of(to, parts, np, wb[1], from, wb[2], wb[3], M,
+                                    C, eps, count, stream);
+    }
+    product(i, tmp, x, wb, C, K, false);
+    fei_layernorm_packed(to, tmp, from, wb[2], wb[3], B, S, C, eps, starts,
+                         stream);
+  };
+  for (int l = 0; l < layers; ++l, w += 12) {
+    product(0, qkv, h, w, 3 * HD, C, false);
+    fei_attn_packed(qkv, att, lens, starts, B, S, H, D, scale, stream);
+    residual(1, h1, h, att, w + 2, HD, p1);
+    product(2, inner, h1, w + 6, I, C, true);
+    residual(3, h, h1, inner, w + 8, I, p2);
+  }
+  hipLaunchKernelGGL(k_pool_unit, dim3(B), dim3(1024), 1024 / (C / 8) * C * 4,
+                     stream, out, (const u16*)h, lens, starts, S, C);
+}
 
 // w: 12 a layer, in the order in which they are read below; h [B * S, C] is
 // replaced by the layers' result; h1 and tmp as h, qkv [B * S, 3 H D],

@@ -637,14 +637,26 @@ void fei_sample_shard(const void* logits, float* out, const int* step,
 // ---------------------------------------------------------------------------
 namespace {
 
-template <int V, bool RES>               // loads of 8 columns a lane
+// PACK: text b of at most S rows has rows starts[b] to starts[b + 1] - 1 of ``out``.
+// ALL_ROWS: x is [texts, S, cols], and the rows that a text has not are left out;
+// PACKED_ROWS: x and res are packed already.
+enum { NO_PACK, ALL_ROWS, PACKED_ROWS };
+template <int V, bool RES, int PACK = NO_PACK>   // V loads of 8 columns a lane
 __global__ void __launch_bounds__(256)
 k_layernorm_wave(u16* __restrict__ out, const u16* __restrict__ x,
                  const u16* __restrict__ res, const u16* __restrict__ w,
-                 const u16* __restrict__ bias, int rows, int cols, float eps) {
+                 const u16* __restrict__ bias, int rows, int cols, float eps,
+                 const int* __restrict__ starts, int S) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
+  int to = row;
+  if (PACK == ALL_ROWS) {
+    const int b = row / S;
+    to = starts[b] + row - b * S;
+    if (to >= starts[b + 1]) return;
+  }
+  if (PACK == PACKED_ROWS && row >= starts[rows / S]) return;
   const int nv = cols >> 3;
   const s16x8* xr = (const s16x8*)(x + (long)row * cols);
   const s16x8* rr = (const s16x8*)(res + (long)row * cols);
@@ -689,7 +701,7 @@ k_layernorm_wave(u16* __restrict__ out, const u16* __restrict__ x,
     for (int j = 0; j < 8; ++j)
       o[j] = (short)f2bf(f[i][j] * inv * bf2f((u16)wv[i][j]) +
                          bf2f((u16)bv[i][j]));
-    ((s16x8*)(out + (long)row * cols))[at] = o;
+    ((s16x8*)(out + (long)to * cols))[at] = o;
   }
 }
 
@@ -759,7 +771,8 @@ void fei_add_layernorm(void* out, const void* x, const void* res,
   auto by_wave = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((rows + 3) / 4), dim3(256), 0, stream,
                        (u16*)out, (const u16*)x, (const u16*)res,
-                       (const u16*)w, (const u16*)bias, rows, cols, eps);
+                       (const u16*)w, (const u16*)bias, rows, cols, eps,
+                       nullptr, 0);
   };
   if (nv >= 1 && nv <= 64)
     return by_wave(has_res ? k_layernorm_wave<1, true>
@@ -775,6 +788,27 @@ void fei_add_layernorm(void* out, const void* x, const void* res,
                      (u16*)out, (const u16*)x, (const u16*)res,
                      (const u16*)w, (const u16*)bias, rows, cols, eps,
                      has_res);
+}
+
+// Of the rows that texts have; starts has texts + 1 values. Without res x is [texts, S,
+// cols], with it x and res are packed. cols % 8 == 0, at most 2048.
+void fei_layernorm_packed(void* out, const void* x, const void* res,
+                          const void* w, const void* bias, int texts, int S,
+                          int cols, float eps, const int* starts,
+                          hipStream_t stream) {
+  const int rows = texts * S, nv = cols >> 3;
+  auto by_wave = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((rows + 3) / 4), dim3(256), 0, stream,
+                       (u16*)out, (const u16*)x, (const u16*)res,
+                       (const u16*)w, (const u16*)bias, rows, cols, eps,
+                       starts, S);
+  };
+#define GO(V) by_wave(res ? k_layernorm_wave<V, true, PACKED_ROWS>           \
+                          : k_layernorm_wave<V, false, ALL_ROWS>)
+  if (nv <= 64) return GO(1);
+  if (nv <= 128) return GO(2);
+  GO(4);
+#undef GO
 }
 
 // GELU, erf form (torch's default). 16384 x 3072: 50 us with erff, 41 with

@@ -39,11 +39,15 @@ enum {
 // the L2: 75 rows 26.6 -> 24.3, 14.9 -> 14.4, 45.9 -> 44.8, 40 rows of the last 43.7
 // -> 38.3; two tiles share what they read (200 rows, 2 x 14336 x 4096 in tiles of
 // 64 columns 92 -> 117).
-template <int XJ, int WI, int S, int EPI, bool ONCE>
+//
+// COUNTED: only the device knows how many of the ``room`` rows there are, and finds the
+// number at ``count``; blocks without a tile leave at once. The others are told their
+// tiles of rows, nm: to look at count and reckon cost 75 rows 0.4 us a launch.
+template <int XJ, int WI, int S, int EPI, bool ONCE, bool COUNTED>
 __global__ void __launch_bounds__(256, S * (XJ + WI) <= 20 ? 2 : 1)
 k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
-       const u16* __restrict__ w, const u16* __restrict__ bias, int M, int N,
-       int K, int nx, int nm) {
+       const u16* __restrict__ w, const u16* __restrict__ bias, int room, int N,
+       int K, int nx, int all_nm, const int* __restrict__ count) {
   constexpr int TM = 32 * XJ, TN = 32 * WI, MX = XJ > WI ? XJ : WI;
   constexpr int CN = EPI == ROWS_SWIGLU ? TN / 2 : TN;   // columns of out
   // whether nothing is asked for past the end, so that 16 steps do not become 20. Else
@@ -55,7 +59,9 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
       WI == 2 || (ONCE && (XJ < 4 || EPI != ROWS_SWIGLU));
   constexpr int BUF = (TM + TN) * 64, LOADS = XJ + WI;
   extern __shared__ __align__(16) u16 buf[];
-  const int total = nx * nm, per = (total + 7) / 8;
+  const int M =
+      COUNTED ? __builtin_amdgcn_readfirstlane(min(*count, room)) : room;
+  const int nm = COUNTED ? (M + TM - 1) / TM : all_nm, total = nx * nm, per = (total + 7) / 8;
   const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || id >= total) return;
   const int g0 = id / (4 * nx) * 4, gm = min(4, nm - g0), gr = id - g0 * nx;
@@ -195,23 +201,24 @@ k_rows(void* __restrict__ outp, const u16* __restrict__ x, long xs,
         }
         __builtin_memcpy((u16*)outp + at, v, sizeof(v));
       } else {
-        *(f32x4*)((float*)outp + (long)blockIdx.y * M * N + at) = acc[i][j];
+        *(f32x4*)((float*)outp + (long)blockIdx.y * room * N + at) = acc[i][j];
       }
     }
   }
 }
 
-template <int XJ, int WI, int S, int EPI, bool ONCE>
+template <int XJ, int WI, int S, int EPI, bool ONCE, bool COUNTED = false>
 void launch(void* out, const void* x, long xs, const void* w, int M, int N,
-            int K, int parts, hipStream_t stream, const void* bias = nullptr) {
+            int K, int parts, hipStream_t stream, const void* bias = nullptr,
+            const int* count = nullptr) {
   constexpr int lds = S * 32 * (XJ + WI) * 128;
   constexpr int CN = EPI == ROWS_SWIGLU ? 16 * WI : 32 * WI;
-  allow_lds(k_rows<XJ, WI, S, EPI, ONCE>, lds);
+  allow_lds(k_rows<XJ, WI, S, EPI, ONCE, COUNTED>, lds);
   const int nx = (N + CN - 1) / CN, nm = (M + 32 * XJ - 1) / (32 * XJ);
-  hipLaunchKernelGGL((k_rows<XJ, WI, S, EPI, ONCE>),
+  hipLaunchKernelGGL((k_rows<XJ, WI, S, EPI, ONCE, COUNTED>),
                      dim3((nx * nm + 7) / 8 * 8, parts), dim3(256), lds, stream,
                      out, (const u16*)x, xs, (const u16*)w, (const u16*)bias, M,
-                     N, K, nx, nm);
+                     N, K, nx, nm, count);
 }
 
 // Four buffers, but three for 128 rows of x and 64 of w, of which two blocks fit a
@@ -289,10 +296,10 @@ __global__ void __launch_bounds__(256)
 k_parts_layernorm(u16* __restrict__ out, const float* __restrict__ parts, int np,
                   const u16* __restrict__ bias, const u16* __restrict__ res,
                   const u16* __restrict__ gain, const u16* __restrict__ shift,
-                  int rows, int cols, float eps) {
+                  int rows, int cols, float eps, const int* __restrict__ count) {
   const int lane = threadIdx.x & 63, nv = cols >> 3;
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (row >= rows) return;
+  if (row >= (count ? min(*count, rows) : rows)) return;
   const long step = (long)rows * cols;
   float v[V][8], sum = 0.f;
 #pragma unroll
@@ -505,6 +512,25 @@ void fei_rows_bias(void* out, const void* x, const void* w, const void* bias,
     launch<2, 2, 3, ROWS_BIAS, false>(out, x, K, w, M, N, K, 1, stream, bias);
 }
 
+// Of as many of the M rows as the device finds at ``count``.
+void fei_rows_bias_of(void* out, const void* x, const void* w, const void* bias,
+                      int M, int N, int K, int gelu, const int* count,
+                      hipStream_t stream) {
+  if (gelu)
+    launch<2, 2, 3, ROWS_GELU, false, true>(out, x, K, w, M, N, K, 1, stream,
+                                            bias, count);
+  else
+    launch<2, 2, 3, ROWS_BIAS, false, true>(out, x, K, w, M, N, K, 1, stream,
+                                            bias, count);
+}
+
+// Float32 [parts, M, N] of as many, in tiles of 64 x 64.
+void fei_rows_parts_of(float* out, const void* x, const void* w, int M, int N,
+                       int K, int parts, const int* count, hipStream_t stream) {
+  launch<2, 2, 4, ROWS_PARTS, false, true>(out, x, K, w, M, N, K, parts, stream,
+                                           nullptr, count);
+}
+
 void fei_parts_norm(void* out, void* res, const float* parts, int np,
                     const void* gain, int rows, int cols, float eps,
                     hipStream_t stream) {
@@ -512,18 +538,26 @@ void fei_parts_norm(void* out, void* res, const float* parts, int np,
                      (u16*)res, parts, np, (const u16*)gain, rows, cols, eps);
 }
 
-// cols % 8 == 0, at most 2048; out may be none of the inputs
-void fei_parts_layernorm(void* out, const float* parts, int np,
-                         const void* bias, const void* res, const void* gain,
-                         const void* shift, int rows, int cols, float eps,
-                         hipStream_t stream) {
+// cols % 8 == 0, at most 2048; out may be none of the inputs; count as above
+void fei_parts_layernorm_of(void* out, const float* parts, int np,
+                            const void* bias, const void* res, const void* gain,
+                            const void* shift, int rows, int cols, float eps,
+                            const int* count, hipStream_t stream) {
 #define GO(V)                                                                \
   hipLaunchKernelGGL(k_parts_layernorm<V>, dim3((rows + 3) / 4), dim3(256), 0, \
                      stream, (u16*)out, parts, np, (const u16*)bias,          \
                      (const u16*)res, (const u16*)gain, (const u16*)shift,    \
-                     rows, cols, eps)
+                     rows, cols, eps, count)
   if (cols <= 1024) GO(2); else GO(4);
 #undef GO
+}
+
+void fei_parts_layernorm(void* out, const float* parts, int np,
+                         const void* bias, const void* res, const void* gain,
+                         const void* shift, int rows, int cols, float eps,
+                         hipStream_t stream) {
+  fei_parts_layernorm_of(out, parts, np, bias, res, gain, shift, rows, cols, eps,
+                         nullptr, stream);
 }
 
 // parts [np][B * S][(Hq + 2 Hkv) * D], q [B * S][Hq][D]; D % 16 == 0, all on 16

@@ -14,6 +14,7 @@ enum {
   TILE_GELU = 2,       // with a bias per column
   TILE_RELU2 = 3,
   TILE_PARTS = 4,      // float32 sums of a part of K, [parts][M][N]
+  TILE_BIAS = 5,       // a bias per column alone
 };
 
 __device__ __forceinline__ int uniform(int v) {
@@ -25,8 +26,9 @@ struct TileArgs {
   const u16* x;
   const u16* w;
   const u16* bias;
+  const int* rows;     // how many of the M rows there are, if only the device knows
   long os, xs;         // rows of out and x are this far apart
-  int M, N, K, nx, nm, parts;
+  int M, N, K, nx, parts;
 };
 
 // A block: 8 waves, two on a SIMD, that share tiles of 32 WM XI rows of x and
@@ -72,8 +74,10 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
   constexpr int STAGE = (TM + TN) * 64;
   extern __shared__ __align__(16) u16 buf[];
   u16* const lbias = buf + 2 * STAGE;                   // [4 tiles][512]
-  const int M = g.M, N = g.N, K = g.K, parts = g.parts;
-  const int total = g.nx * g.nm, tiles = total * parts, per = (tiles + 7) / 8;
+  constexpr bool BIAS = EPI == TILE_GELU || EPI == TILE_BIAS;
+  const int M = g.rows ? uniform(min(*g.rows, g.M)) : g.M;
+  const int N = g.N, K = g.K, parts = g.parts, nm = (M + TM - 1) / TM;
+  const int total = g.nx * nm, tiles = total * parts, per = (tiles + 7) / 8;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
   const int lim = min(per, tiles - xcd * per);          // tiles of the XCD
   if (slot >= lim) return;
@@ -85,7 +89,7 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     int id = xcd * per + i;
     t.part = uniform(id / total);
     id -= t.part * total;
-    const int g0 = uniform(id / (8 * g.nx)) * 8, gm = min(8, g.nm - g0);
+    const int g0 = uniform(id / (8 * g.nx)) * 8, gm = min(8, nm - g0);
     const int gr = id - g0 * g.nx, c = uniform(gr / gm);
     t.n0 = c * CN;
     t.m0 = (g0 + gr - c * gm) * TM;
@@ -126,7 +130,7 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
       const int f = (r & 3) | ((r % (16 * WI) / (4 * WI)) & 1) << 2;
       ob[i] = (u32)min(r, last_b) * (u32)(K * 2) + (c8 ^ f) * 16;
     }
-    if (EPI == TILE_GELU && wid == 0)
+    if (BIAS && wid == 0)
       load_lds_from(g.bias, (u32)min(ld.n0 + (ln & 31) * 8, N - 8) * 2,
                     lds + 4 * STAGE + (ltile & 3) * 1024);
   };
@@ -236,7 +240,7 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     asm volatile("" : "+v"(ln));
     const int nr = b * HB + wn * 16 * WI + V * (ln >> 4), n = t.n0 + nr;
     u16 add[V];
-    if (EPI == TILE_GELU)
+    if (BIAS)
 #pragma unroll
       for (int j = 0; j < WI; ++j)
         __builtin_memcpy(add + 4 * j, lbias + (tile & 3) * 512 + nr + 4 * j, 8);
@@ -245,7 +249,7 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
       const int m = t.m0 + a * HA + wm * 16 * XI + i * 16 + (ln & 15);
       if (m < M && n < N) {
         if (EPI == TILE_PARTS) {
-          float* p = (float*)g.out + ((long)t.part * M + m) * N + n;
+          float* p = (float*)g.out + ((long)t.part * g.M + m) * N + n;
 #pragma unroll
           for (int j = 0; j < WI; ++j)
             if (n + 4 * j < N) *(f32x4*)(p + 4 * j) = acc[a][b][i][j];
@@ -257,7 +261,8 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
             for (int e = 0; e < 4; ++e) {
               float y = acc[a][b][i][j][e];
               if (PAIR) y = swiglu(y, acc[a][1][i][j][e]);
-              if (EPI == TILE_GELU) y = gelu_erf(y + bf2f(add[j * 4 + e]));
+              if (BIAS) y += bf2f(add[j * 4 + e]);
+              if (EPI == TILE_GELU) y = gelu_erf(y);
               if (EPI == TILE_RELU2) y = relu2(y);
               v[j * 4 + e] = El<u16>::st(y);
             }
@@ -344,9 +349,9 @@ void launch(TileArgs g, hipStream_t stream) {
   constexpr int lds = 2 * (TM + TN) * 128 + 4096;
   allow_lds(k_tile<WM, XI, WI, EPI>, lds);
   g.nx = (g.N + CN - 1) / CN;
-  g.nm = (g.M + TM - 1) / TM;
+  const long nm = (g.M + TM - 1) / TM;
   // a block a CU
-  const int blocks = std::min(256L, ((long)g.nx * g.nm * g.parts + 7) / 8 * 8);
+  const int blocks = std::min(256L, (nm * g.nx * g.parts + 7) / 8 * 8);
   hipLaunchKernelGGL((k_tile<WM, XI, WI, EPI>), dim3(blocks), dim3(512), lds,
                      stream, g);
 }
@@ -367,18 +372,20 @@ extern "C" {
 // Rows of x (xs apart) and w on 16 bytes and less than 2^24 values apart, K % 64 == 0
 // and at least 64 a part, N % 8 == 0; rows of out (os apart) on 16 bytes, as the bias. A tile has rows x width
 // rows of x and w: 256 x 256, 192 or 128, 192 x 256, 128 x 256. epi: see above; parts
-// are 1 but for TILE_PARTS.
+// are 1 but for TILE_PARTS. count: null, or where the device finds how many of the M
+// rows there are; blocks without a tile leave at once.
 void fei_tile(void* out, long os, const void* x, long xs, const void* w,
               const void* bias, int M, int N, int K, int epi, int rows,
-              int width, int parts, hipStream_t stream) {
-  const TileArgs g = {out, (const u16*)x, (const u16*)w, (const u16*)bias,
-                      os, xs, M, N, K, 0, 0, parts};
+              int width, int parts, const int* count, hipStream_t stream) {
+  const TileArgs g = {out, (const u16*)x, (const u16*)w, (const u16*)bias, count,
+                      os, xs, M, N, K, 0, parts};
   switch (epi) {
     case TILE_BF16: return by_size<TILE_BF16>(rows, width, g, stream);
     case TILE_SWIGLU: return by_size<TILE_SWIGLU>(rows, width, g, stream);
     case TILE_GELU: return by_size<TILE_GELU>(rows, width, g, stream);
     case TILE_RELU2: return by_size<TILE_RELU2>(rows, width, g, stream);
     case TILE_PARTS: return by_size<TILE_PARTS>(rows, width, g, stream);
+    case TILE_BIAS: return by_size<TILE_BIAS>(rows, width, g, stream);
   }
 }
 

@@ -15,7 +15,7 @@ import fei_amd.ops as _ops     # half made yet: it imports this
 _vp, _i, _l = ctypes.c_void_p, ctypes.c_int, ctypes.c_long
 
 # csrc/tile.hip
-TILE_BF16, TILE_SWIGLU, TILE_GELU, TILE_RELU2, TILE_PARTS = range(5)
+TILE_BF16, TILE_SWIGLU, TILE_GELU, TILE_RELU2, TILE_PARTS, TILE_BIAS = range(6)
 
 CUS = 256
 FAR = 1 << 24        # rows this far apart: what 128 of them span takes more than 32 bits
@@ -26,7 +26,8 @@ TILES = ((256, 256, 1.0, 0.46), (256, 192, 0.875, 0.36), (192, 256, 0.82, 0.34),
 
 
 def declare(lib: ctypes.CDLL) -> None:
-    lib.fei_tile.argtypes = [_vp, _l, _vp, _l, _vp, _vp] + [_i] * 7 + [_vp]
+    lib.fei_tile.argtypes = ([_vp, _l, _vp, _l, _vp, _vp] + [_i] * 7 +
+                             [_vp, _vp])
 
 
 def _p(t: Optional[torch.Tensor]):
@@ -158,7 +159,7 @@ def _launch(out, x, w, N, epi, size, bias=None, parts=1) -> None:
     M, K = x.shape
     _ops.require_lib().fei_tile(
         _p(out), out.stride(-2), _p(x), x.stride(0), _p(w), _p(bias), M, N, K,
-        epi, *size, parts, _ops._stream())
+        epi, *size, parts, None, _ops._stream())
 
 
 def parts_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -204,6 +205,22 @@ def parts_for(M: int, N: int, K: int) -> Tuple[Tuple[int, int], int]:
     tile, p = min(((t, p) for t in TILES for p in range(1, 9)),
                   key=lambda c: _time(M, N, K, c[1], *c[0]) +
                   c[1] * M * N * 1.8e-6)
+    return tile[:2], p
+
+
+@lru_cache(maxsize=1024)
+def parts_up_to(M: int, N: int, K: int, most: int = 8
+                ) -> Tuple[Tuple[int, int], int]:
+    """The same where only the device knows how many of M rows there are, half of them
+    or more, and something reads the results of a product in one part too. All of them
+    count twice: texts are often cut to one length."""
+    def us(m, tile, p):
+        return (_time(m, N, K, p, *tile) +
+                m * N * (1.8e-6 * p if p > 1 else 0.9e-6))
+    ways = [(t, p) for t in TILES for p in range(1, min(most, K // 256) + 1)]
+    times = [[us(M * f // 8, *way) for way in ways] for f in (4, 5, 6, 7, 8, 8)]
+    loss = [sum(row[i] / min(row) for row in times) for i in range(len(ways))]
+    tile, p = ways[loss.index(min(loss))]
     return tile[:2], p
 
 

@@ -720,6 +720,37 @@ def test_encoder_norms_inside_products(lib, B, S, heads, inner):
     assert got.isfinite().all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("B,S,lengths", [
+    (3, 214, [214, 0, 1]), (9, 77, [77, 76, 64, 65, 1, 0, 13, 500, -3]),
+    (2, 512, [1, 512]), (1500, 2, None),         # tiles of 64 x 64
+    (64, 50, None), (40, 200, None), (7, 512, [512, 0, 0, 0, 0, 0, 129])])
+def test_encoder_of_the_rows_that_texts_have(lib, B, S, lengths):
+    """Against all rows with padding; a length is taken at 0 and S where it is less
+    or more, and nobody is asked for the rows behind it."""
+    from fei_amd.models.bge import BgeEncoder
+    m = BgeEncoder(device=torch.device(DEV))
+    g = torch.Generator().manual_seed(B)
+    if lengths is None:
+        lengths = torch.randint(0, S + 1, (B,), generator=g).tolist()
+    ids = torch.randint(0, 1000, (B, S), generator=g).to(DEV)
+    n = torch.tensor(lengths, device=DEV)
+    called = []
+    packed, lib.encoder_packed = lib.encoder_packed, \
+        lambda *a: called.append(packed(*a)) or called[-1]
+    try:
+        got = m.encode_ids(ids, n)
+        lib.encoder_packed = lambda *a: None
+        want = m.encode_ids(ids, n.clamp(0, S))
+    finally:
+        lib.encoder_packed = packed
+    assert called[0] is not None
+    empty = n <= 0
+    assert not got[empty].any()
+    # as between the paths for all rows
+    assert row_err(got[~empty], want[~empty].double()) < 2.0 ** -5
+    assert got.isfinite().all()
+
+
 @pytest.mark.parametrize("gelu", [False, True])
 @pytest.mark.parametrize("M,N,K", [(33, 4, 64), (64, 768, 3072), (65, 100, 128),
                                    (500, 2304, 768)])
