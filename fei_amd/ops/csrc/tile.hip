@@ -31,6 +31,19 @@ struct TileArgs {
   int M, N, K, nx, parts;
 };
 
+// A tile's columns of out, and of W a half of them for gates where there are gates.
+template <int WM, int XI, int WI, int EPI>
+struct Shape {
+  static constexpr int rows = 32 * WM * XI, width = 32 * (8 / WM) * WI;
+  static constexpr int columns = EPI == TILE_SWIGLU ? width / 2 : width;
+};
+
+// A block's part of the work: of its XCD's tiles from id ``first`` on, each in MC * NC
+// pieces, ``count`` in all.
+struct Share {
+  int first, count;
+};
+
 // A block: 8 waves, two on a SIMD, that share tiles of 32 WM XI rows of x and
 // 32 WN WI rows of W (SWIGLU: half of them gates, the others the same of up),
 // WN = 8 / WM, 64 steps of K at a time. Both operands come in halves; a wave has
@@ -63,36 +76,38 @@ struct TileArgs {
 // Against the library, us: 2 x 14336 x 4096 of 2048 rows with SwiGLU 348 (360 + 33
 // for the pass of its own); 3072 x 768 of 16384 with bias and GELU 104 to
 // 109 (68.5 + 52); 4096 x 14336 of 2048 in two parts 170 (204); 8192^3 706 (700).
-template <int WM, int XI, int WI, int EPI>
-__global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
+//
+// B: the Shape in which tiles are counted.
+template <typename B, int WM, int XI, int WI, int EPI>
+__device__ __forceinline__ void run_tiles(const TileArgs& g, const Share share,
+                                          u16* const buf, int M, int nm) {
+  typedef Shape<WM, XI, WI, EPI> P;
   constexpr int WN = 8 / WM;
   constexpr int HA = 16 * WM * XI, HB = 16 * WN * WI;   // rows of a half
   constexpr int TM = 2 * HA, TN = 2 * HB;
   constexpr int PA = HA / 32, PB = HB / 32;             // loads of a wave
   constexpr bool PAIR = EPI == TILE_SWIGLU;
-  constexpr int CN = PAIR ? HB : TN;                    // columns of out
-  constexpr int STAGE = (TM + TN) * 64;
-  extern __shared__ __align__(16) u16 buf[];
-  u16* const lbias = buf + 2 * STAGE;                   // [4 tiles][512]
   constexpr bool BIAS = EPI == TILE_GELU || EPI == TILE_BIAS;
-  const int M = g.rows ? uniform(min(*g.rows, g.M)) : g.M;
-  const int N = g.N, K = g.K, parts = g.parts, nm = (M + TM - 1) / TM;
-  const int total = g.nx * nm, tiles = total * parts, per = (tiles + 7) / 8;
+  constexpr int STAGE = (TM + TN) * 64;
+  constexpr int MC = B::rows / P::rows, NC = B::columns / P::columns;
+  u16* const lbias = buf + 2 * STAGE;                   // [4 tiles][512]
+  const int N = g.N, K = g.K, parts = g.parts;
+  const int total = g.nx * nm;
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, slots = gridDim.x >> 3;
-  const int lim = min(per, tiles - xcd * per);          // tiles of the XCD
+  const int lim = share.count;
   if (slot >= lim) return;
   const int all = K / 64;
   const bool spread = (long)M * K <= 2 << 20;
   struct Tile { int m0, n0, part, first, steps, turn; };
   auto locate = [&](int i) __attribute__((always_inline)) {
     Tile t;
-    int id = xcd * per + i;
+    int id = share.first + i / (MC * NC);
     t.part = uniform(id / total);
     id -= t.part * total;
     const int g0 = uniform(id / (8 * g.nx)) * 8, gm = min(8, nm - g0);
     const int gr = id - g0 * g.nx, c = uniform(gr / gm);
-    t.n0 = c * CN;
-    t.m0 = (g0 + gr - c * gm) * TM;
+    t.n0 = c * B::columns + i % NC * P::columns;
+    t.m0 = (g0 + gr - c * gm) * B::rows + i / NC % MC * P::rows;
     t.first = uniform((int)((u32)(t.part * all) / (u32)parts));
     t.steps = uniform((int)((u32)((t.part + 1) * all) / (u32)parts)) - t.first;
     t.turn = uniform((u32)(xcd * t.steps / 8 + (spread ? 3 * c : 0)) % (u32)t.steps);
@@ -339,29 +354,62 @@ __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
     barrier();
     run(Second{});
   }
+}
+
+// MC * NC = 2: where an XCD's CUs have a last round of tiles for half of them or less, its
+// tiles are cut, rows or columns, so that all CUs have one. A kernel of its own: where
+// nothing is cut the other is faster by 1 to 2 us of 35 to 300. Us, uncut and cut: 2 x
+// 6144 x 2048 with SwiGLU, 1301 rows 70, 66; 2304 x 768 with bias and GELU, 10336 rows
+// 61, 56; 3072 x 768, 6144 rows 48, 46; 2 x 14336 x 4096, 2048 rows, 3 1/2 rounds 362,
+// 361 by itself, 9 less in a model's layers: with CUs idle the others keep a higher clock,
+// so that a long round gains little.
+template <int WM, int XI, int WI, int EPI, int MC, int NC>
+__global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
+  typedef Shape<WM, XI, WI, EPI> B;
+  extern __shared__ __align__(16) u16 buf[];
+  const int M = g.rows ? uniform(min(*g.rows, g.M)) : g.M;
+  const int nm = (M + B::rows - 1) / B::rows;
+  const int tiles = g.nx * nm * g.parts, per = (tiles + 7) / 8;
+  const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
+  const int lim = min(per, tiles - xcd * per);          // tiles of the XCD
+  const int rest = MC * NC > 1 && lim > 0 ? uniform(lim % slots) : 0;
+  const int cut = rest * MC * NC <= slots ? rest : 0;
+  run_tiles<B, WM, XI, WI, EPI>(g, Share{xcd * per, lim - cut}, buf, M, nm);
+  if (MC * NC > 1 && cut) {
+    // what is in LDS has been read
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    run_tiles<B, WM, XI / MC, WI / NC, EPI>(
+        g, Share{xcd * per + lim - cut, cut * MC * NC}, buf, M, nm);
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int WM, int XI, int WI, int EPI>
+template <int WM, int XI, int WI, int EPI, int MC = 1, int NC = 1>
 void launch(TileArgs g, hipStream_t stream) {
-  constexpr int TM = 32 * WM * XI, TN = 32 * (8 / WM) * WI;
-  constexpr int CN = EPI == TILE_SWIGLU ? TN / 2 : TN;
-  constexpr int lds = 2 * (TM + TN) * 128 + 4096;
-  allow_lds(k_tile<WM, XI, WI, EPI>, lds);
-  g.nx = (g.N + CN - 1) / CN;
-  const long nm = (g.M + TM - 1) / TM;
-  // a block a CU
-  const int blocks = std::min(256L, (nm * g.nx * g.parts + 7) / 8 * 8);
-  hipLaunchKernelGGL((k_tile<WM, XI, WI, EPI>), dim3(blocks), dim3(512), lds,
-                     stream, g);
+  typedef Shape<WM, XI, WI, EPI> B;
+  constexpr int lds = 2 * (B::rows + B::width) * 128 + 4096;
+  g.nx = (g.N + B::columns - 1) / B::columns;
+  const long nm = (g.M + B::rows - 1) / B::rows;
+  const long per = (nm * g.nx * g.parts + 7) / 8;       // tiles of an XCD
+  const int slots = (int)std::min(32L, per);            // a block a CU
+  auto go = [&](auto kernel) {
+    allow_lds(kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3(8 * slots), dim3(512), lds, stream, g);
+  };
+  const int rest = (int)(per % slots);
+  // where only the device knows the rows, it may have a rest
+  if (MC * NC > 1 && (g.rows || (rest && rest * MC * NC <= slots)))
+    go(k_tile<WM, XI, WI, EPI, MC, NC>);
+  else
+    go(k_tile<WM, XI, WI, EPI, 1, 1>);
 }
 
 template <int EPI>
 void by_size(int rows, int width, const TileArgs& g, hipStream_t stream) {
-  if (rows == 192) launch<2, 3, 2, EPI>(g, stream);
+  if (rows == 192) launch<2, 3, 2, EPI, 1, 2>(g, stream);
   else if (rows == 128) launch<2, 2, 2, EPI>(g, stream);
-  else if (width == 256) launch<2, 4, 2, EPI>(g, stream);
-  else if (width == 192) launch<4, 2, 3, EPI>(g, stream);
+  else if (width == 256) launch<2, 4, 2, EPI, 2, 1>(g, stream);
+  else if (width == 192) launch<4, 2, 3, EPI, 2, 1>(g, stream);
   else launch<4, 2, 2, EPI>(g, stream);
 }
 

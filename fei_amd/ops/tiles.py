@@ -155,11 +155,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def _launch(out, x, w, N, epi, size, bias=None, parts=1) -> None:
+def _launch(out, x, w, N, epi, size, bias=None, parts=1, rows=None) -> None:
     M, K = x.shape
     _ops.require_lib().fei_tile(
         _p(out), out.stride(-2), _p(x), x.stride(0), _p(w), _p(bias), M, N, K,
-        epi, *size, parts, None, _ops._stream())
+        epi, *size, parts, _p(rows), _ops._stream())
 
 
 def parts_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -127,6 +127,30 @@ def test_tile(M, N, K, size):
         assert err(parts.double().sum(0), g) < 2 ** -24 * max(K ** 0.5, 16)
 
 
+# a few tiles more than the CUs have in whole rounds, which are run in halves: of rows
+# where the last tile has rows for one half alone, and for more; of columns
+@pytest.mark.gpu
+@pytest.mark.parametrize("size,M,N", [((256, 256), 2400, 6664), ((256, 256), 2500, 6664),
+                                      ((256, 192), 2400, 5192), ((192, 256), 2500, 4872),
+                                      ((192, 256), 2500, 5000)])
+@pytest.mark.parametrize("K", [64, 192, 1088])
+@pytest.mark.parametrize("count", [None, 0, 1, 600, 2399, 9999])
+def test_last_round_in_halves(size, M, N, K, count):
+    x, w, b = (rand(M, K, seed=1), rand(2 * N, K, seed=2, scale=K ** -0.5),
+               rand(N, seed=3))
+    n = M if count is None else min(count, M)
+    rows = None if count is None else torch.tensor([count], dtype=torch.int32,
+                                                   device=DEV)
+    y = x[:n].double() @ w.double().t()
+    for epi, bias, want in ((tiles.TILE_BIAS, b, y[:, :N] + b.double()),
+                            (tiles.TILE_SWIGLU, None, F.silu(y[:, :N]) * y[:, N:])):
+        out = torch.full((M, N), 7.0, device=DEV, dtype=torch.bfloat16)
+        ww = w if epi == tiles.TILE_SWIGLU else w[:N]
+        tiles._launch(out, x, ww, N, epi, size, bias, rows=rows)
+        assert n == 0 or err(out[:n], want) < 2 ** -9     # a result is rounded once
+        assert bool((out[n:] == 7).all())
+
+
 @pytest.mark.gpu
 def test_activations_of_every_value():
     """All of bfloat16, and infinities and NaN that sums come to (as no factor, which
