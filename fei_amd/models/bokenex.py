@@ -140,13 +140,17 @@ class BokenexModel(StepModel):
         s, dt = self.spec, self.dtype
         x = ops.embed_pos(batch.tokens, batch.pos, self.emb, self.pos_emb)
         rows = None
+        few = self._few_wanted(batch, on_run)
         for r, (lw, L) in enumerate(zip(self.layers, s.layers)):
             n_mix, mlp = L.mixer.out_cols, lw.mlp
             ff = mlp.act_cols if mlp is not None else 0
-            cat = torch.empty(x.shape[0], n_mix + ff, dtype=dt,
-                              device=x.device)
             h = ops.GainNormed(x, lw.norm, dt, rows)
             rows = None
+            if few and r + 1 == len(self.layers):
+                x = self._last_layer(h, lw, L, batch, cache, r)
+                break
+            cat = torch.empty(x.shape[0], n_mix + ff, dtype=dt,
+                              device=x.device)
             proj, router = ops.parallel_in(
                 h, lw.w_in, L.mixer.in_rows, ff,
                 mlp.router_rows if mlp is not None else 0, cat[:, n_mix:])
@@ -164,7 +168,29 @@ class BokenexModel(StepModel):
                                      mlp.down, mlp.f, s.residual_mult)
             if on_run is not None:
                 on_run(r, x)
-        if batch.want_rows is not None:
+        if batch.want_rows is not None and not few:
             x = x[batch.want_rows]
         return ops.gain_logits(ops.GainNormed(x, self.norm_f, dt),
                                self.lm_head)
+
+    def _last_layer(self, h, lw, L, batch, cache, r) -> torch.Tensor:
+        """The last layer's residual of the wanted rows alone."""
+        want, mlp, n_in = batch.want_rows, lw.mlp, L.mixer.in_rows
+        n_mix, dt, mult = L.mixer.out_cols, self.dtype, self.spec.residual_mult
+        mixed = torch.empty(h.x.shape[0], n_mix, dtype=dt, device=h.x.device)
+        proj, _ = ops.parallel_in(h, lw.w_in, n_in, 0, 0, mixed)
+        lw.mixer.run(proj, mixed, batch, cache, r, {})
+        x = h.x[want]
+        if not want.shape[0]:
+            return x
+        ff = mlp.act_cols if mlp is not None else 0
+        cat = torch.empty(x.shape[0], n_mix + ff, dtype=dt, device=x.device)
+        cat[:, :n_mix] = mixed[want]
+        h, router = ops.GainNormed(x, lw.norm, dt), None
+        if mlp is not None:
+            _, router = ops.parallel_in(h, lw.w_in[n_in:], 0, ff, mlp.router_rows,
+                                        cat[:, n_mix:])
+        if router is None:
+            return ops.residual_linear(x, cat, lw.w_out, mult)
+        return ops.residual_moe(x, h, router, cat, lw.w_out, mlp.up, mlp.down,
+                                mlp.f, mult)

@@ -75,6 +75,16 @@ class StepModel:
     def forward(self, batch, cache: HybridCache, on_run=None) -> torch.Tensor:
         raise NotImplementedError
 
+    def _few_wanted(self, batch, on_run) -> bool:
+        """Whether the last layer run leaves out what only rows make that nobody asks
+        logits of: all but what its mixer keeps and mixes. To take the wanted rows out
+        costs four launches of 3 us; 1301 rows in 16 layer runs gain 140 us of 5260, 1706
+        in 16 layers 70 of 4510; up to some hundred rows the products cost what their
+        weights do."""
+        want = batch.want_rows
+        return (on_run is None and want is not None and bool(batch.portions)
+                and batch.n_rows >= 128 and 4 * want.shape[0] <= batch.n_rows)
+
     # -- weights -------------------------------------------------------------
 
     def _read(self, path: str) -> Get:

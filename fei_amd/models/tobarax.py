@@ -149,6 +149,7 @@ class TobaraxModel(StepModel):
         x0 = x.clone() if s.loop is not None else None
         normed = None
         runs = s.runs            # made anew each time
+        few = self._few_wanted(batch, on_run)
         for r, run in enumerate(runs):
             if run.enters_pass is not None:
                 x = ops.linear_f32(ops.cat_cast(x, x0, dt), self.loop_in,
@@ -157,6 +158,9 @@ class TobaraxModel(StepModel):
             n1, n2 = normed or ops.norm_pair(x, lw.norm1, lw.norm2, s.norm_eps,
                                              dt)
             n_mix, ff = L.mixer.out_cols, L.ff or 0
+            if few and r + 1 == len(runs):
+                x = self._last_run(x, n1, n2, lw, L, batch, cache, r)
+                break
             cat = torch.empty(x.shape[0], n_mix + ff, dtype=dt,
                               device=x.device)
             proj = ops.mix_in(n1, n2, lw.w_in, L.mixer.in_rows, ff,
@@ -172,8 +176,25 @@ class TobaraxModel(StepModel):
                 x, normed = ops.residual_linear(x, cat, lw.w_out), None
             if on_run is not None:
                 on_run(r, x)
-        if batch.want_rows is not None:
+        if batch.want_rows is not None and not few:
             x = x[batch.want_rows]
         y, _ = ops.norm_pair(x, self.norm_f, None, s.norm_eps, dt)
         return ops.logits_head(y, self.lm_head, s.logit_scale,
                                s.logit_softcap)
+
+    def _last_run(self, x, n1, n2, lw, L, batch, cache, r) -> torch.Tensor:
+        """The last run's residual of the wanted rows alone."""
+        want, n_mix, ff = batch.want_rows, L.mixer.out_cols, L.ff or 0
+        T, n, dt = x.shape[0], want.shape[0], self.dtype
+        mixed = torch.empty(T, n_mix, dtype=dt, device=x.device)
+        proj = ops.mix_in(n1, None, lw.w_in, L.mixer.in_rows, 0, mixed)
+        lw.mixer.run(proj, mixed, batch, cache, r, self._rot)
+        x = x[want]
+        if not n:
+            return x
+        cat = torch.empty(n, n_mix + ff, dtype=dt, device=x.device)
+        cat[:, :n_mix] = mixed[want]
+        if ff:
+            n2 = n2[want]
+            ops.mix_in(n2, n2, lw.w_in[L.mixer.in_rows:], 0, ff, cat[:, n_mix:])
+        return ops.residual_linear(x, cat, lw.w_out)

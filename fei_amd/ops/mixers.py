@@ -259,7 +259,8 @@ def mix_in(n1: torch.Tensor, n2: Optional[torch.Tensor], w_in: torch.Tensor,
         n2.shape == n1.shape and plain(n2, w_in) and n2.data_ptr() % 16 == 0))
     if own and skinny_ok(T, K, n1, w_in):
         proj = torch.empty(T, n_mix, dtype=n1.dtype, device=n1.device)
-        skinny(proj, n1, w_in, n_mix, EPI_BF16)
+        if n_mix:
+            skinny(proj, n1, w_in, n_mix, EPI_BF16)
         if ff:
             skinny(None, n2, w_in[n_mix:], ff, EPI_SWIGLU, act=act,
                    stride=act.stride(0))

@@ -665,6 +665,35 @@ def test_prompt_in_parts_matches_whole_products(lib, B, S):
         assert row_err(x.flatten(), y.double().flatten()) < 2.0 ** -6
 
 
+# in parts and by whole products, up to the rows that the last layer's kernels for few
+# take, and one more
+@pytest.mark.parametrize("layers", [1, 2])
+@pytest.mark.parametrize("B,S", [(1, 33), (2, 65), (1, 300), (3, 257), (32, 2), (32, 9),
+                                 (33, 9), (5, 1)])
+def test_last_layer_of_a_prompt(lib, B, S, layers):
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+    spec = dataclasses.replace(get_spec("llama3-1b"), num_layers=layers,
+                               vocab_size=512)
+    m = LlamaModel(spec, torch.device(DEV), torch.bfloat16, seed=1,
+                   max_seq_len=640)
+    toks = torch.randint(0, 512, (B, S), device=DEV)
+    pos0 = torch.arange(B, dtype=torch.int32, device=DEV) * 3
+    new = randbf(layers, B, spec.num_kv_heads, 640, m.D, seed=2)
+
+    def run(everything):
+        kc, vc = new.clone(), -new
+        y = m.forward_prefill(toks, pos0, list(kc), list(vc),
+                              all_positions=everything)
+        return y[:, -1] if everything else y, kc, vc
+    (a, ka, va), (b, kb, vb) = run(False), run(True)
+    assert a.shape == b.shape
+    # one layer's roundings, 2^-9 each, fall otherwise
+    assert row_err(a, b.double()) < 2.0 ** -6
+    assert torch.equal(ka, kb) and torch.equal(va, vb)
+
+
 @pytest.mark.parametrize("B,S,lengths", [(1, 4, None), (1, 24, None),
                                          (4, 8, [8, 1, 3, 5]), (2, 16, [16, 9]),
                                          (32, 1, None), (1, 33, None),

@@ -384,6 +384,49 @@ def test_far_key_among_many(tmp_path, device):
 # -- batches, blocks and slots ---------------------------------------------------------
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_few_wanted_rows(tmp_path, name, device):
+    """The last layer makes the wanted rows alone, if they are few: none, the
+    counts that the products for few rows part at, one twice; and what it keeps is
+    kept of all rows."""
+    net = Net(tmp_path, CONFIGS[name], 41, device)
+    V = net.cfg["vocab"]
+    a, b, c = toks(150, V, 5), toks(60, V, 6), toks(31, V, 7)
+    want = {i: net.want(t) for i, t in enumerate((a, b, c))}
+    for n in (0, 1, 2, 3, 8, 40):
+        r = net.runner()
+        sa, sb, sc = r.admit(), r.admit(), r.admit()
+        r.step([StepEntry(sc, c[:30])])
+        rows = [149, 149, 0][:n] + list(range(1, max(n - 2, 1)))
+        got = r.step([StepEntry(sa, a, rows),
+                      StepEntry(sb, b[:59], [58]), StepEntry(sc, c[30:], [0])])
+        ref = torch.cat([want[0][rows], want[1][58:59], want[2][30:31]])
+        assert err(got, ref) < F32_TOL, n
+        got = r.step([StepEntry(sb, b[59:], [0])])
+        assert err(got, want[1][59:60]) < F32_TOL, n
+        r = net.runner()
+        sa = r.admit()
+        assert r.step([StepEntry(sa, a[:149])]).shape == (0, V)
+        assert err(r.step([StepEntry(sa, a[149:], [0])]), want[0][149:]) < F32_TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(CONFIGS))
+def test_few_wanted_rows_in_bfloat16(tmp_path, name):
+    """Against all rows' logits; the products take other kernels, so that roundings
+    of the last layer differ: of its inputs, 2^-9 each."""
+    net = Net(tmp_path, CONFIGS[name], 41, "cuda", torch.bfloat16)
+    a, b = toks(150, net.cfg["vocab"], 8), toks(50, net.cfg["vocab"], 9)
+    for n in (1, 2, 3, 40):
+        r = net.runner()
+        pair = [r.admit(), r.admit(), r.admit(), r.admit()]
+        rows = list(range(150 - n, 150))
+        got = r.step([StepEntry(pair[0], a, rows), StepEntry(pair[1], b, [49])])
+        ref = r.step([StepEntry(pair[2], a), StepEntry(pair[3], b)], True)
+        assert err(got, ref[rows + [199]].cpu()) < 2 ** -6, n
+
+
+@pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("name", ["odd", "even"])
 def test_mixed_batches(tmp_path, name, device):
     """Unequal requests in one batch, portions beside single tokens, requests
