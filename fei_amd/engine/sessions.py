@@ -317,7 +317,10 @@ class PagedSessionManager:
                 pos, **args)
 
         if m.fused_rows(B):
-            sums = m.fused_layers(h, attend)
+            few = ops.llama_few(h, m.layers, self.pool.k, self.pool.v, m.hq_l, eps,
+                                pos, m.rope, self._splits(B), self._workspace(B),
+                                table)
+            sums = m.fused_layers(h, attend, *few)
             return ops.gemv_norm(h, m.norm_f, m.lm_head, eps, sums=sums)
         x = ops.rmsnorm(h, m.layers[0].norm_attn, eps)
         for li, lw in enumerate(m.layers):

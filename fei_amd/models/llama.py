@@ -258,12 +258,15 @@ class LlamaModel:
             token = token.long()
         return F.embedding(token, self.emb)
 
-    def fused_layers(self, h: torch.Tensor, attend) -> Optional[torch.Tensor]:
+    def fused_layers(self, h: torch.Tensor, attend, done: int = 0,
+                     sums: Optional[torch.Tensor] = None
+                     ) -> Optional[torch.Tensor]:
         """All layers over the residual ``h`` [rows, C], in place; fused_rows
         has to allow the rows. ``attend(layer, qkv)`` gives the attention's
-        output. Returns what a norm's product takes as ``sums``."""
-        eps, sums = self.spec.norm_eps, None
-        for li, lw in enumerate(self.layers):
+        output. ``done`` layers have been run already and left ``sums``. Returns
+        what a norm's product takes as ``sums``."""
+        eps = self.spec.norm_eps
+        for li, lw in enumerate(self.layers[done:], done):
             qkv = ops.gemv_norm(h, lw.norm_attn, lw.wqkv, eps, sums=sums)
             att = attend(li, qkv)
             sums = ops.add_product(att.reshape(h.shape[0], -1), lw.wo, h,
@@ -336,11 +339,16 @@ class LlamaModel:
         if ssq is not None:
             ssq.zero_()
         pf = self.prefetch_mb > 0 and fp8 is None and h.is_cuda
+        done = 0
+        if not (pf or fused_attn) and fp8 is ssq is attn_out is None:
+            done, sums = ops.llama_few(
+                h, self.layers, k_caches, v_caches, self.hq_l, s.norm_eps, pos,
+                self.rope, attn_splits, workspace)
         if pf and self._pf_stream is None:
             self._pf_stream = torch.cuda.Stream()
             self._pf_sink = torch.zeros(1, dtype=torch.float32,
                                         device=h.device)
-        for li, lw in enumerate(self.layers):
+        for li, lw in enumerate(self.layers[done:], done):
             if fp8 is not None:
                 q8 = fp8[li]
                 qkv = ops.gemv_norm_fp8(h, lw.norm_attn, *q8["wqkv"],
@@ -420,7 +428,9 @@ class LlamaModel:
                                     scale=scale)
 
         if self.fused_rows(B * S):
-            sums = self.fused_layers(h.view(B * S, -1), attend)
+            few = ops.llama_few(h.view(B * S, -1), self.layers, k_caches, v_caches,
+                                self.hq_l, s.norm_eps, pos0, self.rope, S=S)
+            sums = self.fused_layers(h.view(B * S, -1), attend, *few)
             if not all_positions and S > 1:
                 h, sums = h[:, -1, :], None
             elif not all_positions:

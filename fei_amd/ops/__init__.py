@@ -19,12 +19,14 @@ from typing import Optional, Tuple
 
 import torch
 
+from fei_amd.ops import layers as _layers
 from fei_amd.ops import mixers as _mixers
 from fei_amd.ops import moe as _moe
 from fei_amd.ops import reference as ref
 from fei_amd.ops import rows as _rows
 from fei_amd.ops import sigmoid_attn as _sigmoid_attn
 from fei_amd.ops import tiles as _tiles
+from fei_amd.ops.layers import llama_few  # noqa: F401
 from fei_amd.ops.mixers import (  # noqa: F401
     GainNorm, GainNormed, cat_cast, check_gla_geometry,
     check_latent_geometry, embed_pos, gain_logits, gla_decode, gla_prefill,
@@ -104,6 +106,7 @@ def _try_load() -> None:
     _mixers.declare(lib)
     _rows.declare(lib)
     _tiles.declare(lib)
+    _layers.declare(lib)
     _moe.declare(lib)
     _sigmoid_attn.declare(lib)
     _LIB = lib

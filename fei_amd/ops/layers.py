@@ -1,0 +1,119 @@
+"""Layers of a Llama-style decoder over few rows, each launched from one call
+(csrc/layers.hip). bfloat16 GPU tensors only."""
+
+from __future__ import annotations
+
+import ctypes
+import math
+from typing import Optional, Sequence, Tuple
+
+import torch
+
+import fei_amd.ops as _ops     # half made yet: it imports this
+from fei_amd.ops import tiles as _tiles
+from fei_amd.ops.mixers import SKINNY_ROWS
+
+_vp, _i, _f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+_BF16 = torch.bfloat16
+
+
+class _FewRows(ctypes.Structure):
+    """FewRows of csrc/layers.hip."""
+    _fields_ = ([(n, _i) for n in ("B", "S", "C", "I", "Hq", "Hkv", "D", "room",
+                                   "bs_log", "W", "splits")] +
+                [("eps", _f), ("scale", _f)] +
+                [(n, _vp) for n in ("pos", "table", "cos_sin", "po", "pml")])
+
+
+def declare(lib: ctypes.CDLL) -> None:
+    lib.fei_llama_few.argtypes = [_vp, _i] + [_vp] * 8
+
+
+def _pointers(tensors, shapes, device: int, grad: bool):
+    """Where kernels find the tensors, 16 bytes at a time, or None if one is not what
+    lies there."""
+    out = []
+    for t, shape in zip(tensors, shapes):
+        p = t.data_ptr()
+        if not (t.dtype is _BF16 and t.shape == shape and t.is_contiguous()
+                and t.get_device() == device and not p % 16
+                and _tiles.types_ok(t) and not (grad and t.requires_grad)):
+            return None
+        out.append(p)
+    return out
+
+
+def llama_few(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor],
+              v_caches: Sequence[torch.Tensor], heads: int, eps: float,
+              pos: torch.Tensor, rope: torch.Tensor, splits: int = 0,
+              workspace=None, table: Optional[torch.Tensor] = None, S: int = 0
+              ) -> Tuple[int, Optional[torch.Tensor]]:
+    """``layers`` over the rows h [M, C], in place: a decoding step's, or (``S``) those
+    of prompts of S tokens. Caches [B, Hkv, room, D], or with a ``table`` pools
+    [blocks, Hkv, size, D]; at pos[b] and on the rows' keys and values are written.
+    ``workspace``: see attn_decode. Returns how many layers are done, up to the first that
+    the kernels for few rows do not take, and what a norm's product behind them takes as
+    ``sums``. The launches, and their order, are those of the operations one by one. A
+    layer a call: the GPU has the first one's while the others are looked at (all 16 looked
+    at first, a step of 20 sessions took 1130 us, 1068 one by one)."""
+    M, C = h.shape
+    lw, grad = layers[0], torch.is_grad_enabled()
+    if not (h.is_cuda and 0 < M <= SKINNY_ROWS and 0 < C <= 16384
+            and k_caches[0].dim() == 4 and (not S or M % S == 0)):
+        return 0, None
+    Hkv, room, D = k_caches[0].shape[1:]
+    HD, width, I = heads * D, (heads + 2 * Hkv) * D, lw.wdown.shape[-1]
+    B, dev, bs_log, W = M // (S or 1), h.get_device(), 0, 0
+    cache = k_caches[0].shape if table is not None else (B, Hkv, room, D)
+    if not (dev == torch.cuda.current_device() and D in (64, 128) and I > 0 < Hkv
+            and heads % Hkv == 0 and heads // Hkv <= 16
+            and not any(n % (64 if M > 1 else 8) for n in (C, HD, I))
+            and _pointers((h,), ((M, C),), dev, grad)
+            and rope.dtype is torch.float32 and pos.dtype is torch.int32
+            and pos.is_contiguous() and rope.is_contiguous()
+            and pos.get_device() == rope.get_device() == dev and pos.numel() == B
+            and not rope.data_ptr() % 16 and _tiles._memory(pos, rope)):
+        return 0, None
+    if table is not None:
+        if not (table.dtype is torch.int32 and table.is_contiguous()
+                and table.shape[0] == B and table.get_device() == dev
+                and not room & (room - 1) and not S):
+            return 0, None
+        bs_log, W = room.bit_length() - 1, table.shape[1]
+        room = W << bs_log
+    if S:
+        splits = _ops._prefill_splits(B, Hkv, S * (heads // Hkv), room)
+        n = M * heads * splits if splits > 1 else 0
+        ws = torch.empty(n * (D + 2), dtype=torch.float32, device=h.device)
+        po, pml = ws.data_ptr(), ws.data_ptr() + n * D * 4
+    else:
+        if not 0 < splits <= 64:
+            return 0, None
+        if workspace is None:
+            workspace = [torch.empty(B, heads, splits, n, dtype=torch.float32,
+                                     device=h.device) for n in (D, 2)]
+        po, pml = (t.data_ptr() for t in workspace)
+        assert all(t.shape[2] == splits for t in workspace)
+
+    def rows(n):
+        return torch.empty(M, n, dtype=h.dtype, device=h.device)
+    room_for = [rows(n) for n in (width, HD, I, C)]
+    sums = torch.empty(M, -(-C // (8 if C <= 2048 else 16)), dtype=torch.float32,
+                       device=h.device)
+    p = _FewRows(B, S, C, I, heads, Hkv, D, room, bs_log, W, splits, eps,
+                 1.0 / math.sqrt(D), pos.data_ptr(),
+                 None if table is None else table.data_ptr(), rope.data_ptr(), po,
+                 pml)
+    args = (h.data_ptr(), *(t.data_ptr() for t in room_for), sums.data_ptr(),
+            ctypes.byref(p), _ops._stream())
+    launch = _ops.require_lib().fei_llama_few
+    shapes = ((C,), (width, C), (C, HD), (C,), (2 * I, C), (C, I), cache, cache)
+    done = 0
+    for lw, kc, vc in zip(layers, k_caches, v_caches):
+        at = _pointers((lw.norm_attn, lw.wqkv, lw.wo, lw.norm_mlp, lw.wgu, lw.wdown,
+                        kc, vc), shapes, dev, grad)
+        if at is None:
+            break
+        launch((_vp * 8)(*at), done, *args)
+        done += 1
+    return done, sums if done and M > 1 else None

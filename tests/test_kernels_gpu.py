@@ -665,6 +665,46 @@ def test_prompt_in_parts_matches_whole_products(lib, B, S):
         assert row_err(x.flatten(), y.double().flatten()) < 2.0 ** -6
 
 
+# one row, one and more groups of 8, prompts and decoding steps; ``odd``: a layer whose
+# weights the kernels for few rows do not read as they lie, from which on the operations
+# run one by one
+@pytest.mark.parametrize("name", ["llama3-1b", "wide"])
+@pytest.mark.parametrize("B,S", [(1, 0), (2, 0), (9, 0), (32, 0), (1, 1), (1, 32),
+                                 (3, 7), (33, 0)])
+@pytest.mark.parametrize("odd", [None, 0, 1])
+def test_layers_of_few_rows_from_one_call(lib, name, B, S, odd, monkeypatch):
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+    sizes = dict(hidden_size=2112, num_heads=8, num_kv_heads=4, head_dim=128,
+                 intermediate_size=448) if name == "wide" else {}
+    spec = dataclasses.replace(get_spec("llama3-1b"), num_layers=3, vocab_size=512,
+                               **sizes)
+    m = LlamaModel(spec, torch.device(DEV), torch.bfloat16, seed=1,
+                   max_seq_len=640)
+    if odd is not None:
+        w = m.layers[odd].wdown
+        m.layers[odd].wdown = torch.cat([w, w], 1)[:, :w.shape[1]]
+    toks = torch.randint(0, 512, (B, S) if S else (B,), device=DEV)
+    pos = torch.arange(B, dtype=torch.int32, device=DEV) * 13 % 500
+    new = randbf(3, B, spec.num_kv_heads, 640, m.D, seed=2)
+    done, few = [], lib.llama_few
+
+    def run(one_call):
+        monkeypatch.setattr(lib, "llama_few", lambda *a, **k: done.append(
+            few(*a, **k) if one_call else (0, None)) or done[-1])
+        kc, vc = new.clone(), -new
+        if S:
+            return m.forward_prefill(toks, pos, list(kc), list(vc)), kc, vc
+        return m.forward_decode(toks, pos, list(kc), list(vc)), kc, vc
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a, b)
+    # the layers before the odd one; none where it is the first, whose weights say
+    # whether this chain is taken at all
+    assert [d for d, _ in done] == ([] if B > 32 or odd == 0
+                                    else [3 if odd is None else odd, 0])
+
+
 # in parts and by whole products, up to the rows that the last layer's kernels for few
 # take, and one more
 @pytest.mark.parametrize("layers", [1, 2])
