@@ -40,6 +40,18 @@ __device__ __forceinline__ int channels(const Geo& g) {
   return g.heads * g.dim + g.kvh * (g.dim + g.vdim);
 }
 
+// Sum over the 8 lanes 8i .. 8i + 7: of pairs, of fours, of a half row and its mirror.
+__device__ __forceinline__ float half16_sum(float v) {
+  auto swap = [](float x, auto ctrl) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                           decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  v += swap(v, std::integral_constant<int, 0xb1>{});
+  v += swap(v, std::integral_constant<int, 0x4e>{});
+  return v + swap(v, std::integral_constant<int, 0x141>{});
+}
+
 // Per-head norm of a group's LG x 8 values of which n count.
 template <int LG>
 __device__ __forceinline__ void head_norm(float (&y)[8], int n, float eps,
@@ -47,7 +59,8 @@ __device__ __forceinline__ void head_norm(float (&y)[8], int n, float eps,
   float ss = 0.f;
 #pragma unroll
   for (int j = 0; j < 8; ++j) ss = fmaf(y[j], y[j], ss);
-  ss = row16_sum(ss);
+  if (LG == 8) ss = half16_sum(ss);
+  else ss = row16_sum(ss);
   if (LG == 32) ss += __shfl_xor(ss, 16);
   const float inv = 1.f / sqrtf(ss / (float)n + eps);
 #pragma unroll
@@ -55,20 +68,23 @@ __device__ __forceinline__ void head_norm(float (&y)[8], int n, float eps,
 }
 
 // Convolution and norms of prompt rows: queries to q, keys and values to
-// their cache rows. A group of LG lanes takes one head of RUN rows one after
-// another, a lane 8 of its channels: the weights and the TAPS - 1 projections
-// before a row stay in registers. spans [.][3]: first row, rows, first
-// position. Sizes are multiples of 8.
-constexpr int RUN = 8;
+// their cache rows. A group of LG lanes takes one head of RUN rows, a lane 8 of its
+// channels: the weights, the rows and the TAPS - 1 before them are in registers, all asked
+// for at once. Sizes are multiples of 8. Bound by the latency of a launch, a row's
+// sequence and its cache row's block: 1700 rows of 48 heads of 64, 4 taps, 9.4 us, of 8
+// rows a group 10.8; with each row's loads behind the row before, and half of the lanes
+// idle, 14.2.
+constexpr int RUN = 4;
 
 template <typename T, int LG, int TAPS>
 __global__ void __launch_bounds__(256)
 k_sig_conv_run(T* __restrict__ q, const T* __restrict__ proj, long ps,
                T* __restrict__ rows, const float* __restrict__ states,
-               Conv cv, const int* __restrict__ spans,
-               const int* __restrict__ row_seq, const int* __restrict__ pos,
-               const int* __restrict__ slots, const int* __restrict__ table,
-               int n_rows, int seq0, int W, int bs_log, Geo g) {
+               Conv cv, const int* __restrict__ row_seq,
+               const int* __restrict__ pos, const int* __restrict__ slots,
+               const int* __restrict__ table, int n_rows, int seq0, int W,
+               int bs_log, Geo g) {
+  constexpr int B = TAPS - 1;
   const int units = g.heads + 2 * g.kvh;
   const int item = blockIdx.x * (256 / LG) + threadIdx.x / LG;
   const int t0 = item / units * RUN, u = item % units;
@@ -82,7 +98,19 @@ k_sig_conv_run(T* __restrict__ q, const T* __restrict__ proj, long ps,
   const int c = (threadIdx.x & (LG - 1)) * 8;
   const bool on = c < n;
   const int ch = ch0 + (on ? c : 0);
-  float w[TAPS][8], wn[8], past[TAPS][8];  // past[a]: a rows back; [0] unused
+  // rows t0 - B .. t0 + RUN - 1; those of another sequence than a row's do not count
+  // for it
+  int seq[RUN + B], p[RUN];
+  typename El<T>::frag x[RUN + B];
+#pragma unroll
+  for (int i = 0; i < RUN + B; ++i) {
+    const int row = seq0 + t0 + i - B, at = min(max(row, 0), seq0 + n_rows - 1);
+    seq[i] = row_seq[at];
+    if (i >= B) p[i - B] = pos[at];
+    x[i] = ld8(proj + (long)at * ps + ch);
+    if (row < 0) seq[i] = -1;
+  }
+  float w[TAPS][8], wn[8];
 #pragma unroll
   for (int i = 0; i < TAPS; ++i) {
     const f32x8 v = ld8(cv.w + (long)i * CH + ch);
@@ -94,55 +122,43 @@ k_sig_conv_run(T* __restrict__ q, const T* __restrict__ proj, long ps,
 #pragma unroll
     for (int j = 0; j < 8; ++j) wn[j] = v[j];
   }
-  int last = -1;
+  long to[RUN];
+#pragma unroll
+  for (int k = 0; k < RUN; ++k)
+    to[k] = is_q ? (long)(t0 + k) * g.heads * g.dim + ch
+                 : cache_row(table, W, seq[k + B], p[k], bs_log) * R +
+                       (ch - g.heads * g.dim);
 #pragma unroll
   for (int k = 0; k < RUN; ++k) {
-    const int t = t0 + k;
-    if (t >= n_rows) return;
-    const int row = seq0 + t, seq = row_seq[row], p = pos[row];
-    if (seq != last) {                     // the run or a portion starts
-      last = seq;
-      const int row0 = spans[(seq - seq0) * 3];
-#pragma unroll
-      for (int a = 1; a < TAPS; ++a) {
-        if (row - a >= row0) {
-          const auto v = ld8(proj + (long)(row - a) * ps + ch);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) past[a][j] = get8(v, j);
-        } else if (p - a >= 0) {
-          const f32x8 v = ld8(states + ((long)slots[seq] * TAPS +
-                                        (p - a) % TAPS) * CH + ch);
-#pragma unroll
-          for (int j = 0; j < 8; ++j) past[a][j] = v[j];
-        } else {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) past[a][j] = 0.f;
-        }
-      }
-    }
-    const auto v = ld8(proj + (long)row * ps + ch);
+    if (t0 + k >= n_rows) return;
     float y[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float x = get8(v, j);
-      y[j] = 0.f;
+    for (int j = 0; j < 8; ++j) y[j] = 0.f;
 #pragma unroll
-      for (int a = TAPS - 1; a > 0; --a)
-        y[j] = fmaf(w[TAPS - 1 - a][j], past[a][j], y[j]);
-      y[j] = on ? fmaf(w[TAPS - 1][j], x, y[j]) : 0.f;
+    for (int a = B; a > 0; --a) {
+      if (seq[k + B - a] == seq[k + B]) {
 #pragma unroll
-      for (int a = TAPS - 1; a > 1; --a) past[a][j] = past[a - 1][j];
-      if (TAPS > 1) past[TAPS > 1 ? 1 : 0][j] = x;
+        for (int j = 0; j < 8; ++j)
+          y[j] = fmaf(w[B - a][j], get8(x[k + B - a], j), y[j]);
+      } else if (p[k] >= a) {              // a portion starts
+        const f32x8 v = ld8(states + ((long)slots[seq[k + B]] * TAPS +
+                                      (p[k] - a) % TAPS) * CH + ch);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[j] = fmaf(w[B - a][j], v[j], y[j]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) y[j] = fmaf(w[B - a][j], 0.f, y[j]);
+      }
     }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      y[j] = on ? fmaf(w[B][j], get8(x[k + B], j), y[j]) : 0.f;
     if (!is_v) head_norm<LG>(y, n, cv.eps, wn);
     if (on) {
-      T* dst = is_q ? q + (long)t * g.heads * g.dim + ch
-                    : rows + cache_row(table, W, seq, p, bs_log) * R +
-                          (ch - g.heads * g.dim);
       typename El<T>::frag o;
 #pragma unroll
       for (int j = 0; j < 8; ++j) o[j] = El<T>::st(y[j]);
-      st8(dst, o);
+      st8((is_q ? q : rows) + to[k], o);
     }
   }
 }
@@ -815,11 +831,13 @@ void run_conv(T* q, const T* proj, long ps, T* rows, float* states, Conv cv,
 #define CONV_RUN(LG, TAPS)                                                   \
   hipLaunchKernelGGL((k_sig_conv_run<T, LG, TAPS>),                          \
                      dim3((runs + 256 / LG - 1) / (256 / LG)), dim3(256), 0, \
-                     stream, q, proj, ps, rows, states, cv, spans, row_seq,  \
-                     pos, slots, table, n_rows, seq0, W, bs_log, g)
+                     stream, q, proj, ps, rows, states, cv, row_seq, pos,    \
+                     slots, table, n_rows, seq0, W, bs_log, g)
 #define BY_LG(TAPS)                                              \
   do {                                                           \
-    if (small) CONV_RUN(16, TAPS); else CONV_RUN(32, TAPS);      \
+    if (g.dim <= 64 && g.vdim <= 64) CONV_RUN(8, TAPS);          \
+    else if (small) CONV_RUN(16, TAPS);                          \
+    else CONV_RUN(32, TAPS);                                     \
   } while (0)
   const long runs = (long)((n_rows + RUN - 1) / RUN) *
                     (g.heads + 2 * g.kvh);
