@@ -85,7 +85,7 @@ def _try_load() -> None:
     lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
                                        [_f, _f, _i] + [_vp] * 3 + [_i, _i, _vp])
     lib.fei_encoder_packed.argtypes = ([_vp, _i] + [_vp] * 12 + [_i] * 6 +
-                                       [_f, _f] + [_vp] * 2 + [_i, _i, _vp])
+                                       [_f, _f, _i, _vp, _i, _i, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
                                           _l, _l, _vp]
@@ -989,12 +989,9 @@ def encoder_packed(emb: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor,
     room = [rows(n) for n in (C, C, C, 3 * HD, HD, inner)]
     starts = torch.empty(B + 1, dtype=torch.int32, device=emb.device)
     out = torch.empty(B, C, dtype=torch.float32, device=emb.device)
-    sizes = parts = None
-    if M > ENCODER_PACKED_ROWS:
-        best = [_tiles.parts_up_to(M, *c) for c in (
-            (3 * HD, C, 1), (C, HD), (inner, C, 1), (C, inner))]
-        sizes = (_i * 8)(*(v for size, _ in best for v in size))
-        p1, p2 = best[1][1], best[3][1]
+    parts, many = None, M > ENCODER_PACKED_ROWS
+    if many:
+        p1, p2 = (_tiles.parts_up_to(M, C, k) for k in (HD, inner))
     else:
         # as in encoder_layers, for two thirds of the rows
         tiles = -(-M * 2 // 3 // 64) * -(-C // 64)
@@ -1007,7 +1004,7 @@ def encoder_packed(emb: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor,
         (_vp * len(weights))(*(t.data_ptr() for t in weights)),
         len(weights) // 12, _ptr(out), _ptr(emb), _ptr(gain), _ptr(shift),
         *(_ptr(t) for t in room), _ptr(lens), _ptr(starts), B, S, heads, dim, C,
-        inner, 1.0 / math.sqrt(dim), eps, sizes,
+        inner, 1.0 / math.sqrt(dim), eps, many,
         None if parts is None else _ptr(parts), p1, p2, _stream())
     return out
 

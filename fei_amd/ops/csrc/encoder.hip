@@ -337,9 +337,9 @@ void fei_parts_layernorm_of(void* out, const float* parts, int np,
                             const void* bias, const void* res, const void* gain,
                             const void* shift, int rows, int cols, float eps,
                             const int* count, hipStream_t stream);
-void fei_tile(void* out, long os, const void* x, long xs, const void* w,
-              const void* bias, int M, int N, int K, int epi, int rows,
-              int width, int parts, const int* count, hipStream_t stream);
+void fei_tile_counted(void* out, long os, const void* x, long xs, const void* w,
+                      const void* bias, int M, int N, int K, int epi, int parts,
+                      const int* count, hipStream_t stream);
 void fei_attn_packed(const void* qkv, void* out, const int* kv_len,
                      const int* starts, int B, int S, int H, int D, float scale,
                      hipStream_t stream);
@@ -352,21 +352,22 @@ void fei_layernorm_packed(void* out, const void* x, const void* res,
 // emb [B, S, C] is what the first norm (gain, shift) takes; w: 12 a layer, as in
 // fei_encoder_layers; h, h1 and tmp have room for B * S rows of C, qkv of 3 H D, att of
 // H D, inner of I; starts for B + 1. How many rows there are only the device knows: grids
-// are made for all B * S, and blocks that have none leave. sizes: rows and width of the
-// tiles (fei_tile) of the four products of a layer; null: tiles of 64 x 64. p1, p2 and
-// parts as in fei_encoder_layers. All on 16 bytes, C and H D and I
+// are made for all B * S, and blocks that have none leave. many: whether
+// products are fei_tile_counted's, else in tiles of 64 x 64. p1, p2 and parts as in
+// fei_encoder_layers. All on 16 bytes, C and H D and I
 // multiples of 64, C <= 2048.
 //
-// 64 texts of 64 to 256 tokens, 10336 rows of 16384, 12 layers of 768: 3000 us; all
-// rows, with the library's products, 4005. Bound by the products, at 0.7 to 0.8 PFLOP/s
-// of tiles that fill the chip one and a half times. To find the number costs each kernel
+// 64 texts of 64 to 256 tokens, 10336 rows of 16384, 12 layers of 768: 2565 us; all
+// rows, with the library's products, 3750. Texts of one length, for which the library's
+// tiles are better: 32 x 128 to 64 x 256 2 to 6 % slower. Bound by the products, at 0.7 to
+// 1 PFLOP/s of tiles that fill the chip one and a half times. To find the number costs each kernel
 // a load before its first, 30 us of the 570 that 320 rows take in all.
 void fei_encoder_packed(const void* const* w, int layers, float* out,
                         const void* emb, const void* gain, const void* shift,
                         void* h, void* h1, void* tmp, void* qkv, void* att,
                         void* inner, const int* lens, int* starts, int B, int S,
                         int H, int D, int C, int I, float scale, float eps,
-                        const int* sizes, float* parts, int p1, int p2,
+                        int many, float* parts, int p1, int p2,
                         hipStream_t stream) {
   const int M = B * S, HD = H * D;
   const int* count = starts + B;
@@ -374,36 +375,36 @@ void fei_encoder_packed(const void* const* w, int layers, float* out,
                      lens, B, S);
   fei_layernorm_packed(h, emb, nullptr, gain, shift, B, S, C, eps, starts,
                        stream);
-  auto product = [&](int i, void* to, const void* x, const void* const* wb,
-                     int N, int K, bool gelu) {
+  auto product = [&](void* to, const void* x, const void* const* wb, int N, int K,
+                     bool gelu) {
     constexpr int TILE_GELU = 2, TILE_BIAS = 5;
-    if (!sizes)
+    if (!many)
       return fei_rows_bias_of(to, x, wb[0], wb[1], M, N, K, gelu, count, stream);
-    fei_tile(to, N, x, K, wb[0], wb[1], M, N, K, gelu ? TILE_GELU : TILE_BIAS,
-             sizes[2 * i], sizes[2 * i + 1], 1, count, stream);
+    fei_tile_counted(to, N, x, K, wb[0], wb[1], M, N, K,
+                     gelu ? TILE_GELU : TILE_BIAS, 1, count, stream);
   };
-  auto residual = [&](int i, void* to, const void* from, const void* x,
+  auto residual = [&](void* to, const void* from, const void* x,
                       const void* const* wb, int K, int np) {
     if (np) {
       constexpr int TILE_PARTS = 4;
-      if (sizes)
-        fei_tile(parts, C, x, K, wb[0], nullptr, M, C, K, TILE_PARTS,
-                 sizes[2 * i], sizes[2 * i + 1], np, count, stream);
+      if (many)
+        fei_tile_counted(parts, C, x, K, wb[0], nullptr, M, C, K, TILE_PARTS, np,
+                         count, stream);
       else
         fei_rows_parts_of(parts, x, wb[0], M, C, K, np, count, stream);
       return fei_parts_layernorm_of(to, parts, np, wb[1], from, wb[2], wb[3], M,
                                     C, eps, count, stream);
     }
-    product(i, tmp, x, wb, C, K, false);
+    product(tmp, x, wb, C, K, false);
     fei_layernorm_packed(to, tmp, from, wb[2], wb[3], B, S, C, eps, starts,
                          stream);
   };
   for (int l = 0; l < layers; ++l, w += 12) {
-    product(0, qkv, h, w, 3 * HD, C, false);
+    product(qkv, h, w, 3 * HD, C, false);
     fei_attn_packed(qkv, att, lens, starts, B, S, H, D, scale, stream);
-    residual(1, h1, h, att, w + 2, HD, p1);
-    product(2, inner, h1, w + 6, I, C, true);
-    residual(3, h, h1, inner, w + 8, I, p2);
+    residual(h1, h, att, w + 2, HD, p1);
+    product(inner, h1, w + 6, I, C, true);
+    residual(h, h1, inner, w + 8, I, p2);
   }
   hipLaunchKernelGGL(k_pool_unit, dim3(B), dim3(1024), 1024 / (C / 8) * C * 4,
                      stream, out, (const u16*)h, lens, starts, S, C);

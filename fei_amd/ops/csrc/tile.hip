@@ -2,6 +2,7 @@
 // out[M, N] = x[M, K] @ W[N, K]^T in bfloat16 with float32 sums, where what follows
 // the product is done on its sums, or K is cut so that all CUs have a tile.
 #include <algorithm>
+#include <type_traits>
 
 #include "fei_epilogue.h"
 #include "fei_mma.h"
@@ -26,10 +27,13 @@ struct TileArgs {
   const u16* x;
   const u16* w;
   const u16* bias;
-  const int* rows;     // how many of the M rows there are, if only the device knows
+  const int* rows;     // k_tile_counted: how many of the M rows there are
   long os, xs;         // rows of out and x are this far apart
   int M, N, K, nx, parts;
 };
+
+template <int N>
+using Int = std::integral_constant<int, N>;
 
 // A tile's columns of out, and of W a half of them for gates where there are gates.
 template <int WM, int XI, int WI, int EPI>
@@ -367,8 +371,7 @@ template <int WM, int XI, int WI, int EPI, int MC, int NC>
 __global__ void __launch_bounds__(512, 2) k_tile(TileArgs g) {
   typedef Shape<WM, XI, WI, EPI> B;
   extern __shared__ __align__(16) u16 buf[];
-  const int M = g.rows ? uniform(min(*g.rows, g.M)) : g.M;
-  const int nm = (M + B::rows - 1) / B::rows;
+  const int M = g.M, nm = (M + B::rows - 1) / B::rows;
   const int tiles = g.nx * nm * g.parts, per = (tiles + 7) / 8;
   const int xcd = blockIdx.x & 7, slots = gridDim.x >> 3;
   const int lim = min(per, tiles - xcd * per);          // tiles of the XCD
@@ -397,11 +400,60 @@ void launch(TileArgs g, hipStream_t stream) {
     hipLaunchKernelGGL(kernel, dim3(8 * slots), dim3(512), lds, stream, g);
   };
   const int rest = (int)(per % slots);
-  // where only the device knows the rows, it may have a rest
-  if (MC * NC > 1 && (g.rows || (rest && rest * MC * NC <= slots)))
+  if (MC * NC > 1 && rest && rest * MC * NC <= slots)
     go(k_tile<WM, XI, WI, EPI, MC, NC>);
   else
     go(k_tile<WM, XI, WI, EPI, 1, 1>);
+}
+
+// The same of as many rows as the device finds, in the tiles that suit them: by the time
+// of a round of each, us of a step of 64 of K with one tile on the chip, what comes on
+// top with one on every CU, and of a round. 12 layers of 768, texts of 64 to 256 tokens,
+// 10336 rows of 16384: 2304 x 768 in tiles of 256 x 256, which suit 16384, 45.6 us, of 192
+// x 256 36.2; 768 x 768 21.5 and, of 128 x 256, 16.3; 768 x 3072 56.3, 46.2; 3072 x 768
+// with GELU 63, 72 of either other. Rests are not cut: with 12 steps of K that gains less
+// than to start anew costs. Blocks without a tile leave at once.
+template <int EPI>
+__global__ void __launch_bounds__(512, 2) k_tile_counted(const TileArgs all) {
+  extern __shared__ __align__(16) u16 buf[];
+  TileArgs g = all;
+  const int M = uniform(min(*g.rows, g.M));
+  const float steps = (float)(g.K / 64 / g.parts);
+  // us of GELU on 256 x 256 sums
+  const float act = EPI == TILE_GELU ? 14.f : 0.f;
+  auto tiles = [&](int rows, int width) {
+    return (M + rows - 1) / rows * ((g.N + width - 1) / width) * g.parts;
+  };
+  auto time = [&](int rows, int width, float alone, float full) {
+    const int n = tiles(rows, width);
+    const float round = steps * alone + 3.f + act * (float)(rows * width) / 65536.f;
+    return (float)((n + 255) / 256) * round + steps * full * (float)n / 256.f;
+  };
+  const float t0 = time(256, 256, 1.f, 0.46f), t1 = time(256, 192, 0.875f, 0.36f);
+  const float t2 = time(192, 256, 0.82f, 0.34f), t3 = time(128, 256, 0.73f, 0.13f);
+  auto run = [&](auto wm, auto xi, auto wi) __attribute__((always_inline)) {
+    typedef Shape<decltype(wm)::value, decltype(xi)::value, decltype(wi)::value, EPI> B;
+    g.nx = (g.N + B::columns - 1) / B::columns;
+    const int nm = (M + B::rows - 1) / B::rows;
+    const int per = (g.nx * nm * g.parts + 7) / 8, xcd = blockIdx.x & 7;
+    run_tiles<B, decltype(wm)::value, decltype(xi)::value, decltype(wi)::value, EPI>(
+        g, Share{xcd * per, min(per, g.nx * nm * g.parts - xcd * per)}, buf, M, nm);
+  };
+  const float best = fminf(fminf(t0, t1), fminf(t2, t3));
+  switch (uniform(best == t0 ? 0 : best == t1 ? 1 : best == t2 ? 2 : 3)) {
+    case 0: run(Int<2>{}, Int<4>{}, Int<2>{}); break;
+    case 1: run(Int<4>{}, Int<2>{}, Int<3>{}); break;
+    case 2: run(Int<2>{}, Int<3>{}, Int<2>{}); break;
+    default: run(Int<2>{}, Int<2>{}, Int<2>{});
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
+template <int EPI>
+void launch_counted(const TileArgs& g, hipStream_t stream) {
+  constexpr int lds = 2 * 512 * 128 + 4096;
+  allow_lds(k_tile_counted<EPI>, lds);
+  hipLaunchKernelGGL(k_tile_counted<EPI>, dim3(256), dim3(512), lds, stream, g);
 }
 
 template <int EPI>
@@ -420,12 +472,11 @@ extern "C" {
 // Rows of x (xs apart) and w on 16 bytes and less than 2^24 values apart, K % 64 == 0
 // and at least 64 a part, N % 8 == 0; rows of out (os apart) on 16 bytes, as the bias. A tile has rows x width
 // rows of x and w: 256 x 256, 192 or 128, 192 x 256, 128 x 256. epi: see above; parts
-// are 1 but for TILE_PARTS. count: null, or where the device finds how many of the M
-// rows there are; blocks without a tile leave at once.
+// are 1 but for TILE_PARTS.
 void fei_tile(void* out, long os, const void* x, long xs, const void* w,
               const void* bias, int M, int N, int K, int epi, int rows,
-              int width, int parts, const int* count, hipStream_t stream) {
-  const TileArgs g = {out, (const u16*)x, (const u16*)w, (const u16*)bias, count,
+              int width, int parts, hipStream_t stream) {
+  const TileArgs g = {out, (const u16*)x, (const u16*)w, (const u16*)bias, nullptr,
                       os, xs, M, N, K, 0, parts};
   switch (epi) {
     case TILE_BF16: return by_size<TILE_BF16>(rows, width, g, stream);
@@ -433,7 +484,20 @@ void fei_tile(void* out, long os, const void* x, long xs, const void* w,
     case TILE_GELU: return by_size<TILE_GELU>(rows, width, g, stream);
     case TILE_RELU2: return by_size<TILE_RELU2>(rows, width, g, stream);
     case TILE_PARTS: return by_size<TILE_PARTS>(rows, width, g, stream);
-    case TILE_BIAS: return by_size<TILE_BIAS>(rows, width, g, stream);
+  }
+}
+
+// The same of as many of the M rows as the device finds at ``count``, in tiles that it
+// chooses: with a bias, and GELU of that, or (TILE_PARTS) float32 [parts, M, N].
+void fei_tile_counted(void* out, long os, const void* x, long xs, const void* w,
+                      const void* bias, int M, int N, int K, int epi, int parts,
+                      const int* count, hipStream_t stream) {
+  const TileArgs g = {out, (const u16*)x, (const u16*)w, (const u16*)bias, count,
+                      os, xs, M, N, K, 0, parts};
+  switch (epi) {
+    case TILE_BIAS: return launch_counted<TILE_BIAS>(g, stream);
+    case TILE_GELU: return launch_counted<TILE_GELU>(g, stream);
+    case TILE_PARTS: return launch_counted<TILE_PARTS>(g, stream);
   }
 }
 

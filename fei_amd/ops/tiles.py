@@ -26,8 +26,9 @@ TILES = ((256, 256, 1.0, 0.46), (256, 192, 0.875, 0.36), (192, 256, 0.82, 0.34),
 
 
 def declare(lib: ctypes.CDLL) -> None:
-    lib.fei_tile.argtypes = ([_vp, _l, _vp, _l, _vp, _vp] + [_i] * 7 +
-                             [_vp, _vp])
+    lib.fei_tile.argtypes = [_vp, _l, _vp, _l, _vp, _vp] + [_i] * 7 + [_vp]
+    lib.fei_tile_counted.argtypes = ([_vp, _l, _vp, _l, _vp, _vp] + [_i] * 5 +
+                                     [_vp, _vp])
 
 
 def _p(t: Optional[torch.Tensor]):
@@ -155,11 +156,11 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def _launch(out, x, w, N, epi, size, bias=None, parts=1, rows=None) -> None:
+def _launch(out, x, w, N, epi, size, bias=None, parts=1) -> None:
     M, K = x.shape
     _ops.require_lib().fei_tile(
         _p(out), out.stride(-2), _p(x), x.stride(0), _p(w), _p(bias), M, N, K,
-        epi, *size, parts, _p(rows), _ops._stream())
+        epi, *size, parts, _ops._stream())
 
 
 def parts_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -209,19 +210,17 @@ def parts_for(M: int, N: int, K: int) -> Tuple[Tuple[int, int], int]:
 
 
 @lru_cache(maxsize=1024)
-def parts_up_to(M: int, N: int, K: int, most: int = 8
-                ) -> Tuple[Tuple[int, int], int]:
-    """The same where only the device knows how many of M rows there are, half of them
-    or more, and something reads the results of a product in one part too. All of them
-    count twice: texts are often cut to one length."""
-    def us(m, tile, p):
-        return (_time(m, N, K, p, *tile) +
+def parts_up_to(M: int, N: int, K: int) -> int:
+    """Parts of K where only the device knows how many of M rows there are, half of them
+    or more, which chooses its tiles, and something reads the results of a product in one
+    part too."""
+    def us(m, p):
+        return (min(_time(m, N, K, p, *t) for t in TILES if t[1] > 128) +
                 m * N * (1.8e-6 * p if p > 1 else 0.9e-6))
-    ways = [(t, p) for t in TILES for p in range(1, min(most, K // 256) + 1)]
-    times = [[us(M * f // 8, *way) for way in ways] for f in (4, 5, 6, 7, 8, 8)]
-    loss = [sum(row[i] / min(row) for row in times) for i in range(len(ways))]
-    tile, p = ways[loss.index(min(loss))]
-    return tile[:2], p
+    times = [[us(M * f // 8, p) for p in range(1, min(8, K // 256) + 1)]
+             for f in range(4, 9)]
+    loss = [sum(row[i] / min(row) for row in times) for i in range(len(times[0]))]
+    return loss.index(min(loss)) + 1
 
 
 def product_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

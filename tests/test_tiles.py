@@ -134,21 +134,42 @@ def test_tile(M, N, K, size):
                                       ((256, 192), 2400, 5192), ((192, 256), 2500, 4872),
                                       ((192, 256), 2500, 5000)])
 @pytest.mark.parametrize("K", [64, 192, 1088])
-@pytest.mark.parametrize("count", [None, 0, 1, 600, 2399, 9999])
-def test_last_round_in_halves(size, M, N, K, count):
-    x, w, b = (rand(M, K, seed=1), rand(2 * N, K, seed=2, scale=K ** -0.5),
-               rand(N, seed=3))
-    n = M if count is None else min(count, M)
-    rows = None if count is None else torch.tensor([count], dtype=torch.int32,
-                                                   device=DEV)
-    y = x[:n].double() @ w.double().t()
-    for epi, bias, want in ((tiles.TILE_BIAS, b, y[:, :N] + b.double()),
-                            (tiles.TILE_SWIGLU, None, F.silu(y[:, :N]) * y[:, N:])):
+def test_last_round_in_halves(size, M, N, K):
+    x, w = rand(M, K, seed=1), rand(2 * N, K, seed=2, scale=K ** -0.5)
+    y = x.double() @ w.double().t()
+    for epi, want in ((tiles.TILE_BF16, y[:, :N]),
+                      (tiles.TILE_SWIGLU, F.silu(y[:, :N]) * y[:, N:])):
         out = torch.full((M, N), 7.0, device=DEV, dtype=torch.bfloat16)
-        ww = w if epi == tiles.TILE_SWIGLU else w[:N]
-        tiles._launch(out, x, ww, N, epi, size, bias, rows=rows)
-        assert n == 0 or err(out[:n], want) < 2 ** -9     # a result is rounded once
-        assert bool((out[n:] == 7).all())
+        tiles._launch(out, x, w if epi == tiles.TILE_SWIGLU else w[:N], N, epi, size)
+        assert err(out, want) < 2 ** -9               # a result is rounded once
+
+
+# each of the tiles that the device chooses from, short of the last row and past it
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(2500, 768, 192), (10336, 768, 64), (9000, 2304, 64),
+                                   (10400, 3080, 128), (16000, 776, 1088)])
+@pytest.mark.parametrize("count", [0, 1, 129, 0.4, 0.63, 1.0, 99999])
+def test_rows_that_the_device_counts(M, N, K, count):
+    x, w, b = rand(M, K, seed=1), rand(N, K, seed=2, scale=K ** -0.5), rand(N, seed=3)
+    count = int(M * count) if isinstance(count, float) else count
+    n, rows = min(count, M), torch.tensor([count], dtype=torch.int32, device=DEV)
+    y = x[:n].double() @ w.double().t()
+
+    def run(out, epi, parts=1):
+        ops.require_lib().fei_tile_counted(
+            out.data_ptr(), N, x.data_ptr(), K, w.data_ptr(), b.data_ptr(), M, N, K,
+            epi, parts, rows.data_ptr(), ops._stream())
+        assert bool((out[..., n:, :] == 7).all())
+        return out[..., :n, :]
+    for epi, want in ((tiles.TILE_BIAS, y + b.double()),
+                      (tiles.TILE_GELU, F.gelu(y + b.double()))):
+        got = run(torch.full((M, N), 7.0, device=DEV, dtype=torch.bfloat16), epi)
+        assert n == 0 or err(got, want) < 2 ** -9     # a result is rounded once
+    for p in (1, 2, 3):
+        if K // 64 >= p:
+            got = run(torch.full((p, M, N), 7.0, device=DEV), tiles.TILE_PARTS, p)
+            # float32 sums in any order, as above
+            assert n == 0 or err(got.double().sum(0), y) < 2 ** -24 * max(K ** 0.5, 16)
 
 
 @pytest.mark.gpu
