@@ -340,10 +340,10 @@ class LlamaModel:
             ssq.zero_()
         pf = self.prefetch_mb > 0 and fp8 is None and h.is_cuda
         done = 0
-        if not (pf or fused_attn) and fp8 is ssq is attn_out is None:
+        if not (pf or fused_attn) and fp8 is ssq is None:
             done, sums = ops.llama_few(
                 h, self.layers, k_caches, v_caches, self.hq_l, s.norm_eps, pos,
-                self.rope, attn_splits, workspace)
+                self.rope, attn_splits, workspace, attn_out=attn_out)
         if pf and self._pf_stream is None:
             self._pf_stream = torch.cuda.Stream()
             self._pf_sink = torch.zeros(1, dtype=torch.float32,
@@ -371,13 +371,19 @@ class LlamaModel:
                 att = ops.attn_decode_fused(q, k, v, k_caches[li],
                                             v_caches[li], pos, self.rope,
                                             scale=scale, out=attn_out)
+            elif fp8 is not None:
+                ops.attn_decode_product_fp8(
+                    q, k_caches[li], v_caches[li], pos, *q8["wo"], h,
+                    splits=attn_splits, scale=scale, workspace=workspace,
+                    out=attn_out, k=k, v=v, table=self.rope)
             else:
                 att = ops.attn_decode(q, k_caches[li], v_caches[li], pos,
                                       splits=attn_splits, scale=scale,
                                       workspace=workspace, out=attn_out,
                                       k=k, v=v, table=self.rope, layer=li)
             if fp8 is not None:
-                ops.gemv_res_fp8(att.reshape(B, -1), *q8["wo"], h)
+                if fused_attn:
+                    ops.gemv_res_fp8(att.reshape(B, -1), *q8["wo"], h)
                 act = ops.gemv_swiglu_norm_fp8(h, lw.norm_mlp, *q8["wgu"],
                                                s.norm_eps)
                 ops.gemv_res_fp8(act, *q8["wdown"], h)

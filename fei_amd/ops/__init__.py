@@ -68,6 +68,9 @@ def _try_load() -> None:
                                         _i, _i, _i, _i, _i, _i, _l, _l, _vp]
     lib.fei_attn_decode.argtypes = ([_vp] * 8 + [_i] * 8 + [_f, _l] +
                                     [_vp] * 3 + [_l, _vp])
+    lib.fei_attn_decode_product.argtypes = ([_vp] * 8 + [_i] * 7 + [_f, _l] +
+                                            [_vp] * 3 + [_l] + [_vp] * 3 +
+                                            [_i, _vp])
     lib.fei_swiglu.argtypes = [_vp, _vp, _l, _i, _vp]
     lib.fei_sample.argtypes = [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _f, _u64,
                                _i, _i, _vp]
@@ -252,8 +255,9 @@ def attn_decode(q, k_cache, v_cache, pos, splits: int = 32,
 
 def _launch_attn_decode(q, kc, vc, blocks, max_seq: int, bs_log: int,
                         Hkv: int, pos, splits: int, scale: float, workspace,
-                        out, k, v, rope) -> torch.Tensor:
-    """Contiguous caches (``blocks`` None) or paged pools."""
+                        out, k, v, rope, product=None) -> torch.Tensor:
+    """Contiguous caches (``blocks`` None) or paged pools. ``product``: (w, its scales or
+    None, res) of an output product that is added to res, of one sequence."""
     B, Hq, D = q.shape
     if workspace is None:
         part_o = torch.empty(B, Hq, splits, D, dtype=torch.float32, device=q.device)
@@ -278,11 +282,17 @@ def _launch_attn_decode(q, kc, vc, blocks, max_seq: int, bs_log: int,
         kv_bs = 0
     if not B:
         return out
-    require_lib().fei_attn_decode(
-        _ptr(q), _ptr(kc), _ptr(vc), None if blocks is None else _ptr(blocks),
-        _ptr(part_o), _ptr(part_ml), _ptr(out), _ptr(pos), B, Hq, Hkv, D,
-        max_seq, bs_log, 0 if blocks is None else blocks.shape[1], splits,
-        scale, q.stride(0), kin, vin, cs, kv_bs, _stream())
+    args = (_ptr(q), _ptr(kc), _ptr(vc), None if blocks is None else _ptr(blocks),
+            _ptr(part_o), _ptr(part_ml), _ptr(out), _ptr(pos))
+    sizes = (Hq, Hkv, D, max_seq, bs_log, 0 if blocks is None else blocks.shape[1],
+             splits, scale, q.stride(0), kin, vin, cs, kv_bs)
+    if product is None:
+        require_lib().fei_attn_decode(*args, B, *sizes, _stream())
+    else:
+        w, wscale, res = product
+        require_lib().fei_attn_decode_product(
+            *args, *sizes, _ptr(res), _ptr(w),
+            None if wscale is None else _ptr(wscale), w.shape[0], _stream())
     return out
 
 
@@ -1082,6 +1092,25 @@ def gemv_res_fp8(x, w8, wscale, res) -> torch.Tensor:
         return res
     _launch_gemv(res, x.contiguous().view(M, K), None, w8, wscale, N, 0.0,
                  _RES)
+    return res
+
+
+def attn_decode_product_fp8(q, k_cache, v_cache, pos, w8, wscale, res,
+                            splits: int = 32, scale: Optional[float] = None,
+                            workspace=None, out=None, k=None, v=None,
+                            table=None) -> torch.Tensor:
+    """attn_decode of one sequence, and gemv_res_fp8 of its result, which may be left to
+    the product to sum: ``out`` need not have it afterwards."""
+    B, Hq, D = q.shape
+    if not (q.is_cuda and B == 1 and Hq * D % 16 == 0 and res.is_contiguous()
+            and res.dtype == torch.bfloat16 and res.numel() == w8.shape[0]):
+        att = attn_decode(q, k_cache, v_cache, pos, splits, scale, workspace, out, k,
+                          v, table)
+        return gemv_res_fp8(att.reshape(B, -1), w8, wscale, res)
+    _launch_attn_decode(q, k_cache, v_cache, None, k_cache.shape[2], 0,
+                        k_cache.shape[1], pos, splits,
+                        scale if scale is not None else 1.0 / math.sqrt(D),
+                        workspace, out, k, v, table, (w8, wscale, res))
     return res
 
 

@@ -441,11 +441,13 @@ inline int whole_keys(int heads, int D) {
   return D == 64 ? 768 : heads < 96 ? 320 : 512;
 }
 
+// Returns how many splits there are to sum, if that was left to the caller (``open``).
 template <int D>
-void launch_decode(DecodeAttn a, int B, hipStream_t stream) {
+int launch_decode(DecodeAttn a, int B, bool open, hipStream_t stream) {
   if (a.max_seq > CHUNK * SHARE && a.max_seq <= whole_keys(a.Hkv * B, D)) {
     a.splits = 1;
-    return launch_waves<D, whole_waves(D)>(a, dim3(a.Hkv, B), stream);
+    launch_waves<D, whole_waves(D)>(a, dim3(a.Hkv, B), stream);
+    return 1;
   }
   // Splits that no sequence can have are not launched, and those beyond 16 come
   // last: a block waits for the position to know that it has no keys, and keeps
@@ -456,9 +458,10 @@ void launch_decode(DecodeAttn a, int B, hipStream_t stream) {
   const int side = min(all, 16);
   launch_waves<D, SHARE>(a, dim3(a.Hkv * side, B, (all + side - 1) / side),
                          stream);
-  if (all > 1)
+  if (all > 1 && !open)
     hipLaunchKernelGGL(k_attn_decode_combine<D>, dim3(B * a.Hkv * a.G),
                        dim3(256), 0, stream, a);
+  return all;
 }
 
 }  // namespace
@@ -467,15 +470,12 @@ void launch_decode(DecodeAttn a, int B, hipStream_t stream) {
 // null) the positions that a row of the table can name. cs null: q is roped and
 // the new token's row is in the cache. Up to 16 query heads a kv head, up to 64
 // splits; D is 64 or 128. Nothing is launched for an empty batch.
-extern "C" void fei_attn_decode(const void* q, void* kc, void* vc,
-                                const int* table, float* po, float* pml,
-                                void* out, const int* pos, int B, int Hq,
-                                int Hkv, int D, int max_seq, int bs_log, int W,
-                                int splits, float scale, long q_bs,
-                                const void* kin, const void* vin,
-                                const float* cs, long kv_bs,
-                                hipStream_t stream) {
-  if (B <= 0 || Hkv <= 0) return;
+static int decode(const void* q, void* kc, void* vc, const int* table, float* po,
+                  float* pml, void* out, const int* pos, int B, int Hq, int Hkv,
+                  int D, int max_seq, int bs_log, int W, int splits, float scale,
+                  long q_bs, const void* kin, const void* vin, const float* cs,
+                  long kv_bs, bool open, hipStream_t stream) {
+  if (B <= 0 || Hkv <= 0) return 1;
   const DecodeAttn a{(const u16*)q, (u16*)kc,         (u16*)vc,
                      table,         po,               pml,
                      (u16*)out,     pos,              (const u16*)kin,
@@ -483,6 +483,52 @@ extern "C" void fei_attn_decode(const void* q, void* kc, void* vc,
                      Hkv,           max_seq,          bs_log,
                      W,             splits,           scale,
                      q_bs,          kv_bs};
-  if (D == 128) launch_decode<128>(a, B, stream);
-  else if (D == 64) launch_decode<64>(a, B, stream);
+  if (D == 128) return launch_decode<128>(a, B, open, stream);
+  if (D == 64) return launch_decode<64>(a, B, open, stream);
+  return 1;
 }
+
+extern "C" {
+
+void fei_attn_decode(const void* q, void* kc, void* vc, const int* table, float* po,
+                     float* pml, void* out, const int* pos, int B, int Hq, int Hkv,
+                     int D, int max_seq, int bs_log, int W, int splits, float scale,
+                     long q_bs, const void* kin, const void* vin, const float* cs,
+                     long kv_bs, hipStream_t stream) {
+  decode(q, kc, vc, table, po, pml, out, pos, B, Hq, Hkv, D, max_seq, bs_log, W,
+         splits, scale, q_bs, kin, vin, cs, kv_bs, false, stream);
+}
+
+void fei_gemv_splits(void* out, const void* x, const void* w, const float* wscale,
+                     int N, int K, const float* po, const float* pml,
+                     const int* pos, int splits, int left, int room, int keys,
+                     int D, hipStream_t stream);
+void fei_gemv(void* out, const void* x, const void* gain, const void* w,
+              const float* wscale, int M, int N, int K, float eps, int epi,
+              float* ssq, hipStream_t stream);
+
+// Decode attention of one sequence and its output product, added to res [1, N]: w [N, Hq
+// D], wscale null or the scales of fp8 rows. Where the splits are few the product sums
+// them (gemv.hip), and out is not written. The rest as above.
+void fei_attn_decode_product(const void* q, void* kc, void* vc, const int* table,
+                             float* po, float* pml, void* out, const int* pos,
+                             int Hq, int Hkv, int D, int max_seq, int bs_log, int W,
+                             int splits, float scale, long q_bs, const void* kin,
+                             const void* vin, const float* cs, long kv_bs,
+                             void* res, const void* w, const float* wscale, int N,
+                             hipStream_t stream) {
+  // of few long rows k_gemv has its waves share them
+  const int K = Hq * D, most = K <= 2048 ? 16 : K <= 4096 && N > 2048 ? 5 : 0;
+  const bool open = min(splits, (max_seq + CHUNK * SHARE - 1) / (CHUNK * SHARE)) <=
+                    most;
+  const int left = decode(q, kc, vc, table, po, pml, out, pos, 1, Hq, Hkv, D,
+                          max_seq, bs_log, W, splits, scale, q_bs, kin, vin, cs,
+                          kv_bs, open, stream);
+  if (open && left > 1)
+    return fei_gemv_splits(res, out, w, wscale, N, K, po, pml, pos, splits, left,
+                           max_seq, CHUNK * SHARE, D, stream);
+  constexpr int GEMV_RES = 1;
+  fei_gemv(res, out, nullptr, w, wscale, 1, N, K, 0.f, GEMV_RES, nullptr, stream);
+}
+
+}  // extern "C"

@@ -13,6 +13,16 @@ namespace {
 
 enum { GEMV_BF16 = 0, GEMV_RES = 1, GEMV_SWIGLU = 2 };
 
+// Decode attention of one row that its product sums itself: what the splits of the keys
+// left (attn_decode.hip), [heads][splits][D] and their maxima (of exponents of 2) and sums,
+// [heads][splits][2]; keys: of a split. Of so few keys that one split had them all, x
+// has the result.
+struct Splits {
+  const float *po, *pml;
+  const int* pos;
+  int splits, room, keys, D;
+};
+
 // Sum over a wave, added in the order of a butterfly from lane ^ 32 down to
 // lane ^ 1, without LDS.
 __device__ __forceinline__ float wave_sum(float v) {
@@ -47,12 +57,20 @@ __device__ __forceinline__ float wave_sum(float v) {
 // (24.9), 128256 x 4096 151 (165). fp8: 7.1 (10), 5.7 (6.5), 20.4 (44.5),
 // 13.7 (13). Two or eight loads a row in flight, four rows a wave, or rows
 // shared by 2 waves are slower at nearly every size.
-template <int M, int KS, bool NORM, int EPI, bool FP8, bool LDS>
-__global__ void __launch_bounds__(256)
-k_gemv(u16* __restrict__ out, const u16* __restrict__ x,
-       const u16* __restrict__ gain, const void* __restrict__ wp,
-       const float* __restrict__ wscale, int N, int K, float eps,
-       float* __restrict__ ssq) {
+//
+// NS: x is the sum of up to NS splits of the keys, which every block makes for itself:
+// a launch less, and the weights are on the way meanwhile. For up to XS * 2048 columns.
+// All blocks read all splits, 4 bytes a column, from the L2s: whole decoding steps, us, 16
+// layers of 2048, 300 keys (3 splits) 685 -> 652, 1000 (8) 703 -> 670, 2000 (16) 702 ->
+// 692; 32 layers of 4096, 300 keys 2889 -> 2870, 600 (5) 2907 -> 2896, 700 (6) 2890 ->
+// 2899, which is left to the launch; fp8 weights, 500 keys 1898 -> 1858.
+template <int M, int KS, bool NORM, int EPI, bool FP8, bool LDS, int NS = 0,
+          int XS = 1>
+__device__ __forceinline__ void
+gemv(u16* __restrict__ out, const u16* __restrict__ x,
+     const u16* __restrict__ gain, const void* __restrict__ wp,
+     const float* __restrict__ wscale, int N, int K, float eps,
+     float* __restrict__ ssq, const Splits* sp) {
   constexpr int E = FP8 ? 16 : 8;          // weights of a 16-byte load
   constexpr int U = KS > 1 ? 2 : 4;        // loads of a row in flight
   constexpr int R = 2;                     // rows of w
@@ -77,17 +95,38 @@ k_gemv(u16* __restrict__ out, const u16* __restrict__ x,
   const int per = KS > 1 ? ((nv + 63) / 64 + KS - 1) / KS * 64 : nv;
   const int lo = ks * per, hi = KS > 1 ? min(nv, lo + per) : nv;
   // x first: loads come back in order
-  constexpr int XV = NORM && M == 1 ? 4 : 8;
+  constexpr int XV = NS ? XS : NORM && M == 1 ? 4 : 8;
   const int nx = M * (K / 8);
   s16x8 x0[XV], g0[NORM ? XV : 1];
   auto gain_at = [&](int c) {
     return ((const s16x8*)gain)[M == 1 ? c : c % (K / 8)];
   };
+  f32x4 po[NS ? XS : 1][NS ? NS : 1][2];
+  f32x2 ml[NS ? XS : 1][NS ? NS : 1];
+  int used = 0;
+  if constexpr (NS > 0) {
 #pragma unroll
-  for (int i = 0; LDS && i < XV; ++i) {
-    const int c = min(tid + i * 256, nx - 1);
-    x0[i] = ((const s16x8*)x)[c];
-    if (NORM) g0[i] = gain_at(c);
+    for (int i = 0; i < XS; ++i) {
+      const int c = min(tid + i * 256, nx - 1), head = c * 8 / sp->D;
+      x0[i] = ((const s16x8*)x)[c];
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const long at = (long)head * sp->splits + min(s, sp->splits - 1);
+        ml[i][s] = ((const f32x2*)sp->pml)[at];
+        const f32x4* p = (const f32x4*)(sp->po + at * sp->D + (c * 8 & (sp->D - 1)));
+        po[i][s][0] = p[0];
+        po[i][s][1] = p[1];
+      }
+    }
+    const int n = min(*sp->pos + 1, sp->room);
+    used = min(sp->splits, (n + sp->keys - 1) / sp->keys);
+  } else {
+#pragma unroll
+    for (int i = 0; LDS && i < XV; ++i) {
+      const int c = min(tid + i * 256, nx - 1);
+      x0[i] = ((const s16x8*)x)[c];
+      if (NORM) g0[i] = gain_at(c);
+    }
   }
   u32x4 v[U][R], nxt[U][R];
   auto fetch = [&](u32x4 (&d)[U][R], int i0) {
@@ -142,6 +181,29 @@ k_gemv(u16* __restrict__ out, const u16* __restrict__ x,
     for (int m = 0; m < M; ++m)
       inv[m] = rsqrtf((ssq ? ssq[m] : red[0][m] + red[1][m] + red[2][m] +
                                           red[3][m]) / (float)K + eps);
+  }
+  if constexpr (NS > 0) {
+    if (used != 1)
+#pragma unroll
+      for (int i = 0; i < XS; ++i) {
+        float m = -3.0e38f, l = 0.f, v[8];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          if (s < used) m = fmaxf(m, ml[i][s][0]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = 0.f;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          if (s < used) {                  // what lies there else is not used
+            const float f = __builtin_amdgcn_exp2f(ml[i][s][0] - m);
+            l = fmaf(f, ml[i][s][1], l);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = fmaf(f, po[i][s][j >> 2][j & 3], v[j]);
+          }
+        const float r = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x0[i][j] = (short)El<u16>::st(v[j] * r);
+      }
   }
   auto stage = [&](int c, s16x8 xv, s16x8 gv) {
     if (NORM) {
@@ -260,6 +322,26 @@ k_gemv(u16* __restrict__ out, const u16* __restrict__ x,
   }
 }
 
+template <int M, int KS, bool NORM, int EPI, bool FP8, bool LDS>
+__global__ void __launch_bounds__(256)
+k_gemv(u16* __restrict__ out, const u16* __restrict__ x,
+       const u16* __restrict__ gain, const void* __restrict__ wp,
+       const float* __restrict__ wscale, int N, int K, float eps,
+       float* __restrict__ ssq) {
+  gemv<M, KS, NORM, EPI, FP8, LDS>(out, x, gain, wp, wscale, N, K, eps, ssq,
+                                   nullptr);
+}
+
+// The output product of an attention, added to a residual: see Splits.
+template <bool FP8, int NS, int XS>
+__global__ void __launch_bounds__(256)
+k_gemv_splits(u16* __restrict__ out, const u16* __restrict__ x,
+              const void* __restrict__ wp, const float* __restrict__ wscale, int N,
+              int K, const Splits sp) {
+  gemv<1, 1, false, GEMV_RES, FP8, true, NS, XS>(out, x, nullptr, wp, wscale, N, K,
+                                                 0.f, nullptr, &sp);
+}
+
 template <int M, bool NORM, int EPI, bool FP8>
 void launch_gemv(void* out, const void* x, const void* gain, const void* w,
                  const float* wscale, int N, int K, float eps, float* ssq,
@@ -338,6 +420,38 @@ void fei_gemv(void* out, const void* x, const void* gain, const void* w,
   };
   if (gain) by_epi(std::true_type{});
   else by_epi(std::false_type{});
+}
+
+// out [1, N] += the attention that ``left`` splits of ``keys`` keys each left in po and
+// pml, where each head has room for ``splits``, (or, one that had all keys, in x) times w
+// [N, K], heads of D one behind another. K up to 2048 and 16 left, or up to 4096 and 5
+// (which fei_attn_decode_product sees to). K % 8 == 0, D a power of two.
+void fei_gemv_splits(void* out, const void* x, const void* w, const float* wscale,
+                     int N, int K, const float* po, const float* pml,
+                     const int* pos, int splits, int left, int room, int keys,
+                     int D, hipStream_t stream) {
+  const Splits sp{po, pml, pos, splits, room, keys, D};
+  auto run = [&](auto ns, auto xs) {
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3((N + 7) / 8), dim3(256), K * 2, stream,
+                         (u16*)out, (const u16*)x, w, wscale, N, K, sp);
+    };
+    if (wscale) go(k_gemv_splits<true, ns.value, xs.value>);
+    else go(k_gemv_splits<false, ns.value, xs.value>);
+  };
+  const std::integral_constant<int, 1> one{};
+  const std::integral_constant<int, 2> two{};
+  const std::integral_constant<int, 4> four{};
+  if (K <= 2048) {
+    if (left <= 2) run(two, one);
+    else if (left <= 4) run(four, one);
+    else if (left <= 8) run(std::integral_constant<int, 8>{}, one);
+    else run(std::integral_constant<int, 16>{}, one);
+  } else {
+    if (left <= 2) run(two, two);
+    else if (left <= 4) run(four, two);
+    else run(std::integral_constant<int, 5>{}, two);
+  }
 }
 
 void fei_prefetch(const void* w, long bytes, void* sink, int n_blocks,

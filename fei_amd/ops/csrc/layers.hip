@@ -25,6 +25,13 @@ void fei_attn_decode(const void* q, void* kc, void* vc, const int* table,
                      int splits, float scale, long q_bs, const void* kin,
                      const void* vin, const float* cs, long kv_bs,
                      hipStream_t stream);
+void fei_attn_decode_product(const void* q, void* kc, void* vc, const int* table,
+                             float* po, float* pml, void* out, const int* pos,
+                             int Hq, int Hkv, int D, int max_seq, int bs_log, int W,
+                             int splits, float scale, long q_bs, const void* kin,
+                             const void* vin, const float* cs, long kv_bs,
+                             void* res, const void* w, const float* wscale, int N,
+                             hipStream_t stream);
 void fei_rope_kv_prefill(void* q, const void* k, const void* v, void* k_cache,
                          void* v_cache, const float* cos_sin, const int* pos0,
                          int B, int S, int Hq, int Hkv, int D, int max_seq,
@@ -89,12 +96,17 @@ void fei_llama_few(const void* const* w, int summed, void* h, void* qkv,
     fei_attn_prefill(qkv, kc, vc, att, a.pos, a.pos, a.B, a.S, a.Hq, a.Hkv, a.D,
                      a.room, a.scale, 1, width, a.splits, a.po, a.pml,
                      (long)a.Hkv * a.room * a.D, (long)a.room * a.D, a.D, stream);
+  } else if (M == 1) {
+    fei_attn_decode_product(qkv, kc, vc, a.table, a.po, a.pml, att, a.pos, a.Hq,
+                            a.Hkv, a.D, a.room, a.bs_log, a.W, a.splits, a.scale,
+                            width, k, v, a.cos_sin, width, h, w[2], nullptr, C,
+                            stream);
   } else {
     fei_attn_decode(qkv, kc, vc, a.table, a.po, a.pml, att, a.pos, a.B, a.Hq,
                     a.Hkv, a.D, a.room, a.bs_log, a.W, a.splits, a.scale, width, k,
                     v, a.cos_sin, width, stream);
   }
-  add(att, w[2], HD);
+  if (a.S || M > 1) add(att, w[2], HD);
   normed_product(act, w[3], w[4], a.I, true);
   add(act, w[5], a.I);
 }

@@ -46,12 +46,14 @@ def _pointers(tensors, shapes, device: int, grad: bool):
 def llama_few(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor],
               v_caches: Sequence[torch.Tensor], heads: int, eps: float,
               pos: torch.Tensor, rope: torch.Tensor, splits: int = 0,
-              workspace=None, table: Optional[torch.Tensor] = None, S: int = 0
+              workspace=None, table: Optional[torch.Tensor] = None, S: int = 0,
+              attn_out: Optional[torch.Tensor] = None
               ) -> Tuple[int, Optional[torch.Tensor]]:
     """``layers`` over the rows h [M, C], in place: a decoding step's, or (``S``) those
     of prompts of S tokens. Caches [B, Hkv, room, D], or with a ``table`` pools
     [blocks, Hkv, size, D]; at pos[b] and on the rows' keys and values are written.
-    ``workspace``: see attn_decode. Returns how many layers are done, up to the first that
+    ``workspace``: see attn_decode; ``attn_out``: room for M rows of its results, if the
+    caller has some. Returns how many layers are done, up to the first that
     the kernels for few rows do not take, and what a norm's product behind them takes as
     ``sums``. The launches, and their order, are those of the operations one by one. A
     layer a call: the GPU has the first one's while the others are looked at (all 16 looked
@@ -97,7 +99,10 @@ def llama_few(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor
 
     def rows(n):
         return torch.empty(M, n, dtype=h.dtype, device=h.device)
-    room_for = [rows(n) for n in (width, HD, I, C)]
+    att = attn_out if attn_out is not None else rows(HD)
+    if not (_pointers((att,), (att.shape,), dev, False) and att.numel() == M * HD):
+        return 0, None
+    room_for = [rows(width), att, rows(I), rows(C)]
     sums = torch.empty(M, -(-C // (8 if C <= 2048 else 16)), dtype=torch.float32,
                        device=h.device)
     p = _FewRows(B, S, C, I, heads, Hkv, D, room, bs_log, W, splits, eps,

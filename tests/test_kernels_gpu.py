@@ -665,6 +665,44 @@ def test_prompt_in_parts_matches_whole_products(lib, B, S):
         assert row_err(x.flatten(), y.double().flatten()) < 2.0 ** -6
 
 
+# as many splits as the product sums itself, and one more, with keys for one split, for
+# all, at their edges, and none
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 64), (16, 4, 128), (32, 8, 128), (6, 2, 64)])
+@pytest.mark.parametrize("room", [128, 256, 320, 512, 640, 1024, 2048, 2112])
+@pytest.mark.parametrize("fp8", [False, True])
+def test_output_product_sums_the_splits(lib, Hq, Hkv, D, room, fp8):
+    W, N = (Hq + 2 * Hkv) * D, 2056
+    w = randbf(N, Hq * D, seed=1, scale=(Hq * D) ** -0.5)
+    w, ws = lib.quant_fp8(w) if fp8 else (w, None)
+    table = torch.randn(room, D // 2, 2, device=DEV)
+    kc, vc = (randbf(1, Hkv, room, D, seed=i) for i in (2, 3))
+    for n in sorted({0, 1, 127, 128, 129, room // 2, room - 1, room}):
+        qkv = randbf(1, W, seed=n + 9)
+        q, k, v = (qkv[:, a * D:b * D].view(1, -1, D) for a, b in (
+            (0, Hq), (Hq, Hq + Hkv), (Hq + Hkv, Hq + 2 * Hkv)))
+        # without RoPE where there is no key to turn
+        rope = dict(k=k, v=v, table=table) if n else {}
+        args = dict(splits=32, scale=D ** -0.5, **rope)
+        pos = torch.tensor([n - 1], dtype=torch.int32, device=DEV)
+        res = randbf(1, N, seed=5)
+        got, want = res.clone(), res.clone()
+        att = lib.attn_decode(q, kc.clone(), vc.clone(), pos, **args)
+        # what no split has written is not read
+        room_for = tuple(torch.full((1, Hq, 32, x), float("nan"), device=DEV)
+                         for x in (D, 2))
+        if fp8:
+            lib.gemv_res_fp8(att.view(1, -1), w, ws, want)
+            lib.attn_decode_product_fp8(q, kc.clone(), vc.clone(), pos, w, ws, got,
+                                        workspace=room_for, **args)
+        else:
+            lib.gemv_res(att.view(1, -1), w, want)
+            lib._launch_attn_decode(q, kc.clone(), vc.clone(), None, room, 0, Hkv, pos,
+                                    32, D ** -0.5, room_for, None, rope.get("k"),
+                                    rope.get("v"), rope.get("table"), (w, None, got))
+        # the attention's sums are rounded to bfloat16 once, in another order here
+        assert row_err(got, want.double()) < 2.0 ** -8, n
+
+
 # one row, one and more groups of 8, prompts and decoding steps; ``odd``: a layer whose
 # weights the kernels for few rows do not read as they lie, from which on the operations
 # run one by one
