@@ -19,7 +19,6 @@ import math
 from typing import List, Optional
 
 import torch
-import torch.nn.functional as F
 
 from fei_amd import ops
 from fei_amd.engine.config import ModelSpec, get_spec
@@ -90,19 +89,18 @@ class BgeEncoder:
         s = self.spec
         B, S = token_ids.shape
         H, D = s.num_heads, s.head_dim
-        h = F.embedding(token_ids.long(), self.tok_emb) + \
-            self.pos_emb[:S].unsqueeze(0)
-        h = h.to(self.dtype)
+        embed = (token_ids.long().contiguous(), self.tok_emb, self.pos_emb,
+                 self.emb_ln_w, self.emb_ln_b)
         kv_len = (lengths.to(torch.int32) if lengths is not None
                   else torch.full((B,), S, dtype=torch.int32, device=self.device))
         weights = [lw[n] for lw in self.layers for n in NAMES]
         if lengths is not None:
-            out = ops.encoder_packed(h, self.emb_ln_w, self.emb_ln_b, weights,
-                                     H, D, s.intermediate_size, kv_len, self.eps)
+            out = ops.encoder_packed(*embed, weights, H, D, s.intermediate_size,
+                                     kv_len, self.eps)
             if out is not None:
                 return out
-        h = ops.layernorm(h, self.emb_ln_w, self.emb_ln_b, self.eps)
-        pos0 = torch.zeros(B, dtype=torch.int32, device=self.device)
+        h = ops.embed_layernorm(*embed, self.eps, self.dtype)
+        pos0 = kv_len                  # of causal attention alone
         few = ops.encoder_layers(h, weights, H, D, s.intermediate_size, pos0,
                                  kv_len, self.eps)
         h = few if few is not None else self._layers(h, pos0, kv_len)

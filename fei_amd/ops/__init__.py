@@ -87,7 +87,9 @@ def _try_load() -> None:
     lib.fei_argmax.argtypes = [_vp] * 3 + [_i] * 4 + [_vp]
     lib.fei_encoder_layers.argtypes = ([_vp, _i] + [_vp] * 8 + [_i] * 6 +
                                        [_f, _f, _i] + [_vp] * 3 + [_i, _i, _vp])
-    lib.fei_encoder_packed.argtypes = ([_vp, _i] + [_vp] * 12 + [_i] * 6 +
+    lib.fei_embed_layernorm.argtypes = ([_vp] * 6 + [_i] * 4 + [_f] + [_vp] * 2)
+    lib.fei_encoder_packed.argtypes = ([_vp, _i] + [_vp] * 4 + [_i] +
+                                       [_vp] * 10 + [_i] * 6 +
                                        [_f, _f, _i, _vp, _i, _i, _vp])
     lib.fei_attn_decode_fused.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp,
                                           _vp, _i, _i, _i, _i, _i, _f,
@@ -971,34 +973,69 @@ ENCODER_PACKED_FROM = 640
 ENCODER_PACKED_ROWS = 3072
 
 
-def encoder_packed(emb: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor,
-                   weights, heads: int, dim: int, inner: int,
-                   lens: torch.Tensor, eps: float) -> Optional[torch.Tensor]:
-    """An encoder over texts of unlike lengths: emb [B, S, C], before the norm with
-    ``gain`` and ``shift``, of which text b has lens[b] rows -> embeddings [B, C]
-    float32, or None where its kernels do not take them. Rows that no text has are left
-    out, without the host's knowing how many those are. ``weights``: see
-    encoder_layers."""
-    B, S, C = emb.shape
-    M, HD = B * S, heads * dim
-    tensors = [emb, gain, shift, *weights]
-    if not (emb.is_cuda and dim in (64, 128) and M > ENCODER_PACKED_FROM
-            and M * max(3 * HD, inner, C) < 1 << 31
-            and C % 64 == HD % 64 == inner % 64 == 0 and C <= 2048
-            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
+def _embedding_ok(ids, tok, pos, gain, shift) -> bool:
+    """Whether a kernel can look up the rows of ids [B, S] and norm them: all on the
+    current device, 16 bytes at a time."""
+    C = tok.shape[-1]
+    tensors = (tok, pos, gain, shift)
+    return (tok.is_cuda and ids.dtype is torch.int64 and ids.is_contiguous()
+            and ids.dim() == 2 and ids.numel() > 0 and ids.numel() * C < 1 << 31
+            and tok.dim() == pos.dim() == 2 and ids.shape[1] <= pos.shape[0]
+            and C % 8 == 0 and 0 < C <= 2048 and pos.shape[1] == C
+            and gain.shape == shift.shape == (C,)
+            and all(t.dtype is torch.bfloat16 and t.is_contiguous()
                     and t.data_ptr() % 16 == 0 for t in tensors)
-            and lens.device == emb.device and lens.dtype == torch.int32
+            and all(t.get_device() == torch.cuda.current_device()
+                    for t in (ids, *tensors))
+            and _tiles._memory(ids, *tensors)
+            and not (torch.is_grad_enabled()
+                     and any(t.requires_grad for t in tensors)))
+
+
+def embed_layernorm(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
+                    gain: torch.Tensor, shift: torch.Tensor, eps: float,
+                    dtype: torch.dtype) -> torch.Tensor:
+    """LayerNorm of tok[ids] + pos[:S], ids [B, S] -> [B, S, C]."""
+    B, S = ids.shape
+    if not (dtype is torch.bfloat16 and _embedding_ok(ids, tok, pos, gain, shift)):
+        h = torch.nn.functional.embedding(ids, tok) + pos[:S].unsqueeze(0)
+        return layernorm(h.to(dtype), gain, shift, eps)
+    out = torch.empty(B, S, tok.shape[1], dtype=dtype, device=ids.device)
+    require_lib().fei_embed_layernorm(
+        _ptr(out), _ptr(ids), _ptr(tok), _ptr(pos), _ptr(gain), _ptr(shift), B, S,
+        tok.shape[1], tok.shape[0], eps, None, _stream())
+    return out
+
+
+def encoder_packed(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
+                   gain: torch.Tensor, shift: torch.Tensor, weights, heads: int,
+                   dim: int, inner: int, lens: torch.Tensor, eps: float
+                   ) -> Optional[torch.Tensor]:
+    """An encoder over texts of unlike lengths: ids [B, S], of which text b has lens[b],
+    and what embed_layernorm takes -> embeddings [B, C] float32, or None where its
+    kernels do not take them. Rows that no text has are left out, without the host's
+    knowing how many those are. ``weights``: see encoder_layers."""
+    B, S = ids.shape
+    C, HD = tok.shape[1], heads * dim
+    M = B * S
+    if not (tok.is_cuda and dim in (64, 128) and M > ENCODER_PACKED_FROM
+            and M * max(3 * HD, inner, C) < 1 << 31
+            and C % 64 == HD % 64 == inner % 64 == 0
+            and _embedding_ok(ids, tok, pos, gain, shift)
+            and all(t.dtype is torch.bfloat16 and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 and t.get_device() == ids.get_device()
+                    for t in weights)
+            and lens.device == ids.device and lens.dtype is torch.int32
             and lens.shape == (B,) and lens.is_contiguous()
-            and emb.get_device() == torch.cuda.current_device()
-            and _tiles._memory(*tensors, lens)
+            and _tiles.types_ok(lens, *weights)
             and _prefill_splits(B, heads, S, S) == 1):
         return None
 
     def rows(n):
-        return torch.empty(M, n, dtype=emb.dtype, device=emb.device)
+        return torch.empty(M, n, dtype=tok.dtype, device=ids.device)
     room = [rows(n) for n in (C, C, C, 3 * HD, HD, inner)]
-    starts = torch.empty(B + 1, dtype=torch.int32, device=emb.device)
-    out = torch.empty(B, C, dtype=torch.float32, device=emb.device)
+    starts = torch.empty(B + 1, dtype=torch.int32, device=ids.device)
+    out = torch.empty(B, C, dtype=torch.float32, device=ids.device)
     parts, many = None, M > ENCODER_PACKED_ROWS
     if many:
         p1, p2 = (_tiles.parts_up_to(M, C, k) for k in (HD, inner))
@@ -1009,10 +1046,11 @@ def encoder_packed(emb: torch.Tensor, gain: torch.Tensor, shift: torch.Tensor,
     p1, p2 = (p if p > 1 else 0 for p in (p1, p2))
     if p1 or p2:
         parts = torch.empty(max(p1, p2) * M * C, dtype=torch.float32,
-                            device=emb.device)
+                            device=ids.device)
     require_lib().fei_encoder_packed(
         (_vp * len(weights))(*(t.data_ptr() for t in weights)),
-        len(weights) // 12, _ptr(out), _ptr(emb), _ptr(gain), _ptr(shift),
+        len(weights) // 12, _ptr(out), _ptr(ids), _ptr(tok), _ptr(pos), tok.shape[0],
+        _ptr(gain), _ptr(shift),
         *(_ptr(t) for t in room), _ptr(lens), _ptr(starts), B, S, heads, dim, C,
         inner, 1.0 / math.sqrt(dim), eps, many,
         None if parts is None else _ptr(parts), p1, p2, _stream())

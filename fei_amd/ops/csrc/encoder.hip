@@ -348,8 +348,13 @@ void fei_layernorm_packed(void* out, const void* x, const void* res,
                           int cols, float eps, const int* starts,
                           hipStream_t stream);
 
+void fei_embed_layernorm(void* out, const long* ids, const void* tok, const void* pos,
+                         const void* w, const void* bias, int texts, int S, int cols,
+                         int vocab, float eps, const int* starts,
+                         hipStream_t stream);
+
 // An encoder over the rows that its texts have, one behind another: out [B, C] float32.
-// emb [B, S, C] is what the first norm (gain, shift) takes; w: 12 a layer, as in
+// ids [B, S] of tok [vocab, C]; pos [S, C]; gain and shift of the first norm; w: 12 a layer, as in
 // fei_encoder_layers; h, h1 and tmp have room for B * S rows of C, qkv of 3 H D, att of
 // H D, inner of I; starts for B + 1. How many rows there are only the device knows: grids
 // are made for all B * S, and blocks that have none leave. many: whether
@@ -363,8 +368,9 @@ void fei_layernorm_packed(void* out, const void* x, const void* res,
 // 1 PFLOP/s of tiles that fill the chip one and a half times. To find the number costs each kernel
 // a load before its first, 30 us of the 570 that 320 rows take in all.
 void fei_encoder_packed(const void* const* w, int layers, float* out,
-                        const void* emb, const void* gain, const void* shift,
-                        void* h, void* h1, void* tmp, void* qkv, void* att,
+                        const long* ids, const void* tok, const void* pos,
+                        int vocab, const void* gain, const void* shift, void* h,
+                        void* h1, void* tmp, void* qkv, void* att,
                         void* inner, const int* lens, int* starts, int B, int S,
                         int H, int D, int C, int I, float scale, float eps,
                         int many, float* parts, int p1, int p2,
@@ -373,8 +379,8 @@ void fei_encoder_packed(const void* const* w, int layers, float* out,
   const int* count = starts + B;
   hipLaunchKernelGGL(k_text_starts, dim3(1), dim3(1024), 0, stream, starts,
                      lens, B, S);
-  fei_layernorm_packed(h, emb, nullptr, gain, shift, B, S, C, eps, starts,
-                       stream);
+  fei_embed_layernorm(h, ids, tok, pos, gain, shift, B, S, C, vocab, eps, starts,
+                      stream);
   auto product = [&](void* to, const void* x, const void* const* wb, int N, int K,
                      bool gelu) {
     constexpr int TILE_GELU = 2, TILE_BIAS = 5;

@@ -640,13 +640,16 @@ namespace {
 // PACK: text b of at most S rows has rows starts[b] to starts[b + 1] - 1 of ``out``.
 // ALL_ROWS: x is [texts, S, cols], and the rows that a text has not are left out;
 // PACKED_ROWS: x and res are packed already.
+// EMBED: of text b's token s x has row ids[b, s], and res row s; their sum is rounded to
+// bfloat16. Two launches less: an encoder of 24 tokens 388 -> 382 us.
 enum { NO_PACK, ALL_ROWS, PACKED_ROWS };
-template <int V, bool RES, int PACK = NO_PACK>   // V loads of 8 columns a lane
-__global__ void __launch_bounds__(256)
+template <int V, bool RES, int PACK = NO_PACK, bool EMBED = false>
+__global__ void __launch_bounds__(256)               // V loads of 8 columns a lane
 k_layernorm_wave(u16* __restrict__ out, const u16* __restrict__ x,
                  const u16* __restrict__ res, const u16* __restrict__ w,
                  const u16* __restrict__ bias, int rows, int cols, float eps,
-                 const int* __restrict__ starts, int S) {
+                 const int* __restrict__ starts, int S,
+                 const long* __restrict__ ids, int vocab) {
   const int lane = threadIdx.x & 63;
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
@@ -658,8 +661,13 @@ k_layernorm_wave(u16* __restrict__ out, const u16* __restrict__ x,
   }
   if (PACK == PACKED_ROWS && row >= starts[rows / S]) return;
   const int nv = cols >> 3;
-  const s16x8* xr = (const s16x8*)(x + (long)row * cols);
-  const s16x8* rr = (const s16x8*)(res + (long)row * cols);
+  long from = row;
+  if (EMBED) {
+    from = ids[row];
+    if (from < 0 || from >= vocab) __builtin_trap();   // as torch's embedding does
+  }
+  const s16x8* xr = (const s16x8*)(x + from * cols);
+  const s16x8* rr = (const s16x8*)(res + (long)(EMBED ? row % S : row) * cols);
   s16x8 xv[V], rv[RES ? V : 1], wv[V], bv[V];
 #pragma unroll
   for (int i = 0; i < V; ++i) {
@@ -680,6 +688,7 @@ k_layernorm_wave(u16* __restrict__ out, const u16* __restrict__ x,
     for (int j = 0; j < 8; ++j) {
       f[i][j] = bf2f((u16)xv[i][j]);
       if (RES) f[i][j] += bf2f((u16)rv[i][j]);
+      if (EMBED) f[i][j] = bf2f(f2bf(f[i][j]));
       if (lane + 64 * i < nv) sum += f[i][j];
     }
   const float mean = wave_reduce_sum(sum) / (float)cols;
@@ -772,7 +781,7 @@ void fei_add_layernorm(void* out, const void* x, const void* res,
     hipLaunchKernelGGL(kernel, dim3((rows + 3) / 4), dim3(256), 0, stream,
                        (u16*)out, (const u16*)x, (const u16*)res,
                        (const u16*)w, (const u16*)bias, rows, cols, eps,
-                       nullptr, 0);
+                       nullptr, 0, nullptr, 0);
   };
   if (nv >= 1 && nv <= 64)
     return by_wave(has_res ? k_layernorm_wave<1, true>
@@ -790,24 +799,43 @@ void fei_add_layernorm(void* out, const void* x, const void* res,
                      has_res);
 }
 
-// Of the rows that texts have; starts has texts + 1 values. Without res x is [texts, S,
-// cols], with it x and res are packed. cols % 8 == 0, at most 2048.
+// LayerNorm of packed x + res: of the rows that texts have; starts has texts + 1 values.
+// cols % 8 == 0, at most 2048.
 void fei_layernorm_packed(void* out, const void* x, const void* res,
                           const void* w, const void* bias, int texts, int S,
                           int cols, float eps, const int* starts,
                           hipStream_t stream) {
   const int rows = texts * S, nv = cols >> 3;
-  auto by_wave = [&](auto kernel) {
+  auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3((rows + 3) / 4), dim3(256), 0, stream,
                        (u16*)out, (const u16*)x, (const u16*)res,
                        (const u16*)w, (const u16*)bias, rows, cols, eps,
-                       starts, S);
+                       starts, S, nullptr, 0);
   };
-#define GO(V) by_wave(res ? k_layernorm_wave<V, true, PACKED_ROWS>           \
-                          : k_layernorm_wave<V, false, ALL_ROWS>)
-  if (nv <= 64) return GO(1);
-  if (nv <= 128) return GO(2);
-  GO(4);
+  if (nv <= 64) go(k_layernorm_wave<1, true, PACKED_ROWS>);
+  else if (nv <= 128) go(k_layernorm_wave<2, true, PACKED_ROWS>);
+  else go(k_layernorm_wave<4, true, PACKED_ROWS>);
+}
+
+// LayerNorm of the sum of the rows of tok [vocab, cols] that ids [texts, S] name and of
+// pos [S, cols]: of all, or with starts those that texts have, packed. All bfloat16 on 16
+// bytes, cols % 8 == 0, at most 2048.
+void fei_embed_layernorm(void* out, const long* ids, const void* tok, const void* pos,
+                         const void* w, const void* bias, int texts, int S, int cols,
+                         int vocab, float eps, const int* starts,
+                         hipStream_t stream) {
+  const int rows = texts * S, nv = cols >> 3;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((rows + 3) / 4), dim3(256), 0, stream,
+                       (u16*)out, (const u16*)tok, (const u16*)pos,
+                       (const u16*)w, (const u16*)bias, rows, cols, eps,
+                       starts, S, ids, vocab);
+  };
+#define GO(V) go(starts ? k_layernorm_wave<V, true, ALL_ROWS, true>           \
+                        : k_layernorm_wave<V, true, NO_PACK, true>)
+  if (nv <= 64) GO(1);
+  else if (nv <= 128) GO(2);
+  else GO(4);
 #undef GO
 }
 

@@ -827,6 +827,27 @@ def test_encoder_norms_inside_products(lib, B, S, heads, inner):
     assert got.isfinite().all() and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("B,S,C", [(1, 1, 8), (2, 3, 512), (5, 7, 520), (3, 9, 768),
+                                   (1, 512, 1032), (2, 2, 2048)])
+def test_embedding_and_its_norm(lib, B, S, C):
+    """The bits of a look-up, a sum and a norm; what it does not read as it lies goes
+    there, and positions that there are not are refused as they were."""
+    ids = torch.randint(0, 100, (B, S), device=DEV)
+    ids[0, 0], ids[-1, -1] = 99, 0
+    tok, pos = randbf(100, C, seed=1), randbf(512, C, seed=2)
+    w, b = 1 + 0.1 * randbf(C, seed=3), randbf(C, seed=4)
+    want = lib.layernorm(torch.nn.functional.embedding(ids, tok) + pos[:S], w, b, 1e-6)
+    args = (w, b, 1e-6, torch.bfloat16)
+    assert lib._embedding_ok(ids, tok, pos, w, b)
+    assert torch.equal(lib.embed_layernorm(ids, tok, pos, *args), want)
+    wide = torch.cat([tok, tok], 1)[:, :C]
+    assert not lib._embedding_ok(ids, wide, pos, w, b)
+    assert torch.equal(lib.embed_layernorm(ids, wide, pos, *args), want)
+    if S > 1:
+        with pytest.raises(RuntimeError):
+            lib.embed_layernorm(ids, tok, pos[:S - 1] if S > 2 else pos[:0], *args)
+
+
 @pytest.mark.parametrize("B,S,lengths", [
     (3, 214, [214, 0, 1]), (9, 77, [77, 76, 64, 65, 1, 0, 13, 500, -3]),
     (2, 512, [1, 512]), (1500, 2, None),         # tiles of 64 x 64
