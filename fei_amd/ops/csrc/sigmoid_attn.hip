@@ -239,22 +239,30 @@ k_sig_conv(T* __restrict__ q, const T* __restrict__ proj, long ps,
   }
 }
 
-// State after the portions: their last projected rows. grid (portions, taps,
-// ceil(channels / 256))
+// State after the portions: their last projected rows, of which ``blocks`` blocks of NT
+// threads each write a share, a row's NT channels at a time. As a launch of its own this
+// took 4.2 us in each of 16 layers, nearly all of it the launch: portions of 1500 and 200 rows
+// and 6 tokens take 4083 us with it in the attention's launch, 4111 before.
 template <typename T>
-__global__ void __launch_bounds__(256)
-k_sig_state(float* __restrict__ states, const T* __restrict__ proj, long ps,
-            const int* __restrict__ spans, const int* __restrict__ slots,
-            int seq0, int taps, int CH) {
-  const int* sp = spans + blockIdx.x * 3;
-  const int a = blockIdx.y, n = sp[1];
-  if (a >= n) return;
-  const int p = sp[2] + n - 1 - a;
-  const T* src = proj + (long)(sp[0] + n - 1 - a) * ps;
-  const int i = blockIdx.z * 256 + threadIdx.x;
-  if (i < CH)
-    states[((long)slots[seq0 + blockIdx.x] * taps + p % taps) * CH + i] =
-        El<T>::ld(src[i]);
+struct States {
+  float* to;           // null: none are kept
+  const T* proj;
+  long ps;
+  const int* slots;
+  int portions, taps, CH;
+};
+template <typename T, int NT>
+__device__ __forceinline__ void write_states(const States<T>& s, const int* spans,
+                                             int seq0, int block, int blocks) {
+  const int parts = (s.CH + NT - 1) / NT;
+  for (int u = block; u < s.portions * s.taps * parts; u += blocks) {
+    const int row = u / parts, pt = row / s.taps, a = row - pt * s.taps;
+    const int n = spans[pt * 3 + 1], p = spans[pt * 3 + 2] + n - 1 - a;
+    const int ch = (u - row * parts) * NT + threadIdx.x;
+    if (a < n && ch < s.CH)
+      s.to[((long)s.slots[seq0 + pt] * s.taps + p % s.taps) * s.CH + ch] =
+          El<T>::ld(s.proj[(long)(spans[pt * 3] + n - 1 - a) * s.ps + ch]);
+  }
 }
 
 // Place of a key of a tile of 64 in the order of the second product.
@@ -262,7 +270,8 @@ __device__ __forceinline__ int key_place(int key) {
   return (key & 32) + ((key & 15) >> 2) * 8 + ((key >> 4) & 1) * 4 + (key & 3);
 }
 
-// Attention of prompt portions. grid (heads, query tiles, 128 / (16 NW QS)); a
+// Attention of prompt portions, whose convolution has read the states already: they are
+// written here. grid (heads, query tiles + 1 if states are kept, 128 / (16 NW QS)); a
 // wave owns QS sets of 16 queries, which share the fragments it reads, the
 // block walks the keys they see in tiles of 64 held in LDS: keys row-major,
 // values transposed. The distance bias depends on query - key alone: a tile's
@@ -276,7 +285,7 @@ k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
               const T* __restrict__ rows, const float* __restrict__ bias,
               const int* __restrict__ spans, const int* __restrict__ tiles,
               const int* __restrict__ table, int seq0, int W, int bs_log,
-              Geo g) {
+              Geo g, const States<T> states) {
   typedef typename El<T>::frag frag;
   constexpr int NP = Parts<T>::n;
   constexpr int NT = NW * 64, NQ = NW * 16 * QS;
@@ -289,7 +298,11 @@ k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
 
   const int h = blockIdx.x, gk = h / (g.heads / g.kvh);
   // a portion's last queries see the most keys: they start first
-  const int tile = gridDim.y - 1 - blockIdx.y;
+  const int tile = (int)gridDim.y - (states.to ? 2 : 1) - (int)blockIdx.y;
+  if (tile < 0) {                          // the last blocks: a launch of 4 us spared
+    if (blockIdx.z == 0) write_states<T, NT>(states, spans, seq0, h, gridDim.x);
+    return;
+  }
   const int pt = tiles[tile * 2];
   const int row0 = spans[pt * 3], cnt = spans[pt * 3 + 1];
   const int pos0 = spans[pt * 3 + 2];
@@ -852,19 +865,13 @@ void run_conv(T* q, const T* proj, long ps, T* rows, float* states, Conv cv,
 #undef BY_LG
 #undef CONV_RUN
 #undef CONV
-  const int CH = g.heads * g.dim + g.kvh * (g.dim + g.vdim);
-  if (states)
-    hipLaunchKernelGGL(k_sig_state<T>,
-                       dim3(n_portions, cv.taps, (CH + 255) / 256), dim3(256),
-                       0, stream, states, proj, ps, spans, slots, seq0,
-                       cv.taps, CH);
 }
 
 template <typename T, int KS, int DC, bool VEC>
 void launch_prefill(T* out, long os, const T* q, const T* rows,
                     const float* bias, const int* spans, const int* tiles,
                     const int* table, int n_tiles, int seq0, int W, int bs_log,
-                    Geo g, hipStream_t stream) {
+                    Geo g, const States<T>& states, hipStream_t stream) {
   // the registers of two sets of queries suffice up to these sizes
   constexpr int QS = sizeof(T) == 2 && KS <= 4 && DC <= 8 ? 2 : 1;
   constexpr int NW = sizeof(T) == 2 ? 8 / QS : 4;
@@ -872,20 +879,20 @@ void launch_prefill(T* out, long os, const T* q, const T* rows,
   const size_t lds = sizeof(T) * (64 * (KS * 32 + 8) + DC * 16 * 64) +
                      16 * (NQ + 68);
   allow_lds(k_sig_prefill<T, KS, DC, NW, QS, VEC>, lds);
-  const dim3 grid(g.heads, n_tiles, 128 / NQ);
+  const dim3 grid(g.heads, n_tiles + (states.to ? 1 : 0), 128 / NQ);
   hipLaunchKernelGGL((k_sig_prefill<T, KS, DC, NW, QS, VEC>), grid,
                      dim3(NW * 64), lds, stream, out, os, q, rows, bias,
-                     spans, tiles, table, seq0, W, bs_log, g);
+                     spans, tiles, table, seq0, W, bs_log, g, states);
 }
 
 template <typename T>
 void run_prefill(T* out, long os, const T* q, const T* rows,
                  const float* bias, const int* spans, const int* tiles,
                  const int* table, int n_tiles, int seq0, int W, int bs_log,
-                 Geo g, hipStream_t stream) {
+                 Geo g, const States<T>& states, hipStream_t stream) {
 #define PRE(KS, DC, VEC)                                                     \
   launch_prefill<T, KS, DC, VEC>(out, os, q, rows, bias, spans, tiles,       \
-                                 table, n_tiles, seq0, W, bs_log, g, stream)
+                                 table, n_tiles, seq0, W, bs_log, g, states, stream)
 #define BY_DC(KS)                             \
   do {                                        \
     if (g.vdim <= 64) PRE(KS, 4, true);       \
@@ -947,15 +954,21 @@ void fei_sig_prefill(void* out, long os, const void* q, const void* rows,
                      const float* bias, const int* spans, const int* tiles,
                      const int* table, int n_tiles, int seq0, int W,
                      int bs_log, int heads, int kvh, int dim, int vdim,
-                     int window, float scale, int f32, hipStream_t stream) {
+                     int window, float scale, float* states, const void* proj,
+                     long ps, const int* slots, int n_portions, int taps, int f32,
+                     hipStream_t stream) {
   const Geo g{heads, kvh, dim, vdim, scale, window};
+  const int CH = heads * dim + kvh * (dim + vdim);
   if (f32)
     run_prefill<float>((float*)out, os, (const float*)q, (const float*)rows,
                        bias, spans, tiles, table, n_tiles, seq0, W, bs_log, g,
+                       {states, (const float*)proj, ps, slots, n_portions, taps, CH},
                        stream);
   else
     run_prefill<u16>((u16*)out, os, (const u16*)q, (const u16*)rows, bias,
-                     spans, tiles, table, n_tiles, seq0, W, bs_log, g, stream);
+                     spans, tiles, table, n_tiles, seq0, W, bs_log, g,
+                     {states, (const u16*)proj, ps, slots, n_portions, taps, CH},
+                     stream);
 }
 
 }  // extern "C"

@@ -639,6 +639,23 @@ def test_mixed_batches(tmp_path, name, device):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("conv", [1, 3, 5])
+def test_states_of_many_portions(tmp_path, conv, device):
+    """Portions shorter and longer than the convolution in one batch, two for
+    each sequence, then a token of each: every slot holds its own last rows."""
+    cfg = make_cfg([(att(heads=2, dim=88, vdim=84, conv=conv), None)])
+    net = Net(tmp_path, cfg, 25, device)
+    r = net.runner(slots=14)
+    tokens = {r.admit(): toks(2 * n + 1, cfg["vocab"], 80 + n) for n in range(1, 15)}
+    for part in range(2):
+        r.step([StepEntry(sid, t[part * (len(t) // 2):][:len(t) // 2])
+                for sid, t in tokens.items()])
+    got = r.step([StepEntry(sid, t[-1:]) for sid, t in tokens.items()])
+    for row, t in zip(got.cpu(), tokens.values()):
+        assert err(row[None], net.want(t)[-1:]) < F32_TOL, len(t)
+
+
+@pytest.mark.parametrize("device", DEVICES)
 def test_decode_batches(tmp_path, device):
     """Single tokens of 1 to 9 sequences of unlike lengths, each as alone."""
     net = Net(tmp_path, CONFIGS["even"], 24, device)
