@@ -153,13 +153,9 @@ class SigmoidAttention(Mixer):
                 "k.conv": ck, "v.conv": cv}
 
     def run(self, proj, out, batch, cache, run, rot) -> None:
-        args = (self.m, self, batch, cache.rows[run], cache.states[run],
-                cache.block_size)
-        n = batch.n_dec
-        if n:
-            ops.sigmoid_attn_decode(proj[:n], out[:n], *args)
-        if batch.portions:
-            ops.sigmoid_attn_prefill(proj, out, *args)
+        ops.sigmoid_attn_mixed(proj, out, self.m, self, batch, cache.rows[run],
+                               cache.states[run], cache.block_size)
+
 
 
 MIXERS = {"latent_attention": LatentAttention, "gla": GatedLinearAttention,

@@ -37,7 +37,8 @@ from fei_amd.ops.moe import (  # noqa: F401
 from fei_amd.ops.rows import (  # noqa: F401
     add_norm_parts, product_parts, rope_kv_parts, rows_ok)
 from fei_amd.ops.sigmoid_attn import (  # noqa: F401
-    check_sigmoid_geometry, sigmoid_attn_decode, sigmoid_attn_prefill)
+    check_sigmoid_geometry, sigmoid_attn_decode, sigmoid_attn_mixed,
+    sigmoid_attn_prefill)
 from fei_amd.ops.tiles import (  # noqa: F401
     parts_ok as tile_parts_ok, parts_pay as tile_parts_pay,
     product_parts as tile_parts)

@@ -18,6 +18,8 @@
 //
 // T is u16 (bfloat16 bits) or float. Scores, weights and sums are float32; a
 // weight enters a bfloat16 product as a high and a low part.
+#include <algorithm>
+
 #include "fei_attn.h"
 
 namespace {
@@ -36,7 +38,7 @@ struct Conv {
   float eps;
 };
 
-__device__ __forceinline__ int channels(const Geo& g) {
+__host__ __device__ __forceinline__ int channels(const Geo& g) {
   return g.heads * g.dim + g.kvh * (g.dim + g.vdim);
 }
 
@@ -271,8 +273,8 @@ __device__ __forceinline__ int key_place(int key) {
 }
 
 // Attention of prompt portions, whose convolution has read the states already: they are
-// written here. grid (heads, query tiles + 1 if states are kept, 128 / (16 NW QS)); a
-// wave owns QS sets of 16 queries, which share the fragments it reads, the
+// written here. Blocks (heads h, query tiles + 1 if states are kept y, 128 / (16 NW QS)
+// z); a wave owns QS sets of 16 queries, which share the fragments it reads, the
 // block walks the keys they see in tiles of 64 held in LDS: keys row-major,
 // values transposed. The distance bias depends on query - key alone: a tile's
 // NW * 16 * QS + 63 values are computed once, in four copies shifted by one
@@ -280,12 +282,12 @@ __device__ __forceinline__ int key_place(int key) {
 // KS >= ceil(dim / 32), DC >= ceil(vdim / 16); queries are zero beyond dim,
 // columns beyond vdim are not stored.
 template <typename T, int KS, int DC, int NW, int QS, bool VEC>
-__global__ void __launch_bounds__(NW * 64, 2)
-k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
+__device__ __forceinline__ void
+prefill_block(T* __restrict__ out, long os, const T* __restrict__ q,
               const T* __restrict__ rows, const float* __restrict__ bias,
               const int* __restrict__ spans, const int* __restrict__ tiles,
               const int* __restrict__ table, int seq0, int W, int bs_log,
-              Geo g, const States<T> states) {
+              const Geo& g, const States<T>& states, int h, int y, int ny, int z) {
   typedef typename El<T>::frag frag;
   constexpr int NP = Parts<T>::n;
   constexpr int NT = NW * 64, NQ = NW * 16 * QS;
@@ -296,17 +298,17 @@ k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
   T* vt = kt + 64 * DS;                    // [DC * 16][64], see vt_at
   float* tb = (float*)(vt + DC * 16 * 64);  // [4][TB]
 
-  const int h = blockIdx.x, gk = h / (g.heads / g.kvh);
+  const int gk = h / (g.heads / g.kvh);
   // a portion's last queries see the most keys: they start first
-  const int tile = (int)gridDim.y - (states.to ? 2 : 1) - (int)blockIdx.y;
+  const int tile = ny - (states.to ? 2 : 1) - y;
   if (tile < 0) {                          // the last blocks: a launch of 4 us spared
-    if (blockIdx.z == 0) write_states<T, NT>(states, spans, seq0, h, gridDim.x);
+    if (z == 0) write_states<T, NT>(states, spans, seq0, h, g.heads);
     return;
   }
   const int pt = tiles[tile * 2];
   const int row0 = spans[pt * 3], cnt = spans[pt * 3 + 1];
   const int pos0 = spans[pt * 3 + 2];
-  const int q0 = tiles[tile * 2 + 1] + blockIdx.z * NQ;
+  const int q0 = tiles[tile * 2 + 1] + z * NQ;
   if (q0 >= cnt) return;
   const int qn = min(NQ, cnt - q0);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -510,6 +512,19 @@ k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
   }
 }
 
+// grid (heads, query tiles + 1 if states are kept, 128 / (16 NW QS))
+template <typename T, int KS, int DC, int NW, int QS, bool VEC>
+__global__ void __launch_bounds__(NW * 64, 2)
+k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
+              const T* __restrict__ rows, const float* __restrict__ bias,
+              const int* __restrict__ spans, const int* __restrict__ tiles,
+              const int* __restrict__ table, int seq0, int W, int bs_log,
+              Geo g, const States<T> states) {
+  prefill_block<T, KS, DC, NW, QS, VEC>(out, os, q, rows, bias, spans, tiles, table,
+                                        seq0, W, bs_log, g, states, blockIdx.x,
+                                        blockIdx.y, gridDim.y, blockIdx.z);
+}
+
 // Keys of a decode row in splits: base (a multiple of 32), keys per split.
 __device__ __forceinline__ void split_of(int p, int window, int splits,
                                          int least, int* base, int* chunk) {
@@ -519,21 +534,21 @@ __device__ __forceinline__ void split_of(int p, int window, int splits,
 }
 
 // Decode: one token of each sequence, from its projections to attention
-// outputs. grid (splits, kvh * ceil(group / 16), B); a block takes the keys of
+// outputs. Blocks (splits, kvh * ceil(group / 16), B); a block takes the keys of
 // one split for up to 16 heads that share a key/value head, a wave 32 keys at
 // a time. Every block makes the queries of its heads; the one whose split
 // ends with the new token also makes its key and value, writes its cache row
 // and reads them from LDS. Split 0 writes the state.
 // A lane holds CPL value columns: CPL * 16 >= vdim. KS >= ceil(dim / 32).
 template <typename T, int KS, int CPL, bool VEC>
-__global__ void
-__launch_bounds__(256, sizeof(T) == 2 && KS <= 4 && CPL <= 8 ? 2 : 1)
-k_sig_decode(T* __restrict__ out, long os, float* __restrict__ part,
+__device__ __forceinline__ void
+decode_block(T* __restrict__ out, long os, float* __restrict__ part,
              const T* __restrict__ proj, long ps, T* __restrict__ rows,
-             float* __restrict__ states, Conv cv,
+             float* __restrict__ states, const Conv& cv,
              const float* __restrict__ bias, const int* __restrict__ pos,
              const int* __restrict__ slots, const int* __restrict__ table,
-             int W, int bs_log, Geo g, int splits, int least) {
+             int W, int bs_log, const Geo& g, int splits, int least, int split, int y,
+             int b) {
   typedef typename El<T>::frag frag;
   constexpr int NP = Parts<T>::n;
   constexpr int DS = KS * 32 + 8;
@@ -544,9 +559,8 @@ k_sig_decode(T* __restrict__ out, long os, float* __restrict__ part,
   T* vn = kn + DS;                         // [VS]
   float* red = (float*)(vn + VS);          // [4][heads of the block][VS + 4]
 
-  const int split = blockIdx.x, b = blockIdx.z;
   const int hg = g.heads / g.kvh, ht = (hg + 15) / 16;
-  const int gk = blockIdx.y / ht, hy = blockIdx.y - gk * ht;
+  const int gk = y / ht, hy = y - gk * ht;
   const int h0 = gk * hg + hy * 16, nh = min(16, hg - hy * 16);
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
   const int l15 = lane & 15, lg = lane >> 4;
@@ -768,6 +782,48 @@ k_sig_decode(T* __restrict__ out, long os, float* __restrict__ part,
   }
 }
 
+template <typename T, int KS, int CPL, bool VEC>
+__global__ void
+__launch_bounds__(256, sizeof(T) == 2 && KS <= 4 && CPL <= 8 ? 2 : 1)
+k_sig_decode(T* __restrict__ out, long os, float* __restrict__ part,
+             const T* __restrict__ proj, long ps, T* __restrict__ rows,
+             float* __restrict__ states, Conv cv,
+             const float* __restrict__ bias, const int* __restrict__ pos,
+             const int* __restrict__ slots, const int* __restrict__ table,
+             int W, int bs_log, Geo g, int splits, int least) {
+  decode_block<T, KS, CPL, VEC>(out, os, part, proj, ps, rows, states, cv, bias, pos,
+                                slots, table, W, bs_log, g, splits, least, blockIdx.x,
+                                blockIdx.y, blockIdx.z);
+}
+
+// Prompt portions and the tokens beside them in one launch: k_sig_prefill's blocks behind
+// k_sig_decode's, of which there are ``nd`` (a multiple of 8: the blocks of a head stay on
+// one XCD). Neither reads a row or a state that the other writes. A token's block is a
+// chain of dependent loads (10 us for 1200 keys in 8 shares, and a sum of 4), a portion's
+// is bound by exponentials: 6 tokens beside 1500 + 200 rows, 32 heads of 64, with the
+// convolution 57.4 -> 46.2 us; a step of 16 layers 4270 -> 4053.
+template <int KS, int DC>
+__global__ void __launch_bounds__(256, 2)
+k_sig_both(u16* out, long os, float* part, const u16* q, const u16* proj, long ps,
+           u16* rows, Conv cv, const float* bias, const int* spans, const int* tiles,
+           const int* pos, const int* slots, const int* table, int B, int W, int bs_log,
+           Geo g, int splits, int least, int nd, const States<u16> states) {
+  const int id = blockIdx.x;
+  if (id < nd) {
+    const int hg = g.heads / g.kvh, ny = g.kvh * ((hg + 15) / 16);
+    const int split = id % splits, y = id / splits % ny, b = id / (splits * ny);
+    if (b < B)
+      decode_block<u16, KS, DC, true>(out, os, part, proj, ps, rows, states.to, cv, bias,
+                                      pos, slots, table, W, bs_log, g, splits, least,
+                                      split, y, b);
+    return;
+  }
+  prefill_block<u16, KS, DC, 4, 2, true>(out, os, q, rows, bias, spans, tiles, table, B, W,
+                                         bs_log, g, states, (id - nd) % g.heads,
+                                         (id - nd) / g.heads, (gridDim.x - nd) / g.heads,
+                                         0);
+}
+
 // Sum of the splits that had keys. grid (ceil(heads * vdim / 256), B)
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -867,6 +923,28 @@ void run_conv(T* q, const T* proj, long ps, T* rows, float* states, Conv cv,
 #undef CONV
 }
 
+template <int KS, int DC>
+void launch_both(u16* out, long os, float* part, const u16* q, u16* rows, const Conv& cv,
+                 const float* bias, const int* spans, const int* tiles, const int* pos,
+                 const int* table, int n_tiles, int B, int W, int bs_log, Geo g,
+                 int splits, int least, const States<u16>& states, hipStream_t stream) {
+  const int hg = g.heads / g.kvh;
+  const size_t lds = std::max(
+      2 * (64 * (KS * 32 + 8) + DC * 16 * 64) + 16 * (128 + 68),
+      2 * (17 * (KS * 32 + 8) + DC * 16) + 4 * 4 * std::min(hg, 16) * (DC * 16 + 4));
+  allow_lds(k_sig_both<KS, DC>, lds);
+  const int nd = (splits * g.kvh * ((hg + 15) / 16) * B + 7) / 8 * 8;
+  hipLaunchKernelGGL((k_sig_both<KS, DC>),
+                     dim3(nd + g.heads * (n_tiles + (states.to ? 1 : 0))), dim3(256), lds,
+                     stream, out, os, part, q, states.proj, states.ps, rows, cv, bias,
+                     spans, tiles, pos, states.slots, table, B, W, bs_log, g, splits,
+                     least, nd, states);
+  const int HV = g.heads * g.vdim;
+  if (splits > 1)
+    hipLaunchKernelGGL(k_sig_combine<u16>, dim3((HV + 255) / 256, B), dim3(256), 0,
+                       stream, out, os, part, pos, g.window, splits, least, HV);
+}
+
 template <typename T, int KS, int DC, bool VEC>
 void launch_prefill(T* out, long os, const T* q, const T* rows,
                     const float* bias, const int* spans, const int* tiles,
@@ -958,7 +1036,7 @@ void fei_sig_prefill(void* out, long os, const void* q, const void* rows,
                      long ps, const int* slots, int n_portions, int taps, int f32,
                      hipStream_t stream) {
   const Geo g{heads, kvh, dim, vdim, scale, window};
-  const int CH = heads * dim + kvh * (dim + vdim);
+  const int CH = channels(g);
   if (f32)
     run_prefill<float>((float*)out, os, (const float*)q, (const float*)rows,
                        bias, spans, tiles, table, n_tiles, seq0, W, bs_log, g,
@@ -969,6 +1047,29 @@ void fei_sig_prefill(void* out, long os, const void* q, const void* rows,
                      spans, tiles, table, n_tiles, seq0, W, bs_log, g,
                      {states, (const u16*)proj, ps, slots, n_portions, taps, CH},
                      stream);
+}
+
+// fei_sig_prefill and fei_sig_decode of the B tokens before the portions: bfloat16, dim and
+// vdim of up to 128, multiples of 8, os of 4.
+void fei_sig_both(void* out, long os, float* part, const void* q, const void* proj,
+                  long ps, void* rows, float* states, const float* conv, const float* qn,
+                  const float* kn, const float* bias, const int* spans, const int* tiles,
+                  const int* pos, const int* slots, const int* table, int n_tiles,
+                  int n_portions, int B, int W, int bs_log, int heads, int kvh, int dim,
+                  int vdim, int taps, int window, float scale, int splits, float eps,
+                  int least, hipStream_t stream) {
+  const Geo g{heads, kvh, dim, vdim, scale, window};
+  const Conv cv{conv, qn, kn, taps, eps};
+  const States<u16> st{states, (const u16*)proj, ps, slots, n_portions, taps, channels(g)};
+#define BOTH(KS, DC)                                                                   \
+  launch_both<KS, DC>((u16*)out, os, part, (const u16*)q, (u16*)rows, cv, bias, spans, \
+                      tiles, pos, table, n_tiles, B, W, bs_log, g, splits, least, st,  \
+                      stream)
+  if (dim <= 64 && vdim <= 64) BOTH(2, 4);
+  else if (dim <= 64) BOTH(2, 8);
+  else if (vdim <= 64) BOTH(4, 4);
+  else BOTH(4, 8);
+#undef BOTH
 }
 
 }  // extern "C"

@@ -9,6 +9,7 @@ import json
 import os
 import subprocess
 import sys
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -19,7 +20,7 @@ import step_helpers
 from fei_amd import ops
 from fei_amd.engine.config import (MODEL_SPECS, BokenexSpec, MoESpec,
                                    get_spec)
-from fei_amd.engine.step import StepEntry
+from fei_amd.engine.step import RaggedBatch, StepEntry
 from fei_amd.models.bokenex import BokenexModel
 from step_helpers import (DEVICES, F32_TOL, err, row_errors, run, run_mixed,
                           serve_sessions, toks)
@@ -653,6 +654,63 @@ def test_states_of_many_portions(tmp_path, conv, device):
     got = r.step([StepEntry(sid, t[-1:]) for sid, t in tokens.items()])
     for row, t in zip(got.cpu(), tokens.values()):
         assert err(row[None], net.want(t)[-1:]) < F32_TOL, len(t)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("conv", [1, 4])
+@pytest.mark.parametrize("window", [None, 100])
+@pytest.mark.parametrize("heads,kv,dim,vdim,dtype", [
+    (4, 2, 64, 64, torch.bfloat16), (5, 1, 24, 72, torch.bfloat16),
+    (34, 2, 72, 40, torch.bfloat16), (8, 8, 128, 128, torch.bfloat16),
+    (4, 2, 136, 64, torch.bfloat16), (5, 5, 67, 85, torch.bfloat16),
+    (4, 2, 64, 64, torch.float32)])
+def test_tokens_beside_portions(heads, kv, dim, vdim, dtype, window, conv):
+    """One call for both, against a call for each: the same bits of portions, cache and
+    states; the tokens', whose keys may be shared out otherwise, up to the rounding of a
+    result: bfloat16 keeps 8 bits."""
+    m = SimpleNamespace(heads=heads, kv_heads=kv, dim=dim, vdim=vdim, window=window,
+                        conv=conv, scale=dim ** -0.5)
+    net_rows = kv * (dim + vdim)
+    n_in = heads * dim + net_rows
+    g = torch.Generator(device="cuda").manual_seed(heads + dim)
+
+    def rand(*size, dtype=torch.float32):
+        return torch.randn(*size, device="cuda", generator=g).to(dtype)
+    w = SimpleNamespace(conv=rand(conv, n_in), qn=rand(dim), kn=rand(dim), eps=1e-5,
+                        bias=rand(3, heads).abs())
+    lens, new = [1, 70, 1030, 650, 37, 260, 129], [1, 1, 1, 1, 2, 130, 129]
+    W = -(-max(lens) // 16)
+    table = torch.randperm(len(lens) * W, device="cuda", generator=g)
+    row = [sum(new[:i]) for i in range(len(new))]
+
+    def ints(x):
+        return torch.tensor(x, dtype=torch.int32, device="cuda")
+    batch = RaggedBatch(
+        tokens=None, pos=ints([p for n, c in zip(lens, new) for p in range(n - c, n)]),
+        row_seq=ints([i for i, c in enumerate(new) for _ in range(c)]),
+        table=table.int().view(len(lens), W), slots=ints([3, 0, 6, 2, 1, 5, 4]),
+        n_dec=4,
+        portions=[(row[i], new[i], lens[i] - new[i]) for i in (4, 5, 6)])
+    batch._upload = lambda rows, width: ints(rows).view(-1, width)
+    proj = rand(sum(new), n_in, dtype=dtype)
+    cache, states = rand(len(lens) * W * 16, net_rows, dtype=dtype), rand(7, conv, n_in)
+    got, want = ([x.clone() for x in (cache, states if conv > 1 else None)
+                  if x is not None] for _ in range(2))
+    outs = [torch.zeros(sum(new), heads * vdim, dtype=dtype, device="cuda")
+            for _ in range(2)]
+    for out, mem, apart in ((outs[0], got, False), (outs[1], want, True)):
+        args = (m, w, batch, mem[0], mem[1] if conv > 1 else None, 16)
+        if apart:
+            ops.sigmoid_attn_decode(proj[:4], out[:4], *args)
+            ops.sigmoid_attn_prefill(proj, out, *args)
+        else:
+            ops.sigmoid_attn_mixed(proj, out, *args)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert torch.equal(outs[0][4:], outs[1][4:])
+    a, b = (o[:4].double() for o in outs)
+    # a rounding of either, and sums in float32 of up to 1030 values below the largest
+    assert ((a - b).abs() <= 2 ** -7 * b.abs() + 2 ** -12 * b.abs().max()).all()
 
 
 @pytest.mark.parametrize("device", DEVICES)
