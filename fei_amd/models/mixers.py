@@ -105,12 +105,7 @@ class GatedLinearAttention(Mixer):
         return {"norm": self.norm, "a2.b": self.bias, "a2": self.a2}
 
     def run(self, proj, out, batch, cache, run, rot) -> None:
-        args = (self.m, self, batch, cache.states[run])
-        n = batch.n_dec
-        if n:
-            ops.gla_decode(proj[:n], out[:n], *args)
-        if batch.portions:
-            ops.gla_prefill(proj, out, *args)
+        ops.gla_mixed(proj, out, self.m, self, batch, cache.states[run])
 
 
 class SigmoidAttention(Mixer):
@@ -155,7 +150,6 @@ class SigmoidAttention(Mixer):
     def run(self, proj, out, batch, cache, run, rot) -> None:
         ops.sigmoid_attn_mixed(proj, out, self.m, self, batch, cache.rows[run],
                                cache.states[run], cache.block_size)
-
 
 
 MIXERS = {"latent_attention": LatentAttention, "gla": GatedLinearAttention,

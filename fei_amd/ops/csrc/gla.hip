@@ -16,7 +16,8 @@
 //   k_gla_chunk   A, and each chunk's own sum for S'
 //   k_gla_scan    start state of every chunk, last state into the slot
 //   k_gla_out     o, head norm, output gate
-// Decode: k_gla_decode updates the state and reads it, k_gla_gate_out norms.
+// Decode: k_gla_decode updates the state and reads it, k_gla_gate_out norms; beside a
+// prompt blocks of k_gla_gate and of k_gla_scan do.
 //
 // A projected row is [q (H dim) | k (H dim) | v (H vdim) | gate (H vdim) |
 // decay input (rank)]; T is u16 (bfloat16 bits) or float.
@@ -42,16 +43,144 @@ __device__ __forceinline__ float log_decay(float z, float inv_tau) {
   return (fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * inv_tau;
 }
 
+// One token per sequence: S <- S diag(alpha) + v k^T, o = S q (float32, to
+// ``o`` [B][H vdim]). Blocks (heads h, ceil(vdim / 16) y, B b), 4 value rows a wave.
+// lpr: lanes that share a value row, a power of two; with vec each takes 4
+// channels at a time, otherwise one.
+template <typename T>
+__device__ __forceinline__ void
+decode_block(float* __restrict__ o, float* __restrict__ states,
+             const T* __restrict__ proj, long ps, const float* __restrict__ a2,
+             const float* __restrict__ bias, const int* __restrict__ pos,
+             const int* __restrict__ slots, const Gla& g, int lpr, int vec, int h,
+             int y, int b) {
+  __shared__ __align__(16) float q[256], k[256], al[256], a1[256];
+  const int tid = threadIdx.x;
+  const T* pr = proj + (long)b * ps;
+  const bool fresh = pos[b] == 0;
+  if (tid < g.rank) a1[tid] = El<T>::ld(pr[g.a_off() + tid]);
+  __syncthreads();
+  if (tid < g.dim) {
+    const int c = h * g.dim + tid;
+    float z = bias[c];
+    for (int r = 0; r < g.rank; ++r) z = fmaf(a2[(long)c * g.rank + r], a1[r], z);
+    al[tid] = expf(log_decay(z, 1.f / g.tau));
+    q[tid] = El<T>::ld(pr[c]) / sqrtf((float)g.dim);
+    k[tid] = El<T>::ld(pr[g.k_off() + c]);
+  }
+  __syncthreads();
+  const int w = tid >> 6, lane = tid & 63;
+  const int rpw = 64 / lpr, sub = lane % lpr, rw = lane / lpr;
+  float* base = states +
+      ((long)slots[b] * g.heads + h) * g.vdim * g.dim;
+  for (int i = 0; i < 4; i += rpw) {
+    const int e = y * 16 + w * 4 + i + rw;
+    const bool on = i + rw < 4 && e < g.vdim;
+    float acc = 0.f;
+    if (on) {
+      float* s = base + (long)e * g.dim;
+      const float v = El<T>::ld(pr[g.v_off() + h * g.vdim + e]);
+      if (vec) {
+        for (int d = sub * 4; d < g.dim; d += lpr * 4) {
+          f32x4 x = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *(f32x4*)(s + d);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            x[j] = fmaf(al[d + j], x[j], v * k[d + j]);
+            acc = fmaf(x[j], q[d + j], acc);
+          }
+          *(f32x4*)(s + d) = x;
+        }
+      } else {
+        for (int d = sub; d < g.dim; d += lpr) {
+          const float x = fmaf(al[d], fresh ? 0.f : s[d], v * k[d]);
+          acc = fmaf(x, q[d], acc);
+          s[d] = x;
+        }
+      }
+    }
+    for (int off = lpr >> 1; off; off >>= 1) acc += __shfl_xor(acc, off);
+    if (on && sub == 0) o[(long)b * g.vo() + h * g.vdim + e] = acc;
+  }
+}
+
+// out = rms(o) * nw * silu(gate) of a head, by one wave.
+template <typename T>
+__device__ __forceinline__ void
+gate_out(T* __restrict__ out, long os, const float* __restrict__ o,
+         const T* __restrict__ proj, long ps, const float* __restrict__ nw,
+         const Gla& g, float eps, int h, int b) {
+  const int lane = threadIdx.x & 63;
+  const float* x = o + (long)b * g.vo() + h * g.vdim;
+  float ss = 0.f;
+  for (int e = lane; e < g.vdim; e += 64) ss = fmaf(x[e], x[e], ss);
+  ss = wave_reduce_sum(ss);
+  const float inv = 1.f / sqrtf(ss / (float)g.vdim + eps);
+  for (int e = lane; e < g.vdim; e += 64) {
+    const float gv = El<T>::ld(proj[(long)b * ps + g.g_off() + h * g.vdim + e]);
+    out[(long)b * os + h * g.vdim + e] =
+        El<T>::st(x[e] * inv * nw[e] * gv * sigmoid_f(gv));
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_gla_decode(float* __restrict__ o, float* __restrict__ states,
+             const T* __restrict__ proj, long ps, const float* __restrict__ a2,
+             const float* __restrict__ bias, const int* __restrict__ pos,
+             const int* __restrict__ slots, Gla g, int lpr, int vec) {
+  decode_block<T>(o, states, proj, ps, a2, bias, pos, slots, g, lpr, vec, blockIdx.x,
+                  blockIdx.y, blockIdx.z);
+}
+
+// grid (heads, B)
+template <typename T>
+__global__ void __launch_bounds__(64)
+k_gla_gate_out(T* __restrict__ out, long os, const float* __restrict__ o,
+               const T* __restrict__ proj, long ps,
+               const float* __restrict__ nw, Gla g, float eps) {
+  gate_out<T>(out, os, o, proj, ps, nw, g, eps, blockIdx.x, blockIdx.y);
+}
+
+// The B tokens that a step has beside its portions: their decay, state and product run in
+// k_gla_gate's launch, their norm in k_gla_scan's, between which nothing else reads them.
+// Launches of their own take 7.3 and 4.9 us, chains of loads on an idle chip. 4 tokens
+// beside 1297 rows, 8 heads of 128 and 256: 38.1 us for the four launches, 27.7 for the
+// two that are left.
+struct Tokens {
+  int B;
+  float* o;                // [B][H vdim]
+  const int* pos;
+  int lpr, vec;
+};
+// Lanes that share a value row of a decode block.
+int lanes_per_row(const Gla& g) {
+  const int need = g.dim % 4 == 0 ? g.dim / 4 : g.dim;
+  int lpr = 16;
+  while (lpr < 64 && lpr < need) lpr <<= 1;
+  return lpr;
+}
+
 // chunks [.][3]: portion, first row, rows. G [T][H dim].
-// grid (chunks, ceil(H dim / 64)): 64 channels x 4 groups of 16 tokens.
+// Blocks: ``heads * ceil(vdim / 16) * B`` of the tokens, then (chunks, ceil(H dim / 64)):
+// 64 channels x 4 groups of 16 rows.
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_gla_gate(float* __restrict__ G, const T* __restrict__ proj, long ps,
            const float* __restrict__ a2, const float* __restrict__ bias,
-           const int* __restrict__ chunks, Gla g) {
+           const int* __restrict__ chunks, int n_chunks, float* __restrict__ states,
+           const int* __restrict__ slots, Gla g, Tokens tk) {
   extern __shared__ float as[];            // [rank][CH]
   __shared__ float tot[4][64];
-  const int row0 = chunks[blockIdx.x * 3 + 1], n = chunks[blockIdx.x * 3 + 2];
+  const int vt = (g.vdim + 15) / 16;
+  const int id = (int)blockIdx.x - tk.B * g.heads * vt;
+  if (id < 0) {
+    const int i = blockIdx.x, y = i / g.heads;
+    decode_block<T>(tk.o, states, proj, ps, a2, bias, tk.pos, slots, g, tk.lpr, tk.vec,
+                    i % g.heads, y % vt, y / vt);
+    return;
+  }
+  const int ch = id % n_chunks;
+  const int row0 = chunks[ch * 3 + 1], n = chunks[ch * 3 + 2];
   for (int i = threadIdx.x; i < CH * g.rank; i += 256) {
     const int t = i / g.rank, r = i - t * g.rank;
     as[r * CH + t] = t < n ? El<T>::ld(proj[(long)(row0 + t) * ps + g.a_off() + r])
@@ -60,7 +189,7 @@ k_gla_gate(float* __restrict__ G, const T* __restrict__ proj, long ps,
   __syncthreads();
   const float inv_tau = 1.f / g.tau;
   const int cx = threadIdx.x & 63, sb = threadIdx.x >> 6;
-  const int c = blockIdx.y * 64 + cx;
+  const int c = id / n_chunks * 64 + cx;
   float z[16];
   if (c < g.kq()) {
     const float b = bias[c];
@@ -332,17 +461,27 @@ k_gla_chunk(float* __restrict__ U, float* __restrict__ A,
 
 // U becomes the start state of each chunk; the last state goes to the slot.
 // spans [P][4]: first chunk, chunks, first position, sequence. grid
-// (state values / 256, P); NB chunks are read ahead of the recurrence.
+// (state values / 256, 1 if there are tokens, whose outputs it makes, + P); NB
+// chunks are read ahead of the recurrence.
+template <typename T>
 __global__ void __launch_bounds__(256)
 k_gla_scan(float* __restrict__ U, const float* __restrict__ G,
            float* __restrict__ states, const int* __restrict__ chunks,
            const int* __restrict__ spans, const int* __restrict__ slots,
-           Gla g) {
+           T* __restrict__ out, long os, const T* __restrict__ proj, long ps,
+           const float* __restrict__ nw, Gla g, float eps, Tokens tk) {
   constexpr int NB = 8;
+  const int pt = (int)blockIdx.y - (tk.B > 0);
+  if (pt < 0) {
+    for (int i = blockIdx.x * 4 + (threadIdx.x >> 6); i < tk.B * g.heads;
+         i += gridDim.x * 4)
+      gate_out<T>(out, os, tk.o, proj, ps, nw, g, eps, i % g.heads, i / g.heads);
+    return;
+  }
   const long size = (long)g.heads * g.vdim * g.dim;
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
   if (i >= size) return;
-  const int* sp = spans + blockIdx.y * 4;
+  const int* sp = spans + pt * 4;
   const int c0 = sp[0], nc = sp[1];
   float* slot = states + (long)slots[sp[3]] * size + i;
   const int hd = (int)(i / ((long)g.vdim * g.dim)) * g.dim + (int)(i % g.dim);
@@ -481,96 +620,14 @@ k_gla_out(T* __restrict__ out, long os, const float* __restrict__ S,
   }
 }
 
-// One token per sequence: S <- S diag(alpha) + v k^T, o = S q (float32, to
-// ``o`` [B][H vdim]). grid (heads, ceil(vdim / 16), B), 4 value rows a wave.
-// lpr: lanes that share a value row, a power of two; with vec each takes 4
-// channels at a time, otherwise one.
-template <typename T>
-__global__ void __launch_bounds__(256)
-k_gla_decode(float* __restrict__ o, float* __restrict__ states,
-             const T* __restrict__ proj, long ps, const float* __restrict__ a2,
-             const float* __restrict__ bias, const int* __restrict__ pos,
-             const int* __restrict__ slots, Gla g, int lpr, int vec) {
-  __shared__ __align__(16) float q[256], k[256], al[256], a1[256];
-  const int h = blockIdx.x, b = blockIdx.z, tid = threadIdx.x;
-  const T* pr = proj + (long)b * ps;
-  const bool fresh = pos[b] == 0;
-  if (tid < g.rank) a1[tid] = El<T>::ld(pr[g.a_off() + tid]);
-  __syncthreads();
-  if (tid < g.dim) {
-    const int c = h * g.dim + tid;
-    float z = bias[c];
-    for (int r = 0; r < g.rank; ++r) z = fmaf(a2[(long)c * g.rank + r], a1[r], z);
-    al[tid] = expf(log_decay(z, 1.f / g.tau));
-    q[tid] = El<T>::ld(pr[c]) / sqrtf((float)g.dim);
-    k[tid] = El<T>::ld(pr[g.k_off() + c]);
-  }
-  __syncthreads();
-  const int w = tid >> 6, lane = tid & 63;
-  const int rpw = 64 / lpr, sub = lane % lpr, rw = lane / lpr;
-  float* base = states +
-      ((long)slots[b] * g.heads + h) * g.vdim * g.dim;
-  for (int i = 0; i < 4; i += rpw) {
-    const int e = blockIdx.y * 16 + w * 4 + i + rw;
-    const bool on = i + rw < 4 && e < g.vdim;
-    float acc = 0.f;
-    if (on) {
-      float* s = base + (long)e * g.dim;
-      const float v = El<T>::ld(pr[g.v_off() + h * g.vdim + e]);
-      if (vec) {
-        for (int d = sub * 4; d < g.dim; d += lpr * 4) {
-          f32x4 x = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : *(f32x4*)(s + d);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            x[j] = fmaf(al[d + j], x[j], v * k[d + j]);
-            acc = fmaf(x[j], q[d + j], acc);
-          }
-          *(f32x4*)(s + d) = x;
-        }
-      } else {
-        for (int d = sub; d < g.dim; d += lpr) {
-          const float x = fmaf(al[d], fresh ? 0.f : s[d], v * k[d]);
-          acc = fmaf(x, q[d], acc);
-          s[d] = x;
-        }
-      }
-    }
-    for (int off = lpr >> 1; off; off >>= 1) acc += __shfl_xor(acc, off);
-    if (on && sub == 0) o[(long)b * g.vo() + h * g.vdim + e] = acc;
-  }
-}
-
-// out = rms(o) * nw * silu(gate) per head. grid (heads, B), one wave.
-template <typename T>
-__global__ void __launch_bounds__(64)
-k_gla_gate_out(T* __restrict__ out, long os, const float* __restrict__ o,
-               const T* __restrict__ proj, long ps,
-               const float* __restrict__ nw, Gla g, float eps) {
-  const int h = blockIdx.x, b = blockIdx.y;
-  const float* x = o + (long)b * g.vo() + h * g.vdim;
-  float ss = 0.f;
-  for (int e = threadIdx.x; e < g.vdim; e += 64) ss = fmaf(x[e], x[e], ss);
-  ss = wave_reduce_sum(ss);
-  const float inv = 1.f / sqrtf(ss / (float)g.vdim + eps);
-  for (int e = threadIdx.x; e < g.vdim; e += 64) {
-    const float gv = El<T>::ld(proj[(long)b * ps + g.g_off() + h * g.vdim + e]);
-    out[(long)b * os + h * g.vdim + e] =
-        El<T>::st(x[e] * inv * nw[e] * gv * sigmoid_f(gv));
-  }
-}
-
 template <typename T>
 void run_gla_decode(T* out, long os, float* o, float* states, const T* proj,
                     long ps, const float* a2, const float* bias,
                     const float* nw, const int* pos, const int* slots, int B,
                     Gla g, float eps, hipStream_t stream) {
-  const int vec = g.dim % 4 == 0;
-  const int need = vec ? g.dim / 4 : g.dim;
-  int lpr = 16;
-  while (lpr < 64 && lpr < need) lpr <<= 1;
   hipLaunchKernelGGL(k_gla_decode<T>, dim3(g.heads, (g.vdim + 15) / 16, B),
                      dim3(256), 0, stream, o, states, proj, ps, a2, bias, pos,
-                     slots, g, lpr, vec);
+                     slots, g, lanes_per_row(g), g.dim % 4 == 0);
   hipLaunchKernelGGL(k_gla_gate_out<T>, dim3(g.heads, B), dim3(64), 0, stream,
                      out, os, o, proj, ps, nw, g, eps);
 }
@@ -605,9 +662,10 @@ void run_gla_prefill(T* out, long os, const T* proj, long ps, const float* a2,
                      const float* bias, const float* nw, float* states,
                      const int* chunks, int n, const int* spans, int P,
                      const int* slots, float* G, float* U, float* A, Gla g,
-                     float eps, hipStream_t stream) {
-  hipLaunchKernelGGL(k_gla_gate<T>, dim3(n, (g.kq() + 63) / 64), dim3(256),
-                     4 * CH * g.rank, stream, G, proj, ps, a2, bias, chunks, g);
+                     float eps, const Tokens& tk, hipStream_t stream) {
+  const int blocks = n * ((g.kq() + 63) / 64) + tk.B * g.heads * ((g.vdim + 15) / 16);
+  hipLaunchKernelGGL(k_gla_gate<T>, dim3(blocks), dim3(256), 4 * CH * g.rank, stream, G,
+                     proj, ps, a2, bias, chunks, n, states, slots, g, tk);
   // quads of q, k, v, G and S lie on 8- and 16-byte borders
   const int vec = g.dim % 4 == 0 && g.vdim % 4 == 0 && ps % 4 == 0 &&
                   (size_t)proj % 16 == 0;
@@ -617,8 +675,9 @@ void run_gla_prefill(T* out, long os, const T* proj, long ps, const float* a2,
   else if (dt <= 8) launch_chunk<T, 8>(U, A, G, proj, ps, chunks, n, g, vec, stream);
   else launch_chunk<T, 16>(U, A, G, proj, ps, chunks, n, g, vec, stream);
   const long size = (long)g.heads * g.vdim * g.dim;
-  hipLaunchKernelGGL(k_gla_scan, dim3((size + 255) / 256, P), dim3(256), 0,
-                     stream, U, G, states, chunks, spans, slots, g);
+  hipLaunchKernelGGL(k_gla_scan<T>, dim3((size + 255) / 256, P + (tk.B > 0)),
+                     dim3(256), 0, stream, U, G, states, chunks, spans, slots, out, os,
+                     proj, ps, nw, g, eps, tk);
 #define OUT(DK, NV)                                                         \
   launch_out<T, DK, NV>(out, os, U, A, G, proj, ps, nw, chunks, n, g, eps,  \
                         vec, stream)
@@ -656,23 +715,25 @@ void fei_gla_decode(void* out, long os, float* o, float* states,
                         bias, nw, pos, slots, B, g, eps, stream);
 }
 
-// Workspaces: G [T][H dim], U [chunks][H][vdim][dim], A [chunks][H][64][64].
+// Workspaces: G [T][H dim], U [chunks][H][vdim][dim], A [chunks][H][64][64]. Of the first
+// B rows each is a token of its sequence, and o [B][H vdim] room for them.
 void fei_gla_prefill(void* out, long os, const void* proj, long ps,
                      const float* a2, const float* bias, const float* nw,
                      float* states, const int* chunks, int n_chunks,
                      const int* spans, int n_spans, const int* slots, float* G,
-                     float* U, float* A, int heads, int dim, int vdim,
-                     int rank, float tau, float eps, int f32,
+                     float* U, float* A, int B, float* o, const int* pos, int heads,
+                     int dim, int vdim, int rank, float tau, float eps, int f32,
                      hipStream_t stream) {
   const Gla g{heads, dim, vdim, rank, tau};
+  const Tokens tk{B, o, pos, lanes_per_row(g), dim % 4 == 0};
   if (f32)
     run_gla_prefill<float>((float*)out, os, (const float*)proj, ps, a2, bias,
                            nw, states, chunks, n_chunks, spans, n_spans, slots,
-                           G, U, A, g, eps, stream);
+                           G, U, A, g, eps, tk, stream);
   else
     run_gla_prefill<u16>((u16*)out, os, (const u16*)proj, ps, a2, bias, nw,
                          states, chunks, n_chunks, spans, n_spans, slots, G, U,
-                         A, g, eps, stream);
+                         A, g, eps, tk, stream);
 }
 
 }  // extern "C"

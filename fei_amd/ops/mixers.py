@@ -51,7 +51,7 @@ def declare(lib: ctypes.CDLL) -> None:
         [_vp, _l, _vp, _vp, _vp, _l] + [_vp] * 5 + [_i] * 5 + [_f, _f, _i, _vp])
     lib.fei_gla_prefill.argtypes = (
         [_vp, _l, _vp, _l] + [_vp] * 5 + [_i, _vp, _i] + [_vp] * 4 +
-        [_i] * 4 + [_f, _f, _i, _vp])
+        [_i, _vp, _vp] + [_i] * 4 + [_f, _f, _i, _vp])
 
 
 def _lib() -> ctypes.CDLL:
@@ -604,6 +604,22 @@ def gla_prefill(proj, out, m, w, batch, states) -> None:
             _gla_cpu(proj[row:row + n], out[row:row + n], m, w,
                      states[int(batch.slots[batch.n_dec + i])], pos0 == 0)
         return
+    _gla_prefill(proj, out, m, w, batch, states, 0)
+
+
+def gla_mixed(proj, out, m, w, batch, states) -> None:
+    """gla_decode of the first n_dec rows and gla_prefill of the others, in the launches
+    of the latter where there are both."""
+    if proj.is_cuda and batch.n_dec and batch.portions:
+        _gla_prefill(proj, out, m, w, batch, states, batch.n_dec)
+        return
+    if batch.n_dec:
+        gla_decode(proj[:batch.n_dec], out[:batch.n_dec], m, w, batch, states)
+    if batch.portions:
+        gla_prefill(proj, out, m, w, batch, states)
+
+
+def _gla_prefill(proj, out, m, w, batch, states, tokens: int) -> None:
     dev = proj.device
     chunks, spans = batch.chunk_plan()
     n = chunks.shape[0]
@@ -611,8 +627,10 @@ def gla_prefill(proj, out, m, w, batch, states) -> None:
     G = torch.empty(proj.shape[0], m.heads * m.dim, **f)
     U = torch.empty(n, m.heads, m.vdim, m.dim, **f)
     A = torch.empty(n, m.heads, 64, 64, **f)
+    o = torch.empty(tokens, m.heads * m.vdim, **f)
     _lib().fei_gla_prefill(
         _p(out), out.stride(0), _p(proj), proj.stride(0), _p(w.a2),
         _p(w.bias), _p(w.norm), _p(states), _p(chunks), n, _p(spans),
-        spans.shape[0], _p(batch.slots), _p(G), _p(U), _p(A), m.heads, m.dim,
-        m.vdim, m.gate_rank, m.tau, w.eps, _f32(proj), _stream())
+        spans.shape[0], _p(batch.slots), _p(G), _p(U), _p(A), tokens,
+        _p(o), _p(batch.pos) if tokens else None, m.heads, m.dim, m.vdim,
+        m.gate_rank, m.tau, w.eps, _f32(proj), _stream())

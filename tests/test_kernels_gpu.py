@@ -978,6 +978,40 @@ def test_gla_prompt_tiles(lib, dim, vdim, dtype, tol):
     assert bool((s[3] == 1).all())
 
 
+@pytest.mark.parametrize("B", [1, 3, 70])
+@pytest.mark.parametrize("H,dim,vdim,rank", [(1, 16, 40, 8), (3, 30, 33, 16),
+                                             (8, 128, 256, 16), (2, 256, 512, 32)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gla_tokens_beside_prompts(lib, B, H, dim, vdim, rank, dtype):
+    """One call for both gives the bits of a call for each."""
+    from types import SimpleNamespace as NS
+    from fei_amd.ops import mixers as mx
+    parts = [(B, 70, 0), (B + 70, 2, 5), (B + 72, 64, 9)]
+    T = B + 136
+    g = torch.Generator(device=DEV).manual_seed(dim + B)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    up = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    m = NS(heads=H, dim=dim, vdim=vdim, gate_rank=rank, tau=8.0)
+    w = NS(a2=rand(H * dim, rank) * 0.3, bias=rand(H * dim), norm=rand(vdim), eps=1e-5)
+    proj = rand(T, 2 * H * dim + 2 * H * vdim + rank).to(dtype)
+    chunks, spans = [], []
+    for i, (row, n, pos0) in enumerate(parts):
+        spans.append([len(chunks), -(-n // 64), pos0, B + i])
+        chunks += [[i, row + a, min(64, n - a)] for a in range(0, n, 64)]
+    slots = torch.randperm(B + 4, generator=g, device=DEV)[:B + 3].int()
+    pos = torch.arange(T, device=DEV).int()      # the first token starts its sequence
+    batch = NS(portions=parts, n_dec=B, slots=slots, pos=pos,
+               chunk_plan=lambda: (up(chunks), up(spans)))
+    states = rand(B + 4, H, vdim, dim)
+    outs, mems = ([x.clone() for _ in range(2)]
+                  for x in (torch.zeros(T, H * vdim, dtype=dtype, device=DEV), states))
+    mx.gla_mixed(proj, outs[0], m, w, batch, mems[0])
+    mx.gla_decode(proj[:B], outs[1][:B], m, w, batch, mems[1])
+    mx.gla_prefill(proj, outs[1], m, w, batch, mems[1])
+    assert torch.equal(*outs) and torch.equal(*mems)
+    assert not torch.equal(mems[0], states)
+
+
 # -- largest values ----------------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
