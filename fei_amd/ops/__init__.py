@@ -968,8 +968,8 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
 # their products run in tiles of 64 x 64, beyond in k_tile's. Us of 12 layers of 768,
 # texts of a quarter to all of the length (all of one length), with padding, in tiles of
 # 64, in k_tile's: 512 rows 618, 636 (670); 768 745, 658 (747); 1500 1631, 800 (1021),
-# 1094 (1136); 2560 1429, 1053 (1265), 1153 (1260); 3200 1431, 1150 (1537), 1250 (1369);
-# 5120 1694, 1550 (2164), 1522 (1747).
+# 1094 (1136); 2560 1429, 1053 (1265), 1153 (1260); 3200 1431, 1150 (1537), 1253 (1406);
+# 5120 1694, 1550 (2164), 1424 (1710).
 ENCODER_PACKED_FROM = 640
 ENCODER_PACKED_ROWS = 3072
 
