@@ -68,13 +68,8 @@ class LatentAttention(Mixer):
 
     def run(self, proj, out, batch, cache, run, rot) -> None:
         m = self.m
-        args = (m, self, rot[m.rot_dim, m.rot_base], batch, cache.rows[run],
-                cache.block_size)
-        n = batch.n_dec
-        if n:
-            ops.latent_attn_decode(proj[:n], out[:n], *args)
-        if batch.portions:
-            ops.latent_attn_prefill(proj, out, *args)
+        ops.latent_attn_mixed(proj, out, m, self, rot[m.rot_dim, m.rot_base], batch,
+                              cache.rows[run], cache.block_size)
 
 
 class GatedLinearAttention(Mixer):

@@ -30,8 +30,8 @@ from fei_amd.ops.layers import llama_few  # noqa: F401
 from fei_amd.ops.mixers import (  # noqa: F401
     GainNorm, GainNormed, cat_cast, check_gla_geometry,
     check_latent_geometry, embed_pos, gain_logits, gla_decode, gla_mixed, gla_prefill,
-    latent_attn_decode, latent_attn_prefill, linear_f32, logits_head, mix_in,
-    norm_pair, parallel_in, residual_linear, residual_norms)
+    latent_attn_decode, latent_attn_mixed, latent_attn_prefill, linear_f32,
+    logits_head, mix_in, norm_pair, parallel_in, residual_linear, residual_norms)
 from fei_amd.ops.moe import (  # noqa: F401
     check_moe_geometry, residual_moe, route)
 from fei_amd.ops.rows import (  # noqa: F401

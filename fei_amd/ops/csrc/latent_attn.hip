@@ -53,16 +53,28 @@ __device__ __forceinline__ void append_row(const T* __restrict__ ckr,
   }
 }
 
-// Prompt rows: cache row, and the rotated part of every query in place.
+// What the prompt portions of a step need before their product, done by blocks of the
+// launches of the tokens beside them, which are few and bound by latency. 4 tokens
+// beside 1297 rows, latents of 512: 33 us for the four launches, 25.6 for the two that are
+// left.
 template <typename T>
-__global__ void __launch_bounds__(256)
-k_latent_append(T* __restrict__ proj, long ps, T* __restrict__ rows,
-                const float* __restrict__ nw, const float* __restrict__ rotab,
-                const int* __restrict__ pos, const int* __restrict__ row_seq,
-                const int* __restrict__ table, int W, int bs_log, Geo g,
-                float eps) {
-  __shared__ float red[4];
-  const int t = blockIdx.x;
+struct Beside {
+  int n;                   // rows of the portions; 0: none
+  T* proj;                 // the first of them
+  const int *pos, *row_seq;
+  int n_keys;              // cached rows that they see, see k_latent_gather
+  T *c, *kr;
+  const int *owner, *spans;
+};
+
+// Prompt row t: cache row, and the rotated part of every query in place.
+template <typename T>
+__device__ __forceinline__ void
+append_prompt(T* __restrict__ proj, long ps, T* __restrict__ rows,
+              const float* __restrict__ nw, const float* __restrict__ rotab,
+              const int* __restrict__ pos, const int* __restrict__ row_seq,
+              const int* __restrict__ table, int W, int bs_log, const Geo& g,
+              float eps, int t, float* red) {
   const int p = pos[t];
   T* pr = proj + (long)t * ps;
   const float* cs = rotab + (long)p * g.rot;
@@ -82,7 +94,45 @@ k_latent_append(T* __restrict__ proj, long ps, T* __restrict__ rows,
   }
 }
 
-// Decode rows: grid (heads + 1, ceil(kr / 128), B). Block x = heads appends
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_latent_append(T* __restrict__ proj, long ps, T* __restrict__ rows,
+                const float* __restrict__ nw, const float* __restrict__ rotab,
+                const int* __restrict__ pos, const int* __restrict__ row_seq,
+                const int* __restrict__ table, int W, int bs_log, Geo g,
+                float eps) {
+  __shared__ float red[4];
+  append_prompt<T>(proj, ps, rows, nw, rotab, pos, row_seq, table, W, bs_log, g, eps,
+                   blockIdx.x, red);
+}
+
+// Cached row of key i of those that the portions see, packed one portion after another:
+// its latents to c [n, kr], its rotated part to kr_out [n, rot], by NL lanes of which this
+// is number l. spans [P][5]: first row, rows, first position, first key, first packed key.
+template <typename T, int NL>
+__device__ __forceinline__ void
+gather_key(T* __restrict__ c, T* __restrict__ kr_out, const T* __restrict__ rows,
+           const int* __restrict__ owner, const int* __restrict__ spans,
+           const int* __restrict__ table, int W, int bs_log, int seq0, const Geo& g,
+           int vec, int i, int l) {
+  const int p = owner[i];
+  const int key = spans[p * 5 + 3] + i - spans[p * 5 + 4];
+  const int R = g.kr + g.rot;
+  const T* src = rows + cache_row(table, W, seq0 + p, key, bs_log) * R;
+  if (vec) {
+    for (int j = l * 8; j < g.kr; j += NL * 8)
+      st8(c + (long)i * g.kr + j, ld8(src + j));
+    for (int j = l * 8; j < g.rot; j += NL * 8)
+      st8(kr_out + (long)i * g.rot + j, ld8(src + g.kr + j));
+  } else {
+    for (int j = l; j < g.kr; j += NL) c[(long)i * g.kr + j] = src[j];
+    for (int j = l; j < g.rot; j += NL)
+      kr_out[(long)i * g.rot + j] = src[g.kr + j];
+  }
+}
+
+// Decode rows: grid (heads + 1, ceil(kr / 128), B, and behind them blocks for the rows of
+// the portions). Block x = heads appends
 // the token's cache row; the others make 128 columns of q' = W_uk^T q of one
 // head (16 groups of 8 columns x 16 groups of rows of W_uk), and block y = 0
 // the rotated query.
@@ -92,10 +142,17 @@ k_latent_absorb(const T* __restrict__ proj, long ps, T* __restrict__ qa,
                 const T* __restrict__ wuk, T* __restrict__ rows,
                 const float* __restrict__ nw, const float* __restrict__ rotab,
                 const int* __restrict__ pos, const int* __restrict__ table,
-                int W, int bs_log, Geo g, float eps) {
+                int B, int W, int bs_log, Geo g, float eps, const Beside<T> bs) {
   __shared__ float qs[256];
   __shared__ float part[16][128];
   const int h = blockIdx.x, b = blockIdx.z, tid = threadIdx.x;
+  if (b >= B) {
+    const int t = ((b - B) * gridDim.y + blockIdx.y) * gridDim.x + h;
+    if (t < bs.n)
+      append_prompt<T>(bs.proj, ps, rows, nw, rotab, bs.pos, bs.row_seq, table, W,
+                       bs_log, g, eps, t, qs);
+    return;
+  }
   const int p = pos[b];
   const int D = g.dim + g.rot, R = g.kr + g.rot;
   const T* pr = proj + (long)b * ps;
@@ -155,7 +212,8 @@ k_latent_absorb(const T* __restrict__ proj, long ps, T* __restrict__ qa,
   }
 }
 
-// Decode partials. grid (splits, ceil(heads / 16 NH), B). The visible
+// Decode partials. grid (splits, ceil(heads / 16 NH), B, and behind them blocks that
+// gather the keys of the portions). The visible
 // keys of row b are cut into ``splits`` chunks of a multiple of KT keys; a
 // block walks its chunk in tiles of KT cached rows held in LDS, which NH groups
 // of 4 waves use for 16 heads each. For the scores a group's waves share out
@@ -168,8 +226,16 @@ __global__ void __launch_bounds__(256 * NH)
 k_latent_decode(const T* __restrict__ qa, const T* __restrict__ rows,
                 float* __restrict__ part_o, float* __restrict__ part_ml,
                 const int* __restrict__ pos, const int* __restrict__ table,
-                int W, int bs_log, Geo g, int splits, int KT, int Rs,
-                int vec) {
+                int B, int W, int bs_log, Geo g, int splits, int KT, int Rs,
+                int vec, const Beside<T> bs) {
+  if ((int)blockIdx.z >= B) {
+    const int e = ((blockIdx.z - B) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    const int i = e * 4 * NH + (threadIdx.x >> 6);
+    if (i < bs.n_keys)
+      gather_key<T, 64>(bs.c, bs.kr, rows, bs.owner, bs.spans, table, W, bs_log, B, g,
+                        g.kr % 8 == 0 && g.rot % 8 == 0, i, threadIdx.x & 63);
+    return;
+  }
   typedef typename El<T>::frag frag;
   constexpr int NP = Parts<T>::n;
   constexpr int NQ = 9;                    // steps per wave: R <= 4 * 9 * 32
@@ -436,31 +502,14 @@ k_latent_out(T* __restrict__ out, long os, const float* __restrict__ part_o,
   }
 }
 
-// Cached rows of the keys that the prompt portions see, packed one portion
-// after another: latents [n, kr] and rotated parts [n, rot].
-// spans [P][5]: first row, rows, first position, first key, first packed key.
 template <typename T>
 __global__ void __launch_bounds__(128)
 k_latent_gather(T* __restrict__ c, T* __restrict__ kr_out,
                 const T* __restrict__ rows, const int* __restrict__ owner,
                 const int* __restrict__ spans, const int* __restrict__ table,
                 int W, int bs_log, int seq0, Geo g, int vec) {
-  const int i = blockIdx.x;
-  const int p = owner[i];
-  const int key = spans[p * 5 + 3] + i - spans[p * 5 + 4];
-  const int R = g.kr + g.rot;
-  const T* src = rows + cache_row(table, W, seq0 + p, key, bs_log) * R;
-  if (vec) {
-    for (int j = threadIdx.x * 8; j < g.kr; j += blockDim.x * 8)
-      st8(c + (long)i * g.kr + j, ld8(src + j));
-    for (int j = threadIdx.x * 8; j < g.rot; j += blockDim.x * 8)
-      st8(kr_out + (long)i * g.rot + j, ld8(src + g.kr + j));
-  } else {
-    for (int j = threadIdx.x; j < g.kr; j += blockDim.x)
-      c[(long)i * g.kr + j] = src[j];
-    for (int j = threadIdx.x; j < g.rot; j += blockDim.x)
-      kr_out[(long)i * g.rot + j] = src[g.kr + j];
-  }
+  gather_key<T, 128>(c, kr_out, rows, owner, spans, table, W, bs_log, seq0, g, vec,
+                     blockIdx.x, threadIdx.x);
 }
 
 // Flash attention of prompt portions over expanded keys and values.
@@ -907,18 +956,19 @@ int run_decode(T* out, long os, const T* proj, long ps, const T* wuk,
                const T* wuv, const float* nw, const float* rotab, T* rows,
                const int* pos, const int* table, T* qa, float* part_o,
                float* part_ml, int B, int W, int bs_log, Geo g, float eps,
-               int splits, int tile, hipStream_t stream) {
+               int splits, int tile, const Beside<T>& bs, hipStream_t stream) {
   const int R = g.kr + g.rot;
   const bool vkr = g.kr % 8 == 0;
-  const dim3 ga(g.heads + 1, (g.kr + 127) / 128, B);
+  const int wa = (g.heads + 1) * ((g.kr + 127) / 128);
+  const dim3 ga(g.heads + 1, (g.kr + 127) / 128, B + (bs.n + wa - 1) / wa);
   if (vkr)
     hipLaunchKernelGGL((k_latent_absorb<T, true>), ga, dim3(256), 0, stream,
-                       proj, ps, qa, wuk, rows, nw, rotab, pos, table, W,
-                       bs_log, g, eps);
+                       proj, ps, qa, wuk, rows, nw, rotab, pos, table, B, W,
+                       bs_log, g, eps, bs);
   else
     hipLaunchKernelGGL((k_latent_absorb<T, false>), ga, dim3(256), 0, stream,
-                       proj, ps, qa, wuk, rows, nw, rotab, pos, table, W,
-                       bs_log, g, eps);
+                       proj, ps, qa, wuk, rows, nw, rotab, pos, table, B, W,
+                       bs_log, g, eps, bs);
 
   const int Rs = (R + 31) / 32 * 32 + 8;
   const int nh = g.heads > 16 ? 2 : 1;     // groups of 16 heads per block
@@ -930,13 +980,15 @@ int run_decode(T* out, long os, const T* proj, long ps, const T* wuk,
   int KT = tile;
   while (KT > 16 && lds(KT) > 160 * 1024) KT >>= 1;
   if (lds(KT) > 160 * 1024 || R > 1152) return 1;
-  const dim3 gd(splits, (g.heads + 16 * nh - 1) / (16 * nh), B);
+  const int hb = (g.heads + 16 * nh - 1) / (16 * nh), wd = splits * hb * 4 * nh;
+  const dim3 gd(splits, hb, B + (bs.n_keys + wd - 1) / wd);
 #define DEC(N, H)                                                            \
   do {                                                                       \
     allow_lds(k_latent_decode<T, N, H>, lds(KT));                            \
     hipLaunchKernelGGL((k_latent_decode<T, N, H>), gd, dim3(256 * H),        \
                        lds(KT), stream, qa, rows, part_o, part_ml, pos,      \
-                       table, W, bs_log, g, splits, KT, Rs, R % 8 == 0);     \
+                       table, B, W, bs_log, g, splits, KT, Rs, R % 8 == 0,   \
+                       bs);                                                  \
   } while (0)
 #define BY_NCT(H)               \
   do {                          \
@@ -1022,7 +1074,9 @@ void run_window(T* out, long os, const T* proj, long ps, const T* kv,
 
 extern "C" {
 
-// tile: keys per LDS tile, 16, 32 or 64; fewer are taken if they do not fit.
+// tile: keys per LDS tile, 16, 32 or 64; fewer are taken if they do not fit. n > 0: also
+// fei_latent_append of the n rows of proj behind the B tokens' and fei_latent_gather of
+// the n_keys that they see; pos has the positions of all rows.
 // Returns 0, or 1 if the sizes do not fit the kernel's LDS tiles.
 int fei_latent_decode(void* out, long os, const void* proj, long ps,
                       const void* wuk, const void* wuv, const float* nw,
@@ -1030,18 +1084,24 @@ int fei_latent_decode(void* out, long os, const void* proj, long ps,
                       const int* table, void* qa, float* part_o,
                       float* part_ml, int B, int W, int bs_log, int heads,
                       int dim, int rot, int vdim, int kr, float scale,
-                      int window, float eps, int splits, int tile, int f32,
+                      int window, float eps, int splits, int tile, int n,
+                      const int* row_seq, int n_keys, void* c, void* krot,
+                      const int* owner, const int* spans, int f32,
                       hipStream_t stream) {
   const Geo g{heads, dim, rot, vdim, kr, scale, window};
   if (f32)
     return run_decode<float>((float*)out, os, (const float*)proj, ps,
                              (const float*)wuk, (const float*)wuv, nw, rotab,
                              (float*)rows, pos, table, (float*)qa, part_o,
-                             part_ml, B, W, bs_log, g, eps, splits, tile, stream);
+                             part_ml, B, W, bs_log, g, eps, splits, tile,
+                             {n, (float*)proj + B * ps, pos + B, row_seq, n_keys,
+                              (float*)c, (float*)krot, owner, spans}, stream);
   return run_decode<u16>((u16*)out, os, (const u16*)proj, ps,
                          (const u16*)wuk, (const u16*)wuv, nw, rotab,
                          (u16*)rows, pos, table, (u16*)qa, part_o, part_ml, B,
-                         W, bs_log, g, eps, splits, tile, stream);
+                         W, bs_log, g, eps, splits, tile,
+                         {n, (u16*)proj + B * ps, pos + B, row_seq, n_keys, (u16*)c,
+                          (u16*)krot, owner, spans}, stream);
 }
 
 void fei_latent_append(void* proj, long ps, void* rows, const float* nw,

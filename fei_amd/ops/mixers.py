@@ -40,7 +40,7 @@ def declare(lib: ctypes.CDLL) -> None:
         [_vp] * 5 + [_f] + [_vp, _l] + [_i] * 5 + [_vp])
     lib.fei_latent_decode.argtypes = (
         [_vp, _l, _vp, _l] + [_vp] * 10 + [_i] * 8 +
-        [_f, _i, _f, _i, _i, _i, _vp])
+        [_f, _i, _f, _i, _i, _i, _vp, _i] + [_vp] * 4 + [_i, _vp])
     lib.fei_latent_decode.restype = _i
     lib.fei_latent_append.argtypes = (
         [_vp, _l] + [_vp] * 6 + [_i] * 8 + [_f, _i, _vp])
@@ -489,7 +489,13 @@ def latent_attn_decode(proj, out, m, w, rot, batch, rows,
                 w.uv, m.scale)[0]
         _latent_out(o, proj, m, out)
         return
-    B, dev = proj.shape[0], proj.device
+    _latent_decode(proj, out, m, w, rot, batch, rows, block_size, proj.shape[0],
+                   (0, None, 0, None, None, None, None))
+
+
+def _latent_decode(proj, out, m, w, rot, batch, rows, block_size: int, B: int,
+                   beside: tuple) -> None:
+    dev = proj.device
     W = batch.table.shape[1]
     n_max = W * block_size
     if m.window is not None:
@@ -509,7 +515,7 @@ def latent_attn_decode(proj, out, m, w, rot, batch, rows,
         _p(w.norm), _p(rot), _p(rows), _p(batch.pos), _p(batch.table), _p(qa),
         _p(part_o), _p(part_ml), B, W, block_size.bit_length() - 1, m.heads,
         m.dim, m.rot_dim, m.vdim, m.kv_rank, m.scale, m.window or 0, w.eps,
-        splits, tile, _f32(proj), _stream())
+        splits, tile, *beside, _f32(proj), _stream())
     if rc:
         raise ValueError(f"no decode tile for {m}")
 
@@ -532,7 +538,7 @@ def latent_attn_prefill(proj, out, m, w, rot, batch, rows,
                 w.uk, w.uv, m.scale)
         _latent_out(o, p_, m, o_)
         return
-    lib, dev, st = _lib(), proj.device, _stream()
+    lib, st = _lib(), _stream()
     W, bs_log = batch.table.shape[1], block_size.bit_length() - 1
     f32, T = _f32(proj), proj.shape[0] - n
     pr = proj[n:]
@@ -540,17 +546,47 @@ def latent_attn_prefill(proj, out, m, w, rot, batch, rows,
         _p(pr), proj.stride(0), _p(rows), _p(w.norm), _p(rot),
         _p(batch.pos[n:]), _p(batch.row_seq[n:]), _p(batch.table), T, W,
         bs_log, m.heads, m.dim, m.rot_dim, m.vdim, m.kv_rank, w.eps, f32, st)
-    spans, n_keys, tiles, owner = batch.key_plan(m.window)
-    c = torch.empty(n_keys, m.kv_rank, dtype=proj.dtype, device=dev)
-    kr = torch.empty(n_keys, m.rot_dim, dtype=proj.dtype, device=dev)
+    spans, n_keys, tiles, owner, c, kr = _key_room(proj, m, batch)
     lib.fei_latent_gather(_p(c), _p(kr), _p(rows), _p(owner), _p(spans),
                           _p(batch.table), n_keys, W, bs_log, n, m.kv_rank,
                           m.rot_dim, f32, st)
+    _window_prefill(proj, out, m, w, spans, tiles, c, kr)
+
+
+def _key_room(proj, m, batch):
+    """batch.key_plan, and room for the keys: latents and rotated parts."""
+    spans, n_keys, tiles, owner = batch.key_plan(m.window)
+    c, kr = (torch.empty(n_keys, k, dtype=proj.dtype, device=proj.device)
+             for k in (m.kv_rank, m.rot_dim))
+    return spans, n_keys, tiles, owner, c, kr
+
+
+def _window_prefill(proj, out, m, w, spans, tiles, c, kr) -> None:
     kv = torch.nn.functional.linear(c, w.ukv)
-    lib.fei_window_prefill(
+    _lib().fei_window_prefill(
         _p(out), out.stride(0), _p(proj), proj.stride(0), _p(kv), _p(kr),
         _p(spans), _p(tiles), tiles.shape[0], m.heads, m.dim, m.rot_dim,
-        m.vdim, m.kv_rank, m.scale, m.window or 0, f32, st)
+        m.vdim, m.kv_rank, m.scale, m.window or 0, _f32(proj), _stream())
+
+
+def latent_attn_mixed(proj, out, m, w, rot, batch, rows, block_size: int) -> None:
+    """latent_attn_decode of the first n_dec rows and latent_attn_prefill of the others,
+    whose rows and keys the former's launches prepare where there are both."""
+    n = batch.n_dec
+    args = (m, w, rot, batch, rows, block_size)
+    # what the third dimension of a grid of few blocks in the others has room for
+    if (proj.is_cuda and 0 < n < 1024 and batch.portions and proj.shape[0] < 1 << 16
+            and batch.key_plan(m.window)[1] < 1 << 17):
+        spans, n_keys, tiles, owner, c, kr = _key_room(proj, m, batch)
+        _latent_decode(proj, out, *args, n, (
+            proj.shape[0] - n, _p(batch.row_seq[n:]), n_keys, _p(c), _p(kr), _p(owner),
+            _p(spans)))
+        _window_prefill(proj, out, m, w, spans, tiles, c, kr)
+        return
+    if n:
+        latent_attn_decode(proj[:n], out[:n], *args)
+    if batch.portions:
+        latent_attn_prefill(proj, out, *args)
 
 
 # -- gated linear attention ----------------------------------------------------------

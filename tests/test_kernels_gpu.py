@@ -1012,6 +1012,50 @@ def test_gla_tokens_beside_prompts(lib, B, H, dim, vdim, rank, dtype):
     assert not torch.equal(mems[0], states)
 
 
+# -- latent attention of tokens and prompts --------------------------------------------
+
+@pytest.mark.parametrize("B", [1, 5, 600])
+@pytest.mark.parametrize("H,dim,rot,vdim,rank,window", [
+    (1, 24, 8, 20, 40, None), (3, 30, 6, 33, 67, 50), (16, 128, 64, 128, 512, 100),
+    (20, 64, 32, 64, 256, None)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_latent_tokens_beside_prompts(lib, B, H, dim, rot, vdim, rank, window, dtype):
+    """One call for both gives the bits of a call for each."""
+    from types import SimpleNamespace as NS
+    from fei_amd.engine.step import RaggedBatch
+    from fei_amd.ops import mixers as mx
+    g = torch.Generator(device=DEV).manual_seed(dim + B)
+    rand = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    up = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    new = [1] * B + [70, 2, 130]
+    lens = [1 + 37 * i % 160 for i in range(B)] + [70, 159, 150]
+    row = [sum(new[:i]) for i in range(B, B + 3)]
+    T, S, W = sum(new), B + 3, 10
+    m = NS(heads=H, dim=dim, rot_dim=rot, vdim=vdim, kv_rank=rank, window=window,
+           scale=dim ** -0.5, row_width=rank + rot)
+    ukv = (rand(H * (dim + vdim), rank) * rank ** -0.5).to(dtype)
+    w = NS(uk=ukv[:H * dim], uv=ukv[H * dim:], ukv=ukv, norm=rand(rank), eps=1e-5)
+    angles = rand(160, rot // 2)
+    rotab = torch.stack([angles.cos(), angles.sin()], -1).flatten(1).contiguous()
+    batch = RaggedBatch(
+        tokens=torch.zeros(T, dtype=torch.int64, device=DEV),
+        pos=up([p for n, c in zip(lens, new) for p in range(n - c, n)]),
+        row_seq=up([i for i, c in enumerate(new) for _ in range(c)]),
+        table=torch.randperm(S * W, generator=g, device=DEV).int().view(S, W),
+        slots=up(list(range(S))), n_dec=B,
+        portions=[(r, new[B + i], lens[B + i] - new[B + i]) for i, r in enumerate(row)])
+    proj = rand(T, H * (dim + rot) + rank + rot + H * vdim).to(dtype)
+    cache = rand(S * W * 16, rank + rot).to(dtype)
+    outs, mems, projs = ([x.clone() for _ in range(2)] for x in (
+        torch.zeros(T, H * vdim, dtype=dtype, device=DEV), cache, proj))
+    mx.latent_attn_mixed(projs[0], outs[0], m, w, rotab, batch, mems[0], 16)
+    args = (m, w, rotab, batch, mems[1], 16)
+    mx.latent_attn_decode(projs[1][:B], outs[1][:B], *args)
+    mx.latent_attn_prefill(projs[1], outs[1], *args)
+    assert torch.equal(*mems) and torch.equal(*projs) and torch.equal(*outs)
+    assert not torch.equal(mems[0], cache) and bool(outs[0].isfinite().all())
+
+
 # -- largest values ----------------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
