@@ -217,8 +217,8 @@ def parts_up_to(M: int, N: int, K: int) -> int:
     def us(m, p):
         return (min(_time(m, N, K, p, *t) for t in TILES if t[1] > 128) +
                 m * N * (1.8e-6 * p if p > 1 else 0.9e-6))
-    times = [[us(M * f // 8, p) for p in range(1, min(8, K // 256) + 1)]
-             for f in range(4, 9)]
+    most = max(1, min(8, K // 256))
+    times = [[us(M * f // 8, p) for p in range(1, most + 1)] for f in range(4, 9)]
     loss = [sum(row[i] / min(row) for row in times) for i in range(len(times[0]))]
     return loss.index(min(loss)) + 1
 

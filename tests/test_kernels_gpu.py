@@ -879,6 +879,33 @@ def test_encoder_of_the_rows_that_texts_have(lib, B, S, lengths):
     assert got.isfinite().all()
 
 
+@pytest.mark.parametrize("B,S", [(20, 40), (64, 60)])    # both kinds of tiles
+@pytest.mark.parametrize("heads,inner", [(1, 64), (2, 192), (3, 128)])
+def test_narrow_encoder_of_the_rows_that_texts_have(lib, B, S, heads, inner):
+    """A K of one to three steps, which no part of K is cut from."""
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.bge import BgeEncoder
+    spec = dataclasses.replace(get_spec("bge-base"), num_layers=3, num_heads=heads,
+                               num_kv_heads=heads, hidden_size=heads * 64,
+                               intermediate_size=inner)
+    m = BgeEncoder(spec, device=torch.device(DEV))
+    ids = torch.randint(0, 1000, (B, S), device=DEV)
+    n = torch.arange(B, device=DEV) * 7 % S + 1
+    called = []
+    packed, lib.encoder_packed = lib.encoder_packed, \
+        lambda *a: called.append(packed(*a)) or called[-1]
+    try:
+        got = m.encode_ids(ids, n)
+        lib.encoder_packed = lambda *a: None
+        want = m.encode_ids(ids, n)
+    finally:
+        lib.encoder_packed = packed
+    assert called[0] is not None
+    # as between the paths for all rows
+    assert row_err(got, want.double()) < 2.0 ** -5
+
+
 @pytest.mark.parametrize("gelu", [False, True])
 @pytest.mark.parametrize("M,N,K", [(33, 4, 64), (64, 768, 3072), (65, 100, 128),
                                    (500, 2304, 768)])

@@ -33,6 +33,13 @@ def test_what_tiles_take():
     assert tiles.size_for(16384, 768, 768) == (256, 192)
 
 
+@pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 768, 3072])
+def test_parts_of_any_k(K):
+    """A part has 256 steps or all that there are."""
+    for M, N in ((2, 64), (3073, 128), (4096, 192), (16384, 768), (131072, 2048)):
+        assert 1 <= tiles.parts_up_to(M, N, K) <= max(1, min(8, K // 256))
+
+
 def test_when_activations_go_into_tiles():
     """Where those fill the CUs: not of few rows and results, whatever K."""
     for M, N, K in ((129, 8, 64), (300, 256, 4096), (1000, 1024, 1024), (8192, 64, 256),
