@@ -94,8 +94,8 @@ def llama_few(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor
         if workspace is None:
             workspace = [torch.empty(B, heads, splits, n, dtype=torch.float32,
                                      device=h.device) for n in (D, 2)]
-        po, pml = (t.data_ptr() for t in workspace)
-        assert all(t.shape[2] == splits for t in workspace)
+        po, pml = (t.data_ptr() for t in workspace[:2])
+        assert all(t.shape[2] == splits for t in workspace[:2])
 
     def rows(n):
         return torch.empty(M, n, dtype=h.dtype, device=h.device)

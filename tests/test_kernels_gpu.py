@@ -743,6 +743,33 @@ def test_layers_of_few_rows_from_one_call(lib, name, B, S, odd, monkeypatch):
                                     else [3 if odd is None else odd, 0])
 
 
+@pytest.mark.parametrize("B", [1, 3])
+def test_workspace_of_a_decoding_step(lib, B):
+    """More entries than the two that attention takes make no difference, nor does
+    what lies there; too small a one is refused."""
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+    spec = dataclasses.replace(get_spec("llama3-1b"), num_layers=2, vocab_size=512)
+    m = LlamaModel(spec, torch.device(DEV), torch.bfloat16, seed=1, max_seq_len=640)
+    toks = torch.randint(0, 512, (B,), device=DEV)
+    pos = torch.arange(B, dtype=torch.int32, device=DEV) * 90 + 300
+    k, v = (randbf(2, B, spec.num_kv_heads, 640, m.D, seed=i) for i in (2, 3))
+
+    def run(ws, splits=16):
+        return m.forward_decode(toks, pos, list(k.clone()), list(v.clone()),
+                                attn_splits=splits, workspace=ws)
+    ws = [torch.full((B, spec.num_heads, 16, n), float("nan"), device=DEV)
+          for n in (m.D, 2)]
+    more = torch.zeros(7, dtype=torch.int32, device=DEV)
+    want = run(None)
+    assert want.isfinite().all()
+    for w in (ws, (*ws, more), [*ws, more, None]):
+        assert torch.equal(run(w), want)
+    with pytest.raises(AssertionError):
+        run(ws, 32)
+
+
 # in parts and by whole products, up to the rows that the last layer's kernels for few
 # take, and one more
 @pytest.mark.parametrize("layers", [1, 2])
