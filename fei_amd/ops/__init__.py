@@ -919,6 +919,23 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor,
 ENCODER_ROWS = 1024
 
 
+def _encoder_weights(weights, C: int, HD: int, inner: int):
+    """Where kernels find an encoder's weights, 12 a layer (see encoder_layers), 16 bytes
+    at a time, or None if one is not of the sizes that they read."""
+    shapes = ((3 * HD, C), (3 * HD,), (C, HD), (C,), (C,), (C,),
+              (inner, C), (inner,), (C, inner), (C,), (C,), (C,))
+    layers, rest = divmod(len(weights), len(shapes))
+    at, low = [], rest
+    for t, shape in zip(weights, shapes * layers):
+        if (t.dtype is not torch.bfloat16 or t.shape != shape
+                or not t.is_contiguous()):
+            return None
+        p = t.data_ptr()
+        at.append(p)
+        low |= p % 16
+    return None if low else at
+
+
 def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
                    pos0: torch.Tensor, kv_len: torch.Tensor,
                    eps: float) -> Optional[torch.Tensor]:
@@ -931,12 +948,10 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
     if not (h.is_cuda and h.is_contiguous() and dim in (64, 128)
             and h.dtype == torch.bfloat16 and 2 < M <= ENCODER_ROWS
             and C % 64 == HD % 64 == inner % 64 == 0
-            and h.data_ptr() % 16 == 0
-            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
-                    for t in weights)):
+            and h.data_ptr() % 16 == 0):
         return None
-    ptrs = [t.data_ptr() for t in weights]
-    if any(p % 16 for p in ptrs):
+    ptrs = _encoder_weights(weights, C, HD, inner)
+    if ptrs is None:
         return None
 
     def rows(n):
@@ -1023,13 +1038,14 @@ def encoder_packed(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
             and M * max(3 * HD, inner, C) < 1 << 31
             and C % 64 == HD % 64 == inner % 64 == 0
             and _embedding_ok(ids, tok, pos, gain, shift)
-            and all(t.dtype is torch.bfloat16 and t.is_contiguous()
-                    and t.data_ptr() % 16 == 0 and t.get_device() == ids.get_device()
-                    for t in weights)
+            and all(t.get_device() == ids.get_device() for t in weights)
             and lens.device == ids.device and lens.dtype is torch.int32
             and lens.shape == (B,) and lens.is_contiguous()
             and _tiles.types_ok(lens, *weights)
             and _prefill_splits(B, heads, S, S) == 1):
+        return None
+    ptrs = _encoder_weights(weights, C, HD, inner)
+    if ptrs is None:
         return None
 
     def rows(n):
@@ -1049,9 +1065,8 @@ def encoder_packed(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
         parts = torch.empty(max(p1, p2) * M * C, dtype=torch.float32,
                             device=ids.device)
     require_lib().fei_encoder_packed(
-        (_vp * len(weights))(*(t.data_ptr() for t in weights)),
-        len(weights) // 12, _ptr(out), _ptr(ids), _ptr(tok), _ptr(pos), tok.shape[0],
-        _ptr(gain), _ptr(shift),
+        (_vp * len(ptrs))(*ptrs), len(ptrs) // 12, _ptr(out), _ptr(ids), _ptr(tok),
+        _ptr(pos), tok.shape[0], _ptr(gain), _ptr(shift),
         *(_ptr(t) for t in room), _ptr(lens), _ptr(starts), B, S, heads, dim, C,
         inner, 1.0 / math.sqrt(dim), eps, many,
         None if parts is None else _ptr(parts), p1, p2, _stream())

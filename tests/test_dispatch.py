@@ -220,3 +220,42 @@ def test_attn_decode_of_an_empty_batch(T):
     torch.cuda.synchronize()
     with pytest.raises(AssertionError):      # what is refused stays so
         ops.attn_decode(q, kc, kc, pos, splits=65)
+
+
+def encoder_shapes(C, HD, inner):
+    return [(3 * HD, C), (3 * HD,), (C, HD), (C,), (C,), (C,),
+            (inner, C), (inner,), (C, inner), (C,), (C,), (C,)]
+
+
+def test_encoder_weights_have_their_sizes():
+    """A kernel reads as much of them as the encoder's sizes say."""
+    C, HD, inner = 128, 64, 192
+    good = [rand(*s) for s in encoder_shapes(C, HD, inner) * 2]
+    assert ops._encoder_weights(good, C, HD, inner) == [t.data_ptr() for t in good]
+    for i, t in enumerate(good):
+        for other in (t[..., :-8].contiguous(), t[:-8].contiguous(), t.float(),
+                      torch.cat([t, t], -1)[..., :t.shape[-1]] if t.dim() == 2
+                      else torch.stack([t, t], 1)[:, 0],
+                      t.t().contiguous() if t.dim() == 2 else t[None],
+                      rand(t.numel() + 1)[1:].view(t.shape)):
+            bad = good[:i] + [other] + good[i + 1:]
+            assert ops._encoder_weights(bad, C, HD, inner) is None, i
+    assert ops._encoder_weights(good[:-1], C, HD, inner) is None
+
+
+# with all rows in one native call, packed in both kinds of tiles, and layer by layer
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,S,lengths", [(2, 30, True), (10, 80, True), (40, 80, True),
+                                         (40, 80, False)])
+@pytest.mark.parametrize("name", ["wqkv", "wo", "wi", "wo2"])
+def test_encoder_weights_of_other_sizes_are_refused(B, S, lengths, name):
+    from fei_amd.models.bge import BgeEncoder
+    m = BgeEncoder(device=torch.device(DEV))
+    ids = torch.zeros(B, S, dtype=torch.long, device=DEV)
+    n = torch.full((B,), S, device=DEV) if lengths else None
+    w = m.layers[-1][name]
+    m.layers[-1][name] = w[:, :-64].contiguous()
+    with pytest.raises(RuntimeError):
+        m.encode_ids(ids, n)
+    m.layers[-1][name] = w
+    assert m.encode_ids(ids, n).isfinite().all()
