@@ -241,10 +241,11 @@ k_sig_conv(T* __restrict__ q, const T* __restrict__ proj, long ps,
   }
 }
 
-// State after the portions: their last projected rows, of which ``blocks`` blocks of NT
-// threads each write a share, a row's NT channels at a time. As a launch of its own this
-// took 4.2 us in each of 16 layers, nearly all of it the launch: portions of 1500 and 200 rows
-// and 6 tokens take 4083 us with it in the attention's launch, 4111 before.
+// State after the portions: their last projected rows. A block of NT threads writes NT times
+// ``wide`` channels of one row, a chain of three loads, 2.6 us. In a loop over its share of
+// them each of a launch's last blocks took as many times that: 64 prompts of 8 rows, 32
+// heads of 128, with the convolution 121 us for 41; 8 of 500, 8 of 256, 72 for 59.
+// As a launch of its own this takes 4 us, nearly all of it the launch.
 template <typename T>
 struct States {
   float* to;           // null: none are kept
@@ -252,277 +253,42 @@ struct States {
   long ps;
   const int* slots;
   int portions, taps, CH;
+  int wide;            // channels of a thread: 8, or 1 where rows do not lie on 16 bytes
+  int blocks;          // that write them
 };
 template <typename T, int NT>
+__host__ __device__ __forceinline__ int parts_of(const States<T>& s) {
+  return (s.CH + NT * s.wide - 1) / (NT * s.wide);
+}
+template <typename T, int NT>
 __device__ __forceinline__ void write_states(const States<T>& s, const int* spans,
-                                             int seq0, int block, int blocks) {
-  const int parts = (s.CH + NT - 1) / NT;
-  for (int u = block; u < s.portions * s.taps * parts; u += blocks) {
-    const int row = u / parts, pt = row / s.taps, a = row - pt * s.taps;
-    const int n = spans[pt * 3 + 1], p = spans[pt * 3 + 2] + n - 1 - a;
-    const int ch = (u - row * parts) * NT + threadIdx.x;
-    if (a < n && ch < s.CH)
-      s.to[((long)s.slots[seq0 + pt] * s.taps + p % s.taps) * s.CH + ch] =
-          El<T>::ld(s.proj[(long)(spans[pt * 3] + n - 1 - a) * s.ps + ch]);
+                                             int seq0, int u) {
+  const int parts = parts_of<T, NT>(s), row = u / parts;
+  const int pt = row / s.taps, a = row - pt * s.taps;
+  if (pt >= s.portions) return;
+  const int n = spans[pt * 3 + 1], p = spans[pt * 3 + 2] + n - 1 - a;
+  const int ch = ((u - row * parts) * NT + threadIdx.x) * s.wide;
+  if (a >= n || ch >= s.CH) return;
+  float* to = s.to + ((long)s.slots[seq0 + pt] * s.taps + p % s.taps) * s.CH + ch;
+  const T* from = s.proj + (long)(spans[pt * 3] + n - 1 - a) * s.ps + ch;
+  if (s.wide == 1) {
+    *to = El<T>::ld(*from);
+  } else {
+    const auto v = ld8(from);
+    st8(to, f32x8{get8(v, 0), get8(v, 1), get8(v, 2), get8(v, 3), get8(v, 4),
+                  get8(v, 5), get8(v, 6), get8(v, 7)});
   }
+}
+
+template <typename T, int NT>
+__global__ void __launch_bounds__(NT)
+k_sig_states(const States<T> s, const int* spans, int seq0) {
+  write_states<T, NT>(s, spans, seq0, blockIdx.x);
 }
 
 // Place of a key of a tile of 64 in the order of the second product.
 __device__ __forceinline__ int key_place(int key) {
   return (key & 32) + ((key & 15) >> 2) * 8 + ((key >> 4) & 1) * 4 + (key & 3);
-}
-
-// Attention of prompt portions, whose convolution has read the states already: they are
-// written here. Blocks (heads h, query tiles + 1 if states are kept y, 128 / (16 NW QS)
-// z); a wave owns QS sets of 16 queries, which share the fragments it reads, the
-// block walks the keys they see in tiles of 64 held in LDS: keys row-major,
-// values transposed. The distance bias depends on query - key alone: a tile's
-// NW * 16 * QS + 63 values are computed once, in four copies shifted by one
-// each, so that a lane reads the four of its keys as one aligned vector.
-// KS >= ceil(dim / 32), DC >= ceil(vdim / 16); queries are zero beyond dim,
-// columns beyond vdim are not stored.
-template <typename T, int KS, int DC, int NW, int QS, bool VEC>
-__device__ __forceinline__ void
-prefill_block(T* __restrict__ out, long os, const T* __restrict__ q,
-              const T* __restrict__ rows, const float* __restrict__ bias,
-              const int* __restrict__ spans, const int* __restrict__ tiles,
-              const int* __restrict__ table, int seq0, int W, int bs_log,
-              const Geo& g, const States<T>& states, int h, int y, int ny, int z) {
-  typedef typename El<T>::frag frag;
-  constexpr int NP = Parts<T>::n;
-  constexpr int NT = NW * 64, NQ = NW * 16 * QS;
-  constexpr int DS = KS * 32 + 8;          // odd count of 16-byte slots
-  constexpr int TB = NQ + 68;
-  extern __shared__ __align__(16) char smem[];
-  T* kt = (T*)smem;                        // [64][DS]
-  T* vt = kt + 64 * DS;                    // [DC * 16][64], see vt_at
-  float* tb = (float*)(vt + DC * 16 * 64);  // [4][TB]
-
-  const int gk = h / (g.heads / g.kvh);
-  // a portion's last queries see the most keys: they start first
-  const int tile = ny - (states.to ? 2 : 1) - y;
-  if (tile < 0) {                          // the last blocks: a launch of 4 us spared
-    if (z == 0) write_states<T, NT>(states, spans, seq0, h, g.heads);
-    return;
-  }
-  const int pt = tiles[tile * 2];
-  const int row0 = spans[pt * 3], cnt = spans[pt * 3 + 1];
-  const int pos0 = spans[pt * 3 + 2];
-  const int q0 = tiles[tile * 2 + 1] + z * NQ;
-  if (q0 >= cnt) return;
-  const int qn = min(NQ, cnt - q0);
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l15 = lane & 15, lg = lane >> 4;
-  const int R = g.kvh * (g.dim + g.vdim);
-  const T* kh = rows + (long)gk * g.dim;
-  const T* vh = rows + (long)g.kvh * g.dim + (long)gk * g.vdim;
-
-  frag bq[QS][KS];
-  f32x4 o[QS][DC];
-#pragma unroll
-  for (int i = 0; i < QS; ++i) {
-    const int r = min((w * QS + i) * 16 + l15, qn - 1);
-    const T* src = q + (long)(row0 - seq0 + q0 + r) * g.heads * g.dim +
-                   (long)h * g.dim;
-#pragma unroll
-    for (int k = 0; k < KS; ++k) {
-      const int c = k * 32 + 8 * lg;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) bq[i][k][j] = 0;
-      if (VEC) {
-        if (c < g.dim) bq[i][k] = ld8(src + c);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (c + j < g.dim) bq[i][k][j] = src[c + j];
-      }
-    }
-#pragma unroll
-    for (int d = 0; d < DC; ++d) o[i][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  // positions of this tile's queries and of the keys any of them sees
-  const int qa = pos0 + q0, qb = qa + qn - 1;
-  const int klo = first_key(qa, g.window) & ~63;
-  // this wave's own range: tiles outside it are staged for the others only
-  const int wa = qa + w * 16 * QS, wb = min(wa + 16 * QS - 1, qb);
-  const int wlo = first_key(wa, g.window);
-  const float r1 = bias[h], r2 = bias[g.heads + h], pb = bias[2 * g.heads + h];
-  const float scale = -g.scale * El<T>::base;
-  const unsigned seen = g.window > 0 ? g.window : 1u << 31;
-
-  // Cached rows of a tile's keys. Keys past the last query are read as that
-  // query's own: their weights are zero, their values have to be finite.
-  const int seq = seq0 + pt;
-  auto tile_row = [&](int t0) {
-    return bs_log >= 6 ? cache_row(table, W, seq, t0, bs_log) : 0L;
-  };
-  auto row_of = [&](long first, int t0, int r) {
-    const int key = min(t0 + r, qb);
-    return bs_log >= 6 ? first + (key - t0)
-                       : cache_row(table, W, seq, key, bs_log);
-  };
-  // vector loads of a tile: all of them before the first store
-  constexpr int NV = KS * 4, NC = DC * 2;
-  constexpr int UK = (64 * NV + NT - 1) / NT, UV = (32 * NC + NT - 1) / NT;
-  frag kf[UK], va[UV], vb[UV];
-  auto load = [&](int t0) {
-    const long first = tile_row(t0);
-#pragma unroll
-    for (int u = 0; u < UK; ++u) {
-      const int i = tid + u * NT;
-      const int r = i / NV, c = (i - r * NV) * 8;
-      kf[u] = ld8(kh + row_of(first, t0, r & 63) * R + (c < g.dim ? c : 0));
-    }
-#pragma unroll
-    for (int u = 0; u < UV; ++u) {
-      const int i = tid + u * NT;
-      const int r = (i / NC * 2) & 63, c = min(i % NC * 8, g.vdim - 8);
-      va[u] = ld8(vh + row_of(first, t0, r) * R + c);
-      vb[u] = ld8(vh + row_of(first, t0, r + 1) * R + c);
-    }
-  };
-  if (VEC) load(klo);
-
-  for (int t0 = klo; t0 <= qb; t0 += 64) {
-    __syncthreads();
-    if (VEC) {
-#pragma unroll
-      for (int u = 0; u < UK; ++u) {
-        const int i = tid + u * NT;
-        const int r = i / NV, c = (i - r * NV) * 8;
-        if (64 * NV % NT == 0 || i < 64 * NV) st8(kt + r * DS + c, kf[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < UV; ++u) {
-        const int i = tid + u * NT;
-        const int r = key_place(i / NC * 2), c = i % NC * 8;
-        if (32 * NC % NT == 0 || i < 32 * NC)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            T two[2] = {(T)va[u][j], (T)vb[u][j]};
-            __builtin_memcpy(vt + vt_at(c + j, r), two, sizeof(two));
-          }
-      }
-    } else {
-      const long first = tile_row(t0);
-      for (int i = tid; i < 64 * KS * 32; i += NT) {
-        const int r = i / (KS * 32), c = i - r * (KS * 32);
-        kt[r * DS + c] = c < g.dim ? kh[row_of(first, t0, r) * R + c]
-                                   : El<T>::st(0.f);
-      }
-      for (int i = tid; i < 64 * DC * 16; i += NT) {
-        const int r = i / (DC * 16), c = i - r * (DC * 16);
-        vt[vt_at(c, key_place(r))] = c < g.vdim
-                                         ? vh[row_of(first, t0, r) * R + c]
-                                         : El<T>::st(0.f);
-      }
-    }
-    for (int i = tid; i < NQ + 63; i += NT) {
-      const int d = max(qa - t0 + NQ - 1 - i, 0);
-      const float v = (r1 * El<T>::ln(1.f + r2 * (float)d) - pb) * El<T>::base;
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-        if (i >= s) tb[s * TB + i - s] = v;
-    }
-    __syncthreads();
-    if (VEC && t0 + 64 <= qb) load(t0 + 64);
-    if (t0 > wb || t0 + 63 < wlo) continue;
-
-    f32x4 s[QS][4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-#pragma unroll
-      for (int i = 0; i < QS; ++i) s[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        const frag a = ld8(kt + (c * 16 + l15) * DS + k * 32 + 8 * lg);
-#pragma unroll
-        for (int i = 0; i < QS; ++i) s[i][c] = mma(a, bq[i][k], s[i][c]);
-      }
-    }
-    // no mask where every query of the wave sees every key of the tile
-    const bool edge = t0 + 63 > wa || (g.window > 0 && wb - t0 >= g.window);
-    const int sh = (3 - l15) & 3;
-#pragma unroll
-    for (int i = 0; i < QS; ++i) {
-      const int qp = wa + i * 16 + l15;
-      const float* tq = tb + sh * TB + 4 * lg - (w * QS + i) * 16 - l15 + NQ -
-                        1 - sh;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const f32x4 b = *(const f32x4*)(tq + c * 16);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          s[i][c][r] =
-              El<T>::inv(1.f + El<T>::exb(fmaf(s[i][c][r], scale, b[r])));
-      }
-      if (edge) {
-        const int d0 = qp - t0 - 4 * lg;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const unsigned d = d0 - c * 16 - r;   // a key ahead: huge
-            if (d >= seen) s[i][c][r] = 0.f;
-          }
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      frag pw[QS][NP];
-#pragma unroll
-      for (int i = 0; i < QS; ++i) {
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = s[i][2 * k + (j >> 2)][j & 3];
-        weight_parts(v, pw[i]);
-      }
-#pragma unroll
-      for (int d = 0; d < DC; ++d) {
-        const frag av = ld8(vt + vt_at(d * 16 + l15, k * 32 + 8 * lg));
-#pragma unroll
-        for (int i = 0; i < QS; ++i)
-#pragma unroll
-          for (int n = 0; n < NP; ++n) o[i][d] = mma(av, pw[i][n], o[i][d]);
-      }
-    }
-  }
-
-#pragma unroll
-  for (int i = 0; i < QS; ++i) {
-    const int r = (w * QS + i) * 16 + l15;
-    if (r >= qn) continue;
-    T* dst = out + (long)(row0 + q0 + r) * os + (long)h * g.vdim;
-#pragma unroll
-    for (int d = 0; d < DC; ++d) {
-      const int c = d * 16 + 4 * lg;
-      T v[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = El<T>::st(o[i][d][j]);
-      if (VEC) {
-        if (c < g.vdim) __builtin_memcpy(dst + c, v, sizeof(v));
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (c + j < g.vdim) dst[c + j] = v[j];
-      }
-    }
-  }
-}
-
-// grid (heads, query tiles + 1 if states are kept, 128 / (16 NW QS))
-template <typename T, int KS, int DC, int NW, int QS, bool VEC>
-__global__ void __launch_bounds__(NW * 64, 2)
-k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
-              const T* __restrict__ rows, const float* __restrict__ bias,
-              const int* __restrict__ spans, const int* __restrict__ tiles,
-              const int* __restrict__ table, int seq0, int W, int bs_log,
-              Geo g, const States<T> states) {
-  prefill_block<T, KS, DC, NW, QS, VEC>(out, os, q, rows, bias, spans, tiles, table,
-                                        seq0, W, bs_log, g, states, blockIdx.x,
-                                        blockIdx.y, gridDim.y, blockIdx.z);
 }
 
 // Keys of a decode row in splits: base (a multiple of 32), keys per split.
@@ -796,32 +562,296 @@ k_sig_decode(T* __restrict__ out, long os, float* __restrict__ part,
                                 blockIdx.y, blockIdx.z);
 }
 
-// Prompt portions and the tokens beside them in one launch: k_sig_prefill's blocks behind
-// k_sig_decode's, of which there are ``nd`` (a multiple of 8: the blocks of a head stay on
-// one XCD). Neither reads a row or a state that the other writes. A token's block is a
-// chain of dependent loads (10 us for 1200 keys in 8 shares, and a sum of 4), a portion's
-// is bound by exponentials: 6 tokens beside 1500 + 200 rows, 32 heads of 64, with the
-// convolution 57.4 -> 46.2 us; a step of 16 layers 4270 -> 4053.
-template <int KS, int DC>
-__global__ void __launch_bounds__(256, 2)
-k_sig_both(u16* out, long os, float* part, const u16* q, const u16* proj, long ps,
-           u16* rows, Conv cv, const float* bias, const int* spans, const int* tiles,
-           const int* pos, const int* slots, const int* table, int B, int W, int bs_log,
-           Geo g, int splits, int least, int nd, const States<u16> states) {
-  const int id = blockIdx.x;
-  if (id < nd) {
-    const int hg = g.heads / g.kvh, ny = g.kvh * ((hg + 15) / 16);
-    const int split = id % splits, y = id / splits % ny, b = id / (splits * ny);
-    if (b < B)
-      decode_block<u16, KS, DC, true>(out, os, part, proj, ps, rows, states.to, cv, bias,
-                                      pos, slots, table, W, bs_log, g, splits, least,
-                                      split, y, b);
-    return;
+// Blocks of queries that share a CU. For three their registers have to be asked for: with a
+// few more than there are, 8 prompts of 2000 rows, 32 heads of 64, take 259 us for 223.
+constexpr int places(int size, int KS, int DC) {
+  return size == 2 && KS == 2 && DC == 4 ? 3 : 2;
+}
+
+// The tokens of a step beside its portions, whose blocks come first in the portions' launch
+// (a multiple of 8 of them: the blocks of a head stay on one XCD). Neither reads a row or a
+// state that the other writes. A token's block is a chain of dependent loads (10 us for
+// 1200 keys in 8 shares, and a sum of 4), a portion's is bound by exponentials: 6 tokens
+// beside 1500 + 200 rows, 32 heads of 64, with the convolution 57.4 -> 46.2 us; a step of
+// 16 layers 4270 -> 4053.
+template <typename T>
+struct Tokens {
+  int blocks, B, splits, least;
+  float* part;
+  T* rows;
+  Conv cv;
+  const int* pos;
+};
+
+// Attention of prompt portions. Blocks: with BOTH those of the tokens; then, for each of
+// 128 / (16 NW QS) parts of a tile of queries, for each of these, the heads; then with KEEP
+// those that write the states, which the convolution has read already: last, so that they
+// take no CU from queries (in front of half of them 4 prompts of 100 rows over 500, float32,
+// took 120 us for 87). The body stands in the kernel: as a function that two kernels call
+// it becomes other code, 2 to 4 % slower over thousands of rows.
+// JOINT: the weights of a wave's QS sets are made before any is masked, which keeps the
+// vector units busier where few waves share them, and takes up to 18 registers more: one
+// prompt of 2000 rows, heads of 64 and 128, 72.7 us for 73.8, 8 of them 243 for 235.
+// A wave owns QS sets of 16 queries, which share the fragments it reads, the
+// block walks the keys they see in tiles of 64 held in LDS: keys row-major,
+// values transposed. The distance bias depends on query - key alone: a tile's
+// NW * 16 * QS + 63 values are computed once, in four copies shifted by one
+// each, so that a lane reads the four of its keys as one aligned vector.
+// KS >= ceil(dim / 32), DC >= ceil(vdim / 16); queries are zero beyond dim,
+// columns beyond vdim are not stored.
+template <typename T, int KS, int DC, int NW, int QS, bool VEC, bool KEEP, bool BOTH,
+          bool JOINT>
+__global__ void __launch_bounds__(NW * 64, JOINT ? 2 : places(sizeof(T), KS, DC))
+k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
+              const T* __restrict__ rows, const float* __restrict__ bias,
+              const int* __restrict__ spans, const int* __restrict__ tiles,
+              const int* __restrict__ table, int seq0, int W, int bs_log,
+              Geo g, const States<T> states, int n_tiles, const Tokens<T> tk) {
+  int id = blockIdx.x;
+  if constexpr (BOTH) {
+    if (id < tk.blocks) {
+      const int hg = g.heads / g.kvh, ny = g.kvh * ((hg + 15) / 16);
+      const int split = id % tk.splits, y = id / tk.splits % ny, b = id / (tk.splits * ny);
+      if (b < tk.B)
+        decode_block<T, KS, DC, true>(out, os, tk.part, states.proj, states.ps, tk.rows,
+                                      states.to, tk.cv, bias, tk.pos, states.slots, table,
+                                      W, bs_log, g, tk.splits, tk.least, split, y, b);
+      return;
+    }
+    id -= tk.blocks;
   }
-  prefill_block<u16, KS, DC, 4, 2, true>(out, os, q, rows, bias, spans, tiles, table, B, W,
-                                         bs_log, g, states, (id - nd) % g.heads,
-                                         (id - nd) / g.heads, (gridDim.x - nd) / g.heads,
-                                         0);
+  typedef typename El<T>::frag frag;
+  constexpr int NP = Parts<T>::n;
+  constexpr int NT = NW * 64, NQ = NW * 16 * QS;
+  constexpr int DS = KS * 32 + 8;          // odd count of 16-byte slots
+  constexpr int TB = NQ + 68;
+  extern __shared__ __align__(16) char smem[];
+  T* kt = (T*)smem;                        // [64][DS]
+  T* vt = kt + 64 * DS;                    // [DC * 16][64], see vt_at
+  float* tb = (float*)(vt + DC * 16 * 64);  // [4][TB]
+
+  const int plane = g.heads * n_tiles, z = id / plane, left = id - z * plane;
+  if (KEEP && z >= 128 / NQ)
+    return write_states<T, NT>(states, spans, seq0, id - plane * (128 / NQ));
+  const int y = left / g.heads, h = left - y * g.heads, gk = h / (g.heads / g.kvh);
+  // a portion's last queries see the most keys: they start first
+  const int tile = n_tiles - 1 - y;
+  const int pt = tiles[tile * 2];
+  const int row0 = spans[pt * 3], cnt = spans[pt * 3 + 1];
+  const int pos0 = spans[pt * 3 + 2];
+  const int q0 = tiles[tile * 2 + 1] + z * NQ;
+  if (q0 >= cnt) return;
+  const int qn = min(NQ, cnt - q0);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l15 = lane & 15, lg = lane >> 4;
+  const int R = g.kvh * (g.dim + g.vdim);
+  const T* kh = rows + (long)gk * g.dim;
+  const T* vh = rows + (long)g.kvh * g.dim + (long)gk * g.vdim;
+
+  frag bq[QS][KS];
+  f32x4 o[QS][DC];
+#pragma unroll
+  for (int i = 0; i < QS; ++i) {
+    const int r = min((w * QS + i) * 16 + l15, qn - 1);
+    const T* src = q + (long)(row0 - seq0 + q0 + r) * g.heads * g.dim +
+                   (long)h * g.dim;
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const int c = k * 32 + 8 * lg;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) bq[i][k][j] = 0;
+      if (VEC) {
+        if (c < g.dim) bq[i][k] = ld8(src + c);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if (c + j < g.dim) bq[i][k][j] = src[c + j];
+      }
+    }
+#pragma unroll
+    for (int d = 0; d < DC; ++d) o[i][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  // positions of this tile's queries and of the keys any of them sees
+  const int qa = pos0 + q0, qb = qa + qn - 1;
+  const int klo = first_key(qa, g.window) & ~63;
+  // this wave's own range: tiles outside it are staged for the others only
+  const int wa = qa + w * 16 * QS, wb = min(wa + 16 * QS - 1, qb);
+  const int wlo = first_key(wa, g.window);
+  const float r1 = bias[h], r2 = bias[g.heads + h], pb = bias[2 * g.heads + h];
+  const float scale = -g.scale * El<T>::base;
+  const unsigned seen = g.window > 0 ? g.window : 1u << 31;
+
+  // Cached rows of a tile's keys. Keys past the last query are read as that
+  // query's own: their weights are zero, their values have to be finite.
+  const int seq = seq0 + pt;
+  auto tile_row = [&](int t0) {
+    return bs_log >= 6 ? cache_row(table, W, seq, t0, bs_log) : 0L;
+  };
+  auto row_of = [&](long first, int t0, int r) {
+    const int key = min(t0 + r, qb);
+    return bs_log >= 6 ? first + (key - t0)
+                       : cache_row(table, W, seq, key, bs_log);
+  };
+  // vector loads of a tile: all of them before the first store
+  constexpr int NV = KS * 4, NC = DC * 2;
+  constexpr int UK = (64 * NV + NT - 1) / NT, UV = (32 * NC + NT - 1) / NT;
+  frag kf[UK], va[UV], vb[UV];
+  auto load = [&](int t0) {
+    const long first = tile_row(t0);
+#pragma unroll
+    for (int u = 0; u < UK; ++u) {
+      const int i = tid + u * NT;
+      const int r = i / NV, c = (i - r * NV) * 8;
+      kf[u] = ld8(kh + row_of(first, t0, r & 63) * R + (c < g.dim ? c : 0));
+    }
+#pragma unroll
+    for (int u = 0; u < UV; ++u) {
+      const int i = tid + u * NT;
+      const int r = (i / NC * 2) & 63, c = min(i % NC * 8, g.vdim - 8);
+      va[u] = ld8(vh + row_of(first, t0, r) * R + c);
+      vb[u] = ld8(vh + row_of(first, t0, r + 1) * R + c);
+    }
+  };
+  if (VEC) load(klo);
+
+  for (int t0 = klo; t0 <= qb; t0 += 64) {
+    __syncthreads();
+    if (VEC) {
+#pragma unroll
+      for (int u = 0; u < UK; ++u) {
+        const int i = tid + u * NT;
+        const int r = i / NV, c = (i - r * NV) * 8;
+        if (64 * NV % NT == 0 || i < 64 * NV) st8(kt + r * DS + c, kf[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < UV; ++u) {
+        const int i = tid + u * NT;
+        const int r = key_place(i / NC * 2), c = i % NC * 8;
+        if (32 * NC % NT == 0 || i < 32 * NC)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            T two[2] = {(T)va[u][j], (T)vb[u][j]};
+            __builtin_memcpy(vt + vt_at(c + j, r), two, sizeof(two));
+          }
+      }
+    } else {
+      const long first = tile_row(t0);
+      for (int i = tid; i < 64 * KS * 32; i += NT) {
+        const int r = i / (KS * 32), c = i - r * (KS * 32);
+        kt[r * DS + c] = c < g.dim ? kh[row_of(first, t0, r) * R + c]
+                                   : El<T>::st(0.f);
+      }
+      for (int i = tid; i < 64 * DC * 16; i += NT) {
+        const int r = i / (DC * 16), c = i - r * (DC * 16);
+        vt[vt_at(c, key_place(r))] = c < g.vdim
+                                         ? vh[row_of(first, t0, r) * R + c]
+                                         : El<T>::st(0.f);
+      }
+    }
+    for (int i = tid; i < NQ + 63; i += NT) {
+      const int d = max(qa - t0 + NQ - 1 - i, 0);
+      const float v = (r1 * El<T>::ln(1.f + r2 * (float)d) - pb) * El<T>::base;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        if (i >= s) tb[s * TB + i - s] = v;
+    }
+    __syncthreads();
+    if (VEC && t0 + 64 <= qb) load(t0 + 64);
+    if (t0 > wb || t0 + 63 < wlo) continue;
+
+    f32x4 s[QS][4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int i = 0; i < QS; ++i) s[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < KS; ++k) {
+        const frag a = ld8(kt + (c * 16 + l15) * DS + k * 32 + 8 * lg);
+#pragma unroll
+        for (int i = 0; i < QS; ++i) s[i][c] = mma(a, bq[i][k], s[i][c]);
+      }
+    }
+    // no mask where every query of the wave sees every key of the tile
+    const bool edge = t0 + 63 > wa || (g.window > 0 && wb - t0 >= g.window);
+    const int sh = (3 - l15) & 3;
+    auto weigh = [&](int i) __attribute__((always_inline)) {
+      const float* tq = tb + sh * TB + 4 * lg - (w * QS + i) * 16 - l15 + NQ -
+                        1 - sh;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const f32x4 b = *(const f32x4*)(tq + c * 16);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          s[i][c][r] =
+              El<T>::inv(1.f + El<T>::exb(fmaf(s[i][c][r], scale, b[r])));
+      }
+    };
+    auto mask = [&](int i) __attribute__((always_inline)) {
+      const int d0 = wa + i * 16 + l15 - t0 - 4 * lg;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const unsigned d = d0 - c * 16 - r;     // a key ahead: huge
+          if (d >= seen) s[i][c][r] = 0.f;
+        }
+    };
+    if (JOINT) {
+#pragma unroll
+      for (int i = 0; i < QS; ++i) weigh(i);
+      if (edge)
+#pragma unroll
+        for (int i = 0; i < QS; ++i) mask(i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < QS; ++i) {
+        weigh(i);
+        if (edge) mask(i);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      frag pw[QS][NP];
+#pragma unroll
+      for (int i = 0; i < QS; ++i) {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = s[i][2 * k + (j >> 2)][j & 3];
+        weight_parts(v, pw[i]);
+      }
+#pragma unroll
+      for (int d = 0; d < DC; ++d) {
+        const frag av = ld8(vt + vt_at(d * 16 + l15, k * 32 + 8 * lg));
+#pragma unroll
+        for (int i = 0; i < QS; ++i)
+#pragma unroll
+          for (int n = 0; n < NP; ++n) o[i][d] = mma(av, pw[i][n], o[i][d]);
+      }
+    }
+  }
+
+#pragma unroll
+  for (int i = 0; i < QS; ++i) {
+    const int r = (w * QS + i) * 16 + l15;
+    if (r >= qn) continue;
+    T* dst = out + (long)(row0 + q0 + r) * os + (long)h * g.vdim;
+#pragma unroll
+    for (int d = 0; d < DC; ++d) {
+      const int c = d * 16 + 4 * lg;
+      T v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = El<T>::st(o[i][d][j]);
+      if (VEC) {
+        if (c < g.vdim) __builtin_memcpy(dst + c, v, sizeof(v));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (c + j < g.vdim) dst[c + j] = v[j];
+      }
+    }
+  }
 }
 
 // Sum of the splits that had keys. grid (ceil(heads * vdim / 256), B)
@@ -846,6 +876,12 @@ k_sig_combine(T* __restrict__ out, long os, const float* __restrict__ part,
   out[(long)b * os + c] = El<T>::st(v);
 }
 
+template <typename T, int KS, int CPL>
+size_t decode_lds(const Geo& g) {
+  return sizeof(T) * (17 * (KS * 32 + 8) + CPL * 16) +
+         4 * 4 * std::min(g.heads / g.kvh, 16) * (CPL * 16 + 4);
+}
+
 template <typename T>
 void run_decode(T* out, long os, float* part, const T* proj, long ps, T* rows,
                 float* states, Conv cv, const float* bias, const int* pos,
@@ -856,8 +892,7 @@ void run_decode(T* out, long os, float* part, const T* proj, long ps, T* rows,
   const bool vec = g.dim % 8 == 0 && g.vdim % 8 == 0;
 #define DEC(KS, CPL, VEC)                                                    \
   do {                                                                       \
-    const size_t lds = sizeof(T) * (17 * (KS * 32 + 8) + CPL * 16) +         \
-                       4 * 4 * (hg < 16 ? hg : 16) * (CPL * 16 + 4);         \
+    const size_t lds = decode_lds<T, KS, CPL>(g);                            \
     allow_lds(k_sig_decode<T, KS, CPL, VEC>, lds);                           \
     hipLaunchKernelGGL((k_sig_decode<T, KS, CPL, VEC>), grid, dim3(256),     \
                        lds, stream, out, os, part, proj, ps, rows, states,   \
@@ -923,44 +958,60 @@ void run_conv(T* q, const T* proj, long ps, T* rows, float* states, Conv cv,
 #undef CONV
 }
 
-template <int KS, int DC>
-void launch_both(u16* out, long os, float* part, const u16* q, u16* rows, const Conv& cv,
-                 const float* bias, const int* spans, const int* tiles, const int* pos,
-                 const int* table, int n_tiles, int B, int W, int bs_log, Geo g,
-                 int splits, int least, const States<u16>& states, hipStream_t stream) {
-  const int hg = g.heads / g.kvh;
-  const size_t lds = std::max(
-      2 * (64 * (KS * 32 + 8) + DC * 16 * 64) + 16 * (128 + 68),
-      2 * (17 * (KS * 32 + 8) + DC * 16) + 4 * 4 * std::min(hg, 16) * (DC * 16 + 4));
-  allow_lds(k_sig_both<KS, DC>, lds);
-  const int nd = (splits * g.kvh * ((hg + 15) / 16) * B + 7) / 8 * 8;
-  hipLaunchKernelGGL((k_sig_both<KS, DC>),
-                     dim3(nd + g.heads * (n_tiles + (states.to ? 1 : 0))), dim3(256), lds,
-                     stream, out, os, part, q, states.proj, states.ps, rows, cv, bias,
-                     spans, tiles, pos, states.slots, table, B, W, bs_log, g, splits,
-                     least, nd, states);
-  const int HV = g.heads * g.vdim;
-  if (splits > 1)
-    hipLaunchKernelGGL(k_sig_combine<u16>, dim3((HV + 255) / 256, B), dim3(256), 0,
-                       stream, out, os, part, pos, g.window, splits, least, HV);
+template <typename T>
+States<T> states_of(float* to, const void* proj, long ps, const int* slots, int portions,
+                    int taps, int CH) {
+  const bool wide = CH % 8 == 0 && ps % 8 == 0 && (size_t)proj % 16 == 0 &&
+                    (size_t)to % 16 == 0;
+  return {to, (const T*)proj, ps, slots, portions, taps, CH, wide ? 8 : 1, 0};
+}
+// The states with as many blocks of NT threads as write them.
+template <int NT, typename T>
+States<T> in_blocks(States<T> s) {
+  if (s.to) s.blocks = s.portions * s.taps * parts_of<T, NT>(s);
+  return s;
 }
 
-template <typename T, int KS, int DC, bool VEC>
+template <typename T, int KS, int DC, bool VEC, bool BOTH = false>
 void launch_prefill(T* out, long os, const T* q, const T* rows,
                     const float* bias, const int* spans, const int* tiles,
                     const int* table, int n_tiles, int seq0, int W, int bs_log,
-                    Geo g, const States<T>& states, hipStream_t stream) {
+                    Geo g, const States<T>& kept, const Tokens<T>& tk,
+                    hipStream_t stream) {
   // the registers of two sets of queries suffice up to these sizes
   constexpr int QS = sizeof(T) == 2 && KS <= 4 && DC <= 8 ? 2 : 1;
   constexpr int NW = sizeof(T) == 2 ? 8 / QS : 4;
   constexpr int NQ = NW * 16 * QS;
-  const size_t lds = sizeof(T) * (64 * (KS * 32 + 8) + DC * 16 * 64) +
-                     16 * (NQ + 68);
-  allow_lds(k_sig_prefill<T, KS, DC, NW, QS, VEC>, lds);
-  const dim3 grid(g.heads, n_tiles + (states.to ? 1 : 0), 128 / NQ);
-  hipLaunchKernelGGL((k_sig_prefill<T, KS, DC, NW, QS, VEC>), grid,
-                     dim3(NW * 64), lds, stream, out, os, q, rows, bias,
-                     spans, tiles, table, seq0, W, bs_log, g, states);
+  const States<T> states = in_blocks<NW * 64>(kept);
+  size_t lds = sizeof(T) * (64 * (KS * 32 + 8) + DC * 16 * 64) + 16 * (NQ + 68);
+  if (BOTH) lds = std::max(lds, decode_lds<T, KS, DC>(g));
+  const int blocks = tk.blocks + g.heads * n_tiles * (128 / NQ);
+  auto launch = [&](auto kernel, int n) {
+    allow_lds(kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3(n), dim3(NW * 64), lds, stream, out, os, q, rows, bias,
+                       spans, tiles, table, seq0, W, bs_log, g, states, n_tiles, tk);
+  };
+  // no registers left: of the plain kernel joint sets spill less (4 prompts of 2000 rows over
+  // 2000 652 us, 666), beside tokens more (694, 650), and to write states here costs 15 to 40
+  constexpr bool LARGE = sizeof(T) == 2 && KS == 4 && DC == 8;
+  auto go = [&](auto keep, int n) {
+    constexpr bool KEEP = decltype(keep)::value;
+    if constexpr (LARGE)
+      launch(k_sig_prefill<T, KS, DC, NW, QS, VEC, KEEP, BOTH, !BOTH>, n);
+    else if (QS == 2 && n <= 512)
+      launch(k_sig_prefill<T, KS, DC, NW, QS, VEC, KEEP, BOTH, QS == 2>, n);
+    else
+      launch(k_sig_prefill<T, KS, DC, NW, QS, VEC, KEEP, BOTH, false>, n);
+  };
+  constexpr bool KEEP = BOTH || !LARGE;
+  if (KEEP && (BOTH || states.to))
+    return go(std::bool_constant<KEEP>{}, blocks + states.blocks);
+  if constexpr (!BOTH) {
+    go(std::false_type{}, blocks);
+    if (states.to)
+      hipLaunchKernelGGL((k_sig_states<T, NW * 64>), dim3(states.blocks), dim3(NW * 64), 0,
+                         stream, states, spans, seq0);
+  }
 }
 
 template <typename T>
@@ -970,7 +1021,7 @@ void run_prefill(T* out, long os, const T* q, const T* rows,
                  Geo g, const States<T>& states, hipStream_t stream) {
 #define PRE(KS, DC, VEC)                                                     \
   launch_prefill<T, KS, DC, VEC>(out, os, q, rows, bias, spans, tiles,       \
-                                 table, n_tiles, seq0, W, bs_log, g, states, stream)
+                                 table, n_tiles, seq0, W, bs_log, g, states, Tokens<T>{}, stream)
 #define BY_DC(KS)                             \
   do {                                        \
     if (g.vdim <= 64) PRE(KS, 4, true);       \
@@ -1040,12 +1091,12 @@ void fei_sig_prefill(void* out, long os, const void* q, const void* rows,
   if (f32)
     run_prefill<float>((float*)out, os, (const float*)q, (const float*)rows,
                        bias, spans, tiles, table, n_tiles, seq0, W, bs_log, g,
-                       {states, (const float*)proj, ps, slots, n_portions, taps, CH},
+                       states_of<float>(states, proj, ps, slots, n_portions, taps, CH),
                        stream);
   else
     run_prefill<u16>((u16*)out, os, (const u16*)q, (const u16*)rows, bias,
                      spans, tiles, table, n_tiles, seq0, W, bs_log, g,
-                     {states, (const u16*)proj, ps, slots, n_portions, taps, CH},
+                     states_of<u16>(states, proj, ps, slots, n_portions, taps, CH),
                      stream);
 }
 
@@ -1059,17 +1110,23 @@ void fei_sig_both(void* out, long os, float* part, const void* q, const void* pr
                   int vdim, int taps, int window, float scale, int splits, float eps,
                   int least, hipStream_t stream) {
   const Geo g{heads, kvh, dim, vdim, scale, window};
-  const Conv cv{conv, qn, kn, taps, eps};
-  const States<u16> st{states, (const u16*)proj, ps, slots, n_portions, taps, channels(g)};
+  const States<u16> st =
+      states_of<u16>(states, proj, ps, slots, n_portions, taps, channels(g));
+  const int per = kvh * ((heads / kvh + 15) / 16), HV = heads * vdim;
+  const Tokens<u16> tk{(splits * per * B + 7) / 8 * 8, B, splits, least, part, (u16*)rows,
+                       Conv{conv, qn, kn, taps, eps}, pos};
 #define BOTH(KS, DC)                                                                   \
-  launch_both<KS, DC>((u16*)out, os, part, (const u16*)q, (u16*)rows, cv, bias, spans, \
-                      tiles, pos, table, n_tiles, B, W, bs_log, g, splits, least, st,  \
-                      stream)
+  launch_prefill<u16, KS, DC, true, true>((u16*)out, os, (const u16*)q,                \
+                                          (const u16*)rows, bias, spans, tiles, table, \
+                                          n_tiles, B, W, bs_log, g, st, tk, stream)
   if (dim <= 64 && vdim <= 64) BOTH(2, 4);
   else if (dim <= 64) BOTH(2, 8);
   else if (vdim <= 64) BOTH(4, 4);
   else BOTH(4, 8);
 #undef BOTH
+  if (splits > 1)
+    hipLaunchKernelGGL(k_sig_combine<u16>, dim3((HV + 255) / 256, B), dim3(256), 0, stream,
+                       (u16*)out, os, part, pos, window, splits, least, HV);
 }
 
 }  // extern "C"

@@ -1119,3 +1119,48 @@ def test_listed_by_the_command_line(capsys):
     from fei_amd.ui.cli import main
     assert main(["models"]) == 0
     assert "bokenex-8b" in capsys.readouterr().out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("portions", [1, 3, 70])
+@pytest.mark.parametrize("heads,kv,dim,vdim,pad,dtype", [
+    (1, 1, 64, 64, 0, torch.bfloat16), (32, 8, 64, 64, 0, torch.bfloat16),
+    (2, 1, 64, 64, 4, torch.bfloat16),      # rows that do not lie on 16 bytes
+    (3, 1, 67, 85, 0, torch.bfloat16), (8, 2, 256, 256, 0, torch.bfloat16),
+    (4, 2, 128, 128, 0, torch.float32), (2, 2, 36, 20, 0, torch.float32)])
+def test_states_that_the_attention_writes(heads, kv, dim, vdim, pad, dtype, portions):
+    """A portion's last rows, whatever number of blocks they take; no others. With a token
+    beside them and without."""
+    taps, CH = 4, heads * dim + kv * (dim + vdim)
+    m = SimpleNamespace(heads=heads, kv_heads=kv, dim=dim, vdim=vdim, window=None,
+                        conv=taps, scale=dim ** -0.5)
+    g = torch.Generator(device="cuda").manual_seed(dim)
+
+    def rand(*size):
+        return torch.randn(*size, device="cuda", generator=g)
+
+    def ints(x):
+        return torch.tensor(x, dtype=torch.int32, device="cuda")
+    w = SimpleNamespace(conv=rand(taps, CH), qn=rand(dim), kn=rand(dim), eps=1e-5,
+                        bias=rand(3, heads).abs())
+    for tokens in (0, 1):
+        new = [1] * tokens + [1 + 5 * i % 9 for i in range(portions)]
+        first = [7] * tokens + [3 * i % 11 for i in range(portions)]
+        row = [sum(new[:i]) for i in range(len(new))]
+        slots = torch.randperm(len(new) + 2, device="cuda", generator=g).int()[:len(new)]
+        batch = RaggedBatch(
+            tokens=None, pos=ints([f + j for f, n in zip(first, new) for j in range(n)]),
+            row_seq=ints([i for i, n in enumerate(new) for _ in range(n)]),
+            table=ints(list(range(2 * len(new)))).view(-1, 2), slots=slots,
+            n_dec=tokens, portions=list(zip(row, new, first))[tokens:])
+        batch._upload = lambda rows, width: ints(rows).view(-1, width)
+        proj = rand(sum(new), CH + pad).to(dtype)[:, :CH]
+        cache = rand(2 * len(new) * 16, kv * (dim + vdim)).to(dtype)
+        states = rand(len(new) + 2, taps, CH)
+        want = states.clone()
+        for s, r, n, f in zip(slots.tolist(), row, new, first):
+            for j in range(max(n - taps, 0), n):
+                want[s, (f + j) % taps] = proj[r + j].float()
+        out = torch.zeros(sum(new), heads * vdim, dtype=dtype, device="cuda")
+        ops.sigmoid_attn_mixed(proj, out, m, w, batch, cache, states, 16)
+        assert torch.equal(states, want)
