@@ -569,14 +569,30 @@ def _window_prefill(proj, out, m, w, spans, tiles, c, kr) -> None:
         m.vdim, m.kv_rank, m.scale, m.window or 0, _f32(proj), _stream())
 
 
+def _keys_beside(m, tokens: int, rows: int, n_keys: int, size: int) -> bool:
+    """Whether the launches of so many tokens prepare the portions' rows and keys, of
+    values of ``size`` bytes. Their blocks gather 4 keys each, 8 where there are more
+    than 16 heads, and few of them fit a CU beside the attention's LDS: by themselves
+    keys take 5 us, here as many as the tokens leave time for. Both launches, beside
+    and in launches of their own, us, rows of 1152 bytes: 16 heads, 2 tokens of 600 keys,
+    8000 gathered 34, 42, 16000 46, 47; 4 of 1500, 8000 34, 42, 16000 51, 48, 64000 115,
+    67; 8 of 600, 4000 37, 39, 6000 41, 41, 12000 50, 43; 64 of 300, 4000 74, 76, 8000 80,
+    78. 32 heads, 4 of 1500, 16000 43 to 48, 48, 64000 84, 68; 8 of 600, 8000 45, 47, 16000
+    51, 50. Rows of 320 to 2176 bytes part at as many bytes or more."""
+    room = 14 if tokens <= 4 else 5
+    return (0 < tokens < 1024 and rows < 1 << 16 and n_keys < 1 << 17   # of a grid
+            and n_keys * m.row_width * size <= room << (21 if m.heads > 16 else 20))
+
+
 def latent_attn_mixed(proj, out, m, w, rot, batch, rows, block_size: int) -> None:
     """latent_attn_decode of the first n_dec rows and latent_attn_prefill of the others,
-    whose rows and keys the former's launches prepare where there are both."""
+    whose rows and keys the former's launches prepare where there are both and that
+    pays."""
     n = batch.n_dec
     args = (m, w, rot, batch, rows, block_size)
-    # what the third dimension of a grid of few blocks in the others has room for
-    if (proj.is_cuda and 0 < n < 1024 and batch.portions and proj.shape[0] < 1 << 16
-            and batch.key_plan(m.window)[1] < 1 << 17):
+    if (proj.is_cuda and n and batch.portions
+            and _keys_beside(m, n, proj.shape[0], batch.key_plan(m.window)[1],
+                             proj.element_size())):
         spans, n_keys, tiles, owner, c, kr = _key_room(proj, m, batch)
         _latent_decode(proj, out, *args, n, (
             proj.shape[0] - n, _p(batch.row_seq[n:]), n_keys, _p(c), _p(kr), _p(owner),

@@ -259,3 +259,21 @@ def test_encoder_weights_of_other_sizes_are_refused(B, S, lengths, name):
         m.encode_ids(ids, n)
     m.layers[-1][name] = w
     assert m.encode_ids(ids, n).isfinite().all()
+
+
+def test_keys_beside_tokens_are_few():
+    """What the tokens' launches prepare of the portions beside them: by bytes, by how
+    many keys a block takes and by how long the tokens take; never past a grid."""
+    from types import SimpleNamespace as NS
+    m, wide = NS(heads=16, row_width=576), NS(heads=32, row_width=576)
+    for spec, tokens, keys, pays in (
+            (m, 1, 12000, True), (m, 4, 8000, True), (m, 4, 16000, False),
+            (m, 5, 4000, True), (m, 64, 4000, True), (m, 8, 8000, False),
+            (wide, 4, 16000, True), (wide, 4, 64000, False), (wide, 8, 8000, True),
+            (wide, 256, 12000, False), (m, 0, 100, False), (m, 1024, 100, False),
+            (NS(heads=16, row_width=320), 32, 8000, True),
+            (NS(heads=16, row_width=1088), 32, 4000, False),
+            (NS(heads=1, row_width=9), 1, 1 << 17, False)):
+        assert mx._keys_beside(spec, tokens, 600, keys, 2) == pays, (spec, tokens, keys)
+    assert not mx._keys_beside(m, 4, 600, 8000, 4)
+    assert not mx._keys_beside(NS(heads=1, row_width=9), 1, 1 << 16, 100, 2)
