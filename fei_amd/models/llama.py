@@ -446,8 +446,10 @@ class LlamaModel:
         x = ops.rmsnorm(h, self.layers[0].norm_attn, s.norm_eps)
         # of the last layer only its keys and values are made of rows that no logits
         # are asked for: 2048 tokens on 8B 25610 -> 24960 us, 6 of 1001 on 1B 10989 ->
-        # 10498, 75 over 1800 on 8B 4301 -> 4275
-        lone = not all_positions and S > 1 and self.fused_rows(B)
+        # 10498, 75 over 1800 on 8B 4299 -> 4266, on 1B 1236 -> 1222. To take the last
+        # rows out costs launches: 33 to 64 tokens on 1B 1121 -> 1129, 32 prompts of 4
+        # 1200 -> 1209, of 9 2326 -> 2312
+        lone = (not all_positions and S >= 8 and B * S > 64 and self.fused_rows(B))
         if self.rows_in_parts(B * S, (*k_caches, *v_caches)):
             x = self._layers_in_parts(x.view(B * S, -1), h.view(B * S, -1), S,
                                       pos0, k_caches, v_caches, lone)

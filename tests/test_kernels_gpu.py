@@ -799,6 +799,29 @@ def test_last_layer_of_a_prompt(lib, B, S, layers):
     assert torch.equal(ka, kb) and torch.equal(va, vb)
 
 
+@pytest.mark.parametrize("B,S,taken", [(1, 64, False), (1, 65, True), (2, 32, False),
+                                       (32, 7, False), (9, 8, True), (1, 300, True),
+                                       (33, 9, False), (4, 8, False)])
+def test_when_a_prompts_last_rows_are_taken_out(lib, B, S, taken, monkeypatch):
+    """Of enough rows for the launches that it costs."""
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+    spec = dataclasses.replace(get_spec("llama3-1b"), num_layers=2, vocab_size=512)
+    m = LlamaModel(spec, torch.device(DEV), torch.bfloat16, seed=1, max_seq_len=320)
+    called, finish = [], m._finish
+    monkeypatch.setattr(m, "_finish", lambda *a: called.append(1) or finish(*a))
+    toks = torch.randint(0, 512, (B, S), device=DEV)
+    pos0 = torch.zeros(B, dtype=torch.int32, device=DEV)
+    kc, vc = (list(randbf(2, B, spec.num_kv_heads, 320, m.D, seed=i)) for i in (2, 3))
+    got = m.forward_prefill(toks, pos0, kc, vc)
+    assert bool(called) == taken
+    if not taken and B * S > 64:
+        # the head's product of the last rows alone may take another kernel
+        want = m.forward_prefill(toks, pos0, kc, vc, all_positions=True)[:, -1]
+        assert row_err(got, want.double()) < 2.0 ** -7
+
+
 @pytest.mark.parametrize("B,S,lengths", [(1, 4, None), (1, 24, None),
                                          (4, 8, [8, 1, 3, 5]), (2, 16, [16, 9]),
                                          (32, 1, None), (1, 33, None),
