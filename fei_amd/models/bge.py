@@ -2,13 +2,14 @@
 (BERT-style: 12 layers, 768 hidden, 12 heads, post-LayerNorm residual
 blocks, GELU MLP, biased linears).
 
-Of more than 640 rows, only those that texts have are run (ops.encoder_packed): padding
-is left out on the device. Up to 1024, and of texts without lengths, all layers are
-launched from one call (ops.encoder_layers); both have their products in this library's
-matrix-core tiles. Beyond, and for one or two rows, the products are the BLAS library's. Bidirectional attention runs in the HIP prompt
-kernel (causal=0), LayerNorm with the residual and GELU in HIP kernels. Weights are
-random-init — there is no network for checkpoints — but the architecture matches
-bge-base so real weights could be loaded via the same tensors.
+Where lengths are given, of more than 640 rows only those that texts have are run
+(ops.encoder_packed): padding is left out on the device. Else, up to 1024 rows, all layers
+are launched from one call (ops.encoder_layers). Both have their products in this library's
+matrix-core tiles; those of more rows without lengths, and of one or two, are the BLAS
+library's (GELU's own). Bidirectional attention runs in the HIP prompt kernel (causal=0),
+LayerNorm with the residual and GELU in HIP kernels. Weights are random-init — there is no
+network for checkpoints — but the architecture matches bge-base so real weights could be
+loaded via the same tensors.
 
 Output: mean-pooled last hidden state, L2-normalised — [B, hidden].
 """
@@ -86,6 +87,11 @@ class BgeEncoder:
                    lengths: Optional[torch.Tensor] = None) -> torch.Tensor:
         """token_ids [B, S] -> embeddings [B, C] (fp32, L2-normalised).
         BERT block: h = LN(h + Attn(h)); h = LN(h + GELU(h Wi + bi) Wo2 + bo2)."""
+        return self._encode(token_ids, lengths, lengths is not None)
+
+    def _encode(self, token_ids: torch.Tensor, lengths: Optional[torch.Tensor],
+                pack: bool) -> torch.Tensor:
+        """``pack``: whether padding may be left out."""
         s = self.spec
         B, S = token_ids.shape
         H, D = s.num_heads, s.head_dim
@@ -94,7 +100,7 @@ class BgeEncoder:
         kv_len = (lengths.to(torch.int32) if lengths is not None
                   else torch.full((B,), S, dtype=torch.int32, device=self.device))
         weights = [lw[n] for lw in self.layers for n in NAMES]
-        if lengths is not None:
+        if pack:
             out = ops.encoder_packed(*embed, weights, H, D, s.intermediate_size,
                                      kv_len, self.eps)
             if out is not None:
@@ -138,11 +144,14 @@ class BgeEncoder:
         for i in range(0, len(texts), batch_size):
             chunk = texts[i:i + batch_size]
             ids = [tok.encode(t)[: self.max_seq_len] for t in chunk]
-            lens = torch.tensor([len(x) for x in ids], device=self.device)
-            S = max(int(lens.max()), 1)
+            n = [len(x) for x in ids]
+            lens = torch.tensor(n, device=self.device)
+            S = max(*n, 1)
             padded = torch.full((len(ids), S), tok.pad_id, dtype=torch.long,
                                 device=self.device)
             for j, row in enumerate(ids):
                 padded[j, :len(row)] = torch.tensor(row, device=self.device)
-            out.append(self.encode_ids(padded, lens))
+            pack = ops.encoder_packing_pays(padded.numel(), sum(n),
+                                            self.spec.intermediate_size)
+            out.append(self._encode(padded, lens, pack))
         return torch.cat(out, dim=0)

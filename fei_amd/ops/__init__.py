@@ -981,12 +981,29 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
 
 # Rows, padding among them, from which those that texts have are packed, and up to which
 # their products run in tiles of 64 x 64, beyond in k_tile's. Us of 12 layers of 768,
-# texts of a quarter to all of the length (all of one length), with padding, in tiles of
-# 64, in k_tile's: 512 rows 618, 636 (670); 768 745, 658 (747); 1500 1631, 800 (1021),
-# 1094 (1136); 2560 1429, 1053 (1265), 1153 (1260); 3200 1431, 1150 (1537), 1253 (1406);
-# 5120 1694, 1550 (2164), 1424 (1710).
+# texts of a quarter to all of the length, with padding, in tiles of 64, in k_tile's: 660
+# rows 712, 645, 1053; 1500 1475, 782, 1088; 2560 1310, 1015, 1145; 3200 1396, 1077, 1202;
+# 3600 1360, 1185, 1249; 4500 1594, 1441, 1396; 6400 1944, -, 1507; 16384 3779, -, 2575.
+# Of as little as a fifth padding 3072 part at: 1336, 1216, 1255, and 3600 1362, 1434, 1361.
 ENCODER_PACKED_FROM = 640
 ENCODER_PACKED_ROWS = 3072
+
+
+def encoder_packing_pays(M: int, texts: int, inner: int) -> bool:
+    """Whether an encoder that could leave out padding is faster so, where the host knows
+    that of the M rows the texts have ``texts``. All rows have fewer launches up to
+    ENCODER_ROWS, the library's tiles beyond, which suit some sizes better. Us, all rows,
+    packed; no padding, a tenth, a fifth: 1024 rows 738, 760; 737, 759; 736, 729. 2560 1314,
+    1211; 1316, 1182; 1306, 1094. 3600 1406, 1506; 1366, 1399; 1362, 1361. 6144 1973, 2071;
+    2000, 2041; 1989, 1771. 9000 2695, 2545. 12800 3507, 3337. Rows whose widest product is
+    whole rounds of the library's tiles: 16384 3791, 3890, of 3 % padding 3801, 3625; 32768
+    7488, 7576, of 3 % 7468, 7345."""
+    if M <= ENCODER_ROWS or 2700 < M <= 8192:
+        return texts <= 0.85 * M
+    if M <= 2700:
+        return True
+    tiles = -(-M // 256) * -(-inner // 256)
+    return texts <= 0.98 * M or tiles % _tiles.CUS != 0
 
 
 def _embedding_ok(ids, tok, pos, gain, shift) -> bool:

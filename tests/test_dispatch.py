@@ -277,3 +277,33 @@ def test_keys_beside_tokens_are_few():
         assert mx._keys_beside(spec, tokens, 600, keys, 2) == pays, (spec, tokens, keys)
     assert not mx._keys_beside(m, 4, 600, 8000, 4)
     assert not mx._keys_beside(NS(heads=1, row_width=9), 1, 1 << 16, 100, 2)
+
+
+def test_when_leaving_out_padding_pays():
+    for M, texts, pays in (
+            (1024, 1024, False), (900, 850, False), (900, 700, True),
+            (1025, 1025, True), (2560, 2560, True),
+            (3600, 3600, False), (4096, 3700, False), (6144, 5000, True),
+            (8192, 8192, False), (9000, 9000, True), (12800, 12800, True),
+            (16384, 16384, False), (16384, 15900, True), (32768, 32768, False),
+            (32768, 0, True)):
+        assert ops.encoder_packing_pays(M, texts, 3072) == pays, (M, texts)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("alike", [True, False])
+def test_texts_of_one_length_are_not_packed(alike, monkeypatch):
+    """The host knows the texts' lengths; either way they are the same embeddings."""
+    from fei_amd.models.bge import BgeEncoder
+    m = BgeEncoder(device=torch.device(DEV))
+    texts = ["ab" * (45 if alike else 1 + i * 11 % 45) for i in range(40)]
+    called, packed = [], ops.encoder_packed
+    monkeypatch.setattr(ops, "encoder_packed",
+                        lambda *a: called.append(1) or packed(*a))
+    got = m.encode_texts(texts, batch_size=40)
+    assert bool(called) != alike
+    monkeypatch.setattr(ops, "encoder_packing_pays", lambda *a: alike)
+    want = m.encode_texts(texts, batch_size=40)
+    assert len(called) == 1
+    # as between the paths for all rows
+    assert row_err(got, want.double()) < 2.0 ** -5
