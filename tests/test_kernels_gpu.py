@@ -743,6 +743,77 @@ def test_layers_of_few_rows_from_one_call(lib, name, B, S, odd, monkeypatch):
                                     else [3 if odd is None else odd, 0])
 
 
+# splits that one kernel sums, and that the output product does, in contiguous caches and in
+# pages, which lie as they happen to
+@pytest.mark.parametrize("B", [1, 3])
+@pytest.mark.parametrize("last", [130, 300, 639])
+@pytest.mark.parametrize("paged", [False, True])
+def test_few_rows_over_many_keys(lib, B, last, paged):
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+    spec = dataclasses.replace(get_spec("llama3-1b"), num_layers=3, vocab_size=512)
+    m = LlamaModel(spec, torch.device(DEV), torch.bfloat16, seed=1, max_seq_len=640)
+    pos = torch.arange(last, last - 13 * B, -13, dtype=torch.int32, device=DEV)
+    shape = (B * 40, spec.num_kv_heads, 16, m.D) if paged else \
+        (B, spec.num_kv_heads, 640, m.D)
+    table = torch.randperm(B * 40, device=DEV).int().view(B, 40) if paged else None
+    k, v = (randbf(3, *shape, seed=i) for i in (2, 3))
+    h = randbf(B, spec.hidden_size, seed=4)
+    eps = spec.norm_eps
+    got, kc, vc = h.clone(), list(k.clone()), list(v.clone())
+    # what no split has written is not read
+    ws = [torch.full((B, spec.num_heads, 16, n), float("nan"), device=DEV)
+          for n in (m.D, 2)]
+    done, sums = lib.llama_few(got, m.layers, kc, vc, m.hq_l, eps, pos, m.rope, 16, ws,
+                               table)
+    assert done == 3 and got.isfinite().all()
+    want, k1, v1 = h.clone(), list(k.clone()), list(v.clone())
+
+    def attend(li, qkv):
+        q, kn, vn = m._qkv_views(qkv, B)
+        args = dict(splits=16, scale=m.D ** -0.5, k=kn, v=vn, table=m.rope)
+        if paged:
+            return lib.attn_decode_paged(q, k1[li], v1[li], table, pos, **args)
+        return lib.attn_decode(q, k1[li], v1[li], pos, **args)
+    want_sums = m.fused_layers(want, attend)
+    if B > 1:
+        assert torch.equal(got, want) and torch.equal(sums, want_sums)
+        assert all(torch.equal(a, b) for a, b in zip(kc + vc, k1 + v1))
+        return
+    # the splits' sums are rounded once, by 2^-9, but in another order: a layer's
+    # attention and the two residuals behind it, three times
+    assert row_err(got, want.double()) < 3 * 3 ** 0.5 * 2.0 ** -9
+    for a, b in zip(kc + vc, k1 + v1):
+        assert row_err(a.flatten(), b.double().flatten()) < 2.0 ** -9
+    assert torch.equal(kc[0], k1[0]) and torch.equal(vc[0], v1[0])
+
+
+@pytest.mark.parametrize("B,S", [(1, 1), (1, 8), (2, 9), (1, 32)])
+def test_few_prompt_rows_over_many_keys(lib, B, S, monkeypatch):
+    """So many that they are cut, into what llama_few makes room for."""
+    import dataclasses
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.llama import LlamaModel
+    spec = dataclasses.replace(get_spec("llama3-1b"), num_layers=2, vocab_size=512)
+    m = LlamaModel(spec, torch.device(DEV), torch.bfloat16, seed=1, max_seq_len=2048)
+    assert lib._prefill_splits(B, spec.num_kv_heads, 4 * S, 2048) > 1
+    toks = torch.randint(0, 512, (B, S), device=DEV)
+    pos0 = 1900 - 300 * torch.arange(B, dtype=torch.int32, device=DEV)
+    k, v = (randbf(2, B, spec.num_kv_heads, 2048, m.D, seed=i) for i in (2, 3))
+    few = lib.llama_few
+
+    def run(one_call):
+        kc, vc, done = list(k.clone()), list(v.clone()), []
+        monkeypatch.setattr(lib, "llama_few", lambda *a, **b: done.append(
+            few(*a, **b) if one_call else (0, None)) or done[-1])
+        y = m.forward_prefill(toks, pos0, kc, vc)
+        assert [d for d, _ in done] == [2 if one_call else 0]
+        return [y, *kc, *vc]
+    for a, b in zip(run(True), run(False)):
+        assert a.isfinite().all() and torch.equal(a, b)
+
+
 @pytest.mark.parametrize("B", [1, 3])
 def test_workspace_of_a_decoding_step(lib, B):
     """More entries than the two that attention takes make no difference, nor does
