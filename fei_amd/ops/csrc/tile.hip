@@ -408,7 +408,7 @@ void launch(TileArgs g, hipStream_t stream) {
 
 // The same of as many rows as the device finds, in the tiles that suit them: by the time
 // of a round of each, us of a step of 64 of K with one tile on the chip, what comes on
-// top with one on every CU, and of a round. 12 layers of 768, texts of 64 to 256 tokens,
+// top with one on every CU (TILES of ops/tiles.py), and of a round. 12 layers of 768, texts of 64 to 256 tokens,
 // 10336 rows of 16384: 2304 x 768 in tiles of 256 x 256, which suit 16384, 45.6 us, of 192
 // x 256 36.2; 768 x 768 21.5 and, of 128 x 256, 16.3; 768 x 3072 56.3, 46.2; 3072 x 768
 // with GELU 63, 72 of either other. Rests are not cut: with 12 steps of K that gains less

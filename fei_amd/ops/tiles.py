@@ -20,7 +20,8 @@ TILE_BF16, TILE_SWIGLU, TILE_GELU, TILE_RELU2, TILE_PARTS, TILE_BIAS = range(6)
 CUS = 256
 FAR = 1 << 24        # rows this far apart: what 128 of them span takes more than 32 bits
 # Rows of x and w a tile, and us of a step of 64 of K: with one tile on the chip, and
-# what comes on top with one on every CU, when the card lowers its clock.
+# what comes on top with one on every CU, when the card lowers its clock. k_tile_counted of
+# csrc/tile.hip has its own copy of those that it chooses from, which a test compares.
 TILES = ((256, 256, 1.0, 0.46), (256, 192, 0.875, 0.36), (192, 256, 0.82, 0.34),
          (256, 128, 0.73, 0.13), (128, 256, 0.73, 0.13))
 
@@ -77,7 +78,8 @@ def tile_ok(M: int, x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def _time(M: int, cols: int, K: int, parts: int, rows: int, width: int,
           alone: float, full: float) -> float:
-    """About how many us a product takes: rounds of tiles over the CUs."""
+    """About how many us a product takes: rounds of tiles over the CUs. A last round that
+    runs in halves counts as a whole one; what it spares is 1 to 5 us of 35 to 360."""
     tiles = -(-M // rows) * -(-cols // width) * parts
     rounds = -(-tiles // CUS)
     return rounds * (-(-K // 64 // parts) * (alone + full * tiles /

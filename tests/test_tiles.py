@@ -40,6 +40,19 @@ def test_parts_of_any_k(K):
         assert 1 <= tiles.parts_up_to(M, N, K) <= max(1, min(8, K // 256))
 
 
+def test_host_and_device_rank_tiles_by_the_same_times():
+    """Parts of K are chosen on the host, the tiles that they run in on the device."""
+    import os
+    import re
+    source = open(os.path.join(os.path.dirname(ops.__file__), "csrc", "tile.hip")).read()
+    times = re.findall(r"= time\((\d+), (\d+), ([\d.]+)f, ([\d.]+)f\)", source)
+    assert [tuple(map(float, t)) for t in times] == [
+        t for t in tiles.TILES if t[1] > 128]
+    # of a round, beside its steps
+    assert "steps * alone + 3.f" in source
+    assert tiles._time(1, 1, 64, 1, 256, 256, 0.0, 0.0) == 3.0
+
+
 def test_when_activations_go_into_tiles():
     """Where those fill the CUs: not of few rows and results, whatever K."""
     for M, N, K in ((129, 8, 64), (300, 256, 4096), (1000, 1024, 1024), (8192, 64, 256),
