@@ -62,8 +62,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 // a launch less, and the weights are on the way meanwhile. For up to XS * 2048 columns.
 // All blocks read all splits, 4 bytes a column, from the L2s: whole decoding steps, us, 16
 // layers of 2048, 300 keys (3 splits) 685 -> 652, 1000 (8) 703 -> 670, 2000 (16) 702 ->
-// 692; 32 layers of 4096, 300 keys 2889 -> 2870, 600 (5) 2907 -> 2896, 700 (6) 2890 ->
-// 2899, which is left to the launch; fp8 weights, 500 keys 1898 -> 1858.
+// 692; 32 layers of 4096, three runs of either in turn, which differ by 2 to 4, 300 keys
+// 2889 -> 2871, 512 (5) 2896 -> 2887, 600 2896 -> 2890, 700 (6) 2890 -> 2899, which is left
+// to the launch; fp8 weights, 300 keys 1889 -> 1849, 512 1892 -> 1864.
 template <int M, int KS, bool NORM, int EPI, bool FP8, bool LDS, int NS = 0,
           int XS = 1>
 __device__ __forceinline__ void
