@@ -630,9 +630,10 @@ k_sig_prefill(T* __restrict__ out, long os, const T* __restrict__ q,
   T* vt = kt + 64 * DS;                    // [DC * 16][64], see vt_at
   float* tb = (float*)(vt + DC * 16 * 64);  // [4][TB]
 
-  const int plane = g.heads * n_tiles, z = id / plane, left = id - z * plane;
-  if (KEEP && z >= 128 / NQ)
+  const int plane = g.heads * n_tiles;
+  if (KEEP && id >= plane * (128 / NQ))
     return write_states<T, NT>(states, spans, seq0, id - plane * (128 / NQ));
+  const int z = id / plane, left = id - z * plane;
   const int y = left / g.heads, h = left - y * g.heads, gk = h / (g.heads / g.kvh);
   // a portion's last queries see the most keys: they start first
   const int tile = n_tiles - 1 - y;
@@ -991,8 +992,9 @@ void launch_prefill(T* out, long os, const T* q, const T* rows,
     hipLaunchKernelGGL(kernel, dim3(n), dim3(NW * 64), lds, stream, out, os, q, rows, bias,
                        spans, tiles, table, seq0, W, bs_log, g, states, n_tiles, tk);
   };
-  // no registers left: of the plain kernel joint sets spill less (4 prompts of 2000 rows over
-  // 2000 652 us, 666), beside tokens more (694, 650), and to write states here costs 15 to 40
+  // no registers left: of the plain kernel joint sets are the faster (4 prompts of 2000 rows
+  // over 2000 652 us, 666), beside tokens the slower (694, 650), and to write states here
+  // costs 15 to 40
   constexpr bool LARGE = sizeof(T) == 2 && KS == 4 && DC == 8;
   auto go = [&](auto keep, int n) {
     constexpr bool KEEP = decltype(keep)::value;
