@@ -5,16 +5,6 @@
 
 namespace {
 
-// Sum over a wave without LDS.
-__device__ __forceinline__ float wave_sum(float v) {
-  f32x2 t = both_halves(v);
-  const u32 b = __builtin_bit_cast(u32, t[0] + t[1]);
-  const auto q = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-  const u32 q0 = q[0], q1 = q[1];
-  return row16_sum(__builtin_bit_cast(float, q0) +
-                   __builtin_bit_cast(float, q1));
-}
-
 // Mean of a text's first len rows, to length 1: out [B, C] float32. A block per
 // text; a thread has 8 columns of every SIDEth row. Bound by latency, and by what
 // one CU loads of a long text (256 rows of 768: 393 KB). starts: null, or the first row

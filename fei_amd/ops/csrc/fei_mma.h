@@ -154,6 +154,20 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v + row_ror<1>(v);
 }
 
+// Sum over a wave, added in the order of a butterfly from lane ^ 32 down to
+// lane ^ 1, without LDS.
+__device__ __forceinline__ float wave_sum(float v) {
+  const u32 a = __builtin_bit_cast(u32, v);
+  const auto p = __builtin_amdgcn_permlane32_swap(a, a, false, false);
+  const u32 p0 = p[0], p1 = p[1];
+  v = __builtin_bit_cast(float, p0) + __builtin_bit_cast(float, p1);
+  const u32 b = __builtin_bit_cast(u32, v);
+  const auto q = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const u32 q0 = q[0], q1 = q[1];
+  return row16_sum(__builtin_bit_cast(float, q0) +
+                   __builtin_bit_cast(float, q1));
+}
+
 // v of the lane's half and of the other (lane ^ 32), in one order in both.
 __device__ __forceinline__ f32x2 both_halves(float v) {
   const u32 u = __builtin_bit_cast(u32, v);

@@ -1,5 +1,6 @@
 """Layers of a Llama-style decoder over few rows, each launched from one call
-(csrc/layers.hip). bfloat16 GPU tensors only."""
+(csrc/layers.hip), and a whole decoding step of one row in one launch
+(csrc/decode_one.hip). bfloat16 GPU tensors only, and fp8 weights."""
 
 from __future__ import annotations
 
@@ -25,8 +26,21 @@ class _FewRows(ctypes.Structure):
                 [(n, _vp) for n in ("pos", "table", "cos_sin", "po", "pml")])
 
 
+class _OneShape(ctypes.Structure):
+    """OneShape of csrc/decode_one.hip."""
+    _fields_ = ([(n, _i) for n in ("layers", "C", "I", "Hq", "Hkv", "D", "room",
+                                   "vocab", "fp8", "blocks")] +
+                [("eps", _f), ("scale", _f)])
+
+
+ONE_BLOCKS = 256               # of decode_one.hip, one a CU
+
+
 def declare(lib: ctypes.CDLL) -> None:
     lib.fei_llama_few.argtypes = [_vp, _i] + [_vp] * 8
+    lib.fei_decode_one_room.argtypes = [_vp]
+    lib.fei_decode_one_room.restype = ctypes.c_long
+    lib.fei_decode_one.argtypes = [_vp] * 8
 
 
 def _pointers(tensors, shapes, device: int, grad: bool):
@@ -124,3 +138,75 @@ def llama_few(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor
         launch((_vp * 8)(*at), done, *args)
         done += 1
     return done, sums if done and M > 1 else None
+
+
+def llama_one(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor],
+              v_caches: Sequence[torch.Tensor], heads: int, eps: float,
+              pos: torch.Tensor, rope: torch.Tensor, norm: torch.Tensor,
+              head: torch.Tensor, fp8: Optional[Sequence] = None,
+              fp8_head: Optional[Tuple[torch.Tensor, torch.Tensor]] = None,
+              blocks: int = ONE_BLOCKS) -> Optional[torch.Tensor]:
+    """A decoding step of one row h [1, C], which is left as it is, in one launch of
+    csrc/decode_one.hip: logits [1, vocab], or None where it does not take the step. Caches
+    [1, Hkv, room, D]; keys and values are written at pos[0]. ``fp8``: of each layer the
+    products' names -> (w, scales). ``blocks``: fewer have items taken by ticket."""
+    M, C = h.shape
+    lw, grad = layers[0], torch.is_grad_enabled()
+    if not (h.is_cuda and M == 1 and k_caches[0].dim() == 4 and len(layers) > 0):
+        return None
+    Hkv, room, D = k_caches[0].shape[1:]
+    I, vocab, dev = lw.wdown.shape[-1], head.shape[0], h.get_device()
+    HD, width, cache = heads * D, (heads + 2 * Hkv) * D, (1, Hkv, room, D)
+    shape = _OneShape(len(layers), C, I, heads, Hkv, D, room, vocab, fp8 is not None,
+                      blocks, eps, 1.0 / math.sqrt(D))
+    lib = _ops.require_lib()
+    if not (Hkv > 0 and dev == torch.cuda.current_device()
+            and torch.cuda.get_device_properties(dev).multi_processor_count >= ONE_BLOCKS
+            and rope.dtype is torch.float32 and pos.dtype is torch.int32
+            and pos.is_contiguous() and rope.is_contiguous() and pos.numel() == 1
+            and pos.get_device() == rope.get_device() == dev
+            and rope.shape == (rope.shape[0], D // 2, 2) and rope.shape[0] >= room
+            and not rope.data_ptr() % 16 and _tiles._memory(pos, rope)):
+        return None
+    size = lib.fei_decode_one_room(ctypes.byref(shape))
+    shapes = ((width, C), (C, HD), (2 * I, C), (C, I))
+    ends = _pointers((h, norm), ((1, C), (C,)), dev, grad)
+    if not size or ends is None:
+        return None
+
+    def weights(names, tensors, pairs):
+        """Where w and its rows' scales lie."""
+        if pairs is None:
+            at = _pointers(tensors, names, dev, grad)
+            return at and (at, [None] * len(at))
+        at = ([], [])
+        for (w, scale), (N, K) in zip(pairs, names):
+            if not (w.dtype is torch.uint8 and w.shape == (N, K) and w.is_contiguous()
+                    and scale.dtype is torch.float32 and scale.numel() == N
+                    and scale.is_contiguous() and not w.data_ptr() % 16
+                    and w.get_device() == scale.get_device() == dev
+                    and _tiles.types_ok(w, scale)):
+                return None
+            at[0].append(w.data_ptr())
+            at[1].append(scale.data_ptr())
+        return at
+
+    table = []
+    for i, (lw, kc, vc) in enumerate(zip(layers, k_caches, v_caches)):
+        q = fp8 and [fp8[i][n] for n in ("wqkv", "wo", "wgu", "wdown")]
+        at = weights(shapes, (lw.wqkv, lw.wo, lw.wgu, lw.wdown), q)
+        rest = _pointers((lw.norm_attn, lw.norm_mlp, kc, vc),
+                         ((C,), (C,), cache, cache), dev, grad)
+        if at is None or rest is None:
+            return None
+        table += [*at[0], *at[1], *rest]
+    at = weights(((vocab, C),), (head,), fp8 and [fp8_head])
+    if at is None or len(table) != 12 * len(layers):
+        return None
+    table += [at[0][0], at[1][0], ends[1]]
+    room_for = torch.empty(size, dtype=torch.uint8, device=h.device)
+    out = torch.empty(1, vocab, dtype=h.dtype, device=h.device)
+    lib.fei_decode_one((_vp * len(table))(*table), ctypes.byref(shape), ends[0],
+                       out.data_ptr(), room_for.data_ptr(), pos.data_ptr(),
+                       rope.data_ptr(), _ops._stream())
+    return out
