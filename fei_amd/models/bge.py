@@ -2,11 +2,11 @@
 (BERT-style: 12 layers, 768 hidden, 12 heads, post-LayerNorm residual
 blocks, GELU MLP, biased linears).
 
-Where lengths are given, of more than 640 rows only those that texts have are run
-(ops.encoder_packed): padding is left out on the device. Else, up to 1024 rows, all layers
-are launched from one call (ops.encoder_layers). Both have their products in this library's
-matrix-core tiles; those of more rows without lengths, and of one or two, are the BLAS
-library's (GELU's own). Bidirectional attention runs in the HIP prompt kernel (causal=0),
+Up to 64 rows take one launch (ops.encoder_one). Where lengths are given, of more than 640
+rows only those that texts have are run (ops.encoder_packed): padding is left out on the
+device. Else, up to 1024 rows, all layers are launched from one call (ops.encoder_layers).
+All have their products in this library's matrix-core tiles; those of more rows without
+lengths are the BLAS library's (GELU's own). Bidirectional attention runs in the HIP prompt kernel (causal=0),
 LayerNorm with the residual and GELU in HIP kernels. Weights are random-init — there is no
 network for checkpoints — but the architecture matches bge-base so real weights could be
 loaded via the same tensors.
@@ -100,6 +100,10 @@ class BgeEncoder:
         kv_len = (lengths.to(torch.int32) if lengths is not None
                   else torch.full((B,), S, dtype=torch.int32, device=self.device))
         weights = [lw[n] for lw in self.layers for n in NAMES]
+        out = ops.encoder_one(*embed, weights, H, D, s.intermediate_size, kv_len,
+                              self.eps)
+        if out is not None:
+            return out
         if pack:
             out = ops.encoder_packed(*embed, weights, H, D, s.intermediate_size,
                                      kv_len, self.eps)

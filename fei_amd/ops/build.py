@@ -16,8 +16,8 @@ from concurrent.futures import ThreadPoolExecutor
 CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 OUT = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libfei_kernels.so")
 SOURCES = ["fei_kernels.hip", "attn_prefill.hip", "attn_decode.hip", "gemv.hip", "decode_one.hip", "attn_decode_fused.hip", "gemv_fp8.hip", "stream_layer.hip",
-           "hybrid.hip", "latent_attn.hip", "gla.hip", "sigmoid_attn.hip", "moe.hip", "rows.hip", "tile.hip", "encoder.hip", "layers.hip"]
-HEADERS = ["fei_common.h", "fei_epilogue.h", "fei_mma.h", "fei_attn.h"]
+           "hybrid.hip", "latent_attn.hip", "gla.hip", "sigmoid_attn.hip", "moe.hip", "rows.hip", "tile.hip", "encoder.hip", "encoder_one.hip", "layers.hip"]
+HEADERS = ["fei_common.h", "fei_epilogue.h", "fei_mma.h", "fei_attn.h", "fei_chain.h"]
 HIPCC = os.environ.get("HIPCC", "hipcc")
 ARCH = os.environ.get("FEI_AMD_ARCH", "gfx950")
 # Packed fp32 VALU instructions are off: some of their forms have returned

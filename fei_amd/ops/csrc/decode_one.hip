@@ -37,6 +37,7 @@
 // 2048, 300 keys 662 -> 609; 32 of 4096, 512 keys 2885 -> 2657; fp8 weights, 3400 keys
 // 2030 -> 1711.
 #include "fei_attn.h"
+#include "fei_chain.h"
 
 namespace {
 
@@ -46,11 +47,7 @@ constexpr int U = 2, DEPTH = 2;          // loads of a row a step; steps in flig
 constexpr int BLOCKS = 256;              // items of a phase
 constexpr int MOST = 32;                 // layers of a launch
 constexpr int CHUNK = 32;                // keys of a wave at a time
-constexpr u32 NONE = 0xffffffffu;         // not there yet
-constexpr int LIMIT = 1 << 20;           // looks
 constexpr float M_NONE = -3.0e38f;       // maximum of no keys
-constexpr int ARRIVED = 0, HOW = 32, TICKET = 64, STATE = 96;    // dwords of a launch's
-enum { FIXED = 1, TICKETS = 2 };
 
 enum { QKV, WO, GU, DOWN, HEAD, ATT, SUM };
 constexpr int PHASES = 6;                // of a layer
@@ -79,26 +76,6 @@ struct One {
   float eps, scale;
 };
 
-template <typename T> __device__ __forceinline__ T ld_sc(const T* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_sc(u32* p, u32 v) {
-  __hip_atomic_store(p, v == NONE ? NONE - 1 : v, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ u32 count(u32* p) {
-  return __hip_atomic_fetch_add(p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Weights stay in flight, unlike at __syncthreads.
-__device__ __forceinline__ void sync_lds() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-__device__ __forceinline__ u32 raised(u32* flag) {
-  return __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-__device__ __forceinline__ void raise(u32* flag) {
-  __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
 // The arguments, read where they are used: kept in registers over all phases they would
 // be spilled.
 typedef const __attribute__((address_space(4))) One Args;
@@ -136,12 +113,6 @@ struct Lds {
 };
 constexpr u32 ALL = 255;
 
-
-__device__ __forceinline__ u32 pack(float x, float y) {
-  return f2bf(x) | (u32)f2bf(y) << 16;
-}
-__device__ __forceinline__ float lo(u32 v) { return bf2f((u16)v); }
-__device__ __forceinline__ float hi(u32 v) { return bf2f((u16)(v >> 16)); }
 __device__ __forceinline__ float as_float(u32 v) { return __builtin_bit_cast(float, v); }
 __device__ __forceinline__ u32 as_u32(float v) { return __builtin_bit_cast(u32, v); }
 
@@ -706,17 +677,7 @@ __global__ void __launch_bounds__(THREADS, 1) k_decode_one(const One) {
   u32* state = a.state;
   if (tid == 0) {
     s.dead = s.late = s.go = 0;
-    const u32 r = count(state + ARRIVED);
-    u32 how = 0;
-    auto decide = [&](u32 to) {          // the first one does
-      u32 none = 0;
-      __hip_atomic_compare_exchange_strong(state + HOW, &none, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-    };
-    if (r == BLOCKS - 1) decide(FIXED);
-    for (int i = 0; (how = ld_sc(state + HOW)) == 0; ++i)
-      if (i >= 100) decide(TICKETS);
-    s.ticket = how == FIXED ? r : NONE;
+    s.ticket = arrive(state, BLOCKS);
   }
   const int last = min(*a.pos + 1, a.room) - 1;
   if (tid < D) s.cs[tid] = a.cs[(long)max(last, 0) * D + tid];

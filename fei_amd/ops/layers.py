@@ -1,6 +1,7 @@
 """Layers of a Llama-style decoder over few rows, each launched from one call
-(csrc/layers.hip), and a whole decoding step of one row in one launch
-(csrc/decode_one.hip). bfloat16 GPU tensors only, and fp8 weights."""
+(csrc/layers.hip), and in one launch a whole decoding step of one row
+(csrc/decode_one.hip) and a whole encoder of few (csrc/encoder_one.hip). bfloat16 GPU
+tensors only, and of the step fp8 weights."""
 
 from __future__ import annotations
 
@@ -33,7 +34,13 @@ class _OneShape(ctypes.Structure):
                 [("eps", _f), ("scale", _f)])
 
 
-ONE_BLOCKS = 256               # of decode_one.hip, one a CU
+class _EncoderShape(ctypes.Structure):
+    """EncoderShape of csrc/encoder_one.hip."""
+    _fields_ = ([(n, _i) for n in ("layers", "B", "S", "H", "C", "I", "blocks")] +
+                [("eps", _f), ("scale", _f)])
+
+
+ONE_BLOCKS = 256               # of decode_one.hip and encoder_one.hip, one a CU
 
 
 def declare(lib: ctypes.CDLL) -> None:
@@ -41,6 +48,9 @@ def declare(lib: ctypes.CDLL) -> None:
     lib.fei_decode_one_room.argtypes = [_vp]
     lib.fei_decode_one_room.restype = ctypes.c_long
     lib.fei_decode_one.argtypes = [_vp] * 8
+    lib.fei_encoder_one_room.argtypes = [_vp]
+    lib.fei_encoder_one_room.restype = ctypes.c_long
+    lib.fei_encoder_one.argtypes = [_vp] * 7
 
 
 def _pointers(tensors, shapes, device: int, grad: bool):
@@ -209,4 +219,39 @@ def llama_one(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor
     lib.fei_decode_one((_vp * len(table))(*table), ctypes.byref(shape), ends[0],
                        out.data_ptr(), room_for.data_ptr(), pos.data_ptr(),
                        rope.data_ptr(), _ops._stream())
+    return out
+
+
+def encoder_one(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
+                gain: torch.Tensor, shift: torch.Tensor, weights, heads: int,
+                dim: int, inner: int, lens: torch.Tensor, eps: float,
+                blocks: int = ONE_BLOCKS) -> Optional[torch.Tensor]:
+    """An encoder over up to 64 rows in one launch of csrc/encoder_one.hip, behind that
+    of the embeddings: arguments and result are encoder_packed's; None where it does not
+    take them. ``blocks``: fewer have items taken by ticket."""
+    if not (tok.is_cuda and ids.dim() == 2 and 0 < ids.numel() <= 64 and dim == 64
+            and _ops._embedding_ok(ids, tok, pos, gain, shift)):
+        return None
+    (B, S), C, dev = ids.shape, tok.shape[1], ids.get_device()
+    shape = _EncoderShape(len(weights) // 12, B, S, heads, C, inner, blocks, eps,
+                          1.0 / math.sqrt(dim))
+    lib = _ops.require_lib()
+    size = lib.fei_encoder_one_room(ctypes.byref(shape))
+    if not (size and torch.cuda.get_device_properties(dev).multi_processor_count
+            >= ONE_BLOCKS
+            and all(t.get_device() == dev for t in weights)
+            and not (torch.is_grad_enabled() and any(t.requires_grad for t in weights))
+            and lens.device == ids.device and lens.dtype is torch.int32
+            and lens.shape == (B,) and lens.is_contiguous()
+            and _tiles.types_ok(lens, *weights)):
+        return None
+    at = _ops._encoder_weights(weights, C, heads * dim, inner)
+    if at is None:
+        return None
+    h = _ops.embed_layernorm(ids, tok, pos, gain, shift, eps, tok.dtype)
+    room = torch.empty(size, dtype=torch.uint8, device=ids.device)
+    out = torch.empty(B, C, dtype=torch.float32, device=ids.device)
+    lib.fei_encoder_one((_vp * len(at))(*at), ctypes.byref(shape), h.data_ptr(),
+                        out.data_ptr(), room.data_ptr(), lens.data_ptr(),
+                        _ops._stream())
     return out
