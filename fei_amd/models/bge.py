@@ -2,7 +2,7 @@
 (BERT-style: 12 layers, 768 hidden, 12 heads, post-LayerNorm residual
 blocks, GELU MLP, biased linears).
 
-Up to 64 rows take one launch (ops.encoder_one). Where lengths are given, of more than 640
+Up to 128 rows take one launch (ops.encoder_one). Where lengths are given, of more than 640
 rows only those that texts have are run (ops.encoder_packed): padding is left out on the
 device. Else, up to 1024 rows, all layers are launched from one call (ops.encoder_layers).
 All have their products in this library's matrix-core tiles; those of more rows without

@@ -1,13 +1,13 @@
-// All layers of an encoder over up to 64 rows, and the texts' means, in one launch (gfx950).
+// All layers of an encoder over up to 128 rows, and the texts' means, in one launch (gfx950).
 //
 // A chain of launches over so few rows is 5 a layer, each of 4 to 8 us for products that
 // take 1: a launch, its first loads, its last blocks. Here 256 blocks of one a CU stay, and
 // hand results on as fei_chain.h says. A layer has five phases, whose items are of 16 rows:
 //   QKV   LayerNorm of what OUT left; 16 T columns of queries, keys and values
 //   ATT   a wave has the queries of a head
-//   MID   16 columns of the output product
+//   MID   16 columns of the output product, of many rows 32 of them
 //   INNER LayerNorm; 16 T columns of the GELU product
-//   OUT   16 columns of the outer product
+//   OUT   16 columns of the outer product, as MID
 // Blocks of QKV and INNER make the norms for themselves, and keep the residual in registers.
 // Eight waves share K; weights, biases and gains are asked for before the input is there,
 // OUT's weights, 96 KB, two phases ahead to LDS. What ATT, MID and OUT read is handed on in
@@ -18,7 +18,8 @@
 // Bound by the seams, 1.5 to 1.8 us each from one phase's end to what the next has read, and
 // by the norms, which take 2.4 us of 16 rows: two rows a wave, whose instructions are 4 cycles
 // each. Whole encoders, 12 layers of 768, us, the chain's (native) first: 8 rows 307 -> 219;
-// 24 371 -> 234; 33 411 -> 273; 64 485 -> 288, 8 texts of 8 486 -> 296. Items of all rows, so that
+// 24 371 -> 234; 33 411 -> 273; 64 485 -> 288, 8 texts of 8 486 -> 296; 80 556 -> 373; 128 567
+// -> 447, and each further tile of 16 rows takes 25 more, where the chain takes 3. Items of all rows, so that
 // a block made the norm of 64, took 376 for 24 and 527 for 64 rows; weights of OUT in
 // registers, asked for behind INNER, 4 us a layer more where blocks have items of both;
 // attention made by each block of MID for itself 440 and 614; biases and gains asked for
@@ -38,6 +39,7 @@ namespace {
 constexpr int NW = 8, THREADS = NW * 64;
 constexpr int BLOCKS = 256;
 constexpr int MOST = 32;                 // layers
+constexpr int ROWS = 128;
 constexpr int D = 64;                    // of a head
 // a lane's groups of 4 columns of C; a wave's steps of 32 of C and H D, and of 64 of I
 constexpr int NC = 3, NEAR = 3, FAR = 6;
@@ -179,18 +181,14 @@ __device__ __forceinline__ u32x2 bias(const u16* b, int tile, int lane) {
   return *(const u32x2*)(b + tile * 16 + (lane >> 4) * 4);
 }
 
-// Sums the waves' shares; wave j < T hands on tile j of columns: lane's 4 (lane / 16) on of row
-// lane % 16, to to(j, row, column / 4 of the tile), null if there is none.
+// Sums the waves' shares of tiles j0 .. j1 of columns, of which a wave hands on one: lane's 4
+// (lane / 16) on of row lane % 16, to to(j, row, column / 4 of the tile), null if there is none.
 template <int T, bool GELU, typename To>
-__device__ __forceinline__ void hand_on(const f32x4 (&acc)[T], const u32x2 (&b)[T], f32x4* red, To to, int tid) {
-  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
-#pragma unroll
-  for (int j = 0; j < T; ++j) red[(j * NW + w) * 64 + lane] = acc[j];
-  sync_lds();
+__device__ __forceinline__ void hand_tiles(int j0, int j1, const u32x2 (&b)[T], const f32x4* red, To to, int lane, int w) {
 #pragma unroll
   for (int j = 0; j < T; ++j)
-    if (w == j) {
-      const f32x4* p = red + j * NW * 64 + lane;
+    if (j >= j0 && j <= j1 && w == j - j0) {
+      const f32x4* p = red + w * NW * 64 + lane;
       f32x4 v = p[0];
 #pragma unroll
       for (int k = 1; k < NW; ++k)
@@ -202,6 +200,21 @@ __device__ __forceinline__ void hand_on(const f32x4 (&acc)[T], const u32x2 (&b)[
       if (GELU) give(at, two(gelu_erf(x[0]), gelu_erf(x[1])), two(gelu_erf(x[2]), gelu_erf(x[3])));
       else give(at, two(x[0], x[1]), two(x[2], x[3]));
     }
+}
+
+// All T of them, in room for PASS at a time.
+constexpr int PASS = 3;
+template <int T, bool GELU, typename To>
+__device__ __forceinline__ void hand_on(const f32x4 (&acc)[T], const u32x2 (&b)[T], f32x4* red, To to, int tid) {
+  const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+  for (int j = 0; j < T; ++j) {
+    if (j && j % PASS == 0) sync_lds();    // it has been read
+    red[(j % PASS * NW + w) * 64 + lane] = acc[j];
+    if (j % PASS < PASS - 1 && j < T - 1) continue;
+    sync_lds();
+    hand_tiles<T, GELU>(j - j % PASS, j, b, red, to, lane, w);
+  }
 }
 
 // xs = LayerNorm of 16 rows of x + res from row0 on, which becomes the new residual. A wave
@@ -297,26 +310,23 @@ __device__ __forceinline__ void attend(Lds* s, u32* at, int u, int lane) {
     const int c = (i >> 2) * H * 16 + head * 16 + (i & 3) * 4 + 3, row = first + S - 1;
     return i < 8 ? at_frag(row, c, 2 * HD) + 1 : a.v + row * (HD / 2) + head * (D / 2) + (i & 3) * 8 + 7;
   }, s, lane);
-  // keys, then queries as fragments; values: the same loads, 8 bytes of two keys
-  constexpr int NF = 2 * KT + 2, NV = 8 * KC;
-  u32x2 g[2 * NF + NV];
-  take(g, at, [&](int i) {
+  // keys, then queries as fragments, 8 bytes at a time; values: columns 4 l15 on of 8 keys.
+  // All at once, but of more keys than there are registers for
+  constexpr int NF = 2 * KT + 2, NV = 8 * KC, NOW = 2 * NF + (KT > 4 ? 0 : NV);
+  auto off = [&](int i) {
     if (i < 2 * NF) {
       const int j = i / 2, row = first + min(16 * (j < 2 * KT ? j / 2 : t) + l15, S - 1);
       return at_frag(row, (j < 2 * KT ? H * 16 : 0) + head * 16 + (j & 1) * 8 + lg * 2, 2 * HD) + (i & 1) * 2;
     }
     const int j = i - 2 * NF, key = j / 8 * 32 + (j & 4) * 4 + 4 * lg + (j & 3);
     return a.v + (first + min(key, S - 1)) * (HD / 2) + head * (D / 2) + 2 * l15;
-  }, [&](int i) { return i < 2 * NF ? i / 2 >= 2 * KT || i / 4 < tiles : (i - 2 * NF) / 8 * 32 < S; }, s);
+  };
+  auto need = [&](int i) { return i < 2 * NF ? i / 2 >= 2 * KT || i / 4 < tiles : (i - 2 * NF) / 8 * 32 < S; };
+  u32x2 g[NOW];
+  take(g, at, off, need, s);
   s16x8 f[NF];
 #pragma unroll
   for (int i = 0; i < NF; ++i) f[i] = __builtin_bit_cast(s16x8, u32x4{g[2 * i][0], g[2 * i][1], g[2 * i + 1][0], g[2 * i + 1][1]});
-  u32x2 v[NV];
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {           // what lies past the keys counts 0
-    const int key = i / 8 * 32 + (i & 4) * 4 + 4 * lg + (i & 3);
-    v[i] = key < n ? g[2 * NF + i] : u32x2{0, 0};
-  }
   float sc[2 * KC][4];
   float m = -1.f / 0.f;
 #pragma unroll
@@ -332,6 +342,18 @@ __device__ __forceinline__ void attend(Lds* s, u32* at, int u, int lane) {
     }
   }
   m = fmaxf(head_max(m) * a.c, M_NONE);
+  u32x2 v[NV];
+  if constexpr (NOW > 2 * NF) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = g[2 * NF + i];
+  } else {
+    take(v, at, [&](int i) { return off(2 * NF + i); }, [&](int i) { return need(2 * NF + i); }, s);
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {           // what lies past the keys counts 0
+    const int key = i / 8 * 32 + (i & 4) * 4 + 4 * lg + (i & 3);
+    if (key >= n) v[i] = u32x2{0, 0};
+  }
   float ls = 0.f;
   f32x4 o[4];
 #pragma unroll
@@ -414,11 +436,13 @@ __device__ __forceinline__ void pool(Lds* s, const u32* rows, int b, int tid) {
 
 template <int T>
 __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
+  // a text's tiles of keys; tiles of rows of MID's and OUT's items, whose weights they share
+  constexpr int KT = T < 3 ? T : T < 4 ? 4 : 8, RP = T < 5 ? 1 : 2;
   extern __shared__ __align__(16) char lds[];
   __shared__ Lds s;
   f32x4* red = (f32x4*)lds;
-  u16* far = (u16*)(lds + T * NW * 1024);
-  u32* xs = (u32*)(lds + T * NW * 1024 + NW * FAR * 2048);
+  u16* far = (u16*)(lds + min(T, PASS) * NW * 1024);
+  u32* xs = (u32*)(lds + min(T, PASS) * NW * 1024 + NW * FAR * 2048);
   u32* state = args().state;
   if (threadIdx.x == 0) {
     s.dead = 0;
@@ -438,7 +462,7 @@ __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
     // items of the phases: of QKV and INNER of one tile of rows, so that a block's residual
     // is; MID's and OUT's from the last block on
     const int gq = (3 * HD / 16 + T - 1) / T, gi = (I / 16 + T - 1) / T, nm = C / 16;
-    const int nq = gq * MT, ni = gi * MT, no = nm * MT;
+    const int nq = gq * MT, ni = gi * MT, no = nm * ((MT + RP - 1) / RP);
     const int units = a.B * a.H * ((a.S + 15) / 16), na = min(units, BLOCKS);
     if (!fixed) {
       __syncthreads();
@@ -551,45 +575,59 @@ __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
       const int out = BLOCKS - 1 - (int)rank;
       if (fixed && out < no) fetch_far(a.layer[ly].wo2, out % nm, I, far, tid);
       const int u = item + BLOCKS * w;
-      if (item < na && u < units) attend<T < 3 ? T : 4>(&s, at, u, lane);
+      if (item < na && u < units) attend<KT>(&s, at, u, lane);
       sync_lds();
       if (lost(&s)) break;
     } else if (kind == POOL) {
       if (item < a.B) pool(&s, at, item, tid);
       if (lost(&s)) break;
     } else if (item < no) {
-      const int rt = item / nm, tile = item - rt * nm;
-      const bool row = rt * 16 + (lane & 15) < a.M, mid = kind == MID;
-      const u32x2 b[1] = {bias(mid ? a.layer[ly].bo : a.layer[ly].bo2, tile, lane)};
-      f32x4 acc[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+      const int rp = item / nm, tile = item - rp * nm;
+      const bool mid = kind == MID;
+      u32x2 b[RP];
+      f32x4 acc[RP];
+#pragma unroll
+      for (int r = 0; r < RP; ++r) {
+        b[r] = bias(mid ? a.layer[ly].bo : a.layer[ly].bo2, tile, lane);
+        acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
       if (mid) {
         const Part p = part(HD, w);
         s16x8 f[NEAR];
         weights(f, a.layer[ly].wo, tile, HD, p, lane);
-        u32x4 x[NEAR];
-        take(x, at + a.att + rt * 8 * HD, [&](int i) { return p.at(i) * 256 + lane * 4; }, [&](int) { return row; }, &s, LATER);
+        u32x4 x[RP * NEAR];
+        take(x, at + a.att, [&](int i) { return (rp * RP + i / NEAR) * 8 * HD + p.at(i % NEAR) * 256 + lane * 4; },
+             [&](int i) { return (rp * RP + i / NEAR) * 16 + (lane & 15) < a.M; }, &s, LATER);
 #pragma unroll
-        for (int i = 0; i < NEAR; ++i) acc[0] = mma(f[i], p.only(i, __builtin_bit_cast(s16x8, x[i])), acc[0]);
+        for (int i = 0; i < RP * NEAR; ++i)
+          acc[i / NEAR] = mma(f[i % NEAR], p.only(i % NEAR, __builtin_bit_cast(s16x8, x[i])), acc[i / NEAR]);
       } else {
         const Far p = far_part(I, w);
         if (!fixed) fetch_far(a.layer[ly].wo2, tile, I, far, tid);
-        const u32* from = at + a.inner + rt * 8 * I;
         if (p.n) {
-          wait<1>(4 * p.n, from, [&](int i) { return at_frag(15, (4 * p.lo + i) * 4 + 3, I) + 1; }, &s, lane);
-          u32x4 x[2 * FAR];
-          take(x, from, [&](int i) { return (2 * p.lo + min(i, 2 * p.n - 1)) * 256 + lane * 4; }, [&](int) { return row; }, &s);
-          // the weights too: they were asked for before what has come
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
           const u16* ws = far + w * FAR * 1024;
 #pragma unroll
-          for (int i = 0; i < 2 * FAR; ++i)
-            if (i < 2 * p.n)
-              acc[0] = mma(ld8(ws + i / 2 * 1024 + (lane & 15) * 64 + (((i & 1) * 4 + (lane >> 4)) ^ (lane & 7)) * 8),
-                           __builtin_bit_cast(s16x8, x[i]), acc[0]);
+          for (int r = 0; r < RP; ++r) {
+            const int rt = rp * RP + r;
+            if (rt >= MT) break;
+            const u32* from = at + a.inner + rt * 8 * I;
+            const bool row = rt * 16 + (lane & 15) < a.M;
+            wait<1>(4 * p.n, from, [&](int i) { return at_frag(15, (4 * p.lo + i) * 4 + 3, I) + 1; }, &s, lane);
+            u32x4 x[2 * FAR];
+            take(x, from, [&](int i) { return (2 * p.lo + min(i, 2 * p.n - 1)) * 256 + lane * 4; }, [&](int) { return row; }, &s);
+            // the weights too: they were asked for before what has come
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int i = 0; i < 2 * FAR; ++i)
+              if (i < 2 * p.n)
+                acc[r] = mma(ld8(ws + i / 2 * 1024 + (lane & 15) * 64 + (((i & 1) * 4 + (lane >> 4)) ^ (lane & 7)) * 8),
+                             __builtin_bit_cast(s16x8, x[i]), acc[r]);
+          }
         }
       }
-      hand_on<1, false>(acc, b, red, [&](int, int r, int c4) {
-        return at + (mid ? a.mid : a.o2) + (rt * 16 + r) * (C / 2) + tile * 8 + 2 * c4;
+      hand_on<RP, false>(acc, b, red, [&](int j, int r, int c4) {
+        const int rt = rp * RP + j;
+        return rt < MT ? at + (mid ? a.mid : a.o2) + (rt * 16 + r) * (C / 2) + tile * 8 + 2 * c4 : nullptr;
       }, tid);
       if (lost(&s)) break;
     }
@@ -634,9 +672,14 @@ inline long room_of(Encoder& a) {
   return (long)o * a.layers + R * a.C / 2;
 }
 
-inline int per_item(int tiles) { return tiles < 3 ? tiles : 3; }
+// T: the fewest tiles of columns an item with which INNER, of up to 192, has no more items
+// than blocks
+inline int per_item(int tiles) { return tiles < 3 ? tiles : tiles < 5 ? 3 : tiles < 8 ? tiles - 1 : 6; }
 // more than half of a CU's: one block each
-inline int lds_of(const Encoder& a) { return per_item(a.tiles) * NW * 1024 + NW * FAR * 2048 + 32 * a.C; }
+inline int lds_of(const Encoder& a) {
+  const int T = per_item(a.tiles);
+  return (T < PASS ? T : PASS) * NW * 1024 + NW * FAR * 2048 + 32 * a.C;
+}
 
 }  // namespace
 
@@ -658,7 +701,7 @@ extern "C" {
 
 // Bytes of room that it takes, 0 where it cannot run it. Heads of 64.
 long fei_encoder_one_room(const EncoderShape* p) {
-  if (p->layers <= 0 || p->layers > MOST || p->B <= 0 || p->S <= 0 || p->B > 64 || p->S > 64 || p->B * p->S > 64 ||
+  if (p->layers <= 0 || p->layers > MOST || p->B <= 0 || p->S <= 0 || p->B > ROWS || p->S > ROWS || p->B * p->S > ROWS ||
       p->H <= 0 || p->H > 12 || p->C <= 0 || p->C > 768 || p->I <= 0 || p->I > 3072 || p->C % 64 || p->I % 64)
     return 0;
   // so that there are no more items of a phase than blocks
@@ -687,7 +730,10 @@ void fei_encoder_one(const void* const* ptrs, const EncoderShape* p, const void*
   switch (per_item(a.tiles)) {
     case 1: return go(k_encoder_one<1>);
     case 2: return go(k_encoder_one<2>);
-    default: return go(k_encoder_one<3>);
+    case 3: return go(k_encoder_one<3>);
+    case 4: return go(k_encoder_one<4>);
+    case 5: return go(k_encoder_one<5>);
+    default: return go(k_encoder_one<6>);
   }
 }
 

@@ -226,10 +226,10 @@ def encoder_one(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
                 gain: torch.Tensor, shift: torch.Tensor, weights, heads: int,
                 dim: int, inner: int, lens: torch.Tensor, eps: float,
                 blocks: int = ONE_BLOCKS) -> Optional[torch.Tensor]:
-    """An encoder over up to 64 rows in one launch of csrc/encoder_one.hip, behind that
+    """An encoder over up to 128 rows in one launch of csrc/encoder_one.hip, behind that
     of the embeddings: arguments and result are encoder_packed's; None where it does not
     take them. ``blocks``: fewer have items taken by ticket."""
-    if not (tok.is_cuda and ids.dim() == 2 and 0 < ids.numel() <= 64 and dim == 64
+    if not (tok.is_cuda and ids.dim() == 2 and 0 < ids.numel() <= 128 and dim == 64
             and _ops._embedding_ok(ids, tok, pos, gain, shift)):
         return None
     (B, S), C, dev = ids.shape, tok.shape[1], ids.get_device()

@@ -1,4 +1,4 @@
-"""An encoder over up to 64 rows in one launch (csrc/encoder_one.hip) against the chain of
+"""An encoder over up to 128 rows in one launch (csrc/encoder_one.hip) against the chain of
 launches, at the edges of its tiles of rows and of the blocks' and waves' shares."""
 
 import dataclasses
@@ -65,7 +65,10 @@ def near(got, want):
 
 @pytest.mark.parametrize("heads,C,inner", SIZES)
 @pytest.mark.parametrize("B,S", [(1, 1), (1, 16), (1, 24), (2, 16), (1, 33), (7, 7),
-                                 (1, 64), (64, 1), (3, 21)])
+                                 (1, 64), (64, 1), (3, 21),
+                                 # each number of tiles of rows, and two an item
+                                 (1, 65), (3, 32), (9, 11), (1, 112), (128, 1), (1, 128),
+                                 (2, 61)])
 def test_sizes(heads, C, inner, B, S):
     m, ids = model(heads, C, inner), texts(B, S)
     lens = torch.arange(B, device=DEV) * 5 % S + 1
@@ -98,7 +101,7 @@ def test_texts_and_padding_stay_apart():
 
 
 @pytest.mark.parametrize("blocks", [1, 50, 255])
-@pytest.mark.parametrize("B,S", [(1, 24), (8, 8)])
+@pytest.mark.parametrize("B,S", [(1, 24), (8, 8), (1, 85), (5, 25)])
 @pytest.mark.parametrize("heads,C,inner", [(1, 64, 64), (12, 768, 3072)])
 def test_items_by_ticket(heads, C, inner, B, S, blocks):
     """Fewer blocks than items, as where something else holds CUs: the same bits."""
@@ -135,10 +138,10 @@ def test_streams_and_replays():
 @pytest.mark.parametrize("change", ["rows", "wide", "inner", "gap", "lengths", "gradient"])
 def test_what_is_left_to_the_chain(change):
     m, ids = model(*{"wide": (13, 832, 64), "inner": (1, 64, 3136)}
-                   .get(change, (2, 192, 128))), texts(5, 12)
-    lens = torch.full((5,), 12, device=DEV)
+                   .get(change, (2, 192, 128))), texts(5, 25)
+    lens = torch.full((5,), 25, device=DEV)
     if change == "rows":
-        ids, lens = texts(5, 13), lens + 1
+        ids, lens = texts(5, 26), lens + 1
     elif change == "gap":
         m.layers[1]["wo"] = torch.cat([m.layers[1]["wo"]] * 2, 1)[:, :128]
     elif change == "lengths":
