@@ -17,9 +17,13 @@
 //
 // Bound by the seams, 1.5 to 1.8 us each from one phase's end to what the next has read, and
 // by the norms, which take 2.4 us of 16 rows: two rows a wave, whose instructions are 4 cycles
-// each. Whole encoders, 12 layers of 768, us, the chain's (native) first: 8 rows 307 -> 219;
-// 24 371 -> 234; 33 411 -> 273; 64 485 -> 288, 8 texts of 8 486 -> 296; 80 556 -> 373; 128 567
-// -> 447, and each further tile of 16 rows takes 25 more, where the chain takes 3. Items of all rows, so that
+// each. Whole encoders, 12 layers of 768, us, the chain's (native) first: 8 rows 307 -> 226;
+// 24 371 -> 238; 40 418 -> 280; 64 485 -> 287, 8 texts of 8 486 -> 297; 80 556 -> 361; 128 567
+// -> 440, and each further tile of 16 rows takes 25 more, where the chain takes 3. What goes
+// into a norm is handed on in float32: in bfloat16, as the chain's up to 64 rows, 24 took 234,
+// and embeddings were over ten seeds 0.391 % from float64, 0.341 now, the chain's 0.378; of
+// 100 rows, where the chain keeps float32 too, 0.292, 0.253, 0.260. Loads of what is handed on
+// for the lanes that have a row alone took 24 rows 250. Items of all rows, so that
 // a block made the norm of 64, took 376 for 24 and 527 for 64 rows; weights of OUT in
 // registers, asked for behind INNER, 4 us a layer more where blocks have items of both;
 // attention made by each block of MID for itself 440 and 614; biases and gains asked for
@@ -60,8 +64,8 @@ struct Encoder {
   u32 *buf, *state;
   int layers, B, S, M, tiles, H, C, I;   // tiles of 16 rows
   // dwords of a layer's room, and to what is handed on in it: queries and keys as fragments;
-  // values as rows; ATT's results as fragments, MID's as rows, INNER's as fragments, OUT's
-  // as rows; by ticket normed rows. Behind the last layer's LAST's rows
+  // values as rows; ATT's results as fragments, MID's as rows of float32, INNER's as fragments,
+  // OUT's as rows of float32; by ticket normed rows. Behind the last layer's LAST's rows
   int stride, v, att, mid, inner, o2, keep1, keep2;
   float eps, c;
 };
@@ -111,6 +115,7 @@ __device__ __forceinline__ void give(u32* p, u32 a, u32 b) {
 // through the L2 (LATER: past it), and until they are there past it. MADE: by another
 // launch, so there.
 enum { THROUGH, LATER, MADE };
+enum { BF16, GELU, F32 };                // what a product's sums become: bfloat16, that of GELU, float32
 template <int N, typename V, typename Off, typename Need>
 __device__ __forceinline__ void take(V (&v)[N], const u32* base, Off off, Need need, Lds* s, int how = THROUGH) {
   auto at = [&](int i) { return (const u32*)((const char*)base + (u32)(off(i) * 4)); };
@@ -183,7 +188,7 @@ __device__ __forceinline__ u32x2 bias(const u16* b, int tile, int lane) {
 
 // Sums the waves' shares of tiles j0 .. j1 of columns, of which a wave hands on one: lane's 4
 // (lane / 16) on of row lane % 16, to to(j, row, column / 4 of the tile), null if there is none.
-template <int T, bool GELU, typename To>
+template <int T, int AS, typename To>
 __device__ __forceinline__ void hand_tiles(int j0, int j1, const u32x2 (&b)[T], const f32x4* red, To to, int lane, int w) {
 #pragma unroll
   for (int j = 0; j < T; ++j)
@@ -197,14 +202,20 @@ __device__ __forceinline__ void hand_tiles(int j0, int j1, const u32x2 (&b)[T], 
       const float x[4] = {v[0] + lo(b[j][0]), v[1] + hi(b[j][0]), v[2] + lo(b[j][1]), v[3] + hi(b[j][1])};
       u32* at = to(j, lane & 15, lane >> 4);
       if (!at) return;
-      if (GELU) give(at, two(gelu_erf(x[0]), gelu_erf(x[1])), two(gelu_erf(x[2]), gelu_erf(x[3])));
-      else give(at, two(x[0], x[1]), two(x[2], x[3]));
+      if (AS == F32) {
+        give(at, __builtin_bit_cast(u32, x[0]), __builtin_bit_cast(u32, x[1]));
+        give(at + 2, __builtin_bit_cast(u32, x[2]), __builtin_bit_cast(u32, x[3]));
+      } else if (AS == GELU) {
+        give(at, two(gelu_erf(x[0]), gelu_erf(x[1])), two(gelu_erf(x[2]), gelu_erf(x[3])));
+      } else {
+        give(at, two(x[0], x[1]), two(x[2], x[3]));
+      }
     }
 }
 
 // All T of them, in room for PASS at a time.
 constexpr int PASS = 3;
-template <int T, bool GELU, typename To>
+template <int T, int AS, typename To>
 __device__ __forceinline__ void hand_on(const f32x4 (&acc)[T], const u32x2 (&b)[T], f32x4* red, To to, int tid) {
   const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
 #pragma unroll
@@ -213,11 +224,11 @@ __device__ __forceinline__ void hand_on(const f32x4 (&acc)[T], const u32x2 (&b)[
     red[(j % PASS * NW + w) * 64 + lane] = acc[j];
     if (j % PASS < PASS - 1 && j < T - 1) continue;
     sync_lds();
-    hand_tiles<T, GELU>(j - j % PASS, j, b, red, to, lane, w);
+    hand_tiles<T, AS>(j - j % PASS, j, b, red, to, lane, w);
   }
 }
 
-// xs = LayerNorm of 16 rows of x + res from row0 on, which becomes the new residual. A wave
+// xs = LayerNorm of 16 rows of x (float32) + res from row0 on, which becomes the new residual. A wave
 // has rows w and w + 8, its lanes columns 4 lane on and every 256 further. gv, sv: their
 // gains and shifts. Not normed: the first layer's rows, as they are. from: by ticket where
 // the residual is; keep: where rows tile and every tiles-th of the new one go to.
@@ -227,11 +238,23 @@ __device__ __forceinline__ void norm(Lds* s, const u32* x, bool normed, const u3
   Args& a = args();
   const int M = a.M, C = a.C, n4 = C / 4, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   auto place = [&](int i) { return (row0 + w + NW * (i / NC)) * (C / 2) + 2 * (lane + 64 * (i % NC)); };
+  // the next one that there is: loads of all lanes cost less than to leave some out
+  auto near = [&](int i) { return min(row0 + w + NW * (i / NC), M - 1) * (C / 2) + 2 * min(lane + 64 * (i % NC), n4 - 1); };
   auto need = [&](int i) { return row0 + w + NW * (i / NC) < M && lane + 64 * (i % NC) < n4; };
   const u32* h = (const u32*)a.h;
-  u32x2 v[2 * NC];
-  take(v, x, place, need, s, x == h ? MADE : THROUGH);
   if (from) take(res, from, place, need, s, from == h ? MADE : THROUGH);
+  u32x2 v[2 * NC];
+  f32x4 y[2 * NC];
+  if (normed) {
+    u32x4 z[2 * NC];
+    take(z, x, [&](int i) { return 2 * near(i); }, [&](int) { return true; }, s);
+#pragma unroll
+    for (int i = 0; i < 2 * NC; ++i) y[i] = need(i) ? __builtin_bit_cast(f32x4, z[i]) : f32x4{0.f, 0.f, 0.f, 0.f};
+  } else {
+    take(v, x, place, need, s, MADE);
+#pragma unroll
+    for (int i = 0; i < 2 * NC; ++i) y[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
   if (normed) {
     float f[2][NC][4], sum[2];
 #pragma unroll
@@ -239,11 +262,12 @@ __device__ __forceinline__ void norm(Lds* s, const u32* x, bool normed, const u3
       float t = 0.f;                       // lanes without columns have 0
 #pragma unroll
       for (int k = 0; k < NC; ++k) {
-        const u32x2 y = v[i * NC + k], r = res[i * NC + k];
-        f[i][k][0] = lo(y[0]) + lo(r[0]);
-        f[i][k][1] = hi(y[0]) + hi(r[0]);
-        f[i][k][2] = lo(y[1]) + lo(r[1]);
-        f[i][k][3] = hi(y[1]) + hi(r[1]);
+        const f32x4 z = y[i * NC + k];
+        const u32x2 r = res[i * NC + k];
+        f[i][k][0] = z[0] + lo(r[0]);
+        f[i][k][1] = z[1] + hi(r[0]);
+        f[i][k][2] = z[2] + lo(r[1]);
+        f[i][k][3] = z[3] + hi(r[1]);
         t += (f[i][k][0] + f[i][k][1]) + (f[i][k][2] + f[i][k][3]);
       }
       sum[i] = t;
@@ -541,7 +565,7 @@ __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
           }
         }
         if (normed) {
-          if (w == 0) wait<1>(nm, x, [&](int i) { return (rt * 16 + 15) * (C / 2) + i * 8 + 7; }, &s, lane);
+          if (w == 0) wait<1>(nm, x, [&](int i) { return (rt * 16 + 15) * C + i * 16 + 15; }, &s, lane);
           sync_lds();
         }
         norm(&s, x, normed, gv, sv, res, xs, from, keep, rt * 16, group, groups, tid);
@@ -559,12 +583,12 @@ __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
             for (int j = 0; j < T; ++j) acc[j] = mma(f[j][i], y, acc[j]);
           }
           if (second) {
-            hand_on<T, true>(acc, b, red, [&](int j, int row, int c4) {
+            hand_on<T, GELU>(acc, b, red, [&](int j, int row, int c4) {
               const int tile = group * T + j;
               return tile > last ? nullptr : at + a.inner + at_frag(rt * 16 + row, tile * 4 + c4, I);
             }, tid);
           } else {
-            hand_on<T, false>(acc, b, red, [&](int j, int row, int c4) {
+            hand_on<T, BF16>(acc, b, red, [&](int j, int row, int c4) {
               const int tile = group * T + j, c = tile * 16 - 2 * HD, r = rt * 16 + row;
               return tile > last ? nullptr : at + (c < 0 ? at_frag(r, tile * 4 + c4, 2 * HD) : a.v + r * (HD / 2) + c / 2 + 2 * c4);
             }, tid);
@@ -596,8 +620,11 @@ __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
         s16x8 f[NEAR];
         weights(f, a.layer[ly].wo, tile, HD, p, lane);
         u32x4 x[RP * NEAR];
-        take(x, at + a.att, [&](int i) { return (rp * RP + i / NEAR) * 8 * HD + p.at(i % NEAR) * 256 + lane * 4; },
-             [&](int i) { return (rp * RP + i / NEAR) * 16 + (lane & 15) < a.M; }, &s, LATER);
+        // the last row stands in for those behind it, which nobody writes
+        take(x, at + a.att, [&](int i) {
+          const int rt = min(rp * RP + i / NEAR, MT - 1);
+          return rt * 8 * HD + p.at(i % NEAR) * 256 + (lane & 48) * 4 + min(lane & 15, a.M - 1 - rt * 16) * 4;
+        }, [&](int) { return true; }, &s, LATER);
 #pragma unroll
         for (int i = 0; i < RP * NEAR; ++i)
           acc[i / NEAR] = mma(f[i % NEAR], p.only(i % NEAR, __builtin_bit_cast(s16x8, x[i])), acc[i / NEAR]);
@@ -611,10 +638,9 @@ __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
             const int rt = rp * RP + r;
             if (rt >= MT) break;
             const u32* from = at + a.inner + rt * 8 * I;
-            const bool row = rt * 16 + (lane & 15) < a.M;
             wait<1>(4 * p.n, from, [&](int i) { return at_frag(15, (4 * p.lo + i) * 4 + 3, I) + 1; }, &s, lane);
             u32x4 x[2 * FAR];
-            take(x, from, [&](int i) { return (2 * p.lo + min(i, 2 * p.n - 1)) * 256 + lane * 4; }, [&](int) { return row; }, &s);
+            take(x, from, [&](int i) { return (2 * p.lo + min(i, 2 * p.n - 1)) * 256 + lane * 4; }, [&](int) { return true; }, &s);
             // the weights too: they were asked for before what has come
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
@@ -625,9 +651,9 @@ __global__ void __launch_bounds__(THREADS, 1) k_encoder_one(const Encoder) {
           }
         }
       }
-      hand_on<RP, false>(acc, b, red, [&](int j, int r, int c4) {
+      hand_on<RP, F32>(acc, b, red, [&](int j, int r, int c4) {
         const int rt = rp * RP + j;
-        return rt < MT ? at + (mid ? a.mid : a.o2) + (rt * 16 + r) * (C / 2) + tile * 8 + 2 * c4 : nullptr;
+        return rt < MT ? at + (mid ? a.mid : a.o2) + (rt * 16 + r) * C + tile * 16 + 4 * c4 : nullptr;
       }, tid);
       if (lost(&s)) break;
     }
@@ -663,9 +689,9 @@ inline long room_of(Encoder& a) {
   room(R * HD);
   a.v = room(R * HD / 2);
   a.att = room(R * HD / 2);
-  a.mid = room(R * a.C / 2);
+  a.mid = room(R * a.C);
   a.inner = room(R * a.I / 2);
-  a.o2 = room(R * a.C / 2);
+  a.o2 = room(R * a.C);
   a.keep1 = room(R * a.C / 2);
   a.keep2 = room(R * a.C / 2);
   a.stride = o;
