@@ -26,6 +26,29 @@ CHUNK = 64           # tokens per chunk of the linear-attention prompt kernels
 Q_TILE = 128         # query rows per workgroup of the prompt attention kernel
 
 
+def upload(arrays: Sequence[np.ndarray], device: torch.device
+           ) -> List[torch.Tensor]:
+    """The arrays on the device, 16-byte aligned views of one copy that the current
+    stream makes and nobody waits for: a copy from ordinary memory holds the host up until
+    the GPU has done all that it was given. A step of prompts made ten of those, while the
+    GPU had little to do: 1297 rows and 4 tokens of tobarax-1b 4846 us, 4654 so; 1700 and 6
+    of bokenex-1b 4090, 3961."""
+    arrays = [np.ascontiguousarray(a) for a in arrays]
+    if device.type != "cuda":
+        return [torch.from_numpy(a).to(device) for a in arrays]
+    at, size = [], 0
+    for a in arrays:
+        at.append(size)
+        size += -(-a.nbytes // 16) * 16
+    host = torch.empty(size, dtype=torch.uint8, pin_memory=True)
+    flat = host.numpy()
+    for a, o in zip(arrays, at):
+        flat[o:o + a.nbytes] = a.reshape(-1).view(np.uint8)
+    dev = host.to(device, non_blocking=True)
+    return [dev[o:o + a.nbytes].view(torch.from_numpy(a).dtype).view(a.shape)
+            for a, o in zip(arrays, at)]
+
+
 @dataclass
 class RaggedBatch:
     """Device tensors of one step. Sequences are numbered 0 .. n_seq-1 in row
@@ -46,44 +69,9 @@ class RaggedBatch:
     def n_rows(self) -> int:
         return self.tokens.shape[0]
 
-    def _upload(self, rows, width: int) -> torch.Tensor:
-        t = torch.from_numpy(np.asarray(rows, dtype=np.int32))
-        return t.view(-1, width).to(self.tokens.device)
-
-    def span_plan(self):
-        """The prompt portions [first row, rows, first position], and their
-        query tiles [portion, first row in it]."""
-        if "spans" not in self._plans:
-            tiles = [[p, q] for p, (_, n, _) in enumerate(self.portions)
-                     for q in range(0, n, Q_TILE)]
-            self._plans["spans"] = (self._upload(self.portions, 3),
-                                    self._upload(tiles, 2))
-        return self._plans["spans"]
-
-    def key_plan(self, window: Optional[int]):
-        """What the prompt portions read through a window: per portion
-        [first row, rows, first position, first key position, first packed
-        key], the number of packed keys, the query tiles [portion, first row
-        in it], and the portion of every packed key."""
-        key = ("keys", window)
-        if key not in self._plans:
-            spans, tiles, owner, at = [], [], [], 0
-            for p, (row, n, pos0) in enumerate(self.portions):
-                k0 = 0 if window is None else max(0, pos0 - window + 1)
-                spans.append([row, n, pos0, k0, at])
-                n_keys = pos0 + n - k0
-                owner.append(np.full(n_keys, p, dtype=np.int32))
-                at += n_keys
-                tiles += [[p, q] for q in range(0, n, Q_TILE)]
-            self._plans[key] = (self._upload(spans, 5), at,
-                                self._upload(tiles, 2),
-                                self._upload(np.concatenate(owner), 1).view(-1))
-        return self._plans[key]
-
-    def chunk_plan(self):
-        """Chunks of the prompt portions [portion, first row, rows], and per
-        portion [first chunk, chunks, first position, state slot index]."""
-        if "chunks" not in self._plans:
+    def plan_arrays(self, key) -> List[np.ndarray]:
+        """Of one of the plans below: "spans", ("keys", window), "chunks"."""
+        if key == "chunks":
             chunks, spans = [], []
             for p, (row, n, pos0) in enumerate(self.portions):
                 first = len(chunks)
@@ -91,9 +79,47 @@ class RaggedBatch:
                            for c in range(0, n, CHUNK)]
                 spans.append([first, len(chunks) - first, pos0,
                               self.n_dec + p])
-            self._plans["chunks"] = (self._upload(chunks, 3),
-                                     self._upload(spans, 4))
-        return self._plans["chunks"]
+            out = [(chunks, 3), (spans, 4)]
+        else:
+            tiles = [[p, q] for p, (_, n, _) in enumerate(self.portions)
+                     for q in range(0, n, Q_TILE)]
+            out = [(self.portions, 3), (tiles, 2)]
+        if key[0] == "keys":
+            spans, owner, at = [], [], 0
+            for p, (row, n, pos0) in enumerate(self.portions):
+                k0 = 0 if key[1] is None else max(0, pos0 - key[1] + 1)
+                spans.append([row, n, pos0, k0, at])
+                owner.append(np.full(pos0 + n - k0, p, dtype=np.int32))
+                at += pos0 + n - k0
+            out = [(spans, 5), (tiles, 2), (np.concatenate(owner), 1)]
+        return [np.asarray(a, dtype=np.int32).reshape(-1, w) for a, w in out]
+
+    def _upload(self, rows: np.ndarray, width: int) -> torch.Tensor:
+        return upload([rows], self.tokens.device)[0].view(-1, width)
+
+    def _plan(self, key) -> List[torch.Tensor]:
+        if key not in self._plans:
+            self._plans[key] = [self._upload(a, a.shape[1])
+                                for a in self.plan_arrays(key)]
+        return self._plans[key]
+
+    def span_plan(self):
+        """The prompt portions [first row, rows, first position], and their
+        query tiles [portion, first row in it]."""
+        return tuple(self._plan("spans"))
+
+    def key_plan(self, window: Optional[int]):
+        """What the prompt portions read through a window: per portion
+        [first row, rows, first position, first key position, first packed
+        key], the number of packed keys, the query tiles [portion, first row
+        in it], and the portion of every packed key."""
+        spans, tiles, owner = self._plan(("keys", window))
+        return spans, owner.shape[0], tiles, owner.view(-1)
+
+    def chunk_plan(self):
+        """Chunks of the prompt portions [portion, first row, rows], and per
+        portion [first chunk, chunks, first position, state slot index]."""
+        return tuple(self._plan("chunks"))
 
 
 @dataclass
@@ -111,6 +137,9 @@ class StepRunner:
         self.cache: HybridCache = model.new_cache(num_blocks, num_slots,
                                                   block_size)
         self.length: Dict[int, int] = {}      # tokens run, by sequence
+        # what its mixers read of a batch's prompt portions
+        self.plans = list(dict.fromkeys(
+            m.plan for m in model.mixers() if m.plan is not None))
 
     # -- sequences -----------------------------------------------------------
 
@@ -137,16 +166,13 @@ class StepRunner:
 
     # -- steps ---------------------------------------------------------------
 
-    def _tables(self, seqs: Sequence[int]) -> Tuple[torch.Tensor, torch.Tensor]:
+    def _tables(self, seqs: Sequence[int]) -> Tuple[np.ndarray, np.ndarray]:
         blocks = [self.cache.table(s).blocks for s in seqs]
         W = max(max((len(b) for b in blocks), default=1), 1)
         host = np.full((len(seqs), W), self.cache.scratch_block, np.int32)
         for i, b in enumerate(blocks):
             host[i, :len(b)] = b
-        table = torch.from_numpy(host)
-        slots = torch.tensor([self.cache.slot(s) for s in seqs],
-                             dtype=torch.int32)
-        return table.to(self.device), slots.to(self.device)
+        return host, np.array([self.cache.slot(s) for s in seqs], np.int32)
 
     def build(self, entries: Sequence[StepEntry],
               all_rows: bool = False) -> RaggedBatch:
@@ -195,12 +221,20 @@ class StepRunner:
         table, slots = self._tables([entries[i].seq for i in order])
         want = [first_row[i] + w for i, e in enumerate(entries)
                 for w in e.want]
-        rows = torch.from_numpy(meta).to(self.device)
-        return RaggedBatch(
-            tokens=rows[0].long(), pos=rows[1], row_seq=rows[2], table=table,
-            slots=slots, n_dec=n_dec, portions=portions,
-            want_rows=None if all_rows else torch.tensor(
-                want, dtype=torch.int64, device=self.device))
+        batch = RaggedBatch(None, None, None, None, None, n_dec, portions)
+        arrays = [meta[0].astype(np.int64), meta[1], meta[2], table, slots,
+                  np.array(want, np.int64)]
+        plans = [batch.plan_arrays(key) for key in self.plans if portions]
+        dev = upload(arrays + sum(plans, []), self.device)
+        (batch.tokens, batch.pos, batch.row_seq, batch.table, batch.slots,
+         batch.want_rows) = dev[:6]
+        if all_rows:
+            batch.want_rows = None
+        at = 6
+        for key, plan in zip(self.plans, plans):
+            batch._plans[key] = dev[at:at + len(plan)]
+            at += len(plan)
+        return batch
 
     @torch.no_grad()
     def step(self, entries: Sequence[StepEntry],
@@ -222,8 +256,9 @@ class StepRunner:
                 raise ValueError("sequence longer than "
                                  f"{self.model.max_seq_len} tokens")
             self.cache.ensure_capacity(s, self.length[s] + room)
-        table, slots = self._tables(seqs)
         dev = self.device
+        table, slots = (torch.from_numpy(a).to(dev)
+                        for a in self._tables(seqs))
         return RaggedBatch(
             tokens=torch.tensor(list(tokens) if tokens is not None
                                 else [0] * len(seqs),

@@ -22,6 +22,7 @@ class Mixer:
     IN: Tuple[str, ...] = ()
     row_width: Optional[int] = None       # cached values per token
     state_shape: Optional[Tuple[int, ...]] = None   # state per sequence
+    plan: object = None                   # what it reads of a RaggedBatch's portions
 
     @staticmethod
     def shapes(m, width: int) -> Dict[str, tuple]:
@@ -61,7 +62,7 @@ class LatentAttention(Mixer):
         self.ukv = torch.cat([mat("uk"), mat("uv")], dim=0).contiguous()
         self.uk = self.ukv[:m.heads * m.dim]
         self.uv = self.ukv[m.heads * m.dim:]
-        self.row_width = m.row_width
+        self.row_width, self.plan = m.row_width, ("keys", m.window)
 
     def own_weights(self) -> Dict[str, torch.Tensor]:
         return {"dkv.norm": self.norm, "uk": self.uk, "uv": self.uv}
@@ -94,7 +95,7 @@ class GatedLinearAttention(Mixer):
         self.norm, self.bias = vec("norm"), vec("a2.b")
         self.a2 = vec("a2")             # small, and feeds the recurrence
         # value-major, so that a value channel's keys are contiguous
-        self.state_shape = (m.heads, m.vdim, m.dim)
+        self.state_shape, self.plan = (m.heads, m.vdim, m.dim), "chunks"
 
     def own_weights(self) -> Dict[str, torch.Tensor]:
         return {"norm": self.norm, "a2.b": self.bias, "a2": self.a2}
@@ -130,7 +131,7 @@ class SigmoidAttention(Mixer):
         # tap-major, so that the channels of a tap are contiguous
         self.conv = torch.cat([vec(n + ".conv") for n in self.IN]).t() \
             .contiguous()
-        self.row_width = m.row_width
+        self.row_width, self.plan = m.row_width, "spans"
         if m.conv > 1:
             self.state_shape = (m.conv, m.in_rows)
 
