@@ -148,12 +148,6 @@ __device__ __forceinline__ void wait(int n, const u32* base, Flag flag, Lds* s, 
   }
 }
 
-// Two results as a dword, rounded to nearest even.
-__device__ __forceinline__ u32 two(float x, float y) {
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-  return __builtin_bit_cast(u32, __builtin_convertvector(f32x2{x, y}, bf16x2));
-}
-
 // Dwords to a place in a product's input as fragments: columns 4 c on of a row of K. In LDS
 // the rows' places are permuted, so that lanes along c spread over the banks.
 __device__ __forceinline__ int at_frag(int row, int c, int K) {
@@ -206,9 +200,9 @@ __device__ __forceinline__ void hand_tiles(int j0, int j1, const u32x2 (&b)[T], 
         give(at, __builtin_bit_cast(u32, x[0]), __builtin_bit_cast(u32, x[1]));
         give(at + 2, __builtin_bit_cast(u32, x[2]), __builtin_bit_cast(u32, x[3]));
       } else if (AS == GELU) {
-        give(at, two(gelu_erf(x[0]), gelu_erf(x[1])), two(gelu_erf(x[2]), gelu_erf(x[3])));
+        give(at, pack(gelu_erf(x[0]), gelu_erf(x[1])), pack(gelu_erf(x[2]), gelu_erf(x[3])));
       } else {
-        give(at, two(x[0], x[1]), two(x[2], x[3]));
+        give(at, pack(x[0], x[1]), pack(x[2], x[3]));
       }
     }
 }
@@ -299,7 +293,7 @@ __device__ __forceinline__ void norm(Lds* s, const u32* x, bool normed, const u3
       for (int k = 0; k < NC; ++k)
 #pragma unroll
         for (int e = 0; e < 2; ++e)
-          v[i * NC + k][e] = two(fmaf(f[i][k][2 * e] * inv, lo(gv[k][e]), lo(sv[k][e])),
+          v[i * NC + k][e] = pack(fmaf(f[i][k][2 * e] * inv, lo(gv[k][e]), lo(sv[k][e])),
                                  fmaf(f[i][k][2 * e + 1] * inv, hi(gv[k][e]), hi(sv[k][e])));
     }
   }
@@ -409,7 +403,7 @@ __device__ __forceinline__ void attend(Lds* s, u32* at, int u, int lane) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
       give(at + a.att + at_frag(first + 16 * t + l15, head * 16 + 4 * lg + r, HD),
-           two(o[0][r] * inv, o[1][r] * inv), two(o[2][r] * inv, o[3][r] * inv));
+           pack(o[0][r] * inv, o[1][r] * inv), pack(o[2][r] * inv, o[3][r] * inv));
 }
 
 // OUT's weights: 16 rows of W in LDS, a wave's steps of 64 of K, whose 16-byte places are

@@ -27,8 +27,10 @@ __device__ __forceinline__ u32 raised(u32* flag) {
 __device__ __forceinline__ void raise(u32* flag) {
   __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
+// Two results as a dword, by the hardware's conversion, round to nearest even.
 __device__ __forceinline__ u32 pack(float x, float y) {
-  return f2bf(x) | (u32)f2bf(y) << 16;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+  return __builtin_bit_cast(u32, __builtin_convertvector(f32x2{x, y}, bf16x2));
 }
 __device__ __forceinline__ float lo(u32 v) { return bf2f((u16)v); }
 __device__ __forceinline__ float hi(u32 v) { return bf2f((u16)(v >> 16)); }
