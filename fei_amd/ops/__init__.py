@@ -347,7 +347,7 @@ def attn_prefill(q, k_cache, v_cache, pos0, scale: Optional[float] = None,
     if not q.numel():
         return out
     k_cache, v_cache = _cache_rows(k_cache, v_cache)
-    splits = _prefill_splits(B, Hkv, S * (Hq // Hkv), k_cache.shape[2])
+    splits = _prefill_splits(B, Hkv, S * (Hq // Hkv), k_cache.shape[2], D)
     po = pml = None
     if splits > 1:
         ws = torch.empty(B * S * Hq * splits * (D + 2), dtype=torch.float32,
@@ -373,18 +373,26 @@ def _cache_rows(k: torch.Tensor, v: torch.Tensor):
     return (t.clone(memory_format=torch.contiguous_format) for t in (k, v))
 
 
-def _prefill_splits(B: int, Hkv: int, rows: int, max_seq: int) -> int:
+def _prefill_splits(B: int, Hkv: int, rows: int, max_seq: int,
+                    dim: int = 64) -> int:
     """Shares of the keys that the prompt attention's blocks of 128 rows are
     cut into, so that few rows over many keys fill the chip's 512 places (two
-    blocks per CU). How many keys there are is known on the device only; the
-    kernel uses fewer shares where one would have under three tiles of 64, and
+    blocks per CU), or of heads of 128 a CU each, if that leaves them three shares and
+    more. One block too many is a round more, and each share's sums are written and read
+    once. 32 layers of 4096 in all, us, 512 places and one block too many, as was, and
+    now: 128 tokens over 1800 5030, 4930; 200 over 1800 6355, 6210; 300 over 2000 7860, 7575;
+    600 over 3000 12070, 11810; 760 over 6000 14250, 13925. Heads of 64 gain up to 2 %
+    from whole rounds, and lose 2 with 256 places.
+
+    How many keys there are is known on the device only; the kernel uses fewer shares where one would have under three tiles of 64, and
     one where there are few keys in all. Of ``max_seq`` that is asked here, for
     half of the ``B`` and one more as if they were long; a launch without shares
     saves 3 us and more."""
     blocks = B * Hkv * -(-rows // 128)
     if blocks > 192 or max_seq <= 64 * 6 + Hkv * rows * (B + 1) // 20:
         return 1
-    return max(1, min(16, -(-512 // blocks), max_seq // 192))
+    places = 256 if dim > 64 and 3 * blocks <= 256 else 512
+    return max(1, min(16, places // blocks, max_seq // 192))
 
 
 def _ref_bidir(q, k_cache, v_cache, kv_len, scale):
@@ -958,7 +966,7 @@ def encoder_layers(h: torch.Tensor, weights, heads: int, dim: int, inner: int,
         return torch.empty(M, n, dtype=h.dtype, device=h.device)
     h1, tmp = rows(C), rows(C)
     qkv, att, mid = rows(3 * HD), rows(HD), rows(inner)
-    splits = _prefill_splits(B, heads, S, S)
+    splits = _prefill_splits(B, heads, S, S, dim)
     po = pml = None
     if splits > 1:
         ws = torch.empty(M * heads * splits * (dim + 2), dtype=torch.float32,
@@ -1059,7 +1067,7 @@ def encoder_packed(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
             and lens.device == ids.device and lens.dtype is torch.int32
             and lens.shape == (B,) and lens.is_contiguous()
             and _tiles.types_ok(lens, *weights)
-            and _prefill_splits(B, heads, S, S) == 1):
+            and _prefill_splits(B, heads, S, S, dim) == 1):
         return None
     ptrs = _encoder_weights(weights, C, HD, inner)
     if ptrs is None:

@@ -110,7 +110,7 @@ def llama_few(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor
         bs_log, W = room.bit_length() - 1, table.shape[1]
         room = W << bs_log
     if S:
-        splits = _ops._prefill_splits(B, Hkv, S * (heads // Hkv), room)
+        splits = _ops._prefill_splits(B, Hkv, S * (heads // Hkv), room, D)
         n = M * heads * splits if splits > 1 else 0
         ws = torch.empty(n * (D + 2), dtype=torch.float32, device=h.device)
         po, pml = ws.data_ptr(), ws.data_ptr() + n * D * 4
