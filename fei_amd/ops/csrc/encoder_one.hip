@@ -17,8 +17,8 @@
 //
 // Bound by the seams, 1.5 to 1.8 us each from one phase's end to what the next has read, and
 // by the norms, which take 2.4 us of 16 rows: two rows a wave, whose instructions are 4 cycles
-// each. Whole encoders, 12 layers of 768, us, the chain's (native) first: 8 rows 307 -> 226;
-// 24 371 -> 238; 40 418 -> 280; 64 485 -> 287, 8 texts of 8 486 -> 297; 80 556 -> 361; 128 567
+// each. Whole encoders, 12 layers of 768, us, the chain's (native) first: 8 rows 307 -> 224;
+// 24 371 -> 236; 40 418 -> 276; 64 485 -> 281, 8 texts of 8 486 -> 297; 80 556 -> 361; 128 567
 // -> 440, and each further tile of 16 rows takes 25 more, where the chain takes 3. What goes
 // into a norm is handed on in float32: in bfloat16, as the chain's up to 64 rows, 24 took 234,
 // and embeddings were over ten seeds 0.391 % from float64, 0.341 now, the chain's 0.378; of
@@ -28,7 +28,7 @@
 // registers, asked for behind INNER, 4 us a layer more where blocks have items of both;
 // attention made by each block of MID for itself 440 and 614; biases and gains asked for
 // behind the wait 1.5 us a phase. All that reads asking past the L2 at once, without flags
-// first: the same; all waves looking at the flags 234 -> 249.
+// first (as ATT and MID do): the same; all waves looking at the flags 234 -> 249.
 //
 // Forward progress: see fei_chain.h. By ticket an item waits only for items of smaller
 // tickets, norms and residual come from memory, and any number of blocks comes to the end.
@@ -323,11 +323,6 @@ __device__ __forceinline__ void attend(Lds* s, u32* at, int u, int lane) {
   const int tiles = (S + 15) / 16, p = u / tiles, t = u - p * tiles;
   const int b = p / H, head = p - b * H, first = b * S;
   const int n = min(max(a.lens[b], 0), S);
-  // the head's tiles of queries, keys and values, in the text's last row
-  wait<1>(12, at, [&](int i) {
-    const int c = (i >> 2) * H * 16 + head * 16 + (i & 3) * 4 + 3, row = first + S - 1;
-    return i < 8 ? at_frag(row, c, 2 * HD) + 1 : a.v + row * (HD / 2) + head * (D / 2) + (i & 3) * 8 + 7;
-  }, s, lane);
   // keys, then queries as fragments, 8 bytes at a time; values: columns 4 l15 on of 8 keys.
   // All at once, but of more keys than there are registers for
   constexpr int NF = 2 * KT + 2, NV = 8 * KC, NOW = 2 * NF + (KT > 4 ? 0 : NV);
@@ -341,7 +336,9 @@ __device__ __forceinline__ void attend(Lds* s, u32* at, int u, int lane) {
   };
   auto need = [&](int i) { return i < 2 * NF ? i / 2 >= 2 * KT || i / 4 < tiles : (i - 2 * NF) / 8 * 32 < S; };
   u32x2 g[NOW];
-  take(g, at, off, need, s);
+  // few read it: asked for past the L2 at once, without flags first (24 rows 234.5 -> 232, 64
+  // 286 -> 280)
+  take(g, at, off, need, s, LATER);
   s16x8 f[NF];
 #pragma unroll
   for (int i = 0; i < NF; ++i) f[i] = __builtin_bit_cast(s16x8, u32x4{g[2 * i][0], g[2 * i][1], g[2 * i + 1][0], g[2 * i + 1][1]});
@@ -365,7 +362,7 @@ __device__ __forceinline__ void attend(Lds* s, u32* at, int u, int lane) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) v[i] = g[2 * NF + i];
   } else {
-    take(v, at, [&](int i) { return off(2 * NF + i); }, [&](int i) { return need(2 * NF + i); }, s);
+    take(v, at, [&](int i) { return off(2 * NF + i); }, [&](int i) { return need(2 * NF + i); }, s, LATER);
   }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {           // what lies past the keys counts 0
