@@ -817,7 +817,7 @@ k_decode_one_begin(u32* ws, long dwords, int stat, const u32* x, int C, int sums
 
 }  // namespace
 
-// vocab: rows of the head. blocks: of a launch, 256 but to have items taken by ticket.
+// vocab: rows of the head. blocks: of a launch, 256, fewer to have items taken by ticket.
 struct OneShape { int layers, C, I, Hq, Hkv, D, room, vocab, fp8, blocks; float eps, scale; };
 
 namespace {
@@ -881,7 +881,8 @@ extern "C" {
 // Bytes of room that a step takes, 0 if this cannot run it.
 long fei_decode_one_room(const OneShape* p) {
   const int HD = p->Hq * p->D, e = p->fp8 ? 16 : 8;
-  if (p->layers <= 0 || p->Hkv <= 0 || p->Hkv > BLOCKS || p->Hq % p->Hkv || p->Hq / p->Hkv > 16 ||
+  // more blocks than items would take rows past the products' ends
+  if (p->blocks < 1 || p->blocks > BLOCKS || p->layers <= 0 || p->Hkv <= 0 || p->Hkv > BLOCKS || p->Hq % p->Hkv || p->Hq / p->Hkv > 16 ||
       (p->D != 64 && p->D != 128) || p->C % e || p->I % e || HD % e || p->vocab % 2 ||
       // each item has rows, and what one wave writes of them it has registers for
       p->C < 512 || p->I < 512 || HD < 512 || p->vocab < 512 || p->C > 16384 || HD > 16384 ||

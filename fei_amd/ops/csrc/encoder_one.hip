@@ -700,7 +700,7 @@ inline int lds_of(const Encoder& a) {
 
 }  // namespace
 
-// blocks: of the launch, 256 but to have items taken by ticket.
+// blocks: of the launch, 256, fewer to have items taken by ticket.
 struct EncoderShape { int layers, B, S, H, C, I, blocks; float eps, scale; };
 
 namespace {
@@ -718,7 +718,8 @@ extern "C" {
 
 // Bytes of room that it takes, 0 where it cannot run it. Heads of 64.
 long fei_encoder_one_room(const EncoderShape* p) {
-  if (p->layers <= 0 || p->layers > MOST || p->B <= 0 || p->S <= 0 || p->B > ROWS || p->S > ROWS || p->B * p->S > ROWS ||
+  // more blocks than items would write in front of the buffers
+  if (p->blocks < 1 || p->blocks > BLOCKS || p->layers <= 0 || p->layers > MOST || p->B <= 0 || p->S <= 0 || p->B > ROWS || p->S > ROWS || p->B * p->S > ROWS ||
       p->H <= 0 || p->H > 12 || p->C <= 0 || p->C > 768 || p->I <= 0 || p->I > 3072 || p->C % 64 || p->I % 64)
     return 0;
   // so that there are no more items of a phase than blocks

@@ -159,7 +159,7 @@ def llama_one(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor
     """A decoding step of one row h [1, C], which is left as it is, in one launch of
     csrc/decode_one.hip: logits [1, vocab], or None where it does not take the step. Caches
     [1, Hkv, room, D]; keys and values are written at pos[0]. ``fp8``: of each layer the
-    products' names -> (w, scales). ``blocks``: fewer have items taken by ticket."""
+    products' names -> (w, scales). ``blocks``: up to 256; fewer have items taken by ticket."""
     M, C = h.shape
     lw, grad = layers[0], torch.is_grad_enabled()
     if not (h.is_cuda and M == 1 and k_caches[0].dim() == 4 and len(layers) > 0):
@@ -228,7 +228,7 @@ def encoder_one(ids: torch.Tensor, tok: torch.Tensor, pos: torch.Tensor,
                 blocks: int = ONE_BLOCKS) -> Optional[torch.Tensor]:
     """An encoder over up to 128 rows in one launch of csrc/encoder_one.hip, behind that
     of the embeddings: arguments and result are encoder_packed's; None where it does not
-    take them. ``blocks``: fewer have items taken by ticket."""
+    take them. ``blocks``: up to 256; fewer have items taken by ticket."""
     if not (tok.is_cuda and ids.dim() == 2 and 0 < ids.numel() <= 128 and dim == 64
             and _ops._embedding_ok(ids, tok, pos, gain, shift)):
         return None
