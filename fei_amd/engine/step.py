@@ -36,6 +36,9 @@ def upload(arrays: Sequence[np.ndarray], device: torch.device
     arrays = [np.ascontiguousarray(a) for a in arrays]
     if device.type != "cuda":
         return [torch.from_numpy(a).to(device) for a in arrays]
+    if torch.cuda.is_current_stream_capturing():
+        # a replay would copy what lies there then
+        raise RuntimeError("a step's batch cannot be built while a stream is captured")
     at, size = [], 0
     for a in arrays:
         at.append(size)

@@ -53,3 +53,10 @@ def test_plans_of_a_batch(model, lens, device):
         rows[i], at = at + lens[i] - 1, at + lens[i]
     assert batch.want_rows.tolist() == [rows[i] for i in range(len(lens))]
     assert runner.build(entries, all_rows=True).want_rows is None
+
+
+def test_upload_is_refused_under_capture(monkeypatch):
+    """A graph would copy again from memory that is others' by then."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    with pytest.raises(RuntimeError, match="captured"):
+        upload([np.zeros(3, np.int32)], torch.device("cuda"))
