@@ -29,10 +29,10 @@ Q_TILE = 128         # query rows per workgroup of the prompt attention kernel
 def upload(arrays: Sequence[np.ndarray], device: torch.device
            ) -> List[torch.Tensor]:
     """The arrays on the device, 16-byte aligned views of one copy that the current
-    stream makes and nobody waits for: a copy from ordinary memory holds the host up until
-    the GPU has done all that it was given. A step of prompts made ten of those, while the
-    GPU had little to do: 1297 rows and 4 tokens of tobarax-1b 4846 us, 4654 so; 1700 and 6
-    of bokenex-1b 4090, 3961."""
+    stream makes and nobody waits for (who reads them on another stream has to): a copy
+    from ordinary memory holds the host up until the GPU has done all that it was given. A
+    step of prompts made ten of those, while the GPU had little to do: 1297 rows and 4
+    tokens of tobarax-1b 4846 us, 4654 so; 1700 and 6 of bokenex-1b 4090, 3961."""
     arrays = [np.ascontiguousarray(a) for a in arrays]
     if device.type != "cuda":
         return [torch.from_numpy(a).to(device) for a in arrays]
@@ -67,10 +67,20 @@ class RaggedBatch:
     want_rows: Optional[torch.Tensor] = None     # [n] int64; None = all rows
     # device tensors that depend on the portions, by key (see below)
     _plans: Dict[object, object] = field(default_factory=dict)
+    # that uploads them all; None = they are there
+    stream: Optional[torch.cuda.Stream] = None
 
     @property
     def n_rows(self) -> int:
         return self.tokens.shape[0]
+
+    def settle(self) -> None:
+        """What runs from now on in the current stream finds the tensors there. A capture
+        begins behind them, and is not to wait for what is not captured."""
+        if self.stream is not None:
+            now = torch.cuda.current_stream(self.stream.device)
+            if now != self.stream and not torch.cuda.is_current_stream_capturing():
+                now.wait_stream(self.stream)
 
     def plan_arrays(self, key) -> List[np.ndarray]:
         """Of one of the plans below: "spans", ("keys", window), "chunks"."""
@@ -98,7 +108,8 @@ class RaggedBatch:
         return [np.asarray(a, dtype=np.int32).reshape(-1, w) for a, w in out]
 
     def _upload(self, rows: np.ndarray, width: int) -> torch.Tensor:
-        return upload([rows], self.tokens.device)[0].view(-1, width)
+        # for whoever asks first, and there when the host goes on
+        return torch.from_numpy(rows).view(-1, width).to(self.tokens.device)
 
     def _plan(self, key) -> List[torch.Tensor]:
         if key not in self._plans:
@@ -229,6 +240,8 @@ class StepRunner:
                   np.array(want, np.int64)]
         plans = [batch.plan_arrays(key) for key in self.plans if portions]
         dev = upload(arrays + sum(plans, []), self.device)
+        if self.device.type == "cuda":
+            batch.stream = torch.cuda.current_stream(self.device)
         (batch.tokens, batch.pos, batch.row_seq, batch.table, batch.slots,
          batch.want_rows) = dev[:6]
         if all_rows:

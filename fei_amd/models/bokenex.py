@@ -138,6 +138,7 @@ class BokenexModel(StepModel):
         """One step -> float32 logits of ``batch.want_rows`` (all rows if
         None). ``on_run(r, residual)`` is called after every layer."""
         s, dt = self.spec, self.dtype
+        batch.settle()
         x = ops.embed_pos(batch.tokens, batch.pos, self.emb, self.pos_emb)
         rows = None
         few = self._few_wanted(batch, on_run)

@@ -145,6 +145,7 @@ class TobaraxModel(StepModel):
         """One step -> float32 logits of ``batch.want_rows`` (all rows if
         None). ``on_run(r, residual)`` is called after every layer run."""
         s, dt = self.spec, self.dtype
+        batch.settle()
         x = torch.nn.functional.embedding(batch.tokens, self.emb).float()
         x0 = x.clone() if s.loop is not None else None
         normed = None

@@ -60,3 +60,26 @@ def test_upload_is_refused_under_capture(monkeypatch):
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
     with pytest.raises(RuntimeError, match="captured"):
         upload([np.zeros(3, np.int32)], torch.device("cuda"))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("model", ["tobarax-tiny", "bokenex-tiny"])
+def test_batch_of_another_stream(model):
+    """Built on a stream that has much to do yet, run on another."""
+    spec = get_spec(model)
+    m = model_class(spec)(spec, torch.device("cuda"))
+    results = []
+    for busy in (False, True):
+        runner = StepRunner(m, 64, 8, 16)
+        entries = [StepEntry(runner.admit(n), list(range(4, 4 + n)), [n - 1])
+                   for n in (70, 1, 9)]
+        torch.cuda.synchronize()
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side if busy else torch.cuda.current_stream()):
+            if busy:
+                torch.cuda._sleep(20_000_000)
+            batch = runner.build(entries)
+        with torch.no_grad():
+            results.append(m.forward(batch, runner.cache).clone())
+        torch.cuda.synchronize()
+    assert torch.equal(*results)
