@@ -339,12 +339,16 @@ class LlamaModel:
         if ssq is not None:
             ssq.zero_()
         pf = self.prefetch_mb > 0 and fp8 is None and h.is_cuda
-        done = 0
+        done, lw = 0, self.layers[0]
         # A step that is captured runs in one launch, whose 12 pointers a layer are looked
         # at before it: 10 us a layer, which a step that is not captured would wait for,
         # while the launches of one layer run under the looks at the next
         if (B == 1 and ssq is None and not (pf or fused_attn) and h.is_cuda
-                and torch.cuda.is_current_stream_capturing()):
+                and torch.cuda.is_current_stream_capturing()
+                and ops.llama_one_pays(
+                    len(self.layers),
+                    sum(w.numel() for w in (lw.wqkv, lw.wo, lw.wgu, lw.wdown)),
+                    self.lm_head.numel(), fp8 is not None)):
             logits = ops.llama_one(
                 h, self.layers, k_caches, v_caches, self.hq_l, s.norm_eps, pos,
                 self.rope, self.norm_f, self.lm_head, fp8,

@@ -26,7 +26,8 @@ from fei_amd.ops import reference as ref
 from fei_amd.ops import rows as _rows
 from fei_amd.ops import sigmoid_attn as _sigmoid_attn
 from fei_amd.ops import tiles as _tiles
-from fei_amd.ops.layers import encoder_one, llama_few, llama_one  # noqa: F401
+from fei_amd.ops.layers import (  # noqa: F401
+    encoder_one, llama_few, llama_one, llama_one_pays)
 from fei_amd.ops.mixers import (  # noqa: F401
     GainNorm, GainNormed, cat_cast, check_gla_geometry,
     check_latent_geometry, embed_pos, gain_logits, gla_decode, gla_mixed, gla_prefill,

@@ -150,6 +150,21 @@ def llama_few(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor
     return done, sums if done and M > 1 else None
 
 
+def llama_one_pays(layers: int, weights: int, head: int, fp8: bool) -> bool:
+    """Whether a captured step of one row is faster in one launch than as a chain, by the
+    numbers of weights of a layer and of the head. The launch costs 10 us more, and gains a
+    layer what the chain's five launches cost beyond their bytes: of few weights nothing, as
+    its seams are no shorter; fp8's are as long for half the bytes. Steps of 30 keys by a
+    graph, us, the chain's first. Layers of 1.8 million weights: 2 of them 46, 58; 24 434,
+    463. Of 6: 12 245, 245, 24 482, 469; of 8.9: 8 171, 174; of 12.8 and 15.9: 8 191, 178
+    and 200, 186; of 44: 24 763, 670; of 61, two and three 83, 85 and 119, 115. fp8: of 12.8
+    24 522, 530; of 25 8 203, 199 (1000 keys 210, 214); of 34.6 8 228, 209; of 44 24 666,
+    597; of 61, two and three 71, 74 and 100, 99. The head's product is no faster: of 262
+    million weights behind layers of 61 takes 4 of them as long, 223, and 8 370, 354."""
+    return (weights >= (32 if fp8 else 10) * 10 ** 6
+            and layers * weights >= max(120 * 10 ** 6, head))
+
+
 def llama_one(h: torch.Tensor, layers: Sequence, k_caches: Sequence[torch.Tensor],
               v_caches: Sequence[torch.Tensor], heads: int, eps: float,
               pos: torch.Tensor, rope: torch.Tensor, norm: torch.Tensor,

@@ -27,3 +27,59 @@ def test_blocks_of_a_launch(kind):
         assert room(kind, blocks) == want
     for blocks in (-1, 0, 257, 512):
         assert room(kind, blocks) == 0
+
+
+def weights(C, I, heads, kv_heads, dim):
+    return C * dim * (2 * heads + 2 * kv_heads) + 3 * C * I
+
+
+# sizes (a layer's and the head's), layers, and whether the one launch was measured to be
+# faster: bfloat16, fp8
+@pytest.mark.parametrize("sizes,vocab,layers,want", [
+    ((512, 512, 8, 8, 64), 512, 24, (False, False)),
+    ((1024, 1024, 16, 4, 64), 1024, 24, (False, False)),
+    ((1024, 2048, 16, 4, 64), 4000, 16, (False, False)),
+    ((1280, 3072, 20, 5, 64), 4000, 8, (True, False)),
+    ((1536, 4096, 12, 4, 128), 1024, 4, (False, False)),
+    ((1536, 6144, 12, 4, 128), 4000, 8, (True, True)),
+    ((2048, 5632, 32, 4, 64), 32000, 1, (False, False)),
+    ((2048, 5632, 32, 4, 64), 32000, 24, (True, True)),
+    ((2048, 8192, 32, 8, 64), 128256, 4, (False, False)),
+    ((2048, 8192, 32, 8, 64), 128256, 16, (True, True)),
+    ((4096, 14336, 32, 8, 128), 128256, 32, (True, True))])
+def test_steps_that_one_launch_is_faster_for(sizes, vocab, layers, want):
+    w, head = weights(*sizes), vocab * sizes[0]
+    assert tuple(ops.llama_one_pays(layers, w, head, f) for f in (False, True)) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layers,C,taken", [(2, 512, False), (12, 512, False),
+                                            (8, 1280, True)])
+def test_route_of_a_captured_step(layers, C, taken, monkeypatch):
+    import torch
+
+    from fei_amd.engine.config import ModelSpec
+    from fei_amd.models.llama import LlamaModel
+    calls, real = [], ops.llama_one
+    monkeypatch.setattr(ops, "llama_one",
+                        lambda *a, **k: calls.append(real(*a, **k)) or calls[-1])
+    spec = ModelSpec("route", 1024, C, layers, C // 64, C // 256, 64, 3 * C)
+    m = LlamaModel(spec, torch.device("cuda:0"), torch.bfloat16, seed=1, max_seq_len=64)
+    tok = torch.tensor([7], dtype=torch.int32, device="cuda:0")
+    pos = torch.tensor([3], dtype=torch.int32, device="cuda:0")
+    kc, vc = m.new_kv_cache(1, 64)
+    with torch.no_grad():
+        want = m.forward_decode(tok, pos, kc, vc)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            got = m.forward_decode(tok, pos, kc, vc)
+    assert len(calls) == taken and all(c is not None for c in calls)
+    for _ in range(3):
+        got.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        if taken:
+            assert (got - want).float().norm() < 2 ** -6 * want.float().norm()
+        else:
+            assert torch.equal(got, want)
