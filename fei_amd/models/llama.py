@@ -349,6 +349,11 @@ class LlamaModel:
                     len(self.layers),
                     sum(w.numel() for w in (lw.wqkv, lw.wo, lw.wgu, lw.wdown)),
                     self.lm_head.numel(), fp8 is not None)):
+            # the chain's, which is refused what it has no room for
+            assert attn_splits <= 64, "at most 64 splits"
+            assert workspace is None or all(
+                t.shape[2] == attn_splits for t in workspace[:2]), \
+                f"workspace of other sizes than {attn_splits} splits"
             logits = ops.llama_one(
                 h, self.layers, k_caches, v_caches, self.hq_l, s.norm_eps, pos,
                 self.rope, self.norm_f, self.lm_head, fp8,

@@ -4,8 +4,11 @@ alone where nothing says gpu."""
 import ctypes
 
 import pytest
+import torch
 
 from fei_amd import ops
+from fei_amd.engine.config import ModelSpec
+from fei_amd.models.llama import LlamaModel
 from fei_amd.ops.layers import _EncoderShape, _OneShape
 
 
@@ -52,19 +55,19 @@ def test_steps_that_one_launch_is_faster_for(sizes, vocab, layers, want):
     assert tuple(ops.llama_one_pays(layers, w, head, f) for f in (False, True)) == want
 
 
+def model(layers, C):
+    spec = ModelSpec("route", 1024, C, layers, C // 64, C // 256, 64, 3 * C)
+    return LlamaModel(spec, torch.device("cuda:0"), torch.bfloat16, seed=1, max_seq_len=64)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layers,C,taken", [(2, 512, False), (12, 512, False),
                                             (8, 1280, True)])
 def test_route_of_a_captured_step(layers, C, taken, monkeypatch):
-    import torch
-
-    from fei_amd.engine.config import ModelSpec
-    from fei_amd.models.llama import LlamaModel
     calls, real = [], ops.llama_one
     monkeypatch.setattr(ops, "llama_one",
                         lambda *a, **k: calls.append(real(*a, **k)) or calls[-1])
-    spec = ModelSpec("route", 1024, C, layers, C // 64, C // 256, 64, 3 * C)
-    m = LlamaModel(spec, torch.device("cuda:0"), torch.bfloat16, seed=1, max_seq_len=64)
+    m = model(layers, C)
     tok = torch.tensor([7], dtype=torch.int32, device="cuda:0")
     pos = torch.tensor([3], dtype=torch.int32, device="cuda:0")
     kc, vc = m.new_kv_cache(1, 64)
@@ -83,3 +86,32 @@ def test_route_of_a_captured_step(layers, C, taken, monkeypatch):
             assert (got - want).float().norm() < 2 ** -6 * want.float().norm()
         else:
             assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [False, True])
+@pytest.mark.parametrize("layers,C", [(2, 512), (8, 2048)])
+@pytest.mark.parametrize("splits,room", [(32, 16), (16, 32), (65, 65)])
+def test_what_a_captured_step_refuses(layers, C, splits, room, fp8):
+    """Where it runs in one launch too, which has no use for a workspace."""
+    m = model(layers, C)
+    if fp8:
+        m.quantize_fp8()
+    tok = torch.tensor([7], dtype=torch.int32, device="cuda:0")
+    pos = torch.tensor([3], dtype=torch.int32, device="cuda:0")
+    kc, vc = m.new_kv_cache(1, 64)
+    ws = [torch.zeros(1, C // 64, room, n, device="cuda:0") for n in (64, 2)]
+
+    def step():
+        with pytest.raises(AssertionError):
+            m.forward_decode(tok, pos, kc, vc, attn_splits=splits, workspace=ws,
+                             fused_norm=fp8)
+        return tok + 1
+    with torch.no_grad():
+        step()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = step()
+    g.replay()
+    assert out.item() == 8
