@@ -100,10 +100,14 @@ class BgeEncoder:
         kv_len = (lengths.to(torch.int32) if lengths is not None
                   else torch.full((B,), S, dtype=torch.int32, device=self.device))
         weights = [lw[n] for lw in self.layers for n in NAMES]
-        out = ops.encoder_one(*embed, weights, H, D, s.intermediate_size, kv_len,
-                              self.eps)
-        if out is not None:
-            return out
+        # of one and two layers the one launch's start costs more than their seams:
+        # captured, us, the chain's first, one layer of 768 and 8 rows 40, 40, 128 64,
+        # 73, two of 128 and 64 rows 64, 62, 100 75, 83; four of 256 and 128 140, 137
+        if len(self.layers) > 2 or B * S <= 32 * len(self.layers):
+            out = ops.encoder_one(*embed, weights, H, D, s.intermediate_size, kv_len,
+                                  self.eps)
+            if out is not None:
+                return out
         if pack:
             out = ops.encoder_packed(*embed, weights, H, D, s.intermediate_size,
                                      kv_len, self.eps)

@@ -115,3 +115,20 @@ def test_what_a_captured_step_refuses(layers, C, splits, room, fp8):
             out = step()
     g.replay()
     assert out.item() == 8
+
+
+@pytest.mark.parametrize("layers,B,S,taken", [(1, 1, 32, True), (1, 3, 11, False),
+                                              (2, 4, 16, True), (2, 5, 13, False),
+                                              (3, 1, 128, True), (12, 128, 1, True)])
+def test_encoders_that_one_launch_is_faster_for(layers, B, S, taken, monkeypatch):
+    import dataclasses
+
+    from fei_amd.engine.config import get_spec
+    from fei_amd.models.bge import BgeEncoder
+    spec = dataclasses.replace(get_spec("bge-base"), num_layers=layers, num_heads=1,
+                               num_kv_heads=1, hidden_size=64, intermediate_size=64)
+    m = BgeEncoder(spec, device=torch.device("cpu"), dtype=torch.float32)
+    asked = []
+    monkeypatch.setattr(ops, "encoder_one", lambda *a: asked.append(1))
+    m.encode_ids(torch.ones(B, S, dtype=torch.int64))
+    assert bool(asked) == taken
