@@ -43,6 +43,10 @@ class BgeEncoder:
         self.dtype = dtype
         self.max_seq_len = min(max_seq_len, self.spec.max_seq_len)
         self.eps = 1e-12 if device.type == "cpu" else 1e-6   # BERT uses 1e-12
+        # Up to 128 rows in one launch, which keeps all CUs while it runs: two encoders on
+        # two streams take 239 us each of 24 tokens, 216 without. Not for those who
+        # run much side by side
+        self.one_launch = True
         self._init_weights(seed)
 
     def _init_weights(self, seed: int) -> None:
@@ -103,7 +107,7 @@ class BgeEncoder:
         # of one and two layers the one launch's start costs more than their seams:
         # captured, us, the chain's first, one layer of 768 and 8 rows 40, 40, 128 64,
         # 73, two of 128 and 64 rows 64, 62, 100 75, 83; four of 256 and 128 140, 137
-        if len(self.layers) > 2 or B * S <= 32 * len(self.layers):
+        if self.one_launch and (len(self.layers) > 2 or B * S <= 32 * len(self.layers)):
             out = ops.encoder_one(*embed, weights, H, D, s.intermediate_size, kv_len,
                                   self.eps)
             if out is not None:

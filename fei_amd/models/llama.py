@@ -78,6 +78,15 @@ class LlamaModel:
         # atomics + block barrier + per-step zeroing cost ~84 us/step.
         # Kept opt-in for re-measurement on future silicon.
         self.norm_precomp = os.environ.get("FEI_NORM_PRECOMP", "0") == "1"
+        # Captured steps of one row run in one launch where that is faster. It keeps all CUs
+        # while it runs, and what is launched beside it waits, where a chain of launches lets
+        # others' in between: two steps on two streams, us each, one launch and without, 1B,
+        # 300 keys 598, 468 (alone 607, 646), 8B, 512 keys 2626, 2322 (2640, 2876); an
+        # embedding of 24 tokens that starts beside 8B's is there after 2140, 830. And its
+        # sums are in another order than those of steps that are not captured: logits of the
+        # same state are alike to 1 %, as those of any two orders, not to the bit. Not for
+        # those who run much side by side, or compare captured with eager steps
+        self.one_launch = True
 
     def resize(self, max_seq_len: int) -> None:
         """Positions up to ``max_seq_len`` - 1 can be run from now on."""
@@ -343,8 +352,8 @@ class LlamaModel:
         # A step that is captured runs in one launch, whose 12 pointers a layer are looked
         # at before it: 10 us a layer, which a step that is not captured would wait for,
         # while the launches of one layer run under the looks at the next
-        if (B == 1 and ssq is None and not (pf or fused_attn) and h.is_cuda
-                and torch.cuda.is_current_stream_capturing()
+        if (self.one_launch and B == 1 and ssq is None and not (pf or fused_attn)
+                and h.is_cuda and torch.cuda.is_current_stream_capturing()
                 and ops.llama_one_pays(
                     len(self.layers),
                     sum(w.numel() for w in (lw.wqkv, lw.wo, lw.wgu, lw.wdown)),

@@ -63,11 +63,15 @@ def model(layers, C):
 @pytest.mark.gpu
 @pytest.mark.parametrize("layers,C,taken", [(2, 512, False), (12, 512, False),
                                             (8, 1280, True)])
-def test_route_of_a_captured_step(layers, C, taken, monkeypatch):
+@pytest.mark.parametrize("wanted", [True, False])
+def test_route_of_a_captured_step(layers, C, taken, wanted, monkeypatch):
+    """In one launch where that is faster and wanted; else with an eager step's bits."""
+    taken = taken and wanted
     calls, real = [], ops.llama_one
     monkeypatch.setattr(ops, "llama_one",
                         lambda *a, **k: calls.append(real(*a, **k)) or calls[-1])
     m = model(layers, C)
+    m.one_launch = wanted
     tok = torch.tensor([7], dtype=torch.int32, device="cuda:0")
     pos = torch.tensor([3], dtype=torch.int32, device="cuda:0")
     kc, vc = m.new_kv_cache(1, 64)
@@ -132,3 +136,6 @@ def test_encoders_that_one_launch_is_faster_for(layers, B, S, taken, monkeypatch
     monkeypatch.setattr(ops, "encoder_one", lambda *a: asked.append(1))
     m.encode_ids(torch.ones(B, S, dtype=torch.int64))
     assert bool(asked) == taken
+    m.one_launch = False
+    m.encode_ids(torch.ones(B, S, dtype=torch.int64))
+    assert len(asked) == taken
