@@ -900,17 +900,20 @@ def test_when_a_prompts_last_rows_are_taken_out(lib, B, S, taken, monkeypatch):
                                          # tiles enough without parts of K
                                          (2, 350, [350, 17]), (2, 512, None),
                                          (5, 205, None)])   # layer by layer
-def test_encoder_layers_from_one_call(lib, B, S, lengths):
+def test_encoder_layers_from_one_call(lib, B, S, lengths, monkeypatch):
     from fei_amd.models.bge import BgeEncoder
     m = BgeEncoder(device=torch.device(DEV))
     ids = torch.randint(0, 1000, (B, S), device=DEV)
     n = None if lengths is None else torch.tensor(lengths, device=DEV)
+    # what one launch, or the rows that texts have, would run
+    monkeypatch.setattr(lib, "encoder_one", lambda *a: None)
+    monkeypatch.setattr(lib, "encoder_packed", lambda *a: None)
+    ran, layers = [], lib.encoder_layers
+    monkeypatch.setattr(lib, "encoder_layers", lambda *a: ran.append(layers(*a)) or ran[-1])
     got = m.encode_ids(ids, n)
-    before, lib.encoder_layers = lib.encoder_layers, lambda *a: None
-    try:
-        want = m.encode_ids(ids, n)
-    finally:
-        lib.encoder_layers = before
+    assert [r is not None for r in ran] == [B * S <= lib.ENCODER_ROWS]
+    monkeypatch.setattr(lib, "encoder_layers", lambda *a: None)
+    want = m.encode_ids(ids, n)
     if not 32 < B * S <= lib.ENCODER_ROWS:   # the same kernels in the same order
         assert torch.equal(got, want)
     else:
@@ -921,7 +924,7 @@ def test_encoder_layers_from_one_call(lib, B, S, lengths):
 
 @pytest.mark.parametrize("B,S", [(3, 1), (1, 8), (1, 9), (2, 8), (1, 17), (5, 5)])
 @pytest.mark.parametrize("heads,inner", [(12, 3072), (1, 64), (16, 128)])
-def test_encoder_norms_inside_products(lib, B, S, heads, inner):
+def test_encoder_norms_inside_products(lib, B, S, heads, inner, monkeypatch):
     """Up to 24 rows: the same sums in the same order as with a launch for each
     norm, at the edges of the rows, and of widths that leave lanes without columns
     or a wave without steps."""
@@ -939,12 +942,13 @@ def test_encoder_norms_inside_products(lib, B, S, heads, inner):
         for n in ("bqkv", "bo", "bi", "bo2", "ln1_b", "ln2_b"):
             lw[n].copy_(randbf(lw[n].numel(), seed=i + 9) * 0.1)
     ids = torch.randint(0, 1000, (B, S), device=DEV)
+    monkeypatch.setattr(lib, "encoder_one", lambda *a: None)
+    ran, layers = [], lib.encoder_layers
+    monkeypatch.setattr(lib, "encoder_layers", lambda *a: ran.append(layers(*a)) or ran[-1])
     got = m.encode_ids(ids)
-    before, lib.encoder_layers = lib.encoder_layers, lambda *a: None
-    try:
-        want = m.encode_ids(ids)
-    finally:
-        lib.encoder_layers = before
+    assert len(ran) == 1 and ran[0] is not None
+    monkeypatch.setattr(lib, "encoder_layers", lambda *a: None)
+    want = m.encode_ids(ids)
     assert got.isfinite().all() and torch.equal(got, want)
 
 
