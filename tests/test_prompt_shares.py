@@ -21,8 +21,21 @@ def test_shares_fill_whole_rounds(dim):
                     blocks = B * Hkv * -(-rows // 128)
                     assert 1 <= n <= 16
                     assert n == 1 or (n * blocks <= 512 and n * 192 <= max_seq)
-                    if n > 1 and dim == 128 and blocks <= 85:
-                        assert n * blocks <= 256
+                    places = 256 if dim == 128 and blocks <= 85 else 512
+                    if n > 1:
+                        assert n * blocks <= places
+                        # and no more do, of 16 and of three tiles of 64 keys each
+                        assert (n == min(16, max_seq // 192)
+                                or (n + 1) * blocks > places)
+
+
+# on both sides of the blocks at which the rule changes
+@pytest.mark.parametrize("blocks,wide,narrow", [
+    (1, 16, 16), (16, 16, 16), (24, 10, 16), (32, 8, 16), (64, 4, 8), (85, 3, 6),
+    (86, 5, 5), (128, 4, 4), (170, 3, 3), (171, 2, 2), (192, 2, 2), (193, 1, 1)])
+def test_shares_of_blocks(blocks, wide, narrow):
+    assert ops._prefill_splits(1, 1, 128 * blocks, 10 ** 6, 128) == wide
+    assert ops._prefill_splits(1, 1, 128 * blocks, 10 ** 6, 64) == narrow
 
 
 # 8 heads of keys, 4 queries each: 10 and 11 blocks of rows a head lie on either side of 85
@@ -37,7 +50,9 @@ def test_shares_against_float32(S, P, D):
     q = torch.randn(1, S, 32, D, generator=g, device=DEV).to(torch.bfloat16)
     k, v = (torch.randn(1, 8, T, D, generator=g, device=DEV).to(torch.bfloat16)
             for _ in range(2))
-    assert ops._prefill_splits(1, 8, 4 * S, T, D) > 1
+    blocks = 8 * -(-4 * S // 128)
+    places = 256 if D == 128 and blocks <= 85 else 512
+    assert ops._prefill_splits(1, 8, 4 * S, T, D) == min(16, T // 192, places // blocks) > 1
     pos0 = torch.tensor([P], dtype=torch.int32, device=DEV)
     got = ops.attn_prefill(q, k, v, pos0, scale=D ** -0.5).float()
     hide = torch.arange(T, device=DEV) > torch.arange(P, T, device=DEV).unsqueeze(1)
