@@ -380,15 +380,18 @@ def _prefill_splits(B: int, Hkv: int, rows: int, max_seq: int,
     cut into, so that few rows over many keys fill the chip's 512 places (two
     blocks per CU), or of heads of 128 a CU each, if that leaves them three shares and
     more. One block too many is a round more, and each share's sums are written and read
-    once. 32 layers of 4096 in all, us, 512 places and one block too many, as was, and
-    now: 128 tokens over 1800 5030, 4930; 200 over 1800 6355, 6210; 300 over 2000 7860, 7575;
-    600 over 3000 12070, 11810; 760 over 6000 14250, 13925. Heads of 64 gain up to 2 %
-    from whole rounds, and lose 2 with 256 places.
+    once. 32 layers of 4096 in all, us, by 512 places and one block too many / 512 / 256:
+    65 tokens over 2500 keys 4262 / 4262 / 4200, over 7500 4550 / 4550 / 4478; 75 4348 /
+    4348 / 4282, 4623 / 4623 / 4539; 96 4540 / 4540 / 4410, 4832 / 4832 / 4703; 128 5090 /
+    5090 / 4925, 5463 / 5463 / 5308; 192 6400 / 6192 / 6037, 6990 / 6708 / 6587; 320 8033 /
+    7743 / 7711, 8979 / 8512 / 8678; four prompts of 40 over 3000 6303 / 6303 / 5975. Heads
+    of 64 gain up to 2 % from whole rounds, and lose with 256 places: 16 layers of 2048, 600
+    over 4000, 2730 / 2711 / 2987.
 
-    How many keys there are is known on the device only; the kernel uses fewer shares where one would have under three tiles of 64, and
-    one where there are few keys in all. Of ``max_seq`` that is asked here, for
-    half of the ``B`` and one more as if they were long; a launch without shares
-    saves 3 us and more."""
+    How many keys there are is known on the device only; the kernel uses fewer
+    shares where one would have under three tiles of 64, and one where there are
+    few keys in all. Of ``max_seq`` that is asked here, for half of the ``B`` and
+    one more as if they were long; a launch without shares saves 3 us and more."""
     blocks = B * Hkv * -(-rows // 128)
     if blocks > 192 or max_seq <= 64 * 6 + Hkv * rows * (B + 1) // 20:
         return 1

@@ -17,25 +17,32 @@
 // the stores 4.0, counters 4.9.
 //
 // The other 8 waves multiply: a step is 2 rows of w times 2 loads of 16 bytes a lane, two
-// steps are in flight a wave and are asked for before the input is there (three, or half of
-// two, are no better: 1813 us, the fp8 case below, 1812 and 1832 then). A CU's loads come
+// steps are in flight a wave and are asked for before the input is there. A CU's loads come
 // back in order, whoever asked, so the serving wave has none of its own, asks only when the
-// weights should have come (1.35 us: at once 1744 us, after 0.8 us 1739, 1.35 1723, 1.9
-// 1739), and goes before the others, whose next loads its results would wait behind (its
-// priority: 1904 -> 1720 us; 642 -> 616 for the first case below).
+// weights should have come (1.35 us), and goes before the others, whose next loads its
+// results would wait behind. Of the three steps below, us, all as it is 604, 2664, 1706; three
+// steps in flight 600, 2588, 1715, half of two 633, 2772, 1763; asking at once 624, 2712, 1733,
+// after 0.8 us 612, 2664, 1722, after 1.9 619, 2642, 1710; nobody before others 617, 2655, 1793.
 //
 // Forward progress. Blocks count themselves at the start. If all 256 are there within 100
 // looks, all of them are on the chip, and each keeps its item of every phase. If not,
 // whatever holds the other CUs, items are taken by ticket, in the order of the phases: an
 // item waits only for items of smaller tickets, which blocks that run have taken, so that
-// any number of blocks, one too, comes to the end. Waits end after LIMIT looks all the
-// same; nothing but a fault of this file would make them, and the logits are NaN then.
+// any number of blocks, one too, comes to the end. Nothing is asked for ahead then: with 255
+// blocks the three take 858, 3785 and 2447. Waits end after LIMIT looks all the same; nothing
+// but a fault of this file would make them, and the logits are NaN then. The launch keeps
+// every CU to its end, so that two steps side by side are slower than as chains, whose
+// launches run in between one another's: two of the first case 598 each and 468, of the
+// second 2626 and 2322.
 //
 // Bound by HBM while products run (27 to 30 KB a us and CU, 7 TB/s) and by the seams, 2 to
 // 3 us each; the eight XCDs get 5 % more or less of it, and all wait for the last. Whole
-// steps by a graph, embedding and sampling left out, us, the chain's first: 16 layers of
-// 2048, 300 keys 662 -> 609; 32 of 4096, 512 keys 2885 -> 2657; fp8 weights, 3400 keys
-// 2030 -> 1711.
+// steps by a graph, which is played again, with the embedding, us, the chain's first: 16
+// layers of 2048, 300 keys 646 -> 604; 32 of 4096, 512 keys 2883 -> 2664; fp8 weights, 3400
+// keys 1996 -> 1706 (each time other keys, from HBM: 2034 -> 1762). Four layers of 2048 and
+// 3400 keys 172 -> 156, 32000 205 -> 186, 131000 349 -> 330, of 4096 365 -> 341, 445 -> 419,
+// 723 -> 710: of so many keys a wave has no loads ahead of the 32 it works on. Which
+// steps are taken: ops.llama_one_pays.
 #include "fei_attn.h"
 #include "fei_chain.h"
 

@@ -442,7 +442,9 @@ void fei_encoder_layers(const void* const* w, int layers, void* h, void* h1,
     fei_add_layernorm(to, tmp, from, wb[2], wb[3], M, C, eps, 1, stream);
   };
   if (M <= 24 && C <= 1024) {
-    // the norms inside the products behind them, but the last
+    // The norms inside the products behind them, but the last. What comes here is what the
+    // one launch of encoder_one.hip does not take: widths beyond 768 (inner ones 3072, 12
+    // heads), more than 32 layers, models that are to leave CUs to others, fewer CUs
     auto behind = [&](void* out, const void* res, const void* const* norm,
                       void* normed, const void* const* wb, int N, bool gelu) {
       auto run = [&](auto launch) {
