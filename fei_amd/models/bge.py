@@ -30,6 +30,11 @@ NAMES = ("wqkv", "bqkv", "wo", "bo", "ln1_w", "ln1_b", "wi", "bi", "wo2", "bo2",
 
 
 class BgeEncoder:
+    # Up to 128 rows in one launch, which keeps all CUs while it runs: two encoders on
+    # two streams take 239 us each of 24 tokens, 216 without. Not for those who
+    # run much side by side
+    one_launch = True
+
     def __init__(self, spec: Optional[ModelSpec] = None,
                  device: Optional[torch.device] = None,
                  dtype: Optional[torch.dtype] = None, seed: int = 42,
@@ -43,10 +48,6 @@ class BgeEncoder:
         self.dtype = dtype
         self.max_seq_len = min(max_seq_len, self.spec.max_seq_len)
         self.eps = 1e-12 if device.type == "cpu" else 1e-6   # BERT uses 1e-12
-        # Up to 128 rows in one launch, which keeps all CUs while it runs: two encoders on
-        # two streams take 239 us each of 24 tokens, 216 without. Not for those who
-        # run much side by side
-        self.one_launch = True
         self._init_weights(seed)
 
     def _init_weights(self, seed: int) -> None:

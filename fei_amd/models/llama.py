@@ -37,6 +37,16 @@ class LayerWeights:
 
 
 class LlamaModel:
+    # Captured steps of one row run in one launch where that is faster. It keeps all CUs
+    # while it runs, and what is launched beside it waits, where a chain of launches lets
+    # others' in between: two steps on two streams, us each, one launch and without, 1B,
+    # 300 keys 598, 468 (alone 607, 646), 8B, 512 keys 2626, 2322 (2640, 2876); an
+    # embedding of 24 tokens that starts beside 8B's is there after 2140, 830. And its
+    # sums are in another order than those of steps that are not captured: logits of the
+    # same state are alike to 1 %, as those of any two orders, not to the bit. Not for
+    # those who run much side by side, or compare captured with eager steps
+    one_launch = True
+
     def __init__(
         self,
         spec: ModelSpec,
@@ -78,15 +88,6 @@ class LlamaModel:
         # atomics + block barrier + per-step zeroing cost ~84 us/step.
         # Kept opt-in for re-measurement on future silicon.
         self.norm_precomp = os.environ.get("FEI_NORM_PRECOMP", "0") == "1"
-        # Captured steps of one row run in one launch where that is faster. It keeps all CUs
-        # while it runs, and what is launched beside it waits, where a chain of launches lets
-        # others' in between: two steps on two streams, us each, one launch and without, 1B,
-        # 300 keys 598, 468 (alone 607, 646), 8B, 512 keys 2626, 2322 (2640, 2876); an
-        # embedding of 24 tokens that starts beside 8B's is there after 2140, 830. And its
-        # sums are in another order than those of steps that are not captured: logits of the
-        # same state are alike to 1 %, as those of any two orders, not to the bit. Not for
-        # those who run much side by side, or compare captured with eager steps
-        self.one_launch = True
 
     def resize(self, max_seq_len: int) -> None:
         """Positions up to ``max_seq_len`` - 1 can be run from now on."""

@@ -139,3 +139,10 @@ def test_encoders_that_one_launch_is_faster_for(layers, B, S, taken, monkeypatch
     m.one_launch = False
     m.encode_ids(torch.ones(B, S, dtype=torch.int64))
     assert len(asked) == taken
+
+
+def test_models_that_were_kept_from_before():
+    """What was pickled without the attribute runs."""
+    from fei_amd.models.bge import BgeEncoder
+    for cls in (LlamaModel, BgeEncoder):
+        assert cls.__new__(cls).one_launch
