@@ -67,8 +67,9 @@ class RaggedBatch:
     want_rows: Optional[torch.Tensor] = None     # [n] int64; None = all rows
     # device tensors that depend on the portions, by key (see below)
     _plans: Dict[object, object] = field(default_factory=dict)
-    # that uploads them all; None = they are there
-    stream: Optional[torch.cuda.Stream] = None
+    # the stream that uploads them all, by its numbers, as batches are copied; None = they
+    # are there
+    stream: Optional[Dict[str, int]] = None
 
     @property
     def n_rows(self) -> int:
@@ -78,9 +79,11 @@ class RaggedBatch:
         """What runs from now on in the current stream finds the tensors there. A capture
         begins behind them, and is not to wait for what is not captured."""
         if self.stream is not None:
-            now = torch.cuda.current_stream(self.stream.device)
-            if now != self.stream and not torch.cuda.is_current_stream_capturing():
-                now.wait_stream(self.stream)
+            now = torch.cuda.current_stream(self.stream["device_index"])
+            if (now.stream_id != self.stream["stream_id"]
+                    and not torch.cuda.is_current_stream_capturing()):
+                now.wait_stream(torch.cuda.Stream(**self.stream))
+                self.table.record_stream(now)    # and all that was uploaded with it
 
     def plan_arrays(self, key) -> List[np.ndarray]:
         """Of one of the plans below: "spans", ("keys", window), "chunks"."""
@@ -241,7 +244,9 @@ class StepRunner:
         plans = [batch.plan_arrays(key) for key in self.plans if portions]
         dev = upload(arrays + sum(plans, []), self.device)
         if self.device.type == "cuda":
-            batch.stream = torch.cuda.current_stream(self.device)
+            now = torch.cuda.current_stream(self.device)
+            batch.stream = {n: getattr(now, n) for n in (
+                "stream_id", "device_index", "device_type")}
         (batch.tokens, batch.pos, batch.row_seq, batch.table, batch.slots,
          batch.want_rows) = dev[:6]
         if all_rows:

@@ -1,6 +1,8 @@
 """What a step's batch is uploaded with (engine/step.py): one copy, from which the plans
 of the model's mixers are views, the same as those made when they are asked for."""
 
+import copy
+
 import numpy as np
 import pytest
 import torch
@@ -65,11 +67,11 @@ def test_upload_is_refused_under_capture(monkeypatch):
 @pytest.mark.gpu
 @pytest.mark.parametrize("model", ["tobarax-tiny", "bokenex-tiny"])
 def test_batch_of_another_stream(model):
-    """Built on a stream that has much to do yet, run on another."""
+    """Built on a stream that has much to do yet, run on another, as is and copied."""
     spec = get_spec(model)
     m = model_class(spec)(spec, torch.device("cuda"))
     results = []
-    for busy in (False, True):
+    for busy in (None, lambda b: b, copy.copy):
         runner = StepRunner(m, 64, 8, 16)
         entries = [StepEntry(runner.admit(n), list(range(4, 4 + n)), [n - 1])
                    for n in (70, 1, 9)]
@@ -79,7 +81,10 @@ def test_batch_of_another_stream(model):
             if busy:
                 torch.cuda._sleep(20_000_000)
             batch = runner.build(entries)
+            waits = batch.stream["stream_id"]
+        assert (waits == torch.cuda.current_stream().stream_id) == (busy is None)
+        batch = busy(batch) if busy else batch
         with torch.no_grad():
             results.append(m.forward(batch, runner.cache).clone())
         torch.cuda.synchronize()
-    assert torch.equal(*results)
+    assert all(torch.equal(r, results[0]) for r in results)
